@@ -18,11 +18,10 @@
 // to the exact factors. Eigenvectors and singular vectors are determined up to a
 // unit phase per vector, which is not fixed by either implementation.
 //
-// How it runs: correctness first, one workgroup per matrix of the batch, the
-// matrix in a contiguous double-precision workspace (the strided, any-dtype
-// operands are brought in and results sent out by nxh_cast).
-//   cholesky      left-looking columns, one row per lane
-//   tri. solve    right-looking substitution, all right-hand sides in parallel
+// How it runs. Cholesky and the triangular solve go by blocks (linalg_blocked.hpp), reading and
+// writing float32 / float64 / complex128 operands where they are. The others: correctness
+// first, one workgroup per matrix of the batch, the matrix in a contiguous double-precision
+// workspace (the strided, any-dtype operands are brought in and results sent out by nxh_cast).
 //   qr            Householder columns, one wave per trailing column
 //   eigh          two-sided Jacobi with a round-robin ordering: n/2 disjoint
 //                 rotations per round, applied as a column phase and a row phase
@@ -53,6 +52,7 @@ struct Sc<double> {
   __device__ __forceinline__ static double abs2(double x) { return x * x; }
   __device__ __forceinline__ static double make(double r, double) { return r; }
   __device__ __forceinline__ static double scale(double x, double r) { return x * r; }
+  __device__ __forceinline__ static double sub_mul(double acc, double x, double y) { return fma(-x, y, acc); }
 };
 template <>
 struct Sc<c64> {
@@ -62,6 +62,7 @@ struct Sc<c64> {
   __device__ __forceinline__ static double abs2(c64 x) { return x.re * x.re + x.im * x.im; }
   __device__ __forceinline__ static c64 make(double r, double i) { return {r, i}; }
   __device__ __forceinline__ static c64 scale(c64 x, double r) { return {x.re * r, x.im * r}; }
+  __device__ __forceinline__ static c64 sub_mul(c64 acc, c64 x, c64 y) { return acc - x * y; }
 };
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -84,81 +85,7 @@ __device__ T block_sum(T v, T *scratch) {
 
 __device__ __forceinline__ void raise(int *status, int code) { atomicMax(status, code); }
 
-// ── cholesky ────────────────────────────────────────────────────────────────
-// Row-major n x n per block. Column j of L from the lower triangle of A and the
-// finished columns to its left; a pivot that is not > 0 (NaN included) stops the
-// matrix (nx_c_tri.c:15-16).
-template <class T>
-__global__ __launch_bounds__(LA_THREADS) void cholesky_kernel(T *all, int n, int upper, int *status) {
-  using S = Sc<T>;
-  T *A = all + (size_t)blockIdx.x * n * n;
-  __shared__ int failed;
-  if (threadIdx.x == 0) failed = 0;
-  for (int j = 0; j < n; j++) {
-    for (int i = j + threadIdx.x; i < n; i += blockDim.x) {
-      T s = A[(size_t)i * n + j];
-      const T *ri = A + (size_t)i * n, *rj = A + (size_t)j * n;
-      for (int k = 0; k < j; k++) s = s - ri[k] * S::conj(rj[k]);
-      A[(size_t)i * n + j] = s;
-    }
-    __syncthreads();
-    const double d = S::re(A[(size_t)j * n + j]);
-    if (threadIdx.x == 0 && !(d > 0.0)) failed = 1;
-    __syncthreads();
-    if (failed) {
-      if (threadIdx.x == 0) raise(status, LA_NOT_PD);
-      return;
-    }
-    const double l = sqrt(d);
-    for (int i = j + threadIdx.x; i < n; i += blockDim.x)
-      A[(size_t)i * n + j] = i == j ? S::make(l, 0.0) : S::scale(A[(size_t)i * n + j], 1.0 / l);
-    __syncthreads();
-  }
-  // the other triangle: zero for L; for U the conjugate transpose moves there first
-  for (int64_t e = threadIdx.x; e < (int64_t)n * n; e += blockDim.x) {
-    const int i = (int)(e / n), k = (int)(e % n);
-    if (i <= k) continue;
-    if (upper) {
-      A[(size_t)k * n + i] = S::conj(A[e]);
-      A[e] = S::make(0.0, 0.0);
-    } else {
-      A[(size_t)k * n + i] = S::make(0.0, 0.0);
-    }
-  }
-}
-
-// ── triangular solve ────────────────────────────────────────────────────────
-// X (n x nrhs) holds B and is solved in place against op(A), op = conjugate
-// transpose when `transpose`. Forward iff upper == transpose (nx_c_tri.c:103-118).
-template <class T>
-__global__ __launch_bounds__(LA_THREADS) void trsm_kernel(const T *a_all, T *x_all, int n, int nrhs, int upper,
-                                                         int transpose, int unit, int *status) {
-  using S = Sc<T>;
-  const T *A = a_all + (size_t)blockIdx.x * n * n;
-  T *X = x_all + (size_t)blockIdx.x * n * nrhs;
-  const bool forward = (upper != 0) == (transpose != 0);
-  for (int ii = 0; ii < n; ii++) {
-    const int i = forward ? ii : n - 1 - ii;
-    if (!unit) {
-      T diag = A[(size_t)i * n + i];
-      if (transpose) diag = S::conj(diag);
-      if (diag == S::make(0.0, 0.0)) {  // uniform: every lane reads the same element
-        if (threadIdx.x == 0) raise(status, LA_SINGULAR);
-        return;
-      }
-      for (int j = threadIdx.x; j < nrhs; j += blockDim.x) X[(size_t)i * nrhs + j] = X[(size_t)i * nrhs + j] / diag;
-      __syncthreads();
-    }
-    const int rest = n - 1 - ii;  // rows not yet solved
-    for (int64_t e = threadIdx.x; e < (int64_t)rest * nrhs; e += blockDim.x) {
-      const int rr = (int)(e / nrhs), j = (int)(e % nrhs);
-      const int r = forward ? i + 1 + rr : i - 1 - rr;
-      const T m = transpose ? S::conj(A[(size_t)i * n + r]) : A[(size_t)r * n + i];
-      X[(size_t)r * nrhs + j] = X[(size_t)r * nrhs + j] - m * X[(size_t)i * nrhs + j];
-    }
-    __syncthreads();
-  }
-}
+#include "linalg_blocked.hpp"
 
 // ── Householder QR on column-major storage ──────────────────────────────────
 // At[c * m + i] = A[i][c]. On return the upper trapezoid holds R, the reflector
@@ -681,96 +608,7 @@ __global__ void la_fill_int(int *p, int count, int value) {
   if (i < count) p[i] = value;
 }
 
-// ── triangular solve over the whole device ──────────────────────────────────
-// Row i of the solution (one launch), then its elimination from the rows not yet
-// solved (another), for every matrix and right-hand side at once.
-template <class T>
-__global__ __launch_bounds__(LA_THREADS) void trsm_wide_scale(const T *a_all, T *x_all, int n, int nrhs, int i, int transpose,
-                                                             int64_t total, int *status) {
-  using S = Sc<T>;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  const int64_t b = e / nrhs;
-  const int j = (int)(e % nrhs);
-  T diag = a_all[(size_t)b * n * n + (size_t)i * n + i];
-  if (transpose) diag = S::conj(diag);
-  if (diag == S::make(0.0, 0.0)) {
-    if (j == 0) raise(status, LA_SINGULAR);
-    return;
-  }
-  T *x = x_all + (size_t)b * n * nrhs + (size_t)i * nrhs + j;
-  *x = *x / diag;
-}
-
-template <class T>
-__global__ __launch_bounds__(LA_THREADS) void trsm_wide_eliminate(const T *a_all, T *x_all, int n, int nrhs, int i, int rest,
-                                                                 int forward, int transpose, int64_t total) {
-  using S = Sc<T>;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  const int j = (int)(e % nrhs), rr = (int)((e / nrhs) % rest);
-  const int64_t b = e / ((int64_t)nrhs * rest);
-  const int r = forward ? i + 1 + rr : i - 1 - rr;
-  const T *A = a_all + (size_t)b * n * n;
-  T *X = x_all + (size_t)b * n * nrhs;
-  const T m = transpose ? S::conj(A[(size_t)i * n + r]) : A[(size_t)r * n + i];
-  X[(size_t)r * nrhs + j] = X[(size_t)r * nrhs + j] - m * X[(size_t)i * nrhs + j];
-}
-
-// ── cholesky and qr over the whole device ───────────────────────────────────
-// Column j of every matrix in one launch, a wave per (matrix, row >= j): the
-// lanes split the dot product along the finished columns (contiguous in the
-// row-major matrix). Every wave recomputes row j's own dot product for the pivot
-// instead of waiting for it.
-template <class T>
-__global__ __launch_bounds__(LA_THREADS) void cholesky_wide_column(T *all, double *diag_all, int n, int j, int64_t waves_total,
-                                                                  int *status) {
-  using S = Sc<T>;
-  const int lane = threadIdx.x & 63;
-  const int64_t item = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (item >= waves_total) return;
-  const int rows = n - j, i = j + (int)(item % rows);
-  T *A = all + (size_t)(item / rows) * n * n;
-  const T *ri = A + (size_t)i * n, *rj = A + (size_t)j * n;
-  T s = S::make(0.0, 0.0);
-  double dj = 0.0;
-  for (int k = lane; k < j; k += 64) {
-    const T ljk = rj[k];
-    s = s + ri[k] * S::conj(ljk);
-    dj += S::abs2(ljk);
-  }
-  s = wave_sum(s);
-  const double d = S::re(rj[j]) - wave_sum(dj);
-  if (!(d > 0.0)) {
-    if (i == j && lane == 0) raise(status, LA_NOT_PD);
-    return;  // later columns see an unfinished factor; the call fails as a whole
-  }
-  const double l = sqrt(d);
-  if (lane != 0) return;
-  // the pivot is kept aside until the end: the other waves of this launch still read A[j][j]
-  if (i == j) diag_all[(item / rows) * n + j] = l;
-  else A[(size_t)i * n + j] = S::scale(A[(size_t)i * n + j] - s, 1.0 / l);
-}
-
-template <class T>
-__global__ __launch_bounds__(LA_THREADS) void cholesky_wide_finish(T *all, const double *diag_all, int n, int upper,
-                                                                  int64_t total) {
-  using S = Sc<T>;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  const int64_t nn2 = (int64_t)n * n;
-  T *A = all + (e / nn2) * nn2;
-  const int i = (int)((e % nn2) / n), k = (int)(e % n);
-  if (i == k) A[(size_t)i * n + i] = S::make(diag_all[(e / nn2) * n + i], 0.0);
-  if (i <= k) return;
-  if (upper) {
-    A[(size_t)k * n + i] = S::conj(A[(size_t)i * n + k]);
-    A[(size_t)i * n + k] = S::make(0.0, 0.0);
-  } else {
-    A[(size_t)k * n + i] = S::make(0.0, 0.0);
-  }
-}
-
+// ── qr over the whole device ────────────────────────────────────────────────
 // Reflector of column j (one workgroup per matrix), then its application to the
 // trailing columns (a wave per (matrix, column)).
 template <class T>
@@ -1324,38 +1162,125 @@ static int svd_wide(nxh_context *ctx, const char *op, Work &work, int64_t batch,
   return NXH_OK;
 }
 
-template <class T>
-static int trsm_wide(nxh_context *ctx, const char *op, int64_t batch, int n, int nrhs, int upper, int transpose, int unit, const T *A,
-                     T *X) {
-  const int forward = (upper != 0) == (transpose != 0);
+// An operand the blocked kernels read or write in place: float32, float64 or complex128 storage
+// whose batch dims are one stride (anything else goes through a workspace and nxh_cast).
+static bool la_direct(const nxh_tensor *t, LaMat *m) {
+  if (t->dtype != NXH_F32 && t->dtype != NXH_F64 && t->dtype != NXH_C64) return false;
+  const int nd = t->ndim;
+  m->rs = t->strides[nd - 2];
+  m->cs = t->strides[nd - 1];
+  m->bs = 0;
+  bool first = true;
+  int64_t expect = 0;
+  for (int d = nd - 3; d >= 0; d--) {
+    if (t->shape[d] == 1) continue;
+    if (first) m->bs = t->strides[d], first = false;
+    else if (t->strides[d] != expect) return false;
+    expect = t->strides[d] * t->shape[d];
+  }
+  const int size = t->dtype == NXH_F32 ? 4 : t->dtype == NXH_F64 ? 8 : 16;
+  m->p = (char *)t->data + t->offset * size;
+  return true;
+}
+
+// The word of pinned memory the blocked kernels report to; zero between calls.
+static int *la_host_status(nxh_context *ctx) { return ctx->fault_flag_host + 8; }
+
+// Waits for the kernels of this call (the results included) and reads their report.
+static int la_collect_host(nxh_context *ctx, const char *op) {
   std::lock_guard<std::mutex> g(ctx->mu);
-  for (int ii = 0; ii < n; ii++) {
-    const int i = forward ? ii : n - 1 - ii, rest = n - 1 - ii;
-    if (!unit)
-      hipLaunchKernelGGL(trsm_wide_scale<T>, dim3(la_blocks(batch * nrhs)), dim3(LA_THREADS), 0, ctx->stream, A, X, n, nrhs, i,
-                         transpose, batch * nrhs, la_status(ctx));
-    const int64_t items = batch * rest * nrhs;
-    if (items > 0)
-      hipLaunchKernelGGL(trsm_wide_eliminate<T>, dim3(la_blocks(items)), dim3(LA_THREADS), 0, ctx->stream, A, X, n, nrhs, i, rest,
-                         forward, transpose, items);
+  NXH_HIP(op, hipGetLastError());
+  NXH_HIP(op, hipStreamSynchronize(ctx->stream));
+  volatile int *host = la_host_status(ctx);
+  const int code = *host;
+  if (code == LA_OK) return NXH_OK;
+  *host = 0;
+  return nxh_fail(NXH_FAILURE, op, LA_MESSAGES[code <= LA_NO_CONVERGE ? code : LA_NO_CONVERGE]);
+}
+
+constexpr int64_t LA_GRID_BATCH = 65535;  // matrices per launch (the grid's y and z extent)
+
+template <class T, class TS>
+static int run_cholesky(nxh_context *ctx, const char *op, int64_t batch, int n, int upper, LaMat x, LaMat out, T *A, T *L) {
+  constexpr int NB = CHOL_NB<T>;
+  auto kern = cholesky_block_kernel<T, TS>;
+  static std::once_flag once;
+  static hipError_t attr = hipSuccess;
+  std::call_once(once, [&] { attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CHOL_LDS<T>); });
+  NXH_HIP(op, attr);
+  std::lock_guard<std::mutex> g(ctx->mu);
+  for (int64_t b0 = 0; b0 < batch; b0 += LA_GRID_BATCH) {
+    const int64_t nbat = std::min(LA_GRID_BATCH, batch - b0);
+    CholArgs<T> a{};
+    a.x = x;
+    a.out = out;
+    a.x.p = (TS *)x.p + b0 * x.bs;
+    a.out.p = (TS *)out.p + b0 * out.bs;
+    a.A = A ? A + (size_t)b0 * n * n : nullptr;
+    a.L = L + (size_t)b0 * n * n;
+    a.n = n;
+    a.upper = upper;
+    a.status = la_host_status(ctx);
+    const int cols = (n + NB - 1) / NB;
+    for (int s = 0; s < cols; s++) {
+      a.s = s;
+      const int64_t panels = cols - s, tiles = panels + (s > 0 ? panels * (panels - 1) / 2 : 0);
+      if (tiles > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "matrix too large for one launch");
+      hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)nbat), dim3(CHOL_THREADS), CHOL_LDS<T>, ctx->stream, a);
+    }
   }
   NXH_HIP(op, hipGetLastError());
   return NXH_OK;
 }
 
+// Rows of a pass: what the LDS holds of sixteen right-hand sides beside the triangles.
 template <class T>
-static int cholesky_wide(nxh_context *ctx, const char *op, Work &work, int64_t batch, int n, int upper, T *A) {
-  void *diag;
-  if (int rc = work.get((size_t)(batch * n) * sizeof(double), &diag)) return rc;
-  std::lock_guard<std::mutex> g(ctx->mu);
-  for (int j = 0; j < n; j++) {
-    const int64_t waves = batch * (n - j);
-    hipLaunchKernelGGL(cholesky_wide_column<T>, dim3(la_blocks(waves, LA_THREADS / 64)), dim3(LA_THREADS), 0, ctx->stream, A,
-                       (double *)diag, n, j, waves, la_status(ctx));
+constexpr int TRSM_PASS = sizeof(T) == 8 ? 1024 : 512;
+
+// b and x may be one workspace (they are where there are several passes: what is passed on between
+// them is in the compute type).
+template <class T, class TS>
+static int run_trsm(nxh_context *ctx, const char *op, int64_t batch, int n, int nrhs, int flags, LaMat m, LaMat b, LaMat x) {
+  const bool upper = flags & 1, transpose = (flags >> 1) & 1, forward = upper == transpose;
+  auto kern = trsm_block_kernel<T, TS>;
+  static std::once_flag once;
+  static hipError_t attr = hipSuccess;
+  std::call_once(once, [&] { attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, TRSM_PASS<T> * 16 * (int)sizeof(T)); });
+  NXH_HIP(op, attr);
+  // in solution order: row t of the solution is matrix row t, or n - 1 - t backwards
+  int64_t ts = transpose ? m.cs : m.rs, us = transpose ? m.rs : m.cs;
+  TS *mp = (TS *)m.p, *bp = (TS *)b.p, *xp = (TS *)x.p;
+  if (!forward) {
+    mp += (n - 1) * (ts + us);
+    bp += (n - 1) * b.rs;
+    xp += (n - 1) * x.rs;
+    ts = -ts, us = -us, b.rs = -b.rs, x.rs = -x.rs;
   }
-  const int64_t total = batch * n * n;
-  hipLaunchKernelGGL(cholesky_wide_finish<T>, dim3(la_blocks(total)), dim3(LA_THREADS), 0, ctx->stream, A, (const double *)diag, n,
-                     upper, total);
+  std::lock_guard<std::mutex> g(ctx->mu);
+  for (int64_t b0 = 0; b0 < batch; b0 += LA_GRID_BATCH) {
+    const unsigned nbat = (unsigned)std::min(LA_GRID_BATCH, batch - b0), groups = (unsigned)((nrhs + 15) / 16);
+    if (groups > 65535u && n > TRSM_PASS<T>) return nxh_fail(NXH_FAILURE, op, "too many elements for one launch");
+    for (int r0 = 0; r0 < n; r0 += TRSM_PASS<T>) {
+      TrsmArgs<T> a{};
+      a.m = mp + b0 * m.bs + r0 * (ts + us);
+      a.ts = ts;
+      a.us = us;
+      a.mbs = m.bs;
+      a.conj = transpose;
+      a.unit = (flags >> 2) & 1;
+      a.b = LaMat{bp + b0 * b.bs + r0 * b.rs, b.rs, b.cs, b.bs};
+      a.x = LaMat{xp + b0 * x.bs + r0 * x.rs, x.rs, x.cs, x.bs};
+      a.rows = std::min(n - r0, TRSM_PASS<T>);
+      a.nrhs = nrhs;
+      a.status = la_host_status(ctx);
+      const int nb = (a.rows + 15) / 16;
+      hipLaunchKernelGGL(kern, dim3(groups, nbat), dim3(64 * TRSM_WAVES), (size_t)nb * 256 * sizeof(T), ctx->stream, a);
+      const int rest = n - r0 - a.rows;
+      if (rest > 0)
+        hipLaunchKernelGGL((trsm_rest_kernel<T, TS>), dim3((unsigned)((rest + 63) / 64), groups, nbat), dim3(256), 0, ctx->stream, a,
+                           LaMat{(TS *)a.x.p + a.rows * a.x.rs, a.x.rs, a.x.cs, a.x.bs}, rest);
+    }
+  }
   NXH_HIP(op, hipGetLastError());
   return NXH_OK;
 }
@@ -1454,22 +1379,28 @@ NXH_EXPORT int nxh_cholesky(nxh_context *ctx, const nxh_tensor *out, const nxh_t
   std::lock_guard<std::mutex> whole_call(ctx->call_mu);
   if ((rc = la_begin(ctx, op))) return rc;
   Work work(ctx);
-  void *A;
-  if ((rc = work.get((size_t)(p.batch * n * n) * p.esize, &A))) return rc;
-  nxh_tensor wa = workspace_tensor(x, A, p.wdt, n, n, false);
-  if ((rc = nxh_cast(ctx, &wa, x))) return rc;
   PathAtExit path{n >= LA_WIDE_FROM ? "cholesky_columns_wide" : "cholesky_columns"};
-  if (n >= LA_WIDE_FROM) {
-    rc = p.cx ? cholesky_wide<c64>(ctx, op, work, p.batch, (int)n, upper, (c64 *)A)
-              : cholesky_wide<double>(ctx, op, work, p.batch, (int)n, upper, (double *)A);
-    if (rc) return rc;
-  } else if (p.cx) {
-    LA_LAUNCH(ctx, cholesky_kernel<c64>, p.batch, 0, (c64 *)A, (int)n, upper, la_status(ctx));
-  } else {
-    LA_LAUNCH(ctx, cholesky_kernel<double>, p.batch, 0, (double *)A, (int)n, upper, la_status(ctx));
+  const size_t mat = (size_t)(p.batch * n * n) * p.esize;
+  void *A = nullptr, *L, *io = nullptr;
+  const int nb = p.cx ? CHOL_NB<c64> : CHOL_NB<double>;
+  if ((rc = work.get(mat, &L)) || (n > 2 * nb && (rc = work.get(mat, &A)))) return rc;
+  LaMat mx{}, mo{};
+  nxh_tensor wio{};
+  const bool direct = x->data != out->data && la_direct(x, &mx) && la_direct(out, &mo);
+  if (!direct) {  // both through one workspace of the compute type
+    if ((rc = work.get(2 * mat, &io))) return rc;
+    wio = workspace_tensor(x, io, p.wdt, n, n, false);
+    if ((rc = nxh_cast(ctx, &wio, x))) return rc;
+    mx = LaMat{io, n, 1, n * n};
+    wio.data = (char *)io + mat;
+    mo = LaMat{wio.data, n, 1, n * n};
   }
-  if ((rc = la_collect(ctx, op))) return rc;
-  return nxh_cast(ctx, out, &wa);
+  if (p.cx) rc = run_cholesky<c64, c64>(ctx, op, p.batch, (int)n, upper, mx, mo, (c64 *)A, (c64 *)L);
+  else if (direct && x->dtype == NXH_F32) rc = run_cholesky<double, float>(ctx, op, p.batch, (int)n, upper, mx, mo, (double *)A, (double *)L);
+  else rc = run_cholesky<double, double>(ctx, op, p.batch, (int)n, upper, mx, mo, (double *)A, (double *)L);
+  if (rc) return rc;
+  if (!direct && (rc = nxh_cast(ctx, out, &wio))) return rc;
+  return la_collect_host(ctx, op);
 }
 
 // nx_c_tri.c:459-562, 580-600. `b` and `out` are matrices of right-hand sides
@@ -1494,23 +1425,26 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
   std::lock_guard<std::mutex> whole_call(ctx->call_mu);
   if ((rc = la_begin(ctx, op))) return rc;
   Work work(ctx);
-  void *A, *X;
-  if ((rc = work.get((size_t)(p.batch * n * n) * p.esize, &A))) return rc;
-  if ((rc = work.get((size_t)(p.batch * n * nrhs) * p.esize, &X))) return rc;
-  nxh_tensor wa = workspace_tensor(a, A, p.wdt, n, n, false);
-  nxh_tensor wx = workspace_tensor(b, X, p.wdt, n, nrhs, false);
-  if ((rc = nxh_cast(ctx, &wa, a)) || (rc = nxh_cast(ctx, &wx, b))) return rc;
   PathAtExit path{n >= LA_WIDE_FROM ? "triangular_substitution_wide" : "triangular_substitution"};
-  const int up = flags & 1, tr = (flags >> 1) & 1, unit = (flags >> 2) & 1;
-  if (n >= LA_WIDE_FROM) {
-    if (p.batch * n * nrhs / LA_THREADS > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "too many elements for one launch");
-    rc = p.cx ? trsm_wide<c64>(ctx, op, p.batch, (int)n, (int)nrhs, up, tr, unit, (const c64 *)A, (c64 *)X)
-              : trsm_wide<double>(ctx, op, p.batch, (int)n, (int)nrhs, up, tr, unit, (const double *)A, (double *)X);
-    if (rc) return rc;
-  } else if (p.cx) LA_LAUNCH(ctx, trsm_kernel<c64>, p.batch, 0, (const c64 *)A, (c64 *)X, (int)n, (int)nrhs, up, tr, unit, la_status(ctx));
-  else LA_LAUNCH(ctx, trsm_kernel<double>, p.batch, 0, (const double *)A, (double *)X, (int)n, (int)nrhs, up, tr, unit, la_status(ctx));
-  if ((rc = la_collect(ctx, op))) return rc;
-  return nxh_cast(ctx, out, &wx);
+  LaMat ma{}, mb{}, mx{};
+  nxh_tensor wx{};
+  const int pass = p.cx ? TRSM_PASS<c64> : TRSM_PASS<double>;
+  const bool direct = n <= pass && out->data != a->data && out->data != b->data && la_direct(a, &ma) && la_direct(b, &mb) && la_direct(out, &mx);
+  if (!direct) {
+    void *A, *X;
+    if ((rc = work.get((size_t)(p.batch * n * n) * p.esize, &A)) || (rc = work.get((size_t)(p.batch * n * nrhs) * p.esize, &X))) return rc;
+    nxh_tensor wa = workspace_tensor(a, A, p.wdt, n, n, false);
+    wx = workspace_tensor(b, X, p.wdt, n, nrhs, false);
+    if ((rc = nxh_cast(ctx, &wa, a)) || (rc = nxh_cast(ctx, &wx, b))) return rc;
+    ma = LaMat{A, n, 1, n * n};
+    mb = mx = LaMat{X, nrhs, 1, n * nrhs};
+  }
+  if (p.cx) rc = run_trsm<c64, c64>(ctx, op, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
+  else if (direct && a->dtype == NXH_F32) rc = run_trsm<double, float>(ctx, op, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
+  else rc = run_trsm<double, double>(ctx, op, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
+  if (rc) return rc;
+  if (!direct && (rc = nxh_cast(ctx, out, &wx))) return rc;
+  return la_collect_host(ctx, op);
 }
 
 // nx_c_qr.c; nx_backend.ml:613-626. q is [..., m, k] (reduced) or [..., m, m]; r is

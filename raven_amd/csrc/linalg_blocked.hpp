@@ -1,0 +1,752 @@
+// linalg_blocked.hpp — cholesky and triangular_solve by blocks (included by linalg.hip,
+// inside its namespace).
+//
+// Both are chains: column j of a factor, row i of a solution, waits for the one before
+// it. A launch per column pays a launch (2 - 4 us) per link of the chain; here a link is
+// some 200 cycles inside a workgroup, and everything that is no link (the updates of what
+// comes later) is a product of 16 x 16 tiles on the f64 matrix instruction.
+#pragma once
+
+typedef __attribute__((ext_vector_type(4))) double la_f64x4;
+
+// A batch of matrices in the storage type TS: element (r, c) of matrix b is p[b bs + r rs + c cs].
+struct LaMat {
+  void *p;
+  int64_t rs, cs, bs;
+};
+
+// A numeric failure goes straight to a word of pinned host memory, which the call reads
+// after its stream wait: no copy of a device word is queued behind the kernels. Every
+// failure of one call has the same code, so a plain store is enough.
+__device__ __forceinline__ void raise_host(int *host_status, int code) {
+  __hip_atomic_store(host_status, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane) {  // `lane` uniform
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane), hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ c64 lane_value(c64 v, int lane) { return {lane_value(v.re, lane), lane_value(v.im, lane)}; }
+
+__device__ __forceinline__ void to_storage(double v, float *p) { *p = (float)v; }
+__device__ __forceinline__ void to_storage(double v, double *p) { *p = v; }
+__device__ __forceinline__ void to_storage(c64 v, c64 *p) { *p = v; }
+
+// sqrt(d) and 1 / sqrt(d) of a positive d, each to the last bit or next to it: one hardware
+// estimate and Newton steps on d scaled into [1/4, 1). The chain of the factorisation runs
+// through this once per column; the library's square root and division are four times as long.
+__device__ __forceinline__ void root_and_inverse(double d, double *root, double *inv) {
+  const int e = (__builtin_amdgcn_frexp_exp(d) + 1) >> 1;
+  const double ds = ldexp(d, -2 * e);
+  double r = __builtin_amdgcn_rsq(ds);
+  const double err = fma(-(ds * r), r, 1.0);
+  r = fma(r * err, fma(0.375, err, 0.5), r);
+  double l = ds * r;
+  l = fma(fma(-l, l, ds), 0.5 * r, l);
+  r = fma(fma(-l, r, 1.0), r, r);
+  *root = d < __builtin_inf() ? ldexp(l, e) : d;
+  *inv = d < __builtin_inf() ? ldexp(r, -e) : 0.0;
+}
+
+// One 16 x 16 tile of accumulators: register v of lane l is row 4 v + l / 16, column l % 16
+// (what v_mfma_f64_16x16x4 produces; the complex form uses the same places).
+template <class T>
+struct LaTile {
+  T v[4];
+};
+
+// acc -= A B^H over K terms: A[row * lda + k], B[col * ldb + k] with the tile's first row and
+// column in the pointers.
+template <int K>
+__device__ __forceinline__ void tile_sub(LaTile<double> &acc, const double *A, int64_t lda, const double *B, int64_t ldb) {
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  la_f64x4 c = {acc.v[0], acc.v[1], acc.v[2], acc.v[3]};
+  const double *pa = A + r * lda + q, *pb = B + r * ldb + q;
+#pragma unroll
+  for (int k = 0; k < K; k += 4) c = __builtin_amdgcn_mfma_f64_16x16x4f64(-pa[k], pb[k], c, 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < 4; i++) acc.v[i] = c[i];
+}
+template <int K>
+__device__ __forceinline__ void tile_sub(LaTile<c64> &acc, const c64 *A, int64_t lda, const c64 *B, int64_t ldb) {
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+#pragma unroll 4
+  for (int k = 0; k < K; k++) {
+    const c64 b = Sc<c64>::conj(B[r * ldb + k]);
+#pragma unroll
+    for (int v = 0; v < 4; v++) acc.v[v] = Sc<c64>::sub_mul(acc.v[v], A[(4 * v + q) * lda + k], b);
+  }
+}
+
+// 1 / d of an ordinary double, to the last bit or next to it.
+__device__ __forceinline__ double inverse_of(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma(fma(-d, r, 1.0), r, r);
+  return fma(fma(-d, r, 1.0), r, r);
+}
+
+// Substitution through a 16 x 16 triangle, four rows at a time on the matrix instruction, for
+// sixteen right-hand sides: register v of lane (q, c) = 16 q + c holds row 4 v + q of side c, which is
+// both where the instruction leaves a result and, for four rows, where it takes its second operand
+// from: nothing moves between lanes. diag_inv[b] is the inverse of the b-th 4 x 4 triangle on
+// the diagonal as a first operand (lane (q, r): element (r - 4 b, q), 0 in other rows), tri[b] columns
+// 4 b .. 4 b + 3 (lane (q, r): element (r, 4 b + q), 0 above the diagonal). The product with the
+// inverse is followed by one step on its remainder, which the update leaves in the same register,
+// so the result is that of a substitution. 16 instructions of 64 cycles; row by row, with a
+// right-hand side a lane, the chain through LDS took 4700 cycles.
+__device__ __forceinline__ void solve16(LaTile<double> &acc, const double (&diag_inv)[4], const double (&tri)[4]) {
+  la_f64x4 c = {acc.v[0], acc.v[1], acc.v[2], acc.v[3]};
+  const la_f64x4 zero = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    const double x = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], c[b], zero, 0, 0, 0)[b];
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64(-tri[b], x, c, 0, 0, 0);
+    const double dx = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], c[b], zero, 0, 0, 0)[b];
+    acc.v[b] = x + dx;
+    if (b < 3) c = __builtin_amdgcn_mfma_f64_16x16x4f64(-tri[b], dx, c, 0, 0, 0);
+  }
+}
+
+// Cholesky of a 16 x 16 tile in that layout (the tile is Hermitian: rows and columns may change
+// places), four columns at a time: every lane factors the 4 x 4 block on the diagonal as L D L^T (the
+// chain is four reciprocals; the roots follow side by side), the matrix instruction does the rest.
+// Leaves the operands of solve16 in diag_inv and tri; tri is the factor itself. `blk`: 64 doubles of LDS.
+__device__ __forceinline__ bool factor16(LaTile<double> acc, double *blk, double (&diag_inv)[4], double (&tri)[4]) {
+  const int lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
+  la_f64x4 t = {acc.v[0], acc.v[1], acc.v[2], acc.v[3]};
+  const la_f64x4 zero = {0.0, 0.0, 0.0, 0.0};
+  bool positive = true;
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    blk[lane] = t[b];
+    __builtin_amdgcn_wave_barrier();
+    double a[4][4];  // a[j][i]: element (4 b + i, 4 b + j)
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int i = j; i < 4; i++) a[j][i] = blk[16 * j + 4 * b + i];
+    __builtin_amdgcn_wave_barrier();
+    double u[4][4], root[4];  // u[j][i]: the unit triangle; root[j]: 1 / sqrt of the pivot
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const double r = inverse_of(a[j][j]);
+#pragma unroll
+      for (int i = j + 1; i < 4; i++) u[j][i] = a[j][i] * r;
+#pragma unroll
+      for (int k = j + 1; k < 4; k++)
+#pragma unroll
+        for (int i = k; i < 4; i++) a[k][i] = fma(-u[j][i], a[j][k], a[k][i]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      double l;
+      positive = positive && a[j][j] > 0.0;
+      root_and_inverse(a[j][j], &l, &root[j]);
+    }
+    // rows of the inverse of the unit triangle, each times its root
+    const double m10 = -u[0][1], m21 = -u[1][2], m32 = -u[2][3];
+    const double m20 = fma(-m10, u[1][2], -u[0][2]), m31 = fma(-m21, u[2][3], -u[1][3]);
+    const double m30 = fma(-m20, u[2][3], fma(-m10, u[1][3], -u[0][3]));
+    const int i = c - 4 * b;
+    double m = q == 0 ? m30 : q == 1 ? m31 : q == 2 ? m32 : 1.0;
+    m = i == 2 ? (q == 0 ? m20 : q == 1 ? m21 : 1.0) : m;
+    m = i == 1 ? (q == 0 ? m10 : 1.0) : m;
+    m = i == 0 ? 1.0 : m;
+    m *= i == 0 ? root[0] : i == 1 ? root[1] : i == 2 ? root[2] : root[3];
+    diag_inv[b] = i >= q && i < 4 ? m : 0.0;
+    double x = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], t[b], zero, 0, 0, 0)[b];
+    x = c >= 4 * b + q ? x : 0.0;
+    t = __builtin_amdgcn_mfma_f64_16x16x4f64(-x, x, t, 0, 0, 0);
+    double dx = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], t[b], zero, 0, 0, 0)[b];
+    // (inside the 4 x 4 block the remainder is that of a product of two unknowns, a rounding of it: left)
+    dx = c >= 4 * b + 4 ? dx : 0.0;
+    if (b < 3) {
+      t = __builtin_amdgcn_mfma_f64_16x16x4f64(-dx, x, t, 0, 0, 0);
+      t = __builtin_amdgcn_mfma_f64_16x16x4f64(-(x + dx), dx, t, 0, 0, 0);
+    }
+    tri[b] = x + dx;
+  }
+  return positive;
+}
+
+// ── cholesky ────────────────────────────────────────────────────────────────
+// NB x NB tiles, one launch per block column s, a workgroup per tile (i, j) with i >= j >= s.
+// Tile (i, j) first takes what block column s - 1 takes from it. Column s then is
+// finished: every workgroup of that column keeps the diagonal tile too, factors it (the same
+// instructions on the same values everywhere), and solves its own tile against it, sixteen
+// columns behind. Factoring the diagonal again in each workgroup costs nothing (it would
+// be waited for) and saves a launch per block column. The factor goes to L, the updated rest to
+// A: nothing that a workgroup of the same launch may still read is overwritten.
+//
+// The chain of a launch is the diagonal tile, sixteen columns at a time: factored by wave 0
+// (factor16), then a wave per sixteen rows below solves against them (solve16), then wave 0
+// updates and factors the next sixteen while the others update the rest and this workgroup's own
+// tile follows, a wave per sixteen rows, one block of columns behind. Complex matrices, with no matrix
+// instruction for them, are factored column by column, a row a lane.
+constexpr int CHOL_THREADS = 512, CHOL_WAVES = CHOL_THREADS / 64;
+template <class T>
+constexpr int CHOL_NB = sizeof(T) == 8 ? 64 : 32;
+constexpr int CHOL_COLUMN = 80;                 // complex: 64 values of one column, and room for reads past them
+constexpr int CHOL_OPERANDS = 64 + 2 * 4 * 256;  // double: factor16's scratch, the operands of solve16 for four blocks of columns
+// four tiles of pitch NB + 2 (66 doubles: sixteen rows on different banks), then those
+template <class T>
+constexpr size_t CHOL_LDS = 4 * CHOL_NB<T> * (CHOL_NB<T> + 2) * sizeof(T) +
+                            (sizeof(T) == 8 ? CHOL_OPERANDS * sizeof(double) : CHOL_COLUMN * sizeof(T) + CHOL_NB<T> * sizeof(double));
+
+template <class T>
+struct CholArgs {
+  LaMat x, out;  // storage types: read by the first two launches, written by all
+  T *A, *L;      // n x n per matrix, row-major
+  int n, s, upper;
+  int *status;
+};
+
+template <class T, class TS>
+__global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T> a) {
+  using S = Sc<T>;
+  constexpr int NB = CHOL_NB<T>, LD = NB + 2, TILES = NB / 16;
+  extern __shared__ double lds_raw[];
+  T *D = (T *)lds_raw, *own = D + NB * LD;  // the diagonal tile, this workgroup's
+  T *ls = own + NB * LD, *li = ls + NB * LD;  // block column s - 1 in the rows of tile (s, .) and of tile (i, .)
+  T *column = li + NB * LD;
+  double *inv = (double *)(column + CHOL_COLUMN);
+  double *blk = (double *)(li + NB * LD), *op_inv = blk + 64, *op_tri = op_inv + 4 * 256;
+  const int n = a.n, s = a.s, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+  const int panels = (n + NB - 1) / NB - s;  // block rows from s down
+  int i, j;
+  if ((int)blockIdx.x < panels) {
+    i = s + blockIdx.x, j = s;
+  } else {  // the others, row by row of the triangle below
+    int t = blockIdx.x - panels, row = 1;
+    while (t >= row) t -= row, row++;
+    i = s + row, j = s + 1 + t;
+  }
+  const TS *x = (const TS *)a.x.p + blockIdx.y * a.x.bs;
+  T *A = a.A + (size_t)blockIdx.y * n * n, *L = a.L + (size_t)blockIdx.y * n * n;
+  // Element (r, c) as the launches before this one left it (lower triangle). Rows and columns
+  // past n read the last one: what comes of them is not kept.
+  auto source = [&](int r, int c) {
+    r = min(r, n - 1), c = min(c, n - 1);
+    return s <= 1 ? T(x[r * a.x.rs + c * a.x.cs]) : A[(size_t)r * n + c];
+  };
+  // What a wave does in 16 x 16 sub-tiles before anything waits: a tile that is not finished in this launch,
+  // or the lower half of the diagonal tile (the own tile of such a workgroup follows in the shadow of the
+  // factorisation; complex: here).
+  const bool panel = j == s, has_own = i > s;
+  const int left = min(n - s * NB, NB), blocks = (left + 15) / 16;
+  constexpr bool OWN_LATER = sizeof(T) == 8;
+  constexpr int LOWER = TILES * (TILES + 1) / 2, ALL = TILES * TILES;
+  auto job = [&](int t, int *diag, int *tr, int *tc) {  // job `t`, and whether there is anything to do
+    *diag = panel && t < LOWER;
+    if (*diag) {
+      *tr = 0;
+      for (int first = 0; first + *tr + 1 <= t; first += ++*tr) *tc = 0;
+      *tc = t - *tr * (*tr + 1) / 2;
+      return *tr < blocks;
+    }
+    t -= panel ? LOWER : 0;
+    *tr = t / TILES, *tc = t % TILES;
+    return t < ALL && (!panel || (has_own && !OWN_LATER)) && i * NB + *tr * 16 < n && j * NB + *tc * 16 < n && (i != j || *tc <= *tr);
+  };
+  constexpr int MOST = OWN_LATER ? ALL : ALL + LOWER, JOBS = (MOST + CHOL_WAVES - 1) / CHOL_WAVES;
+  LaTile<T> acc[JOBS];
+#pragma unroll
+  for (int e = 0; e < JOBS; e++) {  // every load is on its way before the first is waited for
+    int diag, tr, tc;
+    if (!job(e * CHOL_WAVES + wave, &diag, &tr, &tc)) continue;
+#pragma unroll
+    for (int v = 0; v < 4; v++) acc[e].v[v] = source((diag ? s : i) * NB + tr * 16 + 4 * v + q, j * NB + tc * 16 + r16);
+  }
+  constexpr int PER = NB * NB / CHOL_THREADS;
+  const int col_of = threadIdx.x % NB, row_of = threadIdx.x / NB;
+  T mine[PER];
+  if (OWN_LATER && panel && has_own) {
+#pragma unroll
+    for (int e = 0; e < PER; e++) mine[e] = source(i * NB + row_of + e * (CHOL_THREADS / NB), s * NB + col_of);
+  }
+  if (s > 0) {
+    T vj[PER], vi[PER];
+    const int c = col_of, r0 = row_of;
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+      const int r = r0 + e * (CHOL_THREADS / NB);
+      vj[e] = L[(size_t)min(j * NB + r, n - 1) * n + (s - 1) * NB + c];
+      vi[e] = L[(size_t)min(i * NB + r, n - 1) * n + (s - 1) * NB + c];
+    }
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+      const int r = r0 + e * (CHOL_THREADS / NB);
+      ls[r * LD + c] = vj[e];
+      li[r * LD + c] = vi[e];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int e = 0; e < JOBS; e++) {
+    int diag, tr, tc;
+    if (!job(e * CHOL_WAVES + wave, &diag, &tr, &tc)) continue;
+    if (s > 0) tile_sub<NB>(acc[e], (diag ? ls : li) + tr * 16 * LD, LD, ls + tc * 16 * LD, LD);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int r = tr * 16 + 4 * v + q, cc = tc * 16 + r16;
+      if (!panel) {
+        if (i * NB + r < n && j * NB + cc < n) A[(size_t)(i * NB + r) * n + j * NB + cc] = acc[e].v[v];
+      } else if (diag) {  // past n the diagonal tile is the identity
+        D[r * LD + cc] = r < left && cc < left ? acc[e].v[v] : S::make(r == cc ? 1.0 : 0.0, 0.0);
+      } else {
+        own[r * LD + cc] = acc[e].v[v];
+      }
+    }
+  }
+  if (OWN_LATER && panel && has_own) {
+#pragma unroll
+    for (int e = 0; e < PER; e++) own[(row_of + e * (CHOL_THREADS / NB)) * LD + col_of] = mine[e];
+  }
+  if (!panel) return;
+  __syncthreads();
+  bool bad = false;
+  if constexpr (sizeof(T) == 8) {
+    // rows (sixteen, in LDS) against columns 16 jb .. of the diagonal tile; `before`: they still lack the
+    // updates by the columns before those, by block column s - 1 (rows of li at `before`) and in this one
+    auto solve_rows = [&](double *rows, int jb, const double *before) {
+      LaTile<double> t;
+#pragma unroll
+      for (int v = 0; v < 4; v++) t.v[v] = rows[r16 * LD + jb * 16 + 4 * v + q];
+      if (before) {
+        if (s > 0) tile_sub<NB>(t, ls + jb * 16 * LD, LD, before, LD);
+#pragma unroll 1
+        for (int k = 0; k < jb * 16; k += 16) tile_sub<16>(t, D + jb * 16 * LD + k, LD, rows + k, LD);
+      }
+      double di[4], tr[4];
+#pragma unroll
+      for (int v = 0; v < 4; v++) di[v] = op_inv[(jb * 4 + v) * 64 + lane], tr[v] = op_tri[(jb * 4 + v) * 64 + lane];
+      solve16(t, di, tr);
+#pragma unroll
+      for (int v = 0; v < 4; v++) rows[r16 * LD + jb * 16 + 4 * v + q] = t.v[v];
+    };
+    auto solve_own = [&](int jb) {
+      const int tr = wave == 1 ? 3 : wave - 5;  // (not wave 4: it shares a SIMD, and its matrix unit, with wave 0)
+      if (has_own && tr >= 0 && i * NB + tr * 16 < n) solve_rows(own + tr * 16 * LD, jb, li + tr * 16 * LD);
+    };
+#pragma unroll 1
+    for (int jb = 0; jb < blocks; jb++) {
+      if (wave == 0) {
+        double *tile = D + jb * 16 * (LD + 1);
+        LaTile<double> t;
+#pragma unroll
+        for (int v = 0; v < 4; v++) t.v[v] = tile[r16 * LD + 4 * v + q];
+        if (jb > 0) tile_sub<16>(t, tile - 16, LD, tile - 16, LD);
+        // (the lower triangle is what is kept up to date)
+#pragma unroll
+        for (int v = 0; v < 4; v++) tile[r16 * LD + 4 * v + q] = t.v[v];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int v = 0; v < 4; v++) t.v[v] = tile[max(r16, 4 * v + q) * LD + min(r16, 4 * v + q)];
+        double di[4], tr[4];
+        bad = !factor16(t, blk, di, tr) || bad;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          op_inv[(jb * 4 + v) * 64 + lane] = di[v];
+          op_tri[(jb * 4 + v) * 64 + lane] = tr[v];
+          tile[r16 * LD + 4 * v + q] = tr[v];
+        }
+      } else if (jb > 0 && (wave == 2 || wave == 3)) {
+        for (int t = wave - 2; t < TILES * TILES; t += 2) {  // what block jb - 1 takes from the rest of the tile
+          const int tr = t / TILES, tc = t % TILES;
+          if (tc < jb || tc > tr || tr >= blocks || (tc == jb && tr == jb)) continue;
+          LaTile<double> d;
+#pragma unroll
+          for (int v = 0; v < 4; v++) d.v[v] = D[(tr * 16 + 4 * v + q) * LD + tc * 16 + r16];
+          tile_sub<16>(d, D + tr * 16 * LD + (jb - 1) * 16, LD, D + tc * 16 * LD + (jb - 1) * 16, LD);
+#pragma unroll
+          for (int v = 0; v < 4; v++) D[(tr * 16 + 4 * v + q) * LD + tc * 16 + r16] = d.v[v];
+        }
+      } else if (jb > 0) {
+        solve_own(jb - 1);
+      }
+      __syncthreads();
+      if (wave > jb && wave < blocks) solve_rows(D + wave * 16 * LD, jb, nullptr);
+      __syncthreads();
+    }
+    solve_own(blocks - 1);
+  } else {
+    // this workgroup's tile against the finished columns 16 jb .. of the diagonal one: a wave per
+    // sixteen rows (waves 4 and up, beside wave 0's next columns)
+    auto solve_own = [&](int jb) {
+      const int tr = wave - 4;
+      if (!has_own || tr < 0 || tr >= TILES || i * NB + tr * 16 >= n) return;
+      T *rows = own + tr * 16 * LD;
+      if (jb > 0) {
+        LaTile<T> t;
+#pragma unroll
+        for (int v = 0; v < 4; v++) t.v[v] = rows[(4 * v + q) * LD + jb * 16 + r16];
+#pragma unroll 1
+        for (int k = 0; k < jb * 16; k += 16) tile_sub<16>(t, rows + k, LD, D + jb * 16 * LD + k, LD);
+#pragma unroll
+        for (int v = 0; v < 4; v++) rows[(4 * v + q) * LD + jb * 16 + r16] = t.v[v];
+        __builtin_amdgcn_wave_barrier();
+      }
+      T xr[16];
+#pragma unroll
+      for (int c = 0; c < 16; c++) xr[c] = rows[r16 * LD + jb * 16 + c];
+      __builtin_amdgcn_wave_barrier();
+      const T *col = D + jb * 16 * (LD + 1);  // (c, c) of the diagonal block; rows past it are read, their results dropped
+#pragma unroll 1
+      for (int c = 0; c < 16; c++, col += LD + 1) {
+        const T v = S::scale(xr[0], inv[jb * 16 + c]);
+        if (q == 0) rows[r16 * LD + jb * 16 + c] = v;
+#pragma unroll
+        for (int k = 1; k < 16; k++) xr[k - 1] = S::sub_mul(xr[k], v, S::conj(col[k * LD]));
+      }
+    };
+#pragma unroll 1
+    for (int jb = 0; jb < blocks; jb++) {
+      if (wave == 0) {
+        const int c0 = jb * 16, row = min(lane, NB - 1);
+        // `head`: this lane's element of the column at hand, up to date; p: of the columns after
+        // it, which still lack the update by `prev`, the column before it. That column's values come
+        // back from LDS while the square root is under way; only the next column's head waits for a
+        // value of this one, and takes it from its lane (a lane's value costs some 20 cycles a register)
+        T p[16], prev = S::make(0.0, 0.0);
+#pragma unroll
+        for (int c = 0; c < 16; c++) p[c] = D[row * LD + c0 + c];
+        T head = p[0];
+        column[lane] = prev;
+#pragma unroll 1
+        for (int c = c0; c < c0 + 16; c++) {
+          T before[16];
+#pragma unroll
+          for (int k = 1; k < 16; k++) before[k] = column[c + k];
+          const double d = S::re(lane_value(head, c));
+          bad = bad || !(d > 0.0);
+          double l, li1;
+          root_and_inverse(d, &l, &li1);
+#pragma unroll
+          for (int k = 1; k < 16; k++) p[k - 1] = S::sub_mul(p[k], prev, S::conj(before[k]));
+          const T col = lane == c ? S::make(l, 0.0) : S::scale(head, li1);
+          column[lane] = col;
+          if (lane == 0) inv[c] = li1;
+          if (lane < NB && lane >= c0) D[lane * LD + c] = lane < c ? S::make(0.0, 0.0) : col;
+          head = S::sub_mul(p[0], col, S::conj(lane_value(col, (c + 1) & 63)));
+          prev = col;
+        }
+      } else if (jb > 0) {
+        solve_own(jb - 1);
+      }
+      __syncthreads();
+      // what the new columns take from the rest of the diagonal tile
+      for (int t = wave; t < TILES * TILES; t += CHOL_WAVES) {
+        const int tr = t / TILES, tc = t % TILES;
+        if (tc <= jb || tc > tr || tr >= blocks) continue;
+        LaTile<T> d;
+#pragma unroll
+        for (int v = 0; v < 4; v++) d.v[v] = D[(tr * 16 + 4 * v + q) * LD + tc * 16 + r16];
+        tile_sub<16>(d, D + tr * 16 * LD + jb * 16, LD, D + tc * 16 * LD + jb * 16, LD);
+#pragma unroll
+        for (int v = 0; v < 4; v++) D[(tr * 16 + 4 * v + q) * LD + tc * 16 + r16] = d.v[v];
+      }
+      __syncthreads();
+    }
+    solve_own(blocks - 1);
+  }
+  if (bad && wave == 0 && lane == 0) raise_host(a.status, LA_NOT_PD);
+  __syncthreads();
+  // the factor in double for the launches to come, and the result with its zeros. U = L^H.
+  TS *out = (TS *)a.out.p + blockIdx.y * a.out.bs;
+  const T *tile = has_own ? own : D;
+  const int rows = min(n - i * NB, NB);
+  for (int e = threadIdx.x; e < NB * NB; e += CHOL_THREADS) {
+    const int r = e / NB, c = e % NB;
+    if (r >= rows || c >= left) continue;
+    const T v = has_own || c <= r ? tile[r * LD + c] : S::make(0.0, 0.0);
+    L[(size_t)(i * NB + r) * n + s * NB + c] = v;
+    TS *lower = out + (int64_t)(i * NB + r) * a.out.rs + (int64_t)(s * NB + c) * a.out.cs;
+    if (!a.upper) to_storage(v, lower);
+    else if (has_own) to_storage(S::make(0.0, 0.0), lower);
+  }
+  // the tile mirrored across the diagonal, its lanes along that tile's rows
+  if (has_own || a.upper)
+    for (int e = threadIdx.x; e < NB * NB; e += CHOL_THREADS) {
+      const int r = e / NB, c = e % NB;  // of the mirrored tile
+      if (r >= left || c >= rows) continue;
+      const T v = !a.upper ? S::make(0.0, 0.0) : S::conj(has_own || r <= c ? tile[c * LD + r] : S::make(0.0, 0.0));
+      to_storage(v, out + (int64_t)(s * NB + r) * a.out.rs + (int64_t)(i * NB + c) * a.out.cs);
+    }
+}
+
+// ── triangular solve ────────────────────────────────────────────────────────
+// M X = B with M lower triangular after reversing the order where the substitution runs
+// backwards: coefficient (t, u), t > u, is m[t ts + u us] (conjugated for a conjugate
+// transpose). A workgroup solves sixteen right-hand sides, which stay in LDS, sixteen rows a
+// step: wave 0 brings the next sixteen rows up to date and substitutes through their
+// triangle (solve16), while other waves take the step before from the rows further down (a
+// wave per 16 x 16 tile) and one inverts the 4 x 4 triangles of the next step. What is read
+// of the matrix is requested a step or two ahead: it depends on nothing. One barrier a step, no launch.
+// Where an inverse is no ordinary number, and for complex matrices, the substitution goes row by
+// row, a right-hand side a lane.
+// Wave 0 is the chain, wave 4 (of its SIMD) reads and inverts triangles, which takes no matrix
+// instructions from it, the other six bring up to TRSM_TILES tiles each up to date per step: 64 in a pass.
+constexpr int TRSM_WAVES = 8, TRSM_LOADER = 4, TRSM_UPDATERS = 6, TRSM_TILES = 11;
+
+template <class T>
+struct TrsmArgs {
+  const void *m;        // coefficient (0, 0) of this pass, storage type TS
+  int64_t ts, us, mbs;  // strides along t, along u, and from matrix to matrix
+  int conj, unit;
+  LaMat b, x;           // rows from row 0 of the solution order on; b is read, x written (TS)
+  int rows, nrhs;
+  int *status;
+};
+
+template <class T, class TS>
+__device__ __forceinline__ T trsm_coefficient(const TrsmArgs<T> &a, const TS *m, int t, int u) {
+  const T v = T(m[t * a.ts + u * a.us]);
+  return a.conj ? Sc<T>::conj(v) : v;
+}
+
+template <class T, class TS>
+__global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T> a) {
+  using S = Sc<T>;
+  extern __shared__ double lds_raw[];
+  T *X = (T *)lds_raw;  // rows rounded up to 16, times 16
+  // by columns, each from its diagonal on: element r < 16 of column t is coefficient (t + r, t), element
+  // 16 the inverse of the diagonal (reads past a column's end meet the next one: their results are dropped)
+  constexpr int TRI_LD = 18;
+  __shared__ T tri[2][17][TRI_LD];
+  __shared__ double diag_inv[2][4][64];  // operands of solve16, zero outside the 4 x 4 triangles
+  __shared__ int multiply[2];            // whether the inverses are ordinary numbers
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+  const int n = a.rows, nb = (n + 15) / 16, col0 = blockIdx.x * 16;
+  const TS *m = (const TS *)a.m + blockIdx.y * a.mbs;
+  const TS *b = (const TS *)a.b.p + blockIdx.y * a.b.bs;
+  TS *x = (TS *)a.x.p + blockIdx.y * a.x.bs;
+  for (int e = threadIdx.x; e < nb * 256; e += blockDim.x) {
+    const int t = e >> 4, c = col0 + (e & 15);
+    X[e] = t < n && c < a.nrhs ? T(b[t * a.b.rs + c * a.b.cs]) : S::make(0.0, 0.0);
+  }
+  // the triangle of block `k` and the inverses of its diagonal (past n: the identity), by one wave
+  bool singular = false;
+  auto fetch_triangle = [&](int k, TS(&raw)[4]) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) raw[v] = m[min(k * 16 + 4 * v + q, n - 1) * a.ts + min(k * 16 + r16, n - 1) * a.us];
+  };
+  auto place_triangle = [&](int k, const TS(&raw)[4]) {
+    bool ordinary = true;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int t = 4 * v + q;
+      const bool diagonal = t == r16;
+      T val = a.conj ? S::conj(T(raw[v])) : T(raw[v]);
+      if (k * 16 + max(t, r16) >= n || r16 > t || (a.unit && diagonal)) val = S::make(diagonal ? 1.0 : 0.0, 0.0);
+      if (r16 <= t) tri[k & 1][r16][t - r16] = val;
+      if (diagonal) {
+        if (val == S::make(0.0, 0.0)) singular = true;
+        const T di = S::make(1.0, 0.0) / val;
+        tri[k & 1][t][16] = di;
+        const double size = fabs(S::re(di));
+        ordinary = sizeof(T) == 8 && size > 1e-280 && size < 1e280;
+      }
+    }
+    if constexpr (sizeof(T) == 8) {
+      // lane (b, i, j): element (i, j) of the inverse of the b-th 4 x 4 triangle on the diagonal
+      __builtin_amdgcn_wave_barrier();
+      const int bb = lane >> 4, i = (lane >> 2) & 3, j = lane & 3;
+      const T(*t)[TRI_LD] = &tri[k & 1][4 * bb];
+      const double e0 = t[0][16], e1 = t[1][16], e2 = t[2][16], e3 = t[3][16];
+      const double m10 = -e1 * t[0][1] * e0, m21 = -e2 * t[1][1] * e1, m32 = -e3 * t[2][1] * e2;
+      const double m20 = -e2 * fma(t[1][1], m10, t[0][2] * e0), m31 = -e3 * fma(t[2][1], m21, t[1][2] * e1);
+      const double m30 = -e3 * fma(t[2][1], m20, fma(t[1][2], m10, t[0][3] * e0));
+      double v = i == 0 ? e0 : i == 1 ? (j == 0 ? m10 : e1) : i == 2 ? (j == 0 ? m20 : j == 1 ? m21 : e2)
+                                                                     : (j == 0 ? m30 : j == 1 ? m31 : j == 2 ? m32 : e3);
+      v = j <= i ? v : 0.0;
+      ordinary = ordinary && fabs(v) < 1e280;
+      diag_inv[k & 1][bb][j * 16 + 4 * bb + i] = v;
+    }
+    const bool all = __all(ordinary);
+    if (lane == 0) multiply[k & 1] = all;
+  };
+  for (int e = threadIdx.x; e < 512; e += blockDim.x) (&diag_inv[0][0][0])[e] = 0.0;
+  __syncthreads();
+  TS raw[2][4];
+  if (wave == TRSM_LOADER) {
+    fetch_triangle(0, raw[0]);
+    fetch_triangle(1, raw[1]);
+    place_triangle(0, raw[0]);
+    fetch_triangle(2, raw[0]);
+  }
+  // coefficients of tile `t` against block `u`, as the matrix instruction takes them
+  const TS *lane_full = m + r16 * a.ts + q * a.us, *lane_last = m + min(r16, n - 1 - (nb - 1) * 16) * a.ts + q * a.us;
+  auto coefficients = [&](int t, int u, TS(&c)[4]) {
+    if constexpr (sizeof(T) == 8) {
+      const TS *p = (t == nb - 1 ? lane_last : lane_full) + (t * a.ts + u * a.us) * 16;
+      if (u == nb - 1) {  // the last triangle: nothing is read past its columns
+#pragma unroll
+        for (int k = 0; k < 4; k++) c[k] = p[(min(4 * k + q, n - 1 - u * 16) - q) * a.us];
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) c[k] = p[4 * k * a.us];
+      }
+    }
+  };
+  auto load_rows = [&](int t) {
+    LaTile<T> acc;
+#pragma unroll
+    for (int v = 0; v < 4; v++) acc.v[v] = X[(t * 16 + 4 * v + q) * 16 + r16];
+    return acc;
+  };
+  auto store_rows = [&](int t, const LaTile<T> &acc) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) X[(t * 16 + 4 * v + q) * 16 + r16] = acc.v[v];
+  };
+  // what block `u` takes from block `t`, whose coefficients are in `c`
+  auto take = [&](LaTile<T> &acc, int t, int u, const TS(&c)[4]) {
+    if constexpr (sizeof(T) == 8) {
+      la_f64x4 d = {acc.v[0], acc.v[1], acc.v[2], acc.v[3]};
+#pragma unroll
+      for (int k = 0; k < 4; k++) d = __builtin_amdgcn_mfma_f64_16x16x4f64(-(double)c[k], X[(u * 16 + 4 * k + q) * 16 + r16], d, 0, 0, 0);
+#pragma unroll
+      for (int v = 0; v < 4; v++) acc.v[v] = d[v];
+    } else {
+      for (int k = 0; k < 16; k++) {
+        const T xv = X[(u * 16 + k) * 16 + r16];
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          acc.v[v] = S::sub_mul(acc.v[v], trsm_coefficient<T, TS>(a, m, min(t * 16 + 4 * v + q, n - 1), u * 16 + k), xv);
+      }
+    }
+  };
+  __syncthreads();
+  // Three loops with the same barriers: the registers of one role are not the others'. What is read of
+  // the matrix is needed two steps later and has two sets of registers in turn (a copy from one
+  // to the other would wait for it): the first pass over it comes from beyond the L2, some 3500
+  // cycles away.
+  if (wave == 0) {
+    TS left[2][4], on[2][4];  // of the tile left of the triangle, and of the triangle
+    auto step = [&](int k, TS(&cl)[4], TS(&co)[4]) {
+      LaTile<T> acc = load_rows(k);
+      if (k > 0) take(acc, k, k - 1, cl);
+      if (k + 2 < nb) coefficients(k + 2, k + 1, cl);
+      if constexpr (sizeof(T) == 8) {
+        double tr[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const int u = 4 * v + q;
+          tr[v] = r16 < u ? 0.0 : k * 16 + r16 >= n || (a.unit && r16 == u) ? (r16 == u ? 1.0 : 0.0) : (double)co[v];
+        }
+        if (k + 2 < nb) coefficients(k + 2, k + 2, co);
+        if (multiply[k & 1]) {
+          double di[4];
+#pragma unroll
+          for (int v = 0; v < 4; v++) di[v] = diag_inv[k & 1][v][lane];
+          solve16(acc, di, tr);
+          store_rows(k, acc);
+          return;
+        }
+      }
+      store_rows(k, acc);
+      __builtin_amdgcn_wave_barrier();
+      const T(*t16)[TRI_LD] = tri[k & 1];
+      T v[16];  // this lane's right-hand side from row t on; it moves up one place with every row
+#pragma unroll
+      for (int t = 0; t < 16; t++) v[t] = X[(k * 16 + t) * 16 + r16];
+#pragma unroll 1
+      for (int t = 0; t < 16; t++) {
+        const T sol = v[0] / t16[t][0];
+        if (q == 0) X[(k * 16 + t) * 16 + r16] = sol;
+#pragma unroll
+        for (int r = 1; r < 16; r++) v[r - 1] = S::sub_mul(v[r], t16[t][r], sol);
+      }
+    };
+    coefficients(0, 0, on[0]);
+    if (nb > 1) coefficients(1, 0, left[1]), coefficients(1, 1, on[1]);
+#pragma unroll 1
+    for (int k = 0; k < nb; k += 2) {
+      step(k, left[0], on[0]);
+      __syncthreads();
+      if (k + 1 < nb) {
+        step(k + 1, left[1], on[1]);
+        __syncthreads();
+      }
+    }
+  } else if (wave == TRSM_LOADER) {
+    auto step = [&](int k, TS(&r)[4]) {
+      if (k + 1 < nb) place_triangle(k + 1, r);
+      if (k + 3 < nb) fetch_triangle(k + 3, r);
+    };
+#pragma unroll 1
+    for (int k = 0; k < nb; k += 2) {
+      step(k, raw[1]);
+      __syncthreads();
+      if (k + 1 < nb) {
+        step(k + 1, raw[0]);
+        __syncthreads();
+      }
+    }
+  } else {
+    const int first = wave < TRSM_LOADER ? wave : wave - 1;  // 1 .. TRSM_UPDATERS
+    TS c[2][TRSM_TILES][4];
+    auto request = [&](int k, TS(&to)[TRSM_TILES][4]) {  // what step `k` takes
+#pragma unroll
+      for (int i = 0; i < TRSM_TILES; i++) {
+        const int t = k + first + i * TRSM_UPDATERS;
+        if (t < nb) coefficients(t, k - 1, to[i]);
+      }
+    };
+    auto step = [&](int k, TS(&from)[TRSM_TILES][4]) {
+      if (k > 0) {
+#pragma unroll
+        for (int i = 0; i < TRSM_TILES; i++) {
+          const int t = k + first + i * TRSM_UPDATERS;
+          if (t < nb) {
+            LaTile<T> acc = load_rows(t);
+            take(acc, t, k - 1, from[i]);
+            store_rows(t, acc);
+          }
+        }
+      }
+      if (k + 2 < nb) request(k + 2, from);
+    };
+    if (nb > 1) request(1, c[1]);
+#pragma unroll 1
+    for (int k = 0; k < nb; k += 2) {
+      step(k, c[0]);
+      __syncthreads();
+      if (k + 1 < nb) {
+        step(k + 1, c[1]);
+        __syncthreads();
+      }
+    }
+  }
+  if (singular) raise_host(a.status, LA_SINGULAR);
+  for (int e = threadIdx.x; e < n * 16; e += blockDim.x) {
+    const int t = e >> 4, c = col0 + (e & 15);
+    if (c < a.nrhs) to_storage(X[e], x + t * a.x.rs + c * a.x.cs);
+  }
+}
+
+// Rows after a pass: X[t] -= sum_u M(t, u) X[u] over the pass's rows, for the next pass to solve
+// (only systems longer than one pass holds come here). A wave per 16 x 16 tile.
+template <class T, class TS>
+__global__ __launch_bounds__(256) void trsm_rest_kernel(TrsmArgs<T> a, LaMat rest, int rest_rows) {
+  using S = Sc<T>;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
+  const int t0 = (blockIdx.x * 4 + wave) * 16, c = blockIdx.y * 16 + r16;
+  if (t0 >= rest_rows) return;
+  const TS *m = (const TS *)a.m + blockIdx.z * a.mbs;
+  const TS *x = (const TS *)a.x.p + blockIdx.z * a.x.bs;
+  TS *y = (TS *)rest.p + blockIdx.z * rest.bs;
+  const int cc = min(c, a.nrhs - 1);
+  T acc[4];
+#pragma unroll
+  for (int v = 0; v < 4; v++) acc[v] = T(y[min(t0 + 4 * v + q, rest_rows - 1) * rest.rs + cc * rest.cs]);
+  for (int u = 0; u < a.rows; u++) {
+    const T xv = T(x[u * a.x.rs + cc * a.x.cs]);
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+      acc[v] = S::sub_mul(acc[v], trsm_coefficient<T, TS>(a, m, a.rows + min(t0 + 4 * v + q, rest_rows - 1), u), xv);
+  }
+  if (c >= a.nrhs) return;
+#pragma unroll
+  for (int v = 0; v < 4; v++)
+    if (t0 + 4 * v + q < rest_rows) to_storage(acc[v], y + (t0 + 4 * v + q) * rest.rs + c * rest.cs);
+}

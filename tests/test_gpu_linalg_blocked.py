@@ -1,0 +1,114 @@
+"""cholesky and triangular_solve at the edges of their blocks: 16-row steps, 64-row (complex: 32-row)
+tiles, the third block column (the first that reads the updated workspace), 1024-row passes, sixteen
+right-hand sides a workgroup, diagonals whose inverse is no ordinary number.
+
+Bounds: a factor or a solution of n terms per element in double is off by at most n eps of the
+magnitudes summed (Higham, Accuracy and Stability, theorems 10.3 and 8.5, constants below 4 n), float32
+storage by half an ulp of the result on top."""
+
+import numpy as np
+import pytest
+
+from helpers import logical
+from raven_amd import dtype as dt
+
+pytestmark = pytest.mark.gpu
+
+EPS = {"float32": 2.0 ** -24, "float64": 2.0 ** -53, "complex128": 2.0 ** -53}
+
+
+def put(hip, a, d):
+    a = np.ascontiguousarray(a)
+    return hip.reshape(hip.from_host(a, d), a.shape)
+
+
+def H(a):
+    return np.swapaxes(a, -1, -2).conj()
+
+
+def draws(rng, shape, name):
+    a = rng.standard_normal(shape)
+    return a + 1j * rng.standard_normal(shape) if name.startswith("complex") else a
+
+
+@pytest.mark.parametrize("name", ["float32", "float64", "complex128"])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 63, 64, 65, 80, 127, 128, 129, 200, 257])
+def test_cholesky_at_block_edges(hip, name, n):
+    d, rng = dt.BY_NAME[name], np.random.default_rng(n)
+    batch = (3,) if n < 130 else ()
+    g = draws(rng, batch + (n, n), name)
+    a = (g @ H(g) + n * np.eye(n)).astype(d.np_storage)
+    full = np.tril(a) + H(np.tril(a, -1))
+    full[..., np.arange(n), np.arange(n)] = full[..., np.arange(n), np.arange(n)].real
+    seen = np.tril(a) + np.triu(np.full(batch + (n, n), np.nan), 1).astype(a.dtype)  # the upper triangle is not read
+    for upper in (False, True):
+        t = hip.cholesky(put(hip, seen, d), upper)
+        f = logical(t).astype(np.complex128 if d.is_complex else np.float64)
+        assert np.all((np.tril(f, -1) if upper else np.triu(f, 1)) == 0)
+        low = H(f) if upper else f
+        wide = full.astype(low.dtype)
+        scale = np.abs(low) @ np.abs(H(low))  # (|L| |L^H|)_ij <= sqrt(a_ii a_jj)
+        assert np.all(np.abs(low @ H(low) - wide) <= (4 * n * 2.0 ** -53 + 3 * EPS[name]) * scale)
+    # the same matrix through a transposed view
+    k = len(batch)
+    t = hip.cholesky(hip.permute(put(hip, np.swapaxes(seen, -1, -2), d), tuple(range(k)) + (k + 1, k)))
+    assert np.array_equal(logical(t), logical(hip.cholesky(put(hip, seen, d))))
+
+
+@pytest.mark.parametrize("name", ["float32", "float64", "complex128"])
+@pytest.mark.parametrize("n,nrhs", [(1, 1), (15, 3), (16, 16), (17, 17), (33, 1), (64, 40), (113, 5), (512, 16), (1024, 2),
+                                    (1025, 17), (1100, 3)])
+def test_triangular_solve_at_block_edges(hip, name, n, nrhs):
+    d, rng = dt.BY_NAME[name], np.random.default_rng(1000 + n)
+    if d.is_complex and n > 520:
+        n -= 512  # (its passes are half as long)
+    batch = (2,) if n < 130 else ()
+    a = draws(rng, batch + (n, n), name) / np.sqrt(n)
+    a[..., np.arange(n), np.arange(n)] += 2 * np.sign(a[..., np.arange(n), np.arange(n)].real)
+    a, b = a.astype(d.np_storage), draws(rng, batch + (n, nrhs), name).astype(d.np_storage)
+    for upper in (False, True):
+        tri = np.triu(a) if upper else np.tril(a)
+        hidden = np.where(np.triu(np.ones((n, n)), 1).astype(bool).T if upper else np.triu(np.ones((n, n)), 1).astype(bool), np.nan, a)
+        for transpose in (False, True):
+            for unit in (False, True):
+                m = tri.astype(np.complex128 if d.is_complex else np.float64)
+                if unit:
+                    m[..., np.arange(n), np.arange(n)] = 1
+                m = H(m) if transpose else m
+                x = logical(hip.triangular_solve(put(hip, hidden.astype(d.np_storage), d), put(hip, b, d), upper, transpose, unit)).astype(m.dtype)
+                residual = np.abs(m @ x - b.astype(m.dtype))
+                bound = (4 * n * 2.0 ** -53 + 2 * EPS[name]) * (np.abs(m) @ np.abs(x)) + 4 * n * 2.0 ** -53
+                assert np.all(residual <= bound), (upper, transpose, unit, float(np.max(residual / bound)))
+
+
+def test_triangular_solve_without_ordinary_inverses(hip):
+    """Rows scaled far outside the range where a product with the inverse stands for the quotient."""
+    rng = np.random.default_rng(5)
+    n = 40
+    a = np.tril(rng.standard_normal((n, n))) + 4 * np.eye(n)
+    scale = np.ones(n)
+    scale[7], scale[20], scale[33] = 1e-300, 1e290, 3e-309
+    b = rng.standard_normal((n, 3))
+    x = logical(hip.triangular_solve(put(hip, a * scale[:, None], dt.float64), put(hip, b * scale[:, None], dt.float64), False, False, False))
+    plain = np.linalg.solve(a, b)
+    # a subnormal row keeps about 2^-42 of its values
+    assert np.all(np.isfinite(x)) and np.max(np.abs(x - plain)) <= 1e-9 * np.max(np.abs(plain))
+
+
+def test_in_place_and_shared_storage(hip):
+    """Results over the operands' own storage, as the C ABI allows."""
+    import ctypes as C
+    rng = np.random.default_rng(6)
+    n = 150
+    g = rng.standard_normal((n, n))
+    a = g @ g.T + n * np.eye(n)
+    t, want = put(hip, a, dt.float64), logical(hip.cholesky(put(hip, a, dt.float64)))
+    ds = t._desc()
+    hip._check(hip._lib.nxh_cholesky(hip._h, C.byref(ds), C.byref(ds), 0))
+    assert np.array_equal(logical(t), want)
+    b = rng.standard_normal((n, 5))
+    tb, tl = put(hip, b, dt.float64), put(hip, want, dt.float64)
+    x = logical(hip.triangular_solve(tl, put(hip, b, dt.float64), False, False, False))
+    db, dl = tb._desc(), tl._desc()
+    hip._check(hip._lib.nxh_triangular_solve(hip._h, C.byref(db), C.byref(dl), C.byref(db), 0))
+    assert np.array_equal(logical(tb), x)
