@@ -12,12 +12,13 @@
 // the real part of its +sign transform.
 //
 // How it runs here: one axis pass = one launch in which a workgroup owns one
-// line (or several short ones), loads it strided into LDS as double2, does all
-// radix-2 stages there (four at a time, sixteen elements per lane in registers) and stores it strided, so a pass reads and writes the
-// tensor exactly once. Lengths that are not a power of two go through Bluestein's
+// line (or several short ones), loads it into registers as double2, transforms it
+// by butterflies of up to sixteen elements per lane with exchanges through LDS in
+// between, and stores it from registers, so a pass reads and writes the tensor
+// exactly once. Real lines of an even length are transformed as complex lines of
+// half the length. Lengths that are not a power of two go through Bluestein's
 // identity inside the same kernel: chirp on load, a power-of-two convolution of
-// length M >= 2n-1 (forward DIF, multiply by the transformed chirp filter in
-// bit-reversed order, inverse DIT: no reordering pass), chirp on store.
+// length M >= 2n-1, chirp on store.
 // Transforms longer than the LDS holds (power of two above 8192, other lengths
 // above 4096) are staged through a complex128 workspace and done as a four-step
 // (n = n1 x n2) pair of passes of the same kernel.
@@ -32,12 +33,15 @@
 namespace {
 
 constexpr int FFT_MAXD = 8;         // other dims of a tensor's lines after merging
-constexpr int FFT_LDS_MAX = 8192;   // longest transform held in one workgroup's LDS (128 KiB)
-constexpr int FFT_LDS_MIN = 2048;   // LDS elements of a workgroup of short lines
+constexpr int FFT_LOG_MAX = 13;
+constexpr int FFT_LDS_MAX = 1 << FFT_LOG_MAX;  // longest transform held by one workgroup (68 KiB of LDS)
 constexpr int64_t FFT_WORK_ELEMS = int64_t(1) << 25;  // workspace elements per chunk of lines (512 MiB)
 
 enum Kind { K_C32 = 0, K_C64 = 1, K_F32 = 2, K_F64 = 3 };
 enum LoadMode { LOAD_COMPLEX = 0, LOAD_REAL = 1, LOAD_HERMITIAN = 2 };
+// Real lines of an even length 2n go as one complex line of length n whose element j is the pair
+// (2j, 2j + 1), at half the arithmetic and LDS of the transform of the real line itself.
+enum Pack { PACK_NONE = 0, PACK_RFFT = 1, PACK_IRFFT = 2 };
 
 static inline int kind_size(int k) { return k == K_C32 ? 8 : k == K_C64 ? 16 : k == K_F32 ? 4 : 8; }
 
@@ -56,27 +60,29 @@ struct FftArgs {
   int n;                 // transform length
   int M, logM;           // LDS transform length: n, or the Bluestein convolution length
   int n_load, load_mode, herm_s;
-  int n_store;
+  int n_store;           // (PACK_IRFFT: pairs; PACK_RFFT: bins before the last, which goes by itself)
   int sign;              // -1 forward, +1 inverse
+  int pack;              // n is then half the real length
+  int pair_aligned;      // the real side's pairs lie side by side at addresses that are multiples of a pair
   int G;                 // lines per workgroup
   // The workgroup's G lines are neighbours in memory while a line's own elements are strided
   // (a transform down the columns of a row-major tensor): consecutive lanes then take the
   // same element of consecutive lines, so that a wave's accesses are contiguous runs of G
   // elements instead of 64 separate ones. Separately for the load and the store side.
   int in_lines_fast, out_lines_fast;
-  const double2 *tw;     // exp(-2 pi i k / M), k < M/2
+  const double2 *tw;       // at len + k: exp(-2 pi i k / len), for every power of two len <= M
+  const double2 *real_tw;  // packed lines: exp(-2 pi i k / 2n), k < n
   const double2 *chirp;  // Bluestein: exp(sign pi i j^2 / n), j < n
   const double2 *bf;     // Bluestein: forward transform (length M) of the wrapped conjugate chirp
   int64_t tw_total;      // four-step: multiply bin k of a line by exp(sign 2 pi i inner k / tw_total)
 };
 
-// Element i of the lines lives at LDS index i + i / 16: one pad element per 16
-// (per 256 bytes, the width of the banks) turns the power-of-two strides of the
-// butterflies and of the bit-reversed scatter into conflict-free ones.
+// Element i of a line lives at LDS index i + i / 16: one pad element per 16 turns
+// the power-of-two strides of the exchanges into conflict-free ones.
 __device__ __forceinline__ int pad(int i) { return i + (i >> 4); }
 
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
-  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  return make_double2(__builtin_fma(a.x, b.x, -(a.y * b.y)), __builtin_fma(a.x, b.y, a.y * b.x));
 }
 
 __device__ __forceinline__ double2 load_elem(const char *base, int kind, int64_t off) {
@@ -101,8 +107,8 @@ __device__ __forceinline__ int64_t line_offset(const Lines &v, int64_t l, int *i
   int64_t off = 0;
   *inner = 0;
   for (int d = v.nd - 1; d >= 0; d--) {
-    const int64_t c = l % v.dims[d];
-    l /= v.dims[d];
+    const int64_t next = d ? l / v.dims[d] : 0, c = l - next * (d ? v.dims[d] : 0);
+    l = next;
     if (d == v.nd - 1) *inner = (int)c;
     off += c * v.strides[d];
   }
@@ -124,154 +130,348 @@ __device__ __forceinline__ double2 fetch(const FftArgs &a, int64_t off, int j) {
   return load_elem(a.in.base, a.in.kind, off + j * a.in.estride);
 }
 
-// R consecutive radix-2 stages, s .. s + R - 1 (stage s has sub-transform length
-// 2^s), in one pass over the G lines of the workgroup: a lane holds the 2^R
-// elements h = 2^(s-1) apart in registers and does every butterfly among them,
-// so the lines go through LDS once per R stages (the stages are bound by LDS
-// bandwidth: 32 bytes per element and pass). The arithmetic per element is that
-// of R single stages in the same order. DIT (stages upwards): input bit-reversed,
-// output natural. DIF (stages downwards): input natural, output bit-reversed.
-// The twiddle table stays in global memory (small and cache-resident; a copy in
-// LDS measured slower).
-template <bool DIF, int R>
-__device__ __forceinline__ void stages(double2 *lds, const FftArgs &a, int s, int sign) {
-  constexpr int N = 1 << R;
-  const double2 *tw = a.tw;
-  const int h = 1 << (s - 1);
-  const int per_line = a.M >> R;
-  const int total = a.G * per_line;
-  for (int b = threadIdx.x; b < total; b += blockDim.x) {
-    const int g = b >> (a.logM - R);
-    const int r = b & (per_line - 1);
-    const int pos = r & (h - 1);
-    const int i0 = (g << a.logM) + ((r >> (s - 1)) << (s - 1 + R)) + pos;
-    double2 x[N];
+// ── the transform in registers ──────────────────────────────────────────────
+// A line of M = 2^L elements belongs to T = M / E lanes that hold E elements each: slot e of
+// lane t is element t + T e, before the transform, after it, and at the start of every pass (the
+// self-sorting order: natural in, natural out). A pass does the butterflies of radix R <= E that
+// a lane's own slots make up and then redistributes the line through LDS.
+constexpr int log_elems(int L) { return L >= 8 ? 4 : L >= 6 ? 3 : L >= 4 ? 2 : L >= 1 ? 1 : 0; }
+
+// v exp(-2 pi i k / 32), k < 32 known to the compiler
+__device__ __forceinline__ double2 turn(double2 v, int k) {
+  constexpr double c[9] = {1, 0.98078528040323043, 0.92387953251128674, 0.83146961230254524, 0.70710678118654757,
+                           0.55557023301960218, 0.38268343236508978, 0.19509032201612825, 0};
+  if (k & 16) v = make_double2(-v.x, -v.y);
+  if (k & 8) v = make_double2(v.y, -v.x);
+  k &= 7;
+  return k ? cmul(v, make_double2(c[k], -c[8 - k])) : v;
+}
+
+// The forward DFT of length R over x[0], x[G], x[2 G], ... in natural order.
+template <int R, int G, int N>
+__device__ __forceinline__ void dft(double2 (&x)[N], int o) {
+  if constexpr (R == 2) {
+    const double2 u = x[o], v = x[o + G];
+    x[o] = make_double2(u.x + v.x, u.y + v.y);
+    x[o + G] = make_double2(u.x - v.x, u.y - v.y);
+  } else if constexpr (R == 4) {
+    const double2 a = x[o], b = x[o + G], c = x[o + 2 * G], d = x[o + 3 * G];
+    const double2 s0 = make_double2(a.x + c.x, a.y + c.y), d0 = make_double2(a.x - c.x, a.y - c.y);
+    const double2 s1 = make_double2(b.x + d.x, b.y + d.y), d1 = make_double2(b.x - d.x, b.y - d.y);
+    x[o] = make_double2(s0.x + s1.x, s0.y + s1.y);
+    x[o + 2 * G] = make_double2(s0.x - s1.x, s0.y - s1.y);
+    x[o + G] = make_double2(d0.x + d1.y, d0.y - d1.x);
+    x[o + 3 * G] = make_double2(d0.x - d1.y, d0.y + d1.x);
+  } else {
+    // R = P x 4: transforms of length 4 over every P-th element, twiddles, transforms of length P
+    constexpr int P = R / 4;
+    double2 y[R];
 #pragma unroll
-    for (int k = 0; k < N; k++) x[k] = lds[pad(i0 + k * h)];
+    for (int p = 0; p < P; p++) {
+      double2 z[4];
 #pragma unroll
-    for (int qq = 0; qq < R; qq++) {
-      const int q = DIF ? R - 1 - qq : qq, span = 1 << q;
+      for (int b = 0; b < 4; b++) z[b] = x[o + (p + P * b) * G];
+      dft<4, 1>(z, 0);
 #pragma unroll
-      for (int k = 0; k < N; k++) {
-        if (k & span) continue;
-        // the pair's position inside its sub-transform of length 2^(s+q)
-        double2 w = tw[(pos + (k & (span - 1)) * h) << (a.logM - s - q)];
-        if (sign > 0) w.y = -w.y;
-        const double2 u = x[k], v = x[k + span];
-        if (DIF) {
-          x[k] = make_double2(u.x + v.x, u.y + v.y);
-          x[k + span] = cmul(make_double2(u.x - v.x, u.y - v.y), w);
-        } else {
-          const double2 t = cmul(w, v);
-          x[k] = make_double2(u.x + t.x, u.y + t.y);
-          x[k + span] = make_double2(u.x - t.x, u.y - t.y);
-        }
+      for (int q = 0; q < 4; q++) {
+        y[q * P + p] = turn(z[q], p * q * (32 / R));
       }
     }
 #pragma unroll
-    for (int k = 0; k < N; k++) lds[pad(i0 + k * h)] = x[k];
+    for (int q = 0; q < 4; q++) {
+      double2 z[P];
+#pragma unroll
+      for (int p = 0; p < P; p++) z[p] = y[q * P + p];
+      dft<P, 1>(z, 0);
+#pragma unroll
+      for (int p = 0; p < P; p++) x[o + (q + 4 * p) * G] = z[p];
+    }
   }
-  __syncthreads();
 }
 
-// All stages of the lines in LDS, FFT_RADIX_LOG2 at a time; the stages left over
-// (fewer than that) go first in DIT order, last in DIF order.
-constexpr int FFT_RADIX_LOG2 = 4;
-template <bool DIF>
-__device__ __forceinline__ void all_stages(double2 *lds, const FftArgs &a, int sign) {
-  constexpr int R = FFT_RADIX_LOG2;
-  const int rem = a.logM % R;
-  auto odd = [&](int s) {
-    if (rem == 1) stages<DIF, 1>(lds, a, s, sign);
-    else if (rem == 2) stages<DIF, 2>(lds, a, s, sign);
-    else if (rem == 3) stages<DIF, 3>(lds, a, s, sign);
+// Slot e of every lane goes to place `to(e)` of its line, place t + T e comes back into slot e.
+// Real and imaginary parts go one after the other through the same LDS: half the LDS per line,
+// so twice the waves in flight (LDS is what limits them), for the same bytes moved.
+template <int E, int T, class To>
+__device__ __forceinline__ void exchange(double2 (&x)[E], double *line, const double *from, int t, To to) {
+#pragma unroll
+  for (int part = 0; part < 2; part++) {
+    __syncthreads();  // what the LDS held before has been read
+#pragma unroll
+    for (int e = 0; e < E; e++) line[pad(to(e))] = part ? x[e].y : x[e].x;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; e++) (part ? x[e].y : x[e].x) = from[pad(t + T * e)];
+  }
+}
+
+// The forward transform of the workgroup's lines, from sub-transforms of length 2^S on. `line` is
+// the lane's own line in LDS. Element (jm, k) of a pass is turned by w^k, w = exp(-2 pi i jm / 2^(S+r)):
+// w, w^2, w^4 and w^8 of the lane's first butterfly are read from the table (neighbouring lanes,
+// neighbouring entries), everything else is a product of those and of constants. The L1 is what
+// table reads cost: with one for each of the R - 1 powers of every butterfly it stalled for two
+// thirds of the kernel's time. The roundings are those of radix-2 stages, which turn an element
+// once a stage.
+template <int L, int S>
+__device__ __forceinline__ void fft_passes(double2 (&x)[1 << log_elems(L)], double *line, const double2 *tw, int t) {
+  constexpr int E = 1 << log_elems(L), T = (1 << L) / E;
+  constexpr int r = L - S < log_elems(L) ? L - S : log_elems(L), R = 1 << r, G = E / R;
+  if constexpr (R > 1) {
+    if constexpr (S > 0) {
+      static_assert(G == 1 || S + r == L, "only the last pass has several butterflies a lane, T apart");
+      const int jm = t & ((1 << S) - 1);
+      double2 w[R];
+#pragma unroll
+      for (int k = 1; k < R; k++) {
+        const int low = k == 3 ? 1 : k & 3;
+        if (low && low != k) w[k] = cmul(w[k - low], w[low]);
+        else if (k == 12) w[k] = cmul(w[k - 4], w[k - 8]);
+        else w[k] = tw[(1 << (S + r)) / k + jm];  // k = 1, 2, 4, 8
+#pragma unroll
+        for (int g = 0; g < G; g++) x[g + k * G] = cmul(x[g + k * G], turn(w[k], g * k * (32 / E)));
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < G; g++) dft<R, G>(x, g);
+  }
+  if constexpr (S + r < L) {
+    exchange<E, T>(x, line, line, t, [&](int e) {
+      const int j = t + (e % G) * T, k = e / G;
+      return ((j >> S) << (S + r)) + (j & ((1 << S) - 1)) + (k << S);
+    });
+    fft_passes<L, S + r>(x, line, tw, t);
+  }
+}
+
+// exp(-2 pi i k / 2n) for slot e of lane t (k = t + T e). Where n is the transform length itself
+// the T e part is a constant.
+template <int E, int T, bool BLUE>
+__device__ __forceinline__ double2 real_twiddle(const FftArgs &a, int t, int e) {
+  return BLUE ? a.real_tw[t + T * e < a.n ? t + T * e : 0] : turn(a.real_tw[t], e * (16 / E));
+}
+
+template <class V>
+__device__ __forceinline__ double2 widen(V v) {
+  if constexpr (std::is_same_v<V, float> || std::is_same_v<V, double>) return make_double2(v, 0.0);
+  else return make_double2(v.x, v.y);
+}
+
+// The E elements t, t + T, ... of the line at `off`; what a line does not have reads as zero. All
+// loads are issued, from addresses that every line has, before the first value is looked at: with
+// the conversion to double beside each guarded load a wave waited for one load after the other
+// (rfft [8192, 2048] float32: 76 us against 58).
+template <int E, int T, bool BLUE>
+__device__ __forceinline__ void load_line(const FftArgs &a, double2 (&x)[E], int64_t off, int t) {
+  const int64_t es = a.in.estride;
+  constexpr int USED = BLUE ? (E + 1) / 2 : E;  // the second half of a convolution's line is padding
+#pragma unroll
+  for (int e = 0; e < E; e++) x[e] = make_double2(0.0, 0.0);
+  if (a.n_load < 1) return;
+  // load(element number times `per`), for elements below `limit`
+  const auto each = [&](int limit, int per, auto load) {
+    decltype(load(off)) raw[USED];
+    const int64_t at = off + (int64_t)t * per * es, step = (int64_t)T * per * es;
+#pragma unroll
+    for (int e = 0; e < USED; e++) raw[e] = load(t + T * e < limit ? at + e * step : off);
+#pragma unroll
+    for (int e = 0; e < USED; e++)
+      if (t + T * e < limit) x[e] = widen(raw[e]);
   };
-  if (DIF) {
-    for (int s = a.logM - R + 1; s >= rem + 1; s -= R) stages<true, R>(lds, a, s, sign);
-    odd(1);
+  const auto single = [&](auto p) { each(a.n_load < a.n ? a.n_load : a.n, 1, [=](int64_t at) { return p[at]; }); };
+  if (a.pack == PACK_RFFT) {
+    const float *pf = (const float *)a.in.base;
+    const double *pd = (const double *)a.in.base;
+    if (a.in.kind == K_F32 && a.pair_aligned) each(a.n, 2, [=](int64_t at) { return *(const float2 *)(pf + at); });
+    else if (a.in.kind == K_F32) each(a.n, 2, [=](int64_t at) { return make_float2(pf[at], pf[at + es]); });
+    else each(a.n, 2, [=](int64_t at) { return make_double2(pd[at], pd[at + es]); });
+  } else if (a.pack == PACK_IRFFT) {
+    // The spectrum of the packed line, bins j and n - j at a time. The real part of the whole
+    // transform never sees the imaginary parts of bins 0 and n (unless they are no numbers).
+    const auto both = [&](auto p) {
+      constexpr int HALF = (USED + 1) / 2;  // half at a time: twice the values are in registers here
+#pragma unroll
+      for (int e0 = 0; e0 < USED; e0 += HALF) {
+        std::decay_t<decltype(p[0])> u[HALF], v[HALF];
+#pragma unroll
+        for (int e = e0; e < e0 + HALF && e < USED; e++) {
+          const int j = t + T * e, k = a.n - j;
+          u[e - e0] = p[off + (j < a.n_load ? j : 0) * es];
+          v[e - e0] = p[off + (k >= 0 && k < a.n_load ? k : 0) * es];
+        }
+#pragma unroll
+        for (int e = e0; e < e0 + HALF && e < USED; e++) {
+          const int j = t + T * e, k = a.n - j;
+          if (k <= 0) continue;
+          double2 lo = j < a.n_load ? widen(u[e - e0]) : make_double2(0.0, 0.0);
+          double2 hi = k < a.n_load ? widen(v[e - e0]) : make_double2(0.0, 0.0);
+          if (j == 0) lo = make_double2(lo.x + 0.0 * lo.y, 0.0), hi = make_double2(hi.x + 0.0 * hi.y, 0.0);
+          const double2 w = real_twiddle<E, T, BLUE>(a, t, e);
+          const double2 odd = cmul(make_double2(lo.x - hi.x, lo.y + hi.y), make_double2(w.x, -w.y));
+          x[e] = make_double2(lo.x + hi.x - odd.y, lo.y - hi.y + odd.x);
+        }
+      }
+    };
+    if (a.in.kind == K_C32) both((const float2 *)a.in.base);
+    else both((const double2 *)a.in.base);
+  } else if (a.load_mode == LOAD_HERMITIAN) {
+#pragma unroll
+    for (int e = 0; e < USED; e++)
+      if (t + T * e < a.n) x[e] = fetch(a, off, t + T * e);
   } else {
-    odd(1);
-    for (int s = rem + 1; s + R - 1 <= a.logM; s += R) stages<false, R>(lds, a, s, sign);
+    switch (a.in.kind) {
+      case K_C32: single((const float2 *)a.in.base); break;
+      case K_C64: single((const double2 *)a.in.base); break;
+      case K_F32: single((const float *)a.in.base); break;
+      default: single((const double *)a.in.base);
+    }
   }
 }
 
-template <bool BLUE>
-__global__ __launch_bounds__(1024) void fft_lines_kernel(FftArgs a) {
-  extern __shared__ double2 lds[];
-  int64_t *off_in = (int64_t *)(lds + pad(a.G << a.logM) + 1);
-  int64_t *off_out = off_in + a.G;
-  int *inner = (int *)(off_out + a.G);
+template <int E, int T, bool BLUE>
+__device__ __forceinline__ void store_line(const FftArgs &a, const double2 (&x)[E], int64_t off, int t) {
+  const int64_t es = a.out.estride;
+  const auto each = [&](int per, auto store) {
+    const int64_t at = off + (int64_t)t * per * es, step = (int64_t)T * per * es;
+#pragma unroll
+    for (int e = 0; e < E; e++)
+      if ((!BLUE || e < (E + 1) / 2) && t + T * e < a.n_store) store(at + e * step, x[e]);
+  };
+  if (a.pack == PACK_IRFFT) {
+    if (a.out.kind == K_F32 && a.pair_aligned)
+      each(2, [&](int64_t at, double2 v) { *(float2 *)(a.out.base + at * 4) = make_float2((float)v.x, (float)v.y); });
+    else if (a.out.kind == K_F32)
+      each(2, [&](int64_t at, double2 v) { float *p = (float *)a.out.base + at; p[0] = (float)v.x, p[es] = (float)v.y; });
+    else
+      each(2, [&](int64_t at, double2 v) { double *p = (double *)a.out.base + at; p[0] = v.x, p[es] = v.y; });
+    return;
+  }
+  switch (a.out.kind) {
+    case K_C32: each(1, [&](int64_t at, double2 v) { store_elem(a.out.base, K_C32, at, v); }); break;
+    case K_C64: each(1, [&](int64_t at, double2 v) { store_elem(a.out.base, K_C64, at, v); }); break;
+    case K_F32: each(1, [&](int64_t at, double2 v) { store_elem(a.out.base, K_F32, at, v); }); break;
+    default: each(1, [&](int64_t at, double2 v) { store_elem(a.out.base, K_F64, at, v); });
+  }
+}
+
+// +sign transforms run as the forward one between two exchanges of real and imaginary parts.
+__device__ __forceinline__ double2 flip(double2 v) { return make_double2(v.y, v.x); }
+
+// One launch = one pass over the tensor: G lines a workgroup, read straight into registers,
+// transformed, and stored from registers: besides the tensor's own traffic there are 32 bytes of
+// LDS per element and exchange (two exchanges for M = 512 .. 4096). The form before went through
+// LDS after the load, every four stages and before the store, and read a twiddle per butterfly.
+// Measured: rfft [8192, 2048] float32 170 -> 53 us, irfft back 158 -> 46 us
+// (2.5 TB/s; three waves a SIMD by registers, and the waits of a wave's own chain bound it now).
+template <int L, bool BLUE>
+__global__ __launch_bounds__(512) void fft_lines_kernel(FftArgs a) {
+  extern __shared__ double lds[];
+  constexpr int M = 1 << L, E = 1 << log_elems(L), T = M / E, PITCH = M + M / 16 + 1;
   // blocks that share an XCD (ids equal modulo 8) take neighbouring groups of lines: with
   // strided lines a 128-byte line of memory serves several workgroups, which then meet in one L2
   uint32_t bx = blockIdx.x;
-  if ((gridDim.x & 7u) == 0) bx = (bx & 7u) * (gridDim.x >> 3) + (bx >> 3);
+  if ((a.in_lines_fast || a.out_lines_fast) && (gridDim.x & 7u) == 0) bx = (bx & 7u) * (gridDim.x >> 3) + (bx >> 3);
   const int64_t first = (int64_t)bx * a.G;
-  for (int g = threadIdx.x; g < a.G; g += blockDim.x) {
-    const int64_t l = first + g;
-    int in_c = 0, out_c = 0;
-    off_in[g] = l < a.lines ? line_offset(a.in, a.line0 + l, &in_c) : 0;
-    off_out[g] = l < a.lines ? line_offset(a.out, a.line0 + l, &out_c) : 0;
-    inner[g] = out_c;
-  }
-  __syncthreads();
-  const int total = a.G << a.logM;
-  const int shift = 32 - a.logM;
-  for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
-    int g = idx >> a.logM, j = idx & (a.M - 1);
-    if (a.in_lines_fast) j = idx / a.G, g = idx - j * a.G;
-    double2 v = make_double2(0.0, 0.0);
-    if (first + g < a.lines && j < a.n) {
-      v = fetch(a, off_in[g], j);
-      if (BLUE) v = cmul(v, a.chirp[j]);
-    }
-    // the plain transform is decimation in time: it wants its input bit-reversed
-    const int p = BLUE || a.logM == 0 ? j : (int)(__brev((unsigned)j) >> shift);
-    lds[pad((g << a.logM) + p)] = v;
-  }
-  __syncthreads();
+  int g = threadIdx.x / T, t = threadIdx.x & (T - 1), unused;
+  if (a.in_lines_fast) t = threadIdx.x / a.G, g = threadIdx.x - t * a.G;
+  double2 x[E];
+  // lanes beyond the last line work on it once more and store nothing
+  const int64_t from_line = first + g < a.lines ? first + g : a.lines - 1;
+  load_line<E, T, BLUE>(a, x, line_offset(a.in, a.line0 + from_line, &unused), t);
   if (BLUE) {
-    all_stages<true>(lds, a, -1);
-    for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
-      const int p = idx & (a.M - 1);
-      const int k = a.logM == 0 ? 0 : (int)(__brev((unsigned)p) >> shift);
-      lds[pad(idx)] = cmul(lds[pad(idx)], a.bf[k]);
+#pragma unroll
+    for (int e = 0; e < (E + 1) / 2; e++) {
+      const int j = t + T * e;
+      if (j < a.n) x[e] = cmul(x[e], a.chirp[j]);
     }
-    __syncthreads();
-    all_stages<false>(lds, a, +1);
-  } else {
-    all_stages<false>(lds, a, a.sign);
+  } else if (a.sign > 0) {
+#pragma unroll
+    for (int e = 0; e < E; e++) x[e] = flip(x[e]);
   }
-  const double inv_m = 1.0 / (double)a.M;
-  const int stores = a.G * a.n_store;
-  for (int idx = threadIdx.x; idx < stores; idx += blockDim.x) {
-    // whole power-of-two lines (the common case) are decoded without a division
-    int g = a.n_store == a.M ? idx >> a.logM : idx / a.n_store, k = idx - g * a.n_store;
-    if (a.out_lines_fast) {
-      k = idx / a.G, g = idx - k * a.G;
-      if (first + g >= a.lines) continue;
-    } else if (first + g >= a.lines) {
-      break;
+  double *line = lds + g * PITCH;
+  fft_passes<L, 0>(x, line, a.tw, t);
+  if (BLUE) {
+#pragma unroll
+    for (int e = 0; e < E; e++) x[e] = flip(cmul(x[e], a.bf[t + T * e]));
+    fft_passes<L, 0>(x, line, a.tw, t);
+    const double inv_m = 1.0 / (double)M;
+#pragma unroll
+    for (int e = 0; e < (E + 1) / 2; e++) {
+      const int j = t + T * e;
+      x[e] = flip(x[e]);
+      if (j < a.n) {
+        const double2 c = a.chirp[j];
+        x[e] = cmul(x[e], make_double2(c.x * inv_m, c.y * inv_m));
+      }
     }
-    double2 v = lds[pad((g << a.logM) + k)];
-    if (BLUE) {
-      const double2 c = a.chirp[k];
-      v = cmul(v, make_double2(c.x * inv_m, c.y * inv_m));
+  } else if (a.sign > 0) {
+#pragma unroll
+    for (int e = 0; e < E; e++) x[e] = flip(x[e]);
+  }
+  if (a.pack == PACK_RFFT) {
+    // bin k of the real line's transform from bins k and n - k of the packed one
+    const double2 zero = x[0];
+    double odd_im[E];
+#pragma unroll
+    for (int part = 0; part < 2; part++) {
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < E; e++) line[pad(t + T * e)] = part ? x[e].y : x[e].x;
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < E; e++) {
+        const int k = t + T * e;
+        const double m = line[pad(k && k < a.n ? a.n - k : 0)];
+        if (part == 0) {
+          odd_im[e] = 0.5 * (m - x[e].x);
+          x[e].x = 0.5 * (x[e].x + m);
+        } else if (k < a.n) {
+          const double2 w = cmul(make_double2(0.5 * (x[e].y + m), odd_im[e]), real_twiddle<E, T, BLUE>(a, t, e));
+          x[e] = make_double2(x[e].x + w.x, 0.5 * (x[e].y - m) + w.y);
+        }
+      }
     }
-    if (a.tw_total) {
+    if (t == 0 && first + g < a.lines) {  // bin n: the difference of the two halves' sums
+      const int64_t off = line_offset(a.out, a.line0 + first + g, &unused);
+      store_elem(a.out.base, a.out.kind, off + (int64_t)a.n * a.out.estride, make_double2(zero.x - zero.y, 0.0));
+    }
+  }
+  if (a.in_lines_fast != a.out_lines_fast) {  // the store wants the other order of lanes
+    const int from = t;
+    g = threadIdx.x / T, t = threadIdx.x & (T - 1);
+    if (a.out_lines_fast) t = threadIdx.x / a.G, g = threadIdx.x - t * a.G;
+    exchange<E, T>(x, line, lds + g * PITCH, t, [&](int e) { return from + T * e; });
+  }
+  if (first + g >= a.lines) return;
+  int inner;
+  const int64_t off = line_offset(a.out, a.line0 + first + g, &inner);
+  if (a.tw_total) {
+#pragma unroll
+    for (int e = 0; e < E; e++) {
       double sn, cs;
-      sincospi(2.0 * (double)((int64_t)inner[g] * k) / (double)a.tw_total, &sn, &cs);
-      v = cmul(v, make_double2(cs, a.sign > 0 ? sn : -sn));
+      sincospi(2.0 * (double)((int64_t)inner * (t + T * e)) / (double)a.tw_total, &sn, &cs);
+      x[e] = cmul(x[e], make_double2(cs, a.sign > 0 ? sn : -sn));
     }
-    store_elem(a.out.base, a.out.kind, off_out[g] + (int64_t)k * a.out.estride, v);
   }
+  store_line<E, T, BLUE>(a, x, off, t);
 }
 
 // ── tables ──────────────────────────────────────────────────────────────────
-__global__ void twiddle_kernel(double2 *tw, int M) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= M / 2) return;
+// Entry len + k: exp(-2 pi i k / len), len the powers of two (entry 0 is not used).
+__global__ void twiddle_kernel(double2 *tw, int count) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= count) return;
+  const int len = 1 << (31 - __clz(i | 1)), k = i & (len - 1);
   double sn, cs;
-  sincospi(2.0 * (double)k / (double)M, &sn, &cs);  // k / M is exact or correctly rounded: M is a power of two
+  sincospi(2.0 * (double)k / (double)len, &sn, &cs);  // an exact argument
+  tw[i] = make_double2(cs, -sn);
+}
+
+// exp(-2 pi i k / n), k < count
+__global__ void real_twiddle_kernel(double2 *tw, int n, int count) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= count) return;
+  double sn, cs;
+  sincospi(2.0 * (double)k / (double)n, &sn, &cs);
   tw[k] = make_double2(cs, -sn);
 }
 
@@ -346,7 +546,10 @@ static inline int log2_of(int64_t n) {
   return l;
 }
 
-enum TableKind : uint64_t { T_TWIDDLE = 1, T_CHIRP = 2, T_FILTER = 3 };
+// A transform too long for one workgroup is done as n1 x n2.
+static inline int64_t four_step_n1(int64_t M) { return int64_t(1) << ((log2_of(M) + 1) / 2); }
+
+enum TableKind : uint64_t { T_TWIDDLE = 1, T_CHIRP = 2, T_FILTER = 3, T_REAL = 4 };
 static inline uint64_t table_key(TableKind k, int64_t n, int sign) {
   return ((uint64_t)k << 60) | ((uint64_t)(sign > 0) << 59) | (uint64_t)n;
 }
@@ -385,14 +588,19 @@ static void table_drop(nxh_context *ctx, uint64_t key) {
   ctx->device_tables.erase(it);
 }
 
-static int twiddles(nxh_context *ctx, int M, const double2 **out) {
+// The table of transforms of length n: of their stages (T_TWIDDLE), or of packed real lines (T_REAL).
+static int twiddles(nxh_context *ctx, TableKind kind, int n, const double2 **out) {
   double2 *t;
   bool fresh;
-  if (int rc = table_lookup(ctx, table_key(T_TWIDDLE, M, -1), (size_t)(M / 2) * sizeof(double2), &t, &fresh)) return rc;
-  if (fresh && M >= 2) {
-    hipLaunchKernelGGL(twiddle_kernel, dim3((M / 2 + 255) / 256), dim3(256), 0, ctx->stream, t, M);
+  const uint64_t key = table_key(kind, n, -1);
+  const int count = kind == T_TWIDDLE ? 2 * n : n / 2;
+  if (int rc = table_lookup(ctx, key, (size_t)count * sizeof(double2), &t, &fresh)) return rc;
+  if (fresh) {
+    const dim3 grid((count + 255) / 256), block(256);
+    if (kind == T_TWIDDLE) hipLaunchKernelGGL(twiddle_kernel, grid, block, 0, ctx->stream, t, count);
+    else hipLaunchKernelGGL(real_twiddle_kernel, grid, block, 0, ctx->stream, t, n, count);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) {
-      table_drop(ctx, table_key(T_TWIDDLE, M, -1));
+      table_drop(ctx, key);
       return nxh_hip_fail("fft", e);
     }
   }
@@ -414,31 +622,38 @@ static Lines workspace_lines(double2 *w, int64_t outer, int64_t outer_stride, in
   return v;
 }
 
+using LinesKernel = void (*)(FftArgs);
+template <bool BLUE, int... L>
+static LinesKernel lines_kernel(int logM, std::integer_sequence<int, L...>) {
+  static constexpr LinesKernel table[] = {fft_lines_kernel<L, BLUE>...};
+  return table[logM];
+}
+
 static int launch_lines(nxh_context *ctx, FftArgs &a, bool blue) {
-  // short lines share a workgroup of FFT_LDS_MIN elements; long ones get one each
-  a.G = a.M >= FFT_LDS_MIN ? 1 : FFT_LDS_MIN / a.M;
+  // short lines share a wave; a longer line takes a workgroup of its own
+  const int lanes = a.M >> log_elems(a.logM);
+  a.G = lanes >= 64 ? 1 : 64 / lanes;
   // strided lines whose neighbours are adjacent in memory: as many lines per workgroup as make
   // runs of 128 bytes, or as the LDS holds
   auto neighbours = [](const Lines &v) { return v.estride != 1 && v.nd >= 1 && v.strides[v.nd - 1] == 1 && v.dims[v.nd - 1] > 1; };
   a.in_lines_fast = neighbours(a.in);
   a.out_lines_fast = neighbours(a.out);
-  if (a.in_lines_fast || a.out_lines_fast) a.G = std::max(1, std::min(FFT_LDS_MAX / a.M, std::max(16, FFT_LDS_MIN / a.M)));
+  if (a.in_lines_fast || a.out_lines_fast) a.G = std::max(1, std::min(FFT_LDS_MAX / a.M, std::max(16, a.G)));
   if ((int64_t)a.G > a.lines) a.G = (int)a.lines;
   if (a.G == 1) a.in_lines_fast = a.out_lines_fast = 0;
   const int64_t blocks = (a.lines + a.G - 1) / a.G;
   if (blocks > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, "fft", "too many lines for one launch");
-  const int64_t elems = (int64_t)a.G * a.M;
-  const int threads = elems >= 8192 ? 1024 : elems >= 4096 ? 512 : 256;
-  const size_t lds = (size_t)(elems + elems / 16 + 1) * sizeof(double2) + (size_t)a.G * (2 * sizeof(int64_t) + sizeof(int));
-  auto kern = blue ? fft_lines_kernel<true> : fft_lines_kernel<false>;
-  static std::once_flag once[2];
-  static hipError_t attr_status[2] = {hipSuccess, hipSuccess};
-  std::call_once(once[blue], [&] {
-    attr_status[blue] = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                            (int)((FFT_LDS_MAX + FFT_LDS_MAX / 16) * sizeof(double2) + 4096));
+  const size_t lds = (size_t)a.G * (a.M + a.M / 16 + 1) * sizeof(double);
+  constexpr auto lengths = std::make_integer_sequence<int, FFT_LOG_MAX + 1>{};
+  const auto kern = blue ? lines_kernel<true>(a.logM, lengths) : lines_kernel<false>(a.logM, lengths);
+  static std::once_flag once[2][FFT_LOG_MAX + 1];
+  static hipError_t attr_status[2][FFT_LOG_MAX + 1];
+  std::call_once(once[blue][a.logM], [&] {
+    attr_status[blue][a.logM] = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                    (int)((FFT_LDS_MAX + FFT_LDS_MAX / 16) * sizeof(double) + 4096));
   });
-  NXH_HIP("fft", attr_status[blue]);
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(threads), lds, ctx->stream, a);
+  NXH_HIP("fft", attr_status[blue][a.logM]);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(a.G * lanes), lds, ctx->stream, a);
   NXH_HIP("fft", hipGetLastError());
   return NXH_OK;
 }
@@ -455,11 +670,10 @@ static int pow2_workspace(nxh_context *ctx, double2 *src, double2 *dst, int64_t 
     a.lines = lines;
     a.n = a.M = a.n_load = a.n_store = (int)M;
     a.logM = log2_of(M);
-    if (int rc = twiddles(ctx, a.M, &a.tw)) return rc;
+    if (int rc = twiddles(ctx, T_TWIDDLE, a.M, &a.tw)) return rc;
     return launch_lines(ctx, a, false);
   }
-  const int lg = log2_of(M);
-  const int64_t n1 = int64_t(1) << ((lg + 1) / 2), n2 = M / n1;
+  const int64_t n1 = four_step_n1(M), n2 = M / n1;
   if (n1 > FFT_LDS_MAX) return nxh_fail(NXH_FAILURE, "fft", "axis too long (the limit is 2^26 elements)");
   // x[j1 n2 + j2] -> X[k1 + n1 k2]: transforms of length n1 down the columns, a
   // twiddle exp(sign 2 pi i j2 k1 / M), transforms of length n2 along the rows
@@ -468,7 +682,7 @@ static int pow2_workspace(nxh_context *ctx, double2 *src, double2 *dst, int64_t 
   a.n = a.M = a.n_load = a.n_store = (int)n1;
   a.logM = log2_of(n1);
   a.tw_total = M;
-  if (int rc = twiddles(ctx, a.M, &a.tw)) return rc;
+  if (int rc = twiddles(ctx, T_TWIDDLE, a.M, &a.tw)) return rc;
   if (int rc = launch_lines(ctx, a, false)) return rc;
   a.in = workspace_lines(src, lines, M, n1, n2, 1);
   a.out = workspace_lines(dst, lines, M, n1, 1, n1);
@@ -476,7 +690,7 @@ static int pow2_workspace(nxh_context *ctx, double2 *src, double2 *dst, int64_t 
   a.n = a.M = a.n_load = a.n_store = (int)n2;
   a.logM = log2_of(n2);
   a.tw_total = 0;
-  if (int rc = twiddles(ctx, a.M, &a.tw)) return rc;
+  if (int rc = twiddles(ctx, T_TWIDDLE, a.M, &a.tw)) return rc;
   return launch_lines(ctx, a, false);
 }
 
@@ -521,6 +735,25 @@ static int bluestein_tables(nxh_context *ctx, int64_t n, int64_t M, int sign, co
   return NXH_OK;
 }
 
+// Whether the tables of transforms of length n (convolved at length M) exist already.
+static bool tables_present(nxh_context *ctx, int64_t n, int64_t M, int sign) {
+  const auto have = [&](TableKind kind, int64_t len, int s) { return ctx->device_tables.count(table_key(kind, len, s)) != 0; };
+  const bool stages = M <= FFT_LDS_MAX ? have(T_TWIDDLE, M, -1)
+                                       : have(T_TWIDDLE, four_step_n1(M), -1) && have(T_TWIDDLE, M / four_step_n1(M), -1);
+  return stages && (n == M || (have(T_CHIRP, n, sign) && have(T_FILTER, n, sign)));
+}
+
+static int line_tables(nxh_context *ctx, int64_t n, int64_t M, int sign) {
+  if (tables_present(ctx, n, M, sign)) return NXH_OK;
+  const double2 *unused, *unused2;
+  const int64_t n1 = M <= FFT_LDS_MAX ? M : four_step_n1(M);
+  if (n1 > FFT_LDS_MAX) return NXH_OK;  // a length that the general path refuses
+  if (int rc = twiddles(ctx, T_TWIDDLE, (int)n1, &unused)) return rc;
+  if (n1 < M)
+    if (int rc = twiddles(ctx, T_TWIDDLE, (int)(M / n1), &unused)) return rc;
+  return n == M ? NXH_OK : bluestein_tables(ctx, n, M, sign, &unused, &unused2);
+}
+
 // One axis pass: every line of `in` (n_load stored elements, read per
 // `load_mode`) is transformed at length n and its first n_store bins are stored
 // to `out` (their real parts when `out` is real). `in` and `out` may be the same tensor.
@@ -528,25 +761,47 @@ static int transform_lines(nxh_context *ctx, const Lines &in, const Lines &out, 
                            int load_mode, int64_t n_store, int sign) {
   if (lines == 0 || n == 0 || n_store == 0) return NXH_OK;
   if (n > (int64_t(1) << 26)) return nxh_fail(NXH_FAILURE, "fft", "axis too long (the limit is 2^26 elements)");
-  const bool blue = !is_pow2(n);
-  const int64_t M = blue ? int64_t(1) << log2_of(2 * n - 1) : n;
-  if (M > (int64_t(1) << 26)) return nxh_fail(NXH_FAILURE, "fft", "axis too long for a length that is not a power of two (the limit is 2^25 elements)");
+  // real lines of an even length, one side real and the other the half spectrum, go packed
+  const int pack = n % 2 ? PACK_NONE
+                   : load_mode == LOAD_REAL && n_load == n && n_store == n / 2 + 1 ? PACK_RFFT
+                   : load_mode == LOAD_HERMITIAN && out.kind >= K_F32 && n_store == n && n_load <= n / 2 + 1 ? PACK_IRFFT
+                                                                                                          : PACK_NONE;
+  const auto conv_length = [](int64_t len) { return is_pow2(len) ? len : int64_t(1) << log2_of(2 * len - 1); };
   FftArgs a{};
   a.in = in;
   a.out = out;
-  a.n = (int)n;
   a.n_load = n_load;
   a.load_mode = load_mode;
   a.herm_s = (int)n;
   a.n_store = (int)n_store;
   a.sign = sign;
+  const bool have_tables = !ctx->capture || (tables_present(ctx, n / 2, conv_length(n / 2), sign) &&
+                                             ctx->device_tables.count(table_key(T_REAL, n, -1)));
+  if (pack != PACK_NONE && conv_length(n / 2) <= FFT_LDS_MAX && have_tables) {
+    a.pack = pack;
+    // A length counts as used, for every transform that a graph may record later, once any of
+    // its transforms has run: the tables of the line itself are made here too.
+    if (!ctx->capture)
+      if (int rc = line_tables(ctx, n, conv_length(n), sign)) return rc;
+    if (int rc = twiddles(ctx, T_REAL, (int)n, &a.real_tw)) return rc;
+    n /= 2;
+    a.n_store = (int)n;
+    const Lines &real = pack == PACK_RFFT ? in : out;
+    const int pair = 2 * kind_size(real.kind);
+    a.pair_aligned = real.estride == 1 && (uintptr_t)real.base % pair == 0;
+    for (int d = 0; d < real.nd; d++) a.pair_aligned &= real.strides[d] % 2 == 0;
+  }
+  a.n = (int)n;
+  const bool blue = !is_pow2(n);
+  const int64_t M = conv_length(n);
+  if (M > (int64_t(1) << 26)) return nxh_fail(NXH_FAILURE, "fft", "axis too long for a length that is not a power of two (the limit is 2^25 elements)");
   if (blue)
     if (int rc = bluestein_tables(ctx, n, M, sign, &a.chirp, &a.bf)) return rc;
   if (M <= FFT_LDS_MAX) {
     a.lines = lines;
     a.M = (int)M;
     a.logM = log2_of(M);
-    if (int rc = twiddles(ctx, a.M, &a.tw)) return rc;
+    if (int rc = twiddles(ctx, T_TWIDDLE, a.M, &a.tw)) return rc;
     return launch_lines(ctx, a, blue);
   }
   // long transform: chunks of lines through two workspaces

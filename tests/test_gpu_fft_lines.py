@@ -1,0 +1,86 @@
+"""The one-workgroup transforms at the edges of their lane layouts: every power of two that a
+workgroup holds, neighbours that go through the convolution, real lines packed in pairs (aligned,
+odd offsets, strided, flipped) and half spectra that are cut or padded. Against numpy in float64;
+a double-precision transform of length n is off by at most about 4 log2(n) roundings (three
+transforms for a convolution), plus one rounding of a float32 result."""
+
+import numpy as np
+import pytest
+
+from helpers import logical
+from raven_amd import dtype as dt
+
+pytestmark = pytest.mark.gpu
+
+
+def near(got, want, n, single, what):
+    got = logical(got)
+    bound = 3 * 4 * np.log2(2 * n + 2) * 2.0**-53 + (2.0**-24 if single else 0)
+    err = np.linalg.norm(got - want) / max(np.linalg.norm(want), 1e-300)
+    assert got.shape == want.shape and err <= bound, (what, err, bound)
+
+
+POWERS = [1 << k for k in range(15)]
+LENGTHS = sorted({*POWERS, *[n + 1 for n in POWERS], *[n - 1 for n in POWERS[1:]], 6, 10, 100, 1000, 2050, 4098, 8190, 8194})
+
+
+@pytest.mark.parametrize("single", [False, True])
+@pytest.mark.parametrize("n", LENGTHS)
+def test_real_lines(hip, n, single):
+    real, cplx = (dt.float32, dt.complex64) if single else (dt.float64, dt.complex128)
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((5, 2 * n + 3)).astype(real.np_storage)
+    t = hip.reshape(hip.from_host(x, real), x.shape)
+    views = {"rows": (hip.shrink(t, [(0, 5), (0, n)]), x[:, :n]),
+             "odd": (hip.shrink(t, [(0, 5), (1, n + 1)]), x[:, 1:n + 1]),
+             "flipped": (hip.flip(hip.shrink(t, [(0, 5), (0, n)]), (True, True)), x[::-1, n - 1::-1] if n else x)}
+    for name, (v, a) in views.items():
+        near(hip.rfft(v, cplx, [1]), np.fft.rfft(a.astype(np.float64), axis=1), n, single, (name, n))
+    cols = np.ascontiguousarray(x[:, :n].T)
+    tc = hip.reshape(hip.from_host(cols, real), cols.shape)
+    near(hip.rfft(tc, cplx, [0]), np.fft.rfft(cols.astype(np.float64), axis=0), n, single, ("columns", n))
+
+
+@pytest.mark.parametrize("single", [False, True])
+@pytest.mark.parametrize("n", LENGTHS)
+def test_half_spectra(hip, n, single):
+    real, cplx = (dt.float32, dt.complex64) if single else (dt.float64, dt.complex128)
+    rng = np.random.default_rng(n + 1)
+    full = n // 2 + 1
+    for bins in sorted({1, full, max(1, full - 1), full // 2 + 1, full + 2}):
+        z = (rng.standard_normal((3, bins)) + 1j * rng.standard_normal((3, bins))).astype(cplx.np_storage)
+        kept = np.zeros((3, full), np.complex128)
+        m = min(bins, full)
+        kept[:, :m] = z[:, :m]
+        # the imaginary parts of bin 0 and of bin n / 2 do not reach a real part
+        want = np.fft.irfft(kept, n, axis=1) * n
+        for axis, a in ((1, z), (0, np.ascontiguousarray(z.T))):
+            t = hip.reshape(hip.from_host(a, cplx), a.shape)
+            got = hip.irfft(t, real, [axis], [n])
+            near(got, want if axis else want.T, n, single, (n, bins, axis))
+
+
+@pytest.mark.parametrize("n", [2, 8, 60, 2048, 8191, 16384])
+def test_lengths_count_as_used_for_a_later_recording(hip, n):
+    """rfft runs once; fft of the same length may then be recorded, and the other way round."""
+    rng = np.random.default_rng(n)
+    for first, second in ((0, 1), (1, 0)):
+        x = rng.standard_normal((2, n))
+        tr = hip.reshape(hip.from_host(x, dt.float64), x.shape)
+        tz = hip.reshape(hip.from_host(x.astype(np.complex128), dt.complex128), x.shape)
+        ops = [lambda: hip.rfft(tr, dt.complex128, [1]), lambda: hip.fft(tz, [1])]
+        want = [np.fft.rfft(x, axis=1), np.fft.fft(x, axis=1)]
+        ops[first]()
+        if n > 8192:
+            ops[second]()  # a transform that needs a workspace has run once before it is recorded
+        hip.synchronize()
+        hip.capture_begin()
+        try:
+            out = ops[second]()
+        finally:
+            graph = hip.capture_end()
+        for _ in range(3):
+            graph.launch()
+            hip.synchronize()
+            near(out, want[second], n, False, (n, first))
+        graph.destroy()
