@@ -27,8 +27,20 @@ import numpy as np
 
 from . import _ffi
 from . import dtype as dt
-from ._ffi import BINARY_OPS, COMPARE_OPS, REDUCE_OPS, UNARY_OPS, NxhTensor, make_tensor
-from .view import View, numel
+from ._ffi import BINARY_OPS, COMPARE_OPS, REDUCE_OPS, UNARY_OPS, NxhTensor, stamp, view_image
+from .view import _CONTIGUOUS, View, numel
+
+
+_UNARY, _BINARY, _COMPARE, _REDUCE = ({name: i for i, name in enumerate(ops)}
+                                      for ops in (UNARY_OPS, BINARY_OPS, COMPARE_OPS, REDUCE_OPS))
+
+
+def _op(table: dict, name: str) -> int:
+    """An operation's number; an unknown name is a ``ValueError``."""
+    i = table.get(name)
+    if i is None:
+        raise ValueError(f"{name!r} is not in list")
+    return i
 
 
 class DeviceBuffer:
@@ -40,7 +52,9 @@ class DeviceBuffer:
 
     def __init__(self, ctx: "Backend", nbytes: int):
         p = C.c_void_p()
-        ctx._check(ctx._lib.nxh_alloc(ctx._h, nbytes, C.byref(p)))
+        rc = ctx._lib.nxh_alloc(ctx._h, nbytes, C.byref(p))
+        if rc:
+            ctx._check(rc)
         self.ctx = ctx
         self.ptr = p.value
         self.nbytes = nbytes
@@ -55,17 +69,15 @@ class DeviceBuffer:
 class Tensor:
     """The backend's tensor handle (nx_backend.ml:36-43)."""
 
-    __slots__ = ("buffer", "view", "dtype", "context")
+    __slots__ = ("buffer", "view", "shape", "dtype", "context", "_d")
 
     def __init__(self, buffer: DeviceBuffer, view: View, dtype: dt.DType, context: "Backend"):
         self.buffer = buffer
         self.view = view
+        self.shape = view.shape
         self.dtype = dtype
         self.context = context
-
-    @property
-    def shape(self):
-        return self.view.shape
+        self._d = None
 
     @property
     def strides(self):
@@ -76,8 +88,16 @@ class Tensor:
         return self.view.offset
 
     def _desc(self):
-        v = self.view
-        return make_tensor(self.buffer.ptr, self.dtype.tag, v.shape, v.strides, v.offset)
+        """The C descriptor, made once: handle, view and storage do not change. The library reads
+        it during a call and keeps no pointer to it."""
+        d = self._d
+        if d is None:
+            v = self.view
+            image = v.image
+            if image is None:
+                image = v.image = view_image(v.shape, v.strides, v.offset)
+            d = self._d = stamp(self.buffer.ptr, self.dtype.tag, image)
+        return d
 
     def __repr__(self):  # pragma: no cover
         return f"Tensor({self.dtype.name}, shape={self.shape}, strides={self.strides}, offset={self.offset})"
@@ -216,18 +236,22 @@ class Backend:
     # ── creation (backend_intf.ml:120-145) ──────────────────────────────────
     def buffer(self, dtype: dt.DType, shape: Sequence[int]) -> Tensor:
         """Uninitialised C-contiguous tensor."""
-        shape = tuple(int(s) for s in shape)
-        buf = DeviceBuffer(self, dtype.nbytes(numel(shape)))
-        return Tensor(buf, View.create(shape), dtype, self)
+        view = _CONTIGUOUS.get(shape) if type(shape) is tuple else None
+        if view is None:
+            view = View.create(shape)
+        return Tensor(DeviceBuffer(self, dtype.nbytes(numel(view.shape))), view, dtype, self)
 
     def full(self, dtype: dt.DType, shape: Sequence[int], value) -> Tensor:
         """Every element is ``value`` (a Python number, or one already-encoded
         storage element as a numpy array)."""
         out = self.buffer(dtype, shape)
         enc = value if isinstance(value, np.ndarray) else encode_scalar(dtype, value)
-        enc = np.ascontiguousarray(enc.reshape(1))
-        d = out._desc()
-        self._check(self._lib.nxh_fill(self._h, C.byref(d), enc.ctypes.data))
+        if enc.size != 1:
+            raise ValueError("full: the value is one element")
+        # (the bytes object is the element's storage during the call)
+        rc = self._lib.nxh_fill(self._h, out._desc(), enc.tobytes())
+        if rc:
+            self._check(rc)
         return out
 
     def from_host(self, array: np.ndarray, dtype: dt.DType) -> Tensor:
@@ -276,38 +300,50 @@ class Backend:
     def unary(self, op: str, x: Tensor) -> Tensor:
         out = self.buffer(x.dtype, x.shape)
         o, a = out._desc(), x._desc()
-        self._check(self._lib.nxh_unary(self._h, UNARY_OPS.index(op), C.byref(o), C.byref(a)))
+        rc = self._lib.nxh_unary(self._h, _op(_UNARY, op), o, a)
+        if rc:
+            self._check(rc)
         return out
 
     def binary(self, op: str, x: Tensor, y: Tensor) -> Tensor:
         out = self.buffer(x.dtype, x.shape)
         o, a, b = out._desc(), x._desc(), y._desc()
-        self._check(self._lib.nxh_binary(self._h, BINARY_OPS.index(op), C.byref(o), C.byref(a), C.byref(b)))
+        rc = self._lib.nxh_binary(self._h, _op(_BINARY, op), o, a, b)
+        if rc:
+            self._check(rc)
         return out
 
     def compare(self, op: str, x: Tensor, y: Tensor) -> Tensor:
         out = self.buffer(dt.bool_, x.shape)
         o, a, b = out._desc(), x._desc(), y._desc()
-        self._check(self._lib.nxh_compare(self._h, COMPARE_OPS.index(op), C.byref(o), C.byref(a), C.byref(b)))
+        rc = self._lib.nxh_compare(self._h, _op(_COMPARE, op), o, a, b)
+        if rc:
+            self._check(rc)
         return out
 
     def where(self, cond: Tensor, if_true: Tensor, if_false: Tensor) -> Tensor:
         out = self.buffer(if_true.dtype, if_true.shape)
         o, c, a, b = out._desc(), cond._desc(), if_true._desc(), if_false._desc()
-        self._check(self._lib.nxh_where(self._h, C.byref(o), C.byref(c), C.byref(a), C.byref(b)))
+        rc = self._lib.nxh_where(self._h, o, c, a, b)
+        if rc:
+            self._check(rc)
         return out
 
     def cast(self, x: Tensor, dtype: dt.DType) -> Tensor:
         out = self.buffer(dtype, x.shape)
         o, a = out._desc(), x._desc()
-        self._check(self._lib.nxh_cast(self._h, C.byref(o), C.byref(a)))
+        rc = self._lib.nxh_cast(self._h, o, a)
+        if rc:
+            self._check(rc)
         return out
 
     # ── move family (nx_backend.ml:349-357, 399-402) ────────────────────────
     def copy(self, x: Tensor) -> Tensor:
         out = self.buffer(x.dtype, x.shape)
         o, a = out._desc(), x._desc()
-        self._check(self._lib.nxh_copy(self._h, C.byref(o), C.byref(a)))
+        rc = self._lib.nxh_copy(self._h, o, a)
+        if rc:
+            self._check(rc)
         return out
 
     def contiguous(self, x: Tensor) -> Tensor:
@@ -320,7 +356,9 @@ class Backend:
         """Writes ``src`` through ``dst``'s strides (visible through every view
         sharing dst's buffer)."""
         o, a = dst._desc(), src._desc()
-        self._check(self._lib.nxh_copy(self._h, C.byref(o), C.byref(a)))
+        rc = self._lib.nxh_copy(self._h, o, a)
+        if rc:
+            self._check(rc)
 
     def gather(self, data: Tensor, indices: Tensor, axis: int) -> Tensor:
         out = self.buffer(data.dtype, indices.shape)
@@ -367,7 +405,7 @@ class Backend:
     def associative_scan(self, axis: int, op: str, x: Tensor) -> Tensor:
         out = self.buffer(x.dtype, x.shape)
         o, a = out._desc(), x._desc()
-        self._check(self._lib.nxh_scan(self._h, REDUCE_OPS.index(op), C.byref(o), C.byref(a), axis))
+        self._check(self._lib.nxh_scan(self._h, _op(_REDUCE, op), C.byref(o), C.byref(a), axis))
         return out
 
     def threefry(self, key: Tensor, counter: Tensor) -> Tensor:
@@ -641,7 +679,9 @@ class Backend:
         out = self.buffer(x.dtype, oshape)
         arr = (C.c_int32 * max(len(axes), 1))(*axes)
         o, a = out._desc(), x._desc()
-        self._check(self._lib.nxh_reduce(self._h, REDUCE_OPS.index(op), C.byref(o), C.byref(a), arr, len(axes)))
+        rc = self._lib.nxh_reduce(self._h, _op(_REDUCE, op), o, a, arr, len(axes))
+        if rc:
+            self._check(rc)
         return out
 
     def reduce_noalloc(self, op: str, axes: Sequence[int], x: Tensor, out: Tensor) -> Tensor:
@@ -651,7 +691,7 @@ class Backend:
         axes = sorted(int(a) for a in axes)
         arr = (C.c_int32 * max(len(axes), 1))(*axes)
         o, a = out._desc(), x._desc()
-        self._check(self._lib.nxh_reduce_noalloc(self._h, REDUCE_OPS.index(op), C.byref(o), C.byref(a), arr, len(axes)))
+        self._check(self._lib.nxh_reduce_noalloc(self._h, _op(_REDUCE, op), C.byref(o), C.byref(a), arr, len(axes)))
         return out
 
     def _argreduce(self, is_min: bool, x: Tensor, axis: int, keepdims: bool) -> Tensor:
@@ -683,7 +723,9 @@ class Backend:
             batch.append(max(xs[ai] if ai >= 0 else 1, ys[bi] if bi >= 0 else 1))
         out = self._matmul_result(x.dtype, batch + [xs[-2], ys[-1]])
         o, a, b = out._desc(), x._desc(), y._desc()
-        self._check(self._lib.nxh_matmul(self._h, C.byref(o), C.byref(a), C.byref(b)))
+        rc = self._lib.nxh_matmul(self._h, o, a, b)
+        if rc:
+            self._check(rc)
         return out
 
     def _matmul_result(self, dtype: dt.DType, shape) -> Tensor:

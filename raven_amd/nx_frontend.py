@@ -18,16 +18,29 @@ from . import dtype as dt
 from .nx_backend import encode_scalar
 
 
+_BROADCAST: dict = {}  # (shape, shape) -> what they broadcast to
+
+
 def _broadcast_shapes(a: Sequence[int], b: Sequence[int]) -> tuple:
-    if tuple(a) == tuple(b):
-        return tuple(a)
+    a, b = tuple(a), tuple(b)
+    if a == b:
+        return a
+    s = _BROADCAST.get((a, b))
+    if s is None:
+        s = _broadcast_unequal(a, b)
+        if len(_BROADCAST) < 4096:
+            _BROADCAST[a, b] = s
+    return s
+
+
+def _broadcast_unequal(a: tuple, b: tuple) -> tuple:
     n = max(len(a), len(b))
     out = []
     for i in range(n):
         x = a[i - (n - len(a))] if i >= n - len(a) else 1
         y = b[i - (n - len(b))] if i >= n - len(b) else 1
         if x != y and x != 1 and y != 1:
-            raise ValueError(f"broadcast: cannot broadcast {tuple(a)} with {tuple(b)}")
+            raise ValueError(f"broadcast: cannot broadcast {a} with {b}")
         out.append(max(x, y) if min(x, y) != 0 else 0)
     return tuple(out)
 

@@ -8,6 +8,7 @@ counterpart of OCaml's ``Invalid_argument``.
 
 from __future__ import annotations
 
+import math
 from typing import Sequence, Tuple
 
 
@@ -22,10 +23,7 @@ def c_contiguous_strides(shape: Sequence[int]) -> Tuple[int, ...]:
 
 
 def numel(shape: Sequence[int]) -> int:
-    n = 1
-    for s in shape:
-        n *= s
-    return n
+    return math.prod(shape)
 
 
 _CONTIGUOUS: dict = {}  # shape -> its C-contiguous, offset-0 view (views are immutable)
@@ -34,12 +32,13 @@ _CONTIGUOUS: dict = {}  # shape -> its C-contiguous, offset-0 view (views are im
 class View:
     """Immutable by convention: every operation returns a new view."""
 
-    __slots__ = ("shape", "strides", "offset")
+    __slots__ = ("shape", "strides", "offset", "image")
 
     def __init__(self, shape: Tuple[int, ...], strides: Tuple[int, ...], offset: int = 0):
         self.shape = shape
         self.strides = strides
         self.offset = offset
+        self.image = None  # the C descriptor's bytes, made by the first call that needs them
 
     def __eq__(self, other):
         return (isinstance(other, View) and self.shape == other.shape and self.strides == other.strides
@@ -54,7 +53,7 @@ class View:
     # -- construction (view.ml:43-78) -------------------------------------
     @staticmethod
     def create(shape, strides=None, offset=0) -> "View":
-        shape = tuple([int(s) for s in shape])
+        shape = tuple(map(int, shape))
         if strides is None:
             if offset == 0 or 0 in shape:
                 v = _CONTIGUOUS.get(shape)
@@ -65,7 +64,7 @@ class View:
                 return v
             strides = c_contiguous_strides(shape)
         else:
-            strides = tuple([int(s) for s in strides])
+            strides = tuple(map(int, strides))
             if len(strides) != len(shape):
                 raise ValueError(
                     f"create: strides length {len(strides)} != shape length {len(shape)}")
@@ -94,40 +93,37 @@ class View:
 
     # -- movement (view.ml:82-322) ----------------------------------------
     def expand(self, new_shape) -> "View":
-        new_shape = tuple(int(s) for s in new_shape)
-        if self.ndim == 0:
-            return View(new_shape, (0,) * len(new_shape), self.offset)
-        if len(new_shape) != self.ndim:
-            raise ValueError(f"expand: rank mismatch: {len(new_shape)} vs {self.ndim}")
-        if any(s == 0 for s in self.shape):
+        new_shape = tuple(map(int, new_shape))
+        shape, n = self.shape, len(new_shape)
+        if not shape:
+            return View(new_shape, (0,) * n, self.offset)
+        if n != len(shape):
+            raise ValueError(f"expand: rank mismatch: {n} vs {len(shape)}")
+        if 0 in shape:
             return View.create(new_shape)
-        strides = []
-        for i, ns in enumerate(new_shape):
-            s = self.shape[i]
-            if s == ns:
-                strides.append(self.strides[i])
-            elif s == 1:
-                strides.append(0)
-            else:
-                raise ValueError(
-                    f"expand: dimension {i} (size {s}) cannot expand to size {ns}, "
-                    "only singletons expand")
-        return View.create(new_shape, strides, self.offset)
+        strides = list(self.strides)
+        for i in range(n):
+            if shape[i] != new_shape[i]:
+                if shape[i] != 1:
+                    raise ValueError(
+                        f"expand: dimension {i} (size {shape[i]}) cannot expand to size {new_shape[i]}, "
+                        "only singletons expand")
+                strides[i] = 0
+        return View(new_shape, tuple(strides), 0 if 0 in new_shape else self.offset)
 
     def permute(self, axes) -> "View":
-        axes = tuple(int(a) for a in axes)
-        n = self.ndim
+        axes = tuple(map(int, axes))
+        shape, strides = self.shape, self.strides
+        n = len(shape)
         if len(axes) != n:
             raise ValueError(f"permute: axes length {len(axes)} != ndim {n}")
-        seen = [False] * n
-        for ax in axes:
+        for i, ax in enumerate(axes):
             if ax < 0 or ax >= n:
                 raise ValueError(f"permute: axis {ax} out of bounds for {n}D tensor")
-            if seen[ax]:
+            if ax in axes[:i]:
                 raise ValueError(f"permute: duplicate axis {ax}")
-            seen[ax] = True
-        return View.create([self.shape[a] for a in axes],
-                           [self.strides[a] for a in axes], self.offset)
+        return View(tuple([shape[a] for a in axes]), tuple([strides[a] for a in axes]),
+                    0 if 0 in shape else self.offset)
 
     def shrink(self, bounds) -> "View":
         bounds = [(int(b), int(e)) for b, e in bounds]
@@ -154,7 +150,7 @@ class View:
         return View.create(self.shape, strides, off)
 
     def reshape(self, new_shape) -> "View":
-        new_shape = tuple(int(s) for s in new_shape)
+        new_shape = tuple(map(int, new_shape))
         if new_shape == self.shape:
             return self
         old_n, new_n = numel(self.shape), numel(new_shape)
@@ -162,7 +158,7 @@ class View:
             raise ValueError(f"reshape: cannot reshape {list(self.shape)} to {list(new_shape)}")
         if 0 in self.shape or 0 in new_shape:
             return View.create(new_shape, offset=0)
-        if self.strides == c_contiguous_strides(self.shape) or self.is_c_contiguous():
+        if _CONTIGUOUS.get(self.shape) is self or self.is_c_contiguous():
             return View.create(new_shape, offset=self.offset)
         if len(new_shape) == 0:
             return View.create(new_shape, offset=self.offset)
