@@ -1259,7 +1259,6 @@ static int run_trsm(nxh_context *ctx, const char *op, int64_t batch, int n, int 
   std::lock_guard<std::mutex> g(ctx->mu);
   for (int64_t b0 = 0; b0 < batch; b0 += LA_GRID_BATCH) {
     const unsigned nbat = (unsigned)std::min(LA_GRID_BATCH, batch - b0), groups = (unsigned)((nrhs + 15) / 16);
-    if (groups > 65535u && n > TRSM_PASS<T>) return nxh_fail(NXH_FAILURE, op, "too many elements for one launch");
     for (int r0 = 0; r0 < n; r0 += TRSM_PASS<T>) {
       TrsmArgs<T> a{};
       a.m = mp + b0 * m.bs + r0 * (ts + us);
@@ -1277,7 +1276,7 @@ static int run_trsm(nxh_context *ctx, const char *op, int64_t batch, int n, int 
       hipLaunchKernelGGL(kern, dim3(groups, nbat), dim3(64 * TRSM_WAVES), (size_t)nb * 256 * sizeof(T), ctx->stream, a);
       const int rest = n - r0 - a.rows;
       if (rest > 0)
-        hipLaunchKernelGGL((trsm_rest_kernel<T, TS>), dim3((unsigned)((rest + 63) / 64), groups, nbat), dim3(256), 0, ctx->stream, a,
+        hipLaunchKernelGGL((trsm_rest_kernel<T, TS>), dim3(groups, (unsigned)((rest + 63) / 64), nbat), dim3(256), 0, ctx->stream, a,
                            LaMat{(TS *)a.x.p + a.rows * a.x.rs, a.x.rs, a.x.cs, a.x.bs}, rest);
     }
   }

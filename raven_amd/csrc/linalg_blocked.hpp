@@ -725,12 +725,13 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
 }
 
 // Rows after a pass: X[t] -= sum_u M(t, u) X[u] over the pass's rows, for the next pass to solve
-// (only systems longer than one pass holds come here). A wave per 16 x 16 tile.
+// (only systems longer than one pass holds come here). A wave per 16 x 16 tile; right-hand sides
+// in the grid's x extent, which has room for any number of them.
 template <class T, class TS>
 __global__ __launch_bounds__(256) void trsm_rest_kernel(TrsmArgs<T> a, LaMat rest, int rest_rows) {
   using S = Sc<T>;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
-  const int t0 = (blockIdx.x * 4 + wave) * 16, c = blockIdx.y * 16 + r16;
+  const int t0 = (blockIdx.y * 4 + wave) * 16, c = blockIdx.x * 16 + r16;
   if (t0 >= rest_rows) return;
   const TS *m = (const TS *)a.m + blockIdx.z * a.mbs;
   const TS *x = (const TS *)a.x.p + blockIdx.z * a.x.bs;

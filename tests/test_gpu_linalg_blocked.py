@@ -81,6 +81,17 @@ def test_triangular_solve_at_block_edges(hip, name, n, nrhs):
                 assert np.all(residual <= bound), (upper, transpose, unit, float(np.max(residual / bound)))
 
 
+def test_triangular_solve_of_many_sides_in_two_passes(hip):
+    """More groups of sixteen right-hand sides than a grid's y extent holds, and a second pass."""
+    rng, n, nrhs = np.random.default_rng(7), 1025, 16 * 65536 + 3
+    a = put(hip, (rng.standard_normal((n, n)) / np.sqrt(n) + 2 * np.eye(n)).astype(np.float32), dt.float32)
+    b = put(hip, rng.standard_normal((n, 1)).astype(np.float32), dt.float32)
+    want = logical(hip.triangular_solve(a, b, False, False, False))
+    x = hip.triangular_solve(a, hip.expand(b, (n, nrhs)), False, False, False)
+    for low, high in ((0, 1), (nrhs - 1, nrhs)):  # a side's arithmetic does not depend on its place
+        assert np.array_equal(logical(hip.copy(hip.shrink(x, [(0, n), (low, high)]))), want)
+
+
 def test_triangular_solve_without_ordinary_inverses(hip):
     """Rows scaled far outside the range where a product with the inverse stands for the quotient."""
     rng = np.random.default_rng(5)
