@@ -32,6 +32,12 @@ __device__ __forceinline__ void to_storage(double v, float *p) { *p = (float)v; 
 __device__ __forceinline__ void to_storage(double v, double *p) { *p = v; }
 __device__ __forceinline__ void to_storage(c64 v, c64 *p) { *p = v; }
 
+// What the lanes of a wave wrote to LDS before it is there for all of them after it.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // sqrt(d) and 1 / sqrt(d) of a positive d, each to the last bit or next to it: one hardware
 // estimate and Newton steps on d scaled into [1/4, 1). The chain of the factorisation runs
 // through this once per column; the library's square root and division are four times as long.
@@ -91,20 +97,28 @@ __device__ __forceinline__ double inverse_of(double d) {
 // from: nothing moves between lanes. diag_inv[b] is the inverse of the b-th 4 x 4 triangle on
 // the diagonal as a first operand (lane (q, r): element (r - 4 b, q), 0 in other rows), tri[b] columns
 // 4 b .. 4 b + 3 (lane (q, r): element (r, 4 b + q), 0 above the diagonal). The product with the
-// inverse is followed by one step on its remainder, which the update leaves in the same register,
-// so the result is that of a substitution. 16 instructions of 64 cycles; row by row, with a
-// right-hand side a lane, the chain through LDS took 4700 cycles.
-__device__ __forceinline__ void solve16(LaTile<double> &acc, const double (&diag_inv)[4], const double (&tri)[4]) {
+// inverse is followed by one step on its remainder, which the update leaves in the same register.
+// The zeros of the operands meet every row of a group of four: a row that is not finite would make
+// the rows before it no numbers too. So where a result is not finite nothing is changed and the
+// answer is false: the caller substitutes row by row. 15 instructions of 64 cycles; row by row, with
+// a right-hand side a lane, the chain through LDS took 4700 cycles.
+__device__ __forceinline__ bool solve16(LaTile<double> &acc, const double (&diag_inv)[4], const double (&tri)[4]) {
   la_f64x4 c = {acc.v[0], acc.v[1], acc.v[2], acc.v[3]};
   const la_f64x4 zero = {0.0, 0.0, 0.0, 0.0};
+  LaTile<double> sol;
+  bool finite = true;
 #pragma unroll
   for (int b = 0; b < 4; b++) {
     const double x = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], c[b], zero, 0, 0, 0)[b];
     c = __builtin_amdgcn_mfma_f64_16x16x4f64(-tri[b], x, c, 0, 0, 0);
     const double dx = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], c[b], zero, 0, 0, 0)[b];
-    acc.v[b] = x + dx;
+    sol.v[b] = x + dx;
+    finite = finite && fabs(sol.v[b]) < __builtin_inf();
     if (b < 3) c = __builtin_amdgcn_mfma_f64_16x16x4f64(-tri[b], dx, c, 0, 0, 0);
   }
+  if (!__all(finite)) return false;
+  acc = sol;
+  return true;
 }
 
 // Cholesky of a 16 x 16 tile in that layout (the tile is Hermitian: rows and columns may change
@@ -320,9 +334,20 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
       double di[4], tr[4];
 #pragma unroll
       for (int v = 0; v < 4; v++) di[v] = op_inv[(jb * 4 + v) * 64 + lane], tr[v] = op_tri[(jb * 4 + v) * 64 + lane];
-      solve16(t, di, tr);
+      const bool solved = solve16(t, di, tr);
 #pragma unroll
       for (int v = 0; v < 4; v++) rows[r16 * LD + jb * 16 + 4 * v + q] = t.v[v];
+      if (solved) return;
+      // column by column, four lanes a row
+      double *row = rows + r16 * LD + jb * 16;
+      const double *tri = D + jb * 16 * (LD + 1);
+#pragma unroll 1
+      for (int c = 0; c < 16; c++) {
+        wave_sync();
+        const double x = row[c] * op_inv[(jb * 4 + (c >> 2)) * 64 + (c & 3) * 16 + c];
+        if (q == 0) row[c] = x;
+        for (int k = c + 1 + q; k < 16; k += 4) row[k] = fma(-x, tri[k * LD + c], row[k]);
+      }
     };
     auto solve_own = [&](int jb) {
       const int tr = wave == 1 ? 3 : wave - 5;  // (not wave 4: it shares a SIMD, and its matrix unit, with wave 0)
@@ -482,8 +507,8 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
 // triangle (solve16), while other waves take the step before from the rows further down (a
 // wave per 16 x 16 tile) and one inverts the 4 x 4 triangles of the next step. What is read
 // of the matrix is requested a step or two ahead: it depends on nothing. One barrier a step, no launch.
-// Where an inverse is no ordinary number, and for complex matrices, the substitution goes row by
-// row, a right-hand side a lane.
+// Where an inverse is no ordinary number, where a right-hand side or a solution is not finite, and for
+// complex matrices, the substitution goes row by row, a right-hand side a lane.
 // Wave 0 is the chain, wave 4 (of its SIMD) reads and inverts triangles, which takes no matrix
 // instructions from it, the other six bring up to TRSM_TILES tiles each up to date per step: 64 in a pass.
 constexpr int TRSM_WAVES = 8, TRSM_LOADER = 4, TRSM_UPDATERS = 6, TRSM_TILES = 11;
@@ -638,9 +663,10 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
           double di[4];
 #pragma unroll
           for (int v = 0; v < 4; v++) di[v] = diag_inv[k & 1][v][lane];
-          solve16(acc, di, tr);
-          store_rows(k, acc);
-          return;
+          if (solve16(acc, di, tr)) {
+            store_rows(k, acc);
+            return;
+          }
         }
       }
       store_rows(k, acc);

@@ -106,6 +106,41 @@ def test_triangular_solve_without_ordinary_inverses(hip):
     assert np.all(np.isfinite(x)) and np.max(np.abs(x - plain)) <= 1e-9 * np.max(np.abs(plain))
 
 
+def substituted(m, b, lower):
+    """Plain substitution in float64, a row at a time."""
+    x = b.astype(np.float64)
+    n = len(m)
+    with np.errstate(all="ignore"):
+        for i in range(n) if lower else range(n - 1, -1, -1):
+            x[i] = x[i] / m[i, i]
+            rest = slice(i + 1, n) if lower else slice(0, i)
+            x[rest] -= m[rest, i:i + 1] * x[i]
+    return x
+
+
+@pytest.mark.parametrize("name", ["float32", "float64"])
+@pytest.mark.parametrize("upper,transpose", [(False, False), (False, True), (True, False), (True, True)])
+def test_triangular_solve_of_sides_that_are_not_finite(hip, name, upper, transpose):
+    """An infinity or a NaN at every row of a right-hand side: the rows solved before it do not see
+    it, it and the rows after it are what substitution makes of it (n eps of the magnitudes summed)."""
+    d, rng, n = dt.BY_NAME[name], np.random.default_rng(11), 37
+    a = (rng.standard_normal((n, n)) / np.sqrt(n) + 2 * np.eye(n)).astype(d.np_storage)
+    b = np.tile(rng.standard_normal((n, 1)).astype(d.np_storage), (1, 3 * n))
+    for i in range(n):
+        b[i, 3 * i:3 * i + 3] = np.inf, -np.inf, np.nan
+    m = (np.triu(a) if upper else np.tril(a)).astype(np.float64)
+    m = m.T if transpose else m
+    want = substituted(m, b, upper == transpose)
+    got = logical(hip.triangular_solve(put(hip, a, d), put(hip, b, d), upper, transpose, False)).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got) * np.sign(got), np.isinf(want) * np.sign(want), equal_nan=True)
+    finite = np.isfinite(want)
+    w = np.where(finite, want, 0)
+    # |x - x'| <= |M^-1| (bound of the residual); the rows past an infinity are none of the system's
+    room = np.abs(np.linalg.inv(m)) @ ((8 * n * 2.0 ** -53 + 2 * EPS[name]) * (np.abs(m) @ np.abs(w)))
+    assert np.all(np.abs(got[finite] - want[finite]) <= room[finite])
+
+
 def test_in_place_and_shared_storage(hip):
     """Results over the operands' own storage, as the C ABI allows."""
     import ctypes as C
