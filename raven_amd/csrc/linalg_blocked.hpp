@@ -91,32 +91,38 @@ __device__ __forceinline__ double inverse_of(double d) {
   return fma(fma(-d, r, 1.0), r, r);
 }
 
+// Neither holds where x or dx is not finite.
+__device__ __forceinline__ bool small_step(double x, double dx) { return dx == 0.0 || fabs(dx) < 0x1p-28 * fabs(x); }
+
 // Substitution through a 16 x 16 triangle, four rows at a time on the matrix instruction, for
 // sixteen right-hand sides: register v of lane (q, c) = 16 q + c holds row 4 v + q of side c, which is
 // both where the instruction leaves a result and, for four rows, where it takes its second operand
 // from: nothing moves between lanes. diag_inv[b] is the inverse of the b-th 4 x 4 triangle on
 // the diagonal as a first operand (lane (q, r): element (r - 4 b, q), 0 in other rows), tri[b] columns
 // 4 b .. 4 b + 3 (lane (q, r): element (r, 4 b + q), 0 above the diagonal). The product with the
-// inverse is followed by one step on its remainder, which the update leaves in the same register.
-// The zeros of the operands meet every row of a group of four: a row that is not finite would make
-// the rows before it no numbers too. So where a result is not finite nothing is changed and the
-// answer is false: the caller substitutes row by row. 15 instructions of 64 cycles; row by row, with
+// inverse is followed by one step on its remainder, which the instruction leaves in the same register.
+// That stands for a substitution where the step is small: it divides the error of the product by as
+// much as it is smaller than it, so below 2^-28 of every value what is left is less than a rounding.
+// Where it is larger (a diagonal small against what is below it: the inverse grows, and the error of
+// the product with it), or no number (the zeros of the operands meet every row of a group of four: a
+// row that is not finite would make the rows before it NaN), nothing is changed and the answer is
+// false: the caller substitutes row by row. 15 instructions of 64 cycles; row by row, with
 // a right-hand side a lane, the chain through LDS took 4700 cycles.
 __device__ __forceinline__ bool solve16(LaTile<double> &acc, const double (&diag_inv)[4], const double (&tri)[4]) {
   la_f64x4 c = {acc.v[0], acc.v[1], acc.v[2], acc.v[3]};
   const la_f64x4 zero = {0.0, 0.0, 0.0, 0.0};
   LaTile<double> sol;
-  bool finite = true;
+  bool small = true;
 #pragma unroll
   for (int b = 0; b < 4; b++) {
     const double x = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], c[b], zero, 0, 0, 0)[b];
-    c = __builtin_amdgcn_mfma_f64_16x16x4f64(-tri[b], x, c, 0, 0, 0);
-    const double dx = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], c[b], zero, 0, 0, 0)[b];
+    const double rest = __builtin_amdgcn_mfma_f64_16x16x4f64(-tri[b], x, c, 0, 0, 0)[b];
+    const double dx = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], rest, zero, 0, 0, 0)[b];
     sol.v[b] = x + dx;
-    finite = finite && fabs(sol.v[b]) < __builtin_inf();
-    if (b < 3) c = __builtin_amdgcn_mfma_f64_16x16x4f64(-tri[b], dx, c, 0, 0, 0);
+    small = small && small_step(x, dx);
+    if (b < 3) c -= __builtin_amdgcn_mfma_f64_16x16x4f64(tri[b], sol.v[b], zero, 0, 0, 0);
   }
-  if (!__all(finite)) return false;
+  if (!__all(small)) return false;
   acc = sol;
   return true;
 }
@@ -507,8 +513,8 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
 // triangle (solve16), while other waves take the step before from the rows further down (a
 // wave per 16 x 16 tile) and one inverts the 4 x 4 triangles of the next step. What is read
 // of the matrix is requested a step or two ahead: it depends on nothing. One barrier a step, no launch.
-// Where an inverse is no ordinary number, where a right-hand side or a solution is not finite, and for
-// complex matrices, the substitution goes row by row, a right-hand side a lane.
+// Where solve16 refuses, and for complex matrices, the substitution goes row by row, a right-hand
+// side a lane.
 // Wave 0 is the chain, wave 4 (of its SIMD) reads and inverts triangles, which takes no matrix
 // instructions from it, the other six bring up to TRSM_TILES tiles each up to date per step: 64 in a pass.
 constexpr int TRSM_WAVES = 8, TRSM_LOADER = 4, TRSM_UPDATERS = 6, TRSM_TILES = 11;
@@ -535,11 +541,10 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
   extern __shared__ double lds_raw[];
   T *X = (T *)lds_raw;  // rows rounded up to 16, times 16
   // by columns, each from its diagonal on: element r < 16 of column t is coefficient (t + r, t), element
-  // 16 the inverse of the diagonal (reads past a column's end meet the next one: their results are dropped)
+  // 16 (double) the inverse of the diagonal (reads past a column's end meet the next one: their results are dropped)
   constexpr int TRI_LD = 18;
   __shared__ T tri[2][17][TRI_LD];
   __shared__ double diag_inv[2][4][64];  // operands of solve16, zero outside the 4 x 4 triangles
-  __shared__ int multiply[2];            // whether the inverses are ordinary numbers
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
   const int n = a.rows, nb = (n + 15) / 16, col0 = blockIdx.x * 16;
   const TS *m = (const TS *)a.m + blockIdx.y * a.mbs;
@@ -556,7 +561,6 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
     for (int v = 0; v < 4; v++) raw[v] = m[min(k * 16 + 4 * v + q, n - 1) * a.ts + min(k * 16 + r16, n - 1) * a.us];
   };
   auto place_triangle = [&](int k, const TS(&raw)[4]) {
-    bool ordinary = true;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       const int t = 4 * v + q;
@@ -566,10 +570,7 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
       if (r16 <= t) tri[k & 1][r16][t - r16] = val;
       if (diagonal) {
         if (val == S::make(0.0, 0.0)) singular = true;
-        const T di = S::make(1.0, 0.0) / val;
-        tri[k & 1][t][16] = di;
-        const double size = fabs(S::re(di));
-        ordinary = sizeof(T) == 8 && size > 1e-280 && size < 1e280;
+        if constexpr (sizeof(T) == 8) tri[k & 1][t][16] = 1.0 / val;
       }
     }
     if constexpr (sizeof(T) == 8) {
@@ -584,11 +585,8 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
       double v = i == 0 ? e0 : i == 1 ? (j == 0 ? m10 : e1) : i == 2 ? (j == 0 ? m20 : j == 1 ? m21 : e2)
                                                                      : (j == 0 ? m30 : j == 1 ? m31 : j == 2 ? m32 : e3);
       v = j <= i ? v : 0.0;
-      ordinary = ordinary && fabs(v) < 1e280;
       diag_inv[k & 1][bb][j * 16 + 4 * bb + i] = v;
     }
-    const bool all = __all(ordinary);
-    if (lane == 0) multiply[k & 1] = all;
   };
   for (int e = threadIdx.x; e < 512; e += blockDim.x) (&diag_inv[0][0][0])[e] = 0.0;
   __syncthreads();
@@ -659,14 +657,12 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
           tr[v] = r16 < u ? 0.0 : k * 16 + r16 >= n || (a.unit && r16 == u) ? (r16 == u ? 1.0 : 0.0) : (double)co[v];
         }
         if (k + 2 < nb) coefficients(k + 2, k + 2, co);
-        if (multiply[k & 1]) {
-          double di[4];
+        double di[4];
 #pragma unroll
-          for (int v = 0; v < 4; v++) di[v] = diag_inv[k & 1][v][lane];
-          if (solve16(acc, di, tr)) {
-            store_rows(k, acc);
-            return;
-          }
+        for (int v = 0; v < 4; v++) di[v] = diag_inv[k & 1][v][lane];
+        if (solve16(acc, di, tr)) {
+          store_rows(k, acc);
+          return;
         }
       }
       store_rows(k, acc);

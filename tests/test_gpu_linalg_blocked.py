@@ -106,6 +106,27 @@ def test_triangular_solve_without_ordinary_inverses(hip):
     assert np.all(np.isfinite(x)) and np.max(np.abs(x - plain)) <= 1e-9 * np.max(np.abs(plain))
 
 
+@pytest.mark.parametrize("upper,transpose", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("n", [4, 8, 16, 19, 40])
+def test_triangular_solve_with_weak_diagonals(hip, n, upper, transpose):
+    """A 4 x 4 block whose diagonal is 1e-5 .. 1e-14 of what is beside it: its inverse grows with the third
+    power, the backward error of a substitution does not (n + 1 eps, Higham theorem 8.5)."""
+    rng = np.random.default_rng(n)
+    for power in (-2, -5, -6, -7, -8, -10, -14):
+        t = rng.standard_normal((24, n, n)) / np.sqrt(n) + 2 * np.eye(n)
+        for m in t:
+            at = 4 * rng.integers(0, n // 4)
+            block = rng.standard_normal((4, 4))
+            block[range(4), range(4)] *= 10.0 ** power
+            m[at:at + 4, at:at + 4] = block
+        t = np.triu(t) if upper else np.tril(t)
+        m = H(t) if transpose else t
+        b = m @ rng.standard_normal((24, n, 3))
+        x = logical(hip.triangular_solve(put(hip, t, dt.float64), put(hip, b, dt.float64), upper, transpose, False)).astype(np.longdouble)
+        residual = np.abs(m.astype(np.longdouble) @ x - b)
+        assert np.all(residual <= (n + 1) * 2.0 ** -53 * (np.abs(m).astype(np.longdouble) @ np.abs(x))), power
+
+
 def substituted(m, b, lower):
     """Plain substitution in float64, a row at a time."""
     x = b.astype(np.float64)
