@@ -61,34 +61,58 @@ struct LaTile {
   T v[4];
 };
 
-// acc -= A B^H over K terms: A[row * lda + k], B[col * ldb + k] with the tile's first row and
-// column in the pointers.
+// A B^H over K terms: A[row * lda + k], B[col * ldb + k] with the tile's first row and column in the
+// pointers, as sums of four terms that meet pairwise; tile_sub takes it from acc. So there is one
+// rounding at the size of acc per call and not one per term (one chain of fused steps from acc left a
+// Gram matrix of 256 columns with four times the backward error, 0.30 against 0.07 eps).
+template <int K>
+__device__ __forceinline__ la_f64x4 tile_sum(const double *A, int64_t lda, const double *B, int64_t ldb) {
+  if constexpr (K > 4) {
+    const la_f64x4 low = tile_sum<K / 2>(A, lda, B, ldb);
+    return low + tile_sum<K / 2>(A + K / 2, lda, B + K / 2, ldb);
+  } else {
+    const int lane = threadIdx.x & 63, at = lane >> 4;
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(A[(lane & 15) * lda + at], B[(lane & 15) * ldb + at], la_f64x4{0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
+  }
+}
 template <int K>
 __device__ __forceinline__ void tile_sub(LaTile<double> &acc, const double *A, int64_t lda, const double *B, int64_t ldb) {
+  const la_f64x4 sum = tile_sum<K>(A, lda, B, ldb);
+#pragma unroll
+  for (int i = 0; i < 4; i++) acc.v[i] -= sum[i];
+}
+template <int K>
+__device__ __forceinline__ LaTile<c64> tile_sum(const c64 *A, int64_t lda, const c64 *B, int64_t ldb) {  // (with its sign)
   const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
-  la_f64x4 c = {acc.v[0], acc.v[1], acc.v[2], acc.v[3]};
-  const double *pa = A + r * lda + q, *pb = B + r * ldb + q;
+  LaTile<c64> s;
+  if constexpr (K > 4) {
+    s = tile_sum<K / 2>(A, lda, B, ldb);
+    const LaTile<c64> high = tile_sum<K / 2>(A + K / 2, lda, B + K / 2, ldb);
 #pragma unroll
-  for (int k = 0; k < K; k += 4) c = __builtin_amdgcn_mfma_f64_16x16x4f64(-pa[k], pb[k], c, 0, 0, 0);
+    for (int v = 0; v < 4; v++) s.v[v] = s.v[v] + high.v[v];
+  } else {
 #pragma unroll
-  for (int i = 0; i < 4; i++) acc.v[i] = c[i];
+    for (int v = 0; v < 4; v++) s.v[v] = Sc<c64>::make(0.0, 0.0);
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const c64 b = Sc<c64>::conj(B[r * ldb + k]);
+#pragma unroll
+      for (int v = 0; v < 4; v++) s.v[v] = Sc<c64>::sub_mul(s.v[v], A[(4 * v + q) * lda + k], b);
+    }
+  }
+  return s;
 }
 template <int K>
 __device__ __forceinline__ void tile_sub(LaTile<c64> &acc, const c64 *A, int64_t lda, const c64 *B, int64_t ldb) {
-  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
-#pragma unroll 4
-  for (int k = 0; k < K; k++) {
-    const c64 b = Sc<c64>::conj(B[r * ldb + k]);
+  LaTile<c64> sum;
+#pragma unroll 1
+  for (int k = 0; k < K; k += 16) {  // (sixteen terms of code)
+    const LaTile<c64> s = tile_sum<16>(A + k, lda, B + k, ldb);
 #pragma unroll
-    for (int v = 0; v < 4; v++) acc.v[v] = Sc<c64>::sub_mul(acc.v[v], A[(4 * v + q) * lda + k], b);
+    for (int v = 0; v < 4; v++) sum.v[v] = k ? sum.v[v] + s.v[v] : s.v[v];
   }
-}
-
-// 1 / d of an ordinary double, to the last bit or next to it.
-__device__ __forceinline__ double inverse_of(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  r = fma(fma(-d, r, 1.0), r, r);
-  return fma(fma(-d, r, 1.0), r, r);
+#pragma unroll
+  for (int v = 0; v < 4; v++) acc.v[v] = acc.v[v] + sum.v[v];
 }
 
 // Neither holds where x or dx is not finite.
@@ -109,18 +133,19 @@ __device__ __forceinline__ bool small_step(double x, double dx) { return dx == 0
 // false: the caller substitutes row by row. 15 instructions of 64 cycles; row by row, with
 // a right-hand side a lane, the chain through LDS took 4700 cycles.
 __device__ __forceinline__ bool solve16(LaTile<double> &acc, const double (&diag_inv)[4], const double (&tri)[4]) {
-  la_f64x4 c = {acc.v[0], acc.v[1], acc.v[2], acc.v[3]};
   const la_f64x4 zero = {0.0, 0.0, 0.0, 0.0};
+  la_f64x4 taken = zero;  // by the rows before, summed apart from acc: one rounding at its size
   LaTile<double> sol;
   bool small = true;
 #pragma unroll
   for (int b = 0; b < 4; b++) {
-    const double x = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], c[b], zero, 0, 0, 0)[b];
-    const double rest = __builtin_amdgcn_mfma_f64_16x16x4f64(-tri[b], x, c, 0, 0, 0)[b];
+    const double c = b > 0 ? acc.v[b] - taken[b] : acc.v[b];
+    const double x = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], c, zero, 0, 0, 0)[b];
+    const double rest = c - __builtin_amdgcn_mfma_f64_16x16x4f64(tri[b], x, zero, 0, 0, 0)[b];
     const double dx = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], rest, zero, 0, 0, 0)[b];
     sol.v[b] = x + dx;
     small = small && small_step(x, dx);
-    if (b < 3) c -= __builtin_amdgcn_mfma_f64_16x16x4f64(tri[b], sol.v[b], zero, 0, 0, 0);
+    if (b < 3) taken = __builtin_amdgcn_mfma_f64_16x16x4f64(tri[b], sol.v[b], taken, 0, 0, 0);
   }
   if (!__all(small)) return false;
   acc = sol;
@@ -128,41 +153,49 @@ __device__ __forceinline__ bool solve16(LaTile<double> &acc, const double (&diag
 }
 
 // Cholesky of a 16 x 16 tile in that layout (the tile is Hermitian: rows and columns may change
-// places), four columns at a time: every lane factors the 4 x 4 block on the diagonal as L D L^T (the
-// chain is four reciprocals; the roots follow side by side), the matrix instruction does the rest.
-// Leaves the operands of solve16 in diag_inv and tri; tri is the factor itself. `blk`: 64 doubles of LDS.
-__device__ __forceinline__ bool factor16(LaTile<double> acc, double *blk, double (&diag_inv)[4], double (&tri)[4]) {
+// places), four columns at a time: every lane factors the 4 x 4 block on the diagonal, element by
+// element, the matrix instruction does the rest. The tile is acc - before; what its own columns take is
+// summed beside `before`, so that an element of a diagonal block rounds once at its own size.
+// Leaves the operands of solve16 in diag_inv and tri; tri is the factor itself. `blk`: 64 places of LDS.
+__device__ __forceinline__ bool factor16(const LaTile<double> &acc, la_f64x4 before, double2 *blk, double (&diag_inv)[4], double (&tri)[4]) {
   const int lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
-  la_f64x4 t = {acc.v[0], acc.v[1], acc.v[2], acc.v[3]};
   const la_f64x4 zero = {0.0, 0.0, 0.0, 0.0};
+  la_f64x4 taken = zero;
   bool positive = true;
 #pragma unroll
   for (int b = 0; b < 4; b++) {
-    blk[lane] = t[b];
+    const double off = b > 0 ? before[b] + taken[b] : before[b], t = acc.v[b] - off;
+    blk[lane] = make_double2(acc.v[b], off);
     __builtin_amdgcn_wave_barrier();
-    double a[4][4];  // a[j][i]: element (4 b + i, 4 b + j)
+    double a[4][4], sum[4][4];  // a[j][i]: element (4 b + i, 4 b + j); sum: what the columns before take from it
 #pragma unroll
     for (int j = 0; j < 4; j++)
 #pragma unroll
-      for (int i = j; i < 4; i++) a[j][i] = blk[16 * j + 4 * b + i];
+      for (int i = j; i < 4; i++) {
+        const double2 v = blk[16 * j + 4 * b + i];
+        a[j][i] = v.x, sum[j][i] = v.y;
+      }
     __builtin_amdgcn_wave_barrier();
-    double u[4][4], root[4];  // u[j][i]: the unit triangle; root[j]: 1 / sqrt of the pivot
+    double low[4][4], root[4];  // low[j][i]: the factor; root[j]: the inverse of its diagonal
+    double own[4][4];           // what this block's columns take
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      const double r = inverse_of(a[j][j]);
 #pragma unroll
-      for (int i = j + 1; i < 4; i++) u[j][i] = a[j][i] * r;
+      for (int i = j; i < 4; i++) low[j][i] = a[j][i] - (j > 0 ? sum[j][i] + own[j][i] : sum[j][i]);
+      positive = positive && low[j][j] > 0.0;
+      root_and_inverse(low[j][j], &low[j][j], &root[j]);
+#pragma unroll
+      for (int i = j + 1; i < 4; i++) low[j][i] *= root[j];
 #pragma unroll
       for (int k = j + 1; k < 4; k++)
 #pragma unroll
-        for (int i = k; i < 4; i++) a[k][i] = fma(-u[j][i], a[j][k], a[k][i]);
+        for (int i = k; i < 4; i++) own[k][i] = j > 0 ? fma(low[j][i], low[j][k], own[k][i]) : low[j][i] * low[j][k];
     }
+    double u[4][4];  // the unit triangle
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      double l;
-      positive = positive && a[j][j] > 0.0;
-      root_and_inverse(a[j][j], &l, &root[j]);
-    }
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int i = j + 1; i < 4; i++) u[j][i] = low[j][i] * root[j];
     // rows of the inverse of the unit triangle, each times its root
     const double m10 = -u[0][1], m21 = -u[1][2], m32 = -u[2][3];
     const double m20 = fma(-m10, u[1][2], -u[0][2]), m31 = fma(-m21, u[2][3], -u[1][3]);
@@ -174,29 +207,34 @@ __device__ __forceinline__ bool factor16(LaTile<double> acc, double *blk, double
     m = i == 0 ? 1.0 : m;
     m *= i == 0 ? root[0] : i == 1 ? root[1] : i == 2 ? root[2] : root[3];
     diag_inv[b] = i >= q && i < 4 ? m : 0.0;
-    double x = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], t[b], zero, 0, 0, 0)[b];
-    x = c >= 4 * b + q ? x : 0.0;
-    t = __builtin_amdgcn_mfma_f64_16x16x4f64(-x, x, t, 0, 0, 0);
-    double dx = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], t[b], zero, 0, 0, 0)[b];
-    // (inside the 4 x 4 block the remainder is that of a product of two unknowns, a rounding of it: left)
-    dx = c >= 4 * b + 4 ? dx : 0.0;
-    if (b < 3) {
-      t = __builtin_amdgcn_mfma_f64_16x16x4f64(-dx, x, t, 0, 0, 0);
-      t = __builtin_amdgcn_mfma_f64_16x16x4f64(-(x + dx), dx, t, 0, 0, 0);
-    }
-    tri[b] = x + dx;
+    // inside the block the factor itself, elsewhere (rows of the factor below it) the product
+    double in = q == 0 ? low[0][3] : q == 1 ? low[1][3] : q == 2 ? low[2][3] : low[3][3];
+    in = i == 2 ? (q == 0 ? low[0][2] : q == 1 ? low[1][2] : low[2][2]) : in;
+    in = i == 1 ? (q == 0 ? low[0][1] : low[1][1]) : in;
+    in = i == 0 ? low[0][0] : in;
+    const double product = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], t, zero, 0, 0, 0)[b];
+    const bool below = i >= 4;
+    const double x = below ? product : i >= q ? in : 0.0;
+    const double rest = t - __builtin_amdgcn_mfma_f64_16x16x4f64(x, x, zero, 0, 0, 0)[b];
+    const double dx = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], rest, zero, 0, 0, 0)[b];
+    tri[b] = below ? x + dx : x;
+    if (b < 3) taken = __builtin_amdgcn_mfma_f64_16x16x4f64(tri[b], tri[b], taken, 0, 0, 0);
   }
   return positive;
 }
 
 // ── cholesky ────────────────────────────────────────────────────────────────
 // NB x NB tiles, one launch per block column s, a workgroup per tile (i, j) with i >= j >= s.
-// Tile (i, j) first takes what block column s - 1 takes from it. Column s then is
-// finished: every workgroup of that column keeps the diagonal tile too, factors it (the same
+// What block column s - 1 takes from tile (i, j) is first added to what the columns before it took.
+// Column s then is finished: every workgroup of that column keeps the diagonal tile too, factors it (the same
 // instructions on the same values everywhere), and solves its own tile against it, sixteen
 // columns behind. Factoring the diagonal again in each workgroup costs nothing (it would
-// be waited for) and saves a launch per block column. The factor goes to L, the updated rest to
-// A: nothing that a workgroup of the same launch may still read is overwritten.
+// be waited for) and saves a launch per block column. The factor goes to L, the sums to
+// A: nothing that a workgroup of the same launch may still read is overwritten. The sums stay apart from
+// the matrix until its column comes up, so that an element rounds a few times at its own size and not
+// once a column: float64, g g^T + n I, relative error of the factor in eps (2-norm, against long double) for
+// n = 64, 130, 400: 1.52, 2.03, 3.41 with the updates taken from the matrix one by one, 0.55, 0.50, 0.51 so
+// (a column at a time with a wave per element: 1.44, 0.52, 0.52), for 28 us of 200 at n = 512.
 //
 // The chain of a launch is the diagonal tile, sixteen columns at a time: factored by wave 0
 // (factor16), then a wave per sixteen rows below solves against them (solve16), then wave 0
@@ -207,7 +245,7 @@ constexpr int CHOL_THREADS = 512, CHOL_WAVES = CHOL_THREADS / 64;
 template <class T>
 constexpr int CHOL_NB = sizeof(T) == 8 ? 64 : 32;
 constexpr int CHOL_COLUMN = 80;                 // complex: 64 values of one column, and room for reads past them
-constexpr int CHOL_OPERANDS = 64 + 2 * 4 * 256;  // double: factor16's scratch, the operands of solve16 for four blocks of columns
+constexpr int CHOL_OPERANDS = 128 + 3 * 4 * 256;  // double: factor16's scratch, the operands of solve16 for four blocks of columns, diag_sum
 // four tiles of pitch NB + 2 (66 doubles: sixteen rows on different banks), then those
 template <class T>
 constexpr size_t CHOL_LDS = 4 * CHOL_NB<T> * (CHOL_NB<T> + 2) * sizeof(T) +
@@ -215,8 +253,8 @@ constexpr size_t CHOL_LDS = 4 * CHOL_NB<T> * (CHOL_NB<T> + 2) * sizeof(T) +
 
 template <class T>
 struct CholArgs {
-  LaMat x, out;  // storage types: read by the first two launches, written by all
-  T *A, *L;      // n x n per matrix, row-major
+  LaMat x, out;  // storage types
+  T *A, *L;      // n x n per matrix, row-major: what is taken from x, with its sign; the factor
   int n, s, upper;
   int *status;
 };
@@ -230,7 +268,7 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
   T *ls = own + NB * LD, *li = ls + NB * LD;  // block column s - 1 in the rows of tile (s, .) and of tile (i, .)
   T *column = li + NB * LD;
   double *inv = (double *)(column + CHOL_COLUMN);
-  double *blk = (double *)(li + NB * LD), *op_inv = blk + 64, *op_tri = op_inv + 4 * 256;
+  double *blk = (double *)(li + NB * LD), *op_inv = blk + 128, *op_tri = op_inv + 4 * 256, *diag_sum = op_tri + 4 * 256;
   const int n = a.n, s = a.s, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
   const int panels = (n + NB - 1) / NB - s;  // block rows from s down
   int i, j;
@@ -243,12 +281,10 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
   }
   const TS *x = (const TS *)a.x.p + blockIdx.y * a.x.bs;
   T *A = a.A + (size_t)blockIdx.y * n * n, *L = a.L + (size_t)blockIdx.y * n * n;
-  // Element (r, c) as the launches before this one left it (lower triangle). Rows and columns
-  // past n read the last one: what comes of them is not kept.
-  auto source = [&](int r, int c) {
-    r = min(r, n - 1), c = min(c, n - 1);
-    return s <= 1 ? T(x[r * a.x.rs + c * a.x.cs]) : A[(size_t)r * n + c];
-  };
+  // Element (r, c) of the matrix (lower triangle), and what the launches before the last took from
+  // it, with its sign. Rows and columns past n read the last one: what comes of them is not kept.
+  auto element = [&](int r, int c) { return x[min(r, n - 1) * a.x.rs + min(c, n - 1) * a.x.cs]; };
+  auto taken_before = [&](int r, int c) { return s > 1 ? A[(size_t)min(r, n - 1) * n + min(c, n - 1)] : S::make(0.0, 0.0); };
   // What a wave does in 16 x 16 sub-tiles before anything waits: a tile that is not finished in this launch,
   // or the lower half of the diagonal tile (the own tile of such a workgroup follows in the shadow of the
   // factorisation; complex: here).
@@ -270,19 +306,33 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
   };
   constexpr int MOST = OWN_LATER ? ALL : ALL + LOWER, JOBS = (MOST + CHOL_WAVES - 1) / CHOL_WAVES;
   LaTile<T> acc[JOBS];
+  LaTile<TS> raw[JOBS];  // (converted only once it is used: a conversion would wait for its load)
 #pragma unroll
   for (int e = 0; e < JOBS; e++) {  // every load is on its way before the first is waited for
     int diag, tr, tc;
     if (!job(e * CHOL_WAVES + wave, &diag, &tr, &tc)) continue;
 #pragma unroll
-    for (int v = 0; v < 4; v++) acc[e].v[v] = source((diag ? s : i) * NB + tr * 16 + 4 * v + q, j * NB + tc * 16 + r16);
+    for (int v = 0; v < 4; v++) {
+      const int r = (diag ? s : i) * NB + tr * 16 + 4 * v + q, c = j * NB + tc * 16 + r16;
+      acc[e].v[v] = taken_before(r, c);
+      if (panel) raw[e].v[v] = element(r, c);
+    }
   }
+  // Double: what is taken from the diagonal tile is summed apart from it, for a 16 x 16 tile below the
+  // diagonal in the place of its mirror image, transposed; for one on the diagonal in diag_sum.
+  auto taken_at = [&](int tr, int tc) { return (double *)(tr == tc ? diag_sum + tr * 256 + q * 16 + r16 : (double *)D + (tc * 16 + r16) * LD + tr * 16 + q); };
+  auto taken_step = [](int tr, int tc) { return tr == tc ? 64 : 4; };
   constexpr int PER = NB * NB / CHOL_THREADS;
   const int col_of = threadIdx.x % NB, row_of = threadIdx.x / NB;
-  T mine[PER];
+  TS mine[PER];
+  T mine_taken[PER];
   if (OWN_LATER && panel && has_own) {
 #pragma unroll
-    for (int e = 0; e < PER; e++) mine[e] = source(i * NB + row_of + e * (CHOL_THREADS / NB), s * NB + col_of);
+    for (int e = 0; e < PER; e++) {
+      const int r = i * NB + row_of + e * (CHOL_THREADS / NB), c = s * NB + col_of;
+      mine[e] = element(r, c);
+      mine_taken[e] = taken_before(r, c);
+    }
   }
   if (s > 0) {
     T vj[PER], vi[PER];
@@ -309,37 +359,46 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       const int r = tr * 16 + 4 * v + q, cc = tc * 16 + r16;
+      const bool inside = r < left && cc < left;
       if (!panel) {
         if (i * NB + r < n && j * NB + cc < n) A[(size_t)(i * NB + r) * n + j * NB + cc] = acc[e].v[v];
-      } else if (diag) {  // past n the diagonal tile is the identity
-        D[r * LD + cc] = r < left && cc < left ? acc[e].v[v] : S::make(r == cc ? 1.0 : 0.0, 0.0);
-      } else {
-        own[r * LD + cc] = acc[e].v[v];
+      } else if (!diag) {
+        own[r * LD + cc] = T(raw[e].v[v]) + acc[e].v[v];
+      } else {  // past n the diagonal tile is the identity
+        const T val = OWN_LATER ? T(raw[e].v[v]) : T(raw[e].v[v]) + acc[e].v[v];
+        D[r * LD + cc] = inside ? val : S::make(r == cc ? 1.0 : 0.0, 0.0);
+        if constexpr (OWN_LATER) taken_at(tr, tc)[v * taken_step(tr, tc)] = inside ? -acc[e].v[v] : 0.0;
       }
     }
   }
   if (OWN_LATER && panel && has_own) {
 #pragma unroll
-    for (int e = 0; e < PER; e++) own[(row_of + e * (CHOL_THREADS / NB)) * LD + col_of] = mine[e];
+    for (int e = 0; e < PER; e++) own[(row_of + e * (CHOL_THREADS / NB)) * LD + col_of] = T(mine[e]) + mine_taken[e];
   }
   if (!panel) return;
   __syncthreads();
   bool bad = false;
   if constexpr (sizeof(T) == 8) {
-    // rows (sixteen, in LDS) against columns 16 jb .. of the diagonal tile; `before`: they still lack the
-    // updates by the columns before those, by block column s - 1 (rows of li at `before`) and in this one
+    // rows (sixteen, in LDS) against columns 16 jb .. of the diagonal tile; `before`: nothing has summed yet
+    // what the columns before those take, of block column s - 1 (rows of li at `before`) and of this one
     auto solve_rows = [&](double *rows, int jb, const double *before) {
       LaTile<double> t;
 #pragma unroll
       for (int v = 0; v < 4; v++) t.v[v] = rows[r16 * LD + jb * 16 + 4 * v + q];
+      la_f64x4 taken = {0.0, 0.0, 0.0, 0.0};
       if (before) {
-        if (s > 0) tile_sub<NB>(t, ls + jb * 16 * LD, LD, before, LD);
+        if (s > 0) taken = tile_sum<NB>(ls + jb * 16 * LD, LD, before, LD);
 #pragma unroll 1
-        for (int k = 0; k < jb * 16; k += 16) tile_sub<16>(t, D + jb * 16 * LD + k, LD, rows + k, LD);
+        for (int k = 0; k < jb * 16; k += 16) taken += tile_sum<16>(D + jb * 16 * LD + k, LD, rows + k, LD);
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; v++) taken[v] = D[(jb * 16 + 4 * v + q) * LD + wave * 16 + r16];
       }
       double di[4], tr[4];
 #pragma unroll
       for (int v = 0; v < 4; v++) di[v] = op_inv[(jb * 4 + v) * 64 + lane], tr[v] = op_tri[(jb * 4 + v) * 64 + lane];
+#pragma unroll
+      for (int v = 0; v < 4; v++) t.v[v] -= taken[v];
       const bool solved = solve16(t, di, tr);
 #pragma unroll
       for (int v = 0; v < 4; v++) rows[r16 * LD + jb * 16 + 4 * v + q] = t.v[v];
@@ -364,17 +423,14 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
       if (wave == 0) {
         double *tile = D + jb * 16 * (LD + 1);
         LaTile<double> t;
+        la_f64x4 taken = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int v = 0; v < 4; v++) t.v[v] = tile[r16 * LD + 4 * v + q];
-        if (jb > 0) tile_sub<16>(t, tile - 16, LD, tile - 16, LD);
-        // (the lower triangle is what is kept up to date)
+        for (int v = 0; v < 4; v++) t.v[v] = tile[max(r16, 4 * v + q) * LD + min(r16, 4 * v + q)];  // (the lower triangle is what there is)
+        if (jb > 0) taken = tile_sum<16>(tile - 16, LD, tile - 16, LD);
 #pragma unroll
-        for (int v = 0; v < 4; v++) tile[r16 * LD + 4 * v + q] = t.v[v];
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int v = 0; v < 4; v++) t.v[v] = tile[max(r16, 4 * v + q) * LD + min(r16, 4 * v + q)];
+        for (int v = 0; v < 4; v++) taken[v] += taken_at(jb, jb)[64 * v];
         double di[4], tr[4];
-        bad = !factor16(t, blk, di, tr) || bad;
+        bad = !factor16(t, taken, (double2 *)blk, di, tr) || bad;
 #pragma unroll
         for (int v = 0; v < 4; v++) {
           op_inv[(jb * 4 + v) * 64 + lane] = di[v];
@@ -385,12 +441,11 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
         for (int t = wave - 2; t < TILES * TILES; t += 2) {  // what block jb - 1 takes from the rest of the tile
           const int tr = t / TILES, tc = t % TILES;
           if (tc < jb || tc > tr || tr >= blocks || (tc == jb && tr == jb)) continue;
-          LaTile<double> d;
+          la_f64x4 d = tile_sum<16>(D + tr * 16 * LD + (jb - 1) * 16, LD, D + tc * 16 * LD + (jb - 1) * 16, LD);
+          double *to = taken_at(tr, tc);
+          const int step = taken_step(tr, tc);
 #pragma unroll
-          for (int v = 0; v < 4; v++) d.v[v] = D[(tr * 16 + 4 * v + q) * LD + tc * 16 + r16];
-          tile_sub<16>(d, D + tr * 16 * LD + (jb - 1) * 16, LD, D + tc * 16 * LD + (jb - 1) * 16, LD);
-#pragma unroll
-          for (int v = 0; v < 4; v++) D[(tr * 16 + 4 * v + q) * LD + tc * 16 + r16] = d.v[v];
+          for (int v = 0; v < 4; v++) to[v * step] += d[v];
         }
       } else if (jb > 0) {
         solve_own(jb - 1);
@@ -417,15 +472,15 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
         for (int v = 0; v < 4; v++) rows[(4 * v + q) * LD + jb * 16 + r16] = t.v[v];
         __builtin_amdgcn_wave_barrier();
       }
-      T xr[16];
+      T xr[16];  // what the columns so far take from those after them
 #pragma unroll
-      for (int c = 0; c < 16; c++) xr[c] = rows[r16 * LD + jb * 16 + c];
-      __builtin_amdgcn_wave_barrier();
+      for (int c = 0; c < 16; c++) xr[c] = S::make(0.0, 0.0);
+      T *at = rows + r16 * LD + jb * 16;
       const T *col = D + jb * 16 * (LD + 1);  // (c, c) of the diagonal block; rows past it are read, their results dropped
 #pragma unroll 1
       for (int c = 0; c < 16; c++, col += LD + 1) {
-        const T v = S::scale(xr[0], inv[jb * 16 + c]);
-        if (q == 0) rows[r16 * LD + jb * 16 + c] = v;
+        const T v = S::scale(at[c] + xr[0], inv[jb * 16 + c]);
+        if (q == 0) at[c] = v;
 #pragma unroll
         for (int k = 1; k < 16; k++) xr[k - 1] = S::sub_mul(xr[k], v, S::conj(col[k * LD]));
       }
@@ -434,20 +489,21 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
     for (int jb = 0; jb < blocks; jb++) {
       if (wave == 0) {
         const int c0 = jb * 16, row = min(lane, NB - 1);
-        // `head`: this lane's element of the column at hand, up to date; p: of the columns after
-        // it, which still lack the update by `prev`, the column before it. That column's values come
+        // `head`: this lane's element of the column at hand, up to date; p: what the columns so far take
+        // from those after it, still without `prev`, the column before it. That column's values come
         // back from LDS while the square root is under way; only the next column's head waits for a
         // value of this one, and takes it from its lane (a lane's value costs some 20 cycles a register)
         T p[16], prev = S::make(0.0, 0.0);
 #pragma unroll
-        for (int c = 0; c < 16; c++) p[c] = D[row * LD + c0 + c];
-        T head = p[0];
+        for (int c = 0; c < 16; c++) p[c] = S::make(0.0, 0.0);
+        T head = D[row * LD + c0];
         column[lane] = prev;
 #pragma unroll 1
         for (int c = c0; c < c0 + 16; c++) {
           T before[16];
 #pragma unroll
           for (int k = 1; k < 16; k++) before[k] = column[c + k];
+          const T next = D[row * LD + min(c + 1, NB - 1)];
           const double d = S::re(lane_value(head, c));
           bad = bad || !(d > 0.0);
           double l, li1;
@@ -458,7 +514,7 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
           column[lane] = col;
           if (lane == 0) inv[c] = li1;
           if (lane < NB && lane >= c0) D[lane * LD + c] = lane < c ? S::make(0.0, 0.0) : col;
-          head = S::sub_mul(p[0], col, S::conj(lane_value(col, (c + 1) & 63)));
+          head = next + S::sub_mul(p[0], col, S::conj(lane_value(col, (c + 1) & 63)));
           prev = col;
         }
       } else if (jb > 0) {

@@ -127,6 +127,35 @@ def test_triangular_solve_with_weak_diagonals(hip, n, upper, transpose):
         assert np.all(residual <= (n + 1) * 2.0 ** -53 * (np.abs(m).astype(np.longdouble) @ np.abs(x))), power
 
 
+@pytest.mark.parametrize("n", [4, 8, 16, 40, 64, 100, 256])
+def test_cholesky_rounds_a_few_times(hip, n):
+    """float64 against long double, over matrices whose diagonal does not dominate: |A - L L^T| stays
+    under the bound of a factorisation by columns, (n + 1) eps sqrt(a_ii a_jj) (Higham, theorem 10.3). An
+    element rounds a few times at its own size, whatever n is: in a Gram matrix that is n^-1/2 of the
+    bound's off the diagonal, and the n elements on it weigh as much in the mean, so a root mean square of
+    1.5 n^-1/2 eps covers five roundings (an update from the matrix per column: n^1/2 as many). Graded
+    and nearly singular ones keep the first bound."""
+    rng, eps = np.random.default_rng(n), 2.0 ** -53
+    for kind in ("gram", "tall", "graded", "kernel"):
+        squares = []
+        for _ in range(max(2, 256 // n)):
+            g = rng.standard_normal((n, n + (2 if kind == "tall" else 0)))
+            a = g @ g.T
+            if kind == "graded":
+                scale = 10.0 ** rng.uniform(-6, 6, n)
+                a = a * scale[:, None] * scale
+            if kind == "kernel":
+                p = rng.uniform(0, 1, n)
+                a = np.exp(-((p[:, None] - p) * n) ** 2 / 4) + 1e-9 * np.eye(n)
+            a = np.tril(a) + np.tril(a, -1).T
+            low = logical(hip.cholesky(put(hip, a, dt.float64))).astype(np.longdouble)
+            root = np.sqrt(np.diag(a))
+            off = np.abs(low @ low.T - a) / np.outer(root, root) / eps
+            assert np.max(off) <= n + 1, (kind, float(np.max(off)))
+            squares.append(np.mean(off ** 2))
+        assert np.mean(squares) <= 1.5 ** 2 / n or kind in ("graded", "kernel"), (kind, float(np.sqrt(np.mean(squares))))
+
+
 def substituted(m, b, lower):
     """Plain substitution in float64, a row at a time."""
     x = b.astype(np.float64)
