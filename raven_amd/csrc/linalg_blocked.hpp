@@ -157,11 +157,12 @@ __device__ __forceinline__ bool solve16(LaTile<double> &acc, const double (&diag
 // element, the matrix instruction does the rest. The tile is acc - before; what its own columns take is
 // summed beside `before`, so that an element of a diagonal block rounds once at its own size.
 // Leaves the operands of solve16 in diag_inv and tri; tri is the factor itself. `blk`: 64 places of LDS.
+// False where that is not the factor: a pivot that is not positive or not finite, or a step as in solve16.
 __device__ __forceinline__ bool factor16(const LaTile<double> &acc, la_f64x4 before, double2 *blk, double (&diag_inv)[4], double (&tri)[4]) {
   const int lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
   const la_f64x4 zero = {0.0, 0.0, 0.0, 0.0};
   la_f64x4 taken = zero;
-  bool positive = true;
+  bool good = true;
 #pragma unroll
   for (int b = 0; b < 4; b++) {
     const double off = b > 0 ? before[b] + taken[b] : before[b], t = acc.v[b] - off;
@@ -182,7 +183,7 @@ __device__ __forceinline__ bool factor16(const LaTile<double> &acc, la_f64x4 bef
     for (int j = 0; j < 4; j++) {
 #pragma unroll
       for (int i = j; i < 4; i++) low[j][i] = a[j][i] - (j > 0 ? sum[j][i] + own[j][i] : sum[j][i]);
-      positive = positive && low[j][j] > 0.0;
+      good = good && low[j][j] > 0.0 && low[j][j] < __builtin_inf();
       root_and_inverse(low[j][j], &low[j][j], &root[j]);
 #pragma unroll
       for (int i = j + 1; i < 4; i++) low[j][i] *= root[j];
@@ -218,7 +219,30 @@ __device__ __forceinline__ bool factor16(const LaTile<double> &acc, la_f64x4 bef
     const double rest = t - __builtin_amdgcn_mfma_f64_16x16x4f64(x, x, zero, 0, 0, 0)[b];
     const double dx = __builtin_amdgcn_mfma_f64_16x16x4f64(diag_inv[b], rest, zero, 0, 0, 0)[b];
     tri[b] = below ? x + dx : x;
+    good = good && (!below || small_step(x, dx));
     if (b < 3) taken = __builtin_amdgcn_mfma_f64_16x16x4f64(tri[b], tri[b], taken, 0, 0, 0);
+  }
+  return __all(good);
+}
+
+// The same column by column, in place on the lower triangle (the rest becomes 0), for what factor16
+// refuses: pivots that are infinite, tiles close to singular; a failure shows here. 1 / L_cc goes to
+// the place that lane (q, c) of diag_inv[c / 4], q = c % 4, has in `inv`.
+__device__ __forceinline__ bool factor16_columns(double *tile, int ld, double *inv) {
+  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  bool positive = true;
+#pragma unroll 1
+  for (int c = 0; c < 16; c++) {
+    wave_sync();
+    const double d = tile[c * ld + c], own = tile[r * ld + c];
+    positive = positive && d > 0.0;
+    double root, root_inv;
+    root_and_inverse(d, &root, &root_inv);
+    wave_sync();
+    if (q == 0) tile[r * ld + c] = r == c ? root : r > c ? own * root_inv : 0.0;
+    if (lane == 0) inv[(c >> 2) * 64 + (c & 3) * 16 + c] = root_inv;
+    wave_sync();
+    for (int k = c + 1 + q; k <= r; k += 4) tile[r * ld + k] = fma(-tile[r * ld + c], tile[k * ld + c], tile[r * ld + k]);
   }
   return positive;
 }
@@ -430,13 +454,15 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
 #pragma unroll
         for (int v = 0; v < 4; v++) taken[v] += taken_at(jb, jb)[64 * v];
         double di[4], tr[4];
-        bad = !factor16(t, taken, (double2 *)blk, di, tr) || bad;
+        const bool stands = factor16(t, taken, (double2 *)blk, di, tr);
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
+        for (int v = 0; v < 4; v++) tile[r16 * LD + 4 * v + q] = stands ? tr[v] : t.v[v] - taken[v];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {  // (solve16 refuses operands that are no numbers)
           op_inv[(jb * 4 + v) * 64 + lane] = di[v];
-          op_tri[(jb * 4 + v) * 64 + lane] = tr[v];
-          tile[r16 * LD + 4 * v + q] = tr[v];
+          op_tri[(jb * 4 + v) * 64 + lane] = stands ? tr[v] : __builtin_nan("");
         }
+        if (!stands) bad = !factor16_columns(tile, LD, op_inv + jb * 256) || bad;
       } else if (jb > 0 && (wave == 2 || wave == 3)) {
         for (int t = wave - 2; t < TILES * TILES; t += 2) {  // what block jb - 1 takes from the rest of the tile
           const int tr = t / TILES, tc = t % TILES;

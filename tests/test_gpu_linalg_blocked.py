@@ -156,6 +156,49 @@ def test_cholesky_rounds_a_few_times(hip, n):
         assert np.mean(squares) <= 1.5 ** 2 / n or kind in ("graded", "kernel"), (kind, float(np.sqrt(np.mean(squares))))
 
 
+@pytest.mark.parametrize("n", [1, 4, 17, 70])
+def test_cholesky_at_the_ends_of_the_range(hip, n):
+    """Pivots that are subnormal, next to the largest number or infinite factor as their roots do (an
+    infinite one leaves zeros below it); a zero, a negative one and a NaN do not."""
+    rng = np.random.default_rng(n)
+    for name, values in (("float64", (5e-324, 1e-310, 4e-309, 1e-300, 1e300, 1.7e308, np.inf)), ("float32", (1e-45, 1e-40, 3e38, np.inf))):
+        d = dt.BY_NAME[name]
+        for value in values:
+            for at in {0, n // 2, n - 1}:
+                diag = rng.uniform(0.5, 2, n)
+                diag[at] = value
+                a = np.diag(diag).astype(d.np_storage)
+                if np.isinf(value):
+                    a[at + 1:, at], a[at, :at] = 0.25, 0.125 / n  # (the lower triangle is what is read)
+                    a[at, :at] = 0.125 / n
+                low = logical(hip.cholesky(put(hip, a, d))).astype(np.float64)
+                want = np.diag(np.sqrt(np.diag(a).astype(np.float64)))
+                want[at, :at] = a[at, :at].astype(np.float64) / np.diag(want)[:at]
+                assert np.array_equal(np.isfinite(low), np.isfinite(want))
+                f = np.isfinite(want)
+                assert np.all(np.abs(low[f] - want[f]) <= (4 * 2.0 ** -53 + EPS[name]) * np.abs(want[f])), (name, value, at)
+    for value in (0.0, -1e-310, -np.inf, np.nan):
+        a = np.eye(n)
+        a[n // 2, n // 2] = value
+        with pytest.raises(RuntimeError, match="not positive definite"):
+            hip.cholesky(put(hip, a, dt.float64))
+
+
+@pytest.mark.parametrize("n", [8, 16, 40, 100])
+def test_cholesky_close_to_singular(hip, n):
+    """Whole numbers with a repeated row, and 2^-45 of the diagonal on top: the last pivots are far above the
+    n eps by which a factorisation is off, so it is not refused, and off by no more than others."""
+    rng = np.random.default_rng(n)
+    for _ in range(20):
+        g = rng.integers(-3, 4, (n, n)).astype(np.float64)
+        g[n // 2] = g[n // 2 - 1]
+        a = g @ g.T
+        a += np.max(a) * 2.0 ** -45 * np.eye(n)
+        low = logical(hip.cholesky(put(hip, a, dt.float64))).astype(np.longdouble)
+        root = np.sqrt(np.diag(a))
+        assert np.max(np.abs(low @ low.T - a) / np.outer(root, root)) <= (n + 1) * 2.0 ** -53
+
+
 def substituted(m, b, lower):
     """Plain substitution in float64, a row at a time."""
     x = b.astype(np.float64)
