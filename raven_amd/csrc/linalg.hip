@@ -1183,25 +1183,34 @@ static bool la_direct(const nxh_tensor *t, LaMat *m) {
   return true;
 }
 
-// The word of pinned memory the blocked kernels report to; zero between calls.
-static int *la_host_status(nxh_context *ctx) { return ctx->fault_flag_host + 8; }
-
-// Waits for the kernels of this call (the results included) and reads their report.
-static int la_collect_host(nxh_context *ctx, const char *op) {
-  std::lock_guard<std::mutex> g(ctx->mu);
-  NXH_HIP(op, hipGetLastError());
-  NXH_HIP(op, hipStreamSynchronize(ctx->stream));
-  volatile int *host = la_host_status(ctx);
-  const int code = *host;
-  if (code == LA_OK) return NXH_OK;
-  *host = 0;
-  return nxh_fail(NXH_FAILURE, op, LA_MESSAGES[code <= LA_NO_CONVERGE ? code : LA_NO_CONVERGE]);
-}
+// The word of pinned memory the blocked kernels report to. It belongs to one call at a time (the
+// context's call_mu), which clears it first, and waits for the kernels that may still write it also
+// where it returns early.
+struct HostStatus {
+  nxh_context *ctx;
+  bool waited = false;
+  explicit HostStatus(nxh_context *c) : ctx(c) { *(volatile int *)word() = LA_OK; }
+  ~HostStatus() {
+    if (waited) return;
+    std::lock_guard<std::mutex> g(ctx->mu);
+    (void)hipStreamSynchronize(ctx->stream);
+  }
+  int *word() const { return ctx->fault_flag_host + 8; }
+  // Waits for the kernels of this call (the results included) and reads their report.
+  int collect(const char *op) {
+    std::lock_guard<std::mutex> g(ctx->mu);
+    NXH_HIP(op, hipGetLastError());
+    NXH_HIP(op, hipStreamSynchronize(ctx->stream));
+    waited = true;
+    const int code = *(volatile int *)word();
+    return code == LA_OK ? NXH_OK : nxh_fail(NXH_FAILURE, op, LA_MESSAGES[code <= LA_NO_CONVERGE ? code : LA_NO_CONVERGE]);
+  }
+};
 
 constexpr int64_t LA_GRID_BATCH = 65535;  // matrices per launch (the grid's y and z extent)
 
 template <class T, class TS>
-static int run_cholesky(nxh_context *ctx, const char *op, int64_t batch, int n, int upper, LaMat x, LaMat out, T *A, T *L) {
+static int run_cholesky(nxh_context *ctx, const char *op, HostStatus &status, int64_t batch, int n, int upper, LaMat x, LaMat out, T *A, T *L) {
   constexpr int NB = CHOL_NB<T>;
   auto kern = cholesky_block_kernel<T, TS>;
   static std::once_flag once;
@@ -1220,7 +1229,7 @@ static int run_cholesky(nxh_context *ctx, const char *op, int64_t batch, int n, 
     a.L = L + (size_t)b0 * n * n;
     a.n = n;
     a.upper = upper;
-    a.status = la_host_status(ctx);
+    a.status = status.word();
     const int cols = (n + NB - 1) / NB;
     for (int s = 0; s < cols; s++) {
       a.s = s;
@@ -1240,7 +1249,7 @@ constexpr int TRSM_PASS = sizeof(T) == 8 ? 1024 : 512;
 // b and x may be one workspace (they are where there are several passes: what is passed on between
 // them is in the compute type).
 template <class T, class TS>
-static int run_trsm(nxh_context *ctx, const char *op, int64_t batch, int n, int nrhs, int flags, LaMat m, LaMat b, LaMat x) {
+static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, int64_t batch, int n, int nrhs, int flags, LaMat m, LaMat b, LaMat x) {
   const bool upper = flags & 1, transpose = (flags >> 1) & 1, forward = upper == transpose;
   auto kern = trsm_block_kernel<T, TS>;
   static std::once_flag once;
@@ -1271,7 +1280,7 @@ static int run_trsm(nxh_context *ctx, const char *op, int64_t batch, int n, int 
       a.x = LaMat{xp + b0 * x.bs + r0 * x.rs, x.rs, x.cs, x.bs};
       a.rows = std::min(n - r0, TRSM_PASS<T>);
       a.nrhs = nrhs;
-      a.status = la_host_status(ctx);
+      a.status = status.word();
       const int nb = (a.rows + 15) / 16;
       hipLaunchKernelGGL(kern, dim3(groups, nbat), dim3(64 * TRSM_WAVES), (size_t)nb * 256 * sizeof(T), ctx->stream, a);
       const int rest = n - r0 - a.rows;
@@ -1377,6 +1386,7 @@ NXH_EXPORT int nxh_cholesky(nxh_context *ctx, const nxh_tensor *out, const nxh_t
   // one factorisation at a time per context: they share the status word and its host slot
   std::lock_guard<std::mutex> whole_call(ctx->call_mu);
   if ((rc = la_begin(ctx, op))) return rc;
+  HostStatus status(ctx);
   Work work(ctx);
   PathAtExit path{n >= LA_WIDE_FROM ? "cholesky_columns_wide" : "cholesky_columns"};
   const size_t mat = (size_t)(p.batch * n * n) * p.esize;
@@ -1394,12 +1404,12 @@ NXH_EXPORT int nxh_cholesky(nxh_context *ctx, const nxh_tensor *out, const nxh_t
     wio.data = (char *)io + mat;
     mo = LaMat{wio.data, n, 1, n * n};
   }
-  if (p.cx) rc = run_cholesky<c64, c64>(ctx, op, p.batch, (int)n, upper, mx, mo, (c64 *)A, (c64 *)L);
-  else if (direct && x->dtype == NXH_F32) rc = run_cholesky<double, float>(ctx, op, p.batch, (int)n, upper, mx, mo, (double *)A, (double *)L);
-  else rc = run_cholesky<double, double>(ctx, op, p.batch, (int)n, upper, mx, mo, (double *)A, (double *)L);
+  if (p.cx) rc = run_cholesky<c64, c64>(ctx, op, status, p.batch, (int)n, upper, mx, mo, (c64 *)A, (c64 *)L);
+  else if (direct && x->dtype == NXH_F32) rc = run_cholesky<double, float>(ctx, op, status, p.batch, (int)n, upper, mx, mo, (double *)A, (double *)L);
+  else rc = run_cholesky<double, double>(ctx, op, status, p.batch, (int)n, upper, mx, mo, (double *)A, (double *)L);
   if (rc) return rc;
   if (!direct && (rc = nxh_cast(ctx, out, &wio))) return rc;
-  return la_collect_host(ctx, op);
+  return status.collect(op);
 }
 
 // nx_c_tri.c:459-562, 580-600. `b` and `out` are matrices of right-hand sides
@@ -1423,6 +1433,7 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
   // one factorisation at a time per context: they share the status word and its host slot
   std::lock_guard<std::mutex> whole_call(ctx->call_mu);
   if ((rc = la_begin(ctx, op))) return rc;
+  HostStatus status(ctx);
   Work work(ctx);
   PathAtExit path{n >= LA_WIDE_FROM ? "triangular_substitution_wide" : "triangular_substitution"};
   LaMat ma{}, mb{}, mx{};
@@ -1438,12 +1449,12 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
     ma = LaMat{A, n, 1, n * n};
     mb = mx = LaMat{X, nrhs, 1, n * nrhs};
   }
-  if (p.cx) rc = run_trsm<c64, c64>(ctx, op, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
-  else if (direct && a->dtype == NXH_F32) rc = run_trsm<double, float>(ctx, op, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
-  else rc = run_trsm<double, double>(ctx, op, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
+  if (p.cx) rc = run_trsm<c64, c64>(ctx, op, status, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
+  else if (direct && a->dtype == NXH_F32) rc = run_trsm<double, float>(ctx, op, status, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
+  else rc = run_trsm<double, double>(ctx, op, status, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
   if (rc) return rc;
   if (!direct && (rc = nxh_cast(ctx, out, &wx))) return rc;
-  return la_collect_host(ctx, op);
+  return status.collect(op);
 }
 
 // nx_c_qr.c; nx_backend.ml:613-626. q is [..., m, k] (reduced) or [..., m, m]; r is

@@ -87,6 +87,7 @@ NXH_EXPORT int nxh_context_create(nxh_context **out) {
   if (e == hipSuccess) e = hipEventCreate(&ctx->ev_stop);
   if (e == hipSuccess) e = hipMalloc((void **)&ctx->fault_flag, 256);
   if (e == hipSuccess) e = hipHostMalloc((void **)&ctx->fault_flag_host, 256, hipHostMallocDefault);
+  if (e == hipSuccess) memset(ctx->fault_flag_host, 0, 256);
   if (e == hipSuccess)
     e = hipHostMalloc((void **)&ctx->stage, nxh_context::STAGE_SLOTS * nxh_context::STAGE_BYTES, hipHostMallocDefault);
   for (int i = 0; i < nxh_context::STAGE_SLOTS && e == hipSuccess; i++)

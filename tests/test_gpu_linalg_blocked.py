@@ -234,6 +234,28 @@ def test_triangular_solve_of_sides_that_are_not_finite(hip, name, upper, transpo
     assert np.all(np.abs(got[finite] - want[finite]) <= room[finite])
 
 
+def test_first_call_of_a_context(hip):
+    """The word that failures are reported in starts out clear, whatever its memory held before."""
+    import ctypes as C
+    from raven_amd.nx_backend import Backend
+    rt = C.CDLL("libamdhip64.so")
+    blocks = [C.c_void_p() for _ in range(16)]
+    for p in blocks:
+        assert rt.hipHostMalloc(C.byref(p), C.c_size_t(256), C.c_uint(0)) == 0
+        C.memset(p, 1, 256)
+    for p in blocks:
+        assert rt.hipHostFree(p) == 0
+    fresh = Backend()
+    a = 2 * np.eye(5)
+    low = logical(fresh.cholesky(put(fresh, a, dt.float64)))
+    assert np.max(np.abs(low - np.sqrt(a))) <= 2.0 ** -52
+    with pytest.raises(RuntimeError, match="not positive definite"):
+        fresh.cholesky(put(fresh, -a, dt.float64))
+    with pytest.raises(RuntimeError, match="singular"):
+        fresh.triangular_solve(put(fresh, 0 * a, dt.float64), put(fresh, a, dt.float64), False, False, False)
+    assert np.array_equal(logical(fresh.cholesky(put(fresh, a, dt.float64))), low)
+
+
 def test_in_place_and_shared_storage(hip):
     """Results over the operands' own storage, as the C ABI allows."""
     import ctypes as C
