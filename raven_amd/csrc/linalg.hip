@@ -1210,34 +1210,43 @@ struct HostStatus {
 constexpr int64_t LA_GRID_BATCH = 65535;  // matrices per launch (the grid's y and z extent)
 
 template <class T, class TS>
-static int run_cholesky(nxh_context *ctx, const char *op, HostStatus &status, int64_t batch, int n, int upper, LaMat x, LaMat out, T *A, T *L) {
+static int run_cholesky(nxh_context *ctx, const char *op, HostStatus &status, int64_t batch, int n, int upper, LaMat x, LaMat out, void *A,
+                        void *diag) {
   constexpr int NB = CHOL_NB<T>;
+  const int64_t cols = (n + NB - 1) / NB, result_tiles = cols * (cols + 1) / 2;
+  if (result_tiles > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "matrix too large for one launch");
   auto kern = cholesky_block_kernel<T, TS>;
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [&] { attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CHOL_LDS<T>); });
   NXH_HIP(op, attr);
-  std::lock_guard<std::mutex> g(ctx->mu);
-  for (int64_t b0 = 0; b0 < batch; b0 += LA_GRID_BATCH) {
-    const int64_t nbat = std::min(LA_GRID_BATCH, batch - b0);
-    CholArgs<T> a{};
-    a.x = x;
-    a.out = out;
-    a.x.p = (TS *)x.p + b0 * x.bs;
-    a.out.p = (TS *)out.p + b0 * out.bs;
-    a.A = A ? A + (size_t)b0 * n * n : nullptr;
-    a.L = L + (size_t)b0 * n * n;
-    a.n = n;
-    a.upper = upper;
-    a.status = status.word();
-    const int cols = (n + NB - 1) / NB;
+  const auto each_part = [&](auto launch) {  // parts of the batch that a grid holds
+    std::lock_guard<std::mutex> g(ctx->mu);
+    for (int64_t b0 = 0; b0 < batch; b0 += LA_GRID_BATCH) {
+      CholArgs<T> a{};
+      a.x = x;
+      a.out = out;
+      a.x.p = (TS *)x.p + b0 * x.bs;
+      a.out.p = (TS *)out.p + b0 * out.bs;
+      a.A = (T *)A + (size_t)b0 * n * n;
+      a.diag = (T *)diag + (size_t)(b0 * cols) * NB * NB;
+      a.n = n;
+      a.upper = upper;
+      a.status = status.word();
+      launch(a, (unsigned)std::min(LA_GRID_BATCH, batch - b0));
+    }
+  };
+  each_part([&](CholArgs<T> &a, unsigned nbat) {
     for (int s = 0; s < cols; s++) {
       a.s = s;
       const int64_t panels = cols - s, tiles = panels + (s > 0 ? panels * (panels - 1) / 2 : 0);
-      if (tiles > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "matrix too large for one launch");
-      hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)nbat), dim3(CHOL_THREADS), CHOL_LDS<T>, ctx->stream, a);
+      hipLaunchKernelGGL(kern, dim3((unsigned)tiles, nbat), dim3(CHOL_THREADS), CHOL_LDS<T>, ctx->stream, a);
     }
-  }
+  });
+  if (int rc = status.collect(op)) return rc;  // a matrix that has no factor leaves `out` as it was
+  each_part([&](CholArgs<T> &a, unsigned nbat) {
+    hipLaunchKernelGGL((cholesky_result_kernel<T, TS>), dim3((unsigned)result_tiles, nbat), dim3(256), 0, ctx->stream, a);
+  });
   NXH_HIP(op, hipGetLastError());
   return NXH_OK;
 }
@@ -1390,26 +1399,23 @@ NXH_EXPORT int nxh_cholesky(nxh_context *ctx, const nxh_tensor *out, const nxh_t
   Work work(ctx);
   PathAtExit path{n >= LA_WIDE_FROM ? "cholesky_columns_wide" : "cholesky_columns"};
   const size_t mat = (size_t)(p.batch * n * n) * p.esize;
-  void *A = nullptr, *L, *io = nullptr;
-  const int nb = p.cx ? CHOL_NB<c64> : CHOL_NB<double>;
-  if ((rc = work.get(mat, &L)) || (n > 2 * nb && (rc = work.get(mat, &A)))) return rc;
+  const int64_t nb = p.cx ? CHOL_NB<c64> : CHOL_NB<double>;
+  void *A, *diag, *io;
+  if ((rc = work.get(mat, &A)) || (rc = work.get((size_t)(p.batch * ((n + nb - 1) / nb) * nb * nb) * p.esize, &diag))) return rc;
   LaMat mx{}, mo{};
   nxh_tensor wio{};
-  const bool direct = x->data != out->data && la_direct(x, &mx) && la_direct(out, &mo);
+  const bool direct = la_direct(x, &mx) && la_direct(out, &mo);
   if (!direct) {  // both through one workspace of the compute type
-    if ((rc = work.get(2 * mat, &io))) return rc;
+    if ((rc = work.get(mat, &io))) return rc;
     wio = workspace_tensor(x, io, p.wdt, n, n, false);
     if ((rc = nxh_cast(ctx, &wio, x))) return rc;
-    mx = LaMat{io, n, 1, n * n};
-    wio.data = (char *)io + mat;
-    mo = LaMat{wio.data, n, 1, n * n};
+    mx = mo = LaMat{io, n, 1, n * n};
   }
-  if (p.cx) rc = run_cholesky<c64, c64>(ctx, op, status, p.batch, (int)n, upper, mx, mo, (c64 *)A, (c64 *)L);
-  else if (direct && x->dtype == NXH_F32) rc = run_cholesky<double, float>(ctx, op, status, p.batch, (int)n, upper, mx, mo, (double *)A, (double *)L);
-  else rc = run_cholesky<double, double>(ctx, op, status, p.batch, (int)n, upper, mx, mo, (double *)A, (double *)L);
-  if (rc) return rc;
-  if (!direct && (rc = nxh_cast(ctx, out, &wio))) return rc;
-  return status.collect(op);
+  if (p.cx) rc = run_cholesky<c64, c64>(ctx, op, status, p.batch, (int)n, upper, mx, mo, A, diag);
+  else if (direct && x->dtype == NXH_F32) rc = run_cholesky<double, float>(ctx, op, status, p.batch, (int)n, upper, mx, mo, A, diag);
+  else rc = run_cholesky<double, double>(ctx, op, status, p.batch, (int)n, upper, mx, mo, A, diag);
+  if (rc || direct) return rc;
+  return nxh_cast(ctx, out, &wio);
 }
 
 // nx_c_tri.c:459-562, 580-600. `b` and `out` are matrices of right-hand sides

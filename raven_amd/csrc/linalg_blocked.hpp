@@ -253,8 +253,10 @@ __device__ __forceinline__ bool factor16_columns(double *tile, int ld, double *i
 // Column s then is finished: every workgroup of that column keeps the diagonal tile too, factors it (the same
 // instructions on the same values everywhere), and solves its own tile against it, sixteen
 // columns behind. Factoring the diagonal again in each workgroup costs nothing (it would
-// be waited for) and saves a launch per block column. The factor goes to L, the sums to
-// A: nothing that a workgroup of the same launch may still read is overwritten. The sums stay apart from
+// be waited for) and saves a launch per block column. Sums and factor share one workspace: a tile of
+// the factor goes where this workgroup's own sums were, those on the diagonal, whose sums the other
+// workgroups of the column read too, to a place of their own. The matrix itself is only read; the result is
+// written by cholesky_result_kernel, once it is known that there is one. The sums stay apart from
 // the matrix until its column comes up, so that an element rounds a few times at its own size and not
 // once a column: float64, g g^T + n I, relative error of the factor in eps (2-norm, against long double) for
 // n = 64, 130, 400: 1.52, 2.03, 3.41 with the updates taken from the matrix one by one, 0.55, 0.50, 0.51 so
@@ -277,8 +279,9 @@ constexpr size_t CHOL_LDS = 4 * CHOL_NB<T> * (CHOL_NB<T> + 2) * sizeof(T) +
 
 template <class T>
 struct CholArgs {
-  LaMat x, out;  // storage types
-  T *A, *L;      // n x n per matrix, row-major: what is taken from x, with its sign; the factor
+  LaMat x, out;   // storage types
+  T *A, *diag;    // n x n per matrix, row-major: what is taken from x, with its sign, then the factor below the
+                  // diagonal tiles; those tiles, NB x NB each
   int n, s, upper;
   int *status;
 };
@@ -304,7 +307,7 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
     i = s + row, j = s + 1 + t;
   }
   const TS *x = (const TS *)a.x.p + blockIdx.y * a.x.bs;
-  T *A = a.A + (size_t)blockIdx.y * n * n, *L = a.L + (size_t)blockIdx.y * n * n;
+  T *A = a.A + (size_t)blockIdx.y * n * n;
   // Element (r, c) of the matrix (lower triangle), and what the launches before the last took from
   // it, with its sign. Rows and columns past n read the last one: what comes of them is not kept.
   auto element = [&](int r, int c) { return x[min(r, n - 1) * a.x.rs + min(c, n - 1) * a.x.cs]; };
@@ -364,8 +367,8 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
 #pragma unroll
     for (int e = 0; e < PER; e++) {
       const int r = r0 + e * (CHOL_THREADS / NB);
-      vj[e] = L[(size_t)min(j * NB + r, n - 1) * n + (s - 1) * NB + c];
-      vi[e] = L[(size_t)min(i * NB + r, n - 1) * n + (s - 1) * NB + c];
+      vj[e] = A[(size_t)min(j * NB + r, n - 1) * n + (s - 1) * NB + c];
+      vi[e] = A[(size_t)min(i * NB + r, n - 1) * n + (s - 1) * NB + c];
     }
 #pragma unroll
     for (int e = 0; e < PER; e++) {
@@ -564,27 +567,49 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
   }
   if (bad && wave == 0 && lane == 0) raise_host(a.status, LA_NOT_PD);
   __syncthreads();
-  // the factor in double for the launches to come, and the result with its zeros. U = L^H.
-  TS *out = (TS *)a.out.p + blockIdx.y * a.out.bs;
-  const T *tile = has_own ? own : D;
   const int rows = min(n - i * NB, NB);
-  for (int e = threadIdx.x; e < NB * NB; e += CHOL_THREADS) {
-    const int r = e / NB, c = e % NB;
-    if (r >= rows || c >= left) continue;
-    const T v = has_own || c <= r ? tile[r * LD + c] : S::make(0.0, 0.0);
-    L[(size_t)(i * NB + r) * n + s * NB + c] = v;
-    TS *lower = out + (int64_t)(i * NB + r) * a.out.rs + (int64_t)(s * NB + c) * a.out.cs;
-    if (!a.upper) to_storage(v, lower);
-    else if (has_own) to_storage(S::make(0.0, 0.0), lower);
-  }
-  // the tile mirrored across the diagonal, its lanes along that tile's rows
-  if (has_own || a.upper)
+  if (has_own) {
     for (int e = threadIdx.x; e < NB * NB; e += CHOL_THREADS) {
-      const int r = e / NB, c = e % NB;  // of the mirrored tile
-      if (r >= left || c >= rows) continue;
-      const T v = !a.upper ? S::make(0.0, 0.0) : S::conj(has_own || r <= c ? tile[c * LD + r] : S::make(0.0, 0.0));
-      to_storage(v, out + (int64_t)(s * NB + r) * a.out.rs + (int64_t)(i * NB + c) * a.out.cs);
+      const int r = e / NB, c = e % NB;
+      if (r < rows) A[(size_t)(i * NB + r) * n + s * NB + c] = own[r * LD + c];  // (a tile below the diagonal has all its columns)
     }
+  } else {
+    T *to = a.diag + ((size_t)blockIdx.y * (s + panels) + s) * NB * NB;
+    for (int e = threadIdx.x; e < NB * NB; e += CHOL_THREADS) {
+      const int r = e / NB, c = e % NB;
+      if (r < left && c <= r) to[e] = D[r * LD + c];
+    }
+  }
+}
+
+// The result with its zeros, a workgroup per tile (i, j), i >= j, and its mirror image. U = L^H.
+template <class T, class TS>
+__global__ __launch_bounds__(256) void cholesky_result_kernel(CholArgs<T> a) {
+  using S = Sc<T>;
+  constexpr int NB = CHOL_NB<T>;
+  __shared__ T tile[NB][NB + 1];
+  const int n = a.n, cols = (n + NB - 1) / NB;
+  int i = 0, j = blockIdx.x;
+  while (j > i) j -= ++i;
+  const T *A = a.A + (size_t)blockIdx.y * n * n + (size_t)i * NB * n + j * NB;
+  const T *D = a.diag + ((size_t)blockIdx.y * cols + i) * NB * NB;
+  TS *out = (TS *)a.out.p + blockIdx.y * a.out.bs;
+  const int rows = min(n - i * NB, NB), width = min(n - j * NB, NB);
+  for (int e = threadIdx.x; e < NB * NB; e += 256) {
+    const int r = e / NB, c = e % NB;
+    if (r < rows && c < width) tile[r][c] = i > j ? A[(size_t)r * n + c] : c <= r ? D[e] : S::make(0.0, 0.0);
+  }
+  __syncthreads();
+  const T zero = S::make(0.0, 0.0);
+  for (int e = threadIdx.x; e < NB * NB; e += 256) {
+    const int r = e / NB, c = e % NB;
+    if (r < rows && c < width) {  // a diagonal tile is its own mirror image
+      const T v = !a.upper ? tile[r][c] : i > j ? zero : S::conj(tile[c][r]);
+      to_storage(v, out + (int64_t)(i * NB + r) * a.out.rs + (int64_t)(j * NB + c) * a.out.cs);
+    }
+    if (i > j && r < width && c < rows)
+      to_storage(a.upper ? S::conj(tile[c][r]) : zero, out + (int64_t)(j * NB + r) * a.out.rs + (int64_t)(i * NB + c) * a.out.cs);
+  }
 }
 
 // ── triangular solve ────────────────────────────────────────────────────────

@@ -256,6 +256,55 @@ def test_first_call_of_a_context(hip):
     assert np.array_equal(logical(fresh.cholesky(put(fresh, a, dt.float64))), low)
 
 
+def raw_call(hip, name, out, *args):
+    """The C entry itself, the result over storage of the caller's choice."""
+    return getattr(hip._lib, "nxh_" + name)(hip._h, out._desc(), *[a._desc() if hasattr(a, "_desc") else a for a in args])
+
+
+def moved_base(t, bytes_):
+    """The same elements through a descriptor whose storage pointer is `bytes_` further on."""
+    d = type(t._desc()).from_buffer_copy(t._desc())
+    d.data += bytes_
+    d.offset -= bytes_ // t.dtype.itemsize
+
+    class Moved:
+        def _desc(self):
+            return d
+    return Moved()
+
+
+@pytest.mark.parametrize("name", ["float32", "float64", "complex128", "float16"])
+@pytest.mark.parametrize("n", [5, 100])
+def test_a_failing_cholesky_leaves_its_result_alone(hip, name, n):
+    d = dt.BY_NAME[name]
+    a = (2 * np.eye(n) + 0.25).astype(d.np_storage)
+    a[n - 2, n - 2] = -1
+    for upper in (0, 1):
+        t, out = put(hip, a, d), put(hip, np.full((n, n), 7, d.np_storage), d)
+        assert raw_call(hip, "cholesky", t, t, upper) != 0 and np.array_equal(logical(t), a)
+        assert raw_call(hip, "cholesky", out, t, upper) != 0 and np.all(logical(out) == 7)
+        pair = put(hip, np.stack([2 * np.eye(n), a]).astype(d.np_storage), d)  # one of two has a factor
+        assert raw_call(hip, "cholesky", pair, pair, upper) != 0
+        assert np.array_equal(logical(pair), np.stack([2 * np.eye(n), a]).astype(d.np_storage))
+
+
+@pytest.mark.parametrize("n", [5, 100, 200])
+def test_cholesky_over_overlapping_storage(hip, n):
+    """A result that covers the matrix in part, told by base pointers that differ."""
+    rng = np.random.default_rng(n)
+    g = rng.standard_normal((n, n))
+    a = g @ g.T + n * np.eye(n)
+    want = {u: logical(hip.cholesky(put(hip, a, dt.float64), u)) for u in (False, True)}
+    for shift in (0, 1, 7, n * n // 2):
+        for upper in (False, True):
+            whole = put(hip, np.zeros(2 * n * n), dt.float64)
+            x = hip.reshape(hip.shrink(whole, [(0, n * n)]), (n, n))
+            out = hip.reshape(hip.shrink(whole, [(shift, shift + n * n)]), (n, n))
+            hip.assign(x, put(hip, a, dt.float64))
+            assert raw_call(hip, "cholesky", moved_base(out, 8 * shift), x, int(upper)) == 0
+            assert np.array_equal(logical(out), want[upper])
+
+
 def test_in_place_and_shared_storage(hip):
     """Results over the operands' own storage, as the C ABI allows."""
     import ctypes as C
