@@ -1194,6 +1194,9 @@ struct HostStatus {
     if (waited) return;
     std::lock_guard<std::mutex> g(ctx->mu);
     (void)hipStreamSynchronize(ctx->stream);
+    *(volatile int *)word() = LA_OK;
+    (void)hipMemcpyAsync(la_status(ctx), word(), sizeof(int), hipMemcpyHostToDevice, ctx->stream);
+    (void)hipStreamSynchronize(ctx->stream);
   }
   int *word() const { return ctx->fault_flag_host + 8; }
   // Waits for the kernels of this call (the results included) and reads their report.
@@ -1256,9 +1259,10 @@ template <class T>
 constexpr int TRSM_PASS = sizeof(T) == 8 ? 1024 : 512;
 
 // b and x may be one workspace (they are where there are several passes: what is passed on between
-// them is in the compute type).
+// them is in the compute type). Where x is the caller's (`direct`), a singular system leaves it as it was.
 template <class T, class TS>
-static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, int64_t batch, int n, int nrhs, int flags, LaMat m, LaMat b, LaMat x) {
+static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool direct, int64_t batch, int n, int nrhs, int flags, LaMat m,
+                    LaMat b, LaMat x) {
   const bool upper = flags & 1, transpose = (flags >> 1) & 1, forward = upper == transpose;
   auto kern = trsm_block_kernel<T, TS>;
   static std::once_flag once;
@@ -1274,7 +1278,18 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, int64_
     xp += (n - 1) * x.rs;
     ts = -ts, us = -us, b.rs = -b.rs, x.rs = -x.rs;
   }
-  std::lock_guard<std::mutex> g(ctx->mu);
+  std::unique_lock<std::mutex> g(ctx->mu);
+  const bool check = direct && batch > 1 && !((flags >> 2) & 1);  // a workgroup sees the diagonal of its own matrix only
+  if (check) {
+    TrsmArgs<T> a{};
+    a.m = mp;
+    a.ts = ts;
+    a.us = us;
+    a.mbs = m.bs;
+    a.rows = n;
+    a.status = status.word();
+    hipLaunchKernelGGL((trsm_check_kernel<T, TS>), dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, ctx->stream, a, batch, la_status(ctx));
+  }
   for (int64_t b0 = 0; b0 < batch; b0 += LA_GRID_BATCH) {
     const unsigned nbat = (unsigned)std::min(LA_GRID_BATCH, batch - b0), groups = (unsigned)((nrhs + 15) / 16);
     for (int r0 = 0; r0 < n; r0 += TRSM_PASS<T>) {
@@ -1290,6 +1305,7 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, int64_
       a.rows = std::min(n - r0, TRSM_PASS<T>);
       a.nrhs = nrhs;
       a.status = status.word();
+      a.hold = check ? la_status(ctx) : nullptr;
       const int nb = (a.rows + 15) / 16;
       hipLaunchKernelGGL(kern, dim3(groups, nbat), dim3(64 * TRSM_WAVES), (size_t)nb * 256 * sizeof(T), ctx->stream, a);
       const int rest = n - r0 - a.rows;
@@ -1299,7 +1315,10 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, int64_
     }
   }
   NXH_HIP(op, hipGetLastError());
-  return NXH_OK;
+  g.unlock();
+  const int rc = status.collect(op);
+  if (rc && check) (void)la_collect(ctx, op);  // (clears the word on the device)
+  return rc;
 }
 
 // Householder QR of `batch` column-major m x n matrices At, Q's first nq columns to Qt.
@@ -1455,12 +1474,11 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
     ma = LaMat{A, n, 1, n * n};
     mb = mx = LaMat{X, nrhs, 1, n * nrhs};
   }
-  if (p.cx) rc = run_trsm<c64, c64>(ctx, op, status, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
-  else if (direct && a->dtype == NXH_F32) rc = run_trsm<double, float>(ctx, op, status, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
-  else rc = run_trsm<double, double>(ctx, op, status, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
-  if (rc) return rc;
-  if (!direct && (rc = nxh_cast(ctx, out, &wx))) return rc;
-  return status.collect(op);
+  if (p.cx) rc = run_trsm<c64, c64>(ctx, op, status, direct, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
+  else if (direct && a->dtype == NXH_F32) rc = run_trsm<double, float>(ctx, op, status, direct, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
+  else rc = run_trsm<double, double>(ctx, op, status, direct, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
+  if (rc || direct) return rc;
+  return nxh_cast(ctx, out, &wx);
 }
 
 // nx_c_qr.c; nx_backend.ml:613-626. q is [..., m, k] (reduced) or [..., m, m]; r is

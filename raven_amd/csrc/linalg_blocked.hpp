@@ -634,7 +634,21 @@ struct TrsmArgs {
   LaMat b, x;           // rows from row 0 of the solution order on; b is read, x written (TS)
   int rows, nrhs;
   int *status;
+  const int *hold;  // several matrices: where it holds something, one of them is singular and nothing is written
 };
+
+// A wave per matrix: whether an element of its diagonal is zero.
+template <class T, class TS>
+__global__ __launch_bounds__(256) void trsm_check_kernel(TrsmArgs<T> a, int64_t batch, int *found) {
+  const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (b >= batch) return;
+  const TS *m = (const TS *)a.m + b * a.mbs;
+  bool zero = false;
+  for (int t = threadIdx.x & 63; t < a.rows; t += 64) zero = zero || T(m[t * (a.ts + a.us)]) == Sc<T>::make(0.0, 0.0);
+  if (!zero) return;
+  raise(found, LA_SINGULAR);
+  raise_host(a.status, LA_SINGULAR);
+}
 
 template <class T, class TS>
 __device__ __forceinline__ T trsm_coefficient(const TrsmArgs<T> &a, const TS *m, int t, int u) {
@@ -652,6 +666,7 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
   constexpr int TRI_LD = 18;
   __shared__ T tri[2][17][TRI_LD];
   __shared__ double diag_inv[2][4][64];  // operands of solve16, zero outside the 4 x 4 triangles
+  __shared__ int singular;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
   const int n = a.rows, nb = (n + 15) / 16, col0 = blockIdx.x * 16;
   const TS *m = (const TS *)a.m + blockIdx.y * a.mbs;
@@ -661,8 +676,8 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
     const int t = e >> 4, c = col0 + (e & 15);
     X[e] = t < n && c < a.nrhs ? T(b[t * a.b.rs + c * a.b.cs]) : S::make(0.0, 0.0);
   }
+  if (threadIdx.x == 0) singular = 0;
   // the triangle of block `k` and the inverses of its diagonal (past n: the identity), by one wave
-  bool singular = false;
   auto fetch_triangle = [&](int k, TS(&raw)[4]) {
 #pragma unroll
     for (int v = 0; v < 4; v++) raw[v] = m[min(k * 16 + 4 * v + q, n - 1) * a.ts + min(k * 16 + r16, n - 1) * a.us];
@@ -676,7 +691,7 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
       if (k * 16 + max(t, r16) >= n || r16 > t || (a.unit && diagonal)) val = S::make(diagonal ? 1.0 : 0.0, 0.0);
       if (r16 <= t) tri[k & 1][r16][t - r16] = val;
       if (diagonal) {
-        if (val == S::make(0.0, 0.0)) singular = true;
+        if (val == S::make(0.0, 0.0)) singular = 1;
         if constexpr (sizeof(T) == 8) tri[k & 1][t][16] = 1.0 / val;
       }
     }
@@ -846,7 +861,11 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
       }
     }
   }
-  if (singular) raise_host(a.status, LA_SINGULAR);
+  // (every workgroup of a matrix has seen its whole diagonal)
+  if (singular || (a.hold && *a.hold)) {
+    if (threadIdx.x == 0 && singular) raise_host(a.status, LA_SINGULAR);
+    return;
+  }
   for (int e = threadIdx.x; e < n * 16; e += blockDim.x) {
     const int t = e >> 4, c = col0 + (e & 15);
     if (c < a.nrhs) to_storage(X[e], x + t * a.x.rs + c * a.x.cs);

@@ -288,6 +288,27 @@ def test_a_failing_cholesky_leaves_its_result_alone(hip, name, n):
         assert np.array_equal(logical(pair), np.stack([2 * np.eye(n), a]).astype(d.np_storage))
 
 
+@pytest.mark.parametrize("name", ["float32", "float64", "complex128", "float16"])
+@pytest.mark.parametrize("n", [5, 40, 600, 1030])
+def test_a_singular_solve_leaves_its_result_alone(hip, name, n):
+    d, rng = dt.BY_NAME[name], np.random.default_rng(n)
+    a = (np.eye(n) + np.tril(rng.standard_normal((n, n)) / n)).astype(d.np_storage)
+    b = rng.standard_normal((n, 20)).astype(d.np_storage)
+    for at in (0, n - 1):
+        bad = a.copy()
+        bad[at, at] = 0
+        for batch in (1, 3):
+            m, sides = np.stack([a] * (batch - 1) + [bad]), np.stack([b] * batch)
+            t, x, out = put(hip, m, d), put(hip, sides, d), put(hip, np.full(sides.shape, 7, d.np_storage), d)
+            assert raw_call(hip, "triangular_solve", out, t, x, 0) != 0 and np.all(logical(out) == 7)
+            assert raw_call(hip, "triangular_solve", x, t, x, 0) != 0 and np.array_equal(logical(x), sides)
+            assert raw_call(hip, "triangular_solve", out, t, x, 4) == 0 and not np.any(logical(out) == 7)  # (unit diagonal)
+            good = put(hip, np.stack([a] * batch), d)  # the next call knows nothing of it
+            assert raw_call(hip, "triangular_solve", out, good, x, 0) == 0
+            want = np.linalg.solve(a.astype(np.complex128 if d.is_complex else np.float64), sides.astype(np.complex128))
+            assert np.max(np.abs(logical(out).astype(np.complex128) - want)) <= 4e-3 * np.max(np.abs(want))
+
+
 @pytest.mark.parametrize("n", [5, 100, 200])
 def test_cholesky_over_overlapping_storage(hip, n):
     """A result that covers the matrix in part, told by base pointers that differ."""
