@@ -1183,6 +1183,21 @@ static bool la_direct(const nxh_tensor *t, LaMat *m) {
   return true;
 }
 
+// Whether two tensors of one dtype may share bytes: the ranges from their lowest element to their
+// highest meet. (A base pointer says nothing: offsets may make up for it.)
+static bool la_meet(const nxh_tensor *a, const nxh_tensor *b, int size) {
+  const auto range = [&](const nxh_tensor *t, char **low, char **high) {
+    int64_t lo = t->offset, hi = t->offset;
+    for (int d = 0; d < t->ndim; d++) (t->strides[d] < 0 ? lo : hi) += t->strides[d] * (t->shape[d] - 1);
+    *low = (char *)t->data + lo * size;
+    *high = (char *)t->data + (hi + 1) * size;
+  };
+  char *a0, *a1, *b0, *b1;
+  range(a, &a0, &a1);
+  range(b, &b0, &b1);
+  return a0 < b1 && b0 < a1;
+}
+
 // The word of pinned memory the blocked kernels report to. It belongs to one call at a time (the
 // context's call_mu), which clears it first, and waits for the kernels that may still write it also
 // where it returns early.
@@ -1464,7 +1479,9 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
   LaMat ma{}, mb{}, mx{};
   nxh_tensor wx{};
   const int pass = p.cx ? TRSM_PASS<c64> : TRSM_PASS<double>;
-  const bool direct = n <= pass && out->data != a->data && out->data != b->data && la_direct(a, &ma) && la_direct(b, &mb) && la_direct(out, &mx);
+  // the result may be written while other workgroups read: only where it is apart from what they read
+  const int size = a->dtype == NXH_F32 ? 4 : a->dtype == NXH_F64 ? 8 : 16;
+  const bool direct = n <= pass && la_direct(a, &ma) && la_direct(b, &mb) && la_direct(out, &mx) && !la_meet(out, a, size) && !la_meet(out, b, size);
   if (!direct) {
     void *A, *X;
     if ((rc = work.get((size_t)(p.batch * n * n) * p.esize, &A)) || (rc = work.get((size_t)(p.batch * n * nrhs) * p.esize, &X))) return rc;

@@ -326,6 +326,30 @@ def test_cholesky_over_overlapping_storage(hip, n):
             assert np.array_equal(logical(out), want[upper])
 
 
+@pytest.mark.parametrize("n,nrhs", [(5, 3), (100, 40), (16, 48000)])
+def test_triangular_solve_over_overlapping_storage(hip, n, nrhs):
+    """A result that covers the right-hand sides or the matrix in part, told by base pointers that differ;
+    of 48000 sides most are read only after the first are solved."""
+    rng = np.random.default_rng(n)
+    a, b = np.eye(n) + np.tril(rng.standard_normal((n, n)) / n), rng.standard_normal((n, nrhs))
+    room = n * max(n, nrhs)
+    for upper in (False, True):
+        m = a.T if upper else a
+        want = logical(hip.triangular_solve(put(hip, m, dt.float64), put(hip, b, dt.float64), upper, False, False))
+        for over in ("sides", "matrix"):
+            for shift in (1, 16, nrhs, room // 2):
+                whole = put(hip, np.zeros(4 * room), dt.float64)
+                views = {}
+                for key, at, shape in (("sides", 0, (n, nrhs)), ("matrix", 2 * room, (n, n))):
+                    views[key] = hip.reshape(hip.shrink(whole, [(at, at + shape[0] * shape[1])]), shape)
+                at = shift + (0 if over == "sides" else 2 * room)
+                out = hip.reshape(hip.shrink(whole, [(at, at + n * nrhs)]), (n, nrhs))
+                hip.assign(views["matrix"], put(hip, m, dt.float64))
+                hip.assign(views["sides"], put(hip, b, dt.float64))
+                assert raw_call(hip, "triangular_solve", moved_base(out, 8 * at), views["matrix"], views["sides"], int(upper)) == 0
+                assert np.array_equal(logical(out), want), (upper, over, shift)
+
+
 def test_in_place_and_shared_storage(hip):
     """Results over the operands' own storage, as the C ABI allows."""
     import ctypes as C
