@@ -1183,6 +1183,13 @@ static bool la_direct(const nxh_tensor *t, LaMat *m) {
   return true;
 }
 
+// A result whose elements share an address is refused, as nxh_cast refuses it where results go through that.
+static int la_check_out(const char *op, const nxh_tensor *out) {
+  for (int d = 0; d < out->ndim; d++)
+    if (out->shape[d] > 1 && out->strides[d] == 0) return nxh_fail(NXH_INVALID_ARGUMENT, op, NXH_ERR_OUT_ALIASED);
+  return NXH_OK;
+}
+
 // Whether two tensors of one dtype may share bytes: the ranges from their lowest element to their
 // highest meet. (A base pointer says nothing: offsets may make up for it.)
 static bool la_meet(const nxh_tensor *a, const nxh_tensor *b, int size) {
@@ -1426,6 +1433,7 @@ NXH_EXPORT int nxh_cholesky(nxh_context *ctx, const nxh_tensor *out, const nxh_t
   if (rc) return rc;
   const int64_t n = p.rows;
   if (p.batch == 0 || n == 0) return NXH_OK;
+  if ((rc = la_check_out(op, out))) return rc;
   // one factorisation at a time per context: they share the status word and its host slot
   std::lock_guard<std::mutex> whole_call(ctx->call_mu);
   if ((rc = la_begin(ctx, op))) return rc;
@@ -1470,6 +1478,7 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
   const int64_t n = p.rows, nrhs = b->shape[b->ndim - 1];
   if ((rc = same_dims(op, b, a, n, nrhs)) || (rc = same_dims(op, out, a, n, nrhs))) return rc;
   if (p.batch == 0 || n == 0 || nrhs == 0) return NXH_OK;
+  if ((rc = la_check_out(op, out))) return rc;
   // one factorisation at a time per context: they share the status word and its host slot
   std::lock_guard<std::mutex> whole_call(ctx->call_mu);
   if ((rc = la_begin(ctx, op))) return rc;

@@ -350,6 +350,27 @@ def test_triangular_solve_over_overlapping_storage(hip, n, nrhs):
                 assert np.array_equal(logical(out), want), (upper, over, shift)
 
 
+@pytest.mark.parametrize("name", ["float32", "float64", "complex128", "float16"])
+def test_results_over_one_address_are_refused(hip, name):
+    """A result whose elements share an address (a stride of 0 along more than one of them)."""
+    d = dt.BY_NAME[name]
+    a = put(hip, np.stack([2 * np.eye(6)] * 3).astype(d.np_storage), d)
+    b = put(hip, np.ones((3, 6, 4), d.np_storage), d)
+    for shape in ((1, 6, 6), (3, 1, 6), (3, 6, 1)):
+        out = hip.expand(put(hip, np.full(shape, 7, d.np_storage), d), (3, 6, 6))
+        assert raw_call(hip, "cholesky", out, a, 0) == hip._lib.nxh_cast(hip._h, out._desc(), a._desc()) != 0
+        assert np.all(logical(hip.copy(out)) == 7)
+    for shape in ((1, 6, 4), (3, 1, 4), (3, 6, 1)):
+        out = hip.expand(put(hip, np.full(shape, 7, d.np_storage), d), (3, 6, 4))
+        assert raw_call(hip, "triangular_solve", out, a, b, 0) != 0
+        assert np.all(logical(hip.copy(out)) == 7)
+    one = hip.expand(put(hip, np.full((1, 1, 1), 7, d.np_storage), d), (1, 1, 1))
+    assert raw_call(hip, "cholesky", one, put(hip, np.full((1, 1, 1), 4, d.np_storage), d), 0) == 0 and logical(one)[0, 0, 0] == 2
+    # operands may be read through strides of 0
+    wide = hip.expand(put(hip, (2 * np.eye(6)).astype(d.np_storage).reshape(1, 6, 6), d), (3, 6, 6))
+    assert np.array_equal(logical(hip.cholesky(wide)), logical(hip.cholesky(a)))
+
+
 def test_in_place_and_shared_storage(hip):
     """Results over the operands' own storage, as the C ABI allows."""
     import ctypes as C
