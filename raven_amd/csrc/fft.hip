@@ -70,6 +70,7 @@ struct FftArgs {
   // same element of consecutive lines, so that a wave's accesses are contiguous runs of G
   // elements instead of 64 separate ones. Separately for the load and the store side.
   int in_lines_fast, out_lines_fast;
+  int neighbours;  // lines next to each other in memory, whether a workgroup has several of them or one
   const double2 *tw;       // at len + k: exp(-2 pi i k / len), for every power of two len <= M
   const double2 *real_tw;  // packed lines: exp(-2 pi i k / 2n), k < n
   const double2 *chirp;  // Bluestein: exp(sign pi i j^2 / n), j < n
@@ -369,7 +370,7 @@ __global__ __launch_bounds__(512) void fft_lines_kernel(FftArgs a) {
   // blocks that share an XCD (ids equal modulo 8) take neighbouring groups of lines: with
   // strided lines a 128-byte line of memory serves several workgroups, which then meet in one L2
   uint32_t bx = blockIdx.x;
-  if ((a.in_lines_fast || a.out_lines_fast) && (gridDim.x & 7u) == 0) bx = (bx & 7u) * (gridDim.x >> 3) + (bx >> 3);
+  if (a.neighbours && (gridDim.x & 7u) == 0) bx = (bx & 7u) * (gridDim.x >> 3) + (bx >> 3);
   const int64_t first = (int64_t)bx * a.G;
   int g = threadIdx.x / T, t = threadIdx.x & (T - 1), unused;
   if (a.in_lines_fast) t = threadIdx.x / a.G, g = threadIdx.x - t * a.G;
@@ -640,6 +641,7 @@ static int launch_lines(nxh_context *ctx, FftArgs &a, bool blue) {
   a.out_lines_fast = neighbours(a.out);
   if (a.in_lines_fast || a.out_lines_fast) a.G = std::max(1, std::min(FFT_LDS_MAX / a.M, std::max(16, a.G)));
   if ((int64_t)a.G > a.lines) a.G = (int)a.lines;
+  a.neighbours = a.in_lines_fast || a.out_lines_fast;
   if (a.G == 1) a.in_lines_fast = a.out_lines_fast = 0;
   const int64_t blocks = (a.lines + a.G - 1) / a.G;
   if (blocks > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, "fft", "too many lines for one launch");
