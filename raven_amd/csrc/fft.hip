@@ -71,7 +71,7 @@ struct FftArgs {
   // elements instead of 64 separate ones. Separately for the load and the store side.
   int in_lines_fast, out_lines_fast;
   int neighbours;  // lines next to each other in memory, whether a workgroup has several of them or one
-  const double2 *tw;       // at len + k: exp(-2 pi i k / len), for every power of two len <= M
+  const double2 *tw;       // turns between the passes of length M (twiddle_kernel)
   const double2 *real_tw;  // packed lines: exp(-2 pi i k / 2n), k < n
   const double2 *chirp;  // Bluestein: exp(sign pi i j^2 / n), j < n
   const double2 *bf;     // Bluestein: forward transform (length M) of the wrapped conjugate chirp
@@ -136,7 +136,7 @@ __device__ __forceinline__ double2 fetch(const FftArgs &a, int64_t off, int j) {
 // lane t is element t + T e, before the transform, after it, and at the start of every pass (the
 // self-sorting order: natural in, natural out). A pass does the butterflies of radix R <= E that
 // a lane's own slots make up and then redistributes the line through LDS.
-constexpr int log_elems(int L) { return L >= 8 ? 4 : L >= 6 ? 3 : L >= 4 ? 2 : L >= 1 ? 1 : 0; }
+__host__ __device__ constexpr int log_elems(int L) { return L >= 8 ? 4 : L >= 6 ? 3 : L >= 4 ? 2 : L >= 1 ? 1 : 0; }
 
 // v exp(-2 pi i k / 32), k < 32 known to the compiler
 __device__ __forceinline__ double2 turn(double2 v, int k) {
@@ -207,12 +207,10 @@ __device__ __forceinline__ void exchange(double2 (&x)[E], double *line, const do
 }
 
 // The forward transform of the workgroup's lines, from sub-transforms of length 2^S on. `line` is
-// the lane's own line in LDS. Element (jm, k) of a pass is turned by w^k, w = exp(-2 pi i jm / 2^(S+r)):
-// w, w^2, w^4 and w^8 of the lane's first butterfly are read from the table (neighbouring lanes,
-// neighbouring entries), everything else is a product of those and of constants. The L1 is what
-// table reads cost: with one for each of the R - 1 powers of every butterfly it stalled for two
-// thirds of the kernel's time. The roundings are those of radix-2 stages, which turn an element
-// once a stage.
+// the lane's own line in LDS. Element (jm, k) of a pass is turned by exp(-2 pi i k jm / 2^(S+r)), read
+// from the table at (k << S) + jm: neighbouring lanes, neighbouring entries. (Products of the powers
+// 1, 2, 4 and 8 cost the same and are less exact; one table of roots for all powers, read at strides of
+// k, kept the L1 busy for two thirds of the kernel's time.)
 template <int L, int S>
 __device__ __forceinline__ void fft_passes(double2 (&x)[1 << log_elems(L)], double *line, const double2 *tw, int t) {
   constexpr int E = 1 << log_elems(L), T = (1 << L) / E;
@@ -220,17 +218,10 @@ __device__ __forceinline__ void fft_passes(double2 (&x)[1 << log_elems(L)], doub
   if constexpr (R > 1) {
     if constexpr (S > 0) {
       static_assert(G == 1 || S + r == L, "only the last pass has several butterflies a lane, T apart");
-      const int jm = t & ((1 << S) - 1);
-      double2 w[R];
 #pragma unroll
-      for (int k = 1; k < R; k++) {
-        const int low = k == 3 ? 1 : k & 3;
-        if (low && low != k) w[k] = cmul(w[k - low], w[low]);
-        else if (k == 12) w[k] = cmul(w[k - 4], w[k - 8]);
-        else w[k] = tw[(1 << (S + r)) / k + jm];  // k = 1, 2, 4, 8
+      for (int k = 1; k < R; k++)
 #pragma unroll
-        for (int g = 0; g < G; g++) x[g + k * G] = cmul(x[g + k * G], turn(w[k], g * k * (32 / E)));
-      }
+        for (int g = 0; g < G; g++) x[g + k * G] = cmul(tw[(k << S) + ((t + g * T) & ((1 << S) - 1))], x[g + k * G]);
     }
 #pragma unroll
     for (int g = 0; g < G; g++) dft<R, G>(x, g);
@@ -363,8 +354,9 @@ __device__ __forceinline__ double2 flip(double2 v) { return make_double2(v.y, v.
 // LDS after the load, every four stages and before the store, and read a twiddle per butterfly.
 // Measured: rfft [8192, 2048] float32 170 -> 53 us, irfft back 158 -> 46 us
 // (2.5 TB/s; three waves a SIMD by registers, and the waits of a wave's own chain bound it now).
+// (The convolution of length 512 needs 170 registers when left alone, two more than three waves a SIMD have.)
 template <int L, bool BLUE>
-__global__ __launch_bounds__(512) void fft_lines_kernel(FftArgs a) {
+__global__ __launch_bounds__(512, BLUE && L == 9 ? 3 : 2) void fft_lines_kernel(FftArgs a) {
   extern __shared__ double lds[];
   constexpr int M = 1 << L, E = 1 << log_elems(L), T = M / E, PITCH = M + M / 16 + 1;
   // blocks that share an XCD (ids equal modulo 8) take neighbouring groups of lines: with
@@ -457,13 +449,15 @@ __global__ __launch_bounds__(512) void fft_lines_kernel(FftArgs a) {
 }
 
 // ── tables ──────────────────────────────────────────────────────────────────
-// Entry len + k: exp(-2 pi i k / len), len the powers of two (entry 0 is not used).
-__global__ void twiddle_kernel(double2 *tw, int count) {
+// Of a transform of length 2^L: for each of its passes (sub-transforms of length 2^S become 2^(S+r) long),
+// at (k << S) + j: exp(-2 pi i k j / 2^(S+r)), j < 2^S, 0 < k < 2^r. The first pass has none.
+__global__ void twiddle_kernel(double2 *tw, int L) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  const int len = 1 << (31 - __clz(i | 1)), k = i & (len - 1);
+  if (i >= 1 << L) return;
+  const int e = log_elems(L), S = e ? (31 - __clz(i | 1)) / e * e : 0, top = S + e < L ? S + e : L;
+  const int turns = (i >> S) * (i & ((1 << S) - 1)) & ((1 << top) - 1);
   double sn, cs;
-  sincospi(2.0 * (double)k / (double)len, &sn, &cs);  // an exact argument
+  sincospi(2.0 * (double)turns / (double)(1 << top), &sn, &cs);  // an exact argument
   tw[i] = make_double2(cs, -sn);
 }
 
@@ -594,11 +588,11 @@ static int twiddles(nxh_context *ctx, TableKind kind, int n, const double2 **out
   double2 *t;
   bool fresh;
   const uint64_t key = table_key(kind, n, -1);
-  const int count = kind == T_TWIDDLE ? 2 * n : n / 2;
+  const int count = kind == T_TWIDDLE ? n : n / 2;
   if (int rc = table_lookup(ctx, key, (size_t)count * sizeof(double2), &t, &fresh)) return rc;
   if (fresh) {
     const dim3 grid((count + 255) / 256), block(256);
-    if (kind == T_TWIDDLE) hipLaunchKernelGGL(twiddle_kernel, grid, block, 0, ctx->stream, t, count);
+    if (kind == T_TWIDDLE) hipLaunchKernelGGL(twiddle_kernel, grid, block, 0, ctx->stream, t, log2_of(n));
     else hipLaunchKernelGGL(real_twiddle_kernel, grid, block, 0, ctx->stream, t, n, count);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) {
       table_drop(ctx, key);
