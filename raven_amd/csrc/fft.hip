@@ -40,7 +40,11 @@ constexpr int64_t FFT_WORK_ELEMS = int64_t(1) << 25;  // workspace elements per 
 enum Kind { K_C32 = 0, K_C64 = 1, K_F32 = 2, K_F64 = 3 };
 enum LoadMode { LOAD_COMPLEX = 0, LOAD_REAL = 1, LOAD_HERMITIAN = 2 };
 // Real lines of an even length 2n go as one complex line of length n whose element j is the pair
-// (2j, 2j + 1), at half the arithmetic and LDS of the transform of the real line itself.
+// (2j, 2j + 1), at half the arithmetic and LDS of the transform of the real line itself. Of float64
+// lines only where that is no less exact than radix-2 stages over the whole line: spectra of 512 elements on
+// (error in eps, stages / packed: 16 1.05 / 1.13, 256 1.71 / 1.76, 512 1.84 / 1.81, 5000 4.38 / 4.05), and no
+// inverses (a whole transform drops half its error with the imaginary parts: 2048 1.72 / 1.99, 500 2.78 / 4.02).
+// The rounding of float32 covers all of that.
 enum Pack { PACK_NONE = 0, PACK_RFFT = 1, PACK_IRFFT = 2 };
 
 static inline int kind_size(int k) { return k == K_C32 ? 8 : k == K_C64 ? 16 : k == K_F32 ? 4 : 8; }
@@ -63,7 +67,7 @@ struct FftArgs {
   int n_store;           // (PACK_IRFFT: pairs; PACK_RFFT: bins before the last, which goes by itself)
   int sign;              // -1 forward, +1 inverse
   int pack;              // n is then half the real length
-  int pair_aligned;      // the real side's pairs lie side by side at addresses that are multiples of a pair
+  int pair_aligned;      // the real side's float32 pairs lie side by side at addresses that are multiples of a pair
   int G;                 // lines per workgroup
   // The workgroup's G lines are neighbours in memory while a line's own elements are strided
   // (a transform down the columns of a row-major tensor): consecutive lanes then take the
@@ -273,9 +277,9 @@ __device__ __forceinline__ void load_line(const FftArgs &a, double2 (&x)[E], int
   if (a.pack == PACK_RFFT) {
     const float *pf = (const float *)a.in.base;
     const double *pd = (const double *)a.in.base;
-    if (a.in.kind == K_F32 && a.pair_aligned) each(a.n, 2, [=](int64_t at) { return *(const float2 *)(pf + at); });
-    else if (a.in.kind == K_F32) each(a.n, 2, [=](int64_t at) { return make_float2(pf[at], pf[at + es]); });
-    else each(a.n, 2, [=](int64_t at) { return make_double2(pd[at], pd[at + es]); });
+    if (a.in.kind == K_F64) each(a.n, 2, [=](int64_t at) { return make_double2(pd[at], pd[at + es]); });
+    else if (a.pair_aligned) each(a.n, 2, [=](int64_t at) { return *(const float2 *)(pf + at); });
+    else each(a.n, 2, [=](int64_t at) { return make_float2(pf[at], pf[at + es]); });
   } else if (a.pack == PACK_IRFFT) {
     // The spectrum of the packed line, bins j and n - j at a time. The real part of the whole
     // transform never sees the imaginary parts of bins 0 and n (unless they are no numbers).
@@ -329,12 +333,10 @@ __device__ __forceinline__ void store_line(const FftArgs &a, const double2 (&x)[
       if ((!BLUE || e < (E + 1) / 2) && t + T * e < a.n_store) store(at + e * step, x[e]);
   };
   if (a.pack == PACK_IRFFT) {
-    if (a.out.kind == K_F32 && a.pair_aligned)
+    if (a.pair_aligned)
       each(2, [&](int64_t at, double2 v) { *(float2 *)(a.out.base + at * 4) = make_float2((float)v.x, (float)v.y); });
-    else if (a.out.kind == K_F32)
-      each(2, [&](int64_t at, double2 v) { float *p = (float *)a.out.base + at; p[0] = (float)v.x, p[es] = (float)v.y; });
     else
-      each(2, [&](int64_t at, double2 v) { double *p = (double *)a.out.base + at; p[0] = v.x, p[es] = v.y; });
+      each(2, [&](int64_t at, double2 v) { float *p = (float *)a.out.base + at; p[0] = (float)v.x, p[es] = (float)v.y; });
     return;
   }
   switch (a.out.kind) {
@@ -757,10 +759,10 @@ static int transform_lines(nxh_context *ctx, const Lines &in, const Lines &out, 
                            int load_mode, int64_t n_store, int sign) {
   if (lines == 0 || n == 0 || n_store == 0) return NXH_OK;
   if (n > (int64_t(1) << 26)) return nxh_fail(NXH_FAILURE, "fft", "axis too long (the limit is 2^26 elements)");
-  // real lines of an even length, one side real and the other the half spectrum, go packed
+  // real lines of an even length, one side real and the other the half spectrum, go packed (where exact enough)
   const int pack = n % 2 ? PACK_NONE
-                   : load_mode == LOAD_REAL && n_load == n && n_store == n / 2 + 1 ? PACK_RFFT
-                   : load_mode == LOAD_HERMITIAN && out.kind >= K_F32 && n_store == n && n_load <= n / 2 + 1 ? PACK_IRFFT
+                   : load_mode == LOAD_REAL && (in.kind == K_F32 || n >= 512) && n_load == n && n_store == n / 2 + 1 ? PACK_RFFT
+                   : load_mode == LOAD_HERMITIAN && out.kind == K_F32 && n_store == n && n_load <= n / 2 + 1 ? PACK_IRFFT
                                                                                                           : PACK_NONE;
   const auto conv_length = [](int64_t len) { return is_pow2(len) ? len : int64_t(1) << log2_of(2 * len - 1); };
   FftArgs a{};
@@ -783,8 +785,7 @@ static int transform_lines(nxh_context *ctx, const Lines &in, const Lines &out, 
     n /= 2;
     a.n_store = (int)n;
     const Lines &real = pack == PACK_RFFT ? in : out;
-    const int pair = 2 * kind_size(real.kind);
-    a.pair_aligned = real.estride == 1 && (uintptr_t)real.base % pair == 0;
+    a.pair_aligned = real.kind == K_F32 && real.estride == 1 && (uintptr_t)real.base % sizeof(float2) == 0;
     for (int d = 0; d < real.nd; d++) a.pair_aligned &= real.strides[d] % 2 == 0;
   }
   a.n = (int)n;

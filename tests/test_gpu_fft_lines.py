@@ -35,6 +35,27 @@ def test_complex_lines_are_as_exact_as_exact_turns_make_them(hip, n):
         assert err <= 1.05 * 0.6 * 2.0**-53 * np.sqrt(np.log2(n)), (n, err / 2.0**-53)
 
 
+@pytest.mark.parametrize("n", [1, 2, 7, 16, 50, 64, 500, 510, 512, 1024, 2500, 5000, 8192, 16384])
+def test_real_float64_lines(hip, n):
+    """In float64 a real line that would lose by being packed is transformed as the complex line it is: back
+    from a spectrum always, to one below 512 elements. Above, within what exact turns give (as above)."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((max(3, (1 << 16) // n), n))
+    put = lambda a, d: hip.reshape(hip.from_host(np.ascontiguousarray(a), d), a.shape)
+    line = logical(hip.fft(put(x.astype(np.complex128), dt.complex128), [1]))
+    got = logical(hip.rfft(put(x, dt.float64), dt.complex128, [1]))
+    if n < 512:
+        assert np.array_equal(got, line[:, :n // 2 + 1])
+    elif n & (n - 1) == 0:
+        want = np.fft.rfft(x.astype(np.longdouble), axis=1)
+        err = np.linalg.norm((got - want).astype(np.complex128)) / np.linalg.norm(want.astype(np.complex128))
+        assert err <= 1.05 * 0.6 * 2.0**-53 * np.sqrt(np.log2(n)), err / 2.0**-53
+    half = line[:, :n // 2 + 1]
+    whole = np.concatenate([half, half[:, n - n // 2 - 1:0:-1].conj()], axis=1)
+    back = logical(hip.ifft(put(whole, dt.complex128), [1])).real
+    assert np.array_equal(logical(hip.irfft(put(half, dt.complex128), dt.float64, [1], [n])), back)
+
+
 POWERS = [1 << k for k in range(15)]
 LENGTHS = sorted({*POWERS, *[n + 1 for n in POWERS], *[n - 1 for n in POWERS[1:]], 6, 10, 100, 1000, 2050, 4098, 8190, 8194})
 
