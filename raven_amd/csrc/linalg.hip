@@ -1210,10 +1210,10 @@ static bool la_meet(const nxh_tensor *a, const nxh_tensor *b, int size) {
 // where it returns early.
 struct HostStatus {
   nxh_context *ctx;
-  bool waited = false;
+  bool lent = false, waited = false;  // whether kernels have the word; whether they have been waited for
   explicit HostStatus(nxh_context *c) : ctx(c) { *(volatile int *)word() = LA_OK; }
   ~HostStatus() {
-    if (waited) return;
+    if (!lent || waited) return;
     std::lock_guard<std::mutex> g(ctx->mu);
     (void)hipStreamSynchronize(ctx->stream);
     *(volatile int *)word() = LA_OK;
@@ -1221,6 +1221,10 @@ struct HostStatus {
     (void)hipStreamSynchronize(ctx->stream);
   }
   int *word() const { return ctx->fault_flag_host + 8; }
+  int *lend() {
+    lent = true;
+    return word();
+  }
   // Waits for the kernels of this call (the results included) and reads their report.
   int collect(const char *op) {
     std::lock_guard<std::mutex> g(ctx->mu);
@@ -1234,16 +1238,17 @@ struct HostStatus {
 
 constexpr int64_t LA_GRID_BATCH = 65535;  // matrices per launch (the grid's y and z extent)
 
-template <class T, class TS>
-static int run_cholesky(nxh_context *ctx, const char *op, HostStatus &status, int64_t batch, int n, int upper, LaMat x, LaMat out, void *A,
+template <class T, class TS, int ONE>
+static int run_cholesky_as(nxh_context *ctx, const char *op, HostStatus &status, int64_t batch, int n, int upper, LaMat x, LaMat out, void *A,
                         void *diag) {
-  constexpr int NB = CHOL_NB<T>;
+  using C = Chol<T, ONE>;
+  constexpr int NB = C::NB;
   const int64_t cols = (n + NB - 1) / NB, result_tiles = cols * (cols + 1) / 2;
   if (result_tiles > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "matrix too large for one launch");
-  auto kern = cholesky_block_kernel<T, TS>;
+  auto kern = cholesky_block_kernel<T, TS, ONE>;
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
-  std::call_once(once, [&] { attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CHOL_LDS<T>); });
+  std::call_once(once, [&] { attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS); });
   NXH_HIP(op, attr);
   const auto each_part = [&](auto launch) {  // parts of the batch that a grid holds
     std::lock_guard<std::mutex> g(ctx->mu);
@@ -1257,7 +1262,7 @@ static int run_cholesky(nxh_context *ctx, const char *op, HostStatus &status, in
       a.diag = (T *)diag + (size_t)(b0 * cols) * NB * NB;
       a.n = n;
       a.upper = upper;
-      a.status = status.word();
+      a.status = status.lend();
       launch(a, (unsigned)std::min(LA_GRID_BATCH, batch - b0));
     }
   };
@@ -1265,16 +1270,29 @@ static int run_cholesky(nxh_context *ctx, const char *op, HostStatus &status, in
     for (int s = 0; s < cols; s++) {
       a.s = s;
       const int64_t panels = cols - s, tiles = panels + (s > 0 ? panels * (panels - 1) / 2 : 0);
-      hipLaunchKernelGGL(kern, dim3((unsigned)tiles, nbat), dim3(CHOL_THREADS), CHOL_LDS<T>, ctx->stream, a);
+      hipLaunchKernelGGL(kern, dim3((unsigned)tiles, nbat), dim3(C::THREADS), C::LDS, ctx->stream, a);
     }
   });
   if (int rc = status.collect(op)) return rc;  // a matrix that has no factor leaves `out` as it was
   each_part([&](CholArgs<T> &a, unsigned nbat) {
-    hipLaunchKernelGGL((cholesky_result_kernel<T, TS>), dim3((unsigned)result_tiles, nbat), dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL((cholesky_result_kernel<T, TS, ONE>), dim3((unsigned)result_tiles, nbat), dim3(256), 0, ctx->stream, a);
   });
   NXH_HIP(op, hipGetLastError());
   return NXH_OK;
 }
+
+template <class T, class TS>
+static int run_cholesky(nxh_context *ctx, const char *op, HostStatus &status, int64_t batch, int n, int upper, LaMat x, LaMat out, void *A,
+                        void *diag) {
+  const auto run = n <= Chol<T, 1>::NB ? run_cholesky_as<T, TS, 1> : n <= Chol<T, 2>::NB ? run_cholesky_as<T, TS, 2> : run_cholesky_as<T, TS, 0>;
+  return run(ctx, op, status, batch, n, upper, x, out, A, diag);
+}
+
+// Where the small forms of complex systems are the faster ones: from a few hundred matrices on. Measured
+// (us, small / in blocks): factors of [256,64,64] 262 / 122, [1024,17,17] 57 / 103, [2048,64,64] 615 / 836; a solve with
+// 16 sides of [256,32,32] 59 / 38, [1024,17,17] 53 / 105, [2048,64,64] 391 / 394, with one side 150 / 395. Up
+// to 16 rows a block is one wave and the faster form throughout.
+static bool la_many_small(bool complex, int64_t batch, int64_t n) { return complex && batch >= 512 && n > 16 && n <= 64; }
 
 // Rows of a pass: what the LDS holds of sixteen right-hand sides beside the triangles.
 template <class T>
@@ -1286,10 +1304,13 @@ template <class T, class TS>
 static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool direct, int64_t batch, int n, int nrhs, int flags, LaMat m,
                     LaMat b, LaMat x) {
   const bool upper = flags & 1, transpose = (flags >> 1) & 1, forward = upper == transpose;
-  auto kern = trsm_block_kernel<T, TS>;
+  const auto most = trsm_block_kernel<T, TS, TRSM_TILES>, few = trsm_block_kernel<T, TS, TRSM_FEW>, one = trsm_block_kernel<T, TS, 0>;
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
-  std::call_once(once, [&] { attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, TRSM_PASS<T> * 16 * (int)sizeof(T)); });
+  std::call_once(once, [&] {
+    for (const auto kern : {most, few})
+      if (attr == hipSuccess) attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, TRSM_PASS<T> * 16 * (int)sizeof(T));
+  });
   NXH_HIP(op, attr);
   // in solution order: row t of the solution is matrix row t, or n - 1 - t backwards
   int64_t ts = transpose ? m.cs : m.rs, us = transpose ? m.rs : m.cs;
@@ -1309,7 +1330,7 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
     a.us = us;
     a.mbs = m.bs;
     a.rows = n;
-    a.status = status.word();
+    a.status = status.lend();
     hipLaunchKernelGGL((trsm_check_kernel<T, TS>), dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, ctx->stream, a, batch, la_status(ctx));
   }
   for (int64_t b0 = 0; b0 < batch; b0 += LA_GRID_BATCH) {
@@ -1326,10 +1347,12 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
       a.x = LaMat{xp + b0 * x.bs + r0 * x.rs, x.rs, x.cs, x.bs};
       a.rows = std::min(n - r0, TRSM_PASS<T>);
       a.nrhs = nrhs;
-      a.status = status.word();
+      a.status = status.lend();
       a.hold = check ? la_status(ctx) : nullptr;
       const int nb = (a.rows + 15) / 16;
-      hipLaunchKernelGGL(kern, dim3(groups, nbat), dim3(64 * TRSM_WAVES), (size_t)nb * 256 * sizeof(T), ctx->stream, a);
+      const auto kern = nb == 1 ? one : sizeof(T) == 8 && nb <= 2 + TRSM_UPDATERS * TRSM_FEW ? few : most;  // (complex reads nothing ahead)
+      const int threads = nb == 1 ? TRSM_THREADS<0> : TRSM_THREADS<TRSM_FEW>;
+      hipLaunchKernelGGL(kern, dim3(groups, nbat), dim3(threads), (size_t)nb * 256 * sizeof(T), ctx->stream, a);
       const int rest = n - r0 - a.rows;
       if (rest > 0)
         hipLaunchKernelGGL((trsm_rest_kernel<T, TS>), dim3(groups, (unsigned)((rest + 63) / 64), nbat), dim3(256), 0, ctx->stream, a,
@@ -1441,7 +1464,16 @@ NXH_EXPORT int nxh_cholesky(nxh_context *ctx, const nxh_tensor *out, const nxh_t
   Work work(ctx);
   PathAtExit path{n >= LA_WIDE_FROM ? "cholesky_columns_wide" : "cholesky_columns"};
   const size_t mat = (size_t)(p.batch * n * n) * p.esize;
-  const int64_t nb = p.cx ? CHOL_NB<c64> : CHOL_NB<double>;
+  if (la_many_small(p.cx, p.batch, n)) {
+    void *A;
+    if ((rc = work.get(mat, &A))) return rc;
+    nxh_tensor wa = workspace_tensor(x, A, p.wdt, n, n, false);
+    if ((rc = nxh_cast(ctx, &wa, x))) return rc;
+    LA_LAUNCH(ctx, cholesky_small_kernel<c64>, p.batch, 0, (c64 *)A, (int)n, upper, la_status(ctx));
+    if ((rc = la_collect(ctx, op))) return rc;
+    return nxh_cast(ctx, out, &wa);
+  }
+  const int64_t nb = n <= Chol<double, 1>::NB ? Chol<double, 1>::NB : n <= Chol<double, 2>::NB ? Chol<double, 2>::NB : p.cx ? Chol<c64, 0>::NB : Chol<double, 0>::NB;
   void *A, *diag, *io;
   if ((rc = work.get(mat, &A)) || (rc = work.get((size_t)(p.batch * ((n + nb - 1) / nb) * nb * nb) * p.esize, &diag))) return rc;
   LaMat mx{}, mo{};
@@ -1487,10 +1519,11 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
   PathAtExit path{n >= LA_WIDE_FROM ? "triangular_substitution_wide" : "triangular_substitution"};
   LaMat ma{}, mb{}, mx{};
   nxh_tensor wx{};
+  const bool small = la_many_small(p.cx, p.batch, n);
   const int pass = p.cx ? TRSM_PASS<c64> : TRSM_PASS<double>;
   // the result may be written while other workgroups read: only where it is apart from what they read
   const int size = a->dtype == NXH_F32 ? 4 : a->dtype == NXH_F64 ? 8 : 16;
-  const bool direct = n <= pass && la_direct(a, &ma) && la_direct(b, &mb) && la_direct(out, &mx) && !la_meet(out, a, size) && !la_meet(out, b, size);
+  const bool direct = !small && n <= pass && la_direct(a, &ma) && la_direct(b, &mb) && la_direct(out, &mx) && !la_meet(out, a, size) && !la_meet(out, b, size);
   if (!direct) {
     void *A, *X;
     if ((rc = work.get((size_t)(p.batch * n * n) * p.esize, &A)) || (rc = work.get((size_t)(p.batch * n * nrhs) * p.esize, &X))) return rc;
@@ -1499,6 +1532,12 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
     if ((rc = nxh_cast(ctx, &wa, a)) || (rc = nxh_cast(ctx, &wx, b))) return rc;
     ma = LaMat{A, n, 1, n * n};
     mb = mx = LaMat{X, nrhs, 1, n * nrhs};
+  }
+  if (small) {
+    LA_LAUNCH(ctx, trsm_small_kernel<c64>, p.batch, 0, (const c64 *)ma.p, (c64 *)mx.p, (int)n, (int)nrhs, flags & 1, (flags >> 1) & 1,
+              (flags >> 2) & 1, la_status(ctx));
+    if ((rc = la_collect(ctx, op))) return rc;
+    return nxh_cast(ctx, out, &wx);
   }
   if (p.cx) rc = run_trsm<c64, c64>(ctx, op, status, direct, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);
   else if (direct && a->dtype == NXH_F32) rc = run_trsm<double, float>(ctx, op, status, direct, p.batch, (int)n, (int)nrhs, flags, ma, mb, mx);

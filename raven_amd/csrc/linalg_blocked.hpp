@@ -267,15 +267,19 @@ __device__ __forceinline__ bool factor16_columns(double *tile, int ld, double *i
 // updates and factors the next sixteen while the others update the rest and this workgroup's own
 // tile follows, a wave per sixteen rows, one block of columns behind. Complex matrices, with no matrix
 // instruction for them, are factored column by column, a row a lane.
-constexpr int CHOL_THREADS = 512, CHOL_WAVES = CHOL_THREADS / 64;
-template <class T>
-constexpr int CHOL_NB = sizeof(T) == 8 ? 64 : 32;
-constexpr int CHOL_COLUMN = 80;                 // complex: 64 values of one column, and room for reads past them
-constexpr int CHOL_OPERANDS = 128 + 3 * 4 * 256;  // double: factor16's scratch, the operands of solve16 for four blocks of columns, diag_sum
-// four tiles of pitch NB + 2 (66 doubles: sixteen rows on different banks), then those
-template <class T>
-constexpr size_t CHOL_LDS = 4 * CHOL_NB<T> * (CHOL_NB<T> + 2) * sizeof(T) +
-                            (sizeof(T) == 8 ? CHOL_OPERANDS * sizeof(double) : CHOL_COLUMN * sizeof(T) + CHOL_NB<T> * sizeof(double));
+// Matrices of ONE blocks of sixteen columns, 1 or 2, are a single tile: a wave per block, and the LDS of
+// one tile, so that a compute unit holds several. (0: any size, eight waves and four tiles, one
+// workgroup a unit: float64 factors of [16384,16,16] in 361 us against 66, of [1024,17,17] in 57 against 29; the
+// form for one workgroup per matrix in a workspace took 281 and 52.)
+template <class T, int ONE>
+struct Chol {
+  static constexpr int NB = ONE ? 16 * ONE : sizeof(T) == 8 ? 64 : 32, BLOCKS = NB / 16;
+  static constexpr int THREADS = ONE ? 64 * ONE : 512, WAVES = THREADS / 64;
+  static constexpr int LD = NB + 2;                        // 66 doubles: sixteen rows on different banks
+  static constexpr int COLUMN = 80;                        // complex: 64 values of one column, and room for reads past them
+  static constexpr int OPERANDS = 128 + 3 * BLOCKS * 256;  // double: factor16's scratch, the operands of solve16, diag_sum
+  static constexpr size_t LDS = (ONE ? 1 : 4) * NB * LD * sizeof(T) + (sizeof(T) == 8 ? OPERANDS * sizeof(double) : COLUMN * sizeof(T) + NB * sizeof(double));
+};
 
 template <class T>
 struct CholArgs {
@@ -286,16 +290,18 @@ struct CholArgs {
   int *status;
 };
 
-template <class T, class TS>
-__global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T> a) {
+template <class T, class TS, int ONE>
+__global__ __launch_bounds__((Chol<T, ONE>::THREADS)) void cholesky_block_kernel(CholArgs<T> a) {
   using S = Sc<T>;
-  constexpr int NB = CHOL_NB<T>, LD = NB + 2, TILES = NB / 16;
+  using C = Chol<T, ONE>;
+  constexpr int NB = C::NB, LD = C::LD, TILES = C::BLOCKS;
   extern __shared__ double lds_raw[];
-  T *D = (T *)lds_raw, *own = D + NB * LD;  // the diagonal tile, this workgroup's
-  T *ls = own + NB * LD, *li = ls + NB * LD;  // block column s - 1 in the rows of tile (s, .) and of tile (i, .)
-  T *column = li + NB * LD;
-  double *inv = (double *)(column + CHOL_COLUMN);
-  double *blk = (double *)(li + NB * LD), *op_inv = blk + 128, *op_tri = op_inv + 4 * 256, *diag_sum = op_tri + 4 * 256;
+  T *D = (T *)lds_raw;  // the diagonal tile
+  T *column = D + NB * LD;
+  double *inv = (double *)(column + C::COLUMN);
+  double *blk = (double *)(D + NB * LD), *op_inv = blk + 128, *op_tri = op_inv + TILES * 256, *diag_sum = op_tri + TILES * 256;
+  // ONE has neither of these: this workgroup's tile, block column s - 1 in the rows of tile (s, .) and of tile (i, .)
+  T *own = (T *)((char *)lds_raw + C::LDS) - 3 * NB * LD, *ls = own + NB * LD, *li = ls + NB * LD;
   const int n = a.n, s = a.s, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
   const int panels = (n + NB - 1) / NB - s;  // block rows from s down
   int i, j;
@@ -331,13 +337,13 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
     *tr = t / TILES, *tc = t % TILES;
     return t < ALL && (!panel || (has_own && !OWN_LATER)) && i * NB + *tr * 16 < n && j * NB + *tc * 16 < n && (i != j || *tc <= *tr);
   };
-  constexpr int MOST = OWN_LATER ? ALL : ALL + LOWER, JOBS = (MOST + CHOL_WAVES - 1) / CHOL_WAVES;
+  constexpr int MOST = OWN_LATER ? ALL : ALL + LOWER, JOBS = (MOST + C::WAVES - 1) / C::WAVES;
   LaTile<T> acc[JOBS];
   LaTile<TS> raw[JOBS];  // (converted only once it is used: a conversion would wait for its load)
 #pragma unroll
   for (int e = 0; e < JOBS; e++) {  // every load is on its way before the first is waited for
     int diag, tr, tc;
-    if (!job(e * CHOL_WAVES + wave, &diag, &tr, &tc)) continue;
+    if (!job(e * C::WAVES + wave, &diag, &tr, &tc)) continue;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       const int r = (diag ? s : i) * NB + tr * 16 + 4 * v + q, c = j * NB + tc * 16 + r16;
@@ -349,14 +355,14 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
   // diagonal in the place of its mirror image, transposed; for one on the diagonal in diag_sum.
   auto taken_at = [&](int tr, int tc) { return (double *)(tr == tc ? diag_sum + tr * 256 + q * 16 + r16 : (double *)D + (tc * 16 + r16) * LD + tr * 16 + q); };
   auto taken_step = [](int tr, int tc) { return tr == tc ? 64 : 4; };
-  constexpr int PER = NB * NB / CHOL_THREADS;
+  constexpr int PER = NB * NB / C::THREADS;
   const int col_of = threadIdx.x % NB, row_of = threadIdx.x / NB;
   TS mine[PER];
   T mine_taken[PER];
   if (OWN_LATER && panel && has_own) {
 #pragma unroll
     for (int e = 0; e < PER; e++) {
-      const int r = i * NB + row_of + e * (CHOL_THREADS / NB), c = s * NB + col_of;
+      const int r = i * NB + row_of + e * (C::THREADS / NB), c = s * NB + col_of;
       mine[e] = element(r, c);
       mine_taken[e] = taken_before(r, c);
     }
@@ -366,13 +372,13 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
     const int c = col_of, r0 = row_of;
 #pragma unroll
     for (int e = 0; e < PER; e++) {
-      const int r = r0 + e * (CHOL_THREADS / NB);
+      const int r = r0 + e * (C::THREADS / NB);
       vj[e] = A[(size_t)min(j * NB + r, n - 1) * n + (s - 1) * NB + c];
       vi[e] = A[(size_t)min(i * NB + r, n - 1) * n + (s - 1) * NB + c];
     }
 #pragma unroll
     for (int e = 0; e < PER; e++) {
-      const int r = r0 + e * (CHOL_THREADS / NB);
+      const int r = r0 + e * (C::THREADS / NB);
       ls[r * LD + c] = vj[e];
       li[r * LD + c] = vi[e];
     }
@@ -381,7 +387,7 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
 #pragma unroll
   for (int e = 0; e < JOBS; e++) {
     int diag, tr, tc;
-    if (!job(e * CHOL_WAVES + wave, &diag, &tr, &tc)) continue;
+    if (!job(e * C::WAVES + wave, &diag, &tr, &tc)) continue;
     if (s > 0) tile_sub<NB>(acc[e], (diag ? ls : li) + tr * 16 * LD, LD, ls + tc * 16 * LD, LD);
 #pragma unroll
     for (int v = 0; v < 4; v++) {
@@ -400,7 +406,7 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
   }
   if (OWN_LATER && panel && has_own) {
 #pragma unroll
-    for (int e = 0; e < PER; e++) own[(row_of + e * (CHOL_THREADS / NB)) * LD + col_of] = T(mine[e]) + mine_taken[e];
+    for (int e = 0; e < PER; e++) own[(row_of + e * (C::THREADS / NB)) * LD + col_of] = T(mine[e]) + mine_taken[e];
   }
   if (!panel) return;
   __syncthreads();
@@ -551,7 +557,7 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
       }
       __syncthreads();
       // what the new columns take from the rest of the diagonal tile
-      for (int t = wave; t < TILES * TILES; t += CHOL_WAVES) {
+      for (int t = wave; t < TILES * TILES; t += C::WAVES) {
         const int tr = t / TILES, tc = t % TILES;
         if (tc <= jb || tc > tr || tr >= blocks) continue;
         LaTile<T> d;
@@ -569,13 +575,13 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
   __syncthreads();
   const int rows = min(n - i * NB, NB);
   if (has_own) {
-    for (int e = threadIdx.x; e < NB * NB; e += CHOL_THREADS) {
+    for (int e = threadIdx.x; e < NB * NB; e += C::THREADS) {
       const int r = e / NB, c = e % NB;
       if (r < rows) A[(size_t)(i * NB + r) * n + s * NB + c] = own[r * LD + c];  // (a tile below the diagonal has all its columns)
     }
   } else {
     T *to = a.diag + ((size_t)blockIdx.y * (s + panels) + s) * NB * NB;
-    for (int e = threadIdx.x; e < NB * NB; e += CHOL_THREADS) {
+    for (int e = threadIdx.x; e < NB * NB; e += C::THREADS) {
       const int r = e / NB, c = e % NB;
       if (r < left && c <= r) to[e] = D[r * LD + c];
     }
@@ -583,10 +589,10 @@ __global__ __launch_bounds__(CHOL_THREADS) void cholesky_block_kernel(CholArgs<T
 }
 
 // The result with its zeros, a workgroup per tile (i, j), i >= j, and its mirror image. U = L^H.
-template <class T, class TS>
+template <class T, class TS, int ONE>
 __global__ __launch_bounds__(256) void cholesky_result_kernel(CholArgs<T> a) {
   using S = Sc<T>;
-  constexpr int NB = CHOL_NB<T>;
+  constexpr int NB = Chol<T, ONE>::NB;
   __shared__ T tile[NB][NB + 1];
   const int n = a.n, cols = (n + NB - 1) / NB;
   int i = 0, j = blockIdx.x;
@@ -623,8 +629,14 @@ __global__ __launch_bounds__(256) void cholesky_result_kernel(CholArgs<T> a) {
 // Where solve16 refuses, and for complex matrices, the substitution goes row by row, a right-hand
 // side a lane.
 // Wave 0 is the chain, wave 4 (of its SIMD) reads and inverts triangles, which takes no matrix
-// instructions from it, the other six bring up to TRSM_TILES tiles each up to date per step: 64 in a pass.
-constexpr int TRSM_WAVES = 8, TRSM_LOADER = 4, TRSM_UPDATERS = 6, TRSM_TILES = 11;
+// instructions from it, the other six bring up to TILES tiles each up to date per step. What a tile needs
+// of the matrix is in registers two steps ahead, so that TILES decides how many workgroups a compute unit
+// holds (float64: 11 tiles 208 registers, one; 2 tiles 128, two). Eleven make a pass of 64 blocks; systems of
+// 2 + 6 TILES blocks and fewer take two; those of one block, TILES = 0, a single wave, which places
+// the triangle itself.
+constexpr int TRSM_WAVES = 8, TRSM_LOADER = 4, TRSM_UPDATERS = 6, TRSM_TILES = 11, TRSM_FEW = 2;
+template <int TILES>
+constexpr int TRSM_THREADS = TILES > 0 ? 64 * TRSM_WAVES : 64;
 
 template <class T>
 struct TrsmArgs {
@@ -656,16 +668,17 @@ __device__ __forceinline__ T trsm_coefficient(const TrsmArgs<T> &a, const TS *m,
   return a.conj ? Sc<T>::conj(v) : v;
 }
 
-template <class T, class TS>
-__global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T> a) {
+template <class T, class TS, int TILES>
+__global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) void trsm_block_kernel(TrsmArgs<T> a) {
   using S = Sc<T>;
+  constexpr int AHEAD = TILES > 0 ? 2 : 1;  // triangles in LDS
   extern __shared__ double lds_raw[];
   T *X = (T *)lds_raw;  // rows rounded up to 16, times 16
   // by columns, each from its diagonal on: element r < 16 of column t is coefficient (t + r, t), element
   // 16 (double) the inverse of the diagonal (reads past a column's end meet the next one: their results are dropped)
   constexpr int TRI_LD = 18;
-  __shared__ T tri[2][17][TRI_LD];
-  __shared__ double diag_inv[2][4][64];  // operands of solve16, zero outside the 4 x 4 triangles
+  __shared__ T tri[AHEAD][17][TRI_LD];
+  __shared__ double diag_inv[AHEAD][4][64];  // operands of solve16, zero outside the 4 x 4 triangles
   __shared__ int singular;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
   const int n = a.rows, nb = (n + 15) / 16, col0 = blockIdx.x * 16;
@@ -689,17 +702,17 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
       const bool diagonal = t == r16;
       T val = a.conj ? S::conj(T(raw[v])) : T(raw[v]);
       if (k * 16 + max(t, r16) >= n || r16 > t || (a.unit && diagonal)) val = S::make(diagonal ? 1.0 : 0.0, 0.0);
-      if (r16 <= t) tri[k & 1][r16][t - r16] = val;
+      if (r16 <= t) tri[k % AHEAD][r16][t - r16] = val;
       if (diagonal) {
         if (val == S::make(0.0, 0.0)) singular = 1;
-        if constexpr (sizeof(T) == 8) tri[k & 1][t][16] = 1.0 / val;
+        if constexpr (sizeof(T) == 8) tri[k % AHEAD][t][16] = 1.0 / val;
       }
     }
     if constexpr (sizeof(T) == 8) {
       // lane (b, i, j): element (i, j) of the inverse of the b-th 4 x 4 triangle on the diagonal
       __builtin_amdgcn_wave_barrier();
       const int bb = lane >> 4, i = (lane >> 2) & 3, j = lane & 3;
-      const T(*t)[TRI_LD] = &tri[k & 1][4 * bb];
+      const T(*t)[TRI_LD] = &tri[k % AHEAD][4 * bb];
       const double e0 = t[0][16], e1 = t[1][16], e2 = t[2][16], e3 = t[3][16];
       const double m10 = -e1 * t[0][1] * e0, m21 = -e2 * t[1][1] * e1, m32 = -e3 * t[2][1] * e2;
       const double m20 = -e2 * fma(t[1][1], m10, t[0][2] * e0), m31 = -e3 * fma(t[2][1], m21, t[1][2] * e1);
@@ -707,17 +720,17 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
       double v = i == 0 ? e0 : i == 1 ? (j == 0 ? m10 : e1) : i == 2 ? (j == 0 ? m20 : j == 1 ? m21 : e2)
                                                                      : (j == 0 ? m30 : j == 1 ? m31 : j == 2 ? m32 : e3);
       v = j <= i ? v : 0.0;
-      diag_inv[k & 1][bb][j * 16 + 4 * bb + i] = v;
+      diag_inv[k % AHEAD][bb][j * 16 + 4 * bb + i] = v;
     }
   };
-  for (int e = threadIdx.x; e < 512; e += blockDim.x) (&diag_inv[0][0][0])[e] = 0.0;
+  for (int e = threadIdx.x; e < AHEAD * 256; e += blockDim.x) (&diag_inv[0][0][0])[e] = 0.0;
   __syncthreads();
   TS raw[2][4];
-  if (wave == TRSM_LOADER) {
+  if (TILES == 0 || wave == TRSM_LOADER) {
     fetch_triangle(0, raw[0]);
-    fetch_triangle(1, raw[1]);
+    if (TILES > 0) fetch_triangle(1, raw[1]);
     place_triangle(0, raw[0]);
-    fetch_triangle(2, raw[0]);
+    if (TILES > 0) fetch_triangle(2, raw[0]);
   }
   // coefficients of tile `t` against block `u`, as the matrix instruction takes them
   const TS *lane_full = m + r16 * a.ts + q * a.us, *lane_last = m + min(r16, n - 1 - (nb - 1) * 16) * a.ts + q * a.us;
@@ -765,7 +778,7 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
   // the matrix is needed two steps later and has two sets of registers in turn (a copy from one
   // to the other would wait for it): the first pass over it comes from beyond the L2, some 3500
   // cycles away.
-  if (wave == 0) {
+  if (TILES == 0 || wave == 0) {
     TS left[2][4], on[2][4];  // of the tile left of the triangle, and of the triangle
     auto step = [&](int k, TS(&cl)[4], TS(&co)[4]) {
       LaTile<T> acc = load_rows(k);
@@ -781,7 +794,7 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
         if (k + 2 < nb) coefficients(k + 2, k + 2, co);
         double di[4];
 #pragma unroll
-        for (int v = 0; v < 4; v++) di[v] = diag_inv[k & 1][v][lane];
+        for (int v = 0; v < 4; v++) di[v] = diag_inv[k % AHEAD][v][lane];
         if (solve16(acc, di, tr)) {
           store_rows(k, acc);
           return;
@@ -789,7 +802,7 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
       }
       store_rows(k, acc);
       __builtin_amdgcn_wave_barrier();
-      const T(*t16)[TRI_LD] = tri[k & 1];
+      const T(*t16)[TRI_LD] = tri[k % AHEAD];
       T v[16];  // this lane's right-hand side from row t on; it moves up one place with every row
 #pragma unroll
       for (int t = 0; t < 16; t++) v[t] = X[(k * 16 + t) * 16 + r16];
@@ -826,20 +839,20 @@ __global__ __launch_bounds__(64 * TRSM_WAVES) void trsm_block_kernel(TrsmArgs<T>
         __syncthreads();
       }
     }
-  } else {
+  } else if constexpr (TILES > 0) {
     const int first = wave < TRSM_LOADER ? wave : wave - 1;  // 1 .. TRSM_UPDATERS
-    TS c[2][TRSM_TILES][4];
-    auto request = [&](int k, TS(&to)[TRSM_TILES][4]) {  // what step `k` takes
+    TS c[2][TILES][4];
+    auto request = [&](int k, TS(&to)[TILES][4]) {  // what step `k` takes
 #pragma unroll
-      for (int i = 0; i < TRSM_TILES; i++) {
+      for (int i = 0; i < TILES; i++) {
         const int t = k + first + i * TRSM_UPDATERS;
         if (t < nb) coefficients(t, k - 1, to[i]);
       }
     };
-    auto step = [&](int k, TS(&from)[TRSM_TILES][4]) {
+    auto step = [&](int k, TS(&from)[TILES][4]) {
       if (k > 0) {
 #pragma unroll
-        for (int i = 0; i < TRSM_TILES; i++) {
+        for (int i = 0; i < TILES; i++) {
           const int t = k + first + i * TRSM_UPDATERS;
           if (t < nb) {
             LaTile<T> acc = load_rows(t);
@@ -898,4 +911,78 @@ __global__ __launch_bounds__(256) void trsm_rest_kernel(TrsmArgs<T> a, LaMat res
 #pragma unroll
   for (int v = 0; v < 4; v++)
     if (t0 + 4 * v + q < rest_rows) to_storage(acc[v], y + (t0 + 4 * v + q) * rest.rs + c * rest.cs);
+}
+
+// ── many small complex systems ──────────────────────────────────────────────
+// The complex forms above are chains of one wave, with no matrix instruction to shorten them; a thousand of
+// them queue up. Matrices of up to 64 rows then take a workgroup each whose lanes share every link: a
+// column of the factor with a row a lane; a row of the solution, then its elimination from the others,
+// with an element a lane. In place in a workspace of the compute type.
+template <class T>
+__global__ __launch_bounds__(LA_THREADS) void cholesky_small_kernel(T *all, int n, int upper, int *status) {
+  using S = Sc<T>;
+  T *A = all + (size_t)blockIdx.x * n * n;
+  __shared__ int failed;
+  if (threadIdx.x == 0) failed = 0;
+  for (int j = 0; j < n; j++) {
+    for (int i = j + threadIdx.x; i < n; i += blockDim.x) {
+      T s = A[(size_t)i * n + j];
+      const T *ri = A + (size_t)i * n, *rj = A + (size_t)j * n;
+      for (int k = 0; k < j; k++) s = s - ri[k] * S::conj(rj[k]);
+      A[(size_t)i * n + j] = s;
+    }
+    __syncthreads();
+    const double d = S::re(A[(size_t)j * n + j]);
+    if (threadIdx.x == 0 && !(d > 0.0)) failed = 1;
+    __syncthreads();
+    if (failed) {
+      if (threadIdx.x == 0) raise(status, LA_NOT_PD);
+      return;
+    }
+    const double l = sqrt(d);
+    for (int i = j + threadIdx.x; i < n; i += blockDim.x)
+      A[(size_t)i * n + j] = i == j ? S::make(l, 0.0) : S::scale(A[(size_t)i * n + j], 1.0 / l);
+    __syncthreads();
+  }
+  // the other triangle: zero for L; for U the conjugate transpose moves there first
+  for (int64_t e = threadIdx.x; e < (int64_t)n * n; e += blockDim.x) {
+    const int i = (int)(e / n), k = (int)(e % n);
+    if (i <= k) continue;
+    if (upper) {
+      A[(size_t)k * n + i] = S::conj(A[e]);
+      A[e] = S::make(0.0, 0.0);
+    } else {
+      A[(size_t)k * n + i] = S::make(0.0, 0.0);
+    }
+  }
+}
+
+template <class T>
+__global__ __launch_bounds__(LA_THREADS) void trsm_small_kernel(const T *a_all, T *x_all, int n, int nrhs, int upper,
+                                                                int transpose, int unit, int *status) {
+  using S = Sc<T>;
+  const T *A = a_all + (size_t)blockIdx.x * n * n;
+  T *X = x_all + (size_t)blockIdx.x * n * nrhs;
+  const bool forward = (upper != 0) == (transpose != 0);
+  for (int ii = 0; ii < n; ii++) {
+    const int i = forward ? ii : n - 1 - ii;
+    if (!unit) {
+      T diag = A[(size_t)i * n + i];
+      if (transpose) diag = S::conj(diag);
+      if (diag == S::make(0.0, 0.0)) {  // uniform: every lane reads the same element
+        if (threadIdx.x == 0) raise(status, LA_SINGULAR);
+        return;
+      }
+      for (int j = threadIdx.x; j < nrhs; j += blockDim.x) X[(size_t)i * nrhs + j] = X[(size_t)i * nrhs + j] / diag;
+      __syncthreads();
+    }
+    const int rest = n - 1 - ii;  // rows not yet solved
+    for (int64_t e = threadIdx.x; e < (int64_t)rest * nrhs; e += blockDim.x) {
+      const int rr = (int)(e / nrhs), j = (int)(e % nrhs);
+      const int r = forward ? i + 1 + rr : i - 1 - rr;
+      const T m = transpose ? S::conj(A[(size_t)i * n + r]) : A[(size_t)r * n + i];
+      X[(size_t)r * nrhs + j] = X[(size_t)r * nrhs + j] - m * X[(size_t)i * nrhs + j];
+    }
+    __syncthreads();
+  }
 }

@@ -256,6 +256,41 @@ def test_first_call_of_a_context(hip):
     assert np.array_equal(logical(fresh.cholesky(put(fresh, a, dt.float64))), low)
 
 
+@pytest.mark.parametrize("name", ["float32", "float64", "complex128", "complex64"])
+@pytest.mark.parametrize("batch,n", [(511, 17), (512, 17), (512, 64), (512, 65), (700, 16), (700, 1), (513, 33)])
+def test_many_small_systems(hip, name, batch, n):
+    """Either side of the number and the size of matrices where the form changes: every matrix as alone,
+    within the bound of either (4 n eps of the magnitudes summed), failures of one of them as of one."""
+    d, rng = dt.BY_NAME[name], np.random.default_rng(batch + n)
+    eps = {"complex64": 2.0 ** -24}.get(name) or EPS[name]
+    g = draws(rng, (batch, n, n), name)
+    wide = np.complex128 if d.is_complex else np.float64
+    a = (g @ H(g) + n * np.eye(n)).astype(d.np_storage)
+    a[..., np.arange(n), np.arange(n)] = a[..., np.arange(n), np.arange(n)].real
+    full = np.tril(a).astype(wide) + H(np.tril(a, -1)).astype(wide)
+    for upper in (False, True):
+        f = logical(hip.cholesky(put(hip, a, d), upper)).astype(wide)
+        low = H(f) if upper else f
+        assert np.all(np.triu(low, 1) == 0)
+        assert np.all(np.abs(low @ H(low) - full) <= (4 * n * 2.0 ** -53 + 3 * eps) * (np.abs(low) @ np.abs(H(low))))
+    t = np.tril(draws(rng, (batch, n, n), name) / np.sqrt(n) + 2 * np.eye(n)).astype(d.np_storage)
+    b = draws(rng, (batch, n, 5), name).astype(d.np_storage)
+    for transpose in (False, True):
+        for unit in (False, True):
+            m = t.astype(wide)
+            if unit:
+                m[..., np.arange(n), np.arange(n)] = 1
+            m = H(m) if transpose else m
+            x = logical(hip.triangular_solve(put(hip, t, d), put(hip, b, d), False, transpose, unit)).astype(wide)
+            assert np.all(np.abs(m @ x - b) <= (4 * n * 2.0 ** -53 + 2 * eps) * (np.abs(m) @ np.abs(x)) + 4 * n * 2.0 ** -53)
+    out = put(hip, np.full((batch, n, n), 7, d.np_storage), d)
+    a[batch - 3, n - 1, n - 1] = -1
+    assert raw_call(hip, "cholesky", out, put(hip, a, d), 0) != 0 and np.all(logical(out) == 7)
+    t[batch - 3, n - 1, n - 1] = 0
+    sides = put(hip, b, d)
+    assert raw_call(hip, "triangular_solve", sides, put(hip, t, d), sides, 0) != 0 and np.array_equal(logical(sides), b)
+
+
 def raw_call(hip, name, out, *args):
     """The C entry itself, the result over storage of the caller's choice."""
     return getattr(hip._lib, "nxh_" + name)(hip._h, out._desc(), *[a._desc() if hasattr(a, "_desc") else a for a in args])
