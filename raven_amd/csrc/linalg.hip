@@ -1462,9 +1462,10 @@ NXH_EXPORT int nxh_cholesky(nxh_context *ctx, const nxh_tensor *out, const nxh_t
   if ((rc = la_begin(ctx, op))) return rc;
   HostStatus status(ctx);
   Work work(ctx);
-  PathAtExit path{n >= LA_WIDE_FROM ? "cholesky_columns_wide" : "cholesky_columns"};
+  PathAtExit path{"cholesky_blocked"};
   const size_t mat = (size_t)(p.batch * n * n) * p.esize;
   if (la_many_small(p.cx, p.batch, n)) {
+    path.name = "cholesky_small";
     void *A;
     if ((rc = work.get(mat, &A))) return rc;
     nxh_tensor wa = workspace_tensor(x, A, p.wdt, n, n, false);
@@ -1480,6 +1481,7 @@ NXH_EXPORT int nxh_cholesky(nxh_context *ctx, const nxh_tensor *out, const nxh_t
   nxh_tensor wio{};
   const bool direct = la_direct(x, &mx) && la_direct(out, &mo);
   if (!direct) {  // both through one workspace of the compute type
+    path.name = "cholesky_blocked_workspace";
     if ((rc = work.get(mat, &io))) return rc;
     wio = workspace_tensor(x, io, p.wdt, n, n, false);
     if ((rc = nxh_cast(ctx, &wio, x))) return rc;
@@ -1516,7 +1518,7 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
   if ((rc = la_begin(ctx, op))) return rc;
   HostStatus status(ctx);
   Work work(ctx);
-  PathAtExit path{n >= LA_WIDE_FROM ? "triangular_substitution_wide" : "triangular_substitution"};
+  PathAtExit path{"triangular_blocked"};
   LaMat ma{}, mb{}, mx{};
   nxh_tensor wx{};
   const bool small = la_many_small(p.cx, p.batch, n);
@@ -1525,6 +1527,7 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
   const int size = a->dtype == NXH_F32 ? 4 : a->dtype == NXH_F64 ? 8 : 16;
   const bool direct = !small && n <= pass && la_direct(a, &ma) && la_direct(b, &mb) && la_direct(out, &mx) && !la_meet(out, a, size) && !la_meet(out, b, size);
   if (!direct) {
+    path.name = small ? "triangular_small" : n > pass ? "triangular_blocked_passes" : "triangular_blocked_workspace";
     void *A, *X;
     if ((rc = work.get((size_t)(p.batch * n * n) * p.esize, &A)) || (rc = work.get((size_t)(p.batch * n * nrhs) * p.esize, &X))) return rc;
     nxh_tensor wa = workspace_tensor(a, A, p.wdt, n, n, false);

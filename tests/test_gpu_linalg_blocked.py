@@ -43,6 +43,7 @@ def test_cholesky_at_block_edges(hip, name, n):
     seen = np.tril(a) + np.triu(np.full(batch + (n, n), np.nan), 1).astype(a.dtype)  # the upper triangle is not read
     for upper in (False, True):
         t = hip.cholesky(put(hip, seen, d), upper)
+        assert hip.last_path() == "cholesky_blocked"
         f = logical(t).astype(np.complex128 if d.is_complex else np.float64)
         assert np.all((np.tril(f, -1) if upper else np.triu(f, 1)) == 0)
         low = H(f) if upper else f
@@ -75,7 +76,9 @@ def test_triangular_solve_at_block_edges(hip, name, n, nrhs):
                 if unit:
                     m[..., np.arange(n), np.arange(n)] = 1
                 m = H(m) if transpose else m
-                x = logical(hip.triangular_solve(put(hip, hidden.astype(d.np_storage), d), put(hip, b, d), upper, transpose, unit)).astype(m.dtype)
+                t = hip.triangular_solve(put(hip, hidden.astype(d.np_storage), d), put(hip, b, d), upper, transpose, unit)
+                assert hip.last_path() == ("triangular_blocked_passes" if n > (512 if d.is_complex else 1024) else "triangular_blocked")
+                x = logical(t).astype(m.dtype)
                 residual = np.abs(m @ x - b.astype(m.dtype))
                 bound = (4 * n * 2.0 ** -53 + 2 * EPS[name]) * (np.abs(m) @ np.abs(x)) + 4 * n * 2.0 ** -53
                 assert np.all(residual <= bound), (upper, transpose, unit, float(np.max(residual / bound)))
@@ -268,8 +271,11 @@ def test_many_small_systems(hip, name, batch, n):
     a = (g @ H(g) + n * np.eye(n)).astype(d.np_storage)
     a[..., np.arange(n), np.arange(n)] = a[..., np.arange(n), np.arange(n)].real
     full = np.tril(a).astype(wide) + H(np.tril(a, -1)).astype(wide)
+    small = d.is_complex and batch >= 512 and 16 < n <= 64
     for upper in (False, True):
-        f = logical(hip.cholesky(put(hip, a, d), upper)).astype(wide)
+        t = hip.cholesky(put(hip, a, d), upper)
+        assert hip.last_path() == ("cholesky_small" if small else "cholesky_blocked_workspace" if name == "complex64" else "cholesky_blocked")
+        f = logical(t).astype(wide)
         low = H(f) if upper else f
         assert np.all(np.triu(low, 1) == 0)
         assert np.all(np.abs(low @ H(low) - full) <= (4 * n * 2.0 ** -53 + 3 * eps) * (np.abs(low) @ np.abs(H(low))))
@@ -281,7 +287,9 @@ def test_many_small_systems(hip, name, batch, n):
             if unit:
                 m[..., np.arange(n), np.arange(n)] = 1
             m = H(m) if transpose else m
-            x = logical(hip.triangular_solve(put(hip, t, d), put(hip, b, d), False, transpose, unit)).astype(wide)
+            got = hip.triangular_solve(put(hip, t, d), put(hip, b, d), False, transpose, unit)
+            assert hip.last_path() == ("triangular_small" if small else "triangular_blocked_workspace" if name == "complex64" else "triangular_blocked")
+            x = logical(got).astype(wide)
             assert np.all(np.abs(m @ x - b) <= (4 * n * 2.0 ** -53 + 2 * eps) * (np.abs(m) @ np.abs(x)) + 4 * n * 2.0 ** -53)
     out = put(hip, np.full((batch, n, n), 7, d.np_storage), d)
     a[batch - 3, n - 1, n - 1] = -1
@@ -416,10 +424,12 @@ def test_in_place_and_shared_storage(hip):
     t, want = put(hip, a, dt.float64), logical(hip.cholesky(put(hip, a, dt.float64)))
     ds = t._desc()
     hip._check(hip._lib.nxh_cholesky(hip._h, C.byref(ds), C.byref(ds), 0))
+    assert hip.last_path() == "cholesky_blocked"
     assert np.array_equal(logical(t), want)
     b = rng.standard_normal((n, 5))
     tb, tl = put(hip, b, dt.float64), put(hip, want, dt.float64)
     x = logical(hip.triangular_solve(tl, put(hip, b, dt.float64), False, False, False))
     db, dl = tb._desc(), tl._desc()
     hip._check(hip._lib.nxh_triangular_solve(hip._h, C.byref(db), C.byref(dl), C.byref(db), 0))
+    assert hip.last_path() == "triangular_blocked_workspace"
     assert np.array_equal(logical(tb), x)
