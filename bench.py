@@ -332,11 +332,11 @@ def next_ops(hip, W, linalg=False):
     y = bf((b * sq, 3072))
     timed("gelu_tanh [8192,3072] bf16 (fused)", lambda: hip.gelu_tanh(y), 2 * b * sq * 3072 * 2)
     del x, y, gam, bet, q, k, v
-    # Fourier transforms: one pass reads and writes the tensor once; the butterflies run in LDS
+    # Fourier transforms: one pass reads and writes the tensor once; the butterflies run in registers
     cplx = lambda shape: W.dev((rng.standard_normal(shape) + 1j * rng.standard_normal(shape)).astype(np.complex64),
                                dt.complex64)
     z = cplx((16384, 1024))
-    timed("fft [16384,1024] complex64 axis 1 (fft_lines, four radix-2 stages per LDS pass)", lambda: hip.fft(z, [1]), 2 * 16384 * 1024 * 8)
+    timed("fft [16384,1024] complex64 axis 1 (fft_lines, up to sixteen elements a lane)", lambda: hip.fft(z, [1]), 2 * 16384 * 1024 * 8)
     out[-1]["GFLOP/s"] = round(5 * 16384 * 1024 * 10 / out[-1]["ms"] / 1e6, 1)
     z2 = cplx((4096, 4096))
     timed("fft [4096,4096] complex64 axis 0 (strided lines)", lambda: hip.fft(z2, [0]), 2 * 4096 * 4096 * 8)
@@ -349,7 +349,7 @@ def next_ops(hip, W, linalg=False):
     timed("fft [4,2^20] complex64 axis 1 (four-step through a workspace)", lambda: hip.fft(big, [1]),
           2 * 4 * (1 << 20) * 8, iters=5)
     for rec in out[-5:]:
-        rec["bound"] = "lds"
+        rec["bound"] = "latency"  # of a wave's chain of exchanges through LDS
     del z, z2, z3, r, big
     if not linalg:
         return out
