@@ -1288,11 +1288,15 @@ static int run_cholesky(nxh_context *ctx, const char *op, HostStatus &status, in
   return run(ctx, op, status, batch, n, upper, x, out, A, diag);
 }
 
-// Where the small forms of complex systems are the faster ones: from a few hundred matrices on. Measured
-// (us, small / in blocks): factors of [256,64,64] 262 / 122, [1024,17,17] 57 / 103, [2048,64,64] 615 / 836; a solve with
-// 16 sides of [256,32,32] 59 / 38, [1024,17,17] 53 / 105, [2048,64,64] 391 / 394, with one side 150 / 395. Up
-// to 16 rows a block is one wave and the faster form throughout.
-static bool la_many_small(bool complex, int64_t batch, int64_t n) { return complex && batch >= 512 && n > 16 && n <= 64; }
+// Where the small forms of complex systems are the faster ones: where the form in blocks has a thousand workgroups
+// to queue (one per matrix, of a solve one per sixteen sides), there are matrices enough for the chip, and they are
+// more than `single` rows: up to 32 of them are one tile of the factor, up to 16 one wave of the solve. Measured
+// (complex128, us, small / in blocks): factors of [512,64,64] 285 / 239, [1024,48,48] 205 / 363, [1024,64,64] 342 /
+// 427, [1024,32,32] 111 / 51; a solve of [512,32,32] with 16 sides 67 / 62 and with 17 72 / 106, of [512,64,64] 141 /
+// 112 and 146 / 205, of [1024,17,17] 52 / 104, of [2048,64,64] with one side 149 / 392, with 16 389 / 393.
+static bool la_many_small(bool complex, int64_t batch, int64_t n, int64_t single, int64_t nrhs = 1) {
+  return complex && batch >= 512 && batch * ((nrhs + 15) / 16) >= 1024 && n > single && n <= 64;
+}
 
 // Rows of a pass: what the LDS holds of sixteen right-hand sides beside the triangles.
 template <class T>
@@ -1464,7 +1468,7 @@ NXH_EXPORT int nxh_cholesky(nxh_context *ctx, const nxh_tensor *out, const nxh_t
   Work work(ctx);
   PathAtExit path{"cholesky_blocked"};
   const size_t mat = (size_t)(p.batch * n * n) * p.esize;
-  if (la_many_small(p.cx, p.batch, n)) {
+  if (la_many_small(p.cx, p.batch, n, Chol<c64, 2>::NB)) {
     path.name = "cholesky_small";
     void *A;
     if ((rc = work.get(mat, &A))) return rc;
@@ -1521,7 +1525,7 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
   PathAtExit path{"triangular_blocked"};
   LaMat ma{}, mb{}, mx{};
   nxh_tensor wx{};
-  const bool small = la_many_small(p.cx, p.batch, n);
+  const bool small = la_many_small(p.cx, p.batch, n, 16, nrhs);
   const int pass = p.cx ? TRSM_PASS<c64> : TRSM_PASS<double>;
   // the result may be written while other workgroups read: only where it is apart from what they read
   const int size = a->dtype == NXH_F32 ? 4 : a->dtype == NXH_F64 ? 8 : 16;

@@ -260,7 +260,8 @@ def test_first_call_of_a_context(hip):
 
 
 @pytest.mark.parametrize("name", ["float32", "float64", "complex128", "complex64"])
-@pytest.mark.parametrize("batch,n", [(511, 17), (512, 17), (512, 64), (512, 65), (700, 16), (700, 1), (513, 33)])
+@pytest.mark.parametrize("batch,n", [(511, 17), (512, 17), (512, 64), (512, 65), (1023, 17), (1024, 17), (1024, 64), (1024, 65), (1100, 16), (1100, 1), (1025, 32),
+                                     (1025, 33)])
 def test_many_small_systems(hip, name, batch, n):
     """Either side of the number and the size of matrices where the form changes: every matrix as alone,
     within the bound of either (4 n eps of the magnitudes summed), failures of one of them as of one."""
@@ -271,32 +272,31 @@ def test_many_small_systems(hip, name, batch, n):
     a = (g @ H(g) + n * np.eye(n)).astype(d.np_storage)
     a[..., np.arange(n), np.arange(n)] = a[..., np.arange(n), np.arange(n)].real
     full = np.tril(a).astype(wide) + H(np.tril(a, -1)).astype(wide)
-    small = d.is_complex and batch >= 512 and 16 < n <= 64
+    small = lambda single, sides: d.is_complex and batch >= 512 and batch * -(-sides // 16) >= 1024 and single < n <= 64
     for upper in (False, True):
         t = hip.cholesky(put(hip, a, d), upper)
-        assert hip.last_path() == ("cholesky_small" if small else "cholesky_blocked_workspace" if name == "complex64" else "cholesky_blocked")
+        assert hip.last_path() == ("cholesky_small" if small(32, 1) else "cholesky_blocked_workspace" if name == "complex64" else "cholesky_blocked")
         f = logical(t).astype(wide)
         low = H(f) if upper else f
         assert np.all(np.triu(low, 1) == 0)
         assert np.all(np.abs(low @ H(low) - full) <= (4 * n * 2.0 ** -53 + 3 * eps) * (np.abs(low) @ np.abs(H(low))))
     t = np.tril(draws(rng, (batch, n, n), name) / np.sqrt(n) + 2 * np.eye(n)).astype(d.np_storage)
-    b = draws(rng, (batch, n, 5), name).astype(d.np_storage)
-    for transpose in (False, True):
-        for unit in (False, True):
-            m = t.astype(wide)
-            if unit:
-                m[..., np.arange(n), np.arange(n)] = 1
-            m = H(m) if transpose else m
-            got = hip.triangular_solve(put(hip, t, d), put(hip, b, d), False, transpose, unit)
-            assert hip.last_path() == ("triangular_small" if small else "triangular_blocked_workspace" if name == "complex64" else "triangular_blocked")
-            x = logical(got).astype(wide)
-            assert np.all(np.abs(m @ x - b) <= (4 * n * 2.0 ** -53 + 2 * eps) * (np.abs(m) @ np.abs(x)) + 4 * n * 2.0 ** -53)
+    for transpose, unit, sides in ((False, False, 5), (False, True, 17), (True, False, 17), (True, True, 5)):
+        b = draws(rng, (batch, n, sides), name).astype(d.np_storage)
+        m = t.astype(wide)
+        if unit:
+            m[..., np.arange(n), np.arange(n)] = 1
+        m = H(m) if transpose else m
+        got = hip.triangular_solve(put(hip, t, d), put(hip, b, d), False, transpose, unit)
+        assert hip.last_path() == ("triangular_small" if small(16, sides) else "triangular_blocked_workspace" if name == "complex64" else "triangular_blocked")
+        x = logical(got).astype(wide)
+        assert np.all(np.abs(m @ x - b) <= (4 * n * 2.0 ** -53 + 2 * eps) * (np.abs(m) @ np.abs(x)) + 4 * n * 2.0 ** -53)
     out = put(hip, np.full((batch, n, n), 7, d.np_storage), d)
     a[batch - 3, n - 1, n - 1] = -1
     assert raw_call(hip, "cholesky", out, put(hip, a, d), 0) != 0 and np.all(logical(out) == 7)
     t[batch - 3, n - 1, n - 1] = 0
-    sides = put(hip, b, d)
-    assert raw_call(hip, "triangular_solve", sides, put(hip, t, d), sides, 0) != 0 and np.array_equal(logical(sides), b)
+    over = put(hip, b, d)
+    assert raw_call(hip, "triangular_solve", over, put(hip, t, d), over, 0) != 0 and np.array_equal(logical(over), b)
 
 
 def raw_call(hip, name, out, *args):
