@@ -260,7 +260,8 @@ __device__ __forceinline__ bool factor16_columns(double *tile, int ld, double *i
 // the matrix until its column comes up, so that an element rounds a few times at its own size and not
 // once a column: float64, g g^T + n I, relative error of the factor in eps (2-norm, against long double) for
 // n = 64, 130, 400: 1.52, 2.03, 3.41 with the updates taken from the matrix one by one, 0.55, 0.50, 0.51 so
-// (a column at a time with a wave per element: 1.44, 0.52, 0.52), for 28 us of 200 at n = 512.
+// (a column at a time with a wave per element: 1.44, 0.52, 0.52). float64 [512, 512] takes 226 us so, its
+// result written by a launch of its own, against 213.
 //
 // The chain of a launch is the diagonal tile, sixteen columns at a time: factored by wave 0
 // (factor16), then a wave per sixteen rows below solves against them (solve16), then wave 0
@@ -269,7 +270,7 @@ __device__ __forceinline__ bool factor16_columns(double *tile, int ld, double *i
 // instruction for them, are factored column by column, a row a lane.
 // Matrices of ONE blocks of sixteen columns, 1 or 2, are a single tile: a wave per block, and the LDS of
 // one tile, so that a compute unit holds several. (0: any size, eight waves and four tiles, one
-// workgroup a unit: float64 factors of [16384,16,16] in 361 us against 66, of [1024,17,17] in 57 against 29; the
+// workgroup a unit: float64 factors of [16384,16,16] in 361 us against 68, of [1024,17,17] in 51 against 29; the
 // form for one workgroup per matrix in a workspace took 281 and 52.)
 template <class T, int ONE>
 struct Chol {
