@@ -1205,34 +1205,41 @@ static bool la_meet(const nxh_tensor *a, const nxh_tensor *b, int size) {
   return a0 < b1 && b0 < a1;
 }
 
-// The word of pinned memory the blocked kernels report to. It belongs to one call at a time (the
-// context's call_mu), which clears it first, and waits for the kernels that may still write it also
-// where it returns early.
+// The word of pinned memory the blocked kernels report to, and one of device memory by which the kernels of
+// one call hold each other back. Both belong to one call at a time (the context's call_mu): the first is
+// cleared before it is lent, the second (zero between calls, and no other kernel's) after a call that may have
+// set it. A call that returns early waits here for the kernels that may still write them.
 struct HostStatus {
   nxh_context *ctx;
-  bool lent = false, waited = false;  // whether kernels have the word; whether they have been waited for
+  bool lent = false, clean = false, held = false;  // clean: the kernels have been waited for and reported nothing
   explicit HostStatus(nxh_context *c) : ctx(c) { *(volatile int *)word() = LA_OK; }
   ~HostStatus() {
-    if (!lent || waited) return;
+    if (!lent || clean) return;
     std::lock_guard<std::mutex> g(ctx->mu);
     (void)hipStreamSynchronize(ctx->stream);
     *(volatile int *)word() = LA_OK;
-    (void)hipMemcpyAsync(la_status(ctx), word(), sizeof(int), hipMemcpyHostToDevice, ctx->stream);
+    if (!held) return;
+    (void)hipMemcpyAsync(hold(), word(), sizeof(int), hipMemcpyHostToDevice, ctx->stream);
     (void)hipStreamSynchronize(ctx->stream);
   }
   int *word() const { return ctx->fault_flag_host + 8; }
+  int *hold() const { return ctx->fault_flag + 2; }
   int *lend() {
     lent = true;
     return word();
+  }
+  int *lend_hold() {
+    held = true;
+    return hold();
   }
   // Waits for the kernels of this call (the results included) and reads their report.
   int collect(const char *op) {
     std::lock_guard<std::mutex> g(ctx->mu);
     NXH_HIP(op, hipGetLastError());
     NXH_HIP(op, hipStreamSynchronize(ctx->stream));
-    waited = true;
     const int code = *(volatile int *)word();
-    return code == LA_OK ? NXH_OK : nxh_fail(NXH_FAILURE, op, LA_MESSAGES[code <= LA_NO_CONVERGE ? code : LA_NO_CONVERGE]);
+    clean = code == LA_OK;
+    return clean ? NXH_OK : nxh_fail(NXH_FAILURE, op, LA_MESSAGES[code <= LA_NO_CONVERGE ? code : LA_NO_CONVERGE]);
   }
 };
 
@@ -1335,7 +1342,7 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
     a.mbs = m.bs;
     a.rows = n;
     a.status = status.lend();
-    hipLaunchKernelGGL((trsm_check_kernel<T, TS>), dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, ctx->stream, a, batch, la_status(ctx));
+    hipLaunchKernelGGL((trsm_check_kernel<T, TS>), dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, ctx->stream, a, batch, status.lend_hold());
   }
   for (int64_t b0 = 0; b0 < batch; b0 += LA_GRID_BATCH) {
     const unsigned nbat = (unsigned)std::min(LA_GRID_BATCH, batch - b0), groups = (unsigned)((nrhs + 15) / 16);
@@ -1352,7 +1359,7 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
       a.rows = std::min(n - r0, TRSM_PASS<T>);
       a.nrhs = nrhs;
       a.status = status.lend();
-      a.hold = check ? la_status(ctx) : nullptr;
+      a.hold = check ? status.hold() : nullptr;
       const int nb = (a.rows + 15) / 16;
       const auto kern = nb == 1 ? one : sizeof(T) == 8 && nb <= 2 + TRSM_UPDATERS * TRSM_FEW ? few : most;  // (complex reads nothing ahead)
       const int threads = nb == 1 ? TRSM_THREADS<0> : TRSM_THREADS<TRSM_FEW>;
@@ -1365,9 +1372,7 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
   }
   NXH_HIP(op, hipGetLastError());
   g.unlock();
-  const int rc = status.collect(op);
-  if (rc && check) (void)la_collect(ctx, op);  // (clears the word on the device)
-  return rc;
+  return status.collect(op);
 }
 
 // Householder QR of `batch` column-major m x n matrices At, Q's first nq columns to Qt.
