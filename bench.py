@@ -313,7 +313,7 @@ def next_ops(hip, W, linalg=False):
     # fused attention and the row kernels at GPT-2-small's shapes (bf16, batch 8, seq 1024)
     bf = lambda shape: W.dev((rng.standard_normal(shape).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16),
                              dt.bfloat16)
-    mm("matmul bf16 [256,2304] x [32,2304,196] (3x3 windows of [32,256,14,14]; rows of 196 via a padded copy)",
+    mm("matmul bf16 [256,2304] x [32,2304,196] (3x3 windows of [32,256,14,14]; rows of 196)",
        hip.expand(bf((1, 256, 2304)), (32, 256, 2304)), bf((32, 2304, 196)), 2.0 * 32 * 256 * 2304 * 196, 2500.0)
     b, h, sq, hd = 8, 12, 1024, 64
     q, k, v = (hip.permute(hip.reshape(bf((b, sq, h * hd)), (b, sq, h, hd)), (0, 2, 1, 3)) for _ in range(3))

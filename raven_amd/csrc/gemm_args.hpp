@@ -40,3 +40,8 @@ struct GemmArgs {
 // The register-blocked kernel for the dtypes without a matrix-instruction path (gemm_block.hip):
 // NXH_OK, an error status, or -1 when the shape is better left to the one-lane-per-output kernel.
 int nxh_gemm_block(nxh_context *ctx, int dtype, GemmArgs &a, uint32_t nbatch);
+// The general kernel of the dtypes with one (gemm_mfma.hip; float32, bfloat16, float16): any extents,
+// strides and alignment. -1 only for more than 2^31 result tiles or a K beyond 2^31.
+int nxh_gemm_mfma(nxh_context *ctx, int dtype, const GemmArgs &a, uint32_t nbatch);
+// The LDS-tiled kernels on operands of any K and alignment (gemm_ragged.hip); -1 where they do not apply.
+int nxh_gemm_ragged(nxh_context *ctx, int dtype, const GemmArgs &a, uint32_t nbatch);

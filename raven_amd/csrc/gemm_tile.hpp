@@ -145,6 +145,7 @@ struct Args {
   // the launch belongs to member tn / gtn. Offsets of members 1 and 2 from member 0, in elements.
   uint32_t ngroup, gtn;
   int64_t goff_b[2], goff_c[2], goff_bias[2];
+  int64_t ccs;  // RAG kernels: distance of two columns of C
 };
 
 // The arithmetic of the fused linear's epilogue on 16-bit results, two neighbours per
@@ -261,6 +262,38 @@ __device__ __forceinline__ V16 slab_load1(int i, const typename EL::S *p, int64_
     return *reinterpret_cast<const V16 *>(p + (int64_t)(v / VPR) * ld + c);
   }
 }
+// The same vector where the operand is as it comes (RAG kernels): rows start at any element, the
+// vector may run past the row's end. Along M / N that is harmless in every slab but the last: what
+// follows the row in memory is a neighbouring one (the host has checked a pitch of at least a row and
+// rows of at least a vector), and only feeds outputs that are never stored. The last slab (TAIL) reads
+// what exists and nothing else, zeros past K: `kleft` k-values are left at the slab's origin.
+typedef V16 V16a4 __attribute__((aligned(4)));
+typedef V16 V16a2 __attribute__((aligned(2)));
+template <class EL, bool KC, int ROWS, int THREADS, bool TAIL>
+__device__ __forceinline__ V16 slab_load1_ragged(int i, const typename EL::S *p, int64_t ld, int edge, int kleft) {
+  using S = typename EL::S;
+  using V16u = std::conditional_t<EL::F32, V16a4, V16a2>;
+  constexpr int VE = EL::VE, VPR = ROWS / VE;
+  const int v = threadIdx.x + i * THREADS;
+  int row = KC ? v >> 3 : (v % VPR) * VE;  // along M / N: the vector's row, or its first
+  const int k = KC ? (v & 7) * VE : v / VPR;
+  const bool past = row >= edge;
+  row = past ? edge - 1 : row;
+  const S *q = KC ? p + (int64_t)row * ld + k : p + (int64_t)k * ld + row;
+  if constexpr (!TAIL) {
+    return *reinterpret_cast<const V16u *>(q);
+  } else {
+    const int have = KC ? kleft - k : (k < kleft ? edge - row : 0);  // elements of the vector that exist
+    if (have >= VE) return *reinterpret_cast<const V16u *>(q);
+    union {
+      S s[VE];
+      V16 v16;
+    } u;
+#pragma unroll
+    for (int j = 0; j < VE; j++) u.s[j] = j < have ? q[j] : (S)0;
+    return u.v16;
+  }
+}
 template <class EL, bool KC, int ROWS, int THREADS>
 __device__ __forceinline__ void slab_store1(int i, const V16 &r, typename EL::S *lds) {
   using G = Geo<EL>;
@@ -322,7 +355,8 @@ __device__ __forceinline__ void tile_of_block(const Args &a, uint32_t bid, uint3
 
 // OUT32: the f32 sums are stored as they are (C is float, `ldc` and the batch strides in floats):
 // the partial sums of a product cut along K, added up by a second kernel.
-template <class EL, bool A_KC, bool B_KC, class SH, bool EDGE, bool EPI = false, bool OUT32 = false>
+// RAG: any K, any alignment of the operands' rows (slab_load1_ragged), ragged edges.
+template <class EL, bool A_KC, bool B_KC, class SH, bool EDGE, bool EPI = false, bool OUT32 = false, bool RAG = false>
 __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH::WAVES_PER_SIMD))) void kernel(Args a) {
   constexpr int THREADS = SH::THREADS, BM = SH::BM, BN = SH::BN, TM = SH::TM, TN = SH::TN;
   constexpr int NVA = SH::NVA, NVB = SH::NVB, BK = Geo<EL>::BK;
@@ -365,8 +399,8 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
   const int edge_n = EDGE ? (int)(a.N - n0 < BN ? a.N - n0 : BN) : BN;
   // a k-contiguous operand clamps its rows to the logical edge; one contiguous along M / N
   // clamps its vectors to the loadable extent
-  const int ledge_m = EDGE && !A_KC ? (int)(a.Mld - m0 < BM ? a.Mld - m0 : BM) : edge_m;
-  const int ledge_n = EDGE && !B_KC ? (int)(a.Nld - n0 < BN ? a.Nld - n0 : BN) : edge_n;
+  const int ledge_m = EDGE && !A_KC && !RAG ? (int)(a.Mld - m0 < BM ? a.Mld - m0 : BM) : edge_m;
+  const int ledge_n = EDGE && !B_KC && !RAG ? (int)(a.Nld - n0 < BN ? a.Nld - n0 : BN) : edge_n;
   // slab origin and per-slab advance of each operand
   const S *gA = (const S *)a.A + ao + (A_KC ? m0 * a.lda : m0);
   const S *gB = (const S *)a.B + bo + (B_KC ? n0 * a.ldb : n0);
@@ -383,17 +417,32 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
     for (int u = 0; u < TN; u++)
 #pragma unroll
       for (int e = 0; e < 16; e++) acc[t][u][e] = 0.0f;
+  // The one-tile waves of the ragged form sum the odd k-steps apart: half the length of the chain of
+  // roundings, as a product cut in two along K would have it.
+  constexpr bool TWO = RAG && TM * TN == 1;
+  f32x16 odd;
+  if constexpr (TWO) {
+#pragma unroll
+    for (int e = 0; e < 16; e++) odd[e] = 0.0f;
+  }
 
   V16 ra[NVA], rb[NVB];
-  const int nk = (int)(a.K / BK);
+  const int nk = (int)(RAG ? (a.K + BK - 1) / BK : a.K / BK);
+  const int kleft = RAG ? (int)(a.K - (int64_t)(nk - 1) * BK) : BK;  // of the last slab
   // Staged vector i of an operand moves at k-step i % KSTEPS; the prologue uses
   // the same issue order, so the loop's in-order wait counts hold from the start.
-  auto fetch_step = [&](int ks, const S *pA, const S *pB) {
+  auto fetch_step = [&](int ks, const S *pA, const S *pB, auto tail_c, int kleft) {
+    constexpr bool TAIL = decltype(tail_c)::value;
 #pragma unroll
     for (int i = 0; i < (NVA > NVB ? NVA : NVB); i++) {
       if (i % KSTEPS != ks) continue;
-      if (i < NVA) ra[i] = slab_load1<EL, A_KC, BM, THREADS, EDGE>(i, pA, a.lda, ledge_m);
-      if (i < NVB) rb[i] = slab_load1<EL, B_KC, BN, THREADS, EDGE>(i, pB, a.ldb, ledge_n);
+      if constexpr (RAG) {
+        if (i < NVA) ra[i] = slab_load1_ragged<EL, A_KC, BM, THREADS, TAIL>(i, pA, a.lda, ledge_m, kleft);
+        if (i < NVB) rb[i] = slab_load1_ragged<EL, B_KC, BN, THREADS, TAIL>(i, pB, a.ldb, ledge_n, kleft);
+      } else {
+        if (i < NVA) ra[i] = slab_load1<EL, A_KC, BM, THREADS, EDGE>(i, pA, a.lda, ledge_m);
+        if (i < NVB) rb[i] = slab_load1<EL, B_KC, BN, THREADS, EDGE>(i, pB, a.ldb, ledge_n);
+      }
     }
   };
   auto stage_step = [&](int ks, S *nA, S *nB) {
@@ -404,14 +453,23 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
       if (i < NVB) slab_store1<EL, B_KC, BN, THREADS>(i, rb[i], nB);
     }
   };
+  using yes = std::integral_constant<bool, true>;
+  using no = std::integral_constant<bool, false>;
+  auto fetch_slab = [&](int kt) {  // of the prologue
+    const bool last = kt == nk - 1;
+    // (rows that run backwards through memory: what follows the first one is not the operand)
+    if (RAG && (last || (kt == 0 && (a.lda < 0 || a.ldb < 0)))) {
 #pragma unroll
-  for (int ks = 0; ks < KSTEPS; ks++) fetch_step(ks, gA, gB);
+      for (int ks = 0; ks < KSTEPS; ks++) fetch_step(ks, gA + kt * stepA, gB + kt * stepB, yes{}, last ? kleft : BK);
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ks++) fetch_step(ks, gA + kt * stepA, gB + kt * stepB, no{}, BK);
+    }
+  };
+  fetch_slab(0);
 #pragma unroll
   for (int ks = 0; ks < KSTEPS; ks++) stage_step(ks, smem, smem + A_ELEMS);
-  if (nk > 1) {
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) fetch_step(ks, gA + stepA, gB + stepB);
-  }
+  if (nk > 1) fetch_slab(1);
   __syncthreads();
 
   // One K-slab: multiply slab kt out of LDS; when STAGE, move slab kt+1 from
@@ -427,7 +485,8 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
   for (int t = 0; t < TM; t++) fa[0][t] = frag_load<EL, A_KC, BM>(smem, wm + t * 32, 0, lane);
 #pragma unroll
   for (int u = 0; u < TN; u++) fb[0][u] = frag_load<EL, B_KC, BN>(smem + A_ELEMS, wn + u * 32, 0, lane);
-  auto slab = [&](int kt, auto stage_c, auto fetch_c) {
+  // `tail_c`: the slab fetched is the last one of a RAG product.
+  auto slab = [&](int kt, auto stage_c, auto fetch_c, auto tail_c) {
     constexpr bool STAGE = decltype(stage_c)::value, FETCH = decltype(fetch_c)::value;
     const S *sA = smem + (kt & 1) * STAGE_ELEMS;
     const S *sB = sA + A_ELEMS;
@@ -438,7 +497,7 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
     for (int ks = 0; ks < KSTEPS; ks++) {
       const int cur = ks & 1, nxt = cur ^ 1;
       if constexpr (STAGE) stage_step(ks, nA, nB);
-      if constexpr (FETCH) fetch_step(ks, pA, pB);
+      if constexpr (FETCH) fetch_step(ks, pA, pB, tail_c, kleft);
       if (ks + 1 < KSTEPS) {
 #pragma unroll
         for (int t = 0; t < TM; t++) fa[nxt][t] = frag_load<EL, A_KC, BM>(sA, wm + t * 32, ks + 1, lane);
@@ -454,7 +513,7 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
 #pragma unroll
       for (int t = 0; t < TM; t++)
 #pragma unroll
-        for (int u = 0; u < TN; u++) mfma_step<EL>(acc[t][u], fa[cur][t], fb[cur][u]);
+        for (int u = 0; u < TN; u++) mfma_step<EL>(TWO && cur ? odd : acc[t][u], fa[cur][t], fb[cur][u]);
       // The memory instructions of this k-step are issued among its MFMAs, one LDS read, one
       // LDS write and one global load behind each (LDS returns in order, so the wait before the
       // first MFMA only covers the current fragments): queueing them all in front of the step
@@ -469,12 +528,16 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  using yes = std::integral_constant<bool, true>;
-  using no = std::integral_constant<bool, false>;
   int kt = 0;
-  for (; kt + 2 < nk; kt++) slab(kt, yes{}, yes{});
-  if (kt + 1 < nk) slab(kt++, yes{}, no{});
-  slab(kt, no{}, no{});
+  for (; kt + 2 < (RAG ? nk - 1 : nk); kt++) slab(kt, yes{}, yes{}, no{});
+  if constexpr (RAG)
+    if (kt + 2 < nk) slab(kt++, yes{}, yes{}, yes{});
+  if (kt + 1 < nk) slab(kt++, yes{}, no{}, no{});
+  slab(kt, no{}, no{}, no{});
+  if constexpr (TWO) {
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[0][0][e] += odd[e];
+  }
 
   // accumulator element e of lane l is C[(e/4)*8 + (l/32)*4 + e%4][l%32]
   S *C = (S *)a.C + co;
@@ -511,7 +574,7 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
     // buffers and sends it out as whole 16-byte row segments.
     constexpr int WC = TN * 32, WP = WC + 8;  // patch width and its LDS pitch (elements)
     static_assert((size_t)SH::WM * SH::WN * TM * 32 * WP * sizeof(S) <= SH::template lds_bytes<EL>(), "epilogue patch");
-    const bool wide = ((uintptr_t)C % 16) == 0 && a.ldc % 8 == 0 &&
+    const bool wide = ((uintptr_t)C % 16) == 0 && a.ldc % 8 == 0 && (!RAG || a.ccs == 1) &&
                       (!EPI || ((!a.bias || (uintptr_t)a.bias % 16 == 0) &&
                                 (!a.R || (((uintptr_t)((const S *)a.R + ro)) % 16 == 0 && a.ldr % 8 == 0))));
     if (wide) {
@@ -642,7 +705,7 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
       for (int e = 0; e < 16; e++) {
         const int rl = wm + t * 32 + (e >> 2) * 8 + kg * 4 + (e & 3);
         if (EDGE && rl >= edge_m) continue;
-        S *c = C + (m0 + rl) * a.ldc + n0 + cl;
+        S *c = C + (m0 + rl) * a.ldc + (RAG ? (n0 + cl) * a.ccs : n0 + cl);
         S v = narrow(acc[t][u][e]);
         if constexpr (EPI) {
           // the bias add and the residual add of the op-by-op sequence, each rounded to the dtype

@@ -8,13 +8,10 @@
 // k == 0 stores zeros.
 //
 // Kernels
-//   gemm_mfma   bf16 / f16 (v_mfma_f32_32x32x16) and f32 (v_mfma_f32_32x32x2,
-//               true f32, no xf32): 128x128 block tile, four wave64s each
-//               owning 64x64 (2x2 MFMA tiles), K-contiguous LDS tiles with a
-//               16-byte pad per row, global->register prefetch of the next
-//               K-slab while the current one is multiplied. Either operand may
-//               be K-contiguous or M/N-contiguous in memory; the turn happens
-//               on the way into LDS.
+//   gemm_tile, gemm_dl  the LDS-tiled kernels (gemm_tile.hpp, gemm_dl.hpp) on aligned operands;
+//               gemm_ragged.hip instantiates them for operands of any K and alignment.
+//   gemm_mfma   (gemm_mfma.hip) bf16 / f16 / f32 of any extents, strides and alignment: small and
+//               ragged products, straight from memory into the matrix instruction.
 //   gemm_tiny   batches of products of a few elements each: a lane per output.
 //   gemm_rowdot n <= 4 with A's rows along K (matrix x vector): a wave per row of A,
 //               16-byte pieces, float32 sums met through the cross-lane network.
@@ -37,184 +34,25 @@
 #include "gemm_dl.hpp"
 #include "nxh_common.hpp"
 
-typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 // A native vector, not a struct: arrays of these stay in registers.
 typedef __attribute__((ext_vector_type(4))) uint32_t U4;
 
-// Per-dtype MFMA traits. VL = elements per 16-byte vector; one "k-chunk" is
-// 2*VL values of k: lanes 0-31 multiply the first VL of them, lanes 32-63 the
-// second (any fixed assignment of k to lanes is valid as long as A and B agree).
+// Per-dtype traits of the dispatch.
 struct MMbf16 {
   static constexpr int DT = NXH_BF16;
   using S = uint16_t;
-  static constexpr int VL = 8;
-  __device__ __forceinline__ static void mac(f32x16 &acc, const U4 &a, const U4 &b) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
-                                                  acc, 0, 0, 0);
-  }
 };
 struct MMf16 {
   static constexpr int DT = NXH_F16;
   using S = uint16_t;
-  static constexpr int VL = 8;
-  __device__ __forceinline__ static void mac(f32x16 &acc, const U4 &a, const U4 &b) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b),
-                                                 acc, 0, 0, 0);
-  }
 };
 struct MMf32 {
   static constexpr int DT = NXH_F32;
   using S = float;
-  static constexpr int VL = 4;
-  __device__ __forceinline__ static void mac(f32x16 &acc, const U4 &a, const U4 &b) {
-    f32x4 x = __builtin_bit_cast(f32x4, a), y = __builtin_bit_cast(f32x4, b);
-#pragma unroll
-    for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s], y[s], acc, 0, 0, 0);
-  }
 };
-
-constexpr int GM = 128, GN = 128;  // block tile
-constexpr int GT = 256;            // threads
-
-// Loads this lane's two 16-byte pieces of one operand's K-slab into registers.
-// ROWS = 128 rows (m or n) by BK k-values. `kc` says the operand is contiguous
-// along k (then a vector runs along k), otherwise along its row index.
-template <class MM, int BK>
-__device__ __forceinline__ void slab_load(U4 (&r)[2], const typename MM::S *p, int64_t rs, int64_t ks,
-                                          int64_t row0, int64_t k0, int64_t nrows, int64_t K, bool kc,
-                                          bool vec) {
-  using S = typename MM::S;
-  constexpr int VL = MM::VL;
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int v = threadIdx.x + i * GT;
-    int64_t row, k;
-    if (kc) {
-      row = row0 + v / (BK / VL);
-      k = k0 + (v % (BK / VL)) * VL;
-    } else {
-      k = k0 + v / (GM / VL);
-      row = row0 + (v % (GM / VL)) * VL;
-    }
-    const S *q = p + row * rs + k * ks;
-    const bool full = kc ? (row < nrows && k + VL <= K) : (k < K && row + VL <= nrows);
-    if (vec && full) {
-      r[i] = *reinterpret_cast<const U4 *>(q);
-    } else {
-      union {
-        S t[VL];
-        U4 v;
-      } u;
-#pragma unroll
-      for (int j = 0; j < VL; j++) {
-        int64_t rr = kc ? row : row + j, kk = kc ? k + j : k;
-        u.t[j] = (rr < nrows && kk < K) ? q[kc ? j * ks : j * rs] : (S)0;
-      }
-      r[i] = u.v;
-    }
-  }
-}
-
-// Writes the prefetched pieces into the K-contiguous LDS tile [128][LDP].
-template <class MM, int BK, int LDP>
-__device__ __forceinline__ void slab_store(const U4 (&r)[2], typename MM::S *lds, bool kc) {
-  using S = typename MM::S;
-  constexpr int VL = MM::VL;
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int v = threadIdx.x + i * GT;
-    if (kc) {
-      const int row = v / (BK / VL), k = (v % (BK / VL)) * VL;
-      *reinterpret_cast<U4 *>(&lds[row * LDP + k]) = r[i];
-    } else {
-      const int k = v / (GM / VL), row = (v % (GM / VL)) * VL;
-      union {
-        U4 v;
-        S t[VL];
-      } u;
-      u.v = r[i];
-#pragma unroll
-      for (int j = 0; j < VL; j++) lds[(row + j) * LDP + k] = u.t[j];
-    }
-  }
-}
-
-template <class MM>
-__global__ __launch_bounds__(GT) void gemm_mfma_kernel(GemmArgs a) {
-  using S = typename MM::S;
-  constexpr int VL = MM::VL;
-  constexpr int BK = 4 * VL;   // two k-chunks per slab
-  constexpr int LDP = BK + VL; // 16-byte pad: rows land on distinct bank groups
-  __shared__ alignas(16) S sA[GM * LDP];
-  __shared__ alignas(16) S sB[GN * LDP];
-
-  int64_t ao, bo, co;
-  batch_decode(a.batch, a.batch0 + blockIdx.z, ao, bo, co);
-  const S *A = (const S *)a.A + ao;
-  const S *B = (const S *)a.B + bo;
-  const int64_t m0 = (int64_t)blockIdx.y * GM, n0 = (int64_t)blockIdx.x * GN;
-  const bool a_kc = a.acs == 1, b_kc = a.brs == 1;
-
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  const int r32 = lane & 31, kg = lane >> 5;
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int t = 0; t < 2; t++)
-#pragma unroll
-    for (int u = 0; u < 2; u++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) acc[t][u][e] = 0.0f;
-
-  U4 ra[2], rb[2];
-  const int64_t nk = (a.K + BK - 1) / BK;
-  if (nk > 0) {
-    slab_load<MM, BK>(ra, A, a.ars, a.acs, m0, 0, a.M, a.K, a_kc, a.a_vec);
-    // B is addressed as rows = n, so its "row stride" is bcs and k stride brs
-    slab_load<MM, BK>(rb, B, a.bcs, a.brs, n0, 0, a.N, a.K, b_kc, a.b_vec);
-  }
-  for (int64_t kt = 0; kt < nk; kt++) {
-    slab_store<MM, BK, LDP>(ra, sA, a_kc);
-    slab_store<MM, BK, LDP>(rb, sB, b_kc);
-    __syncthreads();
-    if (kt + 1 < nk) {
-      slab_load<MM, BK>(ra, A, a.ars, a.acs, m0, (kt + 1) * BK, a.M, a.K, a_kc, a.a_vec);
-      slab_load<MM, BK>(rb, B, a.bcs, a.brs, n0, (kt + 1) * BK, a.N, a.K, b_kc, a.b_vec);
-    }
-#pragma unroll
-    for (int ch = 0; ch < 2; ch++) {
-      U4 fa[2], fb[2];
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-        fa[t] = *reinterpret_cast<const U4 *>(&sA[(wm + t * 32 + r32) * LDP + ch * 2 * VL + kg * VL]);
-        fb[t] = *reinterpret_cast<const U4 *>(&sB[(wn + t * 32 + r32) * LDP + ch * 2 * VL + kg * VL]);
-      }
-#pragma unroll
-      for (int t = 0; t < 2; t++)
-#pragma unroll
-        for (int u = 0; u < 2; u++) MM::mac(acc[t][u], fa[t], fb[u]);
-    }
-    __syncthreads();
-  }
-
-  // accumulator element e of lane l is C[(e/4)*8 + (l/32)*4 + e%4][l%32]
-  S *C = (S *)a.C + co;
-#pragma unroll
-  for (int t = 0; t < 2; t++)
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-      const int64_t col = n0 + wn + u * 32 + r32;
-#pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const int64_t row = m0 + wm + t * 32 + (e >> 2) * 8 + kg * 4 + (e & 3);
-        if (row < a.M && col < a.N) C[row * a.crs + col * a.ccs] = Tr<MM::DT>::st(acc[t][u][e]);
-      }
-    }
-}
 
 // ── gemm_skinny: m <= 16, B streamed once ───────────────────────────────────
 // HBM-bound on B. A block is 64 column lanes (VN adjacent columns each: one
@@ -832,20 +670,6 @@ static int launch_f64(nxh_context *ctx, GemmArgs &a, uint32_t nbatch) {
   return NXH_OK;
 }
 
-template <class MM>
-static int launch_mfma(nxh_context *ctx, GemmArgs &a, uint32_t nbatch) {
-  nxh_set_path("gemm_mfma");
-  const uint32_t gx = (uint32_t)((a.N + GN - 1) / GN), gy = (uint32_t)((a.M + GM - 1) / GM);
-  if (gy > 65535) return launch_any<MM::DT>(ctx, a, nbatch);
-  for (uint32_t b0 = 0; b0 < nbatch; b0 += 65535) {
-    a.batch0 = b0;
-    hipLaunchKernelGGL((gemm_mfma_kernel<MM>), dim3(gx, gy, std::min<uint32_t>(65535, nbatch - b0)), dim3(GT), 0,
-                       ctx->stream, a);
-    NXH_HIP("matmul", hipGetLastError());
-  }
-  return NXH_OK;
-}
-
 template <int DT, int VN>
 static int launch_skinny(nxh_context *ctx, GemmArgs &g) {
   using S = typename Tr<DT>::S;
@@ -1340,161 +1164,6 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
   return launch_tile_oriented<EL, gemm_tile::Shape256x256, false>(ctx, g, a_kc, b_kc, "gemm_tile_256x256");
 }
 
-// ── padded copies for the tiled kernels ─────────────────────────────────────
-// The tiled kernels read whole 16-byte vectors of whole K-slabs. An operand whose rows are not
-// that (a [.., K, 196] matrix of unfolded 14 x 14 windows, a K of 196) is copied once into a
-// buffer whose contiguous dim is rounded up to whole vectors and whose K is rounded up to
-// whole slabs, the new positions filled with zeros (0 x 0 adds nothing to any sum; both operands
-// are padded along K). A broadcast batch dim stays a zero stride of the copy.
-struct RepackArgs {
-  const void *src;
-  void *dst;
-  int64_t rows, cols;    // logical extents: `cols` is the dim that becomes contiguous
-  int64_t prows, pcols;  // padded extents (pcols a multiple of the vector)
-  int64_t srs, scs;      // source strides of (row, col), elements
-  int nbd;
-  uint32_t bshape[MM_MAXB];
-  int64_t bsrc[MM_MAXB];  // source strides of the batch dims that are not broadcast
-  int64_t total;          // vectors to write
-};
-template <class S>
-__global__ __launch_bounds__(256) void gemm_repack_kernel(RepackArgs a) {
-  constexpr int VE = 16 / (int)sizeof(S);
-  const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (v >= a.total) return;
-  const int64_t vpr = a.pcols / VE;
-  const int64_t t = v / vpr, c0 = (v - t * vpr) * VE;
-  int64_t bidx = t / a.prows;
-  const int64_t r = t - bidx * a.prows;
-  int64_t so = 0;
-  for (int i = a.nbd - 1; i >= 0; i--) {
-    const int64_t q = bidx / a.bshape[i];
-    so += (bidx - q * a.bshape[i]) * a.bsrc[i];
-    bidx = q;
-  }
-  const S *src = (const S *)a.src + so + r * a.srs;
-  union {
-    U4 v4;
-    uint32_t w[4];
-    S s[VE];
-  } o;
-  o.v4 = U4{0, 0, 0, 0};
-  if (r < a.rows) {
-    if constexpr (sizeof(S) == 2) {
-      if (a.scs == 1) {
-        // 16-bit elements of a contiguous row: whole 4-byte words from the word-aligned address
-        // at or below the first element, shifted by one element where the row starts on an odd
-        // one (eight 2-byte loads per lane held this copy at half the memory rate). A word is
-        // read only if its first element belongs to the row; elements past the row's end are
-        // cleared afterwards.
-        const uintptr_t first = (uintptr_t)(src + c0);
-        const uint32_t *wp = (const uint32_t *)(first & ~(uintptr_t)3);
-        const int odd = (int)((first >> 1) & 1);
-        const int64_t left = a.cols - c0 + odd;  // elements from wp's first to the row's end
-        uint32_t w[5];
-#pragma unroll
-        for (int j = 0; j < 5; j++) w[j] = (2 * j < left && (j < 4 || odd)) ? wp[j] : 0u;
-#pragma unroll
-        for (int j = 0; j < 4; j++) o.w[j] = odd ? __builtin_amdgcn_alignbit(w[j + 1], w[j], 16) : w[j];
-#pragma unroll
-        for (int j = 0; j < VE; j++)
-          if (c0 + j >= a.cols) o.s[j] = (S)0;
-        ((U4 *)a.dst)[v] = o.v4;
-        return;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < VE; j++)
-      if (c0 + j < a.cols) o.s[j] = src[(c0 + j) * a.scs];
-  }
-  ((U4 *)a.dst)[v] = o.v4;
-}
-
-// Copies one operand (kc: contiguous along K in the copy, else along its M / N dim) and
-// rewrites its strides in place. `bstr` are the operand's batch strides.
-template <class S>
-static int repack_operand(nxh_context *ctx, const GemmArgs &g, const void *src, bool kc, int64_t rows_mn, int64_t Kp,
-                          int64_t &stride_mn, int64_t &stride_k, int64_t *bstr, int64_t &ld_mn, void **block) {
-  constexpr int VE = 16 / (int)sizeof(S);
-  RepackArgs r{};
-  r.src = src;
-  if (kc) {
-    r.rows = r.prows = rows_mn;
-    r.cols = g.K;
-    r.pcols = Kp;
-    r.srs = stride_mn;
-    r.scs = stride_k;
-  } else {
-    r.rows = g.K;
-    r.prows = Kp;
-    r.cols = rows_mn;
-    r.pcols = (rows_mn + VE - 1) / VE * VE;
-    r.srs = stride_k;
-    r.scs = stride_mn;
-  }
-  // the copy's batch layout: dense over the dims the operand really has
-  int64_t run = r.prows * r.pcols, nstr[MM_MAXB] = {};
-  for (int i = g.batch.n - 1; i >= 0; i--) {
-    if (bstr[i] == 0) continue;
-    nstr[i] = run;
-    run *= g.batch.shape[i];
-  }
-  for (int i = 0; i < g.batch.n; i++) {
-    if (bstr[i] == 0) continue;
-    r.bshape[r.nbd] = g.batch.shape[i];
-    r.bsrc[r.nbd] = bstr[i];
-    r.nbd++;
-  }
-  if (run > ((int64_t)1 << 32)) return -1;  // more than the fast path is worth
-  int rc = nxh_alloc_locked(ctx, (size_t)run * sizeof(S), block);
-  if (rc) return rc;
-  r.dst = *block;
-  r.total = run / VE;
-  hipLaunchKernelGGL((gemm_repack_kernel<S>), dim3((unsigned)((r.total + 255) / 256)), dim3(256), 0, ctx->stream, r);
-  NXH_HIP("matmul", hipGetLastError());
-  if (kc) {
-    stride_mn = Kp;
-    stride_k = 1;
-  } else {
-    stride_mn = 1;
-    stride_k = r.pcols;
-    ld_mn = r.pcols;
-  }
-  for (int i = 0; i < g.batch.n; i++) bstr[i] = nstr[i];
-  return NXH_OK;
-}
-
-// The tiled path over padded copies of the operands that do not fit it as they are. -1: not
-// worth it or not possible (the caller falls back to the general kernel).
-template <class EL>
-static int try_tile_repacked(nxh_context *ctx, const GemmArgs &a0, uint32_t nbatch, bool al_a, bool al_b) {
-  using S = typename EL::S;
-  constexpr int VE = EL::VE, BK = gemm_tile::Geo<EL>::BK;
-  if (a0.ccs != 1 || a0.batch.n > 4 || a0.M < 32 || a0.N < 32 || a0.K < 32) return -1;
-  // two more launches and a pass over the copied operand: only for products that outweigh them
-  if ((double)a0.M * (double)a0.N * (double)a0.K * (double)nbatch < (double)(1 << 27)) return -1;
-  GemmArgs a = a0;
-  const int64_t Kp = (a.K + BK - 1) / BK * BK;
-  const bool a_kc = a.acs == 1, b_kc = a.brs == 1;
-  const bool fit_a = Kp == a.K && al_a && al16(a.A) && (a_kc ? a.ars % VE == 0 : (a.acs % VE == 0 && a.M % VE == 0));
-  const bool fit_b = Kp == a.K && al_b && al16(a.B) && (b_kc ? a.bcs % VE == 0 : (a.brs % VE == 0 && a.N % VE == 0));
-  if (fit_a && fit_b) return -1;  // the tiled path refused for another reason
-  void *blk_a = nullptr, *blk_b = nullptr;
-  int rc = NXH_OK;
-  if (!fit_a) rc = repack_operand<S>(ctx, a, a.A, a_kc, a.M, Kp, a.ars, a.acs, a.batch.a, a.m_ld, &blk_a);
-  if (rc == NXH_OK && !fit_b) rc = repack_operand<S>(ctx, a, a.B, b_kc, a.N, Kp, a.bcs, a.brs, a.batch.b, a.n_ld, &blk_b);
-  if (rc == NXH_OK) {
-    if (blk_a) a.A = blk_a;
-    if (blk_b) a.B = blk_b;
-    a.K = Kp;
-    rc = try_tile<EL>(ctx, a, nbatch, true, true);
-    if (rc == NXH_OK) nxh_set_path("gemm_tile_padded");
-  }
-  if (blk_a) nxh_free_locked(ctx, blk_a);
-  if (blk_b) nxh_free_locked(ctx, blk_b);
-  return rc;
-}
-
 // ── gemm_tiny: many products of matrices of a few elements each ─────────────
 // ([65536, 4, 4] x [65536, 4, 4]: transforms, small covariance blocks.) One lane per output over
 // the whole batch, so a wave holds the outputs of several products and neighbouring lanes share
@@ -1622,7 +1291,17 @@ template <class MM>
 static int run_mfma_dtype(nxh_context *ctx, GemmArgs &a, uint32_t nbatch, bool batch_aligned_a,
                           bool batch_aligned_b) {
   using S = typename MM::S;
-  constexpr int VL = MM::VL;
+  // a result that is contiguous along its rows' index: the transposed product (C^T = B^T A^T) has unit-stride rows
+  if (a.ccs != 1 && a.crs == 1 && a.N > 1) {
+    std::swap(a.A, a.B);
+    std::swap(a.M, a.N);
+    std::swap(a.m_ld, a.n_ld);
+    std::swap(a.ars, a.bcs);
+    std::swap(a.acs, a.brs);
+    std::swap(a.crs, a.ccs);
+    for (int i = 0; i < a.batch.n; i++) std::swap(a.batch.a[i], a.batch.b[i]);
+    std::swap(batch_aligned_a, batch_aligned_b);
+  }
   // many products of a few elements each: a lane per output over the whole batch
   if (a.M * a.N <= 256 && a.K <= 64 && nbatch >= 256) return launch_tiny<MM::DT>(ctx, a, nbatch);
   // matrix x vector (up to four columns), the matrix's rows along K: a wave per row
@@ -1652,18 +1331,26 @@ static int run_mfma_dtype(nxh_context *ctx, GemmArgs &a, uint32_t nbatch, bool b
     }
   }
   const bool a_ok = a.acs == 1 || a.ars == 1, b_ok = a.brs == 1 || a.bcs == 1;
-  if (!a_ok || !b_ok) return launch_any<MM::DT>(ctx, a, nbatch);
-  {
+  if (a_ok && b_ok) {
     using EL = std::conditional_t<MM::DT == NXH_F32, gemm_tile::ElF32,
                                   std::conditional_t<MM::DT == NXH_BF16, gemm_tile::ElBF16, gemm_tile::ElF16>>;
     int rc = try_tile<EL>(ctx, a, nbatch, batch_aligned_a, batch_aligned_b);
-    if (rc == -1) rc = try_tile_repacked<EL>(ctx, a, nbatch, batch_aligned_a, batch_aligned_b);
     if (rc != -1) return rc;
+    // Operands that do not fit it as they are: the ragged form of the same kernels for products of 2^27
+    // terms or whose small blocks occupy the chip, the general kernel below that. float32 [16,200,200]
+    // x [16,200,201] (256 blocks of 64 x 64): 9.3 us against 14.2; [501,501]^2 (64 blocks): 13.9 against
+    // 7.9. bfloat16 [16,300,300]^2 (240 blocks of 128 x 64): 8.2 against 16.6; [501,501]^2 (32): 9.3
+    // against 6.7. A K of one slab is loads and stores, which the general kernel does not stage.
+    const double terms = (double)a.M * (double)a.N * (double)a.K * (double)nbatch;
+    const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256, bm = sizeof(S) == 4 ? 64 : 128;
+    const double blocks = (double)((a.M + bm - 1) / bm) * (double)((a.N + 63) / 64) * nbatch;
+    if (terms >= (double)(1 << 27) || (a.K >= 64 && blocks >= (sizeof(S) == 4 ? 0.75 : 0.6) * (double)cus)) {
+      rc = nxh_gemm_ragged(ctx, MM::DT, a, nbatch);
+      if (rc != -1) return rc;
+    }
   }
-  // 16-byte loads need an aligned base and every other stride a multiple of VL
-  a.a_vec = al16(a.A) && batch_aligned_a && ((a.acs == 1 ? a.ars : a.acs) % VL == 0);
-  a.b_vec = al16(a.B) && batch_aligned_b && ((a.brs == 1 ? a.bcs : a.brs) % VL == 0);
-  return launch_mfma<MM>(ctx, a, nbatch);
+  const int rc = nxh_gemm_mfma(ctx, MM::DT, a, nbatch);
+  return rc != -1 ? rc : launch_any<MM::DT>(ctx, a, nbatch);
 }
 
 // matmul, and with `bias` / `R` the fused linear: C = A B, then + bias[col], then
