@@ -74,7 +74,7 @@ __device__ __forceinline__ void arg_take(C &bv, I &bi, C v, I i) {
 }
 
 // Row form: a group of G lanes per output walks the axis. V > 1 (unit axis
-// stride, aligned rows, no carried indices): 16-byte loads, four in flight.
+// stride, no carried indices): 16-byte loads, four in flight.
 template <class IN, class CMP, int G, int V, bool HAS_IDX>
 __global__ __launch_bounds__(FOLD_THREADS) void arg_row_kernel(ArgArgs a) {
   using T = typename IN::T;
@@ -97,24 +97,49 @@ __global__ __launch_bounds__(FOLD_THREADS) void arg_row_kernel(ArgArgs a) {
   C bv{};
   int64_t bi = -1;
   if constexpr (V > 1) {
+    // Whole vectors at any alignment, then the run's last elements one to a lane; `f(value, index)`
+    // meets a lane's candidates in ascending order.
     const int64_t nv = (r1 - r0) / V;
-    const FVec<T, V> *pv = reinterpret_cast<const FVec<T, V> *>(p + r0);
-    int64_t i = lane;
-    for (; i + 3 * G < nv; i += 4 * G) {
-      FVec<T, V> x[4];
+    auto walk = [&](auto f) {
+      int64_t i = lane;
+      for (; i + 3 * G < nv; i += 4 * G) {
+        FVec<T, V> x[4];
 #pragma unroll
-      for (int j = 0; j < 4; j++) x[j] = pv[i + j * G];
+        for (int j = 0; j < 4; j++) x[j] = fold_load<T, V>(p + r0 + (i + j * G) * V);
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+        for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int k = 0; k < V; k++) arg_take<CMP, C>(bv, bi, IN::ld(x[j].v[k]), r0 + (i + j * G) * V + k);
+          for (int k = 0; k < V; k++) f(IN::ld(x[j].v[k]), (int32_t)(r0 + (i + j * G) * V) + k);
+      }
+      for (; i < nv; i += G) {
+        FVec<T, V> x = fold_load<T, V>(p + r0 + i * V);
+#pragma unroll
+        for (int k = 0; k < V; k++) f(IN::ld(x.v[k]), (int32_t)(r0 + i * V) + k);
+      }
+      for (int64_t r = r0 + nv * V + lane; r < r1; r += G) f(IN::ld(p[r]), (int32_t)r);
+    };
+    bool odd = false;
+    if constexpr (CMP::category == CAT_FLOAT || CMP::category == CAT_SINT || CMP::category == CAT_UINT) {
+      // three instructions per element, as in arg_col_kernel; a lane that met a NaN walks again
+      const int64_t first = lane < nv ? r0 + (int64_t)lane * V : r0 + nv * V + lane;
+      C best = CMP::worst();
+      int32_t at = first < r1 ? (int32_t)first : -1;
+      walk([&](C v, int32_t i) {
+        const bool take = CMP::better(v, best);
+        best = take ? v : best;
+        at = take ? i : at;
+        if constexpr (CMP::category == CAT_FLOAT) odd |= v != v;
+      });
+      bv = best;
+      bi = at;
+    } else {
+      odd = true;
     }
-    for (; i < nv; i += G) {
-      FVec<T, V> x = pv[i];
-#pragma unroll
-      for (int k = 0; k < V; k++) arg_take<CMP, C>(bv, bi, IN::ld(x.v[k]), r0 + i * V + k);
+    if (odd) {
+      int32_t at = -1;
+      walk([&](C v, int32_t i) { arg_take<CMP, C>(bv, at, v, i); });
+      bi = at;
     }
-    for (int64_t r = r0 + nv * V + lane; r < r1; r += G) arg_take<CMP, C>(bv, bi, IN::ld(p[r]), r);
   } else {
     for (int64_t r = r0 + lane; r < r1; r += G) {
       C v = IN::ld(p[r * a.r_stride]);
@@ -165,8 +190,9 @@ __global__ __launch_bounds__(FOLD_THREADS) void arg_col_kernel(ArgArgs a) {
   const uint64_t ob = bx / a.lane_blocks;
   const int c = gridDim.y - 1 - blockIdx.y;
   const uint32_t ln = threadIdx.x % LANES, rg = threadIdx.x / LANES;
-  const uint32_t l = (lb * LANES + ln) * V;
-  const bool live = l < a.L;
+  const uint32_t l0 = (lb * LANES + ln) * V;
+  const bool live = l0 < a.L;
+  const uint32_t l = l0 + V <= a.L ? l0 : a.L - V;  // (L >= V) the last lane's, as in fold_col
   int64_t in_off, out_off;
   fold_decode(a.kept, ob, in_off, out_off);
   const int64_t r0 = (int64_t)c * a.chunk;
@@ -187,7 +213,7 @@ __global__ __launch_bounds__(FOLD_THREADS) void arg_col_kernel(ArgArgs a) {
     for (; r + (U - 1) * RG < r1; r += U * RG) {
       FVec<T, V> x[U];
 #pragma unroll
-      for (int j = 0; j < U; j++) x[j] = *reinterpret_cast<const FVec<T, V> *>(p + (r + j * RG) * a.r_stride);
+      for (int j = 0; j < U; j++) x[j] = fold_load<T, V>(p + (r + j * RG) * a.r_stride);
 #pragma unroll
       for (int j = 0; j < U; j++)
 #pragma unroll
@@ -203,7 +229,7 @@ __global__ __launch_bounds__(FOLD_THREADS) void arg_col_kernel(ArgArgs a) {
       FVec<T, V> x[U - 1];
 #pragma unroll
       for (int j = 0; j < U - 1; j++)
-        if (r + j * RG < r1) x[j] = *reinterpret_cast<const FVec<T, V> *>(p + (r + j * RG) * a.r_stride);
+        if (r + j * RG < r1) x[j] = fold_load<T, V>(p + (r + j * RG) * a.r_stride);
 #pragma unroll
       for (int j = 0; j < U - 1; j++)
         if (r + j * RG < r1)
@@ -226,7 +252,7 @@ __global__ __launch_bounds__(FOLD_THREADS) void arg_col_kernel(ArgArgs a) {
     int32_t xi[U];
 #pragma unroll
     for (int j = 0; j < U; j++) {
-      x[j] = *reinterpret_cast<const FVec<T, V> *>(p + (r + j * RG) * a.r_stride);
+      x[j] = fold_load<T, V>(p + (r + j * RG) * a.r_stride);
       if (HAS_IDX) xi[j] = a.in_idx[in_off + l + (r + j * RG) * a.r_stride];
     }
 #pragma unroll
@@ -243,7 +269,7 @@ __global__ __launch_bounds__(FOLD_THREADS) void arg_col_kernel(ArgArgs a) {
 #pragma unroll
     for (int j = 0; j < U - 1; j++)
       if (r + j * RG < r1) {
-        x[j] = *reinterpret_cast<const FVec<T, V> *>(p + (r + j * RG) * a.r_stride);
+        x[j] = fold_load<T, V>(p + (r + j * RG) * a.r_stride);
         if (HAS_IDX) xi[j] = a.in_idx[in_off + l + (r + j * RG) * a.r_stride];
       }
 #pragma unroll
@@ -316,13 +342,9 @@ static int arg_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, co
   if (lane >= 0 && std::llabs(a.r_stride) > 1 && dims_fill(&a.kept, g.nk, g.kshape, g.kin, g.kout, lane)) {
     const int64_t L = g.kshape[lane], n_outer = g.n_out / L;
     constexpr int V = 16 / (int)sizeof(S) > 0 ? 16 / (int)sizeof(S) : 1;
-    bool vec = V > 1 && aligned_to16(ibase) && L % V == 0 && a.r_stride % V == 0;
-    for (int i = 0; vec && i < g.nk; i++)
-      if (i != lane && g.kin[i] % V != 0) vec = false;
-    const int v = vec ? V : 1;
     const bool rg4 = g.R >= 64;
     const int64_t lanes = rg4 ? FOLD_THREADS / 4 : FOLD_THREADS;
-    const int64_t lane_blocks = (L + lanes * v - 1) / (lanes * v);
+    const int64_t lane_blocks = (L + lanes * V - 1) / (lanes * V);
     const int64_t blocks = lane_blocks * n_outer;
     if (blocks <= 0x7fffffffLL) {
       // four blocks per unit, not eight: fewer partial rows for the second pass ([8192,8192] f32: 48.0 -> 45.6 us)
@@ -347,13 +369,8 @@ static int arg_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, co
       }
       nxh_set_path(nsplit > 1 ? "arg_col_split" : "arg_col");
       dim3 grid((unsigned)blocks, (unsigned)nsplit);
-      if (rg4) {
-        if (vec) hipLaunchKernelGGL((arg_col_kernel<InS<DT>, CMP, V, 4, false>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-        else hipLaunchKernelGGL((arg_col_kernel<InS<DT>, CMP, 1, 4, false>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-      } else {
-        if (vec) hipLaunchKernelGGL((arg_col_kernel<InS<DT>, CMP, V, 1, false>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-        else hipLaunchKernelGGL((arg_col_kernel<InS<DT>, CMP, 1, 1, false>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-      }
+      if (rg4) hipLaunchKernelGGL((arg_col_kernel<InS<DT>, CMP, V, 4, false>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
+      else hipLaunchKernelGGL((arg_col_kernel<InS<DT>, CMP, V, 1, false>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
       NXH_HIP(op, hipGetLastError());
       if (nsplit > 1) {
         ArgArgs b = a;
@@ -404,7 +421,7 @@ static int arg_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, co
   if (blocks > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "too many outputs for one launch");
   int nsplit = wave_rows ? 1 : pick_split(blocks, g.R, 8192, cus);
   int64_t chunk = (g.R + nsplit - 1) / nsplit;
-  if (nsplit > 1) chunk = (chunk + 63) / 64 * 64;  // keeps every chunk start 16-byte aligned
+  if (nsplit > 1) chunk = (chunk + 63) / 64 * 64;  // keeps the chunks of aligned rows aligned
   nsplit = (int)((g.R + chunk - 1) / chunk);
   a.chunk = chunk;
   a.nsplit = nsplit;
@@ -421,9 +438,7 @@ static int arg_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, co
   nxh_set_path(nsplit > 1 ? "arg_row_split" : (wave_rows ? "arg_row_wave" : "arg_row"));
   {
     constexpr int V = 16 / (int)sizeof(S) > 0 ? 16 / (int)sizeof(S) : 1;
-    bool vec = V > 1 && a.r_stride == 1 && aligned_to16(ibase) && (nsplit == 1 || chunk % V == 0);
-    for (int i = 0; vec && i < g.nk; i++)
-      if (g.kin[i] % V != 0) vec = false;
+    const bool vec = V > 1 && a.r_stride == 1;
     if (wave_rows) {
       if (vec) hipLaunchKernelGGL((arg_row_kernel<InS<DT>, CMP, 64, V, false>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
       else hipLaunchKernelGGL((arg_row_kernel<InS<DT>, CMP, 64, 1, false>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);

@@ -68,10 +68,10 @@ __global__ __launch_bounds__(FOLD_THREADS) void fold_row_kernel(RowArgs a) {
   const T *p = (const T *)a.in + in_off + (int64_t)c * a.split_stride;
   C acc0 = CB::init(), acc1 = CB::init(), acc2 = CB::init(), acc3 = CB::init();
   const int64_t nv = (r1 - r0) / V;
-  const FVec<T, V> *pv = reinterpret_cast<const FVec<T, V> *>(p + r0);
+  auto pv = [&](int64_t i) { return fold_load<T, V>(p + r0 + i * V); };
   int64_t i = lane;
   for (; i + 3 * G < nv; i += 4 * G) {
-    FVec<T, V> x0 = pv[i], x1 = pv[i + G], x2 = pv[i + 2 * G], x3 = pv[i + 3 * G];
+    FVec<T, V> x0 = pv(i), x1 = pv(i + G), x2 = pv(i + 2 * G), x3 = pv(i + 3 * G);
 #pragma unroll
     for (int k = 0; k < V; k++) {
       acc0 = CB::apply(acc0, IN::ld(x0.v[k]));
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(FOLD_THREADS) void fold_row_kernel(RowArgs a) {
     }
   }
   for (; i < nv; i += G) {
-    FVec<T, V> x0 = pv[i];
+    FVec<T, V> x0 = pv(i);
 #pragma unroll
     for (int k = 0; k < V; k++) acc0 = CB::apply(acc0, IN::ld(x0.v[k]));
   }
@@ -127,8 +127,11 @@ __global__ __launch_bounds__(FOLD_THREADS) void fold_col_kernel(ColArgs a) {
   const uint64_t ob = bx / a.lane_blocks;
   const int c = gridDim.y - 1 - blockIdx.y;
   const uint32_t ln = threadIdx.x % LANES, rg = threadIdx.x / LANES;
-  const uint32_t l = (lb * LANES + ln) * V;
-  const bool live = l < a.L;
+  const uint32_t l0 = (lb * LANES + ln) * V;
+  const bool live = l0 < a.L;
+  // (L >= V) a last lane whose columns would run over the edge takes the last V instead: the ones it
+  // shares with its neighbour come out of the same rows in the same order
+  const uint32_t l = l0 + V <= a.L ? l0 : a.L - V;
   int64_t in_off, out_off;
   fold_decode(a.outer, ob, in_off, out_off);
   const int64_t r0 = 0, before = (int64_t)c * a.chunk;
@@ -141,7 +144,7 @@ __global__ __launch_bounds__(FOLD_THREADS) void fold_col_kernel(ColArgs a) {
   for (; r + (U - 1) * RG < r1; r += U * RG) {
     FVec<T, V> x[U];
 #pragma unroll
-    for (int j = 0; j < U; j++) x[j] = *reinterpret_cast<const FVec<T, V> *>(p + (r + j * RG) * a.r_stride);
+    for (int j = 0; j < U; j++) x[j] = fold_load<T, V>(p + (r + j * RG) * a.r_stride);
 #pragma unroll
     for (int j = 0; j < U; j++)
 #pragma unroll
@@ -151,7 +154,7 @@ __global__ __launch_bounds__(FOLD_THREADS) void fold_col_kernel(ColArgs a) {
     FVec<T, V> x[U - 1];
 #pragma unroll
     for (int j = 0; j < U - 1; j++)
-      if (r + j * RG < r1) x[j] = *reinterpret_cast<const FVec<T, V> *>(p + (r + j * RG) * a.r_stride);
+      if (r + j * RG < r1) x[j] = fold_load<T, V>(p + (r + j * RG) * a.r_stride);
 #pragma unroll
     for (int j = 0; j < U - 1; j++)
       if (r + j * RG < r1)
@@ -353,15 +356,12 @@ static int fold_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, c
       int64_t chunk = run;
       if (!row_two && nsplit > 1) {
         chunk = (g.R + nsplit - 1) / nsplit;
-        chunk = (chunk + 63) / 64 * 64;  // keeps every chunk start 16-byte aligned
+        chunk = (chunk + 63) / 64 * 64;  // keeps the chunks of aligned rows aligned
         nsplit = (int)((g.R + chunk - 1) / chunk);
       }
       a.chunk = chunk;
       a.split_stride = row_two ? g.rin[1 - row_dim] : chunk;
       a.nsplit = nsplit;
-      bool vec = aligned_to16(ibase) && (!row_two || a.split_stride % V == 0);
-      for (int i = 0; vec && i < g.nk; i++)
-        if (g.kin[i] % V != 0) vec = false;
       if (nsplit > 1) {
         int rc = scratch.get(0, (size_t)g.n_out * nsplit * sizeof(C));
         if (rc) return rc;
@@ -371,13 +371,8 @@ static int fold_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, c
       }
       dim3 grid((unsigned)blocks, (unsigned)nsplit);
       nxh_set_path(row_two ? "fold_row_outer" : nsplit > 1 ? "fold_row_split" : (wave_rows ? "fold_row_wave" : "fold_row"));
-      if (wave_rows) {
-        if (vec) hipLaunchKernelGGL((fold_row_kernel<InS<DT>, CB, OutS<DT>, 64, V>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-        else hipLaunchKernelGGL((fold_row_kernel<InS<DT>, CB, OutS<DT>, 64, 1>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-      } else {
-        if (vec) hipLaunchKernelGGL((fold_row_kernel<InS<DT>, CB, OutS<DT>, 256, V>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-        else hipLaunchKernelGGL((fold_row_kernel<InS<DT>, CB, OutS<DT>, 256, 1>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-      }
+      if (wave_rows) hipLaunchKernelGGL((fold_row_kernel<InS<DT>, CB, OutS<DT>, 64, V>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
+      else hipLaunchKernelGGL((fold_row_kernel<InS<DT>, CB, OutS<DT>, 256, V>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
       NXH_HIP(op, hipGetLastError());
       if (nsplit > 1) {
         RowArgs b = a;
@@ -463,14 +458,11 @@ static int fold_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, c
         dims_fill(&a.outer, g.nk, g.kshape, g.kin, g.kout, lane)) {
       const int64_t L = g.kshape[lane];
       const int64_t n_outer = g.n_out / L;
-      bool vec = aligned_to16(ibase) && L % V == 0 && run_stride % V == 0 && (!col_two || g.rin[1 - walk] % V == 0);
-      for (int i = 0; vec && i < g.nk; i++)
-        if (i != lane && g.kin[i] % V != 0) vec = false;
-      const int v = vec ? V : 1;
       // long reduced runs: 4 row groups per block (see fold_col_kernel)
       const bool rg4 = run >= 64;
       const int64_t lanes = rg4 ? FOLD_THREADS / 4 : FOLD_THREADS;
-      const int64_t lane_blocks = (L + lanes * v - 1) / (lanes * v);
+      static_assert(V <= 16 && VC <= 16, "the lane dim holds a vector");
+      const int64_t lane_blocks = (L + lanes * V - 1) / (lanes * V);
       const int64_t blocks = lane_blocks * n_outer;
       if (blocks <= 0x7fffffffLL) {
         int nsplit = col_two ? (int)g.rshape[1 - walk] : pick_split(blocks, g.R, rg4 ? 64 : 16, cus);
@@ -498,13 +490,8 @@ static int fold_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, c
         }
         dim3 grid((unsigned)blocks, (unsigned)nsplit);
         nxh_set_path(col_two ? "fold_col_outer" : nsplit > 1 ? "fold_col_split" : "fold_col");
-        if (rg4) {
-          if (vec) hipLaunchKernelGGL((fold_col_kernel<InS<DT>, CB, OutS<DT>, V, 4>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-          else hipLaunchKernelGGL((fold_col_kernel<InS<DT>, CB, OutS<DT>, 1, 4>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-        } else {
-          if (vec) hipLaunchKernelGGL((fold_col_kernel<InS<DT>, CB, OutS<DT>, V, 1>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-          else hipLaunchKernelGGL((fold_col_kernel<InS<DT>, CB, OutS<DT>, 1, 1>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
-        }
+        if (rg4) hipLaunchKernelGGL((fold_col_kernel<InS<DT>, CB, OutS<DT>, V, 4>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
+        else hipLaunchKernelGGL((fold_col_kernel<InS<DT>, CB, OutS<DT>, V, 1>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a);
         NXH_HIP(op, hipGetLastError());
         if (nsplit > 1) {
           // the partial rows [nsplit][n_outer * L] are folded the same way
@@ -517,26 +504,17 @@ static int fold_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, c
           b.chunk = nsplit;
           b.split_stride = 0;
           b.nsplit = 1;
-          const bool vec2 = L % VC == 0;
-          const int v2 = vec2 ? VC : 1;
           // 48 partial rows or more: sixteen row groups of four loads each, so that a lane's whole
           // share is in flight at once and four times as many blocks carry the launch (the second
           // pass is all latency: [64][8192] f32 partials, 2 MiB)
           const bool rg16b = nsplit >= 48;
           const bool rg4b = nsplit >= 16;
           const int64_t lanes2 = rg16b ? FOLD_THREADS / 16 : rg4b ? FOLD_THREADS / 4 : FOLD_THREADS;
-          b.lane_blocks = (uint32_t)((L + lanes2 * v2 - 1) / (lanes2 * v2));
+          b.lane_blocks = (uint32_t)((L + lanes2 * VC - 1) / (lanes2 * VC));
           dim3 grid2((unsigned)(b.lane_blocks * n_outer), 1);
-          if (rg16b) {
-            if (vec2) hipLaunchKernelGGL((fold_col_kernel<InC<C>, CB, OutS<DT>, VC, 16, 4>), grid2, dim3(FOLD_THREADS), 0, ctx->stream, b);
-            else hipLaunchKernelGGL((fold_col_kernel<InC<C>, CB, OutS<DT>, 1, 16, 4>), grid2, dim3(FOLD_THREADS), 0, ctx->stream, b);
-          } else if (rg4b) {
-            if (vec2) hipLaunchKernelGGL((fold_col_kernel<InC<C>, CB, OutS<DT>, VC, 4>), grid2, dim3(FOLD_THREADS), 0, ctx->stream, b);
-            else hipLaunchKernelGGL((fold_col_kernel<InC<C>, CB, OutS<DT>, 1, 4>), grid2, dim3(FOLD_THREADS), 0, ctx->stream, b);
-          } else {
-            if (vec2) hipLaunchKernelGGL((fold_col_kernel<InC<C>, CB, OutS<DT>, VC, 1>), grid2, dim3(FOLD_THREADS), 0, ctx->stream, b);
-            else hipLaunchKernelGGL((fold_col_kernel<InC<C>, CB, OutS<DT>, 1, 1>), grid2, dim3(FOLD_THREADS), 0, ctx->stream, b);
-          }
+          if (rg16b) hipLaunchKernelGGL((fold_col_kernel<InC<C>, CB, OutS<DT>, VC, 16, 4>), grid2, dim3(FOLD_THREADS), 0, ctx->stream, b);
+          else if (rg4b) hipLaunchKernelGGL((fold_col_kernel<InC<C>, CB, OutS<DT>, VC, 4>), grid2, dim3(FOLD_THREADS), 0, ctx->stream, b);
+          else hipLaunchKernelGGL((fold_col_kernel<InC<C>, CB, OutS<DT>, VC, 1>), grid2, dim3(FOLD_THREADS), 0, ctx->stream, b);
           NXH_HIP(op, hipGetLastError());
         }
         return NXH_OK;
