@@ -213,6 +213,10 @@ int nxh_gather(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *data,
    that an out-of-bounds index is reported by this call. */
 int nxh_scatter(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *indices,
                 const nxh_tensor *updates, int axis, int mode);
+/* nxh_copy of `from` into `out`, then nxh_scatter (nx_backend.ml:412-416): in one pass
+   over the table where the updates are whole rows of it. */
+int nxh_scatter_from(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *from,
+                     const nxh_tensor *indices, const nxh_tensor *updates, int axis, int mode);
 /* caml_nx_c_pad (nx_c_move.c:203-276): out = x widened by pad_before[d] elements
    in front of every axis d (the rest of out's extent behind it), the border
    holding *fill_value (one storage element of the dtype, host memory; the

@@ -101,6 +101,7 @@ SIGNATURES = {
     "nxh_matmul": (C.c_int, [_CTX, _T, _T, _T]),
     "nxh_copy": (C.c_int, [_CTX, _T, _T]),
     "nxh_scatter": (C.c_int, [_CTX, _T, _T, _T, C.c_int, C.c_int]),
+    "nxh_scatter_from": (C.c_int, [_CTX, _T, _T, _T, _T, C.c_int, C.c_int]),
     "nxh_pad": (C.c_int, [_CTX, _T, _T, C.c_void_p, C.POINTER(C.c_int64)]),
     "nxh_cat": (C.c_int, [_CTX, _T, C.POINTER(_T), C.c_int, C.c_int]),
     "nxh_scan": (C.c_int, [_CTX, C.c_int, _T, _T, C.c_int]),

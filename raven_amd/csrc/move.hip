@@ -37,6 +37,12 @@ struct alignas(16) G16 {
   uint64_t lo, hi;
 };
 
+// The flag is pinned host memory: a plain store of the one value it can take, seen by the host
+// once the stream has been waited for.
+__device__ __forceinline__ void raise_fault(int *flag) {
+  __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 struct GatherRowsArgs {
   const char *data;
   char *out;
@@ -53,7 +59,7 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(GatherRowsArgs a) {
   int64_t index = a.idx[row * a.idx_stride];
   if (index < 0) index += a.axis_len;
   if (index < 0 || index >= a.axis_len) {
-    if ((threadIdx.x & 63) == 0) atomicOr(a.fault, 1);
+    if ((threadIdx.x & 63) == 0) raise_fault(a.fault);
     return;
   }
   const V *src = reinterpret_cast<const V *>(a.data + index * a.data_row_stride * a.esize);
@@ -93,7 +99,7 @@ __global__ __launch_bounds__(256) void gather_any_kernel(GatherAnyArgs a) {
   int64_t index = a.idx[io];
   if (index < 0) index += a.axis_len;
   if (index < 0 || index >= a.axis_len) {
-    atomicOr(a.fault, 1);
+    raise_fault(a.fault);
     return;
   }
   doff += index * a.dstride[a.axis];
@@ -165,7 +171,7 @@ NXH_EXPORT int nxh_gather(nxh_context *ctx, const nxh_tensor *out, const nxh_ten
     a.row_bytes = out->shape[1] * es;
     a.axis_len = data->shape[0];
     a.esize = es;
-    a.fault = ctx->fault_flag;
+    a.fault = ctx->fault_flag_host;
     if (out->shape[0] == 1) a.out_row_stride = 0;
     if (data->shape[0] == 1) a.data_row_stride = 0;
     const unsigned blocks = (unsigned)((a.rows + 3) / 4);
@@ -192,7 +198,7 @@ NXH_EXPORT int nxh_gather(nxh_context *ctx, const nxh_tensor *out, const nxh_ten
       a.istride[d] = indices->strides[d];
       a.ostride[d] = out->strides[d];
     }
-    a.fault = ctx->fault_flag;
+    a.fault = ctx->fault_flag_host;
     if (total > 0x7fffffffLL * 256) return nxh_fail(NXH_FAILURE, op, "too many elements for one launch");
     nxh_set_path("gather_any");
     switch (es) {
@@ -218,6 +224,7 @@ struct ScatterArgs {
   int64_t cshape[NXH_MAX_NDIM];
   int64_t c_ostride[NXH_MAX_NDIM], c_istride[NXH_MAX_NDIM], c_ustride[NXH_MAX_NDIM];
   int64_t a_ostride, a_istride, a_ustride;  // along the scatter axis
+  const char *from;  // scatter_rows: what `out` starts as, laid out as it is (null: out already holds it)
   int *fault;
 };
 // ADD: accumulate in the dtype's compute type; otherwise a byte-exact store.
@@ -267,7 +274,7 @@ __global__ __launch_bounds__(256) void scatter_kernel(ScatterArgs a) {
       u[j] = upd[(i + j) * a.a_ustride];
     }
     if (!ok) {
-      atomicOr(a.fault, 1);
+      raise_fault(a.fault);
       return;
     }
     bool distinct = true;
@@ -298,7 +305,7 @@ __global__ __launch_bounds__(256) void scatter_kernel(ScatterArgs a) {
     int64_t index = idx[i * a.a_istride];
     if (index < 0) index += a.axis_len;
     if (index < 0 || index >= a.axis_len) {
-      atomicOr(a.fault, 1);
+      raise_fault(a.fault);
       return;
     }
     apply(out + index * a.a_ostride, upd[i * a.a_ustride]);
@@ -315,6 +322,8 @@ __global__ __launch_bounds__(256) void scatter_kernel(ScatterArgs a) {
 // at a time when their targets are pairwise distinct. Outputs of different
 // blocks are disjoint and each lane sees its column's updates in the serial
 // order, so the result is the reference's.
+// `from`: the lane first copies its columns of the range's rows from there; the updates that follow
+// find them in L2, and there is one launch instead of a copy and a walk.
 // With V > 1 a lane owns V adjacent columns, moved as one 16-byte vector (the columns of `out`
 // and `updates` are then contiguous and every row starts on a 16-byte boundary: checked on the
 // host); a.columns counts lanes.
@@ -364,6 +373,19 @@ __global__ __launch_bounds__(256) void scatter_rows_kernel(ScatterArgs a, int64_
       return u;
     }
   };
+  if (a.from && live) {
+    const S *from = reinterpret_cast<const S *>(reinterpret_cast<const E *>(a.from) + oo);
+    const int64_t end = hi < a.axis_len ? hi : a.axis_len;
+    int64_t r = lo;
+    for (; r + 8 <= end; r += 8) {
+      S x[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) x[j] = from[(r + j) * a_os];
+#pragma unroll
+      for (int j = 0; j < 8; j++) out[(r + j) * a_os] = x[j];
+    }
+    for (; r < end; r++) out[r * a_os] = from[r * a_os];
+  }
   for (int64_t base = 0; base < a.n_idx; base += SPAN) {
     int t[SCAN];  // targets index an axis of the output checked to fit 31 bits
     bool bad = false;
@@ -377,7 +399,7 @@ __global__ __launch_bounds__(256) void scatter_rows_kernel(ScatterArgs a, int64_
     }
     // also separates this pass's LDS writes from the last pass's reads
     if (__syncthreads_or(bad)) {
-      if (threadIdx.x == 0) atomicOr(a.fault, 1);
+      if (threadIdx.x == 0) raise_fault(a.fault);
       return;
     }
     uint64_t hits[SCAN];
@@ -591,9 +613,10 @@ static int scatter_sorted(nxh_context *ctx, const char *op, const ScatterArgs &a
   return rc;
 }
 
-NXH_EXPORT int nxh_scatter(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *indices,
-                           const nxh_tensor *updates, int axis, int mode) {
-  NXH_DEFER_TOUCH(ctx, 1, out, indices, updates);
+// `from`: null, or a tensor laid out as `out`, of other memory, that out becomes a copy of first; -1 when
+// the call is not one that copies and scatters in one pass.
+static int scatter_impl(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *from, const nxh_tensor *indices,
+                        const nxh_tensor *updates, int axis, int mode) {
   const char *op = "scatter";
   if (!ctx || !out || !indices || !updates) return nxh_fail(NXH_INVALID_ARGUMENT, op, "null argument");
   int rc = nxh_check_tensor(op, out);
@@ -625,17 +648,19 @@ NXH_EXPORT int nxh_scatter(nxh_context *ctx, const nxh_tensor *out, const nxh_te
     a.ncol_dims++;
   }
   a.n_idx = indices->shape[axis];
+  if (from && (a.columns <= 1 || a.n_idx == 0)) return -1;
   if (a.columns == 0 || a.n_idx == 0) return NXH_OK;
   if (a.columns > 0x7fffffffLL * 256) return nxh_fail(NXH_FAILURE, op, "too many elements for one launch");
   const int64_t es = nxh_elem_size(dt);
   a.out = (char *)out->data + out->offset * es;
   a.idx = (const int32_t *)indices->data + indices->offset;
   a.upd = (const char *)updates->data + updates->offset * es;
+  a.from = from ? (const char *)from->data + from->offset * es : nullptr;
   a.axis_len = out->shape[axis];
   a.a_ostride = out->strides[axis];
   a.a_istride = indices->strides[axis];
   a.a_ustride = updates->strides[axis];
-  a.fault = ctx->fault_flag;
+  a.fault = ctx->fault_flag_host;
   struct Table {
     scatter_launch_fn fn[NXH_DTYPE_COUNT] = {};
     Table() {
@@ -651,9 +676,6 @@ NXH_EXPORT int nxh_scatter(nxh_context *ctx, const nxh_tensor *out, const nxh_te
     const int src = scatter_sorted(ctx, op, a, dt, mode == 1);
     if (src != -1) return src;
   }
-  std::lock_guard<std::mutex> guard(ctx->mu);
-  NXH_HIP(op, hipSetDevice(ctx->device));
-  if (int frc = nxh_settle_replay_faults(ctx, op)) return frc;
   // Too few columns to fill the chip and one index per axis position: split the
   // targets over blocks too. The index list is read once per block, so this
   // pays only while the list is short next to the rows it spreads over.
@@ -664,7 +686,7 @@ NXH_EXPORT int nxh_scatter(nxh_context *ctx, const nxh_tensor *out, const nxh_te
   // run, a whole number of vectors long, and every row of both starts on a 16-byte boundary
   // (embedding gradient [8192, 768] f32 into [50257, 768]: 38 -> 33 us)
   bool vec = uniform_index && es < 16 && a.columns % (16 / es) == 0 && a.a_ostride % (16 / es) == 0 &&
-             a.a_ustride % (16 / es) == 0 && ((uintptr_t)a.out | (uintptr_t)a.upd) % 16 == 0;
+             a.a_ustride % (16 / es) == 0 && ((uintptr_t)a.out | (uintptr_t)a.upd | (uintptr_t)a.from) % 16 == 0;
   for (int64_t d = a.ncol_dims - 1, run = 1; d >= 0 && vec; d--) {
     if (a.cshape[d] > 1 && (a.c_ostride[d] != run || a.c_ustride[d] != run)) vec = false;
     run *= a.cshape[d];
@@ -673,18 +695,58 @@ NXH_EXPORT int nxh_scatter(nxh_context *ctx, const nxh_tensor *out, const nxh_te
   const int64_t lanes = vec ? a.columns / (16 / es) : a.columns;
   const int64_t col_blocks = (lanes + 255) / 256;
   const int64_t want_blocks = (int64_t)ctx->compute_units * 3;  // measured best on the embedding-gradient shape
-  if (uniform_index && a.n_idx >= 256 && col_blocks * 4 <= want_blocks) {
+  if (uniform_index && (a.n_idx >= 256 || from) && col_blocks * 4 <= want_blocks) {
     int64_t ranges = want_blocks / col_blocks;
     if (ranges > a.axis_len) ranges = a.axis_len;
     if (ranges > 65535) ranges = 65535;
     if (ranges >= 2) range_rows = (a.axis_len + ranges - 1) / ranges;
   }
+  // One pass pays while a launch and its gap are a share of the call: a table of 64 MiB at most
+  // ([34828,369] float32 with 195 updates, with the gather before it: 102 -> 77 us; [50257,768], 154 MB: the
+  // blocks copy and update in step, 191 us against 145 for two launches).
+  if (from && (range_rows == 0 || a.n_idx > 4 * a.axis_len || a.axis_len * a.columns * es > (64 << 20))) return -1;
+  std::lock_guard<std::mutex> guard(ctx->mu);
+  NXH_HIP(op, hipSetDevice(ctx->device));
+  if (int frc = nxh_settle_replay_faults(ctx, op)) return frc;
   vec = vec && range_rows > 0;
   if (vec) a.columns = lanes;
   nxh_set_path(vec ? "scatter_rows_16B" : range_rows > 0 ? "scatter_rows" : "scatter_columns");
   table[dt](ctx, a, mode == 1, range_rows, vec);
   NXH_HIP(op, hipGetLastError());
   return nxh_collect_index_fault(ctx, op);
+}
+
+NXH_EXPORT int nxh_scatter(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *indices,
+                           const nxh_tensor *updates, int axis, int mode) {
+  NXH_DEFER_TOUCH(ctx, 1, out, indices, updates);
+  return scatter_impl(ctx, out, nullptr, indices, updates, axis, mode);
+}
+
+// out = a copy of `from`, then the updates: nxh_copy and nxh_scatter, in one pass where the updates are
+// whole rows of a dense table that does not overlap `out`.
+NXH_EXPORT int nxh_scatter_from(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *from, const nxh_tensor *indices,
+                                const nxh_tensor *updates, int axis, int mode) {
+  auto dense = [](const nxh_tensor *t) {
+    int64_t s = 1;
+    for (int d = t->ndim - 1; d >= 0; d--) {
+      if (t->shape[d] != 1 && t->strides[d] != s) return (int64_t)0;
+      s *= t->shape[d];
+    }
+    return s;
+  };
+  if (ctx && out && from && nxh_check_tensor("scatter", out) == NXH_OK && nxh_check_tensor("scatter", from) == NXH_OK &&
+      !nxh_is_packed(out->dtype) && out->dtype == from->dtype && out->ndim == from->ndim &&
+      std::equal(out->shape, out->shape + out->ndim, from->shape)) {
+    const int64_t n = dense(out), es = nxh_elem_size(out->dtype);
+    const char *o = (const char *)out->data + out->offset * es, *f = (const char *)from->data + from->offset * es;
+    if (n > 0 && dense(from) == n && (o + n * es <= f || f + n * es <= o)) {
+      NXH_DEFER_TOUCH(ctx, 1, out, from, indices, updates);
+      const int rc = scatter_impl(ctx, out, from, indices, updates, axis, mode);
+      if (rc != -1) return rc;
+    }
+  }
+  if (const int rc = nxh_copy(ctx, out, from)) return rc;
+  return nxh_scatter(ctx, out, indices, updates, axis, mode);
 }
 
 // ── threefry2x32-20 ─────────────────────────────────────────────────────────

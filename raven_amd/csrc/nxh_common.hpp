@@ -41,8 +41,8 @@ struct nxh_context {
   std::map<void *, size_t> live;  // every block handed out or cached -> its class size
   uint64_t in_use = 0, cached = 0, reserved = 0, driver_allocs = 0;
   // one device word, written by kernels that detect a data fault (gather OOB)
-  int *fault_flag = nullptr;       // device
-  int *fault_flag_host = nullptr;  // pinned host mirror for the readback
+  int *fault_flag = nullptr;       // device words of the factorisations
+  int *fault_flag_host = nullptr;  // pinned host words: [0] is raised by gather and scatter, the rest mirror the device's
   // pinned staging slots for small host-to-device uploads: the caller's bytes
   // are copied into a slot and the transfer is queued on the stream, so an
   // upload does not wait for the work already queued

@@ -371,10 +371,9 @@ class Backend:
                 axis: int) -> Tensor:
         """``mode`` is "set" or "add"; ``unique_indices`` is accepted and ignored,
         as in the reference binding. The result starts as a copy of ``template``."""
-        out = self.copy(template)
-        o, i, u = out._desc(), indices._desc(), updates._desc()
-        self._check(self._lib.nxh_scatter(self._h, C.byref(o), C.byref(i), C.byref(u), axis,
-                                          {"set": 0, "add": 1}[mode]))
+        out = self.buffer(template.dtype, template.shape)
+        o, t, i, u = out._desc(), template._desc(), indices._desc(), updates._desc()
+        self._check(self._lib.nxh_scatter_from(self._h, o, t, i, u, axis, {"set": 0, "add": 1}[mode]))
         return out
 
     def pad(self, x: Tensor, padding: Sequence[Sequence[int]], fill_value) -> Tensor:

@@ -95,6 +95,8 @@ external caml_argreduce : bool -> (int32, Dtype.int32_elt) t -> ('a, 'b) t -> in
 external caml_matmul : ('a, 'b) t -> ('a, 'b) t -> ('a, 'b) t -> unit = "caml_nx_hip_matmul"
 external caml_gather : ('a, 'b) t -> ('a, 'b) t -> (int32, Dtype.int32_elt) t -> int -> unit = "caml_nx_hip_gather"
 external caml_scatter : ('a, 'b) t -> (int32, Dtype.int32_elt) t -> ('a, 'b) t -> int -> int -> unit = "caml_nx_hip_scatter"
+external caml_scatter_from : ('a, 'b) t -> ('a, 'b) t -> (int32, Dtype.int32_elt) t -> ('a, 'b) t -> int -> int -> unit
+  = "caml_nx_hip_scatter_from_bc" "caml_nx_hip_scatter_from"
 external caml_pad : ('a, 'b) t -> ('a, 'b) t -> ('a, 'b) Nx_buffer.t -> int array -> unit = "caml_nx_hip_pad"
 external caml_cat : ('a, 'b) t -> ('a, 'b) t array -> int -> unit = "caml_nx_hip_cat"
 external caml_scan : int -> ('a, 'b) t -> ('a, 'b) t -> int -> unit = "caml_nx_hip_scan"
@@ -274,8 +276,8 @@ let cat tensors ~axis =
 
 (* nx_backend.ml:412-416 *)
 let scatter ~mode ~unique_indices:_ template ~indices ~updates ~axis =
-  let out = copy template in
-  caml_scatter out indices updates axis (match mode with `Set -> 0 | `Add -> 1); out
+  let out = create_tensor template.context template.dtype template.shape in
+  caml_scatter_from out template indices updates axis (match mode with `Set -> 0 | `Add -> 1); out
 
 (* nx_backend.ml:474-477 *)
 let threefry key counter =

@@ -33,7 +33,7 @@
   X(context_create) X(context_destroy) X(last_error) X(alloc) X(free)         \
   X(memcpy_h2d) X(memcpy_d2h) X(synchronize) X(fill) X(unary) X(binary)       \
   X(compare) X(where) X(cast) X(reduce) X(argreduce) X(matmul) X(copy)        \
-  X(gather) X(scatter) X(pad) X(cat) X(scan) X(threefry) X(dtype_bytes)       \
+  X(gather) X(scatter) X(scatter_from) X(pad) X(cat) X(scan) X(threefry) X(dtype_bytes)       \
   X(sort) X(argsort) X(unfold) X(fold) X(fft) X(rfft) X(irfft) X(cholesky)    \
   X(triangular_solve) X(qr) X(eigh) X(svd) X(eig) X(device_info)              \
   X(memory_stats) X(trim) X(reduce_noalloc) X(softmax_rows) X(layer_norm_rows) \
@@ -339,6 +339,24 @@ CAMLprim value caml_nx_hip_scatter(value vout, value vidx, value vupd, value vax
   caml_leave_blocking_section();
   check(c, rc);
   CAMLreturn(Val_unit);
+}
+CAMLprim value caml_nx_hip_scatter_from(value vout, value vfrom, value vidx, value vupd, value vaxis, value vmode) {
+  CAMLparam5(vout, vfrom, vidx, vupd, vaxis);
+  CAMLxparam1(vmode);
+  nxh_tensor o, f, i, u;
+  nxh_context *c = extract(vout, &o);
+  extract(vfrom, &f);
+  extract(vidx, &i);
+  extract(vupd, &u);
+  caml_enter_blocking_section();
+  int rc = L.scatter_from(c, &o, &f, &i, &u, Int_val(vaxis), Int_val(vmode));
+  caml_leave_blocking_section();
+  check(c, rc);
+  CAMLreturn(Val_unit);
+}
+CAMLprim value caml_nx_hip_scatter_from_bc(value *argv, int argn) {
+  (void)argn;
+  return caml_nx_hip_scatter_from(argv[0], argv[1], argv[2], argv[3], argv[4], argv[5]);
 }
 /* the fill value arrives as a 1-element host Nx_buffer, like caml_nx_hip_fill */
 CAMLprim value caml_nx_hip_pad(value vout, value vx, value vfill, value vbefore) {
