@@ -464,18 +464,24 @@ __global__ __launch_bounds__(256) void psort_reg_kernel(SortArgs a) {
 // descending value sort wants its ties in descending index order and its NaNs in ascending:
 // it sorts ascending and writes the non-NaN prefix out reversed, which is how the reference
 // defines it (nx_c_sort.c:283-289).
-// One pass is four launches: a histogram of the digit per 4096-word tile, laid out bin by
-// bin ([256][tiles], so that its exclusive scan is a tile's first output position for each
-// digit), the scan in two levels (segments of 4096 entries, then the segment totals), and the
-// scatter, in which every tile ranks its words stably: a wave owns 1024 consecutive words,
-// takes them 64 at a time in order, finds for each lane the lanes with the same digit by
-// eight ballots, and keeps a running count per digit; the waves' counts are then offset
-// against each other. No inter-block waiting anywhere.
+// One pass is two launches: a histogram of the digit per 4096-word tile, and the scatter, in
+// which every tile adds up the slice's histograms for its own first output position of each
+// digit (a 50 257-element slice has 13 tiles: 13 KiB out of L2) and ranks its words stably: a
+// wave owns 1024 consecutive words, takes them 64 at a time in order, finds for each lane the
+// lanes with the same digit by eight ballots, and keeps a running count per digit; the waves'
+// counts are then offset against each other. No inter-block waiting anywhere. The first pass
+// packs its words out of the input and the last one writes the results, so the words cross memory
+// once per pass and no more. Measured at [64,50257] float32, argsort: bound by each pass's latency
+// chain (load, rank, LDS, scattered store) on 3.3 blocks a unit; see radix_run for the figures.
+// Slices of more than RX_SHORT tiles lay the histograms out bin by bin ([256][tiles], so that
+// their exclusive scan is a tile's first output position for each digit) and scan them in two
+// further launches (segments of 4096 entries, then the segment totals).
 // Digits that cannot change the order are skipped: the low bits of a widened 16- or 8-bit
 // float, and the sign-extension bytes of a narrow integer, are functions of higher bits.
 constexpr int RX_TILE = 4096;
 constexpr int RX_ROWS = RX_TILE / 256;
 constexpr int RX_SEG = 4096;
+constexpr int RX_SHORT = 32;  // tiles whose histograms a tile adds up by itself
 
 template <int DT>
 constexpr int rx_pass_mask() {  // bit p: the pass over bits 8p .. 8p+7 of the mapped value is needed
@@ -493,8 +499,9 @@ constexpr int rx_pass_mask() {  // bit p: the pass over bits 8p .. 8p+7 of the m
 struct RadixArgs {
   const uint64_t *src;
   uint64_t *dst;
-  uint32_t *hist;  // [slices][256 * nblk], bin-major; after the scans: exclusive inside its segment
-  uint32_t *seg;   // [slices][nseg]: segment totals, then their exclusive scan
+  uint32_t *hist;  // [slices][nblk][256]; more than RX_SHORT tiles: [slices][256][nblk], after the scans exclusive inside its segment
+  uint32_t *seg;   // (more than RX_SHORT tiles) [slices][nseg]: segment totals, then their exclusive scan
+  uint32_t *nan_count;  // of each slice, where the results need it
   int64_t slices, n;
   int nblk, nseg, shift;
 };
@@ -504,40 +511,45 @@ __global__ __launch_bounds__(256) void rx_zero_kernel(uint32_t *p, int64_t count
   if (i < count) p[i] = 0;
 }
 
-// Packs the slices into words (position = index); counts the NaN words of each slice.
-template <int DT, int PM, bool COUNT_NAN>
-__global__ __launch_bounds__(256) void rx_pack_kernel(SortArgs a, uint64_t *w, uint32_t *nan_count, int nblk) {
-  using TR = Tr<DT>;
-  using S = typename TR::S;
-  const int64_t s = blockIdx.x / nblk, base = (int64_t)(blockIdx.x % nblk) * RX_TILE;
-  int64_t io, oo;
-  slice_offsets(a, s, io, oo);
-  uint32_t nans = 0;
-  for (int e = threadIdx.x; e < RX_TILE; e += 256) {
-    const int64_t i = base + e;
-    if (i >= a.n) break;
-    const uint64_t word = Packed<DT>::template pack<PM>(TR::ld(reinterpret_cast<const S *>(a.in)[io + i * a.in_axis]), (uint32_t)i);
-    w[s * a.n + i] = word;
-    nans += (uint32_t)(word >> 32) == Packed<DT>::K_NAN && TR::cat == CAT_FLOAT;
-  }
-  if constexpr (COUNT_NAN) {
-    if (TR::cat == CAT_FLOAT && nans) atomicAdd(nan_count + s, nans);
+// Word `i` of a slice: packed out of the input (FIRST), or read.
+template <int DT, int PM, bool FIRST>
+__device__ __forceinline__ uint64_t rx_word(const SortArgs &a, const uint64_t *src, int64_t io, int64_t i) {
+  if constexpr (FIRST) {
+    using TR = Tr<DT>;
+    return Packed<DT>::template pack<PM>(TR::ld(reinterpret_cast<const typename TR::S *>(a.in)[io + i * a.in_axis]), (uint32_t)i);
+  } else {
+    return src[i];
   }
 }
 
-__global__ __launch_bounds__(256) void rx_hist_kernel(RadixArgs r) {
+// The digit's histogram of every tile; with COUNT_NAN also the NaN words of each slice.
+template <int DT, int PM, bool FIRST, bool COUNT_NAN>
+__global__ __launch_bounds__(256) void rx_hist_kernel(SortArgs a, RadixArgs r) {
   __shared__ uint32_t h[256];
   const int64_t s = blockIdx.x / r.nblk;
   const int blk = (int)(blockIdx.x % r.nblk);
+  int64_t io = 0, oo = 0;
+  if constexpr (FIRST) slice_offsets(a, s, io, oo);
   h[threadIdx.x] = 0;
   __syncthreads();
   const uint64_t *src = r.src + s * r.n;
-  for (int e = threadIdx.x; e < RX_TILE; e += 256) {
-    const int64_t i = (int64_t)blk * RX_TILE + e;
-    if (i < r.n) atomicAdd(&h[(uint32_t)(src[i] >> r.shift) & 255u], 1u);
+  const int64_t i0 = (int64_t)blk * RX_TILE + threadIdx.x;
+  uint64_t w[RX_ROWS];  // all of a lane's loads are in flight before the first is counted
+#pragma unroll
+  for (int q = 0; q < RX_ROWS; q++)
+    if (i0 + q * 256 < r.n) w[q] = rx_word<DT, PM, FIRST>(a, src, io, i0 + q * 256);
+  uint32_t nans = 0;
+#pragma unroll
+  for (int q = 0; q < RX_ROWS; q++)
+    if (i0 + q * 256 < r.n) {
+      atomicAdd(&h[(uint32_t)(w[q] >> r.shift) & 255u], 1u);
+      if constexpr (COUNT_NAN && Tr<DT>::cat == CAT_FLOAT) nans += (uint32_t)(w[q] >> 32) == Packed<DT>::K_NAN;
+    }
+  if constexpr (COUNT_NAN && Tr<DT>::cat == CAT_FLOAT) {
+    if (nans) atomicAdd(r.nan_count + s, nans);
   }
   __syncthreads();
-  r.hist[s * 256 * r.nblk + (int64_t)threadIdx.x * r.nblk + blk] = h[threadIdx.x];
+  r.hist[s * 256 * r.nblk + (r.nblk <= RX_SHORT ? (int64_t)blk * 256 + threadIdx.x : (int64_t)threadIdx.x * r.nblk + blk)] = h[threadIdx.x];
 }
 
 // Exclusive scan of 256 per-thread values across the block; returns this thread's offset and
@@ -599,7 +611,40 @@ __global__ __launch_bounds__(256) void rx_scan_totals_kernel(RadixArgs r) {
   }
 }
 
-__global__ __launch_bounds__(256) void rx_scatter_kernel(RadixArgs r) {
+// Writes result `i` of a slice from its word.
+template <int DT, int PM>
+__device__ __forceinline__ void rx_store(const SortArgs &a, int64_t io, int64_t oo, int64_t i, uint64_t word) {
+  if constexpr (PM == VALUE_ASC) {
+    // The value is the mapped key read backwards; only a zero (both signs share a key) and a
+    // NaN (its payload is not in the key) are fetched from the input through the index. A
+    // gather for every element cost a third of the whole sort.
+    using TR = Tr<DT>;
+    using C = typename TR::C;
+    using S = typename TR::S;
+    const uint32_t m = (uint32_t)(word >> 32);
+    bool direct = true;
+    C x;
+    if constexpr (TR::cat == CAT_FLOAT) {
+      direct = m != Packed<DT>::K_NAN && m != 0x80000000u;
+      const uint32_t u = (m & 0x80000000u) ? m ^ 0x80000000u : ~m;
+      x = (C)__builtin_bit_cast(float, u);
+    } else if constexpr (TR::cat == CAT_SINT) {
+      x = (C)(int32_t)(m ^ 0x80000000u);
+    } else {
+      x = (C)m;
+    }
+    if (direct) {
+      reinterpret_cast<S *>(a.out)[oo + i * a.out_axis] = TR::st(x);
+      return;
+    }
+  }
+  packed_store<DT, PM>(a, oo, io, i, word);
+}
+
+// One pass over the words. FIRST: they are packed out of the input; LAST: they leave as results
+// (DESC_VALUES: the non-NaN prefix reversed).
+template <int DT, int PM, bool FIRST, bool LAST, bool DESC_VALUES>
+__global__ __launch_bounds__(256) void rx_scatter_kernel(SortArgs a, RadixArgs r) {
   __shared__ uint64_t sorted[RX_TILE];  // the tile in digit order, so that lanes next to each other write next to each other
   __shared__ uint32_t cnt[4][256];
   __shared__ uint32_t base[256];   // first output position of this tile's words with digit d
@@ -610,13 +655,10 @@ __global__ __launch_bounds__(256) void rx_scatter_kernel(RadixArgs r) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int w = 0; w < 4; w++) cnt[w][threadIdx.x] = 0;
-  {
-    const int64_t at = (int64_t)threadIdx.x * r.nblk + blk;  // this tile's entry for digit threadIdx.x
-    base[threadIdx.x] = r.hist[s * 256 * r.nblk + at] + r.seg[s * r.nseg + at / RX_SEG];
-  }
-  __syncthreads();
   const uint64_t *src = r.src + s * r.n;
   uint64_t *dst = r.dst + s * r.n;
+  int64_t io = 0, oo = 0;
+  if constexpr (FIRST || LAST) slice_offsets(a, s, io, oo);
   const int64_t tile0 = (int64_t)blk * RX_TILE;
   const int64_t i0 = tile0 + wave * (RX_ROWS * 64) + lane;
   uint64_t w[RX_ROWS];
@@ -624,8 +666,27 @@ __global__ __launch_bounds__(256) void rx_scatter_kernel(RadixArgs r) {
 #pragma unroll
   for (int q = 0; q < RX_ROWS; q++) {
     const int64_t i = i0 + q * 64;
-    w[q] = i < r.n ? src[i] : ~(uint64_t)0;
+    w[q] = i < r.n ? rx_word<DT, PM, FIRST>(a, src, io, i) : ~(uint64_t)0;
   }
+  if (r.nblk <= RX_SHORT) {  // this thread's digit over the slice's tiles
+    const uint32_t *h = r.hist + s * 256 * r.nblk + threadIdx.x;
+    uint32_t all = 0, before = 0, total;
+    for (int t0 = 0; t0 < r.nblk; t0 += 8) {
+      uint32_t c[8];
+#pragma unroll
+      for (int t = 0; t < 8; t++) c[t] = t0 + t < r.nblk ? h[(t0 + t) * 256] : 0;
+#pragma unroll
+      for (int t = 0; t < 8; t++) {
+        all += c[t];
+        before += t0 + t < blk ? c[t] : 0;
+      }
+    }
+    base[threadIdx.x] = rx_block_scan(all, tmp, total) + before;
+  } else {
+    const int64_t at = (int64_t)threadIdx.x * r.nblk + blk;  // this tile's entry for digit threadIdx.x
+    base[threadIdx.x] = r.hist[s * 256 * r.nblk + at] + r.seg[s * r.nseg + at / RX_SEG];
+  }
+  __syncthreads();
   const uint64_t lower = ((uint64_t)1 << lane) - 1;
 #pragma unroll
   for (int q = 0; q < RX_ROWS; q++) {
@@ -666,19 +727,22 @@ __global__ __launch_bounds__(256) void rx_scatter_kernel(RadixArgs r) {
   }
   __syncthreads();
   const int count = (int)(r.n - tile0 < RX_TILE ? r.n - tile0 : RX_TILE);
+  const int64_t reals = LAST && DESC_VALUES ? a.n - (int64_t)r.nan_count[s] : 0;
 #pragma unroll
   for (int q = 0; q < RX_ROWS; q++) {
     const int p = q * 256 + threadIdx.x;
     if (p < count) {
       const uint64_t word = sorted[p];
       const uint32_t d = (uint32_t)(word >> r.shift) & 255u;
-      dst[base[d] + ((uint32_t)p - first[d])] = word;
+      const uint32_t to = base[d] + ((uint32_t)p - first[d]);
+      if constexpr (LAST) rx_store<DT, PM>(a, io, oo, DESC_VALUES && to < reals ? reals - 1 - to : to, word);
+      else dst[to] = word;
     }
   }
 }
 
-// Writes the sorted words out: indices, or the values they point at. DESC_VALUES: the
-// non-NaN prefix reversed.
+// The results of a sort of one pass, whose only scatter reads the input everywhere: a result may
+// lie over it.
 template <int DT, int PM, bool DESC_VALUES>
 __global__ __launch_bounds__(256) void rx_unpack_kernel(SortArgs a, const uint64_t *w, const uint32_t *nan_count, int nblk) {
   const int64_t s = blockIdx.x / nblk, base = (int64_t)(blockIdx.x % nblk) * RX_TILE;
@@ -688,33 +752,7 @@ __global__ __launch_bounds__(256) void rx_unpack_kernel(SortArgs a, const uint64
   for (int e = threadIdx.x; e < RX_TILE; e += 256) {
     const int64_t i = base + e;
     if (i >= a.n) break;
-    const int64_t from = DESC_VALUES && i < reals ? reals - 1 - i : i;
-    const uint64_t word = w[s * a.n + from];
-    if constexpr (PM == VALUE_ASC) {
-      // The value is the mapped key read backwards; only a zero (both signs share a key) and a
-      // NaN (its payload is not in the key) are fetched from the input through the index. A
-      // gather for every element cost a third of the whole sort.
-      using TR = Tr<DT>;
-      using C = typename TR::C;
-      using S = typename TR::S;
-      const uint32_t m = (uint32_t)(word >> 32);
-      bool direct = true;
-      C x;
-      if constexpr (TR::cat == CAT_FLOAT) {
-        direct = m != Packed<DT>::K_NAN && m != 0x80000000u;
-        const uint32_t u = (m & 0x80000000u) ? m ^ 0x80000000u : ~m;
-        x = (C)__builtin_bit_cast(float, u);
-      } else if constexpr (TR::cat == CAT_SINT) {
-        x = (C)(int32_t)(m ^ 0x80000000u);
-      } else {
-        x = (C)m;
-      }
-      if (direct) {
-        reinterpret_cast<S *>(a.out)[oo + i * a.out_axis] = TR::st(x);
-        continue;
-      }
-    }
-    packed_store<DT, PM>(a, oo, io, i, word);
+    rx_store<DT, PM>(a, io, oo, i, w[s * a.n + (DESC_VALUES && i < reals ? reals - 1 - i : i)]);
   }
 }
 
@@ -736,7 +774,7 @@ int radix_run(nxh_context *ctx, const char *op, SortArgs &a) {
   RadixArgs r{};
   r.hist = (uint32_t *)(p + 2 * words);
   r.seg = (uint32_t *)(p + 2 * words + hist);
-  uint32_t *nan_count = (uint32_t *)(p + 2 * words + hist + seg);
+  r.nan_count = (uint32_t *)(p + 2 * words + hist + seg);
   r.slices = a.slices;
   r.n = a.n;
   r.nblk = (int)nblk;
@@ -744,21 +782,32 @@ int radix_run(nxh_context *ctx, const char *op, SortArgs &a) {
   const dim3 tiles((unsigned)(a.slices * nblk)), block(256);
   nxh_set_path("sort_radix");
   if (DESC_VALUES)
-    hipLaunchKernelGGL(rx_zero_kernel, dim3((unsigned)((a.slices + 255) / 256)), block, 0, ctx->stream, nan_count, a.slices);
-  hipLaunchKernelGGL((rx_pack_kernel<DT, PM, DESC_VALUES>), tiles, block, 0, ctx->stream, a, w0, nan_count, (int)nblk);
-  uint64_t *src = w0, *dst = w1;
+    hipLaunchKernelGGL(rx_zero_kernel, dim3((unsigned)((a.slices + 255) / 256)), block, 0, ctx->stream, r.nan_count, a.slices);
+  // [64,50257] float32, argsort: 180 us as pack, four passes of histogram, two scans and scatter, unpack
+  constexpr int mask = rx_pass_mask<DT>(), passes = __builtin_popcount(mask);
+  uint64_t *src = w0, *dst = w0;
+  int done = 0;
   for (int pass = 0; pass < 4; pass++) {
-    if (!(rx_pass_mask<DT>() >> pass & 1)) continue;
+    if (!(mask >> pass & 1)) continue;
+    const bool first = done == 0, last = ++done == passes;
     r.src = src;
     r.dst = dst;
     r.shift = 32 + 8 * pass;
-    hipLaunchKernelGGL(rx_hist_kernel, tiles, block, 0, ctx->stream, r);
-    hipLaunchKernelGGL(rx_scan_segments_kernel, dim3((unsigned)(a.slices * nseg)), block, 0, ctx->stream, r);
-    hipLaunchKernelGGL(rx_scan_totals_kernel, dim3((unsigned)a.slices), block, 0, ctx->stream, r);
-    hipLaunchKernelGGL(rx_scatter_kernel, tiles, block, 0, ctx->stream, r);
-    std::swap(src, dst);
+    if (first) hipLaunchKernelGGL((rx_hist_kernel<DT, PM, true, DESC_VALUES>), tiles, block, 0, ctx->stream, a, r);
+    else hipLaunchKernelGGL((rx_hist_kernel<NXH_F32, ARG_ASC, false, false>), tiles, block, 0, ctx->stream, a, r);
+    if (nblk > RX_SHORT) {
+      hipLaunchKernelGGL(rx_scan_segments_kernel, dim3((unsigned)(a.slices * nseg)), block, 0, ctx->stream, r);
+      hipLaunchKernelGGL(rx_scan_totals_kernel, dim3((unsigned)a.slices), block, 0, ctx->stream, r);
+    }
+    if (first) hipLaunchKernelGGL((rx_scatter_kernel<DT, PM, true, false, false>), tiles, block, 0, ctx->stream, a, r);
+    else if (last) {
+      if constexpr (passes > 1) hipLaunchKernelGGL((rx_scatter_kernel<DT, PM, false, true, DESC_VALUES>), tiles, block, 0, ctx->stream, a, r);
+    } else hipLaunchKernelGGL((rx_scatter_kernel<NXH_F32, ARG_ASC, false, false, false>), tiles, block, 0, ctx->stream, a, r);
+    src = dst;
+    dst = dst == w0 ? w1 : w0;
   }
-  hipLaunchKernelGGL((rx_unpack_kernel<DT, PM, DESC_VALUES>), tiles, block, 0, ctx->stream, a, src, nan_count, (int)nblk);
+  if constexpr (passes == 1)
+    hipLaunchKernelGGL((rx_unpack_kernel<DT, PM, DESC_VALUES>), tiles, block, 0, ctx->stream, a, src, r.nan_count, (int)nblk);
   NXH_HIP(op, hipGetLastError());
   return NXH_OK;
 }
