@@ -1,7 +1,8 @@
 """Builds ``raven_amd/csrc/libnxhip.so`` for gfx950 with hipcc.
 
 One object per ``.hip`` translation unit (compiled in parallel), linked into a
-single shared library that exports exactly the C ABI of ``include/nxhip.h``.
+single shared library that exports exactly the C ABI of ``include/nxhip.h``; and
+the Python module of its host path, with gcc.
 Cross-compiles without a GPU.
 """
 
@@ -10,6 +11,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -72,7 +74,23 @@ def build_all(force: bool = True, jobs: int | None = None) -> Path:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr}")
+    build_calls()
     return LIB
+
+
+CALLS_SRC = CSRC.parent / "host_c" / "nx_calls.c"
+CALLS_LIB = CSRC.parent / "_nxcalls.so"
+
+
+def build_calls() -> Path:
+    """The Python module of the per-primitive host path (raven_amd/host_c/nx_calls.c): gcc only."""
+    cmd = ["gcc", "-std=gnu11", "-O2", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wextra",
+           "-I", str(CSRC.parent.parent / "include"), "-I", sysconfig.get_paths()["include"],
+           "-o", str(CALLS_LIB), str(CALLS_SRC)]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0 or r.stderr.strip():
+        raise RuntimeError(f"gcc failed on {CALLS_SRC.name}:\n{r.stderr}")
+    return CALLS_LIB
 
 
 ABI_CHECK_SRC = CSRC.parent.parent / "tests" / "abi_c" / "nxh_abi_check.c"

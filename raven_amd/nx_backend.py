@@ -27,6 +27,7 @@ import numpy as np
 
 from . import _ffi
 from . import dtype as dt
+from ._nxcalls import Calls, DeviceBuffer, Tensor, bind, setup  # host_c/nx_calls.c, built beside this file
 from ._ffi import BINARY_OPS, COMPARE_OPS, REDUCE_OPS, UNARY_OPS, NxhTensor, stamp, view_image
 from .view import _CONTIGUOUS, View, numel
 
@@ -41,66 +42,6 @@ def _op(table: dict, name: str) -> int:
     if i is None:
         raise ValueError(f"{name!r} is not in list")
     return i
-
-
-class DeviceBuffer:
-    """One device allocation, shared by every view of a tensor. Returned to the
-    context's caching allocator when the last handle goes away (the OCaml
-    binding does the same from a custom-block finaliser)."""
-
-    __slots__ = ("ctx", "ptr", "nbytes", "__weakref__")
-
-    def __init__(self, ctx: "Backend", nbytes: int):
-        p = C.c_void_p()
-        rc = ctx._lib.nxh_alloc(ctx._h, nbytes, C.byref(p))
-        if rc:
-            ctx._check(rc)
-        self.ctx = ctx
-        self.ptr = p.value
-        self.nbytes = nbytes
-
-    def __del__(self):
-        ctx = getattr(self, "ctx", None)
-        if ctx is not None and ctx._h and self.ptr:
-            ctx._lib.nxh_free(ctx._h, self.ptr)
-            self.ptr = None
-
-
-class Tensor:
-    """The backend's tensor handle (nx_backend.ml:36-43)."""
-
-    __slots__ = ("buffer", "view", "shape", "dtype", "context", "_d")
-
-    def __init__(self, buffer: DeviceBuffer, view: View, dtype: dt.DType, context: "Backend"):
-        self.buffer = buffer
-        self.view = view
-        self.shape = view.shape
-        self.dtype = dtype
-        self.context = context
-        self._d = None
-
-    @property
-    def strides(self):
-        return self.view.strides
-
-    @property
-    def offset(self):
-        return self.view.offset
-
-    def _desc(self):
-        """The C descriptor, made once: handle, view and storage do not change. The library reads
-        it during a call and keeps no pointer to it."""
-        d = self._d
-        if d is None:
-            v = self.view
-            image = v.image
-            if image is None:
-                image = v.image = view_image(v.shape, v.strides, v.offset)
-            d = self._d = stamp(self.buffer.ptr, self.dtype.tag, image)
-        return d
-
-    def __repr__(self):  # pragma: no cover
-        return f"Tensor({self.dtype.name}, shape={self.shape}, strides={self.strides}, offset={self.offset})"
 
 
 def encode_scalar(dtype: dt.DType, value) -> np.ndarray:
@@ -140,12 +81,17 @@ class Graph:
             self._h = None
 
 
-class Backend:
+setup(_CONTIGUOUS, View.create, view_image, stamp, encode_scalar, np.ndarray, dt.bool_, _UNARY, _BINARY, _COMPARE, _REDUCE)
+
+
+class Backend(Calls):
     """An execution context (``create_context``, nx_backend.mli:32-39) plus the
-    operations of ``Backend_intf.S``."""
+    operations of ``Backend_intf.S``. unary, binary, compare, where, cast, copy,
+    assign, full, reduce and matmul are ``Calls``' (host_c/nx_calls.c)."""
 
     def __init__(self):
         self._lib = _ffi.load()
+        bind({name: C.cast(getattr(self._lib, name), C.c_void_p).value for name in _ffi.SIGNATURES})
         self._gelu_constants = {}
         h = C.c_void_p()
         rc = self._lib.nxh_context_create(C.byref(h))
@@ -241,19 +187,6 @@ class Backend:
             view = View.create(shape)
         return Tensor(DeviceBuffer(self, dtype.nbytes(numel(view.shape))), view, dtype, self)
 
-    def full(self, dtype: dt.DType, shape: Sequence[int], value) -> Tensor:
-        """Every element is ``value`` (a Python number, or one already-encoded
-        storage element as a numpy array)."""
-        out = self.buffer(dtype, shape)
-        enc = value if isinstance(value, np.ndarray) else encode_scalar(dtype, value)
-        if enc.size != 1:
-            raise ValueError("full: the value is one element")
-        # (the bytes object is the element's storage during the call)
-        rc = self._lib.nxh_fill(self._h, out._desc(), enc.tobytes())
-        if rc:
-            self._check(rc)
-        return out
-
     def from_host(self, array: np.ndarray, dtype: dt.DType) -> Tensor:
         """Copies a flat, C-contiguous host buffer to the device; the result is
         rank 1 (nx_backend.ml:66-69). The host array may be reused on return."""
@@ -296,69 +229,12 @@ class Backend:
     def flip(self, t, flags):
         return self._of_view(t, t.view.flip(flags))
 
-    # ── map family (nx_backend.ml:170-234) ──────────────────────────────────
-    def unary(self, op: str, x: Tensor) -> Tensor:
-        out = self.buffer(x.dtype, x.shape)
-        o, a = out._desc(), x._desc()
-        rc = self._lib.nxh_unary(self._h, _op(_UNARY, op), o, a)
-        if rc:
-            self._check(rc)
-        return out
-
-    def binary(self, op: str, x: Tensor, y: Tensor) -> Tensor:
-        out = self.buffer(x.dtype, x.shape)
-        o, a, b = out._desc(), x._desc(), y._desc()
-        rc = self._lib.nxh_binary(self._h, _op(_BINARY, op), o, a, b)
-        if rc:
-            self._check(rc)
-        return out
-
-    def compare(self, op: str, x: Tensor, y: Tensor) -> Tensor:
-        out = self.buffer(dt.bool_, x.shape)
-        o, a, b = out._desc(), x._desc(), y._desc()
-        rc = self._lib.nxh_compare(self._h, _op(_COMPARE, op), o, a, b)
-        if rc:
-            self._check(rc)
-        return out
-
-    def where(self, cond: Tensor, if_true: Tensor, if_false: Tensor) -> Tensor:
-        out = self.buffer(if_true.dtype, if_true.shape)
-        o, c, a, b = out._desc(), cond._desc(), if_true._desc(), if_false._desc()
-        rc = self._lib.nxh_where(self._h, o, c, a, b)
-        if rc:
-            self._check(rc)
-        return out
-
-    def cast(self, x: Tensor, dtype: dt.DType) -> Tensor:
-        out = self.buffer(dtype, x.shape)
-        o, a = out._desc(), x._desc()
-        rc = self._lib.nxh_cast(self._h, o, a)
-        if rc:
-            self._check(rc)
-        return out
-
     # ── move family (nx_backend.ml:349-357, 399-402) ────────────────────────
-    def copy(self, x: Tensor) -> Tensor:
-        out = self.buffer(x.dtype, x.shape)
-        o, a = out._desc(), x._desc()
-        rc = self._lib.nxh_copy(self._h, o, a)
-        if rc:
-            self._check(rc)
-        return out
-
     def contiguous(self, x: Tensor) -> Tensor:
         """``x`` itself iff C-contiguous AND offset 0, else a copy."""
         if x.view.is_c_contiguous() and x.view.offset == 0:
             return x
         return self.copy(x)
-
-    def assign(self, dst: Tensor, src: Tensor) -> None:
-        """Writes ``src`` through ``dst``'s strides (visible through every view
-        sharing dst's buffer)."""
-        o, a = dst._desc(), src._desc()
-        rc = self._lib.nxh_copy(self._h, o, a)
-        if rc:
-            self._check(rc)
 
     def gather(self, data: Tensor, indices: Tensor, axis: int) -> Tensor:
         out = self.buffer(data.dtype, indices.shape)
@@ -668,7 +544,8 @@ class Backend:
         return out
 
     # ── fold family (nx_backend.ml:266-307) ─────────────────────────────────
-    def reduce(self, op: str, axes: Sequence[int], x: Tensor) -> Tensor:
+    def _reduce_general(self, op: str, axes: Sequence[int], x: Tensor) -> Tensor:
+        """``reduce`` of any axes: out of order, empty extents, errors."""
         axes = sorted(int(a) for a in axes)
         if op in ("max", "min"):
             for a in axes:
@@ -713,7 +590,8 @@ class Backend:
         return self._argreduce(True, x, axis, keepdims)
 
     # ── matmul (nx_backend.ml:485-500) ──────────────────────────────────────
-    def matmul(self, x: Tensor, y: Tensor) -> Tensor:
+    def _matmul_general(self, x: Tensor, y: Tensor) -> Tensor:
+        """``matmul`` whose batches broadcast or whose rows take a pitch of whole memory lines."""
         xs, ys = x.shape, y.shape
         nd = max(len(xs), len(ys))
         batch = []

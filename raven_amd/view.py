@@ -27,18 +27,20 @@ def numel(shape: Sequence[int]) -> int:
 
 
 _CONTIGUOUS: dict = {}  # shape -> its C-contiguous, offset-0 view (views are immutable)
+_DERIVED = 16  # movements a view remembers the results of
 
 
 class View:
     """Immutable by convention: every operation returns a new view."""
 
-    __slots__ = ("shape", "strides", "offset", "image")
+    __slots__ = ("shape", "strides", "offset", "image", "derived")
 
     def __init__(self, shape: Tuple[int, ...], strides: Tuple[int, ...], offset: int = 0):
         self.shape = shape
         self.strides = strides
         self.offset = offset
         self.image = None  # the C descriptor's bytes, made by the first call that needs them
+        self.derived = None  # (movement, argument) -> view, of views that are shared (see _remembered)
 
     def __eq__(self, other):
         return (isinstance(other, View) and self.shape == other.shape and self.strides == other.strides
@@ -92,7 +94,36 @@ class View:
         return True
 
     # -- movement (view.ml:82-322) ----------------------------------------
+    # A program moves the same few shapes over and over (a bias row against a batch, a weight's
+    # transpose), and a fresh result's view is the one in _CONTIGUOUS: those remember what a tuple of
+    # plain integers made of them.
+    def _remembered(self, movement, make, arg) -> "View":
+        if type(arg) is not tuple:
+            arg = tuple(arg)
+        d = self.derived
+        if d is not None:
+            v = d.get((movement, arg))
+            if v is not None:
+                return v
+        v = make(self, arg)
+        if d is None:
+            if _CONTIGUOUS.get(self.shape) is not self:
+                return v
+            d = self.derived = {}
+        if len(d) < _DERIVED:
+            d[movement, tuple(map(int, arg))] = v
+        return v
+
     def expand(self, new_shape) -> "View":
+        return self._remembered("expand", View._expand, new_shape)
+
+    def permute(self, axes) -> "View":
+        return self._remembered("permute", View._permute, axes)
+
+    def reshape(self, new_shape) -> "View":
+        return self._remembered("reshape", View._reshape, new_shape)
+
+    def _expand(self, new_shape) -> "View":
         new_shape = tuple(map(int, new_shape))
         shape, n = self.shape, len(new_shape)
         if not shape:
@@ -111,7 +142,7 @@ class View:
                 strides[i] = 0
         return View(new_shape, tuple(strides), 0 if 0 in new_shape else self.offset)
 
-    def permute(self, axes) -> "View":
+    def _permute(self, axes) -> "View":
         axes = tuple(map(int, axes))
         shape, strides = self.shape, self.strides
         n = len(shape)
@@ -149,7 +180,7 @@ class View:
                 strides[i] = -strides[i]
         return View.create(self.shape, strides, off)
 
-    def reshape(self, new_shape) -> "View":
+    def _reshape(self, new_shape) -> "View":
         new_shape = tuple(map(int, new_shape))
         if new_shape == self.shape:
             return self
