@@ -22,7 +22,8 @@
 // writing float32 / float64 / complex128 operands where they are. The others: correctness
 // first, one workgroup per matrix of the batch, the matrix in a contiguous double-precision
 // workspace (the strided, any-dtype operands are brought in and results sent out by nxh_cast).
-//   qr            Householder columns, one wave per trailing column
+//   qr            Householder panels and products of them (linalg_qr.hpp); complex, or over 2048
+//                 rows: Householder columns, one wave per trailing column
 //   eigh          two-sided Jacobi with a round-robin ordering: n/2 disjoint
 //                 rotations per round, applied as a column phase and a row phase
 //   svd           one-sided Jacobi on the columns (round-robin, one wave per pair),
@@ -1375,10 +1376,14 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
   return status.collect(op);
 }
 
+#include "linalg_qr.hpp"
+
 // Householder QR of `batch` column-major m x n matrices At, Q's first nq columns to Qt.
 template <class T>
 static int run_qr(nxh_context *ctx, const char *op, int64_t batch, int m, int n, int nq, T *At, T *Qt, T *tau) {
   std::lock_guard<std::mutex> g(ctx->mu);
+  if constexpr (std::is_same<T, double>::value)
+    if (m <= QR_ROWS) return run_qr_blocked(ctx, op, batch, m, n, nq, At, Qt);
   if (std::max(m, n) < LA_WIDE_FROM) {
     hipLaunchKernelGGL(qr_kernel<T>, dim3((unsigned)batch), dim3(LA_THREADS), 0, ctx->stream, At, Qt, tau, m, n, nq);
     NXH_HIP(op, hipGetLastError());
@@ -1587,7 +1592,7 @@ NXH_EXPORT int nxh_qr(nxh_context *ctx, const nxh_tensor *q, const nxh_tensor *r
   if ((rc = work.get((size_t)(p.batch * k) * p.esize, &tau))) return rc;
   nxh_tensor wa = workspace_tensor(x, At, p.wdt, m, n, true);
   if (n > 0 && (rc = nxh_cast(ctx, &wa, x))) return rc;
-  PathAtExit path{std::max(m, n) >= LA_WIDE_FROM ? "qr_householder_wide" : "qr_householder"};
+  PathAtExit path{!p.cx && m <= QR_ROWS ? "qr_blocked" : std::max(m, n) >= LA_WIDE_FROM ? "qr_householder_wide" : "qr_householder"};
   rc = p.cx ? run_qr<c64>(ctx, op, p.batch, (int)m, (int)n, (int)nq, (c64 *)At, (c64 *)Qt, (c64 *)tau)
             : run_qr<double>(ctx, op, p.batch, (int)m, (int)n, (int)nq, (double *)At, (double *)Qt, (double *)tau);
   if (rc) return rc;
