@@ -12,6 +12,7 @@
 //               gemm_ragged.hip instantiates them for operands of any K and alignment.
 //   gemm_mfma   (gemm_mfma.hip) bf16 / f16 / f32 of any extents, strides and alignment: small and
 //               ragged products, straight from memory into the matrix instruction.
+//   gemm_strip  (gemm_strip.hip) bf16 / f16, few result tiles, B in memory order.
 //   gemm_tiny   batches of products of a few elements each: a lane per output.
 //   gemm_rowdot n <= 4 with A's rows along K (matrix x vector): a wave per row of A,
 //               16-byte pieces, float32 sums met through the cross-lane network.
@@ -32,6 +33,7 @@
 #include "gemm_args.hpp"
 #include "gemm_tile.hpp"
 #include "gemm_dl.hpp"
+#include "gemm_strip.hpp"
 #include "nxh_common.hpp"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -895,6 +897,32 @@ struct Epilogue {
   int ngroup = 1;
   int64_t goff_b[2] = {}, goff_c[2] = {}, goff_bias[2] = {};
 };
+// The operands of gemm_strip.hip out of a product's; -1 where its layouts don't hold.
+static int try_strip(nxh_context *ctx, int dtype, const GemmArgs &a, uint32_t nbatch, const Epilogue *epi = nullptr) {
+  if (a.acs != 1 || a.bcs != 1 || a.ccs != 1 || a.batch.n > 4) return -1;
+  gemm_strip::Args g{};
+  g.A = a.A, g.B = a.B, g.C = a.C;
+  g.lda = a.ars, g.ldb = a.brs, g.ldc = a.crs;
+  g.M = a.M, g.N = a.N, g.K = a.K;
+  g.nbatch = nbatch;
+  g.nbd = a.batch.n;
+  g.ngroup = 1;
+  for (int i = 0; i < a.batch.n; i++) {
+    g.bshape[i] = a.batch.shape[i];
+    g.ba[i] = a.batch.a[i], g.bb[i] = a.batch.b[i], g.bc[i] = a.batch.c[i];
+    if (epi) g.br[i] = epi->br[i];
+  }
+  if (epi) {
+    g.bias = epi->bias, g.R = epi->R, g.ldr = epi->ldr;
+    g.ngroup = (uint32_t)epi->ngroup;
+    for (int i = 0; i + 1 < epi->ngroup; i++) {
+      g.goff_b[i] = epi->goff_b[i] / 2;
+      g.goff_c[i] = epi->goff_c[i] / 2;
+      g.goff_bias[i] = epi->goff_bias[i] / 2;
+    }
+  }
+  return nxh_gemm_strip(ctx, dtype, g);
+}
 template <class EL, bool EPI = false>
 static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool al_a, bool al_b,
                     const Epilogue *epi = nullptr) {
@@ -988,6 +1016,19 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
   auto tiles = [&](int bm, int bn) { return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * (int64_t)nbatch; };
   if (tiles(128, 64) * members > 0x7fffffffLL) return -1;
   const int cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
+  if constexpr (!EL::F32) {
+    // Few result tiles under a long K: a strip of B a block (gemm_strip.hip). [48,768] x [768,768] bfloat16
+    // 5.1 us against 7.3 as half blocks, [400,768] x [768,768] (84 tiles of 64 x 64) 6.0 against 7.6. Three
+    // such layers over one input are one launch: from 3/8 of a tile per unit on their tiles outnumber the
+    // units and the kernels below are the faster ones ([1024,768] x 3 [768,768]: 16 us against 20). A plain product
+    // of a longer K is better off cut along it by the rule below ([512,3072] x [3072,768]: 14.0 against 15.0)
+    // unless the strips are cut too ([48,3072] x [3072,768]: 9.5 against 7.8).
+    if (a_kc && !b_kc && !(EPI && epi->gelu) && a.K >= 512 && a.N >= 512 && tiles(64, 64) <= 3 * cus / 8 && !forced_tile() &&
+        (EPI || a.K < 2048 || nxh_gemm_strip_blocks(ctx, a.M, a.N, a.K, nbatch) > 1) && !(a.M <= 128 && (double)a.K * (double)a.N * 2.0 >= (double)(16 << 20))) {
+      const int rc = try_strip(ctx, EL::BF16 ? NXH_BF16 : NXH_F16, a, nbatch, epi);
+      if (rc != -1) return rc;
+    }
+  }
   // Block shape: rounds of resident blocks x relative cost of one block. One
   // 256x256 block (8 waves, 144 KiB of LDS) fills a CU; two 128x128 blocks fit,
   // each a quarter of the work at about 0.8 of the big tile's efficiency.
@@ -1336,13 +1377,29 @@ static int run_mfma_dtype(nxh_context *ctx, GemmArgs &a, uint32_t nbatch, bool b
                                   std::conditional_t<MM::DT == NXH_BF16, gemm_tile::ElBF16, gemm_tile::ElF16>>;
     int rc = try_tile<EL>(ctx, a, nbatch, batch_aligned_a, batch_aligned_b);
     if (rc != -1) return rc;
+    const double terms = (double)a.M * (double)a.N * (double)a.K * (double)nbatch;
+    const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
+    // 16-bit operands of any alignment, B in memory order: a strip of B a block, below 2^27 terms or where
+    // one tile holds all rows. bfloat16 [501,501]^2 5.3 us against 6.2 in the general kernel, [300,1001] x [1001,300]
+    // 6.9 against 8.2, [40,2000]^2 8.1 against 18.2, [8,16383]^2 142 against 208, [8,5093] x [5093,907]
+    // 11.5 against 16.2. Too few blocks leave the units that have one loading all by themselves:
+    // [33,1879] x [1879,500] as 24 blocks took 10.4 against 8.3, and the second launch of a K cut among blocks
+    // wants some 5 MB of B ([7,3992] x [3992,531] 10.7 against 7.2). Below 256 a wave has no whole step of K.
+    if constexpr (sizeof(S) == 2) {
+      const int64_t cols = (a.N + 63) / 64 * (int64_t)nbatch;
+      const int cut = nxh_gemm_strip_blocks(ctx, a.M, a.N, a.K, nbatch);
+      if (a.N >= 64 && a.K >= 256 && ((terms < (double)(1 << 27) && (a.M + 63) / 64 * cols <= 7 * cus / 8) || a.M <= 64) &&
+          (((a.M + 15) / 16 * cols * cut >= 3 * cus / 16 && (cut == 1 || a.K * a.N >= (int64_t)5 << 19)) || a.K <= 512)) {
+        rc = try_strip(ctx, MM::DT, a, nbatch);
+        if (rc != -1) return rc;
+      }
+    }
     // Operands that do not fit it as they are: the ragged form of the same kernels for products of 2^27
     // terms or whose small blocks occupy the chip, the general kernel below that. float32 [16,200,200]
     // x [16,200,201] (256 blocks of 64 x 64): 9.3 us against 14.2; [501,501]^2 (64 blocks): 13.9 against
     // 7.9. bfloat16 [16,300,300]^2 (240 blocks of 128 x 64): 8.2 against 16.6; [501,501]^2 (32): 9.3
     // against 6.7. A K of one slab is loads and stores, which the general kernel does not stage.
-    const double terms = (double)a.M * (double)a.N * (double)a.K * (double)nbatch;
-    const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256, bm = sizeof(S) == 4 ? 64 : 128;
+    const int64_t bm = sizeof(S) == 4 ? 64 : 128;
     const double blocks = (double)((a.M + bm - 1) / bm) * (double)((a.N + 63) / 64) * nbatch;
     if (terms >= (double)(1 << 27) || (a.K >= 64 && blocks >= (sizeof(S) == 4 ? 0.75 : 0.6) * (double)cus)) {
       rc = nxh_gemm_ragged(ctx, MM::DT, a, nbatch);
