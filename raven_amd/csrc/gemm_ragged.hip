@@ -83,6 +83,9 @@ int run(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch) {
   }
   if (pick == 0) return launch_oriented<EL, Shape256x256>(ctx, g, a_kc, b_kc);
   if (pick == 1) return launch_oriented<EL, Shape128x128>(ctx, g, a_kc, b_kc);
+  if constexpr (!EL::F32) {  // two groups of waves a block (gemm_tile.hpp), from eight slabs on
+    if (a.K > 7 * Geo<EL>::BK && tiles(128, 64) <= cus) return launch_oriented<EL, Shape128x64Halves>(ctx, g, a_kc, b_kc);
+  }
   return launch_oriented<EL, std::conditional_t<EL::F32, Shape64x64, Shape128x64>>(ctx, g, a_kc, b_kc);
 }
 }  // namespace

@@ -86,29 +86,37 @@ struct Geo {
   }
 };
 
-template <int WM_, int WN_, int TM_, int TN_>
+// KG: groups of WM x WN waves that share the block's tile, each with a run of K's slabs and stages of its own.
+template <int WM_, int WN_, int TM_, int TN_, int KG_ = 1>
 struct Shape {
-  static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_;
-  static constexpr int BM = WM * TM * 32, BN = WN * TN * 32, THREADS = 64 * WM * WN;
-  // staged 16-byte vectors per lane and slab: rows x 8 vectors / THREADS
-  static constexpr int NVA = BM * 8 / THREADS, NVB = BN * 8 / THREADS;
-  static_assert(NVA >= 1 && NVB >= 1 && NVA * THREADS == BM * 8 && NVB * THREADS == BN * 8, "staging");
+  static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, KG = KG_;
+  static constexpr int BM = WM * TM * 32, BN = WN * TN * 32, GT = 64 * WM * WN, THREADS = GT * KG;
+  // staged 16-byte vectors per lane and slab: rows x 8 vectors / a group's threads
+  static constexpr int NVA = BM * 8 / GT, NVB = BN * 8 / GT;
+  static_assert(NVA >= 1 && NVB >= 1 && NVA * GT == BM * 8 && NVB * GT == BN * 8, "staging");
   // Two blocks of a four-wave shape fit a compute unit's LDS; they also fit its register
   // file when a wave stays within 256 registers (accumulators included), which the
   // kernel asks the compiler for: the second block hides the first one's load latency.
-  static constexpr int WAVES_PER_SIMD = THREADS <= 256 ? 2 : 1;
+  static constexpr int WAVES_PER_SIMD = THREADS <= 256 || KG > 1 ? 2 : 1;
   template <class EL>
   static constexpr int a_elems() { return Geo<EL>::tile_elems(BM); }
   template <class EL>
   static constexpr int stage_elems() { return Geo<EL>::tile_elems(BM) + Geo<EL>::tile_elems(BN); }
   template <class EL>
-  static constexpr size_t lds_bytes() { return 2 * (size_t)stage_elems<EL>() * sizeof(typename EL::S); }
+  static constexpr size_t group_bytes() { return 2 * (size_t)stage_elems<EL>() * sizeof(typename EL::S); }
+  template <class EL>
+  static constexpr size_t lds_bytes() { return KG * group_bytes<EL>(); }
 };
 using Shape256x256 = Shape<4, 2, 2, 4>;
 using Shape128x128 = Shape<2, 2, 2, 2>;
 using Shape256x64 = Shape<4, 1, 2, 2>;
 using Shape128x64 = Shape<2, 2, 2, 1>;
 using Shape64x64 = Shape<2, 2, 1, 1>;
+// For 16-bit products that give a unit one 128 x 64 block: four waves leave each SIMD one, which waits out
+// every fetch and barrier; two groups of them halve the chain of slabs ([2048,3072] x [3072,768] bfloat16:
+// 23.2 -> 19.6 us, 2 x [700,2000]^T [2000,700]^T 24.0 -> 18.9, [667,1394] x [1394,434] 20.7 -> 16.6). float32
+// blocks are all arithmetic and gain nothing ([1024,1024]^2: 23.7 us either way).
+using Shape128x64Halves = Shape<2, 2, 2, 1, 2>;
 
 struct Args {
   const void *A, *B;
@@ -248,9 +256,9 @@ __device__ __forceinline__ void mfma_step(f32x16 &acc, const V16 &a, const V16 &
 // vectors per k-row). `edge` is the number of valid rows from the slab's
 // origin (EDGE only).
 template <class EL, bool KC, int ROWS, int THREADS, bool EDGE>
-__device__ __forceinline__ V16 slab_load1(int i, const typename EL::S *p, int64_t ld, int edge) {
+__device__ __forceinline__ V16 slab_load1(int tid, int i, const typename EL::S *p, int64_t ld, int edge) {
   constexpr int VE = EL::VE;
-  const int v = threadIdx.x + i * THREADS;
+  const int v = tid + i * THREADS;
   if constexpr (KC) {
     int row = v >> 3;
     if constexpr (EDGE) row = row < edge ? row : edge - 1;
@@ -270,11 +278,11 @@ __device__ __forceinline__ V16 slab_load1(int i, const typename EL::S *p, int64_
 typedef V16 V16a4 __attribute__((aligned(4)));
 typedef V16 V16a2 __attribute__((aligned(2)));
 template <class EL, bool KC, int ROWS, int THREADS, bool TAIL>
-__device__ __forceinline__ V16 slab_load1_ragged(int i, const typename EL::S *p, int64_t ld, int edge, int kleft) {
+__device__ __forceinline__ V16 slab_load1_ragged(int tid, int i, const typename EL::S *p, int64_t ld, int edge, int kleft) {
   using S = typename EL::S;
   using V16u = std::conditional_t<EL::F32, V16a4, V16a2>;
   constexpr int VE = EL::VE, VPR = ROWS / VE;
-  const int v = threadIdx.x + i * THREADS;
+  const int v = tid + i * THREADS;
   int row = KC ? v >> 3 : (v % VPR) * VE;  // along M / N: the vector's row, or its first
   const int k = KC ? (v & 7) * VE : v / VPR;
   const bool past = row >= edge;
@@ -295,10 +303,10 @@ __device__ __forceinline__ V16 slab_load1_ragged(int i, const typename EL::S *p,
   }
 }
 template <class EL, bool KC, int ROWS, int THREADS>
-__device__ __forceinline__ void slab_store1(int i, const V16 &r, typename EL::S *lds) {
+__device__ __forceinline__ void slab_store1(int tid, int i, const V16 &r, typename EL::S *lds) {
   using G = Geo<EL>;
   constexpr int VE = EL::VE, VPR = ROWS / VE;
-  const int v = threadIdx.x + i * THREADS;
+  const int v = tid + i * THREADS;
   typename EL::S *q = KC ? lds + (v >> 3) * G::PK + (v & 7) * VE : lds + (v / VPR) * (ROWS + G::padr(ROWS)) + (v % VPR) * VE;
   *reinterpret_cast<V16 *>(q) = r;
 }
@@ -358,12 +366,14 @@ __device__ __forceinline__ void tile_of_block(const Args &a, uint32_t bid, uint3
 // RAG: any K, any alignment of the operands' rows (slab_load1_ragged), ragged edges.
 template <class EL, bool A_KC, bool B_KC, class SH, bool EDGE, bool EPI = false, bool OUT32 = false, bool RAG = false>
 __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH::WAVES_PER_SIMD))) void kernel(Args a) {
-  constexpr int THREADS = SH::THREADS, BM = SH::BM, BN = SH::BN, TM = SH::TM, TN = SH::TN;
+  constexpr int GT = SH::GT, KG = SH::KG, BM = SH::BM, BN = SH::BN, TM = SH::TM, TN = SH::TN;
   constexpr int NVA = SH::NVA, NVB = SH::NVB, BK = Geo<EL>::BK;
   constexpr int A_ELEMS = SH::template a_elems<EL>(), STAGE_ELEMS = SH::template stage_elems<EL>();
   using S = typename EL::S;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  S *smem = reinterpret_cast<S *>(smem_raw);
+  const int group = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / GT) : 0;
+  const int tid = (int)threadIdx.x - group * GT;
+  S *smem = reinterpret_cast<S *>(smem_raw) + group * 2 * STAGE_ELEMS;
   uint32_t batch, tm, tn;
   // tiles are walked from the end: an operand the previous kernel has just written
   // front to back still has its tail in the memory-side cache
@@ -407,7 +417,7 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
   const int64_t stepA = A_KC ? BK : (int64_t)BK * a.lda;
   const int64_t stepB = B_KC ? BK : (int64_t)BK * a.ldb;
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = tid >> 6;
   const int wm = (wave / SH::WN) * (TM * 32), wn = (wave % SH::WN) * (TN * 32);
 
   f32x16 acc[TM][TN];
@@ -427,8 +437,16 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
   }
 
   V16 ra[NVA], rb[NVB];
-  const int nk = (int)(RAG ? (a.K + BK - 1) / BK : a.K / BK);
-  const int kleft = RAG ? (int)(a.K - (int64_t)(nk - 1) * BK) : BK;  // of the last slab
+  const int slabs = (int)(RAG ? (a.K + BK - 1) / BK : a.K / BK);
+  int nk = slabs, k0 = 0;  // this group's run of them (the host has checked that every group has one)
+  if constexpr (KG > 1) {
+    const int more = slabs % KG;
+    nk = slabs / KG + (group < more);
+    k0 = group * (slabs / KG) + (group < more ? group : more);
+    gA += k0 * stepA;
+    gB += k0 * stepB;
+  }
+  const int kleft = RAG && k0 + nk == slabs ? (int)(a.K - (int64_t)(slabs - 1) * BK) : BK;  // of the run's last slab
   // Staged vector i of an operand moves at k-step i % KSTEPS; the prologue uses
   // the same issue order, so the loop's in-order wait counts hold from the start.
   auto fetch_step = [&](int ks, const S *pA, const S *pB, auto tail_c, int kleft) {
@@ -437,11 +455,11 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
     for (int i = 0; i < (NVA > NVB ? NVA : NVB); i++) {
       if (i % KSTEPS != ks) continue;
       if constexpr (RAG) {
-        if (i < NVA) ra[i] = slab_load1_ragged<EL, A_KC, BM, THREADS, TAIL>(i, pA, a.lda, ledge_m, kleft);
-        if (i < NVB) rb[i] = slab_load1_ragged<EL, B_KC, BN, THREADS, TAIL>(i, pB, a.ldb, ledge_n, kleft);
+        if (i < NVA) ra[i] = slab_load1_ragged<EL, A_KC, BM, GT, TAIL>(tid, i, pA, a.lda, ledge_m, kleft);
+        if (i < NVB) rb[i] = slab_load1_ragged<EL, B_KC, BN, GT, TAIL>(tid, i, pB, a.ldb, ledge_n, kleft);
       } else {
-        if (i < NVA) ra[i] = slab_load1<EL, A_KC, BM, THREADS, EDGE>(i, pA, a.lda, ledge_m);
-        if (i < NVB) rb[i] = slab_load1<EL, B_KC, BN, THREADS, EDGE>(i, pB, a.ldb, ledge_n);
+        if (i < NVA) ra[i] = slab_load1<EL, A_KC, BM, GT, EDGE>(tid, i, pA, a.lda, ledge_m);
+        if (i < NVB) rb[i] = slab_load1<EL, B_KC, BN, GT, EDGE>(tid, i, pB, a.ldb, ledge_n);
       }
     }
   };
@@ -449,8 +467,8 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
 #pragma unroll
     for (int i = 0; i < (NVA > NVB ? NVA : NVB); i++) {
       if (i % KSTEPS != ks) continue;
-      if (i < NVA) slab_store1<EL, A_KC, BM, THREADS>(i, ra[i], nA);
-      if (i < NVB) slab_store1<EL, B_KC, BN, THREADS>(i, rb[i], nB);
+      if (i < NVA) slab_store1<EL, A_KC, BM, GT>(tid, i, ra[i], nA);
+      if (i < NVB) slab_store1<EL, B_KC, BN, GT>(tid, i, rb[i], nB);
     }
   };
   using yes = std::integral_constant<bool, true>;
@@ -539,6 +557,26 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
     for (int e = 0; e < 16; e++) acc[0][0][e] += odd[e];
   }
 
+  if constexpr (KG > 1) {
+    // the groups' sums meet in the stages, group 0 adds them in order and is the one that stores
+    static_assert((size_t)SH::WM * SH::WN * TM * TN * 16 * 64 * sizeof(float) <= SH::template group_bytes<EL>(), "a group's sums");
+    if (slabs % KG && group >= slabs % KG) __syncthreads();  // (the others have a slab, and a barrier, more)
+    __syncthreads();  // every wave has read its last fragments
+    float *mine = reinterpret_cast<float *>(smem) + wave * TM * TN * 16 * 64 + lane;
+    if (group > 0) {
+#pragma unroll
+      for (int i = 0; i < TM * TN * 16; i++) mine[i * 64] = acc[i / 16 / TN][i / 16 % TN][i % 16];
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int g = 1; g < KG; g++) {
+      const float *other = mine + g * (SH::template group_bytes<EL>() / sizeof(float));
+#pragma unroll
+      for (int i = 0; i < TM * TN * 16; i++) acc[i / 16 / TN][i / 16 % TN][i % 16] += other[i * 64];
+    }
+  }
+
   // accumulator element e of lane l is C[(e/4)*8 + (l/32)*4 + e%4][l%32]
   S *C = (S *)a.C + co;
   const int r32 = lane & 31, kg = lane >> 5;
@@ -573,12 +611,12 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
     // rounded TM*32 x TN*32 patch in a private piece of the (now idle) stage
     // buffers and sends it out as whole 16-byte row segments.
     constexpr int WC = TN * 32, WP = WC + 8;  // patch width and its LDS pitch (elements)
-    static_assert((size_t)SH::WM * SH::WN * TM * 32 * WP * sizeof(S) <= SH::template lds_bytes<EL>(), "epilogue patch");
+    static_assert((size_t)SH::WM * SH::WN * TM * 32 * WP * sizeof(S) <= SH::template group_bytes<EL>(), "epilogue patch");
     const bool wide = ((uintptr_t)C % 16) == 0 && a.ldc % 8 == 0 && (!RAG || a.ccs == 1) &&
                       (!EPI || ((!a.bias || (uintptr_t)a.bias % 16 == 0) &&
                                 (!a.R || (((uintptr_t)((const S *)a.R + ro)) % 16 == 0 && a.ldr % 8 == 0))));
     if (wide) {
-      __syncthreads();  // every wave has read its last fragments
+      if constexpr (KG == 1) __syncthreads();  // every wave has read its last fragments
       S *patch = smem + wave * (TM * 32 * WP);
 #pragma unroll
       for (int t = 0; t < TM; t++)

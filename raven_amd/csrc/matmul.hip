@@ -1032,41 +1032,51 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
   // Block shape: rounds of resident blocks x relative cost of one block. One
   // 256x256 block (8 waves, 144 KiB of LDS) fills a CU; two 128x128 blocks fit,
   // each a quarter of the work at about 0.8 of the big tile's efficiency.
-  int pick = forced_tile();
-  if (!pick && EL::F32) {
-    // f32: a compute unit's f32 matrix rate is a sixteenth of its 16-bit rate, so a block's time
-    // is all arithmetic and the shapes differ only in what they leave idle: rounds of one block
-    // per unit x the block's area (ragged edges count as whole blocks) x the shape's measured cost
-    // per flop against the 256 x 256 block (4096^3: 138 TFLOP/s there, 123 with half blocks;
-    // 1024^3 on quarter blocks about 100 inside the K loop).
-    struct Cand {
-      int pick, bm, bn;
-      double pen;
-    };
-    const Cand cands[] = {{256, 256, 256, 1.0}, {128, 128, 128, 1.12}, {64, 256, 64, 1.12},
-                          {1264, 128, 64, 1.15}, {6464, 64, 64, 1.3}};
-    double best = 0.0;
-    for (const Cand &c : cands) {
-      if (c.pick == 64 && a.N > 64) continue;
-      if (EPI && epi->gelu && c.pick != 256 && c.pick != 128) continue;
-      const double cost = (double)((tiles(c.bm, c.bn) * members + cus - 1) / cus) * c.bm * c.bn * c.pen;
-      if (!pick || cost < best) {
-        pick = c.pick;
-        best = cost;
+  const auto pick_for = [&](int64_t members) {
+    int pick = 0;
+    if constexpr (EL::F32) {
+      // f32: a compute unit's f32 matrix rate is a sixteenth of its 16-bit rate, so a block's time
+      // is all arithmetic and the shapes differ only in what they leave idle: rounds of one block
+      // per unit x the block's area (ragged edges count as whole blocks) x the shape's measured cost
+      // per flop against the 256 x 256 block (4096^3: 138 TFLOP/s there, 123 with half blocks;
+      // 1024^3 on quarter blocks about 100 inside the K loop).
+      struct Cand {
+        int pick, bm, bn;
+        double pen;
+      };
+      const Cand cands[] = {{256, 256, 256, 1.0}, {128, 128, 128, 1.12}, {64, 256, 64, 1.12},
+                            {1264, 128, 64, 1.15}, {6464, 64, 64, 1.3}};
+      double best = 0.0;
+      for (const Cand &c : cands) {
+        if (c.pick == 64 && a.N > 64) continue;
+        if (EPI && epi->gelu && c.pick != 256 && c.pick != 128) continue;
+        const double cost = (double)((tiles(c.bm, c.bn) * members + cus - 1) / cus) * c.bm * c.bn * c.pen;
+        if (!pick || cost < best) {
+          pick = c.pick;
+          best = cost;
+        }
       }
+    } else {
+      if (a.N <= 64) pick = 64;
+      else {
+        const double c256 = (double)((tiles(256, 256) + cus - 1) / cus);
+        const double c128 = (double)((tiles(128, 128) + 2 * cus - 1) / (2 * cus)) * 0.6;
+        pick = c256 <= c128 ? 256 : 128;
+      }
+      // Fewer blocks than half the compute units: half blocks (128 x 64, four waves of 64 x 32)
+      // put twice as many of them to work (bf16 [1024,768] x [768,768]: 9.5 -> 7.9 us).
+      if (pick != 256 && !(EPI && epi->gelu) && (pick == 64 ? tiles(256, 64) : tiles(128, 128)) * members <= cus / 2)
+        pick = 1264;
     }
-  } else if (!pick) {
-    if (a.N <= 64) pick = 64;
-    else {
-      const double c256 = (double)((tiles(256, 256) + cus - 1) / cus);
-      const double c128 = (double)((tiles(128, 128) + 2 * cus - 1) / (2 * cus)) * 0.6;
-      pick = c256 <= c128 ? 256 : 128;
-    }
-    // Fewer blocks than half the compute units: half blocks (128 x 64, four waves of 64 x 32)
-    // put twice as many of them to work (bf16 [1024,768] x [768,768]: 9.5 -> 7.9 us).
-    if (pick != 256 && !(EPI && epi->gelu) && (pick == 64 ? tiles(256, 64) : tiles(128, 128)) * members <= cus / 2)
-      pick = 1264;
-  }
+    return pick;
+  };
+  // Half blocks one to a unit under a long K: two groups of waves each (Shape128x64Halves). From 24 slabs on (of 12
+  // the groups' meeting takes what they gain: [2048,768] x [768,768] 11.9 us either way). Decided without the
+  // group of linears: a member's sums are those of its own call.
+  const int alone = pick_for(1);
+  const int64_t slabs = a.K / BK;
+  const bool halves = !EL::F32 && !forced_tile() && alone == 1264 && slabs >= 24 && tiles(128, 64) <= cus;
+  int pick = forced_tile() ? forced_tile() : halves ? alone : pick_for(members);
   // Whole tiles of 16-bit operands go straight into LDS (gemm_dl.hpp; load offsets are 32-bit:
   // 256 rows of a k-contiguous operand must stay below 4 GiB, and every row segment the
   // epilogue touches must be 16-byte aligned).
@@ -1147,7 +1157,6 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
       nxh_free_locked(ctx, part);
       return rc;
     };
-    const int64_t slabs = a.K / BK;
     // A 16-bit weight matrix of 16 MiB or more streamed once past at most 128 rows (a decode step
     // of 17 to 128 sequences): memory-bound on B. 128-column blocks keep 256-byte row segments and
     // two slabs of 16 KiB in flight each ([32,4096] x [4096,32000], 250 such blocks, streams B
@@ -1185,6 +1194,10 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
   if constexpr (EL::F32) {
     if (pick == 6464)
       return launch_tile_oriented<EL, gemm_tile::Shape64x64, EPI>(ctx, g, a_kc, b_kc, EPI ? "linear_tile_64x64" : "gemm_tile_64x64");
+  }
+  if constexpr (!EL::F32) {
+    if (pick == 1264 && halves)
+      return launch_tile_oriented<EL, gemm_tile::Shape128x64Halves, EPI>(ctx, g, a_kc, b_kc, EPI ? "linear_tile_128x64" : "gemm_tile_128x64");
   }
   if constexpr (EPI) {
     // Two block shapes are enough for the epilogue family; f16 keeps to the small one (its
