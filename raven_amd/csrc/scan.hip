@@ -161,10 +161,31 @@ __device__ __forceinline__ T shfl_any(T v, int src) {
   return u.t;
 }
 
+// The value of lane `src`, the same for the whole wave (and known to be).
+template <class T>
+__device__ __forceinline__ T lane_any(T v, int src) {
+  constexpr int W = (sizeof(T) + 3) / 4;
+  union {
+    T t;
+    uint32_t w[W];
+  } u;
+  u.w[W - 1] = 0;
+  u.t = v;
+#pragma unroll
+  for (int i = 0; i < W; i++) u.w[i] = __builtin_amdgcn_readlane(u.w[i], src);
+  return u.t;
+}
+
+// Chunks of a line whose carry-in is found by the wave that scans them: it reads the totals before its
+// own, a lane each, and adds them up in their order, where a launch between the two took 10.6 us to do
+// so ([64,50257] float32, 40 chunks a line). With that, 16-byte accesses to rows that start at any element and a
+// step's values on their way while the one before is scanned, that scan takes 13.4 us against 30.
+constexpr int SCAN_OWN_CARRY = 64;
+
 // One wave per line (PHASE 1), or per chunk of a line (blockIdx.y; PHASE 0
-// writes the chunk's total to `carry`, PHASE 2 scans the chunk from its
-// carry-in). VEC: lines and chunks are 16-byte aligned.
-template <int DT, class CB, int V, bool VEC, int PHASE>
+// writes the chunk's total to `carry`, PHASE 2 scans the chunk from its carry-in, PHASE 3 from the
+// totals of the chunks before it). Sixteen bytes a lane at the element's own alignment.
+template <int DT, class CB, int V, int PHASE>
 __global__ __launch_bounds__(FOLD_THREADS) void scan_rows_kernel(ScanArgs a, int64_t chunk, void *carry_v) {
   using TR = Tr<DT>;
   using S = typename TR::S;
@@ -180,17 +201,30 @@ __global__ __launch_bounds__(FOLD_THREADS) void scan_rows_kernel(ScanArgs a, int
   const int64_t k1 = PHASE == 1 ? a.len : (k0 + chunk < a.len ? k0 + chunk : a.len);
   C *slot = PHASE == 1 ? nullptr : (C *)carry_v + (uint64_t)blockIdx.y * a.n_lines + line;
   C carry = PHASE == 2 ? *slot : CB::init();
-  for (int64_t base = k0; base < k1; base += 64 * V) {
+  if constexpr (PHASE == 3) {
+    const int before = blockIdx.y;
+    const C total = lane < before ? ((const C *)carry_v)[(uint64_t)lane * a.n_lines + line] : CB::init();
+    for (int c = 0; c < before; c++) carry = CB::apply(carry, lane_any(total, c));
+  }
+  // a step's values are on their way while the step before is scanned
+  const auto load = [&](int64_t base) {
     const int64_t e0 = base + (int64_t)lane * V;
-    const int n = (int)(k1 - e0 < V ? (k1 - e0 < 0 ? 0 : k1 - e0) : V);  // this lane's live elements
     FVec<S, V> x;
-    if (VEC && n == V) {
-      x = *reinterpret_cast<const FVec<S, V> *>(p + e0);
+    if (e0 + V <= k1) {
+      x = fold_load<S, V>(p + e0);
     } else {
 #pragma unroll
       for (int j = 0; j < V; j++)
-        if (j < n) x.v[j] = p[e0 + j];
+        if (e0 + j < k1) x.v[j] = p[e0 + j];
     }
+    return x;
+  };
+  FVec<S, V> ahead = load(k0);
+  for (int64_t base = k0; base < k1; base += 64 * V) {
+    const int64_t e0 = base + (int64_t)lane * V;
+    const int n = (int)(k1 - e0 < V ? (k1 - e0 < 0 ? 0 : k1 - e0) : V);  // this lane's live elements
+    const FVec<S, V> x = ahead;
+    if (base + 64 * V < k1) ahead = load(base + 64 * V);
     C r[V];
     C t = CB::init();
 #pragma unroll
@@ -211,8 +245,8 @@ __global__ __launch_bounds__(FOLD_THREADS) void scan_rows_kernel(ScanArgs a, int
       FVec<S, V> y;
 #pragma unroll
       for (int j = 0; j < V; j++) y.v[j] = TR::st(CB::apply(excl, r[j]));
-      if (VEC && n == V) {
-        *reinterpret_cast<FVec<S, V> *>(q + e0) = y;
+      if (n == V) {
+        __builtin_memcpy(q + e0, &y, sizeof(S) * V);
       } else {
 #pragma unroll
         for (int j = 0; j < V; j++)
@@ -559,9 +593,6 @@ static int scan_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, c
   if (a.in_step == 1 && a.out_step == 1 && a.len >= 128) {
     const int64_t blocks = (g.n_out + 3) / 4;
     if (blocks > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "too many lines for one launch");
-    bool vec = V > 1 && aligned_to16(a.in) && aligned_to16(a.out);
-    for (int i = 0; vec && i < g.nk; i++)
-      if (g.kin[i] % V != 0 || g.kout[i] % V != 0) vec = false;
     const int cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
     // few long lines: a wave per chunk of 64 * V * k elements instead of per line
     int64_t chunks = std::min<int64_t>(((int64_t)cus * 16 + g.n_out - 1) / g.n_out, a.len / (64 * V * 4));
@@ -575,20 +606,17 @@ static int scan_launch(nxh_context *ctx, const char *op, const nxh_tensor *in, c
       if (rc) return rc;
       const dim3 grid((unsigned)blocks, (unsigned)chunks);
       nxh_set_path("scan_rows_chunks");
-      if (vec) hipLaunchKernelGGL((scan_rows_kernel<DT, CB, V, true, 0>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a, chunk, scratch.p[0]);
-      else hipLaunchKernelGGL((scan_rows_kernel<DT, CB, V, false, 0>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a, chunk, scratch.p[0]);
-      if (g.n_out < 64 && chunks >= 64)
+      hipLaunchKernelGGL((scan_rows_kernel<DT, CB, V, 0>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a, chunk, scratch.p[0]);
+      if (chunks <= SCAN_OWN_CARRY) {
+        hipLaunchKernelGGL((scan_rows_kernel<DT, CB, V, 3>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a, chunk, scratch.p[0]);
+      } else {
         hipLaunchKernelGGL((scan_carry_block_kernel<C, CB>), dim3((unsigned)g.n_out), dim3(FOLD_THREADS), 0, ctx->stream,
                            (C *)scratch.p[0], (uint64_t)g.n_out, (int)chunks);
-      else
-        hipLaunchKernelGGL((scan_carry_kernel<C, CB>), dim3((unsigned)((g.n_out + FOLD_THREADS - 1) / FOLD_THREADS)),
-                           dim3(FOLD_THREADS), 0, ctx->stream, (C *)scratch.p[0], (uint64_t)g.n_out, (int)chunks);
-      if (vec) hipLaunchKernelGGL((scan_rows_kernel<DT, CB, V, true, 2>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a, chunk, scratch.p[0]);
-      else hipLaunchKernelGGL((scan_rows_kernel<DT, CB, V, false, 2>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a, chunk, scratch.p[0]);
+        hipLaunchKernelGGL((scan_rows_kernel<DT, CB, V, 2>), grid, dim3(FOLD_THREADS), 0, ctx->stream, a, chunk, scratch.p[0]);
+      }
     } else {
       nxh_set_path("scan_rows");
-      if (vec) hipLaunchKernelGGL((scan_rows_kernel<DT, CB, V, true, 1>), dim3((unsigned)blocks), dim3(FOLD_THREADS), 0, ctx->stream, a, (int64_t)0, nullptr);
-      else hipLaunchKernelGGL((scan_rows_kernel<DT, CB, V, false, 1>), dim3((unsigned)blocks), dim3(FOLD_THREADS), 0, ctx->stream, a, (int64_t)0, nullptr);
+      hipLaunchKernelGGL((scan_rows_kernel<DT, CB, V, 1>), dim3((unsigned)blocks), dim3(FOLD_THREADS), 0, ctx->stream, a, (int64_t)0, nullptr);
     }
   } else {
     const int64_t blocks = (g.n_out + FOLD_THREADS - 1) / FOLD_THREADS;
