@@ -80,30 +80,46 @@ struct GatherAnyArgs {
 };
 // N: the type the element number is unravelled in (uint32_t when the output holds fewer than 2^32
 // elements). With random indices the reads, not the arithmetic, are what costs: [8192,8192] f32 along
-// axis 1 takes 448 us with either type, every lane of a wave on a cache line of its own.
-template <class E, class N>
-__global__ __launch_bounds__(256) void gather_any_kernel(GatherAnyArgs a) {
-  const int64_t it = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (it >= a.total) return;
-  N rem = (N)it;
-  int64_t io = 0, oo = 0, doff = 0;
-  for (int d = a.ndim - 1; d >= 0; d--) {
-    const N extent = (N)a.shape[d];
-    const N q = rem / extent;
-    const int64_t c = (int64_t)(rem - q * extent);
-    rem = q;
-    io += c * a.istride[d];
-    oo += c * a.ostride[d];
-    if (d != a.axis) doff += c * a.dstride[d];
+// axis 1 took 448 us with either type, every lane of a wave on a cache line of its own.
+// EACH > 1, from 2^20 elements on: a lane has several elements, a block's width apart, so that their reads are under
+// way together ([64,50257] f32 along the rows: 22.8 us to 19.2, [8192,8192]: 434 to 346; below that the
+// longer chain of a lane costs a microsecond). Blocks that share an XCD (ids equal modulo 8) take
+// neighbouring elements: rows that fit its L2 are fetched by one of them.
+template <class E, class N, int EACH>
+__global__ __launch_bounds__(256) void gather_any_kernel(GatherAnyArgs a, uint32_t blocks) {
+  const uint32_t x = blockIdx.x & 7u, run = blocks >> 3, longer = blocks & 7u;
+  const int64_t block = (int64_t)x * run + (x < longer ? x : longer) + (blockIdx.x >> 3);
+  const int64_t it = block * (256 * EACH) + threadIdx.x;
+  int64_t io[EACH], oo[EACH], doff[EACH], index[EACH];
+#pragma unroll
+  for (int j = 0; j < EACH; j++) {
+    const int64_t e = it + j * 256;
+    N rem = (N)(e < a.total ? e : a.total - 1);
+    io[j] = oo[j] = doff[j] = 0;
+    for (int d = a.ndim - 1; d >= 0; d--) {
+      const N extent = (N)a.shape[d];
+      const N q = d ? rem / extent : 0;
+      const int64_t c = (int64_t)(rem - q * extent);
+      rem = q;
+      io[j] += c * a.istride[d];
+      oo[j] += c * a.ostride[d];
+      if (d != a.axis) doff[j] += c * a.dstride[d];
+    }
   }
-  int64_t index = a.idx[io];
-  if (index < 0) index += a.axis_len;
-  if (index < 0 || index >= a.axis_len) {
-    raise_fault(a.fault);
-    return;
+#pragma unroll
+  for (int j = 0; j < EACH; j++) index[j] = a.idx[io[j]];
+  E v[EACH];
+  bool ok[EACH];
+#pragma unroll
+  for (int j = 0; j < EACH; j++) {
+    if (index[j] < 0) index[j] += a.axis_len;
+    ok[j] = index[j] >= 0 && index[j] < a.axis_len;
+    if (!ok[j]) raise_fault(a.fault);
+    else v[j] = reinterpret_cast<const E *>(a.data)[doff[j] + index[j] * a.dstride[a.axis]];
   }
-  doff += index * a.dstride[a.axis];
-  reinterpret_cast<E *>(a.out)[oo] = reinterpret_cast<const E *>(a.data)[doff];
+#pragma unroll
+  for (int j = 0; j < EACH; j++)
+    if (ok[j] && it + j * 256 < a.total) reinterpret_cast<E *>(a.out)[oo[j]] = v[j];
 }
 
 static bool contiguous_off0(const nxh_tensor *a) {
@@ -119,9 +135,12 @@ static bool contiguous_off0(const nxh_tensor *a) {
 
 template <class E>
 static void launch_any_e(nxh_context *ctx, const GatherAnyArgs &a) {
-  const dim3 grid((unsigned)((a.total + 255) / 256));
-  if (a.total <= 0xffffffffLL) hipLaunchKernelGGL((gather_any_kernel<E, uint32_t>), grid, dim3(256), 0, ctx->stream, a);
-  else hipLaunchKernelGGL((gather_any_kernel<E, int64_t>), grid, dim3(256), 0, ctx->stream, a);
+  constexpr int EACH = 4;
+  const bool several = a.total >= (int64_t)1 << 20;
+  const int64_t per = several ? 256 * EACH : 256;
+  const uint32_t blocks = (uint32_t)((a.total + per - 1) / per);
+  const auto kern = !several ? gather_any_kernel<E, uint32_t, 1> : a.total <= 0xffffffffLL ? gather_any_kernel<E, uint32_t, EACH> : gather_any_kernel<E, int64_t, EACH>;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, ctx->stream, a, blocks);
 }
 
 NXH_EXPORT int nxh_gather(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *data,
