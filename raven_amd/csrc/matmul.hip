@@ -1039,13 +1039,14 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
       // is all arithmetic and the shapes differ only in what they leave idle: rounds of one block
       // per unit x the block's area (ragged edges count as whole blocks) x the shape's measured cost
       // per flop against the 256 x 256 block (4096^3: 138 TFLOP/s there, 123 with half blocks;
-      // 1024^3 on quarter blocks about 100 inside the K loop).
+      // 1024^3 on quarter blocks about 100 inside the K loop). Two slabs of K are mostly first loads and
+      // stores, which the small blocks overlap best (32 x [288,64] x [64,784]: 19.8 us on quarter blocks, 23.3 on half).
       struct Cand {
         int pick, bm, bn;
         double pen;
       };
       const Cand cands[] = {{256, 256, 256, 1.0}, {128, 128, 128, 1.12}, {64, 256, 64, 1.12},
-                            {1264, 128, 64, 1.15}, {6464, 64, 64, 1.3}};
+                            {1264, 128, 64, 1.15}, {6464, 64, 64, a.K <= 2 * BK ? 1.15 : 1.3}};
       double best = 0.0;
       for (const Cand &c : cands) {
         if (c.pick == 64 && a.N > 64) continue;
