@@ -44,4 +44,5 @@ int nxh_gemm_block(nxh_context *ctx, int dtype, GemmArgs &a, uint32_t nbatch);
 // strides and alignment. -1 only for more than 2^31 result tiles or a K beyond 2^31.
 int nxh_gemm_mfma(nxh_context *ctx, int dtype, const GemmArgs &a, uint32_t nbatch);
 // The LDS-tiled kernels on operands of any K and alignment (gemm_ragged.hip); -1 where they do not apply.
-int nxh_gemm_ragged(nxh_context *ctx, int dtype, const GemmArgs &a, uint32_t nbatch);
+// kruns > 1 (float32, no batch): C gets the sums [kruns][M][N] of that many equal runs of K's slabs.
+int nxh_gemm_ragged(nxh_context *ctx, int dtype, const GemmArgs &a, uint32_t nbatch, int kruns);

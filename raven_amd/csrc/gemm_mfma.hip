@@ -4,10 +4,14 @@
 // What bounds it: latency. These are the products that are too small or too ragged for the
 // LDS-tiled kernels: a few tiles, so a few waves per compute unit at most, and a chain of loads
 // and matrix instructions along K. A wave therefore owns one small result tile (16 x 16, or
-// 32 x 32 where there are enough of those to fill the chip) and a share of K: the `kw` waves
-// of a group walk their shares side by side and meet in LDS, added in wave order (the same bits
-// on every call). Operands are not staged: a tile's rows are read by few waves and come out
-// of L2, and staging would put a barrier into every step of the chain.
+// 32 x 32 where there are enough of those to fill the chip). Operands are not staged: a tile's rows
+// are read by few waves and come out of L2, and staging would put a barrier into every step of the chain.
+//
+// float32 sums up to K = MAX_CHAIN are one chain of fused steps, in the order of the LDS-tiled kernels (of
+// every eight k-values 0, 4, 1, 5, 2, 6, 3, 7): which kernel a product takes changes no bit of its
+// result, and a select on its sign (max(x w, 0) and the mask of its gradient) falls the same way
+// whatever the sizes. Past MAX_CHAIN, and for 16-bit elements, `kw` waves of a block share a tile's K: they walk
+// their shares side by side and meet in LDS, added in wave order (the same bits on every call).
 //
 // A lane's fragment of a step is VE (four or eight) k-values of one row. An operand that is
 // contiguous along K is read with one 16-byte load at whatever alignment the row has (global
@@ -16,8 +20,9 @@
 // past K are zeros in both operands.
 //
 // Before, these products ran as 128 x 128 blocks: [32,784] x [784,128] float32 was one block,
-// 103 us; here it is 16 blocks of eight waves.
+// 103 us, here 7.5.
 #include <algorithm>
+#include <mutex>
 
 #include "gemm_args.hpp"
 #include "gemm_tile.hpp"
@@ -38,6 +43,15 @@ typedef V16 V16a4 __attribute__((aligned(4)));
 typedef V16 V16a2 __attribute__((aligned(2)));
 
 constexpr int MAXW = 8;  // waves of a block at most
+constexpr int64_t MAX_CHAIN = 2048;  // float32: a longer K is shared by the waves of a block
+
+// Exchanges x of the wave's upper half with y of its lower half.
+__device__ __forceinline__ void swap_halves(float &x, float &y) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, y), false, false);
+  const uint32_t u = p[0], v = p[1];
+  x = __builtin_bit_cast(float, u);
+  y = __builtin_bit_cast(float, v);
+}
 
 // The result tile of a wave. LPG lanes hold the rows of a fragment, 64 / LPG groups of lanes the
 // k-values of a step, VE per lane: step width KS.
@@ -46,13 +60,12 @@ struct Tile {
   static constexpr int GROUPS = 64 / T, VE = EL::VE, KS = GROUPS * VE, NE = T * T / 64;
   using Acc = std::conditional_t<T == 32, f32x16, f32x4>;
   __device__ __forceinline__ static void mac(Acc &acc, const V16 &a, const V16 &b) {
-    if constexpr (EL::F32) {
+    if constexpr (EL::F32 && T == 32) {
       const f32x4 x = __builtin_bit_cast(f32x4, a), y = __builtin_bit_cast(f32x4, b);
 #pragma unroll
-      for (int s = 0; s < 4; s++) {
-        if constexpr (T == 32) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s], y[s], acc, 0, 0, 0);
-        else acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[s], y[s], acc, 0, 0, 0);
-      }
+      for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s], y[s], acc, 0, 0, 0);
+    } else if constexpr (EL::F32) {
+      mac_ordered(acc, ordered(a), ordered(b));
     } else if constexpr (EL::BF16) {
       const bf16x8 x = __builtin_bit_cast(bf16x8, a), y = __builtin_bit_cast(bf16x8, b);
       if constexpr (T == 32) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, acc, 0, 0, 0);
@@ -62,6 +75,18 @@ struct Tile {
       if constexpr (T == 32) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, y, acc, 0, 0, 0);
       else acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, y, acc, 0, 0, 0);
     }
+  }
+  // float32, T = 16. The instruction takes a k-value from each quarter of the wave and adds in that order, where
+  // two of the 32 x 32 form take k-values s, 4 + s, s + 1, 5 + s: the halves trade, and the bits are the same.
+  __device__ __forceinline__ static f32x4 ordered(const V16 &a) {
+    const f32x4 x = __builtin_bit_cast(f32x4, a);
+    float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
+    swap_halves(x0, x1), swap_halves(x2, x3);
+    return f32x4{x0, x2, x1, x3};
+  }
+  __device__ __forceinline__ static void mac_ordered(f32x4 &acc, const f32x4 &x, const f32x4 &y) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[s], y[s], acc, 0, 0, 0);
   }
   // accumulator element e of a lane
   __device__ __forceinline__ static int row(int e, int lane) {
@@ -208,6 +233,104 @@ __global__ __launch_bounds__(64 * MAXW) void kernel(GemmArgs a, uint32_t tiles_m
   }
 }
 
+// A float32 tile of 16 x 16 whose K is one chain, where there are at most two tiles to a unit: the chain is
+// one wave's (54 ns a step of 16 k-values), and what that wave can have in flight by itself does not feed it.
+// All CW waves of the block fetch CS steps each into LDS, in the order in which the instruction takes
+// them, while the round before is summed ([38,1754] x [1754,86]: 12.8 us, a wave by itself 19.4; [32,784] x
+// [784,128]: 7.5 and 10.1; K in eight sums, which is not the same result, 7.4 and 5.2).
+constexpr int CW = 8;
+template <bool A_KC, bool B_KC, int CS>
+__global__ __launch_bounds__(64 * CW) void chain_kernel(GemmArgs a, uint32_t tiles_m, uint32_t tiles_n) {
+  using TT = Tile<ElF32, 16>;
+  constexpr int KS = TT::KS, ROUND = CW * CS;
+  extern __shared__ __attribute__((aligned(16))) f32x4 stage[];  // [2][ROUND][A, B][64]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t per = tiles_m * tiles_n, b = blockIdx.x / per, r = blockIdx.x - b * per;
+  int64_t ao, bo, co;
+  batch_decode(a.batch, b, ao, bo, co);
+  const int64_t m0 = (int64_t)(r / tiles_n) * 16, n0 = (int64_t)(r % tiles_n) * 16;
+  const int kg = lane / 16 * TT::VE;
+  const int64_t aks = A_KC ? 1 : a.acs, bks = B_KC ? 1 : a.brs;
+  const int64_t ra = m0 + lane % 16, rb = n0 + lane % 16;
+  const float *pA = (const float *)a.A + ao + (ra < a.M ? ra : a.M - 1) * a.ars + kg * aks;
+  const float *pB = (const float *)a.B + bo + (rb < a.N ? rb : a.N - 1) * a.bcs + kg * bks;
+  const int steps = (int)((a.K + KS - 1) / KS), full = (int)(a.K / KS);
+  V16 fa[CS], fb[CS];
+  auto fetch = [&](int first) {
+#pragma unroll
+    for (int u = 0; u < CS; u++) {
+      const int s = first + wave * CS + u;
+      const int64_t k = (int64_t)s * KS;
+      if (s < full) {
+        fa[u] = fragment<ElF32, A_KC, false>(pA + k * aks, aks, 0);
+        fb[u] = fragment<ElF32, B_KC, false>(pB + k * bks, bks, 0);
+      } else if (s < steps) {  // the last step of K, not a whole one
+        fa[u] = fragment<ElF32, A_KC, true>(pA + k * aks, aks, (int)(a.K - k) - kg);
+        fb[u] = fragment<ElF32, B_KC, true>(pB + k * bks, bks, (int)(a.K - k) - kg);
+      }
+    }
+  };
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  fetch(0);
+  for (int first = 0, at = 0; first < steps; first += ROUND, at ^= ROUND) {
+    f32x4 *mine = stage + (at + wave * CS) * 128 + lane;
+#pragma unroll
+    for (int u = 0; u < CS; u++) {
+      mine[u * 128] = TT::ordered(fa[u]);
+      mine[u * 128 + 64] = TT::ordered(fb[u]);
+    }
+    fetch(first + ROUND);
+    // (also: wave 0 is through with the stage that the next round is written to)
+    __syncthreads();
+    if (wave == 0) {
+      const f32x4 *p = stage + at * 128 + lane;
+      const int n = steps - first < ROUND ? steps - first : ROUND;
+      // (four steps' operands are on their way while the four before are summed; past n: the stage's own memory)
+      constexpr int AHEAD = CS > 2 ? 4 : 2;
+      f32x4 x[2][AHEAD], y[2][AHEAD];
+      auto take = [&](int set, int s) {
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) x[set][j] = p[(s + j) * 128], y[set][j] = p[(s + j) * 128 + 64];
+      };
+      take(0, 0);
+      for (int s = 0; s < n; s += 2 * AHEAD) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          if (s + (h + 1) * AHEAD < ROUND) take(h ^ 1, s + (h + 1) * AHEAD);
+#pragma unroll
+          for (int j = 0; j < AHEAD; j++)
+            if (s + h * AHEAD + j < n) TT::mac_ordered(acc, x[h][j], y[h][j]);
+        }
+      }
+    }
+  }
+  if (wave > 0) return;
+  float *C = (float *)a.C + co;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int64_t row = m0 + TT::row(e, lane), col = n0 + lane % 16;
+    if (row < a.M && col < a.N) C[row * a.crs + col * a.ccs] = acc[e];
+  }
+}
+template <bool A_KC, bool B_KC, int CS>
+static int launch_chain(nxh_context *ctx, const GemmArgs &a, uint32_t tiles_m, uint32_t tiles_n, uint32_t total) {
+  constexpr int LDS = 2 * CW * CS * 2 * 64 * (int)sizeof(f32x4);
+  auto kern = chain_kernel<A_KC, B_KC, CS>;
+  static std::once_flag once;  // allow > 64 KiB of dynamic LDS
+  static hipError_t attr_status = hipSuccess;
+  std::call_once(once, [&] { attr_status = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS); });
+  NXH_HIP("matmul", attr_status);
+  hipLaunchKernelGGL(kern, dim3(total), dim3(64 * CW), LDS, ctx->stream, a, tiles_m, tiles_n);
+  NXH_HIP("matmul", hipGetLastError());
+  return NXH_OK;
+}
+template <int CS>
+static int launch_chain_oriented(nxh_context *ctx, const GemmArgs &a, uint32_t tiles_m, uint32_t tiles_n, uint32_t total) {
+  if (a.acs == 1) return a.brs == 1 ? launch_chain<true, true, CS>(ctx, a, tiles_m, tiles_n, total) : launch_chain<true, false, CS>(ctx, a, tiles_m, tiles_n, total);
+  return a.brs == 1 ? launch_chain<false, true, CS>(ctx, a, tiles_m, tiles_n, total) : launch_chain<false, false, CS>(ctx, a, tiles_m, tiles_n, total);
+}
+
 template <class EL, int T, int U, int R>
 static void launch(nxh_context *ctx, const GemmArgs &a, uint32_t tiles_m, uint32_t tiles_n, uint32_t total, int kw) {
   const int waves = std::max(kw, 4), per_block = waves / kw;
@@ -226,19 +349,28 @@ static int run(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch) {
   const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
   auto count = [&](int64_t t) { return (double)((a.M + t - 1) / t) * (double)((a.N + t - 1) / t) * nbatch; };
   // Tiles: as large as leaves enough waves. 32 x 32 reads half of what 16 x 16 reads, and from half a
-  // tile per unit on sharing K among eight waves fills the chip ([501,501]^2 float32: 7.9 us against
-  // 8.7); blocks of 2 x 2 waves with 64 x 64 each only where their waves alone do ([2048,2048]^2 into
-  // every second column: 170 us against 283 on 32 x 32; [501,501]^2: 41).
-  const int t = count(64) >= 4.0 * cus && a.M > 64 && a.N > 64 ? 128 : count(32) >= 0.5 * cus ? 32 : 16;
+  // tile per unit on sharing K among eight waves fills the chip; a chain of float32 steps is four times as long in a 32 x 32
+  // tile, which pays from two tiles per unit on ([1554,244] x [244,347]: 9.0 us against 10.6, [500,500]^2: 13.2
+  // against 9.1). Blocks of 2 x 2 waves with 64 x 64 each only where their waves alone fill it ([2048,2048]^2 into
+  // every second column, float32: 170 us against 283 on 32 x 32; [501,501]^2: 41 against 10).
+  const bool chain = EL::F32 && a.K <= MAX_CHAIN;
+  const bool wide = chain ? count(32) >= 2.0 * cus && a.M > 16 && a.N > 16 : count(32) >= 0.5 * cus;
+  const int t = count(64) >= 4.0 * cus && a.M > 64 && a.N > 64 ? 128 : wide ? 32 : 16;
   if (count(t) > (double)0x7fffffff || a.K > (int64_t)0x7fffffff) return -1;
   const uint32_t tm = (uint32_t)((a.M + t - 1) / t), tn = (uint32_t)((a.N + t - 1) / t), total = tm * tn * nbatch;
   const int ks = (t == 16 ? 4 : 2) * EL::VE;
   const int64_t steps = (a.K + ks - 1) / ks;
   // waves that share a tile's K: as many as put two waves on every SIMD, and no fewer than two steps each
   int kw = 1;
-  while (t < 128 && kw < MAXW && (int64_t)total * kw < 8 * cus && steps >= 4 * kw) kw *= 2;
+  while (!chain && t < 128 && kw < MAXW && (int64_t)total * kw < 8 * cus && steps >= 4 * kw) kw *= 2;
   const bool deep = (steps + kw - 1) / kw > 4;  // steps a wave has to have in flight
   nxh_set_path("gemm_mfma");
+  if constexpr (EL::F32) {
+    if (chain && t == 16 && a.K > 128) {
+      if (total <= cus) return launch_chain_oriented<4>(ctx, a, tm, tn, total);
+      if (total <= 2 * cus) return launch_chain_oriented<2>(ctx, a, tm, tn, total);
+    }
+  }
   if (t == 128) launch<EL, 32, 4, 2>(ctx, a, tm, tn, total, 1);
   else if (t == 32 && deep) launch<EL, 32, 8, 1>(ctx, a, tm, tn, total, kw);
   else if (t == 32) launch<EL, 32, 4, 1>(ctx, a, tm, tn, total, kw);

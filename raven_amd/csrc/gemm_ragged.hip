@@ -40,7 +40,7 @@ int launch_oriented(nxh_context *ctx, Args &g, bool a_kc, bool b_kc) {
 }
 
 template <class EL>
-int run(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch) {
+int run(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, int kruns) {
   const bool a_kc = a.acs == 1, b_kc = a.brs == 1;
   if (a.batch.n > 4 || a.M < 32 || a.N < 32 || a.K < 32 || a.K > 0x7fffffff) return -1;
   Args g{};
@@ -64,6 +64,13 @@ int run(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch) {
     g.bb[i] = a.batch.b[i];
     g.bc[i] = a.batch.c[i];
   }
+  if (kruns > 1) {  // (the caller has checked that there is no batch)
+    g.kruns = kruns;
+    g.nbatch = nbatch = (uint32_t)kruns;
+    g.nbd = 1;
+    g.bshape[0] = (uint32_t)kruns;
+    g.bc[0] = a.M * a.N;
+  }
   auto tiles = [&](int bm, int bn) { return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * (int64_t)nbatch; };
   if (tiles(64, 64) > 0x7fffffffLL) return -1;
   const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
@@ -84,14 +91,14 @@ int run(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch) {
   if (pick == 0) return launch_oriented<EL, Shape256x256>(ctx, g, a_kc, b_kc);
   if (pick == 1) return launch_oriented<EL, Shape128x128>(ctx, g, a_kc, b_kc);
   if constexpr (!EL::F32) {  // two groups of waves a block (gemm_tile.hpp), from eight slabs on
-    if (a.K > 7 * Geo<EL>::BK && tiles(128, 64) <= cus) return launch_oriented<EL, Shape128x64Halves>(ctx, g, a_kc, b_kc);
+    if (kruns == 1 && a.K > 7 * Geo<EL>::BK && tiles(128, 64) <= cus) return launch_oriented<EL, Shape128x64Halves>(ctx, g, a_kc, b_kc);
   }
   return launch_oriented<EL, std::conditional_t<EL::F32, Shape64x64, Shape128x64>>(ctx, g, a_kc, b_kc);
 }
 }  // namespace
 
-int nxh_gemm_ragged(nxh_context *ctx, int dtype, const GemmArgs &a, uint32_t nbatch) {
-  if (dtype == NXH_F32) return run<ElF32>(ctx, a, nbatch);
-  if (dtype == NXH_BF16) return run<ElBF16>(ctx, a, nbatch);
-  return run<ElF16>(ctx, a, nbatch);
+int nxh_gemm_ragged(nxh_context *ctx, int dtype, const GemmArgs &a, uint32_t nbatch, int kruns) {
+  if (dtype == NXH_F32) return run<ElF32>(ctx, a, nbatch, kruns);
+  if (dtype == NXH_BF16) return run<ElBF16>(ctx, a, nbatch, 1);
+  return run<ElF16>(ctx, a, nbatch, 1);
 }

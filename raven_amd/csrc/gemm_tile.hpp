@@ -154,6 +154,9 @@ struct Args {
   uint32_t ngroup, gtn;
   int64_t goff_b[2], goff_c[2], goff_bias[2];
   int64_t ccs;  // RAG kernels: distance of two columns of C
+  // RAG kernels, no batch: more than one, and tile batch i is run i of that many equal runs of K's slabs
+  // (their sums [kruns][M][N])
+  int kruns;
 };
 
 // The arithmetic of the fused linear's epilogue on 16-bit results, two neighbours per
@@ -427,18 +430,17 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
     for (int u = 0; u < TN; u++)
 #pragma unroll
       for (int e = 0; e < 16; e++) acc[t][u][e] = 0.0f;
-  // The one-tile waves of the ragged form sum the odd k-steps apart: half the length of the chain of
-  // roundings, as a product cut in two along K would have it.
-  constexpr bool TWO = RAG && TM * TN == 1;
-  f32x16 odd;
-  if constexpr (TWO) {
-#pragma unroll
-    for (int e = 0; e < 16; e++) odd[e] = 0.0f;
-  }
-
   V16 ra[NVA], rb[NVB];
   const int slabs = (int)(RAG ? (a.K + BK - 1) / BK : a.K / BK);
   int nk = slabs, k0 = 0;  // this group's run of them (the host has checked that every group has one)
+  if constexpr (RAG && KG == 1) {
+    if (a.kruns > 1) {
+      nk = slabs / a.kruns;
+      k0 = (int)batch * nk;
+      gA += k0 * stepA;
+      gB += k0 * stepB;
+    }
+  }
   if constexpr (KG > 1) {
     const int more = slabs % KG;
     nk = slabs / KG + (group < more);
@@ -531,7 +533,7 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
 #pragma unroll
       for (int t = 0; t < TM; t++)
 #pragma unroll
-        for (int u = 0; u < TN; u++) mfma_step<EL>(TWO && cur ? odd : acc[t][u], fa[cur][t], fb[cur][u]);
+        for (int u = 0; u < TN; u++) mfma_step<EL>(acc[t][u], fa[cur][t], fb[cur][u]);
       // The memory instructions of this k-step are issued among its MFMAs, one LDS read, one
       // LDS write and one global load behind each (LDS returns in order, so the wait before the
       // first MFMA only covers the current fragments): queueing them all in front of the step
@@ -552,10 +554,6 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(SH:
     if (kt + 2 < nk) slab(kt++, yes{}, yes{}, yes{});
   if (kt + 1 < nk) slab(kt++, yes{}, no{}, no{});
   slab(kt, no{}, no{}, no{});
-  if constexpr (TWO) {
-#pragma unroll
-    for (int e = 0; e < 16; e++) acc[0][0][e] += odd[e];
-  }
 
   if constexpr (KG > 1) {
     // the groups' sums meet in the stages, group 0 adds them in order and is the one that stores

@@ -923,6 +923,53 @@ static int try_strip(nxh_context *ctx, int dtype, const GemmArgs &a, uint32_t nb
   }
   return nxh_gemm_strip(ctx, dtype, g);
 }
+static int64_t block_tiles(const GemmArgs &a, int64_t nbatch, int bm, int bn) {
+  return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * nbatch;
+}
+// The block shape of a float32 product: a compute unit's f32 matrix rate is a sixteenth of its 16-bit rate, so
+// a block's time is all arithmetic and the shapes differ only in what they leave idle: rounds of one block
+// per unit x the block's area (ragged edges count as whole blocks) x the shape's measured cost
+// per flop against the 256 x 256 block (4096^3: 138 TFLOP/s there, 123 with half blocks;
+// 1024^3 on quarter blocks about 100 inside the K loop). Two slabs of K are mostly first loads and
+// stores, which the small blocks overlap best (32 x [288,64] x [64,784]: 19.8 us on quarter blocks, 23.3 on half).
+static int pick_f32(const GemmArgs &a, int64_t nbatch, int64_t members, int64_t cus) {
+  struct Cand {
+    int pick, bm, bn;
+    double pen;
+  };
+  const Cand cands[] = {{256, 256, 256, 1.0}, {128, 128, 128, 1.12}, {64, 256, 64, 1.12},
+                        {1264, 128, 64, 1.15}, {6464, 64, 64, a.K <= 2 * gemm_tile::Geo<gemm_tile::ElF32>::BK ? 1.15 : 1.3}};
+  int pick = 0;
+  double best = 0.0;
+  for (const Cand &c : cands) {
+    if (c.pick == 64 && a.N > 64) continue;
+    const double cost = (double)((block_tiles(a, nbatch, c.bm, c.bn) * members + cus - 1) / cus) * c.bm * c.bn * c.pen;
+    if (!pick || cost < best) {
+      pick = c.pick;
+      best = cost;
+    }
+  }
+  return pick;
+}
+// Runs that a product's K is cut into when its `blocks` leave half of the units idle and K is long (a weight
+// gradient: [768, 8192] x [8192, 768]); 1: stays whole. Worth it when the slabs a block no longer walks (about
+// 0.3 us each for a 16-bit block that has its unit to itself, 0.7 us for f32) outweigh the second launch and
+// the partial sums' trip through memory (bf16 [1000,8192] x [8192,1000]: 57 -> 39 us with two runs; [1024,1024]^2
+// would go from 9.5 to 15 us and stays whole).
+static int64_t runs_along_k(const GemmArgs &a, bool f32, int64_t slabs, int64_t blocks, int64_t cus) {
+  int64_t runs = 1;
+  double best_gain = 0.0;
+  for (int64_t sp = std::min<int64_t>(cus / blocks, slabs / 4); sp >= 2; sp--) {
+    if (slabs % sp) continue;
+    const double saved = (double)slabs * (1.0 - 1.0 / (double)sp) * (f32 ? 0.7 : 0.3);
+    const double cost = 4.0 + (double)sp * (double)a.M * (double)a.N * 8.0 / 4e6;
+    if (saved - 1.2 * cost > best_gain) {
+      best_gain = saved - 1.2 * cost;
+      runs = sp;
+    }
+  }
+  return runs;
+}
 template <class EL, bool EPI = false>
 static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool al_a, bool al_b,
                     const Epilogue *epi = nullptr) {
@@ -1013,7 +1060,7 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
   // tiles of one member: a grouped launch picks the block shape its members would pick alone,
   // so that each member's bits are those of its own call
   const int members = EPI && epi ? epi->ngroup : 1;
-  auto tiles = [&](int bm, int bn) { return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * (int64_t)nbatch; };
+  auto tiles = [&](int bm, int bn) { return block_tiles(a, nbatch, bm, bn); };
   if (tiles(128, 64) * members > 0x7fffffffLL) return -1;
   const int cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
   if constexpr (!EL::F32) {
@@ -1035,28 +1082,7 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
   const auto pick_for = [&](int64_t members) {
     int pick = 0;
     if constexpr (EL::F32) {
-      // f32: a compute unit's f32 matrix rate is a sixteenth of its 16-bit rate, so a block's time
-      // is all arithmetic and the shapes differ only in what they leave idle: rounds of one block
-      // per unit x the block's area (ragged edges count as whole blocks) x the shape's measured cost
-      // per flop against the 256 x 256 block (4096^3: 138 TFLOP/s there, 123 with half blocks;
-      // 1024^3 on quarter blocks about 100 inside the K loop). Two slabs of K are mostly first loads and
-      // stores, which the small blocks overlap best (32 x [288,64] x [64,784]: 19.8 us on quarter blocks, 23.3 on half).
-      struct Cand {
-        int pick, bm, bn;
-        double pen;
-      };
-      const Cand cands[] = {{256, 256, 256, 1.0}, {128, 128, 128, 1.12}, {64, 256, 64, 1.12},
-                            {1264, 128, 64, 1.15}, {6464, 64, 64, a.K <= 2 * BK ? 1.15 : 1.3}};
-      double best = 0.0;
-      for (const Cand &c : cands) {
-        if (c.pick == 64 && a.N > 64) continue;
-        if (EPI && epi->gelu && c.pick != 256 && c.pick != 128) continue;
-        const double cost = (double)((tiles(c.bm, c.bn) * members + cus - 1) / cus) * c.bm * c.bn * c.pen;
-        if (!pick || cost < best) {
-          pick = c.pick;
-          best = cost;
-        }
-      }
+      pick = pick_f32(a, nbatch, members, cus);
     } else {
       if (a.N <= 64) pick = 64;
       else {
@@ -1170,25 +1196,8 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
         if (split >= 2) return cut_along_k(split, 2);
       }
     }
-    // A product whose blocks leave half of the units idle and whose K is long (a weight gradient:
-    // [768, 8192] x [8192, 768]).
     if (nbatch == 1 && a.batch.n == 0 && (pick == 1264 || pick == 6464)) {
-      const int64_t blocks = pick == 6464 ? tiles(64, 64) : tiles(128, 64);
-      // Worth it when the slabs a block no longer walks (about 0.3 us each for a 16-bit block that
-      // has its unit to itself, 0.7 us for f32) outweigh the second launch and the partial sums'
-      // trip through memory (bf16 [1000,8192] x [8192,1000]: 57 -> 39 us with two runs; [1024,1024]^2
-      // would go from 9.5 to 15 us and stays whole).
-      int64_t split = 1;
-      double best_gain = 0.0;
-      for (int64_t sp = std::min<int64_t>(cus / blocks, slabs / 4); sp >= 2; sp--) {
-        if (slabs % sp) continue;
-        const double saved = (double)slabs * (1.0 - 1.0 / (double)sp) * (EL::F32 ? 0.7 : 0.3);
-        const double cost = 4.0 + (double)sp * (double)a.M * (double)a.N * 8.0 / 4e6;
-        if (saved - 1.2 * cost > best_gain) {
-          best_gain = saved - 1.2 * cost;
-          split = sp;
-        }
-      }
+      const int64_t split = runs_along_k(a, EL::F32, slabs, pick == 6464 ? tiles(64, 64) : tiles(128, 64), cus);
       if (split >= 2) return cut_along_k(split, pick == 6464 ? 0 : 1);
     }
   }
@@ -1342,6 +1351,27 @@ static int launch_rowdot(nxh_context *ctx, GemmArgs &a, uint32_t nbatch, bool ba
   return NXH_OK;
 }
 
+// A float32 product of any K and alignment, cut into `runs` equal runs of K's slabs whose sums a second kernel
+// adds in run order (as cut_along_k in try_tile).
+static int ragged_along_k(nxh_context *ctx, const GemmArgs &a, int runs) {
+  void *part = nullptr;
+  int rc = nxh_alloc_locked(ctx, (size_t)runs * a.M * a.N * sizeof(float), &part);
+  if (rc) return rc;
+  GemmArgs g = a;
+  g.C = part;
+  g.crs = a.N;
+  g.ccs = 1;
+  rc = nxh_gemm_ragged(ctx, NXH_F32, g, 1, runs);
+  if (rc == NXH_OK) {
+    hipLaunchKernelGGL((skinny_finish_kernel<NXH_F32>), dim3((unsigned)((a.M * a.N + 1023) / 1024)), dim3(256), 0, ctx->stream,
+                       (const float *)part, a.C, a.M, a.N, runs, a.crs, a.ccs);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) rc = nxh_hip_fail("matmul", e);
+  }
+  nxh_free_locked(ctx, part);
+  return rc;
+}
+
 template <class MM>
 static int run_mfma_dtype(nxh_context *ctx, GemmArgs &a, uint32_t nbatch, bool batch_aligned_a,
                           bool batch_aligned_b) {
@@ -1415,8 +1445,20 @@ static int run_mfma_dtype(nxh_context *ctx, GemmArgs &a, uint32_t nbatch, bool b
     // against 6.7. A K of one slab is loads and stores, which the general kernel does not stage.
     const int64_t bm = sizeof(S) == 4 ? 64 : 128;
     const double blocks = (double)((a.M + bm - 1) / bm) * (double)((a.N + 63) / 64) * nbatch;
+    if constexpr (MM::DT == NXH_F32) {
+      // cut along K where the aligned form of these sizes would be: the same sums
+      const int64_t slabs = (a.K + gemm_tile::Geo<EL>::BK - 1) / gemm_tile::Geo<EL>::BK;
+      const int pick = pick_f32(a, nbatch, 1, cus);
+      if (terms >= (double)(1 << 27) && nbatch == 1 && a.batch.n == 0 && (pick == 6464 || pick == 1264)) {
+        const int64_t runs = runs_along_k(a, true, slabs, pick == 6464 ? block_tiles(a, 1, 64, 64) : block_tiles(a, 1, 128, 64), cus);
+        if (runs > 1) {
+          rc = ragged_along_k(ctx, a, (int)runs);
+          if (rc != -1) return rc;
+        }
+      }
+    }
     if (terms >= (double)(1 << 27) || (a.K >= 64 && blocks >= (sizeof(S) == 4 ? 0.75 : 0.6) * (double)cus)) {
-      rc = nxh_gemm_ragged(ctx, MM::DT, a, nbatch);
+      rc = nxh_gemm_ragged(ctx, MM::DT, a, nbatch, 1);
       if (rc != -1) return rc;
     }
   }
