@@ -1067,11 +1067,14 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
     // Few result tiles under a long K: a strip of B a block (gemm_strip.hip). [48,768] x [768,768] bfloat16
     // 5.1 us against 7.3 as half blocks, [400,768] x [768,768] (84 tiles of 64 x 64) 6.0 against 7.6. Three
     // such layers over one input are one launch: from 3/8 of a tile per unit on their tiles outnumber the
-    // units and the kernels below are the faster ones ([1024,768] x 3 [768,768]: 16 us against 20). A plain product
-    // of a longer K is better off cut along it by the rule below ([512,3072] x [3072,768]: 14.0 against 15.0)
-    // unless the strips are cut too ([48,3072] x [3072,768]: 9.5 against 7.8).
-    if (a_kc && !b_kc && !(EPI && epi->gelu) && a.K >= 512 && a.N >= 512 && tiles(64, 64) <= 3 * cus / 8 && !forced_tile() &&
-        (EPI || a.K < 2048 || nxh_gemm_strip_blocks(ctx, a.M, a.N, a.K, nbatch) > 1) && !(a.M <= 128 && (double)a.K * (double)a.N * 2.0 >= (double)(16 << 20))) {
+    // units and the kernels below are the faster ones ([1024,768] x 3 [768,768]: 16 us against 20). A single plain
+    // product of a longer K is better off cut along it where the rule below cuts it ([512,3072] x [3072,768]: 14.0
+    // against 15.0) unless the strips are cut too ([48,3072] x [3072,768]: 9.5 against 7.8). A batch, which is
+    // not cut, and a fused linear take the same kernel, so that they have the same bits.
+    const bool cut = !EPI && nbatch == 1 && a.batch.n == 0 && a.K >= 2048 && nxh_gemm_strip_blocks(ctx, a.M, a.N, a.K, nbatch) == 1 &&
+                     runs_along_k(a, false, a.K / BK, tiles(128, 64), cus) > 1;
+    if (a_kc && !b_kc && !(EPI && epi->gelu) && a.K >= 512 && a.N >= 512 && tiles(64, 64) <= 3 * cus / 8 && !forced_tile() && !cut &&
+        !(a.M <= 128 && (double)a.K * (double)a.N * 2.0 >= (double)(16 << 20))) {
       const int rc = try_strip(ctx, EL::BF16 ? NXH_BF16 : NXH_F16, a, nbatch, epi);
       if (rc != -1) return rc;
     }

@@ -1,0 +1,39 @@
+"""How K is summed is decided by a product's sizes alone: the plain product of a batch, the fused linear and
+the linear with the GELU behind it have the same bits, on both sides of the rules of gemm_strip.hip (few result
+tiles), of the blocks with two groups of waves and of the columns past the last whole 256."""
+
+import numpy as np
+import pytest
+
+from helpers import encode, pair, same_bits
+from raven_amd import dtype as dt
+from raven_amd.nx_backend import logical
+
+pytestmark = pytest.mark.gpu
+HALVES = [dt.bfloat16, dt.float16]
+
+
+def operands(hip, oracle, d, lead, m, k, n):
+    rng = np.random.default_rng(m + k + n)
+    return [pair(encode(rng.standard_normal(s), d, oracle), d, hip, oracle)[0] for s in ((*lead, m, k), (k, n), (n,))]
+
+
+def primitives(hip, x, w, b):
+    lead, (m, k), n = x.shape[:-2], x.shape[-2:], w.shape[-1]
+    wide = hip.expand(hip.reshape(w, (1,) * len(lead) + (k, n)), (*lead, k, n)) if lead else w
+    p = hip.matmul(x, wide)
+    path = hip.last_path()
+    return hip.binary("add", p, hip.expand(hip.reshape(b, (1,) * (len(lead) + 1) + (n,)), (*lead, m, n))), path
+
+
+@pytest.mark.parametrize("d", HALVES, ids=lambda d: d.name)
+@pytest.mark.parametrize("lead,m,k,n,path", [
+    ((2,), 256, 3072, 768, "strip"),    # a long K, one block a tile
+    ((2,), 192, 2048, 520, "strip"),
+    ((), 256, 2368, 768, "strip"),      # one product: 37 slabs, which no number of runs divides
+])
+def test_linear_of_a_long_k_equals_its_primitives(hip, oracle, d, lead, m, k, n, path):
+    x, w, b = operands(hip, oracle, d, lead, m, k, n)
+    want, plain = primitives(hip, x, w, b)
+    same_bits(logical(hip.linear(x, w, b)), logical(want))
+    assert (plain, hip.last_path()) == (f"gemm_{path}", f"linear_{path}")
