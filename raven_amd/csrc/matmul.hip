@@ -972,15 +972,16 @@ static int64_t runs_along_k(const GemmArgs &a, bool f32, int64_t slabs, int64_t 
 }
 template <class EL, bool EPI = false>
 static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool al_a, bool al_b,
-                    const Epilogue *epi = nullptr) {
+                    const Epilogue *epi = nullptr, bool remainder = false) {
   constexpr int VE = EL::VE, BK = gemm_tile::Geo<EL>::BK;
   if (a.K % BK || a.K < BK || a.M < VE || a.N < VE) return -1;
   if (a.ccs != 1 || a.batch.n > 4 || !al_a || !al_b) return -1;
   const bool a_kc = a.acs == 1, b_kc = a.brs == 1;
   // A wide 16-bit product whose N is no whole number of 256-column blocks (GPT-2's tied head,
   // [8192,768] x [768,50257]): the whole blocks take the direct-to-LDS kernel, which has no
-  // ragged form, and the last columns a launch of their own. Every output element is still
-  // one k-ordered f32 sum rounded once, so the split changes no bit of the result.
+  // ragged form, and the last columns a launch of their own (`remainder`: without K shared by two groups of
+  // waves). Every output element is still one k-ordered f32 sum rounded once, so the split changes no bit of the
+  // result; only the last columns of a single product (no batch) whose K is long enough are cut along it below.
   if constexpr (!EL::F32 && !EPI) {
     const int64_t n0 = a.N / 256 * 256;
     if (a.N % 256 && n0 >= 8 * 256 && a.M % 256 == 0 && a.M >= 1024 && !forced_tile() && a.n_ld == a.N) {
@@ -993,7 +994,7 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
       if (rc == NXH_OK) {
         const char *path = nxh_last_path(ctx);
         // (the right part's B starts n0 columns in: 16-byte aligned, since n0 is a multiple of 256)
-        rc = try_tile<EL, false>(ctx, right, nbatch, al_a, al_b, nullptr);
+        rc = try_tile<EL, false>(ctx, right, nbatch, al_a, al_b, nullptr, true);
         nxh_set_path(path);
       }
       if (rc != -1) return rc;  // (-1: the whole product takes the ordinary path below; what the left part wrote is rewritten)
@@ -1105,7 +1106,7 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
   // group of linears: a member's sums are those of its own call.
   const int alone = pick_for(1);
   const int64_t slabs = a.K / BK;
-  const bool halves = !EL::F32 && !forced_tile() && alone == 1264 && slabs >= 24 && tiles(128, 64) <= cus;
+  const bool halves = !EL::F32 && !remainder && !forced_tile() && alone == 1264 && slabs >= 24 && tiles(128, 64) <= cus;
   int pick = forced_tile() ? forced_tile() : halves ? alone : pick_for(members);
   // Whole tiles of 16-bit operands go straight into LDS (gemm_dl.hpp; load offsets are 32-bit:
   // 256 rows of a k-contiguous operand must stay below 4 GiB, and every row segment the

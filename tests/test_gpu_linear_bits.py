@@ -37,3 +37,11 @@ def test_linear_of_a_long_k_equals_its_primitives(hip, oracle, d, lead, m, k, n,
     want, plain = primitives(hip, x, w, b)
     same_bits(logical(hip.linear(x, w, b)), logical(want))
     assert (plain, hip.last_path()) == (f"gemm_{path}", f"linear_{path}")
+
+
+@pytest.mark.parametrize("d", HALVES, ids=lambda d: d.name)
+@pytest.mark.parametrize("lead,m,k,n", [((2,), 1024, 1536, 2112), ((2,), 1024, 1600, 2056)])
+def test_columns_past_the_last_whole_256(hip, oracle, d, lead, m, k, n):
+    x, w, b = operands(hip, oracle, d, lead, m, k, n)
+    want, _ = primitives(hip, x, w, b)
+    same_bits(logical(hip.linear(x, w, b)), logical(want))
