@@ -93,6 +93,7 @@ __device__ __forceinline__ void put(const Args &a, const Where<EPI> &w, int p, i
       const V8 y = *reinterpret_cast<const V8a2 *>(w.bias + w.col);
       v = V8{gemm_tile::epi_add2<EL>(v[0], y[0]), gemm_tile::epi_add2<EL>(v[1], y[1])};
     }
+    if (a.gelu) v = V8{gemm_tile::epi_gelu2<EL>(v[0], a.gc[0], a.gc[1], a.gc[2], a.gc[3]), gemm_tile::epi_gelu2<EL>(v[1], a.gc[0], a.gc[1], a.gc[2], a.gc[3])};
     if (a.R) {
       const V8 y = *reinterpret_cast<const V8a2 *>((const uint16_t *)a.R + w.ro + row * a.ldr + w.col);
       v = V8{gemm_tile::epi_add2<EL>(v[0], y[0]), gemm_tile::epi_add2<EL>(v[1], y[1])};
@@ -197,7 +198,7 @@ __global__ __launch_bounds__(64 * MAXW) void kernel(Args a, int kw, int parts, u
   }
 
   auto piece = [&](int p) { return f32x4{acc[p >> 2][0][p & 3], acc[p >> 2][1][p & 3], acc[p >> 2][2][p & 3], acc[p >> 2][3][p & 3]}; };
-  if (kw == 1) {
+  if (!EPI && kw == 1) {  // (a linear's K is that of several waves)
 #pragma unroll
     for (int p = 0; p < MT * 4; p++) put<EL, EPI>(a, w, p, lane, piece(p));
     return;
@@ -266,7 +267,7 @@ static int run(nxh_context *ctx, Args &g) {
   // same loads as the first ([512,3072] x [3072,768]: 384 tiles of 16 rows 20.6 us, 192 of 32 rows 15.4;
   // [256,768] x [768,3072]: 768 tiles 10.7, 384 11.3, 192 of 64 rows 8.7)
   auto tiles = [&](int64_t bm) { return ((g.M + bm - 1) / bm) * ((g.N + BN - 1) / BN) * (int64_t)g.nbatch * (EPI ? g.ngroup : 1); };
-  if (tiles(16) > 0x7fffffffLL) return -1;
+  if (tiles(16) > 0x7fffffffLL || (EPI && kw == 1)) return -1;
   if (blocks > 1 || g.M <= 16 || tiles(16) <= cus) return launch<EL, 1, EPI>(ctx, g, kw, blocks);
   if (g.M <= 32 || tiles(32) <= cus) return launch<EL, 2, EPI>(ctx, g, kw, 1);
   return launch<EL, 4, EPI>(ctx, g, kw, 1);
@@ -294,7 +295,7 @@ int nxh_gemm_strip(nxh_context *ctx, int dtype, gemm_strip::Args &g) {
   // what a lane's 32-bit offsets hold: 24 rows of B and a row's columns, 64 rows of A
   if (g.N < 4 || g.ldb < 0 || g.lda < 0 || g.K > 0x7fffffff || g.nbd > 4) return -1;
   if ((double)g.ldb * 48.0 + (double)g.N * 2.0 >= 4294967296.0 || (double)g.lda * 130.0 + 64.0 >= 4294967296.0) return -1;
-  const bool epi = g.bias || g.R;
+  const bool epi = g.bias || g.R || g.gelu;
   if (dtype == NXH_BF16) return epi ? run<ElBF16, true>(ctx, g) : run<ElBF16, false>(ctx, g);
   return epi ? run<ElF16, true>(ctx, g) : run<ElF16, false>(ctx, g);
 }

@@ -12,6 +12,8 @@ struct Args {
   int64_t M, N, K;
   const void *bias, *R;  // null: left out
   int64_t ldr;
+  int gelu;  // no R: then the tanh GELU on the biased product (gemm_tile.hpp)
+  float gc[4];
   uint32_t tiles_m, tiles_n, nbatch;
   int nbd;
   uint32_t bshape[4];

@@ -914,6 +914,10 @@ static int try_strip(nxh_context *ctx, int dtype, const GemmArgs &a, uint32_t nb
   }
   if (epi) {
     g.bias = epi->bias, g.R = epi->R, g.ldr = epi->ldr;
+    if (epi->gelu) {
+      g.gelu = 1;
+      for (int i = 0; i < 4; i++) g.gc[i] = (float)epi->gelu[i];
+    }
     g.ngroup = (uint32_t)epi->ngroup;
     for (int i = 0; i + 1 < epi->ngroup; i++) {
       g.goff_b[i] = epi->goff_b[i] / 2;
@@ -1071,10 +1075,10 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
     // units and the kernels below are the faster ones ([1024,768] x 3 [768,768]: 16 us against 20). A single plain
     // product of a longer K is better off cut along it where the rule below cuts it ([512,3072] x [3072,768]: 14.0
     // against 15.0) unless the strips are cut too ([48,3072] x [3072,768]: 9.5 against 7.8). A batch, which is
-    // not cut, and a fused linear take the same kernel, so that they have the same bits.
+    // not cut, and a fused linear, with the GELU or without, take the same kernel, so that they have the same bits.
     const bool cut = !EPI && nbatch == 1 && a.batch.n == 0 && a.K >= 2048 && nxh_gemm_strip_blocks(ctx, a.M, a.N, a.K, nbatch) == 1 &&
                      runs_along_k(a, false, a.K / BK, tiles(128, 64), cus) > 1;
-    if (a_kc && !b_kc && !(EPI && epi->gelu) && a.K >= 512 && a.N >= 512 && tiles(64, 64) <= 3 * cus / 8 && !forced_tile() && !cut &&
+    if (a_kc && !b_kc && a.K >= 512 && a.N >= 512 && tiles(64, 64) <= 3 * cus / 8 && !forced_tile() && !cut &&
         !(a.M <= 128 && (double)a.K * (double)a.N * 2.0 >= (double)(16 << 20))) {
       const int rc = try_strip(ctx, EL::BF16 ? NXH_BF16 : NXH_F16, a, nbatch, epi);
       if (rc != -1) return rc;
@@ -1083,7 +1087,7 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
   // Block shape: rounds of resident blocks x relative cost of one block. One
   // 256x256 block (8 waves, 144 KiB of LDS) fills a CU; two 128x128 blocks fit,
   // each a quarter of the work at about 0.8 of the big tile's efficiency.
-  const auto pick_for = [&](int64_t members) {
+  const auto pick_for = [&](int64_t members, bool gelu) {
     int pick = 0;
     if constexpr (EL::F32) {
       pick = pick_f32(a, nbatch, members, cus);
@@ -1096,18 +1100,19 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
       }
       // Fewer blocks than half the compute units: half blocks (128 x 64, four waves of 64 x 32)
       // put twice as many of them to work (bf16 [1024,768] x [768,768]: 9.5 -> 7.9 us).
-      if (pick != 256 && !(EPI && epi->gelu) && (pick == 64 ? tiles(256, 64) : tiles(128, 128)) * members <= cus / 2)
+      if (pick != 256 && !gelu && (pick == 64 ? tiles(256, 64) : tiles(128, 128)) * members <= cus / 2)
         pick = 1264;
     }
     return pick;
   };
   // Half blocks one to a unit under a long K: two groups of waves each (Shape128x64Halves). From 24 slabs on (of 12
   // the groups' meeting takes what they gain: [2048,768] x [768,768] 11.9 us either way). Decided without the
-  // group of linears: a member's sums are those of its own call.
-  const int alone = pick_for(1);
+  // group of linears and without the GELU: a member's sums are those of its own call, and the GELU's input is
+  // what the linear stores.
+  const int alone = pick_for(1, false);
   const int64_t slabs = a.K / BK;
   const bool halves = !EL::F32 && !remainder && !forced_tile() && alone == 1264 && slabs >= 24 && tiles(128, 64) <= cus;
-  int pick = forced_tile() ? forced_tile() : halves ? alone : pick_for(members);
+  int pick = forced_tile() ? forced_tile() : halves ? alone : pick_for(members, EPI && epi->gelu);
   // Whole tiles of 16-bit operands go straight into LDS (gemm_dl.hpp; load offsets are 32-bit:
   // 256 rows of a k-contiguous operand must stay below 4 GiB, and every row segment the
   // epilogue touches must be 16-byte aligned).
@@ -1149,7 +1154,7 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
       if (rc != -1) return rc;
     }
   }
-  if (g.gelu && (a.M % 128 || a.N % 128)) return -1;
+  if (g.gelu && !halves && (a.M % 128 || a.N % 128)) return -1;
   if (pick == 192) pick = 128;
   if constexpr (!EPI) {
     // One product (no batch) cut along K: `split` equal runs of whole slabs are walked as a batch

@@ -45,3 +45,16 @@ def test_columns_past_the_last_whole_256(hip, oracle, d, lead, m, k, n):
     x, w, b = operands(hip, oracle, d, lead, m, k, n)
     want, _ = primitives(hip, x, w, b)
     same_bits(logical(hip.linear(x, w, b)), logical(want))
+
+
+@pytest.mark.parametrize("d", HALVES, ids=lambda d: d.name)
+@pytest.mark.parametrize("m,k,n,path", [
+    (128, 768, 3072, "linear_strip"), (256, 512, 576, "linear_strip"), (128, 4096, 512, "linear_strip"),
+    (1024, 1536, 768, "linear_tile_128x64"), (1024, 1600, 576, "linear_tile_128x64"),
+    (128, 1536, 128, "linear_tile_128x64"), (1024, 1472, 768, "linear_dl_128x192"),
+])
+def test_linear_gelu_equals_the_two_calls(hip, oracle, d, m, k, n, path):
+    x, w, b = operands(hip, oracle, d, (), m, k, n)
+    want = logical(hip.gelu_tanh(hip.linear(x, w, b)))
+    same_bits(logical(hip.linear_gelu_tanh(x, w, b)), want)
+    assert hip.last_path() == path
