@@ -517,7 +517,7 @@ __global__ __launch_bounds__(256) void scatter_keys_kernel(const int32_t *idx, i
   int64_t v = idx[i * stride];
   if (v < 0) v += axis_len;
   if (v < 0 || v >= axis_len) {
-    atomicOr(fault, 1);
+    raise_fault(fault);
     v = -1;  // sorts first, applied by nobody
   }
   key[i] = (int32_t)v;
