@@ -44,9 +44,33 @@ __global__ __launch_bounds__(64 * W) void qr_panel_kernel(QrPanelArgs a) {
   double *A = a.at + ((size_t)blockIdx.x * a.n + a.p0) * a.m + a.p0;
   auto row_of = [&](int e) { return 4 * (e * W + wave) + q; };
   constexpr int HEAD = W >= 4 ? 1 : 4 / W;  // elements that may lie in the first sixteen rows
-  double x[E];
+  double x[E], biggest = 0.0;
 #pragma unroll
-  for (int e = 0; e < E; e++) x[e] = c < w && row_of(e) < rows ? A[(size_t)c * a.m + row_of(e)] : 0.0;
+  for (int e = 0; e < E; e++) {
+    x[e] = c < w && row_of(e) < rows ? A[(size_t)c * a.m + row_of(e)] : 0.0;
+    biggest = fmax(biggest, fabs(x[e]));  // (passes over a NaN)
+  }
+  // The products below are of two columns as they come: a column whose square, or whose product with another, would
+  // leave float64's range is worked on times a power of two and stored times its inverse. Columns between
+  // 2^-400 and 2^480 are left alone; the others come to 2^0 and 2^400, the large ones so that their small
+  // elements keep their bits.
+  biggest = fmax(biggest, __shfl_xor(biggest, 16));
+  biggest = fmax(biggest, __shfl_xor(biggest, 32));
+  if constexpr (W > 1) {
+    if (q == 0) part[1][wave][c] = biggest;  // (column 1 is the next to use it, a barrier later)
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < W; i++) biggest = fmax(biggest, part[1][i][c]);
+  }
+  int power = 0;
+  if (biggest > 0.0 && biggest < __builtin_inf()) {
+    const int ex = __builtin_amdgcn_frexp_exp(biggest);
+    power = ex < -400 ? ex : ex > 480 ? ex - 400 : 0;
+  }
+  if (__any(power != 0)) {
+#pragma unroll
+    for (int e = 0; e < E; e++) x[e] = ldexp(x[e], -power);
+  }
   // x / y, rounded, by the reciprocal of y: its own error is the same in every element
   auto divided = [](double x, double y, double inv) {
     const double d = x * inv;
@@ -126,7 +150,7 @@ __global__ __launch_bounds__(64 * W) void qr_panel_kernel(QrPanelArgs a) {
     const double v = !in || row < c ? 0.0 : row == c ? 1.0 : divided(x[e], my_scal, my_rs);
     vtv = __builtin_amdgcn_mfma_f64_16x16x4f64(v, v, vtv, 0, 0, 0);
     if (in) {
-      A[(size_t)c * a.m + row] = row < c ? x[e] : row == c ? (reflected ? my_beta : x[e]) : 0.0;
+      A[(size_t)c * a.m + row] = row > c ? 0.0 : ldexp(row == c && reflected ? my_beta : x[e], power);
       V[row] = v;
     }
   }

@@ -1,0 +1,27 @@
+"""QR of columns whose squares or products leave float64's range."""
+
+import numpy as np
+import pytest
+
+from helpers import logical
+from raven_amd import dtype as dt
+
+pytestmark = pytest.mark.gpu
+
+
+def qr(hip, a):
+    return [logical(t) for t in hip.qr(hip.reshape(hip.from_host(a, dt.float64), a.shape))]
+
+
+@pytest.mark.parametrize("m,n", [(6, 3), (40, 40), (70, 20), (300, 21), (1030, 18)])
+def test_columns_times_powers_of_two(hip, m, n):
+    """A column times a power of two changes nothing but that column of R, to the last bit."""
+    rng = np.random.default_rng(m)
+    a = rng.standard_normal((m, n))
+    q, r = qr(hip, a)
+    for powers in ([-100, -995], [-465, -614], [-399, -401, 479, 481], [-900, 0, 900], [500, 560], [-620]):
+        e = np.resize(powers, n)
+        rng.shuffle(e)
+        qs, rs = qr(hip, np.ldexp(a, e))
+        assert np.array_equal(qs, q), powers
+        assert np.array_equal(rs, np.ldexp(r, e)), powers
