@@ -88,7 +88,8 @@ __global__ __launch_bounds__(64 * W) void qr_panel_kernel(QrPanelArgs a) {
     for (int e = 0; e < E; e++) {
       b[e] = bcast16<j>(x[e]);
       if (e < HEAD) b[e] = row_of(e) > j ? b[e] : 0.0;
-      p4[e & 3] = fma(b[e], x[e], p4[e & 3]);
+      // (rows that are done have no part in the sums: they may hold an infinity)
+      p4[e & 3] = fma(b[e], e < HEAD && row_of(e) <= j ? 0.0 : x[e], p4[e & 3]);
     }
     double s = (p4[0] + p4[1]) + (p4[2] + p4[3]);
     s += __shfl_xor(s, 16);
@@ -247,7 +248,7 @@ __global__ __launch_bounds__(64 * QR_APPLY_WAVES) void qr_apply_kernel(QrApplyAr
     const int i = threadIdx.x >> 4, j = threadIdx.x & 15;
     double sum = 0.0;
 #pragma unroll
-    for (int k = 0; k < 16; k++) sum = fma(tm[i][k], wt[k][j], sum);
+    for (int k = 0; k < 16; k++) sum = tm[i][k] != 0.0 ? fma(tm[i][k], wt[k][j], sum) : sum;  // (no part in it: X may hold an infinity)
     w2[i][j] = sum;
   }
   __syncthreads();

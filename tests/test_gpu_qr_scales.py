@@ -1,4 +1,4 @@
-"""QR of columns whose squares or products leave float64's range."""
+"""QR of columns whose squares or products leave float64's range, and of triangular matrices with infinities."""
 
 import numpy as np
 import pytest
@@ -25,3 +25,11 @@ def test_columns_times_powers_of_two(hip, m, n):
         qs, rs = qr(hip, np.ldexp(a, e))
         assert np.array_equal(qs, q), powers
         assert np.array_equal(rs, np.ldexp(r, e)), powers
+
+
+@pytest.mark.parametrize("n", [7, 16, 40, 100])
+def test_a_triangular_matrix_with_infinities_comes_back(hip, n):
+    a = np.triu(np.random.default_rng(n).standard_normal((n, n)))
+    a[0, n - 1], a[2, 5], a[n // 2, n - 2] = np.inf, -np.inf, np.inf
+    q, r = qr(hip, a)
+    assert np.array_equal(q, np.eye(n)) and np.array_equal(r, a)
