@@ -5,10 +5,10 @@
 // in registers, one barrier a column. Everything else is two products per panel, V^T X and X - V W,
 // on the f64 matrix instruction over the whole device (compact WY: H_0 .. H_15 = I - V T V^T).
 // A launch per column and pass over the matrix, which this replaces, was bound by the launches, and a
-// workgroup per small matrix by its walks over memory: [796,796] float32 11.1 -> 2.05 ms, ten of [44,44]
-// float64 397 -> 74 us, a hundred of [100,100] 1407 -> 211. What bounds it now: the panels' chain (28 us for 512
-// rows of sixteen columns, 20 of them the columns) and two applications of 10 us per panel. |Q^T Q - I| and
-// |Q R - A| are 0.5 to 0.9 of what they were.
+// workgroup per small matrix by its walks over memory: [796,796] float64 11.3 -> 2.1 ms, [2048,2048] 55 -> 26.8, ten of
+// [44,44] 411 -> 106 us, a hundred of [100,100] 1 130 -> 208. What bounds it now: the panels' chain (28 us for 512
+// rows of sixteen columns, 20 of them the columns) and two applications of 10 us per panel. Root mean squares over
+// some hundred normal matrices of 8 to 2048 rows: |Q R - A| 0.62 to 1.00 of what it was, |Q^T Q - I| 0.65 to 1.04.
 #pragma once
 
 constexpr int QR_NB = 16;
@@ -275,6 +275,75 @@ __global__ __launch_bounds__(64 * QR_APPLY_WAVES) void qr_apply_kernel(QrApplyAr
   }
 }
 
+// The same reflector by reflector, X and V in registers as in qr_panel_kernel: a column's chain per panel where
+// the products with T take two passes, and as exact as a reflector at a time was for small matrices too.
+// The products round at the panel's size: |Q^T Q - I| of [16,16] 2.39e-15, so 1.69e-15 (before panels 1.74e-15);
+// [64,64] 5.6, 4.8 and 4.9; [96,96] 7.00, 6.82 and 6.91; from 100 columns on they are as exact ([100,100] 7.05 and
+// 7.12) and |Q R - A| is smaller. Time: [44,44] 85 -> 106 us, [96,96] 163 -> 226 (before panels 396 and 803).
+constexpr int QR_SINGLY = 96;         // columns up to which
+constexpr int QR_SINGLY_ROWS = 1024;  // the tallest panel of which both fit (taller: |Q^T Q - I| 0.4 to 4 % larger than before panels)
+template <class F, int... J>
+__device__ __forceinline__ void qr_each(F &&f, std::integer_sequence<int, J...>) {
+  (f(std::integral_constant<int, J>{}), ...);
+}
+template <int W, int E>
+__global__ __launch_bounds__(64 * W) void qr_reflect_kernel(QrApplyArgs a) {
+  __shared__ double part[2][W][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
+  const int rows = a.m - a.p0, w = min(QR_NB, a.k - a.p0);
+  const int col0 = a.first + (int)blockIdx.x * 16, cols = min(16, a.cols - col0);
+  const double *V = a.v + ((size_t)blockIdx.y * a.k + a.p0 + c) * a.m + a.p0;
+  double *X = a.x + ((size_t)blockIdx.y * a.cols + col0 + c) * a.m + a.p0;
+  const double *T = a.t + ((size_t)blockIdx.y * a.panels + a.p0 / QR_NB) * 256;
+  auto row_of = [&](int e) { return 4 * (e * W + wave) + q; };
+  constexpr int HEAD = W >= 4 ? 1 : 4 / W;
+  double x[E], v[E];
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    x[e] = c < cols && row_of(e) < rows ? X[row_of(e)] : 0.0;
+    v[e] = c < w && row_of(e) < rows ? V[row_of(e)] : 0.0;
+  }
+  const double taus = c < w ? T[c * 17] : 0.0;
+  int buf = 0;
+  auto reflect = [&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    const double tau = bcast16<j>(taus);
+    if (j >= w || tau == 0.0) return;  // (uniform)
+    double p4[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int e = 0; e < E; e++)  // (rows above the reflector have no part in it: they may hold an infinity)
+      p4[e & 3] = fma(bcast16<j>(v[e]), e < HEAD && row_of(e) < j ? 0.0 : x[e], p4[e & 3]);
+    double s = (p4[0] + p4[1]) + (p4[2] + p4[3]);
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    if constexpr (W > 1) {
+      if (q == 0) part[buf][wave][c] = s;
+      __syncthreads();
+      double p[W / 2];
+#pragma unroll
+      for (int i = 0; i < W / 2; i++) p[i] = part[buf][i][c] + part[buf][i + W / 2][c];
+#pragma unroll
+      for (int d = W / 4; d > 0; d /= 2)
+#pragma unroll
+        for (int i = 0; i < d; i++) p[i] += p[i + d];
+      s = p[0];
+      buf ^= 1;
+    }
+    const double wc = tau * s;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+      asm volatile("" : "+v"(v[e]));  // (broadcast again: kept, they would take the registers of x or v)
+      x[e] = fma(-bcast16<j>(v[e]), wc, x[e]);
+      asm volatile("" : "+v"(x[e]));
+    }
+  };
+  if (a.transpose) qr_each(reflect, std::make_integer_sequence<int, QR_NB>{});
+  else qr_each([&](auto jc) { reflect(std::integral_constant<int, QR_NB - 1 - decltype(jc)::value>{}); }, std::make_integer_sequence<int, QR_NB>{});
+#pragma unroll
+  for (int e = 0; e < E; e++)
+    if (c < cols && row_of(e) < rows) X[row_of(e)] = x[e];
+}
+
 // Q R of `batch` column-major matrices of at most QR_ROWS rows: R in At, Q's first nq columns in Qt.
 static int run_qr_blocked(nxh_context *ctx, const char *op, int64_t batch, int m, int n, int nq, double *At, double *Qt) {
   const int k = std::min(m, n), panels = (k + QR_NB - 1) / QR_NB;
@@ -289,8 +358,14 @@ static int run_qr_blocked(nxh_context *ctx, const char *op, int64_t batch, int m
       double *vb = (double *)v + b0 * k * m, *tb = (double *)t + b0 * panels * 256;
       auto apply = [&](int p0, double *x, int cols, int first, int transpose) {
         if (first >= cols) return;
-        QrApplyArgs a{vb, tb, x, m, k, p0, panels, cols, first, transpose};
-        hipLaunchKernelGGL(qr_apply_kernel, dim3((unsigned)((cols - first + 15) / 16), nb), dim3(64 * QR_APPLY_WAVES), 0, ctx->stream, a);
+        const QrApplyArgs a{vb, tb, x, m, k, p0, panels, cols, first, transpose};
+        const dim3 grid((unsigned)((cols - first + 15) / 16), nb);
+        const int rows = m - p0;
+        if (k > QR_SINGLY || m > QR_SINGLY_ROWS) hipLaunchKernelGGL(qr_apply_kernel, grid, dim3(64 * QR_APPLY_WAVES), 0, ctx->stream, a);
+        else if (rows <= 64) hipLaunchKernelGGL((qr_reflect_kernel<1, 16>), grid, dim3(64), 0, ctx->stream, a);
+        else if (rows <= 256) hipLaunchKernelGGL((qr_reflect_kernel<4, 16>), grid, dim3(256), 0, ctx->stream, a);
+        else if (rows <= 512) hipLaunchKernelGGL((qr_reflect_kernel<8, 16>), grid, dim3(512), 0, ctx->stream, a);
+        else hipLaunchKernelGGL((qr_reflect_kernel<8, 32>), grid, dim3(512), 0, ctx->stream, a);
       };
       for (int p0 = 0; p0 < k; p0 += QR_NB) {
         QrPanelArgs a{At + b0 * n * m, vb, tb, m, n, k, p0, panels};
