@@ -5,7 +5,7 @@
 // in registers, one barrier a column. Everything else is two products per panel, V^T X and X - V W,
 // on the f64 matrix instruction over the whole device (compact WY: H_0 .. H_15 = I - V T V^T).
 // A launch per column and pass over the matrix, which this replaces, was bound by the launches, and a
-// workgroup per small matrix by its walks over memory: [796,796] float64 11.3 -> 2.1 ms, [2048,2048] 55 -> 26.8, ten of
+// workgroup per small matrix by its walks over memory: [796,796] float64 11.3 -> 2.1 ms, [2048,2048] 55 -> 11.9, ten of
 // [44,44] 411 -> 106 us, a hundred of [100,100] 1 130 -> 208. What bounds it now: the panels' chain (28 us for 512
 // rows of sixteen columns, 20 of them the columns) and two applications of 10 us per panel. Root mean squares over
 // some hundred normal matrices of 8 to 2048 rows: |Q R - A| 0.62 to 1.00 of what it was, |Q^T Q - I| 0.65 to 1.04.
@@ -44,6 +44,9 @@ __global__ __launch_bounds__(64 * W) void qr_panel_kernel(QrPanelArgs a) {
   double *A = a.at + ((size_t)blockIdx.x * a.n + a.p0) * a.m + a.p0;
   auto row_of = [&](int e) { return 4 * (e * W + wave) + q; };
   constexpr int HEAD = W >= 4 ? 1 : 4 / W;  // elements that may lie in the first sixteen rows
+  // Sixteen waves leave a lane 128 registers, which x fills by half: there the reflector is broadcast again for the
+  // update instead of kept.
+  constexpr bool KEEP = W < 16;
   double x[E], biggest = 0.0;
 #pragma unroll
   for (int e = 0; e < E; e++) {
@@ -83,13 +86,18 @@ __global__ __launch_bounds__(64 * W) void qr_panel_kernel(QrPanelArgs a) {
     if (j >= w) return;
     constexpr int OWNER = W >= 4 ? j / 4 : 0, AT = W >= 4 ? 0 : j / 4;  // where row j is
     if (wave == OWNER && q == j % 4) rowj[buf][c] = x[AT];
-    double b[E], p4[4] = {0.0, 0.0, 0.0, 0.0};
+    // the reflector's element of a lane's row, unscaled, and zero above the row below the diagonal
+    auto reflector = [&](int e) {
+      const double v = bcast16<j>(x[e]);
+      return e < HEAD && row_of(e) <= j ? 0.0 : v;
+    };
+    double b[KEEP ? E : 1], p4[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int e = 0; e < E; e++) {
-      b[e] = bcast16<j>(x[e]);
-      if (e < HEAD) b[e] = row_of(e) > j ? b[e] : 0.0;
+      const double v = reflector(e);
+      if constexpr (KEEP) b[e] = v;
       // (rows that are done have no part in the sums: they may hold an infinity)
-      p4[e & 3] = fma(b[e], e < HEAD && row_of(e) <= j ? 0.0 : x[e], p4[e & 3]);
+      p4[e & 3] = fma(v, e < HEAD && row_of(e) <= j ? 0.0 : x[e], p4[e & 3]);
     }
     double s = (p4[0] + p4[1]) + (p4[2] + p4[3]);
     s += __shfl_xor(s, 16);
@@ -97,11 +105,14 @@ __global__ __launch_bounds__(64 * W) void qr_panel_kernel(QrPanelArgs a) {
     if constexpr (W > 1) {
       if (q == 0) part[buf][wave][c] = s;
       __syncthreads();
-      double p[W];
+      double p[W / 2];
 #pragma unroll
-      for (int i = 0; i < W; i++) p[i] = part[buf][i][c];
+      for (int i = 0; i < W / 2; i++) {
+        p[i] = part[buf][i][c] + part[buf][i + W / 2][c];
+        if (!KEEP && i % 2) __builtin_amdgcn_sched_barrier(0);  // (not all of them in registers at once)
+      }
 #pragma unroll
-      for (int d = W / 2; d > 0; d /= 2)
+      for (int d = W / 4; d > 0; d /= 2)
 #pragma unroll
         for (int i = 0; i < d; i++) p[i] += p[i + d];
       s = p[0];
@@ -118,9 +129,17 @@ __global__ __launch_bounds__(64 * W) void qr_panel_kernel(QrPanelArgs a) {
       const double wc = c > j ? tau * (divided(s, scal, rs) + r) : 0.0, wb = divided(wc, scal, rs);  // v . this lane's column, by tau
 #pragma unroll
       for (int e = 0; e < E; e++) {
-        x[e] = fma(-b[e], wb, x[e]);
+        double v;
+        if constexpr (KEEP) {
+          v = b[e];
+        } else {
+          asm volatile("" : "+v"(x[e]));  // (or the compiler keeps the first broadcast, in scratch memory)
+          v = reflector(e);
+        }
+        x[e] = fma(-v, wb, x[e]);
         if (e < HEAD) x[e] = row_of(e) == j ? x[e] - wc : x[e];
-      }
+        if constexpr (!KEEP) asm volatile("" : "+v"(x[e]));
+        }
       if (c == j) my_scal = scal, my_rs = rs, my_beta = beta, reflected = true;
     }
     if (threadIdx.x == 0) taus[j] = tau;
