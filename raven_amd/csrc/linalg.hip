@@ -1382,9 +1382,9 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
 template <class T>
 static int run_qr(nxh_context *ctx, const char *op, int64_t batch, int m, int n, int nq, T *At, T *Qt, T *tau) {
   std::lock_guard<std::mutex> g(ctx->mu);
-  if constexpr (std::is_same<T, double>::value)
+  if constexpr (std::is_same<T, double>::value) {
     if (m <= QR_ROWS) return run_qr_blocked(ctx, op, batch, m, n, nq, At, Qt);
-  if (std::max(m, n) < LA_WIDE_FROM) {
+  } else if (std::max(m, n) < LA_WIDE_FROM) {
     hipLaunchKernelGGL(qr_kernel<T>, dim3((unsigned)batch), dim3(LA_THREADS), 0, ctx->stream, At, Qt, tau, m, n, nq);
     NXH_HIP(op, hipGetLastError());
     return NXH_OK;
@@ -1586,13 +1586,14 @@ NXH_EXPORT int nxh_qr(nxh_context *ctx, const nxh_tensor *q, const nxh_tensor *r
   std::lock_guard<std::mutex> whole_call(ctx->call_mu);
   if ((rc = la_begin(ctx, op))) return rc;
   Work work(ctx);
-  void *At, *Qt, *tau;
+  const bool blocked = !p.cx && m <= QR_ROWS;
+  void *At, *Qt, *tau = nullptr;
   if ((rc = work.get((size_t)(p.batch * m * n) * p.esize, &At))) return rc;
   if ((rc = work.get((size_t)(p.batch * m * nq) * p.esize, &Qt))) return rc;
-  if ((rc = work.get((size_t)(p.batch * k) * p.esize, &tau))) return rc;
+  if (!blocked && (rc = work.get((size_t)(p.batch * k) * p.esize, &tau))) return rc;
   nxh_tensor wa = workspace_tensor(x, At, p.wdt, m, n, true);
   if (n > 0 && (rc = nxh_cast(ctx, &wa, x))) return rc;
-  PathAtExit path{!p.cx && m <= QR_ROWS ? "qr_blocked" : std::max(m, n) >= LA_WIDE_FROM ? "qr_householder_wide" : "qr_householder"};
+  PathAtExit path{blocked ? "qr_blocked" : std::max(m, n) >= LA_WIDE_FROM ? "qr_householder_wide" : "qr_householder"};
   rc = p.cx ? run_qr<c64>(ctx, op, p.batch, (int)m, (int)n, (int)nq, (c64 *)At, (c64 *)Qt, (c64 *)tau)
             : run_qr<double>(ctx, op, p.batch, (int)m, (int)n, (int)nq, (double *)At, (double *)Qt, (double *)tau);
   if (rc) return rc;
