@@ -84,8 +84,10 @@ static PyObject *raise_status(PyObject *ctx, int rc) {
   return NULL;
 }
 
+/* Handles are seen by the cycle collector: a tensor may be kept by its own context. They have nothing to clear; any
+   such cycle runs through a dict or the like that has. */
 static Buffer *buffer_wrap(PyObject *ctx, void *ptr, Py_ssize_t nbytes) {
-  Buffer *b = PyObject_New(Buffer, &BufferType);
+  Buffer *b = PyObject_GC_New(Buffer, &BufferType);
   if (!b) {
     nxh_context *h = ((Calls *)ctx)->h;
     if (h) L.free(h, ptr);
@@ -96,6 +98,7 @@ static Buffer *buffer_wrap(PyObject *ctx, void *ptr, Py_ssize_t nbytes) {
   b->ptr = ptr;
   b->nbytes = nbytes;
   b->weak = NULL;
+  PyObject_GC_Track(b);
   return b;
 }
 static PyObject *buffer_new(PyTypeObject *type, PyObject *args, PyObject *kw) {
@@ -112,7 +115,12 @@ static PyObject *buffer_new(PyTypeObject *type, PyObject *args, PyObject *kw) {
   if (rc) return raise_status(ctx, rc);
   return (PyObject *)buffer_wrap(ctx, p, nbytes);
 }
+static int buffer_traverse(Buffer *b, visitproc visit, void *arg) {
+  Py_VISIT(b->ctx);
+  return 0;
+}
 static void buffer_dealloc(Buffer *b) {
+  PyObject_GC_UnTrack(b);
   if (b->weak) PyObject_ClearWeakRefs((PyObject *)b);
   nxh_context *h = b->ctx ? ((Calls *)b->ctx)->h : NULL;
   if (h && b->ptr) {
@@ -122,7 +130,7 @@ static void buffer_dealloc(Buffer *b) {
     if (t) PyEval_RestoreThread(t);
   }
   Py_XDECREF(b->ctx);
-  PyObject_Free(b);
+  PyObject_GC_Del(b);
 }
 static PyObject *buffer_ptr(Buffer *b, void *u) {
   (void)u;
@@ -136,7 +144,8 @@ static PyGetSetDef buffer_getset[] = {{"ptr", (getter)buffer_ptr, NULL, NULL, NU
 static PyTypeObject BufferType = {
     PyVarObject_HEAD_INIT(NULL, 0).tp_name = "raven_amd._nxcalls.DeviceBuffer",
     .tp_basicsize = sizeof(Buffer),
-    .tp_flags = Py_TPFLAGS_DEFAULT,
+    .tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC,
+    .tp_traverse = (traverseproc)buffer_traverse,
     .tp_doc = "One device allocation, shared by every view of a tensor. Returned to the context's caching\n"
               "allocator when the last handle goes away (the OCaml binding does the same from a\n"
               "custom-block finaliser).",
@@ -154,7 +163,7 @@ typedef struct {
 } Tensor;
 
 static PyObject *tensor_make(PyObject *buffer, PyObject *view, PyObject *shape, PyObject *dtype, PyObject *context) {
-  Tensor *t = PyObject_New(Tensor, &TensorType);
+  Tensor *t = PyObject_GC_New(Tensor, &TensorType);
   if (!t) return NULL;
   Py_INCREF(buffer), Py_INCREF(view), Py_INCREF(shape), Py_INCREF(dtype), Py_INCREF(context);
   t->buffer = buffer;
@@ -163,6 +172,7 @@ static PyObject *tensor_make(PyObject *buffer, PyObject *view, PyObject *shape, 
   t->dtype = dtype;
   t->context = context;
   t->d = NULL;
+  PyObject_GC_Track(t);
   return (PyObject *)t;
 }
 static PyObject *tensor_new(PyTypeObject *type, PyObject *args, PyObject *kw) {
@@ -176,14 +186,24 @@ static PyObject *tensor_new(PyTypeObject *type, PyObject *args, PyObject *kw) {
   Py_DECREF(shape);
   return t;
 }
+static int tensor_traverse(Tensor *t, visitproc visit, void *arg) {
+  Py_VISIT(t->buffer);
+  Py_VISIT(t->view);
+  Py_VISIT(t->shape);
+  Py_VISIT(t->dtype);
+  Py_VISIT(t->context);
+  Py_VISIT(t->d);
+  return 0;
+}
 static void tensor_dealloc(Tensor *t) {
+  PyObject_GC_UnTrack(t);
   Py_XDECREF(t->buffer);
   Py_XDECREF(t->view);
   Py_XDECREF(t->shape);
   Py_XDECREF(t->dtype);
   Py_XDECREF(t->context);
   Py_XDECREF(t->d);
-  PyObject_Free(t);
+  PyObject_GC_Del(t);
 }
 
 /* The bytes of a view's descriptor (storage pointer and dtype tag zero), made once per view. */
@@ -299,7 +319,8 @@ static PyMethodDef tensor_methods[] = {
 static PyTypeObject TensorType = {
     PyVarObject_HEAD_INIT(NULL, 0).tp_name = "raven_amd._nxcalls.Tensor",
     .tp_basicsize = sizeof(Tensor),
-    .tp_flags = Py_TPFLAGS_DEFAULT,
+    .tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC,
+    .tp_traverse = (traverseproc)tensor_traverse,
     .tp_doc = "The backend's tensor handle (nx_backend.ml:36-43).",
     .tp_new = tensor_new,
     .tp_dealloc = (destructor)tensor_dealloc,
