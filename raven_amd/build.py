@@ -79,7 +79,7 @@ def build_all(force: bool = True, jobs: int | None = None) -> Path:
 
 
 CALLS_SRC = CSRC.parent / "host_c" / "nx_calls.c"
-CALLS_LIB = CSRC.parent / "_nxcalls.so"
+CALLS_LIB = CSRC.parent / ("_nxcalls" + sysconfig.get_config_var("EXT_SUFFIX"))  # found by this Python's ABI only
 
 
 def build_calls() -> Path:

@@ -27,7 +27,14 @@ import numpy as np
 
 from . import _ffi
 from . import dtype as dt
-from ._nxcalls import Calls, DeviceBuffer, Tensor, bind, setup  # host_c/nx_calls.c, built beside this file
+
+try:
+    from ._nxcalls import Calls, DeviceBuffer, Tensor, bind, setup  # host_c/nx_calls.c, built beside this file
+except ModuleNotFoundError as e:
+    if e.name != __package__ + "._nxcalls":
+        raise
+    raise ImportError("raven_amd._nxcalls is not built for this Python: build it with "
+                      "`python -c 'import __graft_entry__ as g; g.build()'`") from e
 from ._ffi import BINARY_OPS, COMPARE_OPS, REDUCE_OPS, UNARY_OPS, NxhTensor, stamp, view_image
 from .view import _CONTIGUOUS, View, numel
 

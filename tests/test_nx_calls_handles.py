@@ -3,9 +3,11 @@
 import gc
 import subprocess
 import sys
+import sysconfig
 import weakref
 from pathlib import Path
 
+from raven_amd import build
 from raven_amd import dtype as dt
 from raven_amd.nx_backend import Tensor
 from raven_amd.view import View
@@ -56,3 +58,17 @@ c.kept = Tensor(DeviceBuffer(c, 64), View.create((16,)), dt.float32, c)
 del c
 gc.collect()
 """) == ["freed", "77", "4096"]
+
+
+def test_the_module_is_this_pythons_and_its_absence_is_named():
+    assert build.CALLS_LIB.name.endswith(sysconfig.get_config_var("EXT_SUFFIX")) and build.CALLS_LIB.exists()
+    assert "cpython" in sys.modules["raven_amd._nxcalls"].__file__
+    out = in_a_process("""
+import sys
+sys.modules["raven_amd._nxcalls"] = None
+try:
+    import raven_amd.nx_backend
+except ImportError as e:
+    print("built" in str(e), "g.build()" in str(e))
+""")
+    assert out == ["True", "True"]
