@@ -1,5 +1,6 @@
 """The handles of the host path in C (raven_amd/host_c/nx_calls.c) as Python objects, and the module as a file."""
 
+import copy
 import gc
 import subprocess
 import sys
@@ -32,6 +33,13 @@ def test_a_tensor_kept_by_its_context_goes_with_it():
     del context
     gc.collect()
     assert ref() is None
+
+
+def test_a_handle_can_be_copied():
+    t = Tensor(Thing(), View.create((2, 3)), dt.float32, Thing())
+    u = copy.copy(t)
+    assert u is not t
+    assert all(getattr(u, name) is getattr(t, name) for name in ("buffer", "view", "shape", "dtype", "context"))
 
 
 def test_storage_kept_by_its_context_goes_back():
