@@ -102,7 +102,10 @@ class View:
             arg = tuple(arg)
         d = self.derived
         if d is not None:
-            v = d.get((movement, arg))
+            try:
+                v = d.get((movement, arg))
+            except TypeError:  # whole numbers that have no hash (arrays of rank 0)
+                v = None
             if v is not None:
                 return v
         v = make(self, arg)
