@@ -33,8 +33,6 @@ struct GemmArgs {
   BatchDims batch;
   uint32_t batch0;   // first batch index of this launch
   int a_vec, b_vec;  // 16-byte loads allowed (alignment + stride multiple)
-  // tiled kernels only: extents that may be loaded along M / N (a padded copy's row length)
-  int64_t m_ld, n_ld;
 };
 
 // The register-blocked kernel for the dtypes without a matrix-instruction path (gemm_block.hip):

@@ -28,7 +28,7 @@ int launch(nxh_context *ctx, Args &g) {
   NXH_HIP("matmul", attr_status);
   g.tiles_m = (uint32_t)((g.M + SH::BM - 1) / SH::BM);
   g.tiles_n = (uint32_t)((g.N + SH::BN - 1) / SH::BN);
-  nxh_set_path("gemm_tile_padded");
+  nxh_set_path("gemm_tile_padded");  // (K is padded in LDS)
   hipLaunchKernelGGL(kern, dim3(g.tiles_m * g.tiles_n * g.nbatch), dim3(SH::THREADS), LDS, ctx->stream, g);
   NXH_HIP("matmul", hipGetLastError());
   return NXH_OK;

@@ -988,10 +988,10 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
   // result; only the last columns of a single product (no batch) whose K is long enough are cut along it below.
   if constexpr (!EL::F32 && !EPI) {
     const int64_t n0 = a.N / 256 * 256;
-    if (a.N % 256 && n0 >= 8 * 256 && a.M % 256 == 0 && a.M >= 1024 && !forced_tile() && a.n_ld == a.N) {
+    if (a.N % 256 && n0 >= 8 * 256 && a.M % 256 == 0 && a.M >= 1024 && !forced_tile()) {
       GemmArgs left = a, right = a;
-      left.N = left.n_ld = n0;
-      right.N = right.n_ld = a.N - n0;
+      left.N = n0;
+      right.N = a.N - n0;
       right.B = (const char *)a.B + n0 * a.bcs * (int64_t)sizeof(typename EL::S);
       right.C = (char *)a.C + n0 * (int64_t)sizeof(typename EL::S);
       int rc = try_tile<EL, false>(ctx, left, nbatch, al_a, al_b, nullptr);
@@ -1013,12 +1013,10 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
   g.ldc = a.crs;
   if (!al16(g.A) || !al16(g.B) || g.lda % VE || g.ldb % VE) return -1;
   // an operand contiguous along M / N is read in whole 16-byte vectors
-  if ((!a_kc && a.m_ld % VE) || (!b_kc && a.n_ld % VE)) return -1;
+  if ((!a_kc && a.M % VE) || (!b_kc && a.N % VE)) return -1;
   g.M = a.M;
   g.N = a.N;
   g.K = a.K;
-  g.Mld = a.m_ld;
-  g.Nld = a.n_ld;
   g.nbatch = nbatch;
   g.nbd = a.batch.n;
   for (int i = 0; i < a.batch.n; i++) {
@@ -1389,7 +1387,6 @@ static int run_mfma_dtype(nxh_context *ctx, GemmArgs &a, uint32_t nbatch, bool b
   if (a.ccs != 1 && a.crs == 1 && a.N > 1) {
     std::swap(a.A, a.B);
     std::swap(a.M, a.N);
-    std::swap(a.m_ld, a.n_ld);
     std::swap(a.ars, a.bcs);
     std::swap(a.acs, a.brs);
     std::swap(a.crs, a.ccs);
@@ -1577,8 +1574,8 @@ static int matmul_entry(nxh_context *ctx, const char *op, const nxh_tensor *C, c
   g.A = (const char *)A->data + A->offset * es;
   g.B = (const char *)B->data + B->offset * es;
   g.C = (char *)C->data + C->offset * es;
-  g.M = g.m_ld = m;
-  g.N = g.n_ld = n;
+  g.M = m;
+  g.N = n;
   g.K = k;
   g.batch.n = nb;
   bool al_a = true, al_b = true;
