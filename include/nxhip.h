@@ -322,10 +322,9 @@ int nxh_attention(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *q,
    add of kaun/examples/04-gpt2/gpt2.ml:165-176, inside the GEMM's epilogue:
      out = (matmul x w + bias) + residual
    each of the three results rounded to the dtype as its primitive would store
-   it. The sums along K are those of nxh_matmul over a batch (x [b,m,k], b > 1) of the
-   same sizes, with which the value equals the op-by-op one of this library bit for bit; a
-   single product that nxh_matmul cuts along K, or streams past at most 16 rows, adds the same
-   terms in another order there. bias:
+   it, so the value equals the op-by-op one of this library bit for bit, but for products
+   that nxh_matmul has a kernel of its own for and sums in another order (a single one, without
+   a batch, that it cuts along K or streams past at most 16 rows; hundreds of tiny ones). bias:
    rank 1 of out's last extent, or NULL; residual: out's shape, or NULL (both
    NULL is nxh_matmul). f16 / bf16 / f32 operands that take the tiled MFMA GEMM
    (K a multiple of 128 bytes of k, 16-byte aligned rows, unit-stride output

@@ -351,7 +351,7 @@ static int run(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch) {
   // Tiles: as large as leaves enough waves. 32 x 32 reads half of what 16 x 16 reads, and from half a
   // tile per unit on sharing K among eight waves fills the chip; a chain of float32 steps is four times as long in a 32 x 32
   // tile, which pays from two tiles per unit on ([1554,244] x [244,347]: 9.0 us against 10.6, [500,500]^2: 13.2
-  // against 9.1). Blocks of 2 x 2 waves with 64 x 64 each only where their waves alone fill it ([2048,2048]^2 into
+  // against 9.8). Blocks of 2 x 2 waves with 64 x 64 each only where their waves alone fill it ([2048,2048]^2 into
   // every second column, float32: 170 us against 283 on 32 x 32; [501,501]^2: 41 against 10).
   const bool chain = EL::F32 && a.K <= MAX_CHAIN;
   const bool wide = chain ? count(32) >= 2.0 * cus && a.M > 16 && a.N > 16 : count(32) >= 0.5 * cus;

@@ -1070,7 +1070,8 @@ static int try_tile(nxh_context *ctx, const GemmArgs &a, uint32_t nbatch, bool a
     // Few result tiles under a long K: a strip of B a block (gemm_strip.hip). [48,768] x [768,768] bfloat16
     // 5.1 us against 7.3 as half blocks, [400,768] x [768,768] (84 tiles of 64 x 64) 6.0 against 7.6. Three
     // such layers over one input are one launch: from 3/8 of a tile per unit on their tiles outnumber the
-    // units and the kernels below are the faster ones ([1024,768] x 3 [768,768]: 16 us against 20). A single plain
+    // units and the kernels below are the faster ones ([1024,768] x 3 [768,768]: 16 us against 20); the line is
+    // the same for a layer by itself and for a plain product, whose bits a member of a group has. A single plain
     // product of a longer K is better off cut along it where the rule below cuts it ([512,3072] x [3072,768]: 14.0
     // against 15.0) unless the strips are cut too ([48,3072] x [3072,768]: 9.5 against 7.8). A batch, which is
     // not cut, and a fused linear, with the GELU or without, take the same kernel, so that they have the same bits.
@@ -1446,9 +1447,9 @@ static int run_mfma_dtype(nxh_context *ctx, GemmArgs &a, uint32_t nbatch, bool b
     }
     // Operands that do not fit it as they are: the ragged form of the same kernels for products of 2^27
     // terms or whose small blocks occupy the chip, the general kernel below that. float32 [16,200,200]
-    // x [16,200,201] (256 blocks of 64 x 64): 9.3 us against 14.2; [501,501]^2 (64 blocks): 13.9 against
-    // 7.9. bfloat16 [16,300,300]^2 (240 blocks of 128 x 64): 8.2 against 16.6; [501,501]^2 (32): 9.3
-    // against 6.7. A K of one slab is loads and stores, which the general kernel does not stage.
+    // x [16,200,201] (256 blocks of 64 x 64): 9.1 us against 9.7; [8,200,200] x [8,200,201] (128): 8.6 against 7.6;
+    // [501,501]^2 (64): 13.4 against 9.8. bfloat16 [16,300,300]^2 (240 blocks of 128 x 64): 8.2 against 16.6; [501,501]^2 (32):
+    // 9.3 against 6.7. A K of one slab is loads and stores, which the general kernel does not stage.
     const int64_t bm = sizeof(S) == 4 ? 64 : 128;
     const double blocks = (double)((a.M + bm - 1) / bm) * (double)((a.N + 63) / 64) * nbatch;
     if constexpr (MM::DT == NXH_F32) {
