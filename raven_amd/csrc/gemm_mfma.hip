@@ -236,14 +236,14 @@ __global__ __launch_bounds__(64 * MAXW) void kernel(GemmArgs a, uint32_t tiles_m
 // A float32 tile of 16 x 16 whose K is one chain, where there are at most two tiles to a unit: the chain is
 // one wave's (54 ns a step of 16 k-values), and what that wave can have in flight by itself does not feed it.
 // All CW waves of the block fetch CS steps each into LDS, in the order in which the instruction takes
-// them, while the round before is summed ([38,1754] x [1754,86]: 12.8 us, a wave by itself 19.4; [32,784] x
+// them, while the stage before is summed ([38,1754] x [1754,86]: 12.8 us, a wave by itself 19.4; [32,784] x
 // [784,128]: 7.5 and 10.1; K in eight sums, which is not the same result, 7.4 and 5.2).
 constexpr int CW = 8;
 template <bool A_KC, bool B_KC, int CS>
 __global__ __launch_bounds__(64 * CW) void chain_kernel(GemmArgs a, uint32_t tiles_m, uint32_t tiles_n) {
   using TT = Tile<ElF32, 16>;
-  constexpr int KS = TT::KS, ROUND = CW * CS;
-  extern __shared__ __attribute__((aligned(16))) f32x4 stage[];  // [2][ROUND][A, B][64]
+  constexpr int KS = TT::KS, PER_STAGE = CW * CS;
+  extern __shared__ __attribute__((aligned(16))) f32x4 stage[];  // [2][PER_STAGE][A, B][64]
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t per = tiles_m * tiles_n, b = blockIdx.x / per, r = blockIdx.x - b * per;
@@ -273,19 +273,19 @@ __global__ __launch_bounds__(64 * CW) void chain_kernel(GemmArgs a, uint32_t til
   };
   f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
   fetch(0);
-  for (int first = 0, at = 0; first < steps; first += ROUND, at ^= ROUND) {
+  for (int first = 0, at = 0; first < steps; first += PER_STAGE, at ^= PER_STAGE) {
     f32x4 *mine = stage + (at + wave * CS) * 128 + lane;
 #pragma unroll
     for (int u = 0; u < CS; u++) {
       mine[u * 128] = TT::ordered(fa[u]);
       mine[u * 128 + 64] = TT::ordered(fb[u]);
     }
-    fetch(first + ROUND);
-    // (also: wave 0 is through with the stage that the next round is written to)
+    fetch(first + PER_STAGE);
+    // (also: wave 0 is through with the stage that is written next)
     __syncthreads();
     if (wave == 0) {
       const f32x4 *p = stage + at * 128 + lane;
-      const int n = steps - first < ROUND ? steps - first : ROUND;
+      const int n = steps - first < PER_STAGE ? steps - first : PER_STAGE;
       // (four steps' operands are on their way while the four before are summed; past n: the stage's own memory)
       constexpr int AHEAD = CS > 2 ? 4 : 2;
       f32x4 x[2][AHEAD], y[2][AHEAD];
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(64 * CW) void chain_kernel(GemmArgs a, uint32_t til
       for (int s = 0; s < n; s += 2 * AHEAD) {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-          if (s + (h + 1) * AHEAD < ROUND) take(h ^ 1, s + (h + 1) * AHEAD);
+          if (s + (h + 1) * AHEAD < PER_STAGE) take(h ^ 1, s + (h + 1) * AHEAD);
 #pragma unroll
           for (int j = 0; j < AHEAD; j++)
             if (s + h * AHEAD + j < n) TT::mac_ordered(acc, x[h][j], y[h][j]);

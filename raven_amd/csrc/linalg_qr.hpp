@@ -8,7 +8,7 @@
 // workgroup per small matrix by its walks over memory: [796,796] float64 11.3 -> 2.1 ms, [2048,2048] 55 -> 11.9, ten of
 // [44,44] 411 -> 106 us, a hundred of [100,100] 1 130 -> 208. What bounds it now: the panels' chain (28 us for 512
 // rows of sixteen columns, 20 of them the columns) and two applications of 10 us per panel. Root mean squares over
-// some hundred normal matrices of 8 to 2048 rows: |Q R - A| 0.62 to 1.00 of what it was, |Q^T Q - I| 0.65 to 1.04.
+// some hundred normal matrices of 8 to 2048 rows: |Q R - A| 0.62 to 1.00 of what it was, |Q^T Q - I| 0.64 to 1.04.
 #pragma once
 
 constexpr int QR_NB = 16;
