@@ -14,8 +14,9 @@
    - strides and offset are in ELEMENTS and may be zero (broadcast) or negative
      (flip) on inputs; rank <= NXH_MAX_NDIM (nx_c.h:45-61).
    - dtype tags equal Nx's Dtype.Packed.tag (nx_c.h:130-200).
-   - every call is asynchronous on the context's stream; nxh_memcpy_d2h,
-     nxh_gather, nxh_scatter and nxh_synchronize wait for it.
+   - every call is asynchronous on the context's stream; nxh_memcpy_d2h and
+     nxh_synchronize wait for it, nxh_gather and nxh_scatter until their indices
+     have been looked through (their result is in stream order, as any other's).
    - return value: NXH_OK, NXH_INVALID_ARGUMENT (the reference raises
      Invalid_argument) or NXH_FAILURE (the reference raises Failure); the
      message, prefixed "<op>: " like the reference's, is read with
@@ -201,16 +202,16 @@ int nxh_matmul(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *a,
 
 /* caml_nx_c_copy (nx_c_move.c:191-201): copy / contiguous / assign. */
 int nxh_copy(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *x);
-/* caml_nx_c_gather (nx_c_move.c:342-458). Waits for the stream so that an
-   out-of-bounds index is reported by this call, as in the reference. */
+/* caml_nx_c_gather (nx_c_move.c:342-458). Waits until the device has looked through
+   the indices, so that one out of bounds is reported by this call, as in the reference. */
 int nxh_gather(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *data,
                const nxh_tensor *indices, int axis);
 
 /* caml_nx_c_scatter (nx_c_move.c:460-586): `out` already holds the template (the
    binding copies it first, nx_backend.ml:412-416). mode 0 = Set (the last update
    in row-major order of the index space wins), 1 = Add (accumulates in that
-   order, in the dtype's compute type). Deterministic. Waits for the stream so
-   that an out-of-bounds index is reported by this call. */
+   order, in the dtype's compute type). Deterministic. Waits until the device has
+   looked through the indices, so that one out of bounds is reported by this call. */
 int nxh_scatter(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *indices,
                 const nxh_tensor *updates, int axis, int mode);
 /* nxh_copy of `from` into `out`, then nxh_scatter (nx_backend.ml:412-416): in one pass

@@ -42,7 +42,8 @@ struct nxh_context {
   uint64_t in_use = 0, cached = 0, reserved = 0, driver_allocs = 0;
   // one device word, written by kernels that detect a data fault (gather OOB)
   int *fault_flag = nullptr;       // device words of the factorisations
-  int *fault_flag_host = nullptr;  // pinned host words: [0] is raised by gather and scatter, the rest mirror the device's
+  int *fault_flag_host = nullptr;  // pinned host words: [0] is raised by recorded gathers and scatters, [1], [2] mirror the device's
+  uint32_t report_seq = 0;         // the last report that was asked for (nxh_report_word)
   // pinned staging slots for small host-to-device uploads: the caller's bytes
   // are copied into a slot and the transfer is queued on the stream, so an
   // upload does not wait for the work already queued
@@ -157,8 +158,23 @@ uint32_t nxh_cache_hints(nxh_context *ctx, int nop, const void *const *base, con
 void nxh_cache_touch(nxh_context *ctx, const nxh_tensor *const *tensors, int n, int n_out);
 // An entry point that may touch blocks it does not name. Takes ctx->mu.
 void nxh_cache_opaque(nxh_context *ctx);
-// the out-of-bounds flag of gather / scatter, read back (or left for the replay) (runtime.hip)
-int nxh_collect_index_fault(nxh_context *ctx, const char *op);
+// How a call learns what its kernels found without waiting for all they do: a kernel stores (number of the
+// report << 8 | code) to a word of pinned memory in ONE store, so nothing is cleared and nothing is ordered against
+// it, and the host looks at the word. 7.2 us from a launch to the answer, 12.0 with hipStreamSynchronize; a kernel that
+// stores early lets its caller go on while it works. NXH_REPORT_INDEX (gather, scatter) belongs to whoever holds ctx->mu,
+// NXH_REPORT_LINALG to whoever holds ctx->call_mu.
+enum { NXH_REPORT_INDEX = 0, NXH_REPORT_LINALG = 1 };
+static inline uint64_t *nxh_report_word(nxh_context *ctx, int which) { return (uint64_t *)ctx->fault_flag_host + 8 * (1 + which); }
+// The number of a new report, never 0. Caller holds ctx->mu.
+static inline uint32_t nxh_next_report(nxh_context *ctx) { return ++ctx->report_seq ? ctx->report_seq : ++ctx->report_seq; }
+// Waits until report `seq` is in `which` (or the stream has run out of work) and reads its code.
+int nxh_await_report(nxh_context *ctx, const char *op, int which, uint32_t seq, int *code);
+// Queues report `seq`, made once the work before it has run: code 1 if *found (device memory) is seq, else 0.
+void nxh_queue_report(nxh_context *ctx, int which, uint32_t seq, const int *found);
+// The report of a gather or scatter as the call's failure (recorded into a graph: left for the replay). Its kernels raise
+// the word nxh_index_found to the report's number, in a graph the host's flag.
+int nxh_collect_index_report(nxh_context *ctx, const char *op, uint32_t seq);
+static inline int *nxh_index_found(nxh_context *ctx) { return ctx->fault_flag + 4; }
 // Before an eager gather / scatter is launched: a fault that a replayed graph left in
 // the flag is reported now, as the replay's, so that this call answers only for itself.
 int nxh_settle_replay_faults(nxh_context *ctx, const char *op);
@@ -256,6 +272,10 @@ static inline int nxh_check_tensor(const char *op, const nxh_tensor *t) {
 }
 
 // ─────────────────────────── device scalar types ────────────────────────────
+
+__device__ __forceinline__ void nxh_report(uint64_t *word, uint32_t seq, int code) {
+  __hip_atomic_store(word, (uint64_t)seq << 8 | (uint64_t)code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 enum Cat { CAT_SINT, CAT_UINT, CAT_FLOAT, CAT_COMPLEX, CAT_BOOL };
 

@@ -8,6 +8,7 @@
 // orders all work, and blocks returned to the allocator are reused only by
 // later work on that same stream.
 
+#include <chrono>
 #include <cstdlib>
 
 #include "nxh_common.hpp"
@@ -466,11 +467,9 @@ NXH_EXPORT int nxh_memcpy_h2d(nxh_context *ctx, void *dst, const void *src, size
   return NXH_OK;
 }
 
-// Looks at the out-of-bounds flag after a gather or scatter launch: the failure is reported by
-// the call that caused it (nx_c_move.c:448-458, 571-586). The flag is a word of pinned host memory that
-// a kernel stores to when it meets such an index, so there is nothing to copy back (a copy kernel
-// and its launch were 8 of a gather's 25 us). A stream that is being recorded cannot be waited
-// for: there the flag stays up and the next synchronize after a replay reports it.
+// The out-of-bounds flag that the kernels of a replayed graph raise: a word of pinned host memory.
+// A stream that is being recorded cannot be waited for, so there the flag stays up and the next
+// synchronize after a replay reports it.
 static int read_fault_flag(nxh_context *ctx, const char *op, const char *message) {
   NXH_HIP(op, hipStreamSynchronize(ctx->stream));
   volatile int *flag = ctx->fault_flag_host;
@@ -479,12 +478,40 @@ static int read_fault_flag(nxh_context *ctx, const char *op, const char *message
   return nxh_fail(NXH_FAILURE, op, message);
 }
 
-int nxh_collect_index_fault(nxh_context *ctx, const char *op) {
+__global__ void report_kernel(uint64_t *word, uint32_t seq, const int *found) {
+  nxh_report(word, seq, *found == (int)seq);
+}
+void nxh_queue_report(nxh_context *ctx, int which, uint32_t seq, const int *found) {
+  hipLaunchKernelGGL(report_kernel, dim3(1), dim3(1), 0, ctx->stream, nxh_report_word(ctx, which), seq, found);
+}
+
+int nxh_await_report(nxh_context *ctx, const char *op, int which, uint32_t seq, int *code) {
+  const uint64_t *word = nxh_report_word(ctx, which);
+  const auto there = [&] {
+    const uint64_t v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+    *code = (int)(v & 0xff);
+    return v >> 8 == seq;
+  };
+  // two milliseconds of looking; behind more work than that, or where the device has failed, the stream's own wait
+  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+  do {
+    for (int i = 0; i < 64; i++) {
+      if (there()) return NXH_OK;
+      __builtin_ia32_pause();
+    }
+  } while (std::chrono::steady_clock::now() < until);
+  NXH_HIP(op, hipStreamSynchronize(ctx->stream));
+  return there() ? NXH_OK : nxh_fail(NXH_FAILURE, op, "the device did not report");
+}
+
+int nxh_collect_index_report(nxh_context *ctx, const char *op, uint32_t seq) {
   if (ctx->capture) {
     ctx->capture->has_index_checks = true;
     return NXH_OK;
   }
-  return read_fault_flag(ctx, op, NXH_ERR_INDEX_OOB);
+  int code = 0;
+  if (int rc = nxh_await_report(ctx, op, NXH_REPORT_INDEX, seq, &code)) return rc;
+  return code ? nxh_fail(NXH_FAILURE, op, NXH_ERR_INDEX_OOB) : NXH_OK;
 }
 
 static int report_deferred_faults(nxh_context *ctx, const char *op) {

@@ -320,7 +320,7 @@ CAMLprim value caml_nx_hip_gather(value vout, value vdata, value vidx, value vax
   nxh_context *c = extract(vout, &o);
   extract(vdata, &d);
   extract(vidx, &i);
-  /* waits for the stream to report an out-of-range index from this call */
+  /* waits for the look through the indices, so that one out of range is reported by this call */
   caml_enter_blocking_section();
   int rc = L.gather(c, &o, &d, &i, Int_val(vaxis));
   caml_leave_blocking_section();
@@ -333,7 +333,7 @@ CAMLprim value caml_nx_hip_scatter(value vout, value vidx, value vupd, value vax
   nxh_context *c = extract(vout, &o);
   extract(vidx, &i);
   extract(vupd, &u);
-  /* waits for the stream to report an out-of-range index from this call */
+  /* waits for the look through the indices, so that one out of range is reported by this call */
   caml_enter_blocking_section();
   int rc = L.scatter(c, &o, &i, &u, Int_val(vaxis), Int_val(vmode));
   caml_leave_blocking_section();
