@@ -287,8 +287,9 @@ struct ScatterArgs {
   int64_t cshape[NXH_MAX_NDIM];
   int64_t c_ostride[NXH_MAX_NDIM], c_istride[NXH_MAX_NDIM], c_ustride[NXH_MAX_NDIM];
   int64_t a_ostride, a_istride, a_ustride;  // along the scatter axis
-  const char *from;  // scatter_rows: what `out` starts as, laid out as it is (null: out already holds it)
+  const char *from;  // scatter_rows, scatter_copy: what `out` starts as, laid out as it is (null: out already holds it)
   IndexFault fault;
+  IndexReport report;  // scatter_copy
 };
 // ADD: accumulate in the dtype's compute type; otherwise a byte-exact store.
 template <int DT, bool ADD>
@@ -523,6 +524,178 @@ __global__ __launch_bounds__(256) void scatter_rows_kernel(ScatterArgs a, int64_
     }
   }
 }
+constexpr int SCATTER_RANGE = 1024;  // rows of a block's range, at most
+// out = a copy of `from`, then whole rows of updates, in one pass over the table. `out` and `from` are dense, one row
+// of `row` elements after another, and start on 16 bytes, as do the blocks' ranges of `range_rows` rows. A block looks
+// through all indices for those of its range (sixteen loads of a lane in flight, out of L2) and puts them in the order
+// of (row, position) by counting the smaller ones. Where rows are whole vectors (V > 1) the copy adds on the way: a
+// vector's first update is requested with the vector itself, and nothing but the vector is written. Ragged rows are
+// copied 16 bytes at a time whatever rows they belong to, and updated after it, a wave to 64 elements of a row; so are
+// blocks with more than LIST updates, in spans of LIST positions. Either way an element's updates come in the order of
+// their positions, each rounded to the storage type. Bound by the copy, which streaming stores decide (`stream`): [50257,
+// 768] f32 with 8 192 updates from the cache 47 us, with plain stores 67 (a copy alone 39); with updates from memory 66,
+// where a copy and scatter_rows take 43 and 33, and scatter_rows with `from`, whose lanes own columns and copy one row
+// after another, some 150.
+template <int DT, bool ADD, int V>
+__global__ __launch_bounds__(256) void scatter_copy_kernel(ScatterArgs a, int64_t range_rows, int64_t row, uint32_t by_wide, int stream) {
+  using TR = Tr<DT>;
+  using E = typename TR::S;
+  using C = typename TR::C;
+  struct alignas(V > 1 ? 16 : alignof(E)) S {
+    E v[V];
+  };
+  constexpr int LIST = 1024, LOOK = 16, EACH = 4, B = 4;
+  __shared__ uint64_t list[LIST];         // (row of the range << 32 | position), in any order
+  __shared__ uint32_t position[LIST];     // in the order of (row, position)
+  __shared__ uint16_t start[SCATTER_RANGE], count[SCATTER_RANGE], updated[LIST];  // of a row; the rows that have updates
+  __shared__ int s_total, s_rows;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t lo = (int64_t)blockIdx.x * range_rows, hi = lo + range_rows < a.axis_len ? lo + range_rows : a.axis_len;
+  // The updates at positions from `begin` to `end` whose row is in the range; their number (more than LIST: not kept).
+  auto collect = [&](int64_t begin, int64_t end, bool *bad) {
+    __syncthreads();
+    if (threadIdx.x == 0) s_total = s_rows = 0;
+    __syncthreads();
+    for (int64_t i0 = begin + threadIdx.x; i0 < end; i0 += 256 * LOOK) {
+      int64_t t[LOOK];
+#pragma unroll
+      for (int j = 0; j < LOOK; j++) t[j] = a.idx[(i0 + j * 256 < end ? i0 + j * 256 : i0) * a.a_istride];
+#pragma unroll
+      for (int j = 0; j < LOOK; j++) {
+        if (t[j] < 0) t[j] += a.axis_len;
+        *bad |= t[j] < 0 || t[j] >= a.axis_len;
+        if (t[j] >= lo && t[j] < hi && i0 + j * 256 < end) {
+          const int at = atomicAdd(&s_total, 1);
+          if (at < LIST) list[at] = (uint64_t)(t[j] - lo) << 32 | (uint64_t)(i0 + j * 256);
+        }
+      }
+    }
+    *bad = __syncthreads_or(*bad);
+    return s_total;
+  };
+  auto order = [&](int n) {
+    for (int r = threadIdx.x; r < range_rows; r += 256) count[r] = 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += 256) {
+      const uint64_t own = list[i];
+      int rank = 0, first = 0, last = 0;  // all are different
+      for (int k = 0; k < n; k++) {
+        rank += list[k] < own;
+        first += list[k] >> 32 < own >> 32;
+        last += list[k] >> 32 <= own >> 32;
+      }
+      position[rank] = (uint32_t)own;
+      if (rank > first) continue;
+      start[own >> 32] = (uint16_t)first;
+      count[own >> 32] = (uint16_t)(last - first);
+      updated[atomicAdd(&s_rows, 1)] = (uint16_t)(own >> 32);
+    }
+    __syncthreads();
+  };
+  auto combine = [](S cur, S u) -> S {
+    if constexpr (ADD) {
+      S r;
+#pragma unroll
+      for (int e = 0; e < V; e++) {
+        const C x = TR::ld(cur.v[e]), y = TR::ld(u.v[e]);
+        if constexpr (TR::cat == CAT_SINT) r.v[e] = TR::st((C)((uint64_t)x + (uint64_t)y));
+        else r.v[e] = TR::st((C)(x + y));
+      }
+      return r;
+    } else {
+      return u;
+    }
+  };
+  auto put = [&](G16 *p, G16 x) {
+    typedef uint64_t pair __attribute__((ext_vector_type(2)));
+    if (stream) __builtin_nontemporal_store(pair{x.lo, x.hi}, reinterpret_cast<pair *>(p));
+    else *p = x;
+  };
+  bool bad = false;
+  const int total = collect(0, a.n_idx, &bad);
+  if (a.report.word && blockIdx.x == 0 && threadIdx.x == 0) nxh_report(a.report.word, a.report.seq, bad);
+  if (bad) return;
+  const int64_t base = lo * row * (int64_t)sizeof(E), bytes = (hi - lo) * row * (int64_t)sizeof(E), whole = bytes / 16, wide = row / V;
+  const int64_t a_us = a.a_ustride / V;
+  const G16 *from = reinterpret_cast<const G16 *>(a.from + base);
+  G16 *out = reinterpret_cast<G16 *>(a.out + base);
+  if constexpr (V > 1) {
+    if (total <= LIST) {
+      order(total);
+      const S *upd = reinterpret_cast<const S *>(a.upd);
+      for (int64_t i0 = threadIdx.x; i0 < whole; i0 += 256 * EACH) {
+        S x[EACH], u[EACH];
+        int n[EACH], at[EACH];
+        int64_t col[EACH];
+#pragma unroll
+        for (int j = 0; j < EACH; j++) {
+          const int64_t i = i0 + 256 * j < whole ? i0 + 256 * j : i0;
+          const uint32_t r = __umulhi(2u * (uint32_t)i, by_wide);  // i / wide (one row: 0)
+          n[j] = count[r];
+          at[j] = start[r];
+          col[j] = i - r * wide;
+          x[j] = reinterpret_cast<const S *>(from)[i];
+          if (n[j]) u[j] = upd[(int64_t)position[at[j]] * a_us + col[j]];
+        }
+#pragma unroll
+        for (int j = 0; j < EACH; j++) {
+          if (n[j]) {
+            x[j] = combine(x[j], u[j]);
+            for (int k = 1; k < n[j]; k++) x[j] = combine(x[j], upd[(int64_t)position[at[j] + k] * a_us + col[j]]);
+          }
+          if (i0 + 256 * j < whole) put(out + i0 + 256 * j, __builtin_bit_cast(G16, x[j]));
+        }
+      }
+      return;
+    }
+  }
+  for (int64_t i0 = threadIdx.x; i0 < whole; i0 += 256 * EACH) {
+    G16 x[EACH];
+#pragma unroll
+    for (int j = 0; j < EACH; j++) x[j] = from[i0 + 256 * j < whole ? i0 + 256 * j : i0];
+#pragma unroll
+    for (int j = 0; j < EACH; j++)
+      if (i0 + 256 * j < whole) put(out + i0 + 256 * j, x[j]);
+  }
+  if (threadIdx.x < bytes % 16) a.out[base + whole * 16 + threadIdx.x] = a.from[base + whole * 16 + threadIdx.x];
+  if (total == 0) return;
+  const int64_t span = total <= LIST ? a.n_idx : LIST;
+  const int chunks = (int)((wide + 63) / 64);
+  for (int64_t begin = 0; begin < a.n_idx; begin += span) {
+    if (total > LIST) (void)collect(begin, begin + span < a.n_idx ? begin + span : a.n_idx, &bad);
+    order(s_total);  // (its barriers: what this block's lanes stored so far is seen by its other lanes)
+    for (int64_t item = wave; item < (int64_t)s_rows * chunks; item += 4) {
+      const int r = updated[item / chunks];
+      const int64_t c = item % chunks * 64 + lane;
+      if (c >= wide) continue;
+      S *o = reinterpret_cast<S *>(reinterpret_cast<E *>(a.out) + (lo + r) * row) + c;
+      const S *upd = reinterpret_cast<const S *>(a.upd) + c;
+      S acc = *o;
+      for (int i = start[r], end = i + count[r]; i < end; i += B) {
+        S u[B];
+#pragma unroll
+        for (int j = 0; j < B; j++) u[j] = upd[(int64_t)position[i + j < end ? i + j : i] * a_us];
+#pragma unroll
+        for (int j = 0; j < B; j++)
+          if (i + j < end) acc = combine(acc, u[j]);
+      }
+      *o = acc;
+    }
+  }
+}
+typedef void (*scatter_copy_fn)(nxh_context *, const ScatterArgs &, bool, int64_t, int64_t, bool);
+template <int DT>
+static void scatter_copy_launch(nxh_context *ctx, const ScatterArgs &a, bool add, int64_t range, int64_t row, bool vec) {
+  constexpr int V = 16 / (int)sizeof(typename Tr<DT>::S);
+  const auto kern = vec ? (add ? scatter_copy_kernel<DT, true, V> : scatter_copy_kernel<DT, false, V>)
+                        : (add ? scatter_copy_kernel<DT, true, 1> : scatter_copy_kernel<DT, false, 1>);
+  const int64_t bytes = a.axis_len * row * (int64_t)sizeof(typename Tr<DT>::S), wide = row / V;
+  // i / wide = i by_wide >> 31 of i < range wide < 2^16, since i wide < 2^31 where there is more than one row; 0: one row
+  const uint32_t by_wide = vec && range > 1 ? (uint32_t)(((uint64_t)1 << 31) / (uint64_t)wide) + 1 : 0;
+  // a table that the L2s hold is left there for whoever reads it next
+  const int stream = bytes > (32 << 20);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((a.axis_len + range - 1) / range)), dim3(256), 0, ctx->stream, a, range, row, by_wide, stream);
+}
 typedef void (*scatter_launch_fn)(nxh_context *, const ScatterArgs &, bool, int64_t, bool);
 // range_rows > 0 selects the kernel that also splits the targets into ranges; `vec` its form
 // with 16 bytes of columns per lane (a.columns then counts lanes).
@@ -726,10 +899,12 @@ static int scatter_impl(nxh_context *ctx, const nxh_tensor *out, const nxh_tenso
   a.a_ostride = out->strides[axis];
   a.a_istride = indices->strides[axis];
   a.a_ustride = updates->strides[axis];
+  a.report = {nullptr, 0};
   struct Table {
     scatter_launch_fn fn[NXH_DTYPE_COUNT] = {};
+    scatter_copy_fn copy[NXH_DTYPE_COUNT] = {};
     Table() {
-#define NXH_SC(DT) fn[DT] = &scatter_launch<DT>;
+#define NXH_SC(DT) fn[DT] = &scatter_launch<DT>, copy[DT] = &scatter_copy_launch<DT>;
       NXH_FOR_COMPUTE_DTYPES(NXH_SC)
 #undef NXH_SC
     }
@@ -747,6 +922,39 @@ static int scatter_impl(nxh_context *ctx, const nxh_tensor *out, const nxh_tenso
   bool uniform_index = a.axis_len <= 0x7fffffffLL;
   for (int d = 0; d < a.ncol_dims; d++)
     if (a.cshape[d] > 1 && a.c_istride[d] != 0) uniform_index = false;
+  if (from && uniform_index && !ctx->capture) {
+    // One pass over a dense table of rows (axis 0, or what is like it). A block's range is 48 KiB, or 6 bytes an index,
+    // so that what it reads of the indices (out of L2) stays below what it copies; smaller where the table has too
+    // few such ranges for the chip, down to 4 KiB.
+    const int64_t line = a.columns * es, bytes = a.axis_len * line;
+    int64_t run = 1;
+    bool rows = a.a_ostride == a.columns || a.axis_len == 1;
+    for (int d = a.ncol_dims - 1; d >= 0; d--) {
+      if (a.cshape[d] > 1 && (a.c_ostride[d] != run || a.c_ustride[d] != run)) rows = false;
+      run *= a.cshape[d];
+    }
+    const bool rows16 = es < 16 && line % 16 == 0 && a.a_ustride * es % 16 == 0 && (uintptr_t)a.upd % 16 == 0;
+    int64_t range = std::min(std::max<int64_t>(48 << 10, a.n_idx * 6), std::max<int64_t>(4 << 10, bytes / (2 * ctx->compute_units)));
+    range = std::min<int64_t>(SCATTER_RANGE, std::max<int64_t>(1, range / line));
+    if (rows16) {
+      if (range * (line / 16) >= 1 << 16) range = std::max<int64_t>(1, 65535 / (line / 16));
+    } else {
+      range = (range + 15) / 16 * 16;  // whole vectors, whatever the row
+    }
+    if (rows && ((uintptr_t)a.out | (uintptr_t)a.from) % 16 == 0 && a.n_idx <= 4 * a.axis_len && a.n_idx <= 0x7fffffff) {
+      std::lock_guard<std::mutex> guard(ctx->mu);
+      if (ctx->capture) return -1;
+      NXH_HIP(op, hipSetDevice(ctx->device));
+      if (int frc = nxh_settle_replay_faults(ctx, op)) return frc;
+      const uint32_t seq = nxh_next_report(ctx);
+      a.fault = {nullptr, 0};
+      a.report = {nxh_report_word(ctx, NXH_REPORT_INDEX), seq};
+      nxh_set_path("scatter_copy");
+      table_.copy[dt](ctx, a, mode == 1, range, a.columns, rows16);
+      NXH_HIP(op, hipGetLastError());
+      return nxh_collect_index_report(ctx, op, seq);
+    }
+  }
   // 16 bytes of columns per lane: the off-axis dims of `out` and `updates` are one contiguous
   // run, a whole number of vectors long, and every row of both starts on a 16-byte boundary
   // (embedding gradient [8192, 768] f32 into [50257, 768]: 38 -> 33 us)
@@ -766,9 +974,9 @@ static int scatter_impl(nxh_context *ctx, const nxh_tensor *out, const nxh_tenso
     if (ranges > 65535) ranges = 65535;
     if (ranges >= 2) range_rows = (a.axis_len + ranges - 1) / ranges;
   }
-  // One pass pays while a launch and its gap are a share of the call: a table of 64 MiB at most
-  // ([34828,369] float32 with 195 updates, with the gather before it: 102 -> 77 us; [50257,768], 154 MB: the
-  // blocks copy and update in step, 191 us against 145 for two launches).
+  // What scatter_copy does not take (columns that are no contiguous run, rows that start off 16 bytes). One pass in
+  // this kernel pays while a launch and its gap are a share of the call, for a table of 64 MiB at most ([34828,369]
+  // float32 with 195 updates: 102 -> 77 us; 154 MB: the blocks copy and update in step, 191 us against 145 for two launches).
   if (from && (range_rows == 0 || a.n_idx > 4 * a.axis_len || a.axis_len * a.columns * es > (64 << 20))) return -1;
   std::lock_guard<std::mutex> guard(ctx->mu);
   NXH_HIP(op, hipSetDevice(ctx->device));

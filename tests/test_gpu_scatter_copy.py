@@ -1,0 +1,53 @@
+"""The one-pass copy and scatter of whole rows (scatter_copy) where its blocks, lists and vectors end: against a copy
+followed by a scatter, bit for bit, and against a serial sum."""
+
+import numpy as np
+import pytest
+
+from helpers import same_bits
+from raven_amd import dtype as dt
+from raven_amd.nx_backend import logical
+
+pytestmark = pytest.mark.gpu
+
+
+def rows_of(hip, ids, cols):
+    return hip.expand(hip.reshape(hip.from_host(ids.astype(np.int32), dt.int32), (len(ids), 1)), (len(ids), cols))
+
+
+@pytest.mark.parametrize("d", [dt.float32, dt.bfloat16, dt.int64], ids=lambda d: d.name)
+@pytest.mark.parametrize("rows,cols,n,spread", [
+    (1, 8, 1, 1), (15, 1024, 60, 15), (16, 1024, 64, 2), (17, 1023, 64, 17), (600, 16, 1024, 600), (600, 16, 1025, 600),
+    (600, 17, 2400, 1), (3000, 260, 2049, 3), (50257, 96, 8192, 50257), (5000, 7, 16385, 40)])
+def test_equals_copy_then_scatter(hip, d, rows, cols, n, spread):
+    """`spread`: how many different rows are hit; lists of up to 1024 updates and of more, in one block."""
+    rng = np.random.default_rng(rows * 7 + cols + n)
+
+    def tensor(shape):
+        if d is dt.bfloat16:
+            return hip.cast(hip.reshape(hip.from_host(rng.standard_normal(shape).astype(np.float32), dt.float32), shape), d)
+        return hip.reshape(hip.from_host(rng.integers(-9, 9, shape).astype(d.np_storage), d), shape)
+
+    template, updates = tensor((rows, cols)), tensor((n, cols))
+    ids = rng.integers(0, spread, n) - rng.integers(0, 2, n) * rows
+    index = rows_of(hip, ids, cols)
+    for mode in ("add", "set"):
+        got = hip.scatter(mode, False, template, index, updates, 0)
+        assert hip.last_path() == "scatter_copy"
+        want = hip.copy(template)
+        hip._check(hip._lib.nxh_scatter(hip._h, want._desc(), index._desc(), updates._desc(), 0, {"set": 0, "add": 1}[mode]))
+        same_bits(logical(got), logical(want), mode)
+
+
+def test_sums_in_the_order_of_positions(hip):
+    rng = np.random.default_rng(3)
+    rows, cols, n = 40, 1000, 160
+    t, u = rng.standard_normal((rows, cols)).astype(np.float32), rng.standard_normal((n, cols)).astype(np.float32)
+    ids = rng.integers(0, 5, n)
+    template = hip.reshape(hip.from_host(t, dt.float32), (rows, cols))
+    got = hip.scatter("add", False, template, rows_of(hip, ids, cols), hip.reshape(hip.from_host(u, dt.float32), (n, cols)), 0)
+    assert hip.last_path() == "scatter_copy"
+    want = t.copy()
+    for i, r in enumerate(ids):
+        want[r] += u[i]
+    same_bits(logical(got), want, "serial")
