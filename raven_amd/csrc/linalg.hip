@@ -1206,41 +1206,25 @@ static bool la_meet(const nxh_tensor *a, const nxh_tensor *b, int size) {
   return a0 < b1 && b0 < a1;
 }
 
-// The word of pinned memory the blocked kernels report to, and one of device memory by which the kernels of
-// one call hold each other back. Both belong to one call at a time (the context's call_mu): the first is
-// cleared before it is lent, the second (zero between calls, and no other kernel's) after a call that may have
-// set it. A call that returns early waits here for the kernels that may still write them.
+// The report of a blocked call (of whoever holds the context's call_mu): its number, and where its kernels put what they find.
 struct HostStatus {
   nxh_context *ctx;
-  bool lent = false, clean = false, held = false;  // clean: the kernels have been waited for and reported nothing
-  explicit HostStatus(nxh_context *c) : ctx(c) { *(volatile int *)word() = LA_OK; }
-  ~HostStatus() {
-    if (!lent || clean) return;
+  uint32_t seq;
+  explicit HostStatus(nxh_context *c) : ctx(c) {
     std::lock_guard<std::mutex> g(ctx->mu);
-    (void)hipStreamSynchronize(ctx->stream);
-    *(volatile int *)word() = LA_OK;
-    if (!held) return;
-    (void)hipMemcpyAsync(hold(), word(), sizeof(int), hipMemcpyHostToDevice, ctx->stream);
-    (void)hipStreamSynchronize(ctx->stream);
+    seq = nxh_next_report(ctx);
   }
-  int *word() const { return ctx->fault_flag_host + 8; }
-  int *hold() const { return ctx->fault_flag + 2; }
-  int *lend() {
-    lent = true;
-    return word();
-  }
-  int *lend_hold() {
-    held = true;
-    return hold();
-  }
-  // Waits for the kernels of this call (the results included) and reads their report.
-  int collect(const char *op) {
+  int *found() const { return ctx->fault_flag + 2; }
+  LaFailure failure(bool reports) const { return {found(), reports ? nxh_report_word(ctx, NXH_REPORT_LINALG) : nullptr, seq}; }
+  // For calls none of whose kernels reports: once the work queued so far has run.
+  void queue() const { nxh_queue_report(ctx, NXH_REPORT_LINALG, seq, found()); }
+  // Waits for the report. `code`: what a queued one stands for.
+  int collect(const char *op, int code) const {
     std::lock_guard<std::mutex> g(ctx->mu);
     NXH_HIP(op, hipGetLastError());
-    NXH_HIP(op, hipStreamSynchronize(ctx->stream));
-    const int code = *(volatile int *)word();
-    clean = code == LA_OK;
-    return clean ? NXH_OK : nxh_fail(NXH_FAILURE, op, LA_MESSAGES[code <= LA_NO_CONVERGE ? code : LA_NO_CONVERGE]);
+    int reported = LA_OK;
+    if (int rc = nxh_await_report(ctx, op, NXH_REPORT_LINALG, seq, &reported)) return rc;
+    return reported == LA_OK ? NXH_OK : nxh_fail(NXH_FAILURE, op, LA_MESSAGES[code]);
   }
 };
 
@@ -1270,7 +1254,7 @@ static int run_cholesky_as(nxh_context *ctx, const char *op, HostStatus &status,
       a.diag = (T *)diag + (size_t)(b0 * cols) * NB * NB;
       a.n = n;
       a.upper = upper;
-      a.status = status.lend();
+      a.failure = status.failure(b0 == 0);
       launch(a, (unsigned)std::min(LA_GRID_BATCH, batch - b0));
     }
   };
@@ -1281,12 +1265,11 @@ static int run_cholesky_as(nxh_context *ctx, const char *op, HostStatus &status,
       hipLaunchKernelGGL(kern, dim3((unsigned)tiles, nbat), dim3(C::THREADS), C::LDS, ctx->stream, a);
     }
   });
-  if (int rc = status.collect(op)) return rc;  // a matrix that has no factor leaves `out` as it was
+  // (a matrix that has no factor leaves `out` as it was)
   each_part([&](CholArgs<T> &a, unsigned nbat) {
     hipLaunchKernelGGL((cholesky_result_kernel<T, TS, ONE>), dim3((unsigned)result_tiles, nbat), dim3(256), 0, ctx->stream, a);
   });
-  NXH_HIP(op, hipGetLastError());
-  return NXH_OK;
+  return status.collect(op, LA_NOT_PD);
 }
 
 template <class T, class TS>
@@ -1342,9 +1325,11 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
     a.us = us;
     a.mbs = m.bs;
     a.rows = n;
-    a.status = status.lend();
-    hipLaunchKernelGGL((trsm_check_kernel<T, TS>), dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, ctx->stream, a, batch, status.lend_hold());
+    a.failure = status.failure(false);
+    hipLaunchKernelGGL((trsm_check_kernel<T, TS>), dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, ctx->stream, a, batch);
+    status.queue();  // (the solve's kernels find nothing more)
   }
+  const bool reports = direct && !check;  // one matrix and one pass, or unit diagonals: the solve's first workgroup
   for (int64_t b0 = 0; b0 < batch; b0 += LA_GRID_BATCH) {
     const unsigned nbat = (unsigned)std::min(LA_GRID_BATCH, batch - b0), groups = (unsigned)((nrhs + 15) / 16);
     for (int r0 = 0; r0 < n; r0 += TRSM_PASS<T>) {
@@ -1359,8 +1344,8 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
       a.x = LaMat{xp + b0 * x.bs + r0 * x.rs, x.rs, x.cs, x.bs};
       a.rows = std::min(n - r0, TRSM_PASS<T>);
       a.nrhs = nrhs;
-      a.status = status.lend();
-      a.hold = check ? status.hold() : nullptr;
+      a.failure = status.failure(reports && b0 == 0);
+      a.checked = check;
       const int nb = (a.rows + 15) / 16;
       const auto kern = nb == 1 ? one : sizeof(T) == 8 && nb <= 2 + TRSM_UPDATERS * TRSM_FEW ? few : most;  // (complex reads nothing ahead)
       const int threads = nb == 1 ? TRSM_THREADS<0> : TRSM_THREADS<TRSM_FEW>;
@@ -1371,9 +1356,9 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
                            LaMat{(TS *)a.x.p + a.rows * a.x.rs, a.x.rs, a.x.cs, a.x.bs}, rest);
     }
   }
-  NXH_HIP(op, hipGetLastError());
+  if (!check && !reports) status.queue();
   g.unlock();
-  return status.collect(op);
+  return status.collect(op, LA_SINGULAR);
 }
 
 #include "linalg_qr.hpp"

@@ -15,12 +15,16 @@ struct LaMat {
   int64_t rs, cs, bs;
 };
 
-// A numeric failure goes straight to a word of pinned host memory, which the call reads
-// after its stream wait: no copy of a device word is queued behind the kernels. Every
-// failure of one call has the same code, so a plain store is enough.
-__device__ __forceinline__ void raise_host(int *host_status, int code) {
-  __hip_atomic_store(host_status, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
+// A numeric failure of a call (every one of a call has the same meaning): a kernel stores the call's number to `found`,
+// in device memory, and kernels after it that see that number there write nothing. Nothing is cleared between calls.
+// The call reads it from a report (nxh_report_word), which a kernel stores to `report` as soon as it is known.
+struct LaFailure {
+  int *found;
+  uint64_t *report;  // null: this kernel does not report
+  uint32_t seq;
+  __device__ __forceinline__ void raise() const { __hip_atomic_store(found, (int)seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+  __device__ __forceinline__ bool raised() const { return *found == (int)seq; }
+};
 
 __device__ __forceinline__ double lane_value(double v, int lane) {  // `lane` uniform
   const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane), hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
@@ -256,7 +260,7 @@ __device__ __forceinline__ bool factor16_columns(double *tile, int ld, double *i
 // be waited for) and saves a launch per block column. Sums and factor share one workspace: a tile of
 // the factor goes where this workgroup's own sums were, those on the diagonal, whose sums the other
 // workgroups of the column read too, to a place of their own. The matrix itself is only read; the result is
-// written by cholesky_result_kernel, once it is known that there is one. The sums stay apart from
+// written by cholesky_result_kernel, where there is one. The sums stay apart from
 // the matrix until its column comes up, so that an element rounds a few times at its own size and not
 // once a column: float64, g g^T + n I, relative error of the factor in eps (2-norm, against long double) for
 // n = 64, 130, 400: 1.52, 2.03, 3.41 with the updates taken from the matrix one by one, 0.55, 0.50, 0.51 so
@@ -288,7 +292,7 @@ struct CholArgs {
   T *A, *diag;    // n x n per matrix, row-major: what is taken from x, with its sign, then the factor below the
                   // diagonal tiles; those tiles, NB x NB each
   int n, s, upper;
-  int *status;
+  LaFailure failure;
 };
 
 template <class T, class TS, int ONE>
@@ -572,7 +576,7 @@ __global__ __launch_bounds__((Chol<T, ONE>::THREADS)) void cholesky_block_kernel
     }
     solve_own(blocks - 1);
   }
-  if (bad && wave == 0 && lane == 0) raise_host(a.status, LA_NOT_PD);
+  if (bad && wave == 0 && lane == 0) a.failure.raise();
   __syncthreads();
   const int rows = min(n - i * NB, NB);
   if (has_own) {
@@ -589,7 +593,10 @@ __global__ __launch_bounds__((Chol<T, ONE>::THREADS)) void cholesky_block_kernel
   }
 }
 
-// The result with its zeros, a workgroup per tile (i, j), i >= j, and its mirror image. U = L^H.
+// The result with its zeros, a workgroup per tile (i, j), i >= j, and its mirror image. U = L^H. It is queued behind the
+// factorisation and writes nothing where that failed; its first workgroup tells the host, which goes on meanwhile ([512,512]
+// f32 and two solves: 413 us where each call waited for the stream and the result's launch for the host, 373 so; 300 of
+// [40,40] f64 100 -> 66).
 template <class T, class TS, int ONE>
 __global__ __launch_bounds__(256) void cholesky_result_kernel(CholArgs<T> a) {
   using S = Sc<T>;
@@ -605,6 +612,9 @@ __global__ __launch_bounds__(256) void cholesky_result_kernel(CholArgs<T> a) {
   const T zero = S::make(0.0, 0.0);
   constexpr int PER = NB * NB / 256;
   T v[PER];
+  const bool failed = a.failure.raised();
+  if (a.failure.report && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) nxh_report(a.failure.report, a.failure.seq, failed ? LA_NOT_PD : LA_OK);
+  if (failed) return;
 #pragma unroll
   for (int k = 0; k < PER; k++) {  // every load is on its way before the first is waited for: 10.4 -> 6.2 us at n = 512
     const int e = threadIdx.x + 256 * k, r = e / NB, c = e % NB;
@@ -652,21 +662,19 @@ struct TrsmArgs {
   int conj, unit;
   LaMat b, x;           // rows from row 0 of the solution order on; b is read, x written (TS)
   int rows, nrhs;
-  int *status;
-  const int *hold;  // several matrices: where it holds something, one of them is singular and nothing is written
+  LaFailure failure;
+  bool checked;  // trsm_check_kernel has looked through the batch: where it found a singular matrix, nothing is written
 };
 
 // A wave per matrix: whether an element of its diagonal is zero.
 template <class T, class TS>
-__global__ __launch_bounds__(256) void trsm_check_kernel(TrsmArgs<T> a, int64_t batch, int *found) {
+__global__ __launch_bounds__(256) void trsm_check_kernel(TrsmArgs<T> a, int64_t batch) {
   const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (b >= batch) return;
   const TS *m = (const TS *)a.m + b * a.mbs;
   bool zero = false;
   for (int t = threadIdx.x & 63; t < a.rows; t += 64) zero = zero || T(m[t * (a.ts + a.us)]) == Sc<T>::make(0.0, 0.0);
-  if (!zero) return;
-  raise(found, LA_SINGULAR);
-  raise_host(a.status, LA_SINGULAR);
+  if (zero) a.failure.raise();
 }
 
 template <class T, class TS>
@@ -731,6 +739,22 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
     }
   };
   for (int e = threadIdx.x; e < AHEAD * 256; e += blockDim.x) (&diag_inv[0][0][0])[e] = 0.0;
+  // One matrix (`report`): a wave that has nothing to do yet looks through its diagonal, and the host goes on.
+  if (a.failure.report && blockIdx.x == 0 && blockIdx.y == 0 && wave == (TILES > 0 ? TRSM_WAVES - 1 : 0)) {
+    bool zero = false;
+    if (!a.unit) {
+      constexpr int LOOK = 8;
+      for (int t0 = lane; t0 < n; t0 += 64 * LOOK) {
+        TS d[LOOK];
+#pragma unroll
+        for (int j = 0; j < LOOK; j++) d[j] = m[min(t0 + 64 * j, n - 1) * (a.ts + a.us)];
+#pragma unroll
+        for (int j = 0; j < LOOK; j++) zero = zero || T(d[j]) == S::make(0.0, 0.0);
+      }
+    }
+    zero = __any(zero);
+    if (lane == 0) nxh_report(a.failure.report, a.failure.seq, zero ? LA_SINGULAR : LA_OK);
+  }
   __syncthreads();
   TS raw[2][4];
   if (TILES == 0 || wave == TRSM_LOADER) {
@@ -882,8 +906,8 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
     }
   }
   // (every workgroup of a matrix has seen its whole diagonal)
-  if (singular || (a.hold && *a.hold)) {
-    if (threadIdx.x == 0 && singular) raise_host(a.status, LA_SINGULAR);
+  if (singular || (a.checked && a.failure.raised())) {
+    if (threadIdx.x == 0 && singular) a.failure.raise();
     return;
   }
   for (int e = threadIdx.x; e < n * 16; e += blockDim.x) {
