@@ -812,6 +812,347 @@ int radix_run(nxh_context *ctx, const char *op, SortArgs &a) {
   return NXH_OK;
 }
 
+// ── slices of some tiles: sorted tiles, split evenly, sorted again ──────────
+// Up to SPLIT_TILES tiles of 4096 words: (1) every tile is sorted by a network in one block; (2) a block per slice takes
+// every 32nd word of each sorted tile, sorts these and picks evenly spaced ones that cut the slice into parts, and finds
+// where each cuts each tile; (3) a block per part gathers its T runs, sorts them and writes the results. All words of
+// a slice differ, so the parts are bounded whatever the values are: a cut with R samples at or below it has between
+// 32 R and 32 R + 31 T words at or below it, and the cuts are taken so that 32 (R' - R) + 31 T <= 4096. The words cross
+// memory twice, against once per eight bits in the radix sort, and there are three launches for eight: [64,50257]
+// float32, argsort: 33 + 15 + 36 us, where the radix sort takes 36 for its histograms and 84 for its scatters. Bound by the
+// exchanges: 78 steps of two instructions, some eight clocks each, for every two words, with sixteen waves a compute unit.
+//
+// The words are doubles here: bits 0 - 19 the index, 20 - 51 the mapped key of Packed, above them one exponent for all
+// elements and the next one for padding, so an exchange inside a lane is a minimum and a maximum (two instructions;
+// on 64-bit integers a comparison and four selections), and a run that descends is an ascending one with its signs turned.
+constexpr int SPLIT_TILES = 32, SPLIT_EVERY = 32, SPLIT_SAMPLES = 4096 / SPLIT_EVERY;
+constexpr uint64_t FWORD = 0x2000000000000000ull, FWORD_PAD = FWORD + (1ull << 52);
+constexpr uint32_t FWORD_INDEX = 0xFFFFF;
+
+// The word of Packed, without a branch: `desc` all ones for a descending sort, `back` for the descending value sort.
+template <int DT>
+__device__ __forceinline__ double fword(typename Tr<DT>::C x, uint32_t index, uint32_t desc, uint32_t back) {
+  using TR = Tr<DT>;
+  uint32_t m;
+  if constexpr (TR::cat == CAT_FLOAT) {
+    uint32_t u = __builtin_bit_cast(uint32_t, (float)x);
+    const bool nan = u << 1 > 0xFF000000u;
+    u = u << 1 ? u : 0;  // -0 and +0 compare equal
+    m = nan ? Packed<DT>::K_NAN : u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u) ^ desc;
+    index ^= nan ? 0 : back;  // (FWORD_INDEX - index)
+  } else {
+    m = (TR::cat == CAT_SINT ? (uint32_t)(int32_t)x ^ 0x80000000u : (uint32_t)x) ^ desc;
+    index ^= back;
+  }
+  return __builtin_bit_cast(double, FWORD | (uint64_t)m << 20 | index);
+}
+__device__ __forceinline__ double fword_pad(uint32_t i) { return __builtin_bit_cast(double, FWORD_PAD | i); }
+
+// Sorts 4096 words held by 256 lanes, 16 each, in any order; afterwards lane t has places 16 t .. 16 t + 15. Bitonic:
+// level k brings runs of 2^k in alternating order, by exchanges at distances 2^(k-1) .. 1. Exchanges are made where the
+// four bits of a word's place that they concern number the registers of a lane: (A) bits 0 - 3, (B) 4 - 7 or (C) 8 - 11;
+// between these the words go through LDS, inside a wave between A and B. The first two levels past the lane
+// take data-parallel moves instead.
+// Places in `buf` are padded by one word in sixteen: sixteen lanes meet sixteen pairs of banks in A, B and C.
+constexpr int NET_LDS = 4096 + 256;
+__device__ __forceinline__ int net_place(int i) { return i + (i >> 4); }
+__device__ __forceinline__ void net_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+// (In place of fmin and fmax, which make every operand that comes from LDS a quiet number first, an instruction each:
+// no word is a NaN.)
+__device__ __forceinline__ double net_min(double x, double y) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
+}
+__device__ __forceinline__ double net_max(double x, double y) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+  return r;
+}
+template <int BITS>  // exchanges at register distances 2^(BITS-1) .. 1, ascending
+__device__ __forceinline__ void net_lane(double (&e)[16]) {
+#pragma unroll
+  for (int j = 1 << (BITS - 1); j >= 1; j >>= 1)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      if (r & j) continue;
+      const double x = e[r], y = e[r | j];
+      e[r] = net_min(x, y);
+      e[r | j] = net_max(x, y);
+    }
+}
+template <int LEVEL>
+__device__ __forceinline__ void net_first(double (&e)[16]) {  // levels inside the lane: the order alternates by register
+#pragma unroll
+  for (int j = 1 << (LEVEL - 1); j >= 1; j >>= 1)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      if (r & j) continue;
+      const double x = e[r], y = e[r | j];
+      const bool down = r >> LEVEL & 1;
+      e[r] = down ? net_max(x, y) : net_min(x, y);
+      e[r | j] = down ? net_min(x, y) : net_max(x, y);
+    }
+}
+template <int M>  // with the lane M = 1 or 2 places away, ascending
+__device__ __forceinline__ void net_near(double (&e)[16]) {
+  const bool keep_max = threadIdx.x & M;
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const double y = __builtin_bit_cast(double, lane_xor64(__builtin_bit_cast(uint64_t, e[r]), M));
+    e[r] = ((y < e[r]) != keep_max) ? y : e[r];
+  }
+}
+template <int LEVEL>
+__device__ __forceinline__ void net_level(double (&e)[16], double *buf) {
+  const int t = threadIdx.x, c = t >> 4, low = t & 15;
+  // runs that descend at this level and did not at the last one, or the other way round
+  const uint32_t turn = (uint32_t)((t >> (LEVEL - 4)) ^ (LEVEL > 4 ? t >> (LEVEL - 5) : 0)) << 31;
+#pragma unroll
+  for (int r = 0; r < 16; r++) e[r] = __hiloint2double(__double2hiint(e[r]) ^ turn, __double2loint(e[r]));
+  if constexpr (LEVEL == 6) net_near<2>(e);
+  if constexpr (LEVEL == 5 || LEVEL == 6) net_near<1>(e);
+  if constexpr (LEVEL > 6) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) buf[t * 17 + r] = e[r];
+    if constexpr (LEVEL > 8) {
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 16; r++) e[r] = buf[r * 272 + t + c];
+      net_lane<LEVEL - 8>(e);
+#pragma unroll
+      for (int r = 0; r < 16; r++) buf[r * 272 + t + c] = e[r];
+      __syncthreads();
+    } else {
+      net_wave_sync();
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) e[r] = buf[c * 272 + r * 17 + low];
+    net_lane<LEVEL < 8 ? LEVEL - 4 : 4>(e);
+#pragma unroll
+    for (int r = 0; r < 16; r++) buf[c * 272 + r * 17 + low] = e[r];
+    net_wave_sync();
+#pragma unroll
+    for (int r = 0; r < 16; r++) e[r] = buf[t * 17 + r];
+  }
+  net_lane<4>(e);
+}
+__device__ __forceinline__ void net_sort(double (&e)[16], double *buf) {
+  net_first<1>(e), net_first<2>(e), net_first<3>(e);
+  net_level<4>(e, buf), net_level<5>(e, buf), net_level<6>(e, buf), net_level<7>(e, buf), net_level<8>(e, buf);
+  net_level<9>(e, buf), net_level<10>(e, buf), net_level<11>(e, buf), net_level<12>(e, buf);
+}
+// Hands the sorted words out, lanes of a wave next to each other: f(place, word).
+template <class F>
+__device__ __forceinline__ void net_each(const double (&e)[16], double *buf, F f) {
+  const int t = threadIdx.x, lane = t & 63, first = t >> 6 << 10;
+#pragma unroll
+  for (int r = 0; r < 16; r++) buf[t * 17 + r] = e[r];
+  net_wave_sync();
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    const int i = first + q * 64 + lane;
+    f(i, buf[net_place(i)]);
+  }
+}
+
+struct SplitArgs {
+  double *words;   // [slices][tiles][4096]
+  uint32_t *cuts;  // [slices][parts + 1][tiles]: the words of a tile before a part
+  int tiles, parts;
+  uint32_t desc, back;  // of fword
+};
+
+template <int DT>
+__global__ __launch_bounds__(256) void split_tiles_kernel(SortArgs a, SplitArgs p) {
+  using TR = Tr<DT>;
+  __shared__ double buf[NET_LDS];
+  const int64_t s = blockIdx.x / p.tiles;
+  const int tile = (int)(blockIdx.x % p.tiles);
+  int64_t io, oo;
+  slice_offsets(a, s, io, oo);
+  const typename TR::S *in = reinterpret_cast<const typename TR::S *>(a.in) + io;
+  typename TR::S x[16];
+  double e[16];
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const int64_t i = tile * 4096 + r * 256 + threadIdx.x;
+    x[r] = in[(i < a.n ? i : a.n - 1) * a.in_axis];
+  }
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const uint32_t i = (uint32_t)(tile * 4096 + r * 256 + threadIdx.x);
+    e[r] = i < a.n ? fword<DT>(TR::ld(x[r]), i, p.desc, p.back) : fword_pad(i);
+  }
+  net_sort(e, buf);
+  double *to = p.words + (int64_t)blockIdx.x * 4096;
+  net_each(e, buf, [&](int i, double w) { to[i] = w; });
+}
+
+__global__ __launch_bounds__(256) void split_cuts_kernel(SplitArgs p) {
+  __shared__ double buf[NET_LDS], sample[4096];
+  const double *words = p.words + (int64_t)blockIdx.x * p.tiles * 4096;
+  uint32_t *cuts = p.cuts + (int64_t)blockIdx.x * (p.parts + 1) * p.tiles;
+  const int samples = p.tiles * SPLIT_SAMPLES;
+  double e[16];
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const int q = r * 256 + threadIdx.x;
+    e[r] = q < samples ? words[(int64_t)q * SPLIT_EVERY + SPLIT_EVERY - 1] : fword_pad((1u << 20) + q);
+  }
+#pragma unroll
+  for (int r = 0; r < 16; r++) sample[r * 256 + threadIdx.x] = e[r];
+  net_sort(e, buf);
+  net_each(e, buf, [](int, double) {});  // (places the sorted samples in buf)
+  __syncthreads();
+  for (int pair = threadIdx.x; pair < (p.parts + 1) * p.tiles; pair += 256) {
+    const int k = pair / p.tiles, tile = pair % p.tiles;
+    uint32_t at = k == 0 ? 0 : 4096;
+    if (k > 0 && k < p.parts) {
+      const double cut = buf[net_place(k * samples / p.parts - 1)];
+      const double *own = sample + tile * SPLIT_SAMPLES, *tw = words + (int64_t)tile * 4096;
+      int lo = 0, hi = SPLIT_SAMPLES;  // samples at or below the cut
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (own[mid] <= cut) lo = mid + 1;
+        else hi = mid;
+      }
+      int first = lo * SPLIT_EVERY, last = lo < SPLIT_SAMPLES ? first + SPLIT_EVERY - 1 : first;  // the words up to the next sample
+      while (first < last) {
+        const int mid = (first + last) >> 1;
+        if (tw[mid] <= cut) first = mid + 1;
+        else last = mid;
+      }
+      at = (uint32_t)first;
+    }
+    cuts[pair] = at;
+  }
+}
+
+template <int DT, bool ARG>
+__global__ __launch_bounds__(256) void split_parts_kernel(SortArgs a, SplitArgs p) {
+  using TR = Tr<DT>;
+  using S = typename TR::S;
+  __shared__ double buf[NET_LDS];
+  __shared__ int begin[SPLIT_TILES], before[SPLIT_TILES + 1];  // of each run: its first word; where it lies in buf
+  __shared__ int64_t first_place;
+  const int64_t s = blockIdx.x / p.parts;
+  const int part = (int)(blockIdx.x % p.parts), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t *cuts = p.cuts + (s * (p.parts + 1) + part) * p.tiles;
+  if (wave == 0) {
+    const int lo = lane < p.tiles ? (int)cuts[lane] : 0, n = lane < p.tiles ? (int)cuts[lane + p.tiles] - lo : 0;
+    int sum = n, all = lo;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(sum, d, 64), q = __shfl_xor(all, d, 64);
+      if (lane >= d) sum += o;
+      all += q;
+    }
+    if (lane < p.tiles) begin[lane] = lo, before[lane + 1] = sum;
+    if (lane == 0) before[0] = 0, first_place = all;
+  }
+  __syncthreads();
+  const int64_t place0 = first_place;
+  if (place0 >= a.n) return;  // nothing but padding
+  const double *words = p.words + s * p.tiles * 4096;
+  // a wave to two runs at a time, six loads of a lane of each in flight
+  for (int tile = wave; tile < p.tiles; tile += 8) {
+    const int other = tile + 4 < p.tiles ? tile + 4 : tile;
+    const int at[2] = {before[tile], before[other]}, n[2] = {before[tile + 1] - at[0], other > tile ? before[other + 1] - at[1] : 0};
+    const double *run[2] = {words + (int64_t)tile * 4096 + begin[tile], words + (int64_t)other * 4096 + begin[other]};
+    for (int i0 = lane; i0 < max(n[0], n[1]); i0 += 64 * 6) {
+      double w[2][6];
+#pragma unroll
+      for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int j = 0; j < 6; j++) w[k][j] = i0 + 64 * j < n[k] ? run[k][i0 + 64 * j] : 0.0;
+#pragma unroll
+      for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int j = 0; j < 6; j++)
+          if (i0 + 64 * j < n[k]) buf[at[k] + i0 + 64 * j] = w[k][j];
+    }
+  }
+  __syncthreads();
+  const int count = before[p.tiles];
+  double e[16];
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const int i = r * 256 + threadIdx.x;
+    e[r] = i < count ? buf[i] : fword_pad((1u << 20) + i);
+  }
+  __syncthreads();
+  net_sort(e, buf);
+  int64_t io, oo;
+  slice_offsets(a, s, io, oo);
+  const int64_t left = a.n - place0;
+  const int live = left < count ? (int)left : count;
+  net_each(e, buf, [&](int i, double word) {
+    if (i >= live) return;
+    const uint64_t w = __builtin_bit_cast(uint64_t, word);
+    const uint32_t m = (uint32_t)(w >> 20), low = (uint32_t)w & FWORD_INDEX;
+    const bool nan = TR::cat == CAT_FLOAT && m == Packed<DT>::K_NAN;
+    if constexpr (ARG) {  // (no value is looked at: one instantiation for all types)
+      reinterpret_cast<int32_t *>(a.out)[oo + (place0 + i) * a.out_axis] = (int32_t)low;
+    } else {
+      const uint32_t index = nan ? low : low ^ p.back;
+      S *out = reinterpret_cast<S *>(a.out) + oo + (place0 + i) * a.out_axis;
+      const uint32_t up = m ^ p.desc;
+      if (nan || (TR::cat == CAT_FLOAT && up == 0x80000000u)) {  // a payload, a sign of zero: not in the key
+        *out = TR::st(TR::ld(reinterpret_cast<const S *>(a.in)[io + (int64_t)index * a.in_axis]));
+      } else if constexpr (TR::cat == CAT_FLOAT) {
+        *out = TR::st((typename TR::C)__builtin_bit_cast(float, (up & 0x80000000u) ? up ^ 0x80000000u : ~up));
+      } else if constexpr (TR::cat == CAT_SINT) {
+        *out = TR::st((typename TR::C)(int32_t)(up ^ 0x80000000u));
+      } else {
+        *out = TR::st((typename TR::C)up);
+      }
+    }
+  });
+}
+
+// Whether the results may lie over the input (its blocks read it after others have written).
+template <int DT>
+bool sort_meets_input(const SortArgs &a, int out_size) {
+  int64_t in_lo = 0, in_hi = 0, out_lo = 0, out_hi = 0;
+  const auto grow = [](int64_t &lo, int64_t &hi, int64_t stride, int64_t extent) { (stride < 0 ? lo : hi) += stride * (extent - 1); };
+  grow(in_lo, in_hi, a.in_axis, a.n);
+  grow(out_lo, out_hi, a.out_axis, a.n);
+  for (int d = 0; d < a.nk; d++) {
+    grow(in_lo, in_hi, a.k_in[d], a.kshape[d]);
+    grow(out_lo, out_hi, a.k_out[d], a.kshape[d]);
+  }
+  const int in_size = (int)sizeof(typename Tr<DT>::S);
+  return a.in + in_lo * in_size < a.out + (out_hi + 1) * out_size && a.out + out_lo * out_size < a.in + (in_hi + 1) * in_size;
+}
+
+template <int DT, int MODE>
+int split_run(nxh_context *ctx, const char *op, SortArgs &a) {
+  constexpr bool ARG = MODE >= ARG_ASC;
+  SplitArgs p;
+  p.desc = MODE == VALUE_DESC || MODE == ARG_DESC ? ~0u : 0;
+  p.back = MODE == VALUE_DESC ? FWORD_INDEX : 0;
+  p.tiles = (int)((a.n + 4095) / 4096);
+  const int samples = p.tiles * SPLIT_SAMPLES, most = (4096 - (SPLIT_EVERY - 1) * p.tiles) / SPLIT_EVERY;  // samples of a part
+  p.parts = (samples + most - 1) / most;
+  if (a.slices * std::max(p.tiles, p.parts) > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "too many elements for one launch");
+  Scratch scratch(ctx);
+  if (scratch.get(0, (size_t)(a.slices * p.tiles) * 4096 * sizeof(double)) ||
+      scratch.get(1, (size_t)(a.slices * (p.parts + 1) * p.tiles) * sizeof(uint32_t)))
+    return nxh_fail(NXH_FAILURE, op, NXH_ERR_ALLOC);
+  p.words = (double *)scratch.p[0];
+  p.cuts = (uint32_t *)scratch.p[1];
+  nxh_set_path("sort_radix");  // the name of every long form of packed words
+  hipLaunchKernelGGL((split_tiles_kernel<DT>), dim3((unsigned)(a.slices * p.tiles)), dim3(256), 0, ctx->stream, a, p);
+  hipLaunchKernelGGL(split_cuts_kernel, dim3((unsigned)a.slices), dim3(256), 0, ctx->stream, p);
+  hipLaunchKernelGGL((split_parts_kernel<ARG ? NXH_F32 : DT, ARG>), dim3((unsigned)(a.slices * p.parts)), dim3(256), 0, ctx->stream, a, p);
+  NXH_HIP(op, hipGetLastError());
+  return NXH_OK;
+}
+
 template <int DT, int MODE>
 int psort_run(nxh_context *ctx, const char *op, SortArgs &a) {
   if (a.n_pad <= 4096) {
@@ -831,6 +1172,13 @@ int psort_run(nxh_context *ctx, const char *op, SortArgs &a) {
     }
     NXH_HIP(op, hipGetLastError());
     return NXH_OK;
+  }
+  // Sorted tiles and parts against a radix sort that needs all four of its passes (argsort, us): [64,50257] 85 / 117, [1,50257]
+  // 43 / 57, [1,4097] 41 / 50, [200,6000] 66 / 78, [24,131072] 101 / 110, [1000,9000] 221 / 254. Of three passes (float16)
+  // 83 / 93, 44 / 46, 41 / 42, 64 / 62, 100 / 87, 210 / 201, of two (bfloat16) 86 / 64: those stay.
+  if constexpr (__builtin_popcount(rx_pass_mask<DT>()) == 4) {
+    if (a.n <= SPLIT_TILES * 4096 && !sort_meets_input<DT>(a, MODE >= ARG_ASC ? 4 : (int)sizeof(typename Tr<DT>::S)))
+      return split_run<DT, MODE>(ctx, op, a);
   }
   return radix_run<DT, MODE>(ctx, op, a);
 }

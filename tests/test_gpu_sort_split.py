@@ -1,0 +1,65 @@
+"""Slices of some tiles of 32-bit keys: parts stay within a tile whatever the values, and ties, NaNs and padding keep
+their places. Lengths at the edges of tiles and of the number of tiles."""
+
+import numpy as np
+import pytest
+
+from helpers import same_bits
+from raven_amd import dtype as dt
+from raven_amd.nx_backend import logical
+
+pytestmark = pytest.mark.gpu
+
+
+def shapes_of_values(rng, slices, n):
+    ramp = np.arange(n, dtype=np.float64) - n // 2
+    return {"constant": np.zeros((slices, n)), "ascending": np.tile(ramp, (slices, 1)), "descending": np.tile(-ramp, (slices, 1)),
+            "three": rng.integers(-1, 2, (slices, n)).astype(float), "saw": np.tile(ramp % 4096, (slices, 1)),
+            "interleaved": np.tile(ramp.reshape(-1) * 4099 % (n | 1), (slices, 1)), "random": rng.permutation(slices * n).reshape(slices, n) - 5.0,
+            "one apart": np.where(np.arange(n) == n - 1, -1.0, 1.0)[None].repeat(slices, 0)}
+
+
+@pytest.mark.parametrize("d", [dt.float32, dt.int32, dt.uint32], ids=lambda d: d.name)
+@pytest.mark.parametrize("slices,n", [(3, 4097), (2, 8191), (2, 8193), (1, 53249), (1, 131072)])
+def test_any_distribution(hip, d, slices, n):
+    rng = np.random.default_rng(n)
+    for name, v in shapes_of_values(rng, slices, n).items():
+        if d is dt.uint32:
+            v = v + 2.0**31
+        raw = v.astype(d.np_storage)
+        x = hip.reshape(hip.from_host(raw, d), (slices, n))
+        for desc in (False, True):
+            order = np.stack([np.argsort(-r.astype(np.float64) if desc else r, kind="stable") for r in raw])
+            same_bits(logical(hip.argsort(x, 1, desc)), order.astype(np.int32), f"{name} {desc}")
+            same_bits(logical(hip.sort(x, 1, desc)), np.take_along_axis(raw, order, 1), f"{name} {desc}")
+
+
+@pytest.mark.parametrize("n", [4097, 50257])
+def test_numbers_that_are_none_and_zeros(hip, n):
+    rng = np.random.default_rng(n)
+    bits = rng.integers(0, 2**32, (2, n), dtype=np.uint64).astype(np.uint32)  # every pattern: NaNs of both signs, infinities
+    bits[:, ::3] = rng.choice(np.array([0, 0x80000000, 0x7F800000, 0xFF800000, 0x7FC00001, 0xFFC00002, 1, 0x80000001], np.uint32), bits[:, ::3].shape)
+    v = bits.view(np.float32)
+    x = hip.reshape(hip.from_host(v, dt.float32), (2, n))
+    for desc in (False, True):
+        wide = np.nan_to_num(v, nan=0.0, posinf=np.inf, neginf=-np.inf).astype(np.float64)
+        order = np.stack([np.lexsort((-w if desc else w, np.isnan(r))) for w, r in zip(wide, v)])
+        same_bits(logical(hip.argsort(x, 1, desc)), order.astype(np.int32), f"{desc}")
+        got = logical(hip.sort(x, 1, desc)).view(np.uint32)
+        finite = ~np.isnan(np.take_along_axis(v, order, 1))
+        want = np.take_along_axis(bits, order, 1)
+        same = (got == want) | ((got << 1 == 0) & (want << 1 == 0))  # which zero comes first is open
+        assert np.all(same | ~finite) and np.all(np.isnan(got.view(np.float32)) == ~finite)
+        assert np.array_equal(np.sort(got, axis=1), np.sort(bits, axis=1)), "every element once, zeros and payloads too"
+
+
+def test_in_place_and_views(hip):
+    rng = np.random.default_rng(1)
+    v = rng.standard_normal((6000, 3)).astype(np.float32)
+    v[::7] = -0.0
+    x = hip.permute(hip.reshape(hip.from_host(v, dt.float32), (6000, 3)), (1, 0))
+    same_bits(logical(hip.argsort(x, 1, False)), np.argsort(v.T, axis=1, kind="stable").astype(np.int32), "a strided slice")
+    v[::7] = 0.5  # (in place, the sign of a zero may be that of another one)
+    y = hip.copy(hip.permute(hip.reshape(hip.from_host(v, dt.float32), (6000, 3)), (1, 0)))
+    hip._check(hip._lib.nxh_sort(hip._h, y._desc(), y._desc(), 1, 0))
+    assert np.array_equal(logical(y), np.sort(v.T, axis=1))
