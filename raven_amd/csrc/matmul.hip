@@ -271,7 +271,9 @@ __global__ __launch_bounds__(256) void gemm_skinny_mfma_kernel(SkinnyArgs a) {
 }
 
 // ── gemm_skinny_mfma_k8: the same stream when N alone fills the chip ────────
-// One block of eight waves owns 64 columns; the waves split K eight ways and fold their
+// One block of eight waves owns 64 columns; the waves take the steps of K in turn, so that a block reads
+// rows that follow each other ([8,4096] x [4096,16384] bfloat16 with weights from memory: 27.2 us; a
+// contiguous eighth of K a wave, 16 MB from one to the next, took 29.1), and fold their
 // accumulators through LDS in wave order at the end, so there are no f32 partials in memory
 // and no second launch. A (at most 16 x K, a few dozen KiB, resident in L2) is not staged:
 // each lane reads its 16-byte fragment of the step straight from memory, three steps ahead
@@ -285,9 +287,9 @@ __global__ __launch_bounds__(64 * SM8_WAVES) void gemm_skinny_mfma_k8_kernel(Ski
   extern __shared__ __attribute__((aligned(16))) uint16_t sm_lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t n0 = (int64_t)blockIdx.x * SM_WN;
-  const int64_t k0 = (int64_t)wave * a.kchunk;
-  const int64_t k1 = k0 + a.kchunk < a.K ? k0 + a.kchunk : a.K;
-  const int kn = k1 > k0 ? (int)(k1 - k0) : 0;  // a multiple of 8 (K is)
+  // step s of this wave: rows [(8 s + wave) SM_KS, .. + SM_KS) of B, as far as they are below K (a multiple of 8)
+  const int64_t k0 = (int64_t)wave * SM_KS, kn = a.K - k0;
+  constexpr int64_t STRIDE = SM8_WAVES * SM_KS;
   const uint16_t *A = (const uint16_t *)a.A;
   const uint16_t *B = (const uint16_t *)a.B;
   uint16_t *sB = sm_lds + wave * (2 * SM_TILE);
@@ -301,11 +303,11 @@ __global__ __launch_bounds__(64 * SM8_WAVES) void gemm_skinny_mfma_k8_kernel(Ski
   auto load = [&](U4 (&r)[4], U4 &x, int step) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int kk = step * SM_KS + rbase + i * 8;
-      r[i] = (col_ok && kk < kn) ? *reinterpret_cast<const U4 *>(bp + (int64_t)kk * a.brs) : U4{0, 0, 0, 0};
+      const int64_t kk = step * STRIDE + rbase + i * 8;
+      r[i] = (col_ok && kk < kn) ? *reinterpret_cast<const U4 *>(bp + kk * a.brs) : U4{0, 0, 0, 0};
     }
-    const int ka = step * SM_KS + g * 8;
-    x = (row_ok && ka < kn) ? *reinterpret_cast<const U4 *>(ap + step * SM_KS) : U4{0, 0, 0, 0};
+    const int64_t ka = step * STRIDE + g * 8;
+    x = (row_ok && ka < kn) ? *reinterpret_cast<const U4 *>(ap + step * STRIDE) : U4{0, 0, 0, 0};
   };
   auto store = [&](const U4 (&r)[4], int buf) {
 #pragma unroll
@@ -315,7 +317,7 @@ __global__ __launch_bounds__(64 * SM8_WAVES) void gemm_skinny_mfma_k8_kernel(Ski
   f32x4 acc[4];
 #pragma unroll
   for (int t = 0; t < 4; t++) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  const int nsteps = (kn + SM_KS - 1) / SM_KS;
+  const int nsteps = kn > 0 ? (int)((kn + STRIDE - 1) / STRIDE) : 0;
   // step s multiplies the tile in LDS buffer s & 1 by the A fragment of slot s % 3; slot (s + 1) % 3
   // is stored for step s + 1 and refilled with step s + 4
   auto step = [&](int s, auto slot_c) {
@@ -380,7 +382,7 @@ __global__ __launch_bounds__(64 * SM8_WAVES) void gemm_skinny_mfma_k8_kernel(Ski
 // lane / 16 per lane; that MFMA j then holds columns 4 l + j instead of l is undone at the
 // store. The A operand of the same instructions is A[lane % 16][k], one 4-byte load from L2
 // (rows >= M read as zero). A wave so covers 64 columns by 4 k-rows per load instruction,
-// 256 contiguous bytes per row; the eight waves of a block split K and fold through LDS.
+// 256 contiguous bytes per row; the eight waves of a block take the steps of K in turn and fold through LDS.
 constexpr int SF_U = 8;  // steps (of 4 k-rows) in flight per wave
 __global__ __launch_bounds__(64 * SM8_WAVES) void gemm_skinny_f32_k8_kernel(SkinnyArgs a) {
   typedef __attribute__((ext_vector_type(4))) float f32x4_t;
@@ -388,8 +390,6 @@ __global__ __launch_bounds__(64 * SM8_WAVES) void gemm_skinny_f32_k8_kernel(Skin
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int kg = lane >> 4, l = lane & 15;
   const int64_t n0 = (int64_t)blockIdx.x * 64;
-  const int64_t k0 = (int64_t)wave * a.kchunk;
-  const int64_t k1 = k0 + a.kchunk < a.K ? k0 + a.kchunk : a.K;
   const float *A = (const float *)a.A;
   const float *B = (const float *)a.B;
   const bool col_ok = n0 + 4 * l < a.N;  // N is a multiple of 4: vectors are whole or absent
@@ -399,13 +399,13 @@ __global__ __launch_bounds__(64 * SM8_WAVES) void gemm_skinny_f32_k8_kernel(Skin
   f32x4_t acc[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) acc[j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int64_t kb = k0; kb < k1; kb += 4 * SF_U) {
+  for (int64_t kb = (int64_t)wave * (4 * SF_U); kb < a.K; kb += SM8_WAVES * 4 * SF_U) {
     f32x4_t b[SF_U];
     float av[SF_U];
 #pragma unroll
     for (int u = 0; u < SF_U; u++) {
       const int64_t k = kb + 4 * u + kg;
-      const bool in = k < k1;
+      const bool in = k < a.K;
       b[u] = (in && col_ok) ? *reinterpret_cast<const f32x4_t *>(bp + k * a.brs) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
       av[u] = (in && row_ok) ? ap[k * a.acs] : 0.0f;
     }
@@ -692,7 +692,6 @@ static int launch_skinny(nxh_context *ctx, GemmArgs &g) {
     const int64_t strips = (g.N + 63) / 64;
     if (strips >= cus && strips <= 0x7fffffffLL && g.N % 4 == 0 && g.brs % 4 == 0 && ((uintptr_t)g.B % 16) == 0 &&
         g.K >= 4 * SF_U * SM8_WAVES) {
-      a.kchunk = ((g.K + SM8_WAVES - 1) / SM8_WAVES + 3) / 4 * 4;
       a.nsplit = 1;
       a.C = g.C;
       nxh_set_path("gemm_skinny_f32_k8");
@@ -765,7 +764,6 @@ static int launch_skinny_mfma(nxh_context *ctx, GemmArgs &g) {
       attr_status = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS);
     });
     NXH_HIP("matmul", attr_status);
-    a.kchunk = ((g.K + SM8_WAVES - 1) / SM8_WAVES + SM_KS - 1) / SM_KS * SM_KS;
     a.nsplit = 1;
     a.C = g.C;
     nxh_set_path("gemm_skinny_mfma_k8");
