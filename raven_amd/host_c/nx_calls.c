@@ -10,7 +10,8 @@
  *   DeviceBuffer  one allocation of a context, given back when the last handle goes
  *   Tensor        buffer, view, dtype, context (nx_backend.ml:36-43)
  *   Calls         the base class of Backend: unary, binary, compare, where, cast, copy, assign, full,
- *                 reduce, matmul. A call whose arguments are out of the ordinary (axes that are no
+ *                 reduce, matmul; and what the frontend makes of them over operands that broadcast:
+ *                 broadcast_binary, broadcast_where, reduce_keep. A call whose arguments are out of the ordinary (axes that are no
  *                 plain integers, batches that broadcast, ...) goes to the Python method of the same
  *                 name with `_general` behind it.
  */
@@ -560,6 +561,89 @@ static PyObject *calls_full(Calls *self, Args args, Py_ssize_t n, PyObject *kw) 
   if (result_plan(&r, a[1], a[0])) return NULL;
   RUN(r, self, L.fill(h, &r.d, value));
 }
+/* ── operands that broadcast ───────────────────────────────────────────────── */
+/* The frontend's rule (frontend.ml:293-296, view.ml expand) applied to descriptors: no reshaped and expanded
+ * handles are made of the operands (a forward of GPT-2, 48 tokens, issued call by call: 429 such steps, 74 reductions
+ * that keep their axes, 73 products whose batches broadcast: 2119 us -> 1512). What is out of the ordinary (no plain
+ * Tensor, extents that do not fit, empty results) answers NotImplemented, and the frontend goes the long way. */
+static int broadcast_extents(int64_t *shape, int *ndim, const nxh_tensor *t) {
+  const int n = *ndim > t->ndim ? *ndim : t->ndim;
+  for (int i = 0; i < n; i++) { /* from the last dim on */
+    const int64_t a = i < *ndim ? shape[NXH_MAX_NDIM - 1 - i] : 1, b = i < t->ndim ? t->shape[t->ndim - 1 - i] : 1;
+    if (a != b && a != 1 && b != 1) return 0;
+    shape[NXH_MAX_NDIM - 1 - i] = a == 1 ? b : a;
+    if (a == 0 || b == 0) return 0;
+  }
+  *ndim = n;
+  return 1;
+}
+/* `t` seen with `ndim` extents: a dim that is not there, or is 1 where the other is not, is read in place. */
+static void broadcast_view(nxh_tensor *t, const int64_t *shape, int ndim) {
+  const int pad = ndim - t->ndim;
+  for (int i = ndim - 1; i >= 0; i--) {
+    t->strides[i] = i >= pad && t->shape[i - pad] == shape[i] ? t->strides[i - pad] : 0;
+    t->shape[i] = shape[i];
+  }
+  t->ndim = ndim;
+}
+static int same_extents(const nxh_tensor *t, const int64_t *shape, int ndim) {
+  return t->ndim == ndim && !memcmp(t->shape, shape, sizeof(int64_t) * (size_t)ndim);
+}
+/* Describes n operands, broadcast together, and plans a result of their extents. 0: go the long way; -1: an error. */
+static int broadcast_plan(Result *r, nxh_tensor *t, PyObject *const *a, int n, PyObject *dtype) {
+  int64_t extents[NXH_MAX_NDIM];
+  int ndim = 0;
+  for (int i = 0; i < n; i++)
+    if (Py_TYPE(a[i]) != &TensorType) return 0;
+  for (int i = 0; i < n; i++) {
+    if (describe(&t[i], a[i])) return -1;
+    if (!broadcast_extents(extents, &ndim, &t[i])) return 0;
+  }
+  const int64_t *shape = extents + NXH_MAX_NDIM - ndim;
+  PyObject *like = NULL; /* the extents as a tuple: an operand's where one has them */
+  for (int i = 0; i < n; i++) {
+    if (!same_extents(&t[i], shape, ndim)) broadcast_view(&t[i], shape, ndim);
+    else if (!like) like = ((Tensor *)a[i])->shape;
+  }
+  if (like) return result_plan(r, like, dtype) ? -1 : 1;
+  if (!(like = PyTuple_New(ndim))) return -1;
+  for (int i = 0; i < ndim; i++) {
+    PyObject *e = PyLong_FromLongLong(shape[i]);
+    if (!e) {
+      Py_DECREF(like);
+      return -1;
+    }
+    PyTuple_SET_ITEM(like, i, e);
+  }
+  const int bad = result_plan(r, like, dtype);
+  Py_DECREF(like);
+  return bad ? -1 : 1;
+}
+static PyObject *calls_broadcast_binary(Calls *self, Args args, Py_ssize_t n, PyObject *kw) {
+  static const char *const names[] = {"op", "x", "y"};
+  PyObject *a[3];
+  if (take("broadcast_binary", names, 3, args, n, kw, a)) return NULL;
+  int op = op_number(op_binary, a[0]);
+  if (op < 0) return NULL;
+  Result r;
+  nxh_tensor t[2];
+  const int planned = Py_TYPE(a[1]) == &TensorType ? broadcast_plan(&r, t, a + 1, 2, ((Tensor *)a[1])->dtype) : 0;
+  if (planned < 0) return NULL;
+  if (!planned) Py_RETURN_NOTIMPLEMENTED;
+  RUN(r, self, L.binary(h, op, &r.d, &t[0], &t[1]));
+}
+static PyObject *calls_broadcast_where(Calls *self, Args args, Py_ssize_t n, PyObject *kw) {
+  static const char *const names[] = {"cond", "if_true", "if_false"};
+  PyObject *a[3];
+  if (take("broadcast_where", names, 3, args, n, kw, a)) return NULL;
+  Result r;
+  nxh_tensor t[3];
+  const int planned = Py_TYPE(a[1]) == &TensorType ? broadcast_plan(&r, t, a, 3, ((Tensor *)a[1])->dtype) : 0;
+  if (planned < 0) return NULL;
+  if (!planned) Py_RETURN_NOTIMPLEMENTED;
+  RUN(r, self, L.where(h, &r.d, &t[0], &t[1], &t[2]));
+}
+
 static PyObject *general(Calls *self, const char *name, PyObject **a, Py_ssize_t n) {
   PyObject *m = PyObject_GetAttrString((PyObject *)self, name);
   if (!m) return NULL;
@@ -567,10 +651,31 @@ static PyObject *general(Calls *self, const char *name, PyObject **a, Py_ssize_t
   Py_DECREF(m);
   return r;
 }
-static PyObject *calls_reduce(Calls *self, Args args, Py_ssize_t n, PyObject *kw) {
-  static const char *const names[] = {"op", "axes", "x"};
-  PyObject *a[3];
-  if (take("reduce", names, 3, args, n, kw, a)) return NULL;
+/* The view of a result whose reduced axes stay as dims of extent 1 (a fresh result is contiguous either way). */
+static int keep_axes(Result *r, PyObject *shape, const int32_t *axes, Py_ssize_t na) {
+  const Py_ssize_t nd = PyTuple_GET_SIZE(shape);
+  PyObject *kept = PyTuple_New(nd);
+  if (!kept) return -1;
+  for (Py_ssize_t i = 0, k = 0; i < nd; i++) {
+    PyObject *e = k < na && axes[k] == i ? PyLong_FromLong(1) : PyTuple_GET_ITEM(shape, i);
+    if (k < na && axes[k] == i) k++;
+    else Py_INCREF(e);
+    PyTuple_SET_ITEM(kept, i, e);
+  }
+  PyObject *view = PyDict_GetItemWithError(contiguous_views, kept);
+  if (view) Py_INCREF(view);
+  else if (!PyErr_Occurred()) view = PyObject_CallOneArg(view_create, kept);
+  Py_DECREF(kept);
+  PyObject *own = view ? PyObject_GetAttr(view, s_shape) : NULL;
+  if (!own) {
+    Py_XDECREF(view);
+    return -1;
+  }
+  Py_SETREF(r->view, view);
+  Py_SETREF(r->shape, own);
+  return 0;
+}
+static PyObject *reduce_over(Calls *self, PyObject **a, int keep) {
   int op = op_number(op_reduce, a[0]);
   if (op < 0) return NULL;
   if (Py_TYPE(a[2]) == &TensorType && (PyList_CheckExact(a[1]) || PyTuple_CheckExact(a[1]))) {
@@ -606,10 +711,25 @@ static PyObject *calls_reduce(Calls *self, Args args, Py_ssize_t n, PyObject *kw
       int bad = result_plan(&r, kept, ((Tensor *)a[2])->dtype);
       Py_DECREF(kept);
       if (bad) return NULL;
+      if (keep && keep_axes(&r, shape, axes, na)) {
+        result_drop(&r);
+        return NULL;
+      }
       RUN(r, self, L.reduce(h, op, &r.d, &x, axes, (int)na));
     }
   }
+  if (keep) Py_RETURN_NOTIMPLEMENTED;
   return general(self, "_reduce_general", a, 3);
+}
+static PyObject *calls_reduce(Calls *self, Args args, Py_ssize_t n, PyObject *kw) {
+  static const char *const names[] = {"op", "axes", "x"};
+  PyObject *a[3];
+  return take("reduce", names, 3, args, n, kw, a) ? NULL : reduce_over(self, a, 0);
+}
+static PyObject *calls_reduce_keep(Calls *self, Args args, Py_ssize_t n, PyObject *kw) {
+  static const char *const names[] = {"op", "axes", "x"};
+  PyObject *a[3];
+  return take("reduce_keep", names, 3, args, n, kw, a) ? NULL : reduce_over(self, a, 1);
 }
 static PyObject *calls_matmul(Calls *self, Args args, Py_ssize_t n, PyObject *kw) {
   static const char *const names[] = {"x", "y"};
@@ -618,14 +738,18 @@ static PyObject *calls_matmul(Calls *self, Args args, Py_ssize_t n, PyObject *kw
   if (Py_TYPE(a[0]) == &TensorType && Py_TYPE(a[1]) == &TensorType) {
     nxh_tensor x, y;
     if (describe(&x, a[0]) || describe(&y, a[1])) return NULL;
-    /* equal batches, and rows that take no padded pitch */
-    int fine = x.ndim >= 2 && x.ndim == y.ndim && y.shape[y.ndim - 1] < 4096;
-    for (int i = 0; i < x.ndim - 2; i++) fine = fine && x.shape[i] == y.shape[i];
-    if (fine) {
-      PyObject *sx = ((Tensor *)a[0])->shape, *sy = ((Tensor *)a[1])->shape, *shape = PyTuple_New(x.ndim);
+    /* rows that take no padded pitch; a batch extent is the larger one, as the library checks it */
+    if (x.ndim >= 2 && y.ndim >= 2 && y.shape[y.ndim - 1] < 4096) {
+      PyObject *sx = ((Tensor *)a[0])->shape, *sy = ((Tensor *)a[1])->shape;
+      const int nd = x.ndim > y.ndim ? x.ndim : y.ndim;
+      PyObject *shape = PyTuple_New(nd);
       if (!shape) return NULL;
-      for (int i = 0; i < x.ndim; i++) {
-        PyObject *e = i + 1 < x.ndim ? PyTuple_GET_ITEM(sx, i) : PyTuple_GET_ITEM(sy, i);
+      for (int i = 0; i < nd; i++) {
+        const int ix = i - (nd - x.ndim), iy = i - (nd - y.ndim);
+        PyObject *e = i == nd - 2   ? PyTuple_GET_ITEM(sx, ix)
+                      : i == nd - 1 ? PyTuple_GET_ITEM(sy, iy)
+                      : ix < 0      ? PyTuple_GET_ITEM(sy, iy)
+                      : iy < 0 || x.shape[ix] >= y.shape[iy] ? PyTuple_GET_ITEM(sx, ix) : PyTuple_GET_ITEM(sy, iy);
         Py_INCREF(e);
         PyTuple_SET_ITEM(shape, i, e);
       }
@@ -653,6 +777,12 @@ static PyMethodDef calls_methods[] = {
      "full($self, dtype, shape, value)\n--\n\nEvery element is ``value`` (a Python number, or one already-encoded storage element as a numpy array)."},
     {"reduce", (PyCFunction)(void (*)(void))calls_reduce, FAST, "reduce($self, op, axes, x)\n--\n\n"},
     {"matmul", (PyCFunction)(void (*)(void))calls_matmul, FAST, "matmul($self, x, y)\n--\n\n"},
+    {"broadcast_binary", (PyCFunction)(void (*)(void))calls_broadcast_binary, FAST,
+     "broadcast_binary($self, op, x, y)\n--\n\nbinary of operands broadcast together; NotImplemented where that is out of the ordinary."},
+    {"broadcast_where", (PyCFunction)(void (*)(void))calls_broadcast_where, FAST,
+     "broadcast_where($self, cond, if_true, if_false)\n--\n\nwhere, likewise."},
+    {"reduce_keep", (PyCFunction)(void (*)(void))calls_reduce_keep, FAST,
+     "reduce_keep($self, op, axes, x)\n--\n\nreduce whose reduced axes (ascending) stay as dims of extent 1; NotImplemented likewise."},
     {NULL, NULL, 0, NULL}};
 static PyGetSetDef calls_getset[] = {{"_h", (getter)calls_get_h, (setter)calls_set_h, NULL, NULL}, {NULL, NULL, NULL, NULL, NULL}};
 static PyTypeObject CallsType = {

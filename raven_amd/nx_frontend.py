@@ -15,7 +15,7 @@ from typing import Sequence
 import numpy as np
 
 from . import dtype as dt
-from .nx_backend import encode_scalar
+from .nx_backend import Backend, encode_scalar
 
 
 _BROADCAST: dict = {}  # (shape, shape) -> what they broadcast to
@@ -48,11 +48,27 @@ def _broadcast_unequal(a: tuple, b: tuple) -> tuple:
 _ENCODED: dict = {}  # (dtype name, Python value) -> its encoded storage element
 
 
+def _left(*operands):
+    return NotImplemented
+
+
+def _in_one_call(backend, name, steps):
+    """The call of the device backend that makes several steps one (nx_calls.c), where all of them are the device
+    backend's own; elsewhere (another backend, one that wraps it or changes a step) nothing is taken together."""
+    cls = type(backend)
+    if isinstance(backend, Backend) and all(getattr(cls, s) is getattr(Backend, s) and s not in vars(backend) for s in steps):
+        return getattr(backend, name)
+    return _left
+
+
 class Nx:
     """Frontend functions bound to one backend."""
 
     def __init__(self, backend):
         self.B = backend
+        self._broadcast_binary = _in_one_call(backend, "broadcast_binary", ("reshape", "expand", "binary"))
+        self._broadcast_where = _in_one_call(backend, "broadcast_where", ("reshape", "expand", "where"))
+        self._reduce_keep = _in_one_call(backend, "reduce_keep", ("reshape", "reduce"))
 
     # ── creation ────────────────────────────────────────────────────────────
     def create(self, dtype: dt.DType, shape, host: np.ndarray):
@@ -116,8 +132,11 @@ class Nx:
 
     # ── elementwise (frontend.ml:417-534) ───────────────────────────────────
     def _binop(self, op, a, b):
-        a, b = self.broadcasted(a, b)
-        return self.B.binary(op, a, b)
+        r = self._broadcast_binary(op, a, b)
+        if r is NotImplemented:
+            a, b = self.broadcasted(a, b)
+            r = self.B.binary(op, a, b)
+        return r
 
     def add(self, a, b):
         return self._binop("add", a, b)
@@ -143,6 +162,9 @@ class Nx:
 
     def where(self, cond, if_true, if_false):
         """frontend.ml:612-618."""
+        r = self._broadcast_where(cond, if_true, if_false)
+        if r is not NotImplemented:
+            return r
         s = _broadcast_shapes(_broadcast_shapes(if_true.shape, if_false.shape), cond.shape)
         return self.B.where(self.broadcast_to(s, cond), self.broadcast_to(s, if_true),
                             self.broadcast_to(s, if_false))
@@ -163,7 +185,11 @@ class Nx:
     # ── reductions (frontend.ml:642-708) ────────────────────────────────────
     def _reduce(self, op, x, axes, keepdims):
         r = len(x.shape)
-        axes = sorted(a % r for a in axes)
+        axes = sorted([a % r for a in axes])
+        if keepdims:
+            out = self._reduce_keep(op, axes, x)
+            if out is not NotImplemented:
+                return out
         out = self.B.reduce(op, axes, x)
         if keepdims:
             out = self.B.reshape(out, tuple(1 if i in axes else s for i, s in enumerate(x.shape)))
