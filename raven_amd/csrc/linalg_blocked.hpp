@@ -42,6 +42,14 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// A value that is there before what follows is chosen: keeps the compiler from turning a choice between two short
+// computations, or the loading of one operand, into a branch of the wave and a wait behind it.
+__device__ __forceinline__ double at_hand(double v) {
+  asm("" : "+v"(v));
+  return v;
+}
+__device__ __forceinline__ c64 at_hand(c64 v) { return v; }
+
 // sqrt(d) and 1 / sqrt(d) of a positive d, each to the last bit or next to it: one hardware
 // estimate and Newton steps on d scaled into [1/4, 1). The chain of the factorisation runs
 // through this once per column; the library's square root and division are four times as long.
@@ -641,16 +649,21 @@ __global__ __launch_bounds__(256) void cholesky_result_kernel(CholArgs<T> a) {
 // transpose). A workgroup solves sixteen right-hand sides, which stay in LDS, sixteen rows a
 // step: wave 0 brings the next sixteen rows up to date and substitutes through their
 // triangle (solve16), while other waves take the step before from the rows further down (a
-// wave per 16 x 16 tile) and one inverts the 4 x 4 triangles of the next step. What is read
+// wave per 16 x 16 tile) and one lays out what wave 0 needs of the matrix for the next step. What is read
 // of the matrix is requested a step or two ahead: it depends on nothing. One barrier a step, no launch.
 // Where solve16 refuses, and for complex matrices, the substitution goes row by row, a right-hand
 // side a lane.
-// Wave 0 is the chain, wave 4 (of its SIMD) reads and inverts triangles, which takes no matrix
-// instructions from it, the other six bring up to TILES tiles each up to date per step. What a tile needs
+// Wave 0 is the chain: it neither reads memory nor works out an address. Wave 4 (of its SIMD) reads the triangle and
+// the tile left of it, inverts the 4 x 4 triangles and puts all of it in LDS as the operands that wave 0 takes, without
+// a matrix instruction; the other six bring up to TILES tiles each up to date per step, up to six at a time, so that
+// their products do not wait for each other. What a tile needs
 // of the matrix is in registers two steps ahead, so that TILES decides how many workgroups a compute unit
-// holds (float64: 11 tiles 208 registers, one; 2 tiles 128, two). Eleven make a pass of 64 blocks; systems of
+// holds (11 tiles one, 2 tiles two). Eleven make a pass of 64 blocks; systems of
 // 2 + 6 TILES blocks and fewer take two; those of one block, TILES = 0, a single wave, which places
 // the triangle itself.
+// [512,512] float32, sixteen sides: 74 us while wave 0 took 3 400 clocks a step (0.6 the tile to the left in one chain, 0.7
+// addresses and conversions, 2.0 solve16) and waited for the others, tile after tile, up to 6 400; 62 so, 3 000 a step but for the first ten, whose products keep the matrix units busy.
+// (The 4 x 4 triangles row by row on the vector unit, four products in the chain for fifteen: 2.3 for solve16's 2.0.)
 constexpr int TRSM_WAVES = 8, TRSM_LOADER = 4, TRSM_UPDATERS = 6, TRSM_TILES = 11, TRSM_FEW = 2;
 template <int TILES>
 constexpr int TRSM_THREADS = TILES > 0 ? 64 * TRSM_WAVES : 64;
@@ -693,7 +706,9 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
   // 16 (double) the inverse of the diagonal (reads past a column's end meet the next one: their results are dropped)
   constexpr int TRI_LD = 18;
   __shared__ T tri[AHEAD][17][TRI_LD];
-  __shared__ double diag_inv[AHEAD][4][64];  // operands of solve16, zero outside the 4 x 4 triangles
+  constexpr int REAL = sizeof(T) == 8 ? AHEAD : 1;      // (complex has none of these)
+  __shared__ double diag_inv[REAL][4][64], op_tri[REAL][4][64];  // operands of solve16, the first zero outside the 4 x 4 triangles
+  __shared__ double op_left[REAL][4][64];               // the tile to the left of the triangle
   __shared__ int singular;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
   const int n = a.rows, nb = (n + 15) / 16, col0 = blockIdx.x * 16;
@@ -707,38 +722,49 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
   if (threadIdx.x == 0) singular = 0;
   // the triangle of block `k` and the inverses of its diagonal (past n: the identity), by one wave
   auto fetch_triangle = [&](int k, TS(&raw)[4]) {
+    const int last = min(15, n - 1 - k * 16);
+    const TS *p = m + k * 16 * (a.ts + a.us) + min(r16, last) * a.us;
 #pragma unroll
-    for (int v = 0; v < 4; v++) raw[v] = m[min(k * 16 + 4 * v + q, n - 1) * a.ts + min(k * 16 + r16, n - 1) * a.us];
+    for (int v = 0; v < 4; v++) raw[v] = p[min(4 * v + q, last) * a.ts];
   };
   auto place_triangle = [&](int k, const TS(&raw)[4]) {
+    T own = S::make(1.0, 0.0);  // the diagonal element of a lane that has one
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       const int t = 4 * v + q;
       const bool diagonal = t == r16;
-      T val = a.conj ? S::conj(T(raw[v])) : T(raw[v]);
-      if (k * 16 + max(t, r16) >= n || r16 > t || (a.unit && diagonal)) val = S::make(diagonal ? 1.0 : 0.0, 0.0);
+      T val = at_hand(a.conj ? S::conj(T(raw[v])) : T(raw[v]));
+      const T edge = S::make(diagonal ? 1.0 : 0.0, 0.0);
+      val = k * 16 + max(t, r16) >= n || r16 > t || (a.unit && diagonal) ? edge : val;
       if (r16 <= t) tri[k % AHEAD][r16][t - r16] = val;
-      if (diagonal) {
-        if (val == S::make(0.0, 0.0)) singular = 1;
-        if constexpr (sizeof(T) == 8) tri[k % AHEAD][t][16] = 1.0 / val;
-      }
+      own = diagonal ? val : own;
     }
+    if (own == S::make(0.0, 0.0)) singular = 1;
     if constexpr (sizeof(T) == 8) {
+      const double inverse = at_hand(1.0 / at_hand(own));
+      if ((r16 & 3) == q) tri[k % AHEAD][r16][16] = inverse;
       // lane (b, i, j): element (i, j) of the inverse of the b-th 4 x 4 triangle on the diagonal
-      __builtin_amdgcn_wave_barrier();
+      wave_sync();
       const int bb = lane >> 4, i = (lane >> 2) & 3, j = lane & 3;
       const T(*t)[TRI_LD] = &tri[k % AHEAD][4 * bb];
-      const double e0 = t[0][16], e1 = t[1][16], e2 = t[2][16], e3 = t[3][16];
-      const double m10 = -e1 * t[0][1] * e0, m21 = -e2 * t[1][1] * e1, m32 = -e3 * t[2][1] * e2;
-      const double m20 = -e2 * fma(t[1][1], m10, t[0][2] * e0), m31 = -e3 * fma(t[2][1], m21, t[1][2] * e1);
-      const double m30 = -e3 * fma(t[2][1], m20, fma(t[1][2], m10, t[0][3] * e0));
-      double v = i == 0 ? e0 : i == 1 ? (j == 0 ? m10 : e1) : i == 2 ? (j == 0 ? m20 : j == 1 ? m21 : e2)
-                                                                     : (j == 0 ? m30 : j == 1 ? m31 : j == 2 ? m32 : e3);
-      v = j <= i ? v : 0.0;
-      diag_inv[k % AHEAD][bb][j * 16 + 4 * bb + i] = v;
+      double column[4];  // of the operand of a product with the triangle
+#pragma unroll
+      for (int u = 0; u < 4; u++) column[u] = at_hand(tri[k % AHEAD][4 * u + q][max(r16 - 4 * u - q, 0)]);
+      const double e0 = at_hand(t[0][16]), e1 = at_hand(t[1][16]), e2 = at_hand(t[2][16]), e3 = at_hand(t[3][16]);
+      const double l10 = at_hand(t[0][1]), l20 = at_hand(t[0][2]), l30 = at_hand(t[0][3]), l21 = at_hand(t[1][1]), l31 = at_hand(t[1][2]), l32 = at_hand(t[2][1]);
+      const double m10 = at_hand(-e1 * l10 * e0), m21 = at_hand(-e2 * l21 * e1), m32 = at_hand(-e3 * l32 * e2);
+      const double m20 = at_hand(-e2 * fma(l21, m10, l20 * e0)), m31 = at_hand(-e3 * fma(l32, m21, l31 * e1));
+      const double m30 = at_hand(-e3 * fma(l32, m20, fma(l31, m10, l30 * e0)));
+      double v = j == 0 ? m30 : j == 1 ? m31 : j == 2 ? m32 : e3;
+      v = i == 2 ? (j == 0 ? m20 : j == 1 ? m21 : e2) : v;
+      v = i == 1 ? (j == 0 ? m10 : e1) : v;
+      v = i == 0 ? e0 : v;
+      diag_inv[k % AHEAD][bb][j * 16 + 4 * bb + i] = j <= i ? v : 0.0;
+#pragma unroll
+      for (int u = 0; u < 4; u++) op_tri[k % AHEAD][u][lane] = r16 >= 4 * u + q ? column[u] : 0.0;
     }
   };
-  for (int e = threadIdx.x; e < AHEAD * 256; e += blockDim.x) (&diag_inv[0][0][0])[e] = 0.0;
+  for (int e = threadIdx.x; e < REAL * 256; e += blockDim.x) (&diag_inv[0][0][0])[e] = 0.0;
   // One matrix (`report`): a wave that has nothing to do yet looks through its diagonal, and the host goes on.
   if (a.failure.report && blockIdx.x == 0 && blockIdx.y == 0 && wave == (TILES > 0 ? TRSM_WAVES - 1 : 0)) {
     bool zero = false;
@@ -756,13 +782,6 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
     if (lane == 0) nxh_report(a.failure.report, a.failure.seq, zero ? LA_SINGULAR : LA_OK);
   }
   __syncthreads();
-  TS raw[2][4];
-  if (TILES == 0 || wave == TRSM_LOADER) {
-    fetch_triangle(0, raw[0]);
-    if (TILES > 0) fetch_triangle(1, raw[1]);
-    place_triangle(0, raw[0]);
-    if (TILES > 0) fetch_triangle(2, raw[0]);
-  }
   // coefficients of tile `t` against block `u`, as the matrix instruction takes them
   const TS *lane_full = m + r16 * a.ts + q * a.us, *lane_last = m + min(r16, n - 1 - (nb - 1) * 16) * a.ts + q * a.us;
   auto coefficients = [&](int t, int u, TS(&c)[4]) {
@@ -804,32 +823,70 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
       }
     }
   };
+  // The tile to the left of block k's triangle, k > 0 (real only). Nothing the loader does depends on a branch: behind one,
+  // a wait for loads is a wait for all of them, also those of the step just before.
+  auto fetch_left = [&](int k, TS(&c)[4]) {
+    if constexpr (sizeof(T) == 8) {
+      const TS *p = (k == nb - 1 ? lane_last : lane_full) + (k * a.ts + (k - 1) * a.us) * 16;
+#pragma unroll
+      for (int v = 0; v < 4; v++) c[v] = p[4 * v * a.us];
+    }
+  };
+  auto place_left = [&](int k, const TS(&c)[4]) {
+    if constexpr (sizeof(T) == 8) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) op_left[k % AHEAD][v][lane] = (double)c[v];
+    }
+  };
+  TS raw[2][4], left[2][4];
+  if (TILES == 0 || wave == TRSM_LOADER) {
+    fetch_triangle(0, raw[0]);
+    if constexpr (TILES > 0) fetch_left(1, left[1]), fetch_triangle(1, raw[1]);
+    place_triangle(0, raw[0]);
+    if constexpr (TILES > 0) fetch_left(min(2, nb - 1), left[0]), fetch_triangle(min(2, nb - 1), raw[0]);
+  }
   __syncthreads();
   // Three loops with the same barriers: the registers of one role are not the others'. What is read of
   // the matrix is needed two steps later and has two sets of registers in turn (a copy from one
   // to the other would wait for it): the first pass over it comes from beyond the L2, some 3500
   // cycles away.
   if (TILES == 0 || wave == 0) {
-    TS left[2][4], on[2][4];  // of the tile left of the triangle, and of the triangle
-    auto step = [&](int k, TS(&cl)[4], TS(&co)[4]) {
+    LaTile<T> before;    // the rows solved last,
+    bool known = false;  // where they are
+    auto step = [&](int k) {
       LaTile<T> acc = load_rows(k);
-      if (k > 0) take(acc, k, k - 1, cl);
-      if (k + 2 < nb) coefficients(k + 2, k + 1, cl);
       if constexpr (sizeof(T) == 8) {
-        double tr[4];
+        double di[4], tr[4];
+        if (k > 0) {  // what the tile to the left takes, in two chains and apart from acc
+          double l[4], x[4];
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int u = 4 * v + q;
-          tr[v] = r16 < u ? 0.0 : k * 16 + r16 >= n || (a.unit && r16 == u) ? (r16 == u ? 1.0 : 0.0) : (double)co[v];
+          for (int v = 0; v < 4; v++) l[v] = op_left[k % AHEAD][v][lane], x[v] = before.v[v];
+          if (!known) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) x[v] = X[((k - 1) * 16 + 4 * v + q) * 16 + r16];
+          }
+          const la_f64x4 zero = {0.0, 0.0, 0.0, 0.0};
+          la_f64x4 even = __builtin_amdgcn_mfma_f64_16x16x4f64(l[0], x[0], zero, 0, 0, 0);
+          la_f64x4 odd = __builtin_amdgcn_mfma_f64_16x16x4f64(l[1], x[1], zero, 0, 0, 0);
+          even = __builtin_amdgcn_mfma_f64_16x16x4f64(l[2], x[2], even, 0, 0, 0);
+          odd = __builtin_amdgcn_mfma_f64_16x16x4f64(l[3], x[3], odd, 0, 0, 0);
+#pragma unroll
+          for (int v = 0; v < 4; v++) di[v] = diag_inv[k % AHEAD][v][lane], tr[v] = op_tri[k % AHEAD][v][lane];
+#pragma unroll
+          for (int v = 0; v < 4; v++) acc.v[v] -= even[v] + odd[v];
+        } else {
+#pragma unroll
+          for (int v = 0; v < 4; v++) di[v] = diag_inv[k % AHEAD][v][lane], tr[v] = op_tri[k % AHEAD][v][lane];
         }
-        if (k + 2 < nb) coefficients(k + 2, k + 2, co);
-        double di[4];
-#pragma unroll
-        for (int v = 0; v < 4; v++) di[v] = diag_inv[k % AHEAD][v][lane];
-        if (solve16(acc, di, tr)) {
+        known = solve16(acc, di, tr);
+        if (known) {
           store_rows(k, acc);
+          before = acc;
           return;
         }
+      } else {
+        TS none[4];
+        if (k > 0) take(acc, k, k - 1, none);
       }
       store_rows(k, acc);
       __builtin_amdgcn_wave_barrier();
@@ -845,28 +902,22 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
         for (int r = 1; r < 16; r++) v[r - 1] = S::sub_mul(v[r], t16[t][r], sol);
       }
     };
-    coefficients(0, 0, on[0]);
-    if (nb > 1) coefficients(1, 0, left[1]), coefficients(1, 1, on[1]);
 #pragma unroll 1
-    for (int k = 0; k < nb; k += 2) {
-      step(k, left[0], on[0]);
+    for (int k = 0; k < nb; k++) {
+      step(k);
       __syncthreads();
-      if (k + 1 < nb) {
-        step(k + 1, left[1], on[1]);
-        __syncthreads();
-      }
     }
   } else if (wave == TRSM_LOADER) {
-    auto step = [&](int k, TS(&r)[4]) {
-      if (k + 1 < nb) place_triangle(k + 1, r);
-      if (k + 3 < nb) fetch_triangle(k + 3, r);
+    auto step = [&](int k, TS(&r)[4], TS(&l)[4]) {
+      place_left(k + 1, l), place_triangle(k + 1, r);  // (past the last: the identity, for nobody)
+      fetch_left(min(k + 3, nb - 1), l), fetch_triangle(min(k + 3, nb - 1), r);
     };
 #pragma unroll 1
     for (int k = 0; k < nb; k += 2) {
-      step(k, raw[1]);
+      step(k, raw[1], left[1]);
       __syncthreads();
       if (k + 1 < nb) {
-        step(k + 1, raw[0]);
+        step(k + 1, raw[0], left[0]);
         __syncthreads();
       }
     }
@@ -877,11 +928,56 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
 #pragma unroll
       for (int i = 0; i < TILES; i++) {
         const int t = k + first + i * TRSM_UPDATERS;
-        if (t < nb) coefficients(t, k - 1, to[i]);
+        if (t >= nb) break;
+        coefficients(t, k - 1, to[i]);
+      }
+    };
+    // G tiles from tile t on, every TRSM_UPDATERS: their rows less what the solved block x takes from them (coefficients: from)
+    auto tiles = [&](auto g_c, int t, const double(&x)[4], const TS(*from)[4]) {
+      constexpr int G = decltype(g_c)::value;
+      if constexpr (sizeof(T) == 8) {
+        la_f64x4 d[G];
+#pragma unroll
+        for (int i = 0; i < G; i++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) d[i][v] = X[((t + i * TRSM_UPDATERS) * 16 + 4 * v + q) * 16 + r16];
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+#pragma unroll
+          for (int i = 0; i < G; i++) d[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(-(double)from[i][v], x[v], d[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < G; i++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) X[((t + i * TRSM_UPDATERS) * 16 + 4 * v + q) * 16 + r16] = d[i][v];
       }
     };
     auto step = [&](int k, TS(&from)[TILES][4]) {
-      if (k > 0) {
+      if constexpr (sizeof(T) == 8) {
+        if (k > 0) {
+          double x[4];
+#pragma unroll
+          for (int v = 0; v < 4; v++) x[v] = X[((k - 1) * 16 + 4 * v + q) * 16 + r16];
+          constexpr int MOST = TILES < 6 ? TILES : 6;
+#pragma unroll
+          for (int i = 0; i < TILES; i += MOST) {
+            const int t = k + first + i * TRSM_UPDATERS;
+            if (t >= nb) break;
+            const int more = min((nb - 1 - t) / TRSM_UPDATERS + 1, min(TILES - i, MOST));
+            const auto some = [&](auto g_c) {
+              constexpr int G = decltype(g_c)::value;
+              if constexpr (G <= MOST && (TILES % MOST == 0 || G <= TILES)) tiles(g_c, t, x, &from[i]);
+            };
+            switch (more) {
+              case 1: some(std::integral_constant<int, 1>{}); break;
+              case 2: some(std::integral_constant<int, 2>{}); break;
+              case 3: some(std::integral_constant<int, 3>{}); break;
+              case 4: some(std::integral_constant<int, 4>{}); break;
+              case 5: some(std::integral_constant<int, 5>{}); break;
+              default: some(std::integral_constant<int, 6>{}); break;
+            }
+          }
+        }
+      } else if (k > 0) {
 #pragma unroll
         for (int i = 0; i < TILES; i++) {
           const int t = k + first + i * TRSM_UPDATERS;
