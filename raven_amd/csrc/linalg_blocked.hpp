@@ -50,18 +50,25 @@ __device__ __forceinline__ double at_hand(double v) {
 }
 __device__ __forceinline__ c64 at_hand(c64 v) { return v; }
 
-// sqrt(d) and 1 / sqrt(d) of a positive d, each to the last bit or next to it: one hardware
-// estimate and Newton steps on d scaled into [1/4, 1). The chain of the factorisation runs
-// through this once per column; the library's square root and division are four times as long.
+// sqrt(d) and 1 / sqrt(d) of a positive d far from the ends of the exponents, each to the last bit or next to it: one
+// hardware estimate and Newton steps. The chain of the factorisation runs through this once per column; the library's
+// square root and division are four times as long, and scaling d first a good tenth of the chain (sixteen columns of
+// [512,512] f32: 6 350 clocks scaled, 5 690 so; 28.3 us a launch -> 27.5).
+__device__ __forceinline__ void plain_root_and_inverse(double d, double *root, double *inv) {
+  double r = __builtin_amdgcn_rsq(d);
+  const double err = fma(-(d * r), r, 1.0);
+  r = fma(r * err, fma(0.375, err, 0.5), r);
+  double l = d * r;
+  l = fma(fma(-l, l, d), 0.5 * r, l);
+  r = fma(fma(-l, r, 1.0), r, r);
+  *root = l;
+  *inv = r;
+}
+// The same of any positive d, scaled into [1/4, 1) by a power of four, which changes no digit.
 __device__ __forceinline__ void root_and_inverse(double d, double *root, double *inv) {
   const int e = (__builtin_amdgcn_frexp_exp(d) + 1) >> 1;
-  const double ds = ldexp(d, -2 * e);
-  double r = __builtin_amdgcn_rsq(ds);
-  const double err = fma(-(ds * r), r, 1.0);
-  r = fma(r * err, fma(0.375, err, 0.5), r);
-  double l = ds * r;
-  l = fma(fma(-l, l, ds), 0.5 * r, l);
-  r = fma(fma(-l, r, 1.0), r, r);
+  double l, r;
+  plain_root_and_inverse(ldexp(d, -2 * e), &l, &r);
   *root = d < __builtin_inf() ? ldexp(l, e) : d;
   *inv = d < __builtin_inf() ? ldexp(r, -e) : 0.0;
 }
@@ -77,14 +84,30 @@ struct LaTile {
 // pointers, as sums of four terms that meet pairwise; tile_sub takes it from acc. So there is one
 // rounding at the size of acc per call and not one per term (one chain of fused steps from acc left a
 // Gram matrix of 256 columns with four times the backward error, 0.30 against 0.07 eps).
+// Up to eight products are under way before the first is added: left to itself, the compiler waits for each of them,
+// some 140 clocks, and for its operands ([512,512] f32: the sums of a block column's last rows 470 clocks -> 260, those ahead
+// of its diagonal tile, which the matrix units bound, 7 700 -> 7 350).
 template <int K>
 __device__ __forceinline__ la_f64x4 tile_sum(const double *A, int64_t lda, const double *B, int64_t ldb) {
-  if constexpr (K > 4) {
+  if constexpr (K > 32) {
     const la_f64x4 low = tile_sum<K / 2>(A, lda, B, ldb);
     return low + tile_sum<K / 2>(A + K / 2, lda, B + K / 2, ldb);
   } else {
+    constexpr int N = K / 4;
     const int lane = threadIdx.x & 63, at = lane >> 4;
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(A[(lane & 15) * lda + at], B[(lane & 15) * ldb + at], la_f64x4{0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
+    double x[N], y[N];
+    la_f64x4 p[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) x[i] = A[(lane & 15) * lda + 4 * i + at], y[i] = B[(lane & 15) * ldb + 4 * i + at];
+    if constexpr (N > 4) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < N; i++) p[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i], y[i], la_f64x4{0.0, 0.0, 0.0, 0.0}, 0, 0, 0);
+    if constexpr (N > 4) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d = 1; d < N; d *= 2)
+#pragma unroll
+      for (int i = 0; i + d < N; i += 2 * d) p[i] = p[i] + p[i + d];
+    return p[0];
   }
 }
 template <int K>
@@ -169,7 +192,7 @@ __device__ __forceinline__ bool solve16(LaTile<double> &acc, const double (&diag
 // element, the matrix instruction does the rest. The tile is acc - before; what its own columns take is
 // summed beside `before`, so that an element of a diagonal block rounds once at its own size.
 // Leaves the operands of solve16 in diag_inv and tri; tri is the factor itself. `blk`: 64 places of LDS.
-// False where that is not the factor: a pivot that is not positive or not finite, or a step as in solve16.
+// False where that is not the factor: a pivot that is not positive or near the ends of the exponents, or a step as in solve16.
 __device__ __forceinline__ bool factor16(const LaTile<double> &acc, la_f64x4 before, double2 *blk, double (&diag_inv)[4], double (&tri)[4]) {
   const int lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
   const la_f64x4 zero = {0.0, 0.0, 0.0, 0.0};
@@ -195,8 +218,8 @@ __device__ __forceinline__ bool factor16(const LaTile<double> &acc, la_f64x4 bef
     for (int j = 0; j < 4; j++) {
 #pragma unroll
       for (int i = j; i < 4; i++) low[j][i] = a[j][i] - (j > 0 ? sum[j][i] + own[j][i] : sum[j][i]);
-      good = good && low[j][j] > 0.0 && low[j][j] < __builtin_inf();
-      root_and_inverse(low[j][j], &low[j][j], &root[j]);
+      good = good && low[j][j] > 0x1p-900 && low[j][j] < 0x1p900;
+      plain_root_and_inverse(low[j][j], &low[j][j], &root[j]);
 #pragma unroll
       for (int i = j + 1; i < 4; i++) low[j][i] *= root[j];
 #pragma unroll
@@ -238,7 +261,7 @@ __device__ __forceinline__ bool factor16(const LaTile<double> &acc, la_f64x4 bef
 }
 
 // The same column by column, in place on the lower triangle (the rest becomes 0), for what factor16
-// refuses: pivots that are infinite, tiles close to singular; a failure shows here. 1 / L_cc goes to
+// refuses: pivots that are infinite or near it, or next to zero, tiles close to singular; a failure shows here. 1 / L_cc goes to
 // the place that lane (q, c) of diag_inv[c / 4], q = c % 4, has in `inv`.
 __device__ __forceinline__ bool factor16_columns(double *tile, int ld, double *inv) {
   const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
@@ -782,18 +805,13 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
     if (lane == 0) nxh_report(a.failure.report, a.failure.seq, zero ? LA_SINGULAR : LA_OK);
   }
   __syncthreads();
-  // coefficients of tile `t` against block `u`, as the matrix instruction takes them
+  // coefficients of tile `t` against block `u` < `t`, as the matrix instruction takes them
   const TS *lane_full = m + r16 * a.ts + q * a.us, *lane_last = m + min(r16, n - 1 - (nb - 1) * 16) * a.ts + q * a.us;
   auto coefficients = [&](int t, int u, TS(&c)[4]) {
     if constexpr (sizeof(T) == 8) {
       const TS *p = (t == nb - 1 ? lane_last : lane_full) + (t * a.ts + u * a.us) * 16;
-      if (u == nb - 1) {  // the last triangle: nothing is read past its columns
 #pragma unroll
-        for (int k = 0; k < 4; k++) c[k] = p[(min(4 * k + q, n - 1 - u * 16) - q) * a.us];
-      } else {
-#pragma unroll
-        for (int k = 0; k < 4; k++) c[k] = p[4 * k * a.us];
-      }
+      for (int k = 0; k < 4; k++) c[k] = p[4 * k * a.us];
     }
   };
   auto load_rows = [&](int t) {
@@ -806,15 +824,9 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
 #pragma unroll
     for (int v = 0; v < 4; v++) X[(t * 16 + 4 * v + q) * 16 + r16] = acc.v[v];
   };
-  // what block `u` takes from block `t`, whose coefficients are in `c`
-  auto take = [&](LaTile<T> &acc, int t, int u, const TS(&c)[4]) {
-    if constexpr (sizeof(T) == 8) {
-      la_f64x4 d = {acc.v[0], acc.v[1], acc.v[2], acc.v[3]};
-#pragma unroll
-      for (int k = 0; k < 4; k++) d = __builtin_amdgcn_mfma_f64_16x16x4f64(-(double)c[k], X[(u * 16 + 4 * k + q) * 16 + r16], d, 0, 0, 0);
-#pragma unroll
-      for (int v = 0; v < 4; v++) acc.v[v] = d[v];
-    } else {
+  // what block `u` takes from block `t` (complex)
+  auto take = [&](LaTile<T> &acc, int t, int u) {
+    if constexpr (sizeof(T) != 8) {
       for (int k = 0; k < 16; k++) {
         const T xv = X[(u * 16 + k) * 16 + r16];
 #pragma unroll
@@ -823,15 +835,8 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
       }
     }
   };
-  // The tile to the left of block k's triangle, k > 0 (real only). Nothing the loader does depends on a branch: behind one,
+  // The tile to the left of block k's triangle (real only). Nothing the loader does depends on a branch: behind one,
   // a wait for loads is a wait for all of them, also those of the step just before.
-  auto fetch_left = [&](int k, TS(&c)[4]) {
-    if constexpr (sizeof(T) == 8) {
-      const TS *p = (k == nb - 1 ? lane_last : lane_full) + (k * a.ts + (k - 1) * a.us) * 16;
-#pragma unroll
-      for (int v = 0; v < 4; v++) c[v] = p[4 * v * a.us];
-    }
-  };
   auto place_left = [&](int k, const TS(&c)[4]) {
     if constexpr (sizeof(T) == 8) {
 #pragma unroll
@@ -841,9 +846,9 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
   TS raw[2][4], left[2][4];
   if (TILES == 0 || wave == TRSM_LOADER) {
     fetch_triangle(0, raw[0]);
-    if constexpr (TILES > 0) fetch_left(1, left[1]), fetch_triangle(1, raw[1]);
+    if constexpr (TILES > 0) coefficients(1, 0, left[1]), fetch_triangle(1, raw[1]);
     place_triangle(0, raw[0]);
-    if constexpr (TILES > 0) fetch_left(min(2, nb - 1), left[0]), fetch_triangle(min(2, nb - 1), raw[0]);
+    if constexpr (TILES > 0) coefficients(min(2, nb - 1), min(2, nb - 1) - 1, left[0]), fetch_triangle(min(2, nb - 1), raw[0]);
   }
   __syncthreads();
   // Three loops with the same barriers: the registers of one role are not the others'. What is read of
@@ -885,8 +890,7 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
           return;
         }
       } else {
-        TS none[4];
-        if (k > 0) take(acc, k, k - 1, none);
+        if (k > 0) take(acc, k, k - 1);
       }
       store_rows(k, acc);
       __builtin_amdgcn_wave_barrier();
@@ -910,7 +914,8 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
   } else if (wave == TRSM_LOADER) {
     auto step = [&](int k, TS(&r)[4], TS(&l)[4]) {
       place_left(k + 1, l), place_triangle(k + 1, r);  // (past the last: the identity, for nobody)
-      fetch_left(min(k + 3, nb - 1), l), fetch_triangle(min(k + 3, nb - 1), r);
+      const int ahead = min(k + 3, nb - 1);
+      coefficients(ahead, ahead - 1, l), fetch_triangle(ahead, r);
     };
 #pragma unroll 1
     for (int k = 0; k < nb; k += 2) {
@@ -983,7 +988,7 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
           const int t = k + first + i * TRSM_UPDATERS;
           if (t < nb) {
             LaTile<T> acc = load_rows(t);
-            take(acc, t, k - 1, from[i]);
+            take(acc, t, k - 1);
             store_rows(t, acc);
           }
         }
