@@ -86,6 +86,14 @@ __device__ __forceinline__ float xor32(float v) {
   return __builtin_bit_cast(float, __shfl_xor(__builtin_bit_cast(int, v), 32, 64));
 }
 
+// Exchanges x of the wave's upper half with y of its lower half.
+__device__ __forceinline__ void swap_halves(float &x, float &y) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, y), false, false);
+  const uint32_t u = p[0], v = p[1];
+  x = __builtin_bit_cast(float, u);
+  y = __builtin_bit_cast(float, v);
+}
+
 template <class EL, int DHEAD, bool ONLINE>
 __global__ __launch_bounds__(128) void attention_kernel(AttArgs a) {
   using S = uint16_t;
@@ -434,17 +442,26 @@ __global__ __launch_bounds__(128) void attention_kernel(AttArgs a) {
 // reference, O = O_a 2^((m_a - m) c) + O_b 2^((m_b - m) c) and the same for the row sum, before
 // the one division. Rounding points are those of the two-wave form; only the f32 sums of the
 // output and of the row sum are added in another order.
-// (Asking the compiler for four waves per SIMD at head dim 64, 128 registers instead of the 136
-// it takes, changed nothing at batch 8 or 16: the kernel is bound by what it issues.)
+// What bounds it now is what a SIMD issues: 122 vector instructions and 16 exponentials a half tile,
+// 600 of some 1000 cycles, beside 256 of the matrix pipe. So: a register budget under which
+// the compiler keeps the sums in registers that vector instructions reach (it had them
+// in the other file, 80 moves a step); the exchanges with lane ^ 32 as register swaps instead of trips
+// through LDS; the reference's update behind a branch that most steps do not take; two stages for
+// heads of up to 64, one barrier a tile; four neighbouring mask bytes by one load. The results are
+// the same bits. Start -> now, us: [b,12,1024,64] bfloat16 causal, b = 1 / 2 / 4 / 8 / 16: 18.7 / 20.2 / 22.8 / 38.5
+// / 77 -> 15.8 / 17.5 / 20.4 / 33.8 / 61; without a mask, b = 8: 62.6 -> 55.5; a mask tensor, b = 4: 106 -> 41;
+// [8,12,1024,64] float16 causal 51.6 -> 46.6, [8,16,1000,32] 31.2 -> 28.0, [8,8,2048,128] 152 -> 142.
+// Four waves a SIMD (128 registers) against three: b = 16 61 against 67, b = 8 33.8 and 34.1.
 template <class EL, int DHEAD>
-__global__ __launch_bounds__(256) void attention_split_kernel(AttArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DHEAD <= 64 ? 4 : 2))) void attention_split_kernel(AttArgs a) {
   using S = uint16_t;
   constexpr int KSTEPS = DHEAD / 16, OT = DHEAD / 32, PK = DHEAD + 8, PV = DHEAD + 16, VPR = DHEAD / 8;
-  __shared__ __attribute__((aligned(16))) S Ks[KEYS * PK];
-  __shared__ __attribute__((aligned(16))) S Vs[KEYS * PV];
-  __shared__ float mrg[2][OT * 16 + 2][64];
+  constexpr int NBUF = DHEAD <= 64 ? 2 : 1, STAGE = KEYS * (PK + PV);
+  __shared__ __attribute__((aligned(16))) S stages[NBUF * STAGE];
+  float(*mrg)[OT * 16 + 2][64] = reinterpret_cast<float(*)[OT * 16 + 2][64]>(stages);  // (after the last tile)
+  static_assert(sizeof(float) * 2 * (OT * 16 + 2) * 64 <= sizeof(stages), "the odd waves' results fit the stages");
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c32 = lane & 31, g = lane >> 5;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c32 = lane & 31, g = lane >> 5;
   const int qh = wave >> 1, kh = wave & 1;
   const int64_t bid = blockIdx.x;
   const int tile = a.qtiles - 1 - (int)(bid / a.batches);  // late (long) tiles first
@@ -483,96 +500,128 @@ __global__ __launch_bounds__(256) void attention_split_kernel(AttArgs a) {
 #pragma unroll
     for (int e = 0; e < 16; e++) oacc[t][e] = 0.0f;
 
-  // t[e]: the unscaled score of key j0 + (e/4)*8 + g*4 + e%4 against query qi, -inf where masked
-  auto scores = [&](int j0, float (&t)[16], bool inner) {
-    f32x16 acc;
+  // where this lane reads its rows of K and V inside a stage
+  const int kr_at = (kh * 32 + c32) * PK + g * 8;
+  const int vs_at = KEYS * PK + (kh * 32 + g * 8 + ((lane & 15) >> 2)) * PV + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+  // The unscaled scores of keys j0 + (e/4)*8 + g*4 + e%4 against query qi, -inf where masked (the fill of this form)
+  auto scores = [&](const S *Ks, int j0, bool inner) {
+    f32x16 t;
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[e] = 0.0f;
-    const S *kr = Ks + (j0 % KEYS + c32) * PK + g * 8;
+    for (int e = 0; e < 16; e++) t[e] = 0.0f;
+    const S *kr = Ks + kr_at;
 #pragma unroll
     for (int s = 0; s < KSTEPS; s++) {
       const V16 kf = *reinterpret_cast<const V16 *>(kr + s * 16);
-      gemm_tile::mfma_step<EL>(acc, kf, qf[s]);
+      gemm_tile::mfma_step<EL>(t, kf, qf[s]);
     }
-    if (inner) {
+    if (inner) return t;
+    const int first = j0 + g * 4;
+    if (a.causal || !a.has_mask) {
+      const int last = (a.causal && qi < a.sk - 1 ? qi : a.sk - 1) - first;
 #pragma unroll
-      for (int e = 0; e < 16; e++) t[e] = acc[e];
-      return;
+      for (int e = 0; e < 16; e++) t[e] = (e >> 2) * 8 + (e & 3) <= last ? t[e] : -__builtin_inff();
+      return t;
+    }
+    int mrow = qrow;
+    asm volatile("" : "+v"(mrow));  // (the addresses of the rare forms are made where they are used and hold no registers)
+    const uint8_t *mr = M + (int64_t)mrow * a.mask.row;
+    if (a.mask_col == 1 && j0 + 32 <= a.sk) {  // four neighbouring keys of a lane are one load, of any alignment
+      typedef uint32_t u32a1 __attribute__((aligned(1)));
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const uint32_t four = *reinterpret_cast<const u32a1 *>(mr + first + q * 8);
+#pragma unroll
+        for (int e = 0; e < 4; e++) t[q * 4 + e] = (four >> (8 * e)) & 0xffu ? t[q * 4 + e] : -__builtin_inff();
+      }
+      return t;
     }
 #pragma unroll
     for (int e = 0; e < 16; e++) {
-      const int j = j0 + (e >> 2) * 8 + g * 4 + (e & 3);
-      bool keep = true;
-      if (a.causal) keep = j <= qi;
-      else if (a.has_mask) keep = M[(int64_t)qrow * a.mask.row + (int64_t)(j < a.sk ? j : a.sk - 1) * a.mask_col] != 0;
-      t[e] = keep && j < a.sk ? acc[e] : -__builtin_inff();  // (the fill of this form is -inf)
+      const int j = first + (e >> 2) * 8 + (e & 3);
+      const bool keep = mr[(int64_t)(j < a.sk ? j : a.sk - 1) * a.mask_col] != 0;
+      t[e] = keep && j < a.sk ? t[e] : -__builtin_inff();
     }
+    return t;
   };
 
-  constexpr int NV = KEYS * VPR / 256;
+  // A thread's vectors of a key tile: column vc of rows vr, vr + VS, ...
+  constexpr int NV = KEYS * VPR / 256, VS = 256 / VPR;
   static_assert(NV >= 1 && NV * 256 == KEYS * VPR, "whole vectors per lane");
+  const int vr = threadIdx.x / VPR, vc = (threadIdx.x % VPR) * 8;
   V16 kpre[NV], vpre[NV];
-  // this lane's vectors inside a key tile as element offsets from the tile's first row: a whole
-  // tile then costs one uniform base per operand and no address arithmetic per load
-  uint32_t koff[NV], voff[NV];
+  // from a tile's first row in bytes: a whole tile costs one uniform base per load and no address arithmetic
   const bool short_offsets = (int64_t)KEYS * a.k.row < ((int64_t)1 << 31) && (int64_t)KEYS * a.v.row < ((int64_t)1 << 31) &&
                              a.k.row >= 0 && a.v.row >= 0;
-#pragma unroll
-  for (int i = 0; i < NV; i++) {
-    const int v = threadIdx.x + i * 256;
-    const int r = v / VPR, c = (v % VPR) * 8;
-    koff[i] = (uint32_t)(r * a.k.row + c);
-    voff[i] = (uint32_t)(r * a.v.row + c);
-  }
+  const uint32_t koff = ((uint32_t)vr * (uint32_t)a.k.row + (uint32_t)vc) * 2u, voff = ((uint32_t)vr * (uint32_t)a.v.row + (uint32_t)vc) * 2u;
   auto prefetch = [&](int kt) {
     if (short_offsets && (kt + 1) * KEYS <= a.sk) {  // uniform: every key of the tile exists
-      const S *kb = K + (int64_t)kt * KEYS * a.k.row, *vb = V + (int64_t)kt * KEYS * a.v.row;
 #pragma unroll
       for (int i = 0; i < NV; i++) {
-        kpre[i] = *reinterpret_cast<const V16 *>(kb + koff[i]);
-        vpre[i] = *reinterpret_cast<const V16 *>(vb + voff[i]);
+        const int64_t row = (int64_t)kt * KEYS + i * VS;
+        kpre[i] = *reinterpret_cast<const V16 *>(reinterpret_cast<const char *>(K + row * a.k.row) + koff);
+        vpre[i] = *reinterpret_cast<const V16 *>(reinterpret_cast<const char *>(V + row * a.v.row) + voff);
       }
       return;
     }
+    int row = vr, col = vc;
+    asm volatile("" : "+v"(row), "+v"(col));
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-      const int v = threadIdx.x + i * 256;
-      const int r = v / VPR, c = (v % VPR) * 8;
-      int key = kt * KEYS + r;
+      int key = kt * KEYS + row + i * VS;
       key = key < a.sk ? key : a.sk - 1;
-      kpre[i] = *reinterpret_cast<const V16 *>(K + (int64_t)key * a.k.row + c);
-      vpre[i] = *reinterpret_cast<const V16 *>(V + (int64_t)key * a.v.row + c);
+      kpre[i] = *reinterpret_cast<const V16 *>(K + (int64_t)key * a.k.row + col);
+      vpre[i] = *reinterpret_cast<const V16 *>(V + (int64_t)key * a.v.row + col);
+    }
+    asm volatile("");  // (the two forms' loads stay two: merged, the first pays for the second's addresses)
+  };
+  const int lay_k = vr * PK + vc, lay_v = KEYS * PK + vr * PV + vc;
+  auto lay = [&](S *at) {
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+      *reinterpret_cast<V16 *>(at + lay_k + i * VS * PK) = kpre[i];
+      *reinterpret_cast<V16 *>(at + lay_v + i * VS * PV) = vpre[i];
     }
   };
   prefetch(0);
+  if constexpr (NBUF == 2) {
+    lay(stages);
+    if (ktiles > 1) prefetch(1);
+  }
+  // -m_run c2: +inf before the first score, where the exponentials take 0
+  float lim = __builtin_inff(), mc = 0.0f;
   for (int kt = 0; kt < ktiles; kt++) {
-    __syncthreads();  // the previous tile has been consumed
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-      const int v = threadIdx.x + i * 256;
-      const int r = v / VPR, c = (v % VPR) * 8;
-      *reinterpret_cast<V16 *>(Ks + r * PK + c) = kpre[i];
-      *reinterpret_cast<V16 *>(Vs + r * PV + c) = vpre[i];
+    __syncthreads();  // the tile before has been consumed (two stages: and this one is there)
+    const S *Ks = stages;
+    if constexpr (NBUF == 2) {
+      Ks += (kt & 1) * STAGE;
+      if (kt + 1 < ktiles) {
+        lay(stages + ((kt + 1) & 1) * STAGE);
+        if (kt + 2 < ktiles) prefetch(kt + 2);
+      }
+    } else {
+      lay(stages);
+      __syncthreads();
+      if (kt + 1 < ktiles) prefetch(kt + 1);
     }
-    __syncthreads();
-    if (kt + 1 < ktiles) prefetch(kt + 1);
     const int j0 = kt * KEYS + kh * 32;
     // nothing of this wave's half of the tile is visible to its queries
     if (j0 >= a.sk || (a.causal && j0 > qw + 31)) continue;
-    float t[16];
-    scores(j0, t, j0 + 32 <= a.sk && !a.has_mask && (!a.causal || j0 + 31 <= qw));
+    const f32x16 t = scores(Ks, j0, j0 + 32 <= a.sk && !a.has_mask && (!a.causal || j0 + 31 <= qw));
     float tm = t[0];
 #pragma unroll
     for (int e = 1; e < 16; e++) tm = __builtin_fmaxf(tm, t[e]);
-    tm = __builtin_fmaxf(tm, xor32(tm));  // this query's maximum over the half tile, both lane halves agree
-    // the reference follows the maximum lazily, as in the two-wave kernel
-    const bool first = m_run == -__builtin_inff();
-    const bool grow = tm > m_run && (first || __builtin_fmaf(tm, a.c2, -m_run * a.c2) > 8.0f);
-    const float m_new = grow ? tm : m_run;
-    const float m_ref = m_new == -__builtin_inff() ? 0.0f : m_new;
-    const float mc = -m_ref * a.c2;
-    const float alpha = grow ? __builtin_amdgcn_exp2f(__builtin_fmaf(m_run, a.c2, mc)) : 1.0f;
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+    float tm_other = tm;
+    swap_halves(tm, tm_other);
+    tm = __builtin_fmaxf(tm, tm_other);  // this query's maximum over the half tile, both lane halves agree
+    // the reference follows the maximum lazily, as in the two-wave kernel; most tiles move no query's
+    const bool grow = tm > m_run && __builtin_fmaf(tm, a.c2, lim) > 8.0f;  // (before the first score: +inf)
+    float alpha = 1.0f;
+    if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+      const float mc_new = -tm * a.c2;
+      alpha = grow ? __builtin_amdgcn_exp2f(__builtin_fmaf(m_run, a.c2, mc_new)) : 1.0f;
+      m_run = grow ? tm : m_run;
+      mc = grow ? mc_new : mc;
+      lim = grow ? mc_new : lim;
 #pragma unroll
       for (int ot = 0; ot < OT; ot++)
 #pragma unroll
@@ -584,23 +633,19 @@ __global__ __launch_bounds__(256) void attention_split_kernel(AttArgs a) {
     for (int e = 0; e < 16; e += 2) {
       const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(t[e], a.c2, mc));
       const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(t[e + 1], a.c2, mc));
-      sum = sum + p0 + p1;
+      sum = e == 0 ? p0 + p1 : sum + p0 + p1;
       pk[e >> 1] = narrow2<EL>(p0, p1);
     }
     // O^T += V^T P^T for this wave's 32 keys (the B operand wants keys g*8 + 0..7 per k-step: the
     // accumulator gave g*4 + 0..3 and 8 + g*4 + 0..3, so one half is swapped with lane ^ 32)
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) {
-      const uint32_t a0 = pk[ks * 4 + 0], a1 = pk[ks * 4 + 1];
-      const uint32_t b0 = pk[ks * 4 + 2], b1 = pk[ks * 4 + 3];
-      const uint32_t s0 = g == 0 ? b0 : a0, s1 = g == 0 ? b1 : a1;
-      const uint32_t r0 = (uint32_t)__shfl_xor((int)s0, 32, 64), r1 = (uint32_t)__shfl_xor((int)s1, 32, 64);
-      const V16 pf = g == 0 ? V16{a0, a1, r0, r1} : V16{r0, r1, b0, b1};
+      const auto x = __builtin_amdgcn_permlane32_swap(pk[ks * 4 + 0], pk[ks * 4 + 2], false, false);
+      const auto y = __builtin_amdgcn_permlane32_swap(pk[ks * 4 + 1], pk[ks * 4 + 3], false, false);
+      const V16 pf = {x[0], y[0], x[1], y[1]};
 #pragma unroll
       for (int ot = 0; ot < OT; ot++) {
-        const int kk = kh * 32 + ks * 16 + g * 8 + ((lane & 15) >> 2);
-        const int rr = ot * 32 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
-        const S *src = Vs + kk * PV + rr;
+        const S *src = Ks + vs_at + ks * 16 * PV + ot * 32;
         const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)src);
         const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(src + 4 * PV));
         typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
@@ -609,9 +654,9 @@ __global__ __launch_bounds__(256) void attention_split_kernel(AttArgs a) {
       }
     }
     l_run = __builtin_fmaf(l_run, alpha, sum);
-    m_run = m_new;
   }
   // the odd wave of a pair hands over, the even one merges, divides and stores
+  __syncthreads();  // the stages have been read
   if (kh == 1) {
 #pragma unroll
     for (int ot = 0; ot < OT; ot++)
@@ -667,7 +712,7 @@ int attention_launch(nxh_context *ctx, const char *op, const AttArgs &a, int hd)
   if (blocks > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "too many elements for one launch");
   const dim3 grid((unsigned)blocks), block(128);
   if constexpr (ONLINE) {
-    if (a.raw) {  // the four-wave form ([b,12,1024,64] causal, b = 1 / 2 / 4 / 8 / 16: 19.9 / 20.9 / 23.4 / 37.3 / 74.0 us
+    if (a.raw) {  // the four-wave form ([b,12,1024,64] causal, b = 1 / 2 / 4 / 8 / 16: 15.8 / 17.5 / 20.4 / 33.8 / 61 us
                   // against 29.2 / 30.4 / 32.4 / 42.5 / 80.8 us with two waves per tile)
       switch (hd) {
         case 32: hipLaunchKernelGGL((attention_split_kernel<EL, 32>), grid, dim3(256), 0, ctx->stream, a); break;
