@@ -53,3 +53,17 @@ def test_one_mask_in_all_its_forms(hip, oracle, monkeypatch, d, sq, sk, hd, caus
     want, size = reference(*(decode(x, d, oracle) for x in host), keep)
     unit = 2.0 ** (-8 if d is dt.bfloat16 else -11)
     assert np.all(np.abs(decode(got, d, oracle) - want) <= 1.1 * 2 * unit * size + 2.0 ** -25 * 6 * sk)
+
+
+@pytest.mark.parametrize("heads,sq,hd", [(24, 64, 128), (27, 130, 128), (50, 70, 64)], ids=str)
+def test_tiles_handed_out_in_groups(hip, oracle, monkeypatch, heads, sq, hd):
+    """Keys and values of more heads than three times what the L2s hold: the same bits as a few heads at a time."""
+    monkeypatch.delenv("NXH_ATTENTION", raising=False)
+    rng = np.random.default_rng(heads)
+    q, k, v = (pair(encode(rng.standard_normal((heads, n, hd)), dt.bfloat16, oracle), dt.bfloat16, hip, oracle)[0]
+               for n in (sq, 8192, 8192))
+    got = logical(hip.attention(q, k, v, 0.125))
+    for first in range(0, heads, 9):
+        last = min(first + 9, heads)
+        part = [hip.shrink(t, ((first, last), (0, t.shape[1]), (0, hd))) for t in (q, k, v)]
+        assert got[first:last].tobytes() == logical(hip.attention(*part, 0.125)).tobytes(), first
