@@ -443,15 +443,14 @@ __global__ __launch_bounds__(128) void attention_kernel(AttArgs a) {
 // reference, O = O_a 2^((m_a - m) c) + O_b 2^((m_b - m) c) and the same for the row sum, before
 // the one division. Rounding points are those of the two-wave form; only the f32 sums of the
 // output and of the row sum are added in another order.
-// What bounds it now is what a SIMD issues: 122 vector instructions and 16 exponentials a half tile,
-// 600 of some 1000 cycles, beside 256 of the matrix pipe. So: a register budget under which
-// the compiler keeps the sums in registers that vector instructions reach (it had them
-// in the other file, 80 moves a step); the exchanges with lane ^ 32 as register swaps instead of trips
-// through LDS; the reference's update behind a branch that most steps do not take; two stages for
-// heads of up to 64, one barrier a tile; four neighbouring mask bytes by one load. The results are
-// the same bits. Start -> now, us: [b,12,1024,64] bfloat16 causal, b = 1 / 2 / 4 / 8 / 16: 18.7 / 20.2 / 22.8 / 38.5
-// / 77 -> 15.8 / 17.5 / 20.4 / 33.8 / 61; without a mask, b = 8: 62.6 -> 55.5; a mask tensor, b = 4: 106 -> 41;
-// [8,12,1024,64] float16 causal 51.6 -> 46.6, [8,16,1000,32] 31.2 -> 28.0, [8,8,2048,128] 152 -> 142.
+// What bounds it is what a SIMD issues: 125 vector instructions a half tile and wave, 16 exponentials and 8 products
+// among them, 589 of 978 cycles, beside 256 of the matrix pipe ([8,12,1024,64] without a mask, by counters). So the
+// exchanges with lane ^ 32 are register swaps and no trips through LDS; the reference's update is behind a
+// branch that most steps do not take; heads of up to 64 have two stages and one barrier a tile; a thread's loads and
+// stores have one address each and immediate offsets; four neighbouring mask bytes are one load. The results are the same bits.
+// Before -> now, us: [b,12,1024,64] bfloat16 causal, b = 1 / 2 / 4 / 8 / 16: 18.7 / 20.2 / 22.9 / 39.1 / 74.3 -> 15.5 / 17.4 /
+// 20.3 / 33.8 / 63.3; without a mask, b = 8: 62.2 -> 53.8; a mask tensor, b = 4: 105.6 -> 41.2;
+// [8,12,1024,64] float16 causal 53.2 -> 46.1, [8,16,1000,32] 31.4 -> 28.0, [8,8,2048,128] 154 -> 141.
 // Four waves a SIMD (128 registers) against three: b = 16 61 against 67, b = 8 33.8 and 34.1.
 template <class EL, int DHEAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DHEAD <= 64 ? 4 : 2))) void attention_split_kernel(AttArgs a) {
@@ -719,7 +718,7 @@ int attention_launch(nxh_context *ctx, const char *op, const AttArgs &a, int hd)
   if (blocks > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "too many elements for one launch");
   const dim3 grid((unsigned)blocks), block(128);
   if constexpr (ONLINE) {
-    if (a.raw) {  // the four-wave form ([b,12,1024,64] causal, b = 1 / 2 / 4 / 8 / 16: 15.8 / 17.5 / 20.4 / 33.8 / 61 us
+    if (a.raw) {  // the four-wave form ([b,12,1024,64] causal, b = 1 / 2 / 4 / 8 / 16: 15.5 / 17.4 / 20.3 / 33.8 / 63.3 us
                   // against 29.2 / 30.4 / 32.4 / 42.5 / 80.8 us with two waves per tile)
       switch (hd) {
         case 32: hipLaunchKernelGGL((attention_split_kernel<EL, 32>), grid, dim3(256), 0, ctx->stream, a); break;
