@@ -813,13 +813,13 @@ int radix_run(nxh_context *ctx, const char *op, SortArgs &a) {
 }
 
 // ── slices of some tiles: sorted tiles, split evenly, sorted again ──────────
-// Up to SPLIT_TILES tiles of 4096 words: (1) every tile is sorted by a network in one block; (2) a block per slice takes
-// every 32nd word of each sorted tile, sorts these and picks evenly spaced ones that cut the slice into parts, and finds
+// Up to SPLIT_TILES tiles of 4096 words: (1) every tile is sorted by a network in one block; (2) every 32nd word of
+// each sorted tile is ranked among those of its slice, evenly spaced ranks cut the slice into parts, and it is found
 // where each cuts each tile; (3) a block per part gathers its T runs, sorts them and writes the results. All words of
 // a slice differ, so the parts are bounded whatever the values are: a cut with R samples at or below it has between
 // 32 R and 32 R + 31 T words at or below it, and the cuts are taken so that 32 (R' - R) + 31 T <= 4096. The words cross
 // memory twice, against once per eight bits in the radix sort, and there are three launches for eight: [64,50257]
-// float32, argsort: 33 + 15 + 36 us, where the radix sort takes 36 for its histograms and 84 for its scatters. Bound by the
+// float32, argsort: 33 + 11 + 36 us, where the radix sort takes 36 for its histograms and 84 for its scatters. Bound by the
 // exchanges: 78 steps of two instructions, some eight clocks each, for every two words, with sixteen waves a compute unit.
 //
 // The words are doubles here: bits 0 - 19 the index, 20 - 51 the mapped key of Packed, above them one exponent for all
@@ -961,6 +961,7 @@ __device__ __forceinline__ void net_each(const double (&e)[16], double *buf, F f
 
 struct SplitArgs {
   double *words;   // [slices][tiles][4096]
+  double *samples;  // [slices][tiles][SPLIT_SAMPLES]: every 32nd word of each sorted tile
   uint32_t *cuts;  // [slices][parts + 1][tiles]: the words of a tile before a part
   int tiles, parts;
   uint32_t desc, back;  // of fword
@@ -989,46 +990,67 @@ __global__ __launch_bounds__(256) void split_tiles_kernel(SortArgs a, SplitArgs 
   }
   net_sort(e, buf);
   double *to = p.words + (int64_t)blockIdx.x * 4096;
-  net_each(e, buf, [&](int i, double w) { to[i] = w; });
+  double *sample = p.samples + (int64_t)blockIdx.x * SPLIT_SAMPLES;
+  net_each(e, buf, [&](int i, double w) {
+    to[i] = w;
+    if (i % SPLIT_EVERY == SPLIT_EVERY - 1) sample[i / SPLIT_EVERY] = w;
+  });
 }
 
+// A block per tile: every one of its samples finds its place among all samples of the slice, by a bisection of each
+// tile's; one that is where a cut lies then looks how many words of each tile are at or below it. Nothing is sorted and every chain
+// is short: eight reads of LDS, a load. (One block a slice that sorted the samples took 14.9 us for [64,50257], this 10.9; argsort
+// of [1,4097] 40.5 and 32.2, of [200,6000] 66 and 56, of [1000,9000] 220 and 198.)
 __global__ __launch_bounds__(256) void split_cuts_kernel(SplitArgs p) {
-  __shared__ double buf[NET_LDS], sample[4096];
-  const double *words = p.words + (int64_t)blockIdx.x * p.tiles * 4096;
-  uint32_t *cuts = p.cuts + (int64_t)blockIdx.x * (p.parts + 1) * p.tiles;
-  const int samples = p.tiles * SPLIT_SAMPLES;
-  double e[16];
-#pragma unroll
-  for (int r = 0; r < 16; r++) {
-    const int q = r * 256 + threadIdx.x;
-    e[r] = q < samples ? words[(int64_t)q * SPLIT_EVERY + SPLIT_EVERY - 1] : fword_pad((1u << 20) + q);
+  __shared__ double sample[SPLIT_TILES * SPLIT_SAMPLES];
+  __shared__ uint8_t below[SPLIT_TILES][SPLIT_SAMPLES];  // samples of a tile below this one
+  __shared__ int partial[SPLIT_SAMPLES], found[SPLIT_SAMPLES][2], n_found;
+  static_assert(SPLIT_SAMPLES == 128 && SPLIT_EVERY == 32, "two threads a sample, half a wave a run of words");
+  const int64_t slice = blockIdx.x / p.tiles;
+  const int own = (int)(blockIdx.x % p.tiles), samples = p.tiles * SPLIT_SAMPLES;
+  const double *words = p.words + slice * p.tiles * 4096, *from = p.samples + slice * samples;
+  uint32_t *cuts = p.cuts + slice * (p.parts + 1) * p.tiles;
+  for (int q = threadIdx.x; q < samples; q += 256) sample[q] = from[q];
+  if (threadIdx.x == 0) {
+    n_found = 0;
+    cuts[own] = 0;
+    cuts[p.parts * p.tiles + own] = 4096;
   }
-#pragma unroll
-  for (int r = 0; r < 16; r++) sample[r * 256 + threadIdx.x] = e[r];
-  net_sort(e, buf);
-  net_each(e, buf, [](int, double) {});  // (places the sorted samples in buf)
   __syncthreads();
-  for (int pair = threadIdx.x; pair < (p.parts + 1) * p.tiles; pair += 256) {
-    const int k = pair / p.tiles, tile = pair % p.tiles;
-    uint32_t at = k == 0 ? 0 : 4096;
-    if (k > 0 && k < p.parts) {
-      const double cut = buf[net_place(k * samples / p.parts - 1)];
-      const double *own = sample + tile * SPLIT_SAMPLES, *tw = words + (int64_t)tile * 4096;
-      int lo = 0, hi = SPLIT_SAMPLES;  // samples at or below the cut
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (own[mid] <= cut) lo = mid + 1;
-        else hi = mid;
-      }
-      int first = lo * SPLIT_EVERY, last = lo < SPLIT_SAMPLES ? first + SPLIT_EVERY - 1 : first;  // the words up to the next sample
-      while (first < last) {
-        const int mid = (first + last) >> 1;
-        if (tw[mid] <= cut) first = mid + 1;
-        else last = mid;
-      }
-      at = (uint32_t)first;
+  const int m = threadIdx.x % SPLIT_SAMPLES, half = threadIdx.x / SPLIT_SAMPLES;
+  const double mine = sample[own * SPLIT_SAMPLES + m];
+  int rank = 0;
+#pragma unroll 4
+  for (int tile = half; tile < p.tiles; tile += 2) {
+    const double *other = sample + tile * SPLIT_SAMPLES;
+    int lo = 0;
+#pragma unroll
+    for (int step = SPLIT_SAMPLES / 2; step > 0; step >>= 1) lo += other[lo + step - 1] < mine ? step : 0;
+    lo += other[lo] < mine;  // (lo is at most 127 here)
+    below[tile][m] = (uint8_t)lo;
+    rank += lo;
+  }
+  if (half) partial[m] = rank;
+  __syncthreads();
+  if (!half) {
+    // cut k is the sample with k * samples / parts samples at or below it
+    const int at = rank + partial[m] + 1, k = (at * p.parts + samples - 1) / samples;
+    if (k < p.parts && k * samples / p.parts == at) {
+      const int f = atomicAdd(&n_found, 1);
+      found[f][0] = m, found[f][1] = k;
     }
-    cuts[pair] = at;
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, j = lane & 31;
+  for (int base = 0; base < n_found * p.tiles; base += 8) {  // (every lane of a wave takes every turn)
+    const int pair = base + (threadIdx.x >> 5);
+    const bool live = pair < n_found * p.tiles;
+    const int f = live ? pair / p.tiles : 0, tile = live ? pair % p.tiles : 0, s = found[f][0];
+    const int lo = below[tile][s] + (tile == own);  // samples at or below the cut
+    const bool under = lo < SPLIT_SAMPLES && words[(int64_t)tile * 4096 + lo * SPLIT_EVERY + j] <= sample[own * SPLIT_SAMPLES + s];
+    const uint64_t all = __builtin_amdgcn_ballot_w64(under);  // (the run's last word is the next sample, above the cut)
+    const uint32_t run = (uint32_t)(all >> (lane & 32));
+    if (live && j == 0) cuts[found[f][1] * p.tiles + tile] = (uint32_t)(lo * SPLIT_EVERY + __builtin_popcount(run));
   }
 }
 
@@ -1141,13 +1163,14 @@ int split_run(nxh_context *ctx, const char *op, SortArgs &a) {
   if (a.slices * std::max(p.tiles, p.parts) > 0x7fffffffLL) return nxh_fail(NXH_FAILURE, op, "too many elements for one launch");
   Scratch scratch(ctx);
   if (scratch.get(0, (size_t)(a.slices * p.tiles) * 4096 * sizeof(double)) ||
-      scratch.get(1, (size_t)(a.slices * (p.parts + 1) * p.tiles) * sizeof(uint32_t)))
+      scratch.get(1, (size_t)(a.slices * p.tiles) * (SPLIT_SAMPLES * sizeof(double) + (size_t)(p.parts + 1) * sizeof(uint32_t))))
     return nxh_fail(NXH_FAILURE, op, NXH_ERR_ALLOC);
   p.words = (double *)scratch.p[0];
-  p.cuts = (uint32_t *)scratch.p[1];
+  p.samples = (double *)scratch.p[1];
+  p.cuts = (uint32_t *)(p.samples + a.slices * p.tiles * SPLIT_SAMPLES);
   nxh_set_path("sort_radix");  // the name of every long form of packed words
   hipLaunchKernelGGL((split_tiles_kernel<DT>), dim3((unsigned)(a.slices * p.tiles)), dim3(256), 0, ctx->stream, a, p);
-  hipLaunchKernelGGL(split_cuts_kernel, dim3((unsigned)a.slices), dim3(256), 0, ctx->stream, p);
+  hipLaunchKernelGGL(split_cuts_kernel, dim3((unsigned)(a.slices * p.tiles)), dim3(256), 0, ctx->stream, p);
   hipLaunchKernelGGL((split_parts_kernel<ARG ? NXH_F32 : DT, ARG>), dim3((unsigned)(a.slices * p.parts)), dim3(256), 0, ctx->stream, a, p);
   NXH_HIP(op, hipGetLastError());
   return NXH_OK;
@@ -1173,9 +1196,9 @@ int psort_run(nxh_context *ctx, const char *op, SortArgs &a) {
     NXH_HIP(op, hipGetLastError());
     return NXH_OK;
   }
-  // Sorted tiles and parts against a radix sort that needs all four of its passes (argsort, us): [64,50257] 85 / 117, [1,50257]
-  // 43 / 57, [1,4097] 41 / 50, [200,6000] 66 / 78, [24,131072] 101 / 110, [1000,9000] 221 / 254. Of three passes (float16)
-  // 83 / 93, 44 / 46, 41 / 42, 64 / 62, 100 / 87, 210 / 201, of two (bfloat16) 86 / 64: those stay.
+  // Sorted tiles and parts against a radix sort that needs all four of its passes (argsort, us): [64,50257] 84 / 117, [1,50257]
+  // 41 / 57, [1,4097] 32 / 50, [200,6000] 56 / 78, [24,131072] 96 / 110, [1000,9000] 198 / 254. Of three passes (float16), with cuts
+  // that took up to 20 us more, 83 / 93, 44 / 46, 41 / 42, 64 / 62, 100 / 87, 210 / 201, of two (bfloat16) 86 / 64: those stay.
   if constexpr (__builtin_popcount(rx_pass_mask<DT>()) == 4) {
     if (a.n <= SPLIT_TILES * 4096 && !sort_meets_input<DT>(a, MODE >= ARG_ASC ? 4 : (int)sizeof(typename Tr<DT>::S)))
       return split_run<DT, MODE>(ctx, op, a);
