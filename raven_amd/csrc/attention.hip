@@ -712,6 +712,7 @@ bool two_pass_wanted() {
   return e && strcmp(e, "twopass") == 0;
 }
 
+// hd: 32, 64 or 128, as the entry point has checked.
 template <class EL, bool ONLINE>
 int attention_launch(nxh_context *ctx, const char *op, const AttArgs &a, int hd) {
   const int64_t blocks = a.batches * a.qtiles;
@@ -723,8 +724,7 @@ int attention_launch(nxh_context *ctx, const char *op, const AttArgs &a, int hd)
       switch (hd) {
         case 32: hipLaunchKernelGGL((attention_split_kernel<EL, 32>), grid, dim3(256), 0, ctx->stream, a); break;
         case 64: hipLaunchKernelGGL((attention_split_kernel<EL, 64>), grid, dim3(256), 0, ctx->stream, a); break;
-        case 128: hipLaunchKernelGGL((attention_split_kernel<EL, 128>), grid, dim3(256), 0, ctx->stream, a); break;
-        default: return nxh_fail(NXH_FAILURE, op, "head dimension must be 32, 64 or 128");
+        default: hipLaunchKernelGGL((attention_split_kernel<EL, 128>), grid, dim3(256), 0, ctx->stream, a); break;
       }
       return NXH_OK;
     }
@@ -732,8 +732,7 @@ int attention_launch(nxh_context *ctx, const char *op, const AttArgs &a, int hd)
   switch (hd) {
     case 32: hipLaunchKernelGGL((attention_kernel<EL, 32, ONLINE>), grid, block, 0, ctx->stream, a); break;
     case 64: hipLaunchKernelGGL((attention_kernel<EL, 64, ONLINE>), grid, block, 0, ctx->stream, a); break;
-    case 128: hipLaunchKernelGGL((attention_kernel<EL, 128, ONLINE>), grid, block, 0, ctx->stream, a); break;
-    default: return nxh_fail(NXH_FAILURE, op, "head dimension must be 32, 64 or 128");
+    default: hipLaunchKernelGGL((attention_kernel<EL, 128, ONLINE>), grid, block, 0, ctx->stream, a); break;
   }
   return NXH_OK;
 }
@@ -798,6 +797,7 @@ NXH_EXPORT int nxh_attention(nxh_context *ctx, const nxh_tensor *out, const nxh_
     if (out->shape[d] > 1 && out->strides[d] == 0) return nxh_fail(NXH_INVALID_ARGUMENT, op, NXH_ERR_OUT_ALIASED);
   if (!rows_aligned(q, 16) || !rows_aligned(k, 16) || !rows_aligned(v, 16) || !rows_aligned(out, 8))
     return nxh_fail(NXH_FAILURE, op, "rows must be contiguous and 16-byte aligned");
+  if (hd != 32 && hd != 64 && hd != 128) return nxh_fail(NXH_FAILURE, op, "head dimension must be 32, 64 or 128");
   auto operand = [&](const nxh_tensor *t, AttOperand &o, int es) {
     o.base = t ? (const char *)t->data + t->offset * es : nullptr;
     for (int d = 0; d < ATT_MAXB; d++) o.outer[d] = (t && d < nd - 2) ? t->strides[d] : 0;

@@ -67,3 +67,13 @@ def test_tiles_handed_out_in_groups(hip, oracle, monkeypatch, heads, sq, hd):
         last = min(first + 9, heads)
         part = [hip.shrink(t, ((first, last), (0, t.shape[1]), (0, hd))) for t in (q, k, v)]
         assert got[first:last].tobytes() == logical(hip.attention(*part, 0.125)).tobytes(), first
+
+
+@pytest.mark.parametrize("hd", [0, 1, 8, 16, 96, 256])
+@pytest.mark.parametrize("form", ["", "twopass"])
+def test_other_head_dimensions_are_refused(hip, monkeypatch, hd, form):
+    """None too, which no quotient on the way may meet."""
+    monkeypatch.setenv("NXH_ATTENTION", form)
+    t = hip.full(dt.bfloat16, (1, 1, 1, hd), 1.0)
+    with pytest.raises(RuntimeError, match="head dimension must be 32, 64 or 128"):
+        hip.attention(t, t, t, 0.125)
