@@ -1214,16 +1214,15 @@ struct HostStatus {
     std::lock_guard<std::mutex> g(ctx->mu);
     seq = nxh_next_report(ctx);
   }
-  int *found() const { return ctx->fault_flag + 2; }
-  LaFailure failure(bool reports) const { return {found(), reports ? nxh_report_word(ctx, NXH_REPORT_LINALG) : nullptr, seq}; }
+  LaFailure failure(bool reports) const { return {nxh_found(ctx, NXH_REPORT_CALL), reports ? nxh_report_word(ctx, NXH_REPORT_CALL) : nullptr, seq}; }
   // For calls none of whose kernels reports: once the work queued so far has run.
-  void queue() const { nxh_queue_report(ctx, NXH_REPORT_LINALG, seq, found()); }
+  void queue() const { nxh_queue_report(ctx, NXH_REPORT_CALL, seq); }
   // Waits for the report. `code`: what a queued one stands for.
   int collect(const char *op, int code) const {
     std::lock_guard<std::mutex> g(ctx->mu);
     NXH_HIP(op, hipGetLastError());
     int reported = LA_OK;
-    if (int rc = nxh_await_report(ctx, op, NXH_REPORT_LINALG, seq, &reported)) return rc;
+    if (int rc = nxh_await_report(ctx, op, NXH_REPORT_CALL, seq, &reported)) return rc;
     return reported == LA_OK ? NXH_OK : nxh_fail(NXH_FAILURE, op, LA_MESSAGES[code]);
   }
 };

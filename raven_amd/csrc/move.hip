@@ -49,7 +49,7 @@ __device__ __forceinline__ void raise_fault(const IndexFault &f) {
 }
 static IndexFault index_fault(nxh_context *ctx, uint32_t seq) {
   if (ctx->capture) return {ctx->fault_flag_host, 1};
-  return {nxh_index_found(ctx), (int)seq};
+  return {nxh_found(ctx, NXH_REPORT_INDEX), (int)seq};
 }
 // A report of the launch's first block. word: null where there is none.
 struct IndexReport {
@@ -271,7 +271,7 @@ NXH_EXPORT int nxh_gather(nxh_context *ctx, const nxh_tensor *out, const nxh_ten
       default: launch_any_e<G16>(ctx, a); break;
     }
   }
-  if (!reported) nxh_queue_report(ctx, NXH_REPORT_INDEX, seq, nxh_index_found(ctx));
+  if (!reported) nxh_queue_report(ctx, NXH_REPORT_INDEX, seq);
   NXH_HIP(op, hipGetLastError());
   // Data faults surface from this call (nx_c_move.c:448-458).
   return nxh_collect_index_report(ctx, op, seq);
@@ -823,9 +823,11 @@ static int scatter_sorted(nxh_context *ctx, const char *op, const ScatterArgs &a
     std::lock_guard<std::mutex> guard(ctx->mu);
     rc = nxh_settle_replay_faults(ctx, op);
     if (!rc) {
+      // (the context's other calls come in between these steps: the report is the whole call's, and not under ctx->mu)
       seq = nxh_next_report(ctx);
       hipLaunchKernelGGL(scatter_keys_kernel, dim3((unsigned)((a.n_idx + 255) / 256)), dim3(256), 0, ctx->stream, a.idx,
-                         a.a_istride, a.n_idx, a.axis_len, (int32_t *)key, index_fault(ctx, seq));
+                         a.a_istride, a.n_idx, a.axis_len, (int32_t *)key, IndexFault{nxh_found(ctx, NXH_REPORT_CALL), (int)seq});
+      nxh_queue_report(ctx, NXH_REPORT_CALL, seq);
       if (hipGetLastError() != hipSuccess) rc = nxh_fail(NXH_FAILURE, op, "launch failed");
     }
   }
@@ -843,9 +845,8 @@ static int scatter_sorted(nxh_context *ctx, const char *op, const ScatterArgs &a
     std::lock_guard<std::mutex> guard(ctx->mu);
     nxh_set_path("scatter_sorted");
     table.fn[dt](ctx, (const int32_t *)key, (const int32_t *)perm, a, add);
-    nxh_queue_report(ctx, NXH_REPORT_INDEX, seq, nxh_index_found(ctx));
     if (hipGetLastError() != hipSuccess) rc = nxh_fail(NXH_FAILURE, op, "launch failed");
-    else rc = nxh_collect_index_report(ctx, op, seq);
+    else rc = nxh_collect_index_report(ctx, op, seq, NXH_REPORT_CALL);
   }
   if (key) (void)nxh_free(ctx, key);
   if (perm) (void)nxh_free(ctx, perm);
@@ -987,7 +988,7 @@ static int scatter_impl(nxh_context *ctx, const nxh_tensor *out, const nxh_tenso
   if (vec) a.columns = lanes;
   nxh_set_path(vec ? "scatter_rows_16B" : range_rows > 0 ? "scatter_rows" : "scatter_columns");
   table[dt](ctx, a, mode == 1, range_rows, vec);
-  if (!ctx->capture) nxh_queue_report(ctx, NXH_REPORT_INDEX, seq, nxh_index_found(ctx));
+  if (!ctx->capture) nxh_queue_report(ctx, NXH_REPORT_INDEX, seq);
   NXH_HIP(op, hipGetLastError());
   return nxh_collect_index_report(ctx, op, seq);
 }

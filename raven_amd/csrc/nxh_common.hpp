@@ -161,20 +161,21 @@ void nxh_cache_opaque(nxh_context *ctx);
 // How a call learns what its kernels found without waiting for all they do: a kernel stores (number of the
 // report << 8 | code) to a word of pinned memory in ONE store, so nothing is cleared and nothing is ordered against
 // it, and the host looks at the word. 7.2 us from a launch to the answer, 12.0 with hipStreamSynchronize; a kernel that
-// stores early lets its caller go on while it works. NXH_REPORT_INDEX (gather, scatter) belongs to whoever holds ctx->mu,
-// NXH_REPORT_LINALG to whoever holds ctx->call_mu.
-enum { NXH_REPORT_INDEX = 0, NXH_REPORT_LINALG = 1 };
+// stores early lets its caller go on while it works. NXH_REPORT_INDEX (gathers and scatters of one locked step) belongs to
+// whoever holds ctx->mu, NXH_REPORT_CALL (the factorisations, the scatter that sorts: they let go of mu between their steps) to
+// whoever holds ctx->call_mu; so do the device words nxh_found, which the kernels before a queued report raise to its number.
+enum { NXH_REPORT_INDEX = 0, NXH_REPORT_CALL = 1 };
 static inline uint64_t *nxh_report_word(nxh_context *ctx, int which) { return (uint64_t *)ctx->fault_flag_host + 8 * (1 + which); }
 // The number of a new report, never 0. Caller holds ctx->mu.
 static inline uint32_t nxh_next_report(nxh_context *ctx) { return ++ctx->report_seq ? ctx->report_seq : ++ctx->report_seq; }
 // Waits until report `seq` is in `which` (or the stream has run out of work) and reads its code.
 int nxh_await_report(nxh_context *ctx, const char *op, int which, uint32_t seq, int *code);
-// Queues report `seq`, made once the work before it has run: code 1 if *found (device memory) is seq, else 0.
-void nxh_queue_report(nxh_context *ctx, int which, uint32_t seq, const int *found);
-// The report of a gather or scatter as the call's failure (recorded into a graph: left for the replay). Its kernels raise
-// the word nxh_index_found to the report's number, in a graph the host's flag.
-int nxh_collect_index_report(nxh_context *ctx, const char *op, uint32_t seq);
-static inline int *nxh_index_found(nxh_context *ctx) { return ctx->fault_flag + 4; }
+static inline int *nxh_found(nxh_context *ctx, int which) { return ctx->fault_flag + 2 + which; }
+// Queues report `seq`, made once the work before it has run: code 1 if nxh_found is seq, else 0.
+void nxh_queue_report(nxh_context *ctx, int which, uint32_t seq);
+// The report of a gather or scatter as the call's failure (recorded into a graph, where its kernels raise the host's flag:
+// left for the replay).
+int nxh_collect_index_report(nxh_context *ctx, const char *op, uint32_t seq, int which = NXH_REPORT_INDEX);
 // Before an eager gather / scatter is launched: a fault that a replayed graph left in
 // the flag is reported now, as the replay's, so that this call answers only for itself.
 int nxh_settle_replay_faults(nxh_context *ctx, const char *op);

@@ -481,8 +481,8 @@ static int read_fault_flag(nxh_context *ctx, const char *op, const char *message
 __global__ void report_kernel(uint64_t *word, uint32_t seq, const int *found) {
   nxh_report(word, seq, *found == (int)seq);
 }
-void nxh_queue_report(nxh_context *ctx, int which, uint32_t seq, const int *found) {
-  hipLaunchKernelGGL(report_kernel, dim3(1), dim3(1), 0, ctx->stream, nxh_report_word(ctx, which), seq, found);
+void nxh_queue_report(nxh_context *ctx, int which, uint32_t seq) {
+  hipLaunchKernelGGL(report_kernel, dim3(1), dim3(1), 0, ctx->stream, nxh_report_word(ctx, which), seq, nxh_found(ctx, which));
 }
 
 int nxh_await_report(nxh_context *ctx, const char *op, int which, uint32_t seq, int *code) {
@@ -504,13 +504,13 @@ int nxh_await_report(nxh_context *ctx, const char *op, int which, uint32_t seq, 
   return there() ? NXH_OK : nxh_fail(NXH_FAILURE, op, "the device did not report");
 }
 
-int nxh_collect_index_report(nxh_context *ctx, const char *op, uint32_t seq) {
+int nxh_collect_index_report(nxh_context *ctx, const char *op, uint32_t seq, int which) {
   if (ctx->capture) {
     ctx->capture->has_index_checks = true;
     return NXH_OK;
   }
   int code = 0;
-  if (int rc = nxh_await_report(ctx, op, NXH_REPORT_INDEX, seq, &code)) return rc;
+  if (int rc = nxh_await_report(ctx, op, which, seq, &code)) return rc;
   return code ? nxh_fail(NXH_FAILURE, op, NXH_ERR_INDEX_OOB) : NXH_OK;
 }
 
