@@ -530,9 +530,12 @@ constexpr int SCATTER_RANGE = 1024;  // rows of a block's range, at most
 // through all indices for those of its range (sixteen loads of a lane in flight, out of L2) and puts them in the order
 // of (row, position) by counting the smaller ones. Where rows are whole vectors (V > 1) the copy adds on the way: a
 // vector's first update is requested with the vector itself, and nothing but the vector is written. Ragged rows are
-// copied 16 bytes at a time whatever rows they belong to, and updated after it, a wave to 64 elements of a row; so are
-// blocks with more than LIST updates, in spans of LIST positions. Either way an element's updates come in the order of
-// their positions, each rounded to the storage type. Bound by the copy, which streaming stores decide (`stream`): [50257,
+// copied 16 bytes at a time whatever rows they belong to, and updated after it, an element a lane; so are rows with more
+// than DIRECT updates, whose lanes request a dozen at a time, and blocks with more than LIST updates, in spans of positions that
+// the list takes. Either way an element's updates come in the order of their positions, each rounded to the storage
+// type; of those that are set only the last is read. What one row takes is one block's work (8 192 updates of one row of 768 f32: 613 us,
+// 1 920 in scatter_rows; one at a time and 1 024 positions a span 3 260; [1048576,2] with a million updates 1 470, 1 980
+// and 4 700). Bound by the copy, which streaming stores decide (`stream`): [50257,
 // 768] f32 with 8 192 updates from the cache 47 us, with plain stores 67 (a copy alone 39); with updates from memory 66,
 // where a copy and scatter_rows take 43 and 33, and scatter_rows with `from`, whose lanes own columns and copy one row
 // after another, some 150.
@@ -544,12 +547,11 @@ __global__ __launch_bounds__(256) void scatter_copy_kernel(ScatterArgs a, int64_
   struct alignas(V > 1 ? 16 : alignof(E)) S {
     E v[V];
   };
-  constexpr int LIST = 1024, LOOK = 16, EACH = 4, B = 4;
-  __shared__ uint64_t list[LIST];         // (row of the range << 32 | position), in any order
-  __shared__ uint32_t position[LIST];     // in the order of (row, position)
-  __shared__ uint16_t start[SCATTER_RANGE], count[SCATTER_RANGE], updated[LIST];  // of a row; the rows that have updates
+  constexpr int LIST = 1024, LOOK = 16, EACH = 4, DIRECT = 16;
+  __shared__ uint64_t list[LIST];         // (row of the range << 32 | position), in any order, then in theirs
+  __shared__ uint32_t position[LIST];     // the positions alone
+  __shared__ uint16_t start[SCATTER_RANGE], stop[SCATTER_RANGE], updated[LIST];  // a row's part of it; rows that `apply` updates
   __shared__ int s_total, s_rows;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t lo = (int64_t)blockIdx.x * range_rows, hi = lo + range_rows < a.axis_len ? lo + range_rows : a.axis_len;
   // The updates at positions from `begin` to `end` whose row is in the range; their number (more than LIST: not kept).
   auto collect = [&](int64_t begin, int64_t end, bool *bad) {
@@ -573,22 +575,32 @@ __global__ __launch_bounds__(256) void scatter_copy_kernel(ScatterArgs a, int64_
     *bad = __syncthreads_or(*bad);
     return s_total;
   };
-  auto order = [&](int n) {
-    for (int r = threadIdx.x; r < range_rows; r += 256) count[r] = 0;
-    __syncthreads();
+  // `updated`: the rows that have more than `direct` updates.
+  auto order = [&](int n, int direct) {
+    for (int r = threadIdx.x; r < range_rows; r += 256) start[r] = stop[r] = 0;
+    const auto place = [&](auto each_c) {  // every word to its rank (all are different), a lane's words side by side
+      constexpr int OWN = decltype(each_c)::value;
+      uint64_t own[OWN];
+      int rank[OWN];
+#pragma unroll
+      for (int j = 0; j < OWN; j++) own[j] = list[min((int)threadIdx.x + 256 * j, n - 1)], rank[j] = 0;
+      for (int k = 0; k < n; k++)
+#pragma unroll
+        for (int j = 0; j < OWN; j++) rank[j] += list[k] < own[j];
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < OWN; j++)
+        if ((int)threadIdx.x + 256 * j < n) list[rank[j]] = own[j], position[rank[j]] = (uint32_t)own[j];
+      __syncthreads();
+    };
+    if (n > 256) place(std::integral_constant<int, LIST / 256>{});
+    else if (n > 0) place(std::integral_constant<int, 1>{});
     for (int i = threadIdx.x; i < n; i += 256) {
-      const uint64_t own = list[i];
-      int rank = 0, first = 0, last = 0;  // all are different
-      for (int k = 0; k < n; k++) {
-        rank += list[k] < own;
-        first += list[k] >> 32 < own >> 32;
-        last += list[k] >> 32 <= own >> 32;
-      }
-      position[rank] = (uint32_t)own;
-      if (rank > first) continue;
-      start[own >> 32] = (uint16_t)first;
-      count[own >> 32] = (uint16_t)(last - first);
-      updated[atomicAdd(&s_rows, 1)] = (uint16_t)(own >> 32);
+      const int r = (int)(list[i] >> 32);
+      if (i == n - 1 || (int)(list[i + 1] >> 32) != r) stop[r] = (uint16_t)(i + 1);
+      if (i > 0 && (int)(list[i - 1] >> 32) == r) continue;
+      start[r] = (uint16_t)i;
+      if (direct == 0 || (i + direct < n && (int)(list[i + direct] >> 32) == r)) updated[atomicAdd(&s_rows, 1)] = (uint16_t)r;
     }
     __syncthreads();
   };
@@ -606,6 +618,37 @@ __global__ __launch_bounds__(256) void scatter_copy_kernel(ScatterArgs a, int64_
       return u;
     }
   };
+  const int64_t wide = row / V, a_us = a.a_ustride / V;
+  // The rows in `updated` as they are in memory, an element a lane.
+  auto apply = [&]() {
+    for (uint32_t item = threadIdx.x; item < (uint32_t)s_rows * (uint32_t)wide; item += 256) {
+      const int r = updated[item / (uint32_t)wide];
+      const int64_t c = item % (uint32_t)wide;
+      S *o = reinterpret_cast<S *>(reinterpret_cast<E *>(a.out) + (lo + r) * row) + c;
+      const S *upd = reinterpret_cast<const S *>(a.upd) + c;
+      const int last = stop[r];
+      if constexpr (ADD) {
+        S acc = *o;
+        int i = start[r];
+        const auto some = [&](auto n_c) {
+          constexpr int B = decltype(n_c)::value;
+          S u[B];
+#pragma unroll
+          for (int j = 0; j < B; j++) u[j] = upd[(int64_t)position[i + j < last ? i + j : i] * a_us];
+#pragma unroll
+          for (int j = 0; j < B; j++)
+            if (i + j < last) acc = combine(acc, u[j]);
+          i += B;
+        };
+        constexpr int MANY = V > 8 ? 8 : 12;  // (more would cost the copy a wave a SIMD)
+        while (i + MANY <= last) some(std::integral_constant<int, MANY>{});
+        while (i < last) some(std::integral_constant<int, 4>{});
+        *o = acc;
+      } else {
+        *o = upd[(int64_t)position[last - 1] * a_us];
+      }
+    }
+  };
   auto put = [&](G16 *p, G16 x) {
     typedef uint64_t pair __attribute__((ext_vector_type(2)));
     if (stream) __builtin_nontemporal_store(pair{x.lo, x.hi}, reinterpret_cast<pair *>(p));
@@ -615,13 +658,12 @@ __global__ __launch_bounds__(256) void scatter_copy_kernel(ScatterArgs a, int64_
   const int total = collect(0, a.n_idx, &bad);
   if (a.report.word && blockIdx.x == 0 && threadIdx.x == 0) nxh_report(a.report.word, a.report.seq, bad);
   if (bad) return;
-  const int64_t base = lo * row * (int64_t)sizeof(E), bytes = (hi - lo) * row * (int64_t)sizeof(E), whole = bytes / 16, wide = row / V;
-  const int64_t a_us = a.a_ustride / V;
+  const int64_t base = lo * row * (int64_t)sizeof(E), bytes = (hi - lo) * row * (int64_t)sizeof(E), whole = bytes / 16;
   const G16 *from = reinterpret_cast<const G16 *>(a.from + base);
   G16 *out = reinterpret_cast<G16 *>(a.out + base);
   if constexpr (V > 1) {
     if (total <= LIST) {
-      order(total);
+      order(total, ADD ? DIRECT : LIST);
       const S *upd = reinterpret_cast<const S *>(a.upd);
       for (int64_t i0 = threadIdx.x; i0 < whole; i0 += 256 * EACH) {
         S x[EACH], u[EACH];
@@ -631,8 +673,10 @@ __global__ __launch_bounds__(256) void scatter_copy_kernel(ScatterArgs a, int64_
         for (int j = 0; j < EACH; j++) {
           const int64_t i = i0 + 256 * j < whole ? i0 + 256 * j : i0;
           const uint32_t r = __umulhi(2u * (uint32_t)i, by_wide);  // i / wide (one row: 0)
-          n[j] = count[r];
+          n[j] = stop[r] - start[r];
           at[j] = start[r];
+          if (ADD && n[j] > DIRECT) n[j] = 0;
+          if (!ADD && n[j] > 1) at[j] = stop[r] - 1, n[j] = 1;  // the last one is what stays
           col[j] = i - r * wide;
           x[j] = reinterpret_cast<const S *>(from)[i];
           if (n[j]) u[j] = upd[(int64_t)position[at[j]] * a_us + col[j]];
@@ -646,6 +690,9 @@ __global__ __launch_bounds__(256) void scatter_copy_kernel(ScatterArgs a, int64_
           if (i0 + 256 * j < whole) put(out + i0 + 256 * j, __builtin_bit_cast(G16, x[j]));
         }
       }
+      if (s_rows == 0) return;
+      __syncthreads();  // what this block's lanes stored is seen by its other lanes
+      apply();
       return;
     }
   }
@@ -659,28 +706,18 @@ __global__ __launch_bounds__(256) void scatter_copy_kernel(ScatterArgs a, int64_
   }
   if (threadIdx.x < bytes % 16) a.out[base + whole * 16 + threadIdx.x] = a.from[base + whole * 16 + threadIdx.x];
   if (total == 0) return;
-  const int64_t span = total <= LIST ? a.n_idx : LIST;
-  const int chunks = (int)((wide + 63) / 64);
-  for (int64_t begin = 0; begin < a.n_idx; begin += span) {
-    if (total > LIST) (void)collect(begin, begin + span < a.n_idx ? begin + span : a.n_idx, &bad);
-    order(s_total);  // (its barriers: what this block's lanes stored so far is seen by its other lanes)
-    for (int64_t item = wave; item < (int64_t)s_rows * chunks; item += 4) {
-      const int r = updated[item / chunks];
-      const int64_t c = item % chunks * 64 + lane;
-      if (c >= wide) continue;
-      S *o = reinterpret_cast<S *>(reinterpret_cast<E *>(a.out) + (lo + r) * row) + c;
-      const S *upd = reinterpret_cast<const S *>(a.upd) + c;
-      S acc = *o;
-      for (int i = start[r], end = i + count[r]; i < end; i += B) {
-        S u[B];
-#pragma unroll
-        for (int j = 0; j < B; j++) u[j] = upd[(int64_t)position[i + j < end ? i + j : i] * a_us];
-#pragma unroll
-        for (int j = 0; j < B; j++)
-          if (i + j < end) acc = combine(acc, u[j]);
-      }
-      *o = acc;
+  // Half of what the list takes is expected in a span; where its updates are denser than elsewhere it is halved.
+  int64_t span = total <= LIST ? a.n_idx : max((int64_t)LIST, a.n_idx / total * (LIST / 2));
+  for (int64_t begin = 0; begin < a.n_idx;) {
+    const int64_t end = min(begin + span, a.n_idx);
+    if (total > LIST && collect(begin, end, &bad) > LIST) {
+      span = max((int64_t)LIST, span / 2);
+      continue;
     }
+    begin = end;
+    if (s_total == 0) continue;
+    order(s_total, 0);  // (its barriers: what this block's lanes stored so far is seen by its other lanes)
+    apply();
   }
 }
 typedef void (*scatter_copy_fn)(nxh_context *, const ScatterArgs &, bool, int64_t, int64_t, bool);
@@ -942,7 +979,8 @@ static int scatter_impl(nxh_context *ctx, const nxh_tensor *out, const nxh_tenso
     } else {
       range = (range + 15) / 16 * 16;  // whole vectors, whatever the row
     }
-    if (rows && ((uintptr_t)a.out | (uintptr_t)a.from) % 16 == 0 && a.n_idx <= 4 * a.axis_len && a.n_idx <= 0x7fffffff) {
+    if (rows && ((uintptr_t)a.out | (uintptr_t)a.from) % 16 == 0 && a.n_idx <= 4 * a.axis_len && a.n_idx <= 0x7fffffff &&
+        range * a.columns <= 0x7fffffff) {
       std::lock_guard<std::mutex> guard(ctx->mu);
       if (ctx->capture) return -1;
       NXH_HIP(op, hipSetDevice(ctx->device));

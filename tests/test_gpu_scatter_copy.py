@@ -1,6 +1,8 @@
 """The one-pass copy and scatter of whole rows (scatter_copy) where its blocks, lists and vectors end: against a copy
 followed by a scatter, bit for bit, and against a serial sum."""
 
+import time
+
 import numpy as np
 import pytest
 
@@ -51,3 +53,51 @@ def test_sums_in_the_order_of_positions(hip):
     for i, r in enumerate(ids):
         want[r] += u[i]
     same_bits(logical(got), want, "serial")
+
+
+def two_launches(hip, mode, template, index, updates):
+    out = hip.copy(template)
+    hip._check(hip._lib.nxh_scatter(hip._h, out._desc(), index._desc(), updates._desc(), 0, {"set": 0, "add": 1}[mode]))
+    return out
+
+
+@pytest.mark.parametrize("cols", [8, 7])
+@pytest.mark.parametrize("most", [15, 16, 17, 29, 1024, 1025, 3000])
+def test_rows_that_many_updates_hit(hip, cols, most):
+    """`most` updates of one row, next to each other and apart: those added on the way, those added after the copy, lists
+    that don't take them all, and spans of positions that are halved until they do."""
+    rng = np.random.default_rng(most)
+    rows, n = 5000, 20000
+    template = hip.reshape(hip.from_host(rng.standard_normal((rows, cols)).astype(np.float32), dt.float32), (rows, cols))
+    updates = hip.reshape(hip.from_host(rng.standard_normal((n, cols)).astype(np.float32), dt.float32), (n, cols))
+    for name, places in (("together", np.arange(most)), ("at the end", n - 1 - np.arange(most)), ("apart", rng.permutation(n)[:most])):
+        ids = rng.integers(0, rows, n)
+        ids[places] = 3
+        index = rows_of(hip, ids, cols)
+        for mode in ("add", "set"):
+            got = hip.scatter(mode, False, template, index, updates, 0)
+            assert hip.last_path() == "scatter_copy"
+            same_bits(logical(got), logical(two_launches(hip, mode, template, index, updates)), f"{name} {mode}")
+
+
+@pytest.mark.parametrize("mode", ["add", "set"])
+@pytest.mark.parametrize("cols", [768, 770])
+def test_one_row_for_all_costs_no_more_than_two_launches(hip, mode, cols):
+    """As a padding token's: 8 192 updates of one row, which one block adds up (0.6 ms and 1.5, set 0.25; two launches 1.8 and
+    1.9, set 0.6 and 0.9)."""
+    template, updates = hip.full(dt.float32, (50257, cols), 0.0), hip.full(dt.float32, (8192, cols), 1.0)
+    index = rows_of(hip, np.full(8192, 7), cols)
+
+    def seconds(f):
+        best = 1.0
+        for _ in range(5):
+            hip.synchronize()
+            t = time.perf_counter()
+            f()
+            hip.synchronize()
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    one = seconds(lambda: hip.scatter(mode, False, template, index, updates, 0))
+    assert hip.last_path() == "scatter_copy"
+    assert one < seconds(lambda: two_launches(hip, mode, template, index, updates))
