@@ -963,7 +963,12 @@ static int scatter_impl(nxh_context *ctx, const nxh_tensor *out, const nxh_tenso
   if (from && uniform_index && !ctx->capture) {
     // One pass over a dense table of rows (axis 0, or what is like it). A block's range is 48 KiB, or 6 bytes an index,
     // so that what it reads of the indices (out of L2) stays below what it copies; smaller where the table has too
-    // few such ranges for the chip, down to 4 KiB.
+    // few such ranges for the chip, down to 4 KiB, and where rows are so short that SCATTER_RANGE of them are less.
+    // Rows that make it much longer than that leave the chip to a few blocks, and go the older ways: whole vectors from 64 KiB
+    // on ([1024,16384] f32, 1 024 updates, 71 -> 41 us and [4,16384], 4 updates, 17 -> 14 in one pass; but [16,32768], 16
+    // updates, 17 against 24, [128,65536], 128 updates, 42 against 83, [4,4194304], 8 updates, 100 against 3 800), ragged rows,
+    // which are updated after the copy, from 12 288 elements on ([3000,1025], 3 000 updates, 35 -> 27; but
+    // [1000,4099], 1 000 updates, 35 against 48, [15,1000001], 8 updates, 49 against 22 700).
     const int64_t line = a.columns * es, bytes = a.axis_len * line;
     int64_t run = 1;
     bool rows = a.a_ostride == a.columns || a.axis_len == 1;
@@ -972,15 +977,16 @@ static int scatter_impl(nxh_context *ctx, const nxh_tensor *out, const nxh_tenso
       run *= a.cshape[d];
     }
     const bool rows16 = es < 16 && line % 16 == 0 && a.a_ustride * es % 16 == 0 && (uintptr_t)a.upd % 16 == 0;
-    int64_t range = std::min(std::max<int64_t>(48 << 10, a.n_idx * 6), std::max<int64_t>(4 << 10, bytes / (2 * ctx->compute_units)));
-    range = std::min<int64_t>(SCATTER_RANGE, std::max<int64_t>(1, range / line));
+    const int64_t aim = std::min(std::max<int64_t>(48 << 10, a.n_idx * 6), std::max<int64_t>(4 << 10, bytes / (2 * ctx->compute_units)));
+    int64_t range = std::min<int64_t>(SCATTER_RANGE, std::max<int64_t>(1, aim / line));
     if (rows16) {
       if (range * (line / 16) >= 1 << 16) range = std::max<int64_t>(1, 65535 / (line / 16));
     } else {
-      range = (range + 15) / 16 * 16;  // whole vectors, whatever the row
+      const int64_t some = std::max<int64_t>(1, 16 / es);
+      range = (range + some - 1) / some * some;  // whole vectors, whatever the row
     }
-    if (rows && ((uintptr_t)a.out | (uintptr_t)a.from) % 16 == 0 && a.n_idx <= 4 * a.axis_len && a.n_idx <= 0x7fffffff &&
-        range * a.columns <= 0x7fffffff) {
+    const bool fits = range * line <= aim + aim / 4 || (rows16 ? range * line <= 64 << 10 : range * a.columns <= 12288);
+    if (rows && fits && ((uintptr_t)a.out | (uintptr_t)a.from) % 16 == 0 && a.n_idx <= 4 * a.axis_len && a.n_idx <= 0x7fffffff) {
       std::lock_guard<std::mutex> guard(ctx->mu);
       if (ctx->capture) return -1;
       NXH_HIP(op, hipSetDevice(ctx->device));

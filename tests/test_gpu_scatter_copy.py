@@ -101,3 +101,19 @@ def test_one_row_for_all_costs_no_more_than_two_launches(hip, mode, cols):
     one = seconds(lambda: hip.scatter(mode, False, template, index, updates, 0))
     assert hip.last_path() == "scatter_copy"
     assert one < seconds(lambda: two_launches(hip, mode, template, index, updates))
+
+
+@pytest.mark.parametrize("rows,cols,n,one_pass", [
+    (16, 16384, 16, True), (2, 16388, 2, False), (16, 32768, 16, False), (1, 262144, 4, False), (128, 65536, 128, False),
+    (64, 3071, 64, True), (4, 4099, 4, False), (64, 3073, 64, False), (100, 10001, 100, False), (15, 100001, 8, False),
+    (3000, 1025, 3000, True), (1000, 4099, 1000, False)])
+def test_long_rows_are_not_left_to_a_few_blocks(hip, rows, cols, n, one_pass):
+    """A row, or as many as are whole vectors, is one block's work at the least: past some 64 KiB it is copied by the whole chip."""
+    rng = np.random.default_rng(cols)
+    template = hip.reshape(hip.from_host(rng.standard_normal((rows, cols)).astype(np.float32), dt.float32), (rows, cols))
+    updates = hip.reshape(hip.from_host(rng.standard_normal((n, cols)).astype(np.float32), dt.float32), (n, cols))
+    index = rows_of(hip, rng.integers(0, rows, n), cols)
+    for mode in ("add", "set"):
+        got = hip.scatter(mode, False, template, index, updates, 0)
+        assert (hip.last_path() == "scatter_copy") == one_pass, hip.last_path()
+        same_bits(logical(got), logical(two_launches(hip, mode, template, index, updates)), mode)
