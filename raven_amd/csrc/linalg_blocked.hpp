@@ -758,9 +758,10 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
       const bool diagonal = t == r16;
       T val = at_hand(a.conj ? S::conj(T(raw[v])) : T(raw[v]));
       const T edge = S::make(diagonal ? 1.0 : 0.0, 0.0);
-      val = k * 16 + max(t, r16) >= n || r16 > t || (a.unit && diagonal) ? edge : val;
+      // (assigned, not chosen: of two complex values a choice is one of two addresses, and both go to scratch memory)
+      if (k * 16 + max(t, r16) >= n || r16 > t || (a.unit && diagonal)) val = edge;
       if (r16 <= t) tri[k % AHEAD][r16][t - r16] = val;
-      own = diagonal ? val : own;
+      if (diagonal) own = val;
     }
     if (own == S::make(0.0, 0.0)) singular = 1;
     if constexpr (sizeof(T) == 8) {

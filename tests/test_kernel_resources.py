@@ -1,0 +1,48 @@
+"""What the compiler gave the kernels of the built library, from the metadata that the code objects carry: registers that
+spill and choices between objects go to scratch memory, which no result shows."""
+
+import re
+import struct
+
+import msgpack
+import pytest
+
+from raven_amd import build
+
+
+def metadata(image):
+    """name -> the kernel's entry of every AMD GPU code object (an ELF with the note of type 32) in the library."""
+    found = {}
+    for at in (m.start() for m in re.finditer(rb"\x7fELF\x02\x01\x01\x40", image)):
+        if struct.unpack_from("<H", image, at + 18)[0] != 224:
+            continue
+        (table,), (size, count) = struct.unpack_from("<Q", image, at + 32), struct.unpack_from("<HH", image, at + 54)
+        for p in range(at + table, at + table + size * count, size):
+            if struct.unpack_from("<I", image, p)[0] != 4:  # a segment of notes
+                continue
+            q = at + struct.unpack_from("<Q", image, p + 8)[0]
+            end = q + struct.unpack_from("<Q", image, p + 32)[0]
+            while q < end:
+                name, desc, kind = struct.unpack_from("<III", image, q)
+                q += 12 + (name + 3) // 4 * 4
+                if kind == 32:
+                    for k in msgpack.unpackb(image[q:q + desc])["amdhsa.kernels"]:
+                        found[k[".name"]] = k
+                q += (desc + 3) // 4 * 4
+    return found
+
+
+@pytest.fixture(scope="module")
+def kernels():
+    return metadata(build.LIB.read_bytes())
+
+
+def named(kernels, part):
+    (name,) = [n for n in kernels if part in n]
+    return kernels[name]
+
+
+@pytest.mark.parametrize("part", ["trsm_block_kernelI4cplxIdES2_Li11E", "trsm_block_kernelI4cplxIdES2_Li0E"])
+def test_no_scratch(kernels, part):
+    k = named(kernels, part)
+    assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_spill_count"] == 0
