@@ -911,6 +911,11 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
     for (int k = 0; k < nb; k++) {
       step(k);
       __syncthreads();
+      if constexpr (sizeof(T) != 8) {  // two steps a turn: [512,512] complex64 852 -> 837 us
+        if (++k == nb) break;
+        step(k);
+        __syncthreads();
+      }
     }
   } else if (wave == TRSM_LOADER) {
     auto step = [&](int k, TS(&r)[4], TS(&l)[4]) {
