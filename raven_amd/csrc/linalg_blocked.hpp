@@ -678,10 +678,10 @@ __global__ __launch_bounds__(256) void cholesky_result_kernel(CholArgs<T> a) {
 // side a lane.
 // Wave 0 is the chain: it neither reads memory nor works out an address. Wave 4 (of its SIMD) reads the triangle and
 // the tile left of it, inverts the 4 x 4 triangles and puts all of it in LDS as the operands that wave 0 takes, without
-// a matrix instruction; the other six bring up to TILES tiles each up to date per step, up to six at a time, so that
-// their products do not wait for each other. What a tile needs
+// a matrix instruction; the other six bring up to TILES tiles each up to date per step, up to six at a time (float64 four: six are 22 registers
+// too many, [1000,1000] with sixteen sides 245 us against 240), so that their products do not wait for each other. What a tile needs
 // of the matrix is in registers two steps ahead, so that TILES decides how many workgroups a compute unit
-// holds (11 tiles one, 2 tiles two). Eleven make a pass of 64 blocks; systems of
+// holds (11 tiles, 177 registers, float64 244: one, 2 tiles, 90 and 120: two). Eleven make a pass of 64 blocks; systems of
 // 2 + 6 TILES blocks and fewer take two; those of one block, TILES = 0, a single wave, which places
 // the triangle itself.
 // [512,512] float32, sixteen sides: 74 us while wave 0 took 3 400 clocks a step (0.6 the tile to the left in one chain, 0.7
@@ -968,7 +968,7 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
           double x[4];
 #pragma unroll
           for (int v = 0; v < 4; v++) x[v] = X[((k - 1) * 16 + 4 * v + q) * 16 + r16];
-          constexpr int MOST = TILES < 6 ? TILES : 6;
+          constexpr int AT_ONCE = sizeof(TS) == 8 ? 4 : 6, MOST = TILES < AT_ONCE ? TILES : AT_ONCE;
 #pragma unroll
           for (int i = 0; i < TILES; i += MOST) {
             const int t = k + first + i * TRSM_UPDATERS;
@@ -976,7 +976,8 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
             const int more = min((nb - 1 - t) / TRSM_UPDATERS + 1, min(TILES - i, MOST));
             const auto some = [&](auto g_c) {
               constexpr int G = decltype(g_c)::value;
-              if constexpr (G <= MOST && (TILES % MOST == 0 || G <= TILES)) tiles(g_c, t, x, &from[i]);
+              if constexpr (G <= MOST)
+                if (G <= TILES - i) tiles(g_c, t, x, &from[i]);
             };
             switch (more) {
               case 1: some(std::integral_constant<int, 1>{}); break;

@@ -42,7 +42,8 @@ def named(kernels, part):
     return kernels[name]
 
 
-@pytest.mark.parametrize("part", ["trsm_block_kernelI4cplxIdES2_Li11E", "trsm_block_kernelI4cplxIdES2_Li0E"])
+@pytest.mark.parametrize("part", ["trsm_block_kernelI4cplxIdES2_Li11E", "trsm_block_kernelI4cplxIdES2_Li0E", "trsm_block_kernelIddLi11E",
+                                  "trsm_block_kernelIddLi2E", "trsm_block_kernelIddLi0E"])
 def test_no_scratch(kernels, part):
     k = named(kernels, part)
     assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_spill_count"] == 0
