@@ -1298,11 +1298,13 @@ template <class T, class TS>
 static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool direct, int64_t batch, int n, int nrhs, int flags, LaMat m,
                     LaMat b, LaMat x) {
   const bool upper = flags & 1, transpose = (flags >> 1) & 1, forward = upper == transpose;
-  const auto most = trsm_block_kernel<T, TS, TRSM_TILES>, few = trsm_block_kernel<T, TS, TRSM_FEW>, one = trsm_block_kernel<T, TS, 0>;
+  constexpr int SOME = sizeof(TS) == 4 ? TRSM_SOME : TRSM_FEW;
+  const auto most = trsm_block_kernel<T, TS, TRSM_TILES>, some = trsm_block_kernel<T, TS, SOME>, few = trsm_block_kernel<T, TS, TRSM_FEW>,
+             one = trsm_block_kernel<T, TS, 0>;
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [&] {
-    for (const auto kern : {most, few})
+    for (const auto kern : {most, some, few})
       if (attr == hipSuccess) attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, TRSM_PASS<T> * 16 * (int)sizeof(T));
   });
   NXH_HIP(op, attr);
@@ -1346,7 +1348,7 @@ static int run_trsm(nxh_context *ctx, const char *op, HostStatus &status, bool d
       a.failure = status.failure(reports && b0 == 0);
       a.checked = check;
       const int nb = (a.rows + 15) / 16;
-      const auto kern = nb == 1 ? one : sizeof(T) == 8 && nb <= 2 + TRSM_UPDATERS * TRSM_FEW ? few : most;  // (complex reads nothing ahead)
+      const auto kern = nb == 1 ? one : sizeof(T) != 8 ? most : nb <= 2 + TRSM_UPDATERS * TRSM_FEW ? few : nb <= 2 + TRSM_UPDATERS * SOME ? some : most;  // (complex reads nothing ahead)
       const int threads = nb == 1 ? TRSM_THREADS<0> : TRSM_THREADS<TRSM_FEW>;
       hipLaunchKernelGGL(kern, dim3(groups, nbat), dim3(threads), (size_t)nb * 256 * sizeof(T), ctx->stream, a);
       const int rest = n - r0 - a.rows;

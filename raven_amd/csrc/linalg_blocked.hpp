@@ -681,13 +681,15 @@ __global__ __launch_bounds__(256) void cholesky_result_kernel(CholArgs<T> a) {
 // a matrix instruction; the other six bring up to TILES tiles each up to date per step, up to six at a time (float64 four: six are 22 registers
 // too many, [1000,1000] with sixteen sides 245 us against 240), so that their products do not wait for each other. What a tile needs
 // of the matrix is in registers two steps ahead, so that TILES decides how many workgroups a compute unit
-// holds (11 tiles, 177 registers, float64 244: one, 2 tiles, 90 and 120: two). Eleven make a pass of 64 blocks; systems of
-// 2 + 6 TILES blocks and fewer take two; those of one block, TILES = 0, a single wave, which places
-// the triangle itself.
+// holds (11 tiles, 177 registers, float64 244: one; float32 with 5 tiles, 116, and 2 tiles, 90 and float64 120: two). A form
+// serves systems of 2 + 6 TILES blocks and fewer, eleven tiles those of a pass, 64; systems of one block, TILES = 0, have a
+// single wave, which places the triangle itself. Five tiles against eleven, float32, us: 1 000 systems of 300 rows 109 / 147,
+// of 512 rows, which two workgroups' LDS just holds, 268 / 326, one system of 300 rows 30.8 / 32.3. (513 to 560 rows would fit
+// twice without wave 0's operands in LDS: 1 000 of 530 rows 306 then, 344 so, one 91 and 68.)
 // [512,512] float32, sixteen sides: 74 us while wave 0 took 3 400 clocks a step (0.6 the tile to the left in one chain, 0.7
 // addresses and conversions, 2.0 solve16) and waited for the others, tile after tile, up to 6 400; 62 so, 3 000 a step but for the first ten, whose products keep the matrix units busy.
 // (The 4 x 4 triangles row by row on the vector unit, four products in the chain for fifteen: 2.3 for solve16's 2.0.)
-constexpr int TRSM_WAVES = 8, TRSM_LOADER = 4, TRSM_UPDATERS = 6, TRSM_TILES = 11, TRSM_FEW = 2;
+constexpr int TRSM_WAVES = 8, TRSM_LOADER = 4, TRSM_UPDATERS = 6, TRSM_TILES = 11, TRSM_SOME = 5, TRSM_FEW = 2;
 template <int TILES>
 constexpr int TRSM_THREADS = TILES > 0 ? 64 * TRSM_WAVES : 64;
 
@@ -731,7 +733,7 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
   __shared__ T tri[AHEAD][17][TRI_LD];
   constexpr int REAL = sizeof(T) == 8 ? AHEAD : 1;      // (complex has none of these)
   __shared__ double diag_inv[REAL][4][64], op_tri[REAL][4][64];  // operands of solve16, the first zero outside the 4 x 4 triangles
-  __shared__ double op_left[REAL][4][64];               // the tile to the left of the triangle
+  __shared__ TS op_left[REAL][4][64];                   // the tile to the left of the triangle (float: two workgroups of 512 rows fit)
   __shared__ int singular;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
   const int n = a.rows, nb = (n + 15) / 16, col0 = blockIdx.x * 16;
@@ -841,7 +843,7 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
   auto place_left = [&](int k, const TS(&c)[4]) {
     if constexpr (sizeof(T) == 8) {
 #pragma unroll
-      for (int v = 0; v < 4; v++) op_left[k % AHEAD][v][lane] = (double)c[v];
+      for (int v = 0; v < 4; v++) op_left[k % AHEAD][v][lane] = c[v];
     }
   };
   TS raw[2][4], left[2][4];
@@ -866,7 +868,7 @@ __global__ __launch_bounds__(TRSM_THREADS<TILES>, TILES == TRSM_TILES ? 2 : 4) v
         if (k > 0) {  // what the tile to the left takes, in two chains and apart from acc
           double l[4], x[4];
 #pragma unroll
-          for (int v = 0; v < 4; v++) l[v] = op_left[k % AHEAD][v][lane], x[v] = before.v[v];
+          for (int v = 0; v < 4; v++) l[v] = (double)op_left[k % AHEAD][v][lane], x[v] = before.v[v];
           if (!known) {
 #pragma unroll
             for (int v = 0; v < 4; v++) x[v] = X[((k - 1) * 16 + 4 * v + q) * 16 + r16];

@@ -433,3 +433,10 @@ def test_in_place_and_shared_storage(hip):
     hip._check(hip._lib.nxh_triangular_solve(hip._h, C.byref(db), C.byref(dl), C.byref(db), 0))
     assert hip.last_path() == "triangular_blocked_workspace"
     assert np.array_equal(logical(tb), x)
+
+
+@pytest.mark.parametrize("name", ["float32", "float64"])
+@pytest.mark.parametrize("n", [223, 224, 225, 241, 496, 497, 511, 512, 513])
+def test_triangular_solve_where_its_forms_change(hip, name, n):
+    """Fourteen blocks of rows, thirty-two (float32), and one more."""
+    test_triangular_solve_at_block_edges(hip, name, n, 17)

@@ -43,7 +43,14 @@ def named(kernels, part):
 
 
 @pytest.mark.parametrize("part", ["trsm_block_kernelI4cplxIdES2_Li11E", "trsm_block_kernelI4cplxIdES2_Li0E", "trsm_block_kernelIddLi11E",
-                                  "trsm_block_kernelIddLi2E", "trsm_block_kernelIddLi0E"])
+                                  "trsm_block_kernelIddLi2E", "trsm_block_kernelIddLi0E", "trsm_block_kernelIdfLi11E", "trsm_block_kernelIdfLi5E",
+                                  "trsm_block_kernelIdfLi2E", "trsm_block_kernelIdfLi0E"])
 def test_no_scratch(kernels, part):
     k = named(kernels, part)
     assert k[".private_segment_fixed_size"] == 0 and k[".vgpr_spill_count"] == 0
+
+
+def test_two_float32_solves_share_a_unit(kernels):
+    """Workgroups of eight waves and up to 512 rows of sixteen sides in float64: 512 registers a lane of a SIMD, 160 KB of LDS."""
+    k = named(kernels, "trsm_block_kernelIdfLi5E")
+    assert k[".vgpr_count"] + k[".agpr_count"] <= 128 and k[".group_segment_fixed_size"] + 512 * 16 * 8 <= 80 << 10
