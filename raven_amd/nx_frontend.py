@@ -45,7 +45,8 @@ def _broadcast_unequal(a: tuple, b: tuple) -> tuple:
     return tuple(out)
 
 
-_ENCODED: dict = {}  # (dtype name, Python value) -> its encoded storage element
+# (dtype name, type, Python value, its text where equal values may differ: zeros and complex numbers) -> its encoded storage element
+_ENCODED: dict = {}
 
 
 def _left(*operands):
@@ -77,7 +78,8 @@ class Nx:
 
     def scalar(self, dtype: dt.DType, value):
         """frontend.ml:360: ``B.full ctx dt [||] value``."""
-        key = (dtype.name, value)
+        kind = type(value)
+        key = (dtype.name, kind, value, "" if value and (kind is float or kind is int) else repr(value))
         enc = _ENCODED.get(key)
         if enc is None:
             enc = encode_scalar(dtype, value)
