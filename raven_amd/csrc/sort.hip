@@ -25,6 +25,9 @@
 //                chunks are sorted in LDS, then each merge level runs its
 //                long-distance exchanges as passes over global memory and
 //                finishes the short-distance ones in LDS;
+//   sort_split   slices of up to 131072 packed words whose keys have four digits:
+//                tiles are sorted, cut into even parts and sorted again (see "slices
+//                of some tiles" below);
 //   sort_radix   longer slices of packed words: a stable radix sort over the key
 //                half (see "a radix sort" below).
 
@@ -1168,7 +1171,7 @@ int split_run(nxh_context *ctx, const char *op, SortArgs &a) {
   p.words = (double *)scratch.p[0];
   p.samples = (double *)scratch.p[1];
   p.cuts = (uint32_t *)(p.samples + a.slices * p.tiles * SPLIT_SAMPLES);
-  nxh_set_path("sort_radix");  // the name of every long form of packed words
+  nxh_set_path("sort_split");
   hipLaunchKernelGGL((split_tiles_kernel<DT>), dim3((unsigned)(a.slices * p.tiles)), dim3(256), 0, ctx->stream, a, p);
   hipLaunchKernelGGL(split_cuts_kernel, dim3((unsigned)(a.slices * p.tiles)), dim3(256), 0, ctx->stream, p);
   hipLaunchKernelGGL((split_parts_kernel<ARG ? NXH_F32 : DT, ARG>), dim3((unsigned)(a.slices * p.parts)), dim3(256), 0, ctx->stream, a, p);
@@ -1197,7 +1200,8 @@ int psort_run(nxh_context *ctx, const char *op, SortArgs &a) {
     return NXH_OK;
   }
   // Sorted tiles and parts against a radix sort that needs all four of its passes (argsort, us): [64,50257] 84 / 117, [1,50257]
-  // 41 / 57, [1,4097] 32 / 50, [200,6000] 56 / 78, [24,131072] 96 / 110, [1000,9000] 198 / 254. Of three passes (float16), with cuts
+  // 41 / 57, [1,4097] 32 / 50, [200,6000] 56 / 78, [24,131072] 96 / 110, [1000,9000] 198 / 254; with nearly half of
+  // the words padding, in many slices, [20000,4097] 1 921 / 2 839. Of three passes (float16), with cuts
   // that took up to 20 us more, 83 / 93, 44 / 46, 41 / 42, 64 / 62, 100 / 87, 210 / 201, of two (bfloat16) 86 / 64: those stay.
   if constexpr (__builtin_popcount(rx_pass_mask<DT>()) == 4) {
     if (a.n <= SPLIT_TILES * 4096 && !sort_meets_input<DT>(a, MODE >= ARG_ASC ? 4 : (int)sizeof(typename Tr<DT>::S)))

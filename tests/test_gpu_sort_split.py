@@ -31,6 +31,7 @@ def test_any_distribution(hip, d, slices, n):
         for desc in (False, True):
             order = np.stack([np.argsort(-r.astype(np.float64) if desc else r, kind="stable") for r in raw])
             same_bits(logical(hip.argsort(x, 1, desc)), order.astype(np.int32), f"{name} {desc}")
+            assert hip.last_path() == "sort_split"
             same_bits(logical(hip.sort(x, 1, desc)), np.take_along_axis(raw, order, 1), f"{name} {desc}")
 
 
@@ -45,6 +46,7 @@ def test_numbers_that_are_none_and_zeros(hip, n):
         wide = np.nan_to_num(v, nan=0.0, posinf=np.inf, neginf=-np.inf).astype(np.float64)
         order = np.stack([np.lexsort((-w if desc else w, np.isnan(r))) for w, r in zip(wide, v)])
         same_bits(logical(hip.argsort(x, 1, desc)), order.astype(np.int32), f"{desc}")
+        assert hip.last_path() == "sort_split"
         got = logical(hip.sort(x, 1, desc)).view(np.uint32)
         finite = ~np.isnan(np.take_along_axis(v, order, 1))
         want = np.take_along_axis(bits, order, 1)
@@ -62,4 +64,17 @@ def test_in_place_and_views(hip):
     v[::7] = 0.5  # (in place, the sign of a zero may be that of another one)
     y = hip.copy(hip.permute(hip.reshape(hip.from_host(v, dt.float32), (6000, 3)), (1, 0)))
     hip._check(hip._lib.nxh_sort(hip._h, y._desc(), y._desc(), 1, 0))
+    assert hip.last_path() == "sort_radix", "parts read the tiles' elements after other parts have been written"
     assert np.array_equal(logical(y), np.sort(v.T, axis=1))
+
+
+@pytest.mark.parametrize("d,n,path", [
+    (dt.float32, 4096, "sort_registers"), (dt.float32, 4097, "sort_split"), (dt.float32, 131072, "sort_split"), (dt.float32, 131073, "sort_radix"),
+    (dt.int32, 131072, "sort_split"), (dt.uint32, 131073, "sort_radix"), (dt.float16, 4097, "sort_radix"), (dt.bfloat16, 8192, "sort_radix"),
+    (dt.int16, 5000, "sort_radix")], ids=str)
+def test_which_slices_are_split(hip, d, n, path):
+    x = hip.cast(hip.reshape(hip.from_host(np.arange(n, 0, -1).astype(np.float32), dt.float32), (1, n)), d)
+    hip.sort(x, 1, False)
+    assert hip.last_path() == path
+    hip.argsort(x, 1, True)
+    assert hip.last_path() == path

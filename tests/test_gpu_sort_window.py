@@ -89,8 +89,8 @@ def test_sort_and_argsort_match_oracle(hip, oracle, d):
 
 def path_for(n):
     # packed dtypes ((key, index) pairs take sort_lds / sort_global): slices that pad to 4096 elements
-    # or fewer are sorted in registers, longer ones by radix
-    return "sort_registers" if n <= 4096 else "sort_radix"
+    # or fewer are sorted in registers, float32 ones of up to 32 such tiles as tiles and parts, longer ones by radix
+    return "sort_registers" if n <= 4096 else "sort_split" if n <= 32 * 4096 else "sort_radix"
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 64, 65, 128, 129, 300, 512, 1000, 1024, 1025, 2048, 2049, 4096, 4097, 12000, 16383, 16384, 16385, 20000, 70001])
@@ -119,7 +119,7 @@ def test_radix_sort_matches_oracle(hip, oracle, d):
     ties, both zeros, NaNs and the extremes, both directions, sort and argsort, two slices of a
     length that is no multiple of the tile, and a strided axis."""
     rng = np.random.default_rng(600 + d.tag)
-    n = 16384 + 4096 + 37
+    n = (32 * 4096 if d in (dt.float32, dt.int32, dt.uint32) else 16384 + 4096) + 37  # (shorter ones of four digits are not sorted by radix)
     x = values_for(d, (2, n), rng, oracle)
     h, o = pair(x, d, hip, oracle)
     for desc in (False, True):
