@@ -16,7 +16,8 @@
    - dtype tags equal Nx's Dtype.Packed.tag (nx_c.h:130-200).
    - every call is asynchronous on the context's stream; nxh_memcpy_d2h and
      nxh_synchronize wait for it, nxh_gather and nxh_scatter until their indices
-     have been looked through (their result is in stream order, as any other's).
+     have been looked through (their result is in stream order, as any other's),
+     the linear algebra calls as said there.
    - return value: NXH_OK, NXH_INVALID_ARGUMENT (the reference raises
      Invalid_argument) or NXH_FAILURE (the reference raises Failure); the
      message, prefixed "<op>: " like the reference's, is read with
@@ -377,7 +378,10 @@ int nxh_irfft(nxh_context *ctx, const nxh_tensor *out, const nxh_tensor *x,
    text as the message's tail (nx_c_linalg.h:29-36; nx_backend.ml:573-591 lifts
    them to Linalg_error by that suffix): "matrix is not positive definite",
    "triangular matrix is singular", "eigenvalue iteration did not converge".
-   Every call waits for the stream (the failure belongs to the call). */
+   The failure belongs to the call: nxh_cholesky and nxh_triangular_solve wait
+   until it is known whether there is one, nxh_qr has none, and their results are
+   in stream order, as any other call's (nothing but this context may read them
+   before nxh_synchronize); the others wait for the stream. */
 
 /* cholesky (backend_intf.ml:640-646; nx_c_tri.c:303-400): reads the lower
    triangle; out = L (upper == 0) or U = L^H, the other triangle zero. */

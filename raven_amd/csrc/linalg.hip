@@ -1049,7 +1049,7 @@ static int *la_status(nxh_context *ctx) { return ctx->fault_flag + 1; }
 
 static int la_begin(nxh_context *ctx, const char *op) {
   std::lock_guard<std::mutex> g(ctx->mu);
-  if (ctx->capture) return nxh_fail(NXH_FAILURE, op, "factorisations report numeric failures by waiting for the stream: not recorded into a graph");
+  if (ctx->capture) return nxh_fail(NXH_FAILURE, op, "factorisations fail where a matrix does, which a recorded call cannot: not recorded into a graph");
   NXH_HIP(op, hipSetDevice(ctx->device));
   return NXH_OK;
 }
@@ -1457,7 +1457,8 @@ NXH_EXPORT int nxh_cholesky(nxh_context *ctx, const nxh_tensor *out, const nxh_t
   const int64_t n = p.rows;
   if (p.batch == 0 || n == 0) return NXH_OK;
   if ((rc = la_check_out(op, out))) return rc;
-  // one factorisation at a time per context: they share the status word and its host slot
+  // one factorisation at a time per context: they share the word that a failure is put in and its report (or, where many
+  // small complex matrices take a workgroup each, the status word and its host slot)
   std::lock_guard<std::mutex> whole_call(ctx->call_mu);
   if ((rc = la_begin(ctx, op))) return rc;
   HostStatus status(ctx);
@@ -1513,7 +1514,7 @@ NXH_EXPORT int nxh_triangular_solve(nxh_context *ctx, const nxh_tensor *out, con
   if ((rc = same_dims(op, b, a, n, nrhs)) || (rc = same_dims(op, out, a, n, nrhs))) return rc;
   if (p.batch == 0 || n == 0 || nrhs == 0) return NXH_OK;
   if ((rc = la_check_out(op, out))) return rc;
-  // one factorisation at a time per context: they share the status word and its host slot
+  // one factorisation at a time per context, as above
   std::lock_guard<std::mutex> whole_call(ctx->call_mu);
   if ((rc = la_begin(ctx, op))) return rc;
   HostStatus status(ctx);
@@ -1568,7 +1569,7 @@ NXH_EXPORT int nxh_qr(nxh_context *ctx, const nxh_tensor *q, const nxh_tensor *r
   if (m == 0 || n == 0) {  // nothing to factor: Q is the identity (if it has elements), R is empty
     if (m == 0 || nq == 0) return NXH_OK;
   }
-  // one factorisation at a time per context: they share the status word and its host slot
+  // several locked steps: no capture may begin between them
   std::lock_guard<std::mutex> whole_call(ctx->call_mu);
   if ((rc = la_begin(ctx, op))) return rc;
   Work work(ctx);
