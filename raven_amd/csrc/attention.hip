@@ -451,7 +451,7 @@ __global__ __launch_bounds__(128) void attention_kernel(AttArgs a) {
 // Before -> now, us: [b,12,1024,64] bfloat16 causal, b = 1 / 2 / 4 / 8 / 16: 18.7 / 20.2 / 22.9 / 39.1 / 74.3 -> 15.5 / 17.4 /
 // 20.3 / 33.8 / 63.3; without a mask, b = 8: 62.2 -> 53.8; a mask tensor, b = 4: 105.6 -> 41.2;
 // [8,12,1024,64] float16 causal 53.2 -> 46.1, [8,16,1000,32] 31.4 -> 28.0, [8,8,2048,128] 154 -> 141.
-// Four waves a SIMD (128 registers) against three: b = 16 61 against 67, b = 8 33.8 and 34.1.
+// Four waves a SIMD (128 registers) against three, in turn on one card: b = 16 61 against 67, b = 8 33.8 and 34.1.
 template <class EL, int DHEAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DHEAD <= 64 ? 4 : 2))) void attention_split_kernel(AttArgs a) {
   using S = uint16_t;
