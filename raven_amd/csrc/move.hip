@@ -84,15 +84,19 @@ struct GatherRowsArgs {
 };
 // With a report, block 0 does nothing but look through the indices, and the caller goes on while the others still move
 // rows: a gather of 8 192 rows of 3 KB, a fill and a scatter into [50257, 768] f32, one after the other: 146 us where
-// gather and scatter waited for the stream, 133 with their reports.
-template <class V>
+// gather and scatter waited for the stream, 133 with their reports. Without one (more rows than a block looks through in time, a
+// recorded graph) the kernel is another one: the look's 53 registers for 11 cost waves that have a short
+// row each (a million rows of [1000000,2] float32: 143 us before the look, 164 with its registers, 140).
+template <class V, bool LOOKS>
 __global__ __launch_bounds__(256) void gather_rows_kernel(GatherRowsArgs a) {
-  if (a.report.word && blockIdx.x == 0) {
-    const bool bad = any_out_of_range(a.idx, a.idx_stride, a.rows, a.axis_len);
-    if (threadIdx.x == 0) nxh_report(a.report.word, a.report.seq, bad);
-    return;
+  if constexpr (LOOKS) {
+    if (blockIdx.x == 0) {
+      const bool bad = any_out_of_range(a.idx, a.idx_stride, a.rows, a.axis_len);
+      if (threadIdx.x == 0) nxh_report(a.report.word, a.report.seq, bad);
+      return;
+    }
   }
-  const int64_t row = (int64_t)(blockIdx.x - (a.report.word != nullptr)) * 4 + (threadIdx.x >> 6);
+  const int64_t row = (int64_t)(blockIdx.x - LOOKS) * 4 + (threadIdx.x >> 6);
   if (row >= a.rows) return;
   int64_t index = a.idx[row * a.idx_stride];
   if (index < 0) index += a.axis_len;
@@ -240,11 +244,16 @@ NXH_EXPORT int nxh_gather(nxh_context *ctx, const nxh_tensor *out, const nxh_ten
     nxh_set_path("gather_rows");
     const bool v16 = a.row_bytes % 16 == 0 && ((uintptr_t)dbase % 16) == 0 && ((uintptr_t)obase % 16) == 0 &&
                      (a.data_row_stride * es) % 16 == 0 && (a.out_row_stride * es) % 16 == 0;
-    if (v16) hipLaunchKernelGGL((gather_rows_kernel<G16>), dim3(blocks), dim3(256), 0, ctx->stream, a);
-    else if (es == 8 || es == 16) hipLaunchKernelGGL((gather_rows_kernel<uint64_t>), dim3(blocks), dim3(256), 0, ctx->stream, a);
-    else if (es == 4) hipLaunchKernelGGL((gather_rows_kernel<uint32_t>), dim3(blocks), dim3(256), 0, ctx->stream, a);
-    else if (es == 2) hipLaunchKernelGGL((gather_rows_kernel<uint16_t>), dim3(blocks), dim3(256), 0, ctx->stream, a);
-    else hipLaunchKernelGGL((gather_rows_kernel<uint8_t>), dim3(blocks), dim3(256), 0, ctx->stream, a);
+    const auto launch = [&](auto looks_c) {
+      constexpr bool LOOKS = decltype(looks_c)::value;
+      const auto kern = v16                  ? gather_rows_kernel<G16, LOOKS>
+                        : es == 8 || es == 16 ? gather_rows_kernel<uint64_t, LOOKS>
+                        : es == 4            ? gather_rows_kernel<uint32_t, LOOKS>
+                        : es == 2            ? gather_rows_kernel<uint16_t, LOOKS>
+                                             : gather_rows_kernel<uint8_t, LOOKS>;
+      hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, ctx->stream, a);
+    };
+    looks ? launch(std::true_type{}) : launch(std::false_type{});
   } else {
     GatherAnyArgs a;
     a.data = dbase;

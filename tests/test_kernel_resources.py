@@ -54,3 +54,9 @@ def test_two_float32_solves_share_a_unit(kernels):
     """Workgroups of eight waves and up to 512 rows of sixteen sides in float64: 512 registers a lane of a SIMD, 160 KB of LDS."""
     k = named(kernels, "trsm_block_kernelIdfLi5E")
     assert k[".vgpr_count"] + k[".agpr_count"] <= 128 and k[".group_segment_fixed_size"] + 512 * 16 * 8 <= 80 << 10
+
+
+@pytest.mark.parametrize("vector", ["h", "t", "j", "m", "3G16"])
+def test_gathers_that_do_not_look_have_few_registers(kernels, vector):
+    """A wave has a row, often a short one: what it needs before its first load is what many rows cost."""
+    assert named(kernels, f"gather_rows_kernelI{vector}Lb0E")[".vgpr_count"] <= 16
