@@ -534,6 +534,7 @@ __global__ __launch_bounds__(256) void scatter_rows_kernel(ScatterArgs a, int64_
   }
 }
 constexpr int SCATTER_RANGE = 1024;  // rows of a block's range, at most
+constexpr int SCATTER_LIST = 1024;   // updates that a block orders at a time
 // out = a copy of `from`, then whole rows of updates, in one pass over the table. `out` and `from` are dense, one row
 // of `row` elements after another, and start on 16 bytes, as do the blocks' ranges of `range_rows` rows. A block looks
 // through all indices for those of its range (sixteen loads of a lane in flight, out of L2) and puts them in the order
@@ -543,8 +544,7 @@ constexpr int SCATTER_RANGE = 1024;  // rows of a block's range, at most
 // than DIRECT updates, whose lanes request a dozen at a time, and blocks with more than LIST updates, in spans of positions that
 // the list takes. Either way an element's updates come in the order of their positions, each rounded to the storage
 // type; of those that are set only the last is read. What one row takes is one block's work (8 192 updates of one row of 768 f32: 613 us,
-// 1 920 in scatter_rows; one at a time and 1 024 positions a span 3 260; [1048576,2] with a million updates 1 470, 1 980
-// and 4 700). Bound by the copy, which streaming stores decide (`stream`): [50257,
+// 1 920 in scatter_rows; one at a time and 1 024 positions a span 3 260). Bound by the copy, which streaming stores decide (`stream`): [50257,
 // 768] f32 with 8 192 updates from the cache 47 us, with plain stores 67 (a copy alone 39); with updates from memory 66,
 // where a copy and scatter_rows take 43 and 33, and scatter_rows with `from`, whose lanes own columns and copy one row
 // after another, some 150.
@@ -556,7 +556,7 @@ __global__ __launch_bounds__(256) void scatter_copy_kernel(ScatterArgs a, int64_
   struct alignas(V > 1 ? 16 : alignof(E)) S {
     E v[V];
   };
-  constexpr int LIST = 1024, LOOK = 16, EACH = 4, DIRECT = 16;
+  constexpr int LIST = SCATTER_LIST, LOOK = 16, EACH = 4, DIRECT = 16;
   __shared__ uint64_t list[LIST];         // (row of the range << 32 | position), in any order, then in theirs
   __shared__ uint32_t position[LIST];     // the positions alone
   __shared__ uint16_t start[SCATTER_RANGE], stop[SCATTER_RANGE], updated[LIST];  // a row's part of it; rows that `apply` updates
@@ -988,14 +988,30 @@ static int scatter_impl(nxh_context *ctx, const nxh_tensor *out, const nxh_tenso
     const bool rows16 = es < 16 && line % 16 == 0 && a.a_ustride * es % 16 == 0 && (uintptr_t)a.upd % 16 == 0;
     const int64_t aim = std::min(std::max<int64_t>(48 << 10, a.n_idx * 6), std::max<int64_t>(4 << 10, bytes / (2 * ctx->compute_units)));
     int64_t range = std::min<int64_t>(SCATTER_RANGE, std::max<int64_t>(1, aim / line));
+    // A list that does not take all of a block's updates costs a second look through the indices and a turn a span: what it
+    // holds with a margin (`hold` rows) bounds the range, unless that is over twice the blocks of a full chip; fewer
+    // blocks than the chip takes are made down to a quarter of the list, a word a lane. Float32 add, us, copy and scatter /
+    // without this / so: 4 000 updates into [1000,2] 23 / 74 / 12, 40 000 into [10000,2] 86 / 120 / 29, 400 000 into [100000,2] 747 / 416 / 211; 2 000 000 into
+    // [2000000,3] bfloat16 3 640 / 4 460 / 2 740.
+    const int64_t hold = SCATTER_LIST * 7 / 8 * a.axis_len / a.n_idx, chip = a.axis_len / (2 * ctx->compute_units);
+    const int64_t dense = std::max(hold / 4, 2 * hold >= range ? std::min(chip, hold) : chip);
+    range = std::max<int64_t>(1, std::min(range, dense));
     if (rows16) {
       if (range * (line / 16) >= 1 << 16) range = std::max<int64_t>(1, 65535 / (line / 16));
     } else {
       const int64_t some = std::max<int64_t>(1, 16 / es);
       range = (range + some - 1) / some * some;  // whole vectors, whatever the row
+      if (range > hold && range > some) range -= some;
     }
     const bool fits = range * line <= aim + aim / 4 || (rows16 ? range * line <= 64 << 10 : range * a.columns <= 12288);
-    if (rows && fits && ((uintptr_t)a.out | (uintptr_t)a.from) % 16 == 0 && a.n_idx <= 4 * a.axis_len && a.n_idx <= 0x7fffffff) {
+    // Every block looks through all indices, the older forms' three a unit do too, at a quarter of the rate: more looks than
+    // twelve a unit have to be worth less than the copy they save, 2 bytes for each of the table's, or 40 up to 64 MiB,
+    // where the older form is one pass that moves short rows one after another. Float32 add, us, older / here:
+    // 3 000 updates into [10000000,2] 49 / 36, 10 000 63 / 78, into [10000000,8] 145 / 112, 30 000 190 / 196; 100 000 into
+    // [5000000,3] 444 / 285, 1 000 000 2 160 / 2 720; 2 100 000 into [3000000,2] 4 046 / 3 654, 4 500 000 8 550 / 12 350.
+    const int64_t looks = (a.axis_len + range - 1) / range * (range > hold ? 2 : 1);
+    const bool seen = (double)(looks - 12 * ctx->compute_units) * 4.0 * (double)a.n_idx <= (double)bytes * (bytes > (64 << 20) ? 2.0 : 40.0);
+    if (rows && fits && seen && ((uintptr_t)a.out | (uintptr_t)a.from) % 16 == 0 && a.n_idx <= 4 * a.axis_len && a.n_idx <= 0x7fffffff) {
       std::lock_guard<std::mutex> guard(ctx->mu);
       if (ctx->capture) return -1;
       NXH_HIP(op, hipSetDevice(ctx->device));

@@ -80,6 +80,17 @@ def test_rows_that_many_updates_hit(hip, cols, most):
             same_bits(logical(got), logical(two_launches(hip, mode, template, index, updates)), f"{name} {mode}")
 
 
+def seconds(hip, f):
+    best = 1.0
+    for _ in range(5):
+        hip.synchronize()
+        t = time.perf_counter()
+        f()
+        hip.synchronize()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
 @pytest.mark.parametrize("mode", ["add", "set"])
 @pytest.mark.parametrize("cols", [768, 770])
 def test_one_row_for_all_costs_no_more_than_two_launches(hip, mode, cols):
@@ -88,19 +99,9 @@ def test_one_row_for_all_costs_no_more_than_two_launches(hip, mode, cols):
     template, updates = hip.full(dt.float32, (50257, cols), 0.0), hip.full(dt.float32, (8192, cols), 1.0)
     index = rows_of(hip, np.full(8192, 7), cols)
 
-    def seconds(f):
-        best = 1.0
-        for _ in range(5):
-            hip.synchronize()
-            t = time.perf_counter()
-            f()
-            hip.synchronize()
-            best = min(best, time.perf_counter() - t)
-        return best
-
-    one = seconds(lambda: hip.scatter(mode, False, template, index, updates, 0))
+    one = seconds(hip, lambda: hip.scatter(mode, False, template, index, updates, 0))
     assert hip.last_path() == "scatter_copy"
-    assert one < seconds(lambda: two_launches(hip, mode, template, index, updates))
+    assert one < seconds(hip, lambda: two_launches(hip, mode, template, index, updates))
 
 
 @pytest.mark.parametrize("rows,cols,n,one_pass", [
@@ -117,3 +118,28 @@ def test_long_rows_are_not_left_to_a_few_blocks(hip, rows, cols, n, one_pass):
         got = hip.scatter(mode, False, template, index, updates, 0)
         assert (hip.last_path() == "scatter_copy") == one_pass, hip.last_path()
         same_bits(logical(got), logical(two_launches(hip, mode, template, index, updates)), mode)
+
+
+@pytest.mark.parametrize("rows,cols,n,one_pass", [
+    (1000, 2, 4000, True), (10000, 3, 40000, True), (224, 4, 896, True), (225, 7, 900, True), (120001, 4, 120000, True), (1000000, 3, 1500000, True),
+    (120001, 3, 480004, True), (3300000, 2, 200000, True), (3300000, 2, 3300000, False), (8400000, 2, 8400, False)])
+def test_dense_updates_of_narrow_tables(hip, rows, cols, n, one_pass):
+    """Ranges that a block's list bounds, and tables whose many blocks would read more indices than the copy they save is worth."""
+    rng = np.random.default_rng(n)
+    template = hip.reshape(hip.from_host(rng.standard_normal((rows, cols)).astype(np.float32), dt.float32), (rows, cols))
+    updates = hip.reshape(hip.from_host(rng.standard_normal((n, cols)).astype(np.float32), dt.float32), (n, cols))
+    index = rows_of(hip, rng.integers(-rows, rows, n), cols)
+    for mode in ("add", "set"):
+        got = hip.scatter(mode, False, template, index, updates, 0)
+        assert (hip.last_path() == "scatter_copy") == one_pass, hip.last_path()
+        same_bits(logical(got), logical(two_launches(hip, mode, template, index, updates)), mode)
+
+
+def test_dense_updates_cost_no_more_than_two_launches(hip):
+    """Four updates a row of a narrow table (12 us a call among others; copied and scattered 23)."""
+    rows, n = 1000, 4000
+    template, updates = hip.full(dt.float32, (rows, 2), 0.0), hip.full(dt.float32, (n, 2), 1.0)
+    index = rows_of(hip, np.arange(n) % rows, 2)
+    one = seconds(hip, lambda: hip.scatter("add", False, template, index, updates, 0))
+    assert hip.last_path() == "scatter_copy"
+    assert one < seconds(hip, lambda: two_launches(hip, "add", template, index, updates))
