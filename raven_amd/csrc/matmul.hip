@@ -272,8 +272,9 @@ __global__ __launch_bounds__(256) void gemm_skinny_mfma_kernel(SkinnyArgs a) {
 
 // ── gemm_skinny_mfma_k8: the same stream when N alone fills the chip ────────
 // One block of eight waves owns 64 columns; the waves take the steps of K in turn, so that a block reads
-// rows that follow each other ([8,4096] x [4096,16384] bfloat16 with weights from memory: 27.2 us; a
-// contiguous eighth of K a wave, 16 MB from one to the next, took 29.1), and fold their
+// rows that follow each other ([8,4096] x [4096,16384] bfloat16 with weights from memory: 26.9 us; a
+// contiguous eighth of K a wave, 16 MB from one to the next, took 29.1). Rows are numbered in 32 bits (K is
+// below 2^31 here): in 64 a long K took longer than the eighths did (K = 16384 104 us, 102 and now 101). The waves fold their
 // accumulators through LDS in wave order at the end, so there are no f32 partials in memory
 // and no second launch. A (at most 16 x K, a few dozen KiB, resident in L2) is not staged:
 // each lane reads its 16-byte fragment of the step straight from memory, three steps ahead
@@ -288,14 +289,14 @@ __global__ __launch_bounds__(64 * SM8_WAVES) void gemm_skinny_mfma_k8_kernel(Ski
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t n0 = (int64_t)blockIdx.x * SM_WN;
   // step s of this wave: rows [(8 s + wave) SM_KS, .. + SM_KS) of B, as far as they are below K (a multiple of 8)
-  const int64_t k0 = (int64_t)wave * SM_KS, kn = a.K - k0;
-  constexpr int64_t STRIDE = SM8_WAVES * SM_KS;
+  const int k0 = wave * SM_KS, kn = (int)a.K - k0;
+  constexpr int STRIDE = SM8_WAVES * SM_KS;
   const uint16_t *A = (const uint16_t *)a.A;
   const uint16_t *B = (const uint16_t *)a.B;
   uint16_t *sB = sm_lds + wave * (2 * SM_TILE);
   const int c8 = (lane & 7) * 8, rbase = lane >> 3;
   const bool col_ok = n0 + c8 < a.N;
-  const uint16_t *bp = B + k0 * a.brs + n0 + c8;
+  const uint16_t *bp = B + (int64_t)k0 * a.brs + n0 + c8;
   const int g = lane >> 4, L = lane & 15;
   const uint16_t *ap = A + (int64_t)L * a.ars + k0 + g * 8;  // rows >= M read as zero
   const bool row_ok = L < a.M;
@@ -303,10 +304,10 @@ __global__ __launch_bounds__(64 * SM8_WAVES) void gemm_skinny_mfma_k8_kernel(Ski
   auto load = [&](U4 (&r)[4], U4 &x, int step) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int64_t kk = step * STRIDE + rbase + i * 8;
-      r[i] = (col_ok && kk < kn) ? *reinterpret_cast<const U4 *>(bp + kk * a.brs) : U4{0, 0, 0, 0};
+      const int kk = step * STRIDE + rbase + i * 8;
+      r[i] = (col_ok && kk < kn) ? *reinterpret_cast<const U4 *>(bp + (int64_t)kk * a.brs) : U4{0, 0, 0, 0};
     }
-    const int64_t ka = step * STRIDE + g * 8;
+    const int ka = step * STRIDE + g * 8;
     x = (row_ok && ka < kn) ? *reinterpret_cast<const U4 *>(ap + step * STRIDE) : U4{0, 0, 0, 0};
   };
   auto store = [&](const U4 (&r)[4], int buf) {
@@ -317,7 +318,7 @@ __global__ __launch_bounds__(64 * SM8_WAVES) void gemm_skinny_mfma_k8_kernel(Ski
   f32x4 acc[4];
 #pragma unroll
   for (int t = 0; t < 4; t++) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  const int nsteps = kn > 0 ? (int)((kn + STRIDE - 1) / STRIDE) : 0;
+  const int nsteps = kn > 0 ? (kn + STRIDE - 1) / STRIDE : 0;
   // step s multiplies the tile in LDS buffer s & 1 by the A fragment of slot s % 3; slot (s + 1) % 3
   // is stored for step s + 1 and refilled with step s + 4
   auto step = [&](int s, auto slot_c) {
@@ -753,7 +754,7 @@ static int launch_skinny_mfma(nxh_context *ctx, GemmArgs &g) {
   const int cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
   // N alone fills the chip with 64-column blocks: K is split inside the block, one launch
   const int64_t strips = (g.N + SM_WN - 1) / SM_WN;
-  if (strips >= cus && g.K % 8 == 0 && g.K >= SM8_WAVES * 2 * SM_KS && (g.M == 1 || (g.acs == 1 && g.ars % 8 == 0)) &&
+  if (strips >= cus && g.K % 8 == 0 && g.K >= SM8_WAVES * 2 * SM_KS && g.K < 0x70000000 && (g.M == 1 || (g.acs == 1 && g.ars % 8 == 0)) &&
       (g.M > 1 || g.acs == 1) && ((uintptr_t)g.A % 16) == 0 && strips <= 0x7fffffffLL) {
     auto kern = gemm_skinny_mfma_k8_kernel<DT == NXH_BF16>;
     constexpr size_t LDS = sizeof(uint16_t) * (size_t)(SM8_WAVES * 2 * SM_TILE);

@@ -193,6 +193,20 @@ def test_matmul_skinny_wide_output(hip, oracle, d, m, k, n):
     assert np.array_equal(logical(hip.matmul(ha, hb)), logical(hip.matmul(ha, hb)))
 
 
+@pytest.mark.parametrize("d", [dt.bfloat16, dt.float16], ids=lambda d: d.name)
+@pytest.mark.parametrize("m,k", [(16, 8184), (8, 8192), (8, 8200), (1, 8448), (13, 8456), (3, 12008)])
+def test_matmul_skinny_wide_output_long_k(hip, oracle, d, m, k):
+    """Waves that take the steps of K in turn, the last turn whole, for some waves only, and cut: whole numbers, whose sums are
+    exact in float32 and rounded once, so that no k-value may be left out or taken twice."""
+    rng = np.random.default_rng(k + m)
+    a, b = rng.integers(-2, 3, (m, k)).astype(np.float32), rng.integers(-2, 3, (k, 2049)).astype(np.float32)
+    want = np.tile(encode(a @ b, d, oracle), (1, 8))
+    ha, hb = pair(encode(a, d, oracle), d, hip, oracle)[0], pair(np.tile(encode(b, d, oracle), (1, 8)), d, hip, oracle)[0]
+    got = logical(hip.matmul(ha, hb))
+    assert hip.last_path() == "gemm_skinny_mfma_k8"
+    assert np.array_equal(got, want)
+
+
 @pytest.mark.parametrize("m,k,n", [(8, 1024, 16384), (1, 515, 16388), (16, 4096, 16384), (13, 770, 17000)],
                          ids=lambda v: str(v))
 def test_matmul_skinny_wide_output_f32(hip, oracle, m, k, n):

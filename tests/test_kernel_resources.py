@@ -60,3 +60,9 @@ def test_two_float32_solves_share_a_unit(kernels):
 def test_gathers_that_do_not_look_have_few_registers(kernels, vector):
     """A wave has a row, often a short one: what it needs before its first load is what many rows cost."""
     assert named(kernels, f"gather_rows_kernelI{vector}Lb0E")[".vgpr_count"] <= 16
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+def test_decoding_products_number_their_rows_in_32_bits(kernels, bf16):
+    """142 registers and as many more instructions a step in 64 bits, which a long K paid for."""
+    assert named(kernels, f"gemm_skinny_mfma_k8_kernelILb{bf16}E")[".vgpr_count"] <= 136
